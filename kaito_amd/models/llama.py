@@ -164,17 +164,19 @@ class LlamaAttention(nn.Module):
                                   meta.slot_mapping)
         sinks = getattr(self, "sinks", None)
         if meta.is_prefill:
+            tiles = None if meta.tile_seq is None else \
+                (meta.tile_seq, meta.tile_qbase)
             if meta.kv_lens is not None:
                 # suffix-query attention over the paged cache (the suffix
                 # K/V was just written by reshape_and_cache above)
                 out = ops.context_attention(qh, kv_cache[0], kv_cache[1],
                                             meta.cu_seqlens, meta.kv_lens,
                                             meta.block_tables, self.scale,
-                                            self.window, sinks)
+                                            self.window, sinks, tiles)
             else:
                 out = ops.prefill_attention(qh, kh, vh, meta.cu_seqlens,
                                             self.scale, meta.max_seqlen,
-                                            self.window, sinks)
+                                            self.window, sinks, tiles)
         else:
             out = ops.paged_attention(qh, kv_cache[0], kv_cache[1],
                                       meta.block_tables, meta.seq_lens,

@@ -24,11 +24,11 @@ for the CDNA4 memory system rather than translated:
     re-gathering over xGMI). At deepseek-v3 scale (128 heads, TP=8)
     each rank holds 16 heads == exactly one kernel head-tile.
   * Prefill runs NON-absorbed: k_nope/v are decompressed from the
-    fresh c_kv (bmm), q/k padded 192->256 and v 128->256 with zeros
-    (exact — zero dims contribute nothing) through the existing
-    D=256 prefill_attention MFMA kernel. MLA prompts are scheduled
-    whole (scheduler.whole_prompt_only), so no context-attention
-    (chunked suffix) variant is needed.
+    fresh c_kv and read, beside the shared rotated key dims, where the
+    projections left them (ops.mla_prefill_attention: 128 + 64 key and
+    128 value dims). Other head layouts are padded with zeros (exact —
+    zero dims contribute nothing) to prefill_attention's 256 dims.
+    Suffixes of chunked prompts attend in the absorbed space.
 
 HF config fields covered: q_lora_rank (0 = direct q projection,
 V2-Lite), kv_lora_rank, qk_nope_head_dim, qk_rope_head_dim, v_head_dim,
@@ -229,13 +229,21 @@ class MLAAttention(nn.Module):
     def _prefill(self, q_nope, q_pe, c_kv, k_pe, meta) -> torch.Tensor:
         T = q_nope.size(0)
         Hl = self.num_heads
-        # decompress: k_nope [Hl, nope, T] = w_kc [Hl, nope, r] @ c_kv^T
-        k_nope = torch.matmul(self.w_kc, c_kv.t().to(self.w_kc.dtype))
-        k_nope = k_nope.permute(2, 0, 1)                # [T, Hl, nope]
+        tiles = None if meta.tile_seq is None else \
+            (meta.tile_seq, meta.tile_qbase)
+        # decompress: k_nope [T, Hl, nope], v [Hl, T, v]
+        k_nope = torch.nn.functional.linear(
+            c_kv.to(self.w_kc.dtype), self.w_kc.view(Hl * self.nope, self.r)
+        ).view(T, Hl, self.nope)
         v = torch.matmul(c_kv.to(self.w_vc.dtype).unsqueeze(0), self.w_vc)
         v = v.transpose(0, 1)                           # [T, Hl, v]
+        if q_nope.is_cuda and q_nope.dtype == torch.bfloat16 and \
+                (self.nope, self.rope, self.v_dim) == (128, 64, 128):
+            return ops.mla_prefill_attention(
+                q_nope, q_pe, k_nope, k_pe, v, meta.cu_seqlens, self.scale,
+                tiles)
 
-        pad = 256                                       # D=256 MFMA kernel
+        pad = 256                                       # other head layouts
         qf = torch.zeros(T, Hl, pad, dtype=q_nope.dtype,
                          device=q_nope.device)
         kf = torch.zeros_like(qf)
@@ -246,5 +254,5 @@ class MLAAttention(nn.Module):
         kf[..., self.nope:self.qk_dim] = k_pe.unsqueeze(1)  # broadcast heads
         vf[..., :self.v_dim] = v
         out = ops.prefill_attention(qf, kf, vf, meta.cu_seqlens, self.scale,
-                                    meta.max_seqlen)
+                                    meta.max_seqlen, tiles=tiles)
         return out[..., :self.v_dim].contiguous()       # [T, Hl, v]

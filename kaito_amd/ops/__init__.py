@@ -26,7 +26,7 @@ for _g, _names in {
              "gelu_and_mul gelu layer_norm fused_add_layer_norm "
              "reshape_and_cache topk"),
     "attn": ("paged_attention paged_attention_sp prefill_attention "
-             "context_attention mfma_tile_gemm paged_read_bw"),
+             "mla_prefill_attention context_attention mfma_tile_gemm paged_read_bw"),
     "mla": "mla_decode mla_cache_write",
     "moe": "moe_gate_silu moe_down_scatter",
     "route": "moe_route moe_sort",
@@ -208,10 +208,13 @@ def mla_cache_write(cache: torch.Tensor, c_kv: torch.Tensor,
 def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                       cu_seqlens: torch.Tensor, scale: float,
                       max_seqlen: int | None = None, window: int = 0,
-                      sinks: torch.Tensor | None = None) -> torch.Tensor:
+                      sinks: torch.Tensor | None = None,
+                      tiles=None) -> torch.Tensor:
+    """Causal attention of whole prompts. `tiles` = (tile_seq, tile_qbase)
+    of build_query_tiles spares a read of cu_seqlens on the host."""
     if q.is_cuda:
         out = torch.empty_like(q)
-        tile_seq, tile_qbase = _build_tiles(cu_seqlens)
+        tile_seq, tile_qbase = tiles or _build_tiles(cu_seqlens)
         _K.prefill_attention(out, q, k, v, tile_seq, tile_qbase,
                                           cu_seqlens, scale, window,
                                           _sinks_arg(sinks, q.device))
@@ -220,16 +223,30 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                                        sinks)
 
 
+def mla_prefill_attention(q, q_pe, k, k_pe, v, cu_seqlens, scale: float,
+                          tiles=None) -> torch.Tensor:
+    """Causal latent attention of whole prompts (GPU, bf16): q [T, H, 128]
+    beside q_pe [T, H, 64], k [T, H, 128] beside k_pe [T, 64] shared by the
+    heads, v [T, H, 128]; token and head strides are free. -> [T, H, 128]."""
+    out = torch.empty(v.shape, dtype=v.dtype, device=v.device)
+    tile_seq, tile_qbase = tiles or _build_tiles(cu_seqlens)
+    _K.mla_prefill_attention(out, q, q_pe, k, k_pe, v, tile_seq, tile_qbase,
+                             cu_seqlens, scale)
+    return out
+
+
 def context_attention(q: torch.Tensor, k_cache: torch.Tensor,
                       v_cache: torch.Tensor, cu_seqlens_q: torch.Tensor,
                       kv_lens: torch.Tensor, block_tables: torch.Tensor,
                       scale: float, window: int = 0,
-                      sinks: torch.Tensor | None = None) -> torch.Tensor:
+                      sinks: torch.Tensor | None = None,
+                      tiles=None) -> torch.Tensor:
     """Suffix-query causal attention over the paged cache (chunked
-    prefill / prefix-cache continuation)."""
+    prefill / prefix-cache continuation). `tiles` as in
+    prefill_attention."""
     if q.is_cuda:
         out = torch.empty_like(q)
-        tile_seq, tile_qbase = _build_tiles(cu_seqlens_q)
+        tile_seq, tile_qbase = tiles or _build_tiles(cu_seqlens_q)
         _K.context_attention(out, q, k_cache, v_cache, tile_seq,
                                           tile_qbase, cu_seqlens_q, kv_lens,
                                           block_tables, scale, window,
@@ -288,21 +305,14 @@ def mfma_tile_gemm(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     return _K.mfma_tile_gemm(a, b)
 
 
-QTILE = 64  # must match prefill_attention.hip
+QTILE = 64  # query tiles of a step's chunks: flash_prefill.h TILE
 
 
 def _build_tiles(cu_seqlens: torch.Tensor):
-    """Map varlen batch → list of 64-row Q tiles: (seq_idx, q_base)."""
+    """build_query_tiles for callers that hold the offsets on the device."""
     cs = cu_seqlens.tolist()
-    seqs, bases = [], []
-    for i in range(len(cs) - 1):
-        L = cs[i + 1] - cs[i]
-        for q0 in range(0, L, QTILE):
-            seqs.append(i)
-            bases.append(q0)
-    dev = cu_seqlens.device
-    return (torch.tensor(seqs, dtype=torch.int32, device=dev),
-            torch.tensor(bases, dtype=torch.int32, device=dev))
+    return build_query_tiles([b - a for a, b in zip(cs, cs[1:])],
+                             cu_seqlens.device)
 
 
 def moe_gate_silu(act: torch.Tensor, x: torch.Tensor,

@@ -32,7 +32,8 @@
 // weights and the output accumulation are f32.
 //
 // Three kernels share these semantics:
-//   window_attention_mfma_kernel   bf16 prompt portions, 64-row query tiles
+//   flash_prefill_kernel           bf16 prompt portions, 64-row query tiles
+//                                  (flash_prefill.h)
 //   window_attention_decode_kernel single rows (and f32 portions), the
 //                                  heads of a kv group in one pass
 //   window_attention_kernel        any sizes: one workgroup per (row, head),
@@ -41,6 +42,7 @@
 //                                  thread-per-value-dim
 // All fold key tiles with the running-max (online softmax) recurrence, so
 // any window length works.
+#include "flash_prefill.h"
 #include "mix_common.h"
 
 namespace kaito {
@@ -404,236 +406,6 @@ __global__ void window_attention_kernel(
   for (int i = 0; i < MAXV; i++) {
     const int j = tid + i * KT;
     if (j < V) act_st(orow + j, acc[i] * inv);
-  }
-}
-
-// ---- MFMA prompt-portion kernel (bf16) -------------------------------------
-// One workgroup = 64 query rows of one chunk x one head; 4 waves x 16 rows.
-// Keys come 32 at a time through LDS: the K tile XOR-swizzled for
-// conflict-free 16-byte fragment reads, the V tile transposed so the P.V
-// B-fragments are contiguous. S = Q K^T and O += P V run on
-// v_mfma_f32_16x16x32_bf16; scaling, capping, the distance penalty, the
-// window/causal mask and the online softmax are f32 on the accumulator
-// fragments; the f32 weights enter the P.V product as a bf16 value +
-// remainder pair. Key and value sizes are separate template parameters.
-constexpr int WQ_TILE = 64;
-constexpr int WKV_TILE = 32;
-constexpr int WPAD = 40;
-
-// DB: distance-bias table and query temperature (a softmax variant)
-template <int D, int DV, bool SIG, bool DB>
-__global__ __launch_bounds__(256, 2) void window_attention_mfma_kernel(
-    short* __restrict__ out,              // [T, H, DV]
-    const short* __restrict__ q,          // [T, H, D]
-    const short* __restrict__ k_cache,    // [blocks, G, BS, D]
-    const short* __restrict__ v_cache,    // [blocks, G, BS, DV]
-    const int* __restrict__ tile_seq, const int* __restrict__ tile_qbase,
-    const int* __restrict__ cu, const int* __restrict__ starts,
-    const int* __restrict__ block_tables, const int max_blocks,
-    const float scale, const float softcap, const float* __restrict__ r1,
-    const float* __restrict__ r2, const int window, const int H, const int G,
-    const int BS, const int keep_first, const float* __restrict__ sinks,
-    const int chunk, const float* __restrict__ pb,
-    const short* __restrict__ gate, const int64_t gate_s0,
-    const float* __restrict__ db, const int db_n, const float temp_coef,
-    const int temp_every) {
-  constexpr int KK = D / 32;
-  constexpr int DT = DV / 16;
-  const int tile = blockIdx.x;
-  const int h = blockIdx.y;
-  const int g = h / (H / G);
-  const int seq = tile_seq[tile];
-  const int q0 = tile_qbase[tile];
-  const int tok0 = cu[seq];
-  const int q_len = cu[seq + 1] - tok0;
-  const int q_abs0 = starts[seq];          // position of the chunk's row 0
-  const int kv_len = q_abs0 + q_len;
-  const int* bt = block_tables + (int64_t)seq * max_blocks;
-  const float hr1 = r1 ? r1[h] : 0.f, hr2 = r1 ? r2[h] : 0.f;
-  const float inv_cap = softcap > 0.f ? 1.0f / softcap : 0.f;
-  const float hpb = SIG ? pb[h] : 0.f;
-
-  const int wave = threadIdx.x >> 6;
-  const int lane = threadIdx.x & 63;
-  const int hi = lane >> 4;
-  const int lo = lane & 15;
-
-  __shared__ short lds_k[WKV_TILE * D];
-  __shared__ short lds_vt[DV * WPAD];
-  // softmax weights as a bf16 pair (value + remainder): two MFMAs per value
-  // tile keep ~16 mantissa bits of the f32 weight in the P.V product
-  __shared__ short lds_p[4][16 * WPAD];
-  __shared__ short lds_pl[4][16 * WPAD];
-  // the tile's bias by q row - key + WKV_TILE - 1
-  __shared__ float lds_db[DB ? WQ_TILE + WKV_TILE : 1];
-
-  const int qrow = q0 + wave * 16 + lo;
-  const int qtok = tok0 + (qrow < q_len ? qrow : q_len - 1);
-  bf16x8 qfrag[KK];
-#pragma unroll
-  for (int kk = 0; kk < KK; kk++)
-    qfrag[kk] = *reinterpret_cast<const bf16x8*>(
-        q + ((int64_t)qtok * H + h) * D + kk * 32 + hi * 8);
-
-  float mrow[4], lrow[4], qsc[4];
-#pragma unroll
-  for (int r = 0; r < 4; r++)
-    qsc[r] = DB ? scale * query_temp(q_abs0 + q0 + wave * 16 + hi * 4 + r,
-                                     temp_coef, temp_every) : scale;
-  f32x4 ofrag[DT];
-#pragma unroll
-  for (int r = 0; r < 4; r++) {
-    mrow[r] = sinks ? sinks[h] : -1e30f;
-    lrow[r] = sinks || SIG ? 1.0f : 0.f;
-  }
-#pragma unroll
-  for (int dt = 0; dt < DT; dt++) ofrag[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int kv_end = min(kv_len, q_abs0 + q0 + WQ_TILE);
-  // first key any row of the tile may see: the window's start of the
-  // tile's first row, or the start of that row's chunk
-  const int vis0 = chunk > 0 ? ((q_abs0 + q0) / chunk) * chunk
-      : (window > 0 ? q_abs0 + q0 - window + 1 : 0);
-  const int kv_begin = vis0 > 0 ? (vis0 / WKV_TILE) * WKV_TILE : 0;
-  // key tiles: those that hold kept first tokens, then the window's
-  const int first_end =
-      min((keep_first + WKV_TILE - 1) / WKV_TILE * WKV_TILE, kv_begin);
-  auto next_tile = [&](const int kv0) {
-    return kv0 + WKV_TILE == first_end ? kv_begin : kv0 + WKV_TILE;
-  };
-  const int kv_first = first_end > 0 ? 0 : kv_begin;
-  // this thread's entry of a tile's bias, fetched a tile ahead
-  auto tile_bias = [&](const int kv0) {
-    const int dist = q_abs0 + q0 - kv0 + (int)threadIdx.x - (WKV_TILE - 1);
-    return DB && threadIdx.x < WQ_TILE + WKV_TILE - 1
-        ? db[(int64_t)h * db_n + min(max(dist, 0), db_n - 1)] : 0.f;
-  };
-  float bias_nxt = DB ? tile_bias(kv_first) : 0.f;
-  for (int kv0 = kv_first; kv0 < kv_end; kv0 = next_tile(kv0)) {
-    for (int i = threadIdx.x; i < WKV_TILE * D / 8; i += 256) {
-      const int row = (i * 8) / D;
-      const int col = (i * 8) % D;
-      const int kvp = min(kv0 + row, kv_len - 1);
-      const int64_t src =
-          (((int64_t)bt[kvp / BS] * G + g) * BS + (kvp % BS)) * D + col;
-      const short8_t kd = *reinterpret_cast<const short8_t*>(k_cache + src);
-      const int swz = (col * 2) ^ ((row & 7) << 4);
-      *reinterpret_cast<short8_t*>(&lds_k[row * D + swz / 2]) = kd;
-    }
-    for (int i = threadIdx.x; i < WKV_TILE * DV / 8; i += 256) {
-      const int row = (i * 8) / DV;
-      const int col = (i * 8) % DV;
-      const int kvp = min(kv0 + row, kv_len - 1);
-      const int64_t src =
-          (((int64_t)bt[kvp / BS] * G + g) * BS + (kvp % BS)) * DV + col;
-      const short8_t vd = *reinterpret_cast<const short8_t*>(v_cache + src);
-#pragma unroll
-      for (int j = 0; j < 8; j++) lds_vt[(col + j) * WPAD + row] = vd[j];
-    }
-    if (DB && threadIdx.x < WQ_TILE + WKV_TILE - 1)
-      lds_db[threadIdx.x] = bias_nxt;
-    __syncthreads();
-    if (DB) bias_nxt = tile_bias(next_tile(kv0));
-
-    f32x4 sfrag[2];
-#pragma unroll
-    for (int kt = 0; kt < 2; kt++) {
-      sfrag[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kk = 0; kk < KK; kk++) {
-        const int krow = kt * 16 + lo;
-        const int swz = ((kk * 32 + hi * 8) * 2) ^ ((krow & 7) << 4);
-        const bf16x8 kf =
-            *reinterpret_cast<const bf16x8*>(&lds_k[krow * D + swz / 2]);
-        sfrag[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            qfrag[kk], kf, sfrag[kt], 0, 0, 0);
-      }
-    }
-
-    float p[2][4];
-#pragma unroll
-    for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int qr = q0 + wave * 16 + hi * 4 + r;
-        const int q_abs = q_abs0 + qr;
-        const int kvp = kv0 + kt * 16 + lo;
-        float sv = sfrag[kt][r] * (DB ? qsc[r] : scale);
-        if (softcap > 0.f)          // cap * tanh(s / cap), via exp
-          sv = softcap * (1.0f - 2.0f / (__expf(2.0f * sv * inv_cap) + 1.0f));
-        const int dist = q_abs - kvp;
-        if (r1) sv -= hr1 * __logf(1.0f + hr2 * (float)max(dist, 0));
-        if (DB) sv += lds_db[wave * 16 + hi * 4 + r - kt * 16 - lo +
-                             WKV_TILE - 1];
-        if (dist < 0 || kvp >= kv_len || qr >= q_len ||
-            (window > 0 && dist >= window && kvp >= keep_first) ||
-            (chunk > 0 && kvp < (q_abs / chunk) * chunk)) sv = -1e30f;
-        // exp of a masked score's 1e30 is infinite: weight zero
-        p[kt][r] = SIG ? 1.0f / (1.0f + __expf(-(sv + hpb))) : sv;
-      }
-#pragma unroll
-    for (int r = 0; r < (SIG ? 0 : 4); r++) {
-      float mx = fmaxf(p[0][r], p[1][r]);
-#pragma unroll
-      for (int off = 1; off < 16; off <<= 1)
-        mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-      const float mnew = fmaxf(mrow[r], mx);
-      const float corr = __expf(mrow[r] - mnew);
-      lrow[r] *= corr;
-#pragma unroll
-      for (int dt = 0; dt < DT; dt++) ofrag[dt][r] *= corr;
-      mrow[r] = mnew;
-      float ps = 0.f;
-#pragma unroll
-      for (int kt = 0; kt < 2; kt++) {
-        p[kt][r] = __expf(p[kt][r] - mnew);
-        ps += p[kt][r];
-      }
-#pragma unroll
-      for (int off = 1; off < 16; off <<= 1) ps += __shfl_xor(ps, off, 64);
-      lrow[r] += ps;
-    }
-    {
-      short* ph = lds_p[wave];
-      short* pl = lds_pl[wave];
-#pragma unroll
-      for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const short hi16 = f32_to_bf16(p[kt][r]);
-          const int at = (hi * 4 + r) * WPAD + kt * 16 + lo;
-          ph[at] = hi16;
-          pl[at] = f32_to_bf16(p[kt][r] - bf16_to_f32(hi16));
-        }
-    }
-    __builtin_amdgcn_s_waitcnt(0);
-    const bf16x8 pfrag = *reinterpret_cast<const bf16x8*>(
-        &lds_p[wave][lo * WPAD + hi * 8]);
-    const bf16x8 pfrag_lo = *reinterpret_cast<const bf16x8*>(
-        &lds_pl[wave][lo * WPAD + hi * 8]);
-#pragma unroll
-    for (int dt = 0; dt < DT; dt++) {
-      const bf16x8 vf = *reinterpret_cast<const bf16x8*>(
-          &lds_vt[(dt * 16 + lo) * WPAD + hi * 8]);
-      ofrag[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pfrag, vf,
-                                                          ofrag[dt], 0, 0, 0);
-      ofrag[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pfrag_lo, vf,
-                                                          ofrag[dt], 0, 0, 0);
-    }
-    __syncthreads();
-  }
-
-#pragma unroll
-  for (int r = 0; r < 4; r++) {
-    const int qr = q0 + wave * 16 + hi * 4 + r;
-    if (qr >= q_len) continue;
-    float inv = 1.f / fmaxf(lrow[r], 1e-30f);
-    if (gate)
-      inv *= sigmoid_f(bf16_to_f32(gate[(int64_t)(tok0 + qr) * gate_s0 + h]));
-    const int64_t obase = ((int64_t)(tok0 + qr) * H + h) * DV;
-#pragma unroll
-    for (int dt = 0; dt < DT; dt++)
-      out[obase + dt * 16 + lo] = f32_to_bf16(ofrag[dt][r] * inv);
   }
 }
 
@@ -1224,20 +996,40 @@ void window_attention_tiles(at::Tensor out, at::Tensor q, at::Tensor k_cache,
   const int ntiles = tile_seq.size(0);
   if (ntiles == 0 || T == 0) return;
   auto stream = at::hip::getCurrentHIPStream();
+  flash::Args a{};
+  a.out = (short*)out.data_ptr();
+  a.q = (const short*)q.data_ptr();
+  a.k = k_cache.data_ptr();
+  a.v = v_cache.data_ptr();
+  a.q_ts = (int64_t)H * D; a.q_hs = D;
+  a.tile_seq = tile_seq.data_ptr<int>();
+  a.tile_qbase = tile_qbase.data_ptr<int>();
+  a.cu = cu_seqlens.data_ptr<int>();
+  a.starts = seq_starts.data_ptr<int>();
+  a.block_tables = block_tables.data_ptr<int>();
+  a.max_blocks = (int)block_tables.size(1);
+  a.BS = BS; a.KH = G; a.QH = H;
+  // a distance-bias table belongs to one head: no flattening
+  a.gs = db ? 0 : flash::group_shift(H, G);
+  a.scale = (float)scale;
+  a.window = (int)window;
+  a.sinks = has_sinks ? sinks.data_ptr<float>() : nullptr;
+  a.keep_first = kf;
+  a.chunk = (int)chunk;
+  a.softcap = (float)softcap;
+  a.r1 = bias ? r1.data_ptr<float>() : nullptr;
+  a.r2 = bias ? r2.data_ptr<float>() : nullptr;
+  a.pb = pb;
+  a.gate = gated ? (const short*)gate.data_ptr() : nullptr;
+  a.gate_s0 = gated ? gate.stride(0) : 0;
+  a.db = db; a.db_n = db_n;
+  a.temp_coef = (float)temp_coef;
+  a.temp_every = (int)temp_every;
+  const dim3 grid(flash::grid_size(a, ntiles));
 #define KAITO_WIN_LAUNCH(D_, DV_, SIG_, DB_)                                 \
-    hipLaunchKernelGGL((window_attention_mfma_kernel<D_, DV_, SIG_, DB_>),   \
-        dim3(ntiles, H), dim3(256), 0, stream, (short*)out.data_ptr(),       \
-        (const short*)q.data_ptr(), (const short*)k_cache.data_ptr(),        \
-        (const short*)v_cache.data_ptr(), tile_seq.data_ptr<int>(),          \
-        tile_qbase.data_ptr<int>(), cu_seqlens.data_ptr<int>(),              \
-        seq_starts.data_ptr<int>(), block_tables.data_ptr<int>(),            \
-        (int)block_tables.size(1), (float)scale, (float)softcap,             \
-        bias ? r1.data_ptr<float>() : nullptr,                               \
-        bias ? r2.data_ptr<float>() : nullptr, (int)window, H, G, BS, kf,    \
-        has_sinks ? sinks.data_ptr<float>() : nullptr, (int)chunk, pb,       \
-        gated ? (const short*)gate.data_ptr() : nullptr,                     \
-        gated ? gate.stride(0) : 0, db, db_n, (float)temp_coef,              \
-        (int)temp_every)
+    hipLaunchKernelGGL((flash::flash_prefill_kernel<D_, DV_,                 \
+                            flash::PAGED_BF16, true, SIG_, DB_>),            \
+        grid, dim3(256), 0, stream, a)
 #define KAITO_WIN_CASE(D_, DV_)                                              \
   if (D == D_ && V == DV_) {                                                 \
     if (pb) KAITO_WIN_LAUNCH(D_, DV_, true, false);                          \

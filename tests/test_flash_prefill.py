@@ -1,0 +1,157 @@
+"""The MFMA prompt attention (ops/csrc/flash_prefill.h) at the edges of its
+tiles: 32-row waves, workgroups of 128 flattened rows, 64- (wide heads 32-)
+key tiles, head groups that are flattened and groups that are not. Outputs
+are bf16 of values whose weights entered the second product as bf16: two
+roundings of 2^-9 each relative to the largest terms."""
+import math
+
+import pytest
+import torch
+
+from kaito_amd import ops
+from kaito_amd.ops import torch_ref as R
+
+DEV = "cuda"
+TOL = 2 * 2.0 ** -8          # of the values' magnitude (up to about 3)
+
+
+def _bf16(*shape):
+    return torch.randn(*shape, device=DEV).to(torch.bfloat16)
+
+
+def _cu(lens):
+    return torch.tensor([0] + list(torch.tensor(lens).cumsum(0)),
+                        dtype=torch.int32, device=DEV)
+
+
+def _check(out, ref):
+    assert torch.isfinite(out).all()
+    assert (out.cpu().float() - ref).abs().max().item() < 3 * TOL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("QH,KH,D,lens,window,sink", [
+    (4, 1, 128, [1, 31, 32, 33], 0, False),
+    (8, 2, 128, [63, 64, 65, 129], 0, True),
+    (3, 3, 128, [127, 128, 129, 193], 0, False),     # one head per group
+    (6, 2, 64, [1, 200, 70], 0, False),              # group of 3
+    (16, 1, 64, [9, 40, 100], 33, False),
+    (8, 1, 96, [64, 65, 130], 0, False),
+    (2, 1, 256, [31, 33, 150], 64, True),
+    (4, 4, 256, [64, 96, 129], 0, False),
+    (8, 2, 128, [300], 1, False),
+    (5, 1, 128, [260, 3], 100, True),
+])
+@pytest.mark.parametrize("scale_sign", [1.0, -1.0])
+def test_whole_prompts(QH, KH, D, lens, window, sink, scale_sign):
+    torch.manual_seed(len(lens) + D)
+    T = sum(lens)
+    qkv = _bf16(T, (QH + 2 * KH) * D)        # rows of a fused projection
+    q, k, v = qkv.split([QH * D, KH * D, KH * D], -1)
+    q, k, v = (t.unflatten(-1, (-1, D)) for t in (q, k, v))
+    sinks = torch.randn(QH, device=DEV) if sink else None
+    scale = scale_sign / math.sqrt(D)
+    out = ops.prefill_attention(q, k, v, _cu(lens), scale, window=window,
+                                sinks=sinks)
+    ref = R.prefill_attention(
+        q.cpu().float(), k.cpu().float(), v.cpu().float(), _cu(lens).cpu(),
+        scale, window, sinks.cpu() if sink else None)
+    _check(out, ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("QH,KH,D,pairs,window", [
+    (4, 1, 128, [(64, 64), (65, 1), (191, 33)], 0),
+    (8, 8, 128, [(300, 129), (128, 128)], 0),
+    (8, 1, 64, [(90, 17), (257, 64)], 50),
+    (2, 2, 256, [(97, 33), (32, 32)], 0),
+])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_suffixes_over_pages(QH, KH, D, pairs, window, fp8):
+    torch.manual_seed(D + QH)
+    kv, ql = [p[0] for p in pairs], [p[1] for p in pairs]
+    mb = -(-max(kv) // 16)
+    bt = torch.randperm(len(kv) * mb, device=DEV).int().view(len(kv), mb)
+    kc, vc = (_bf16(len(kv) * mb, KH, 16, D) for _ in range(2))
+    if fp8:
+        k8, v8 = (t.to(torch.float8_e4m3fn) for t in (kc, vc))
+        kc, vc = k8.to(torch.bfloat16), v8.to(torch.bfloat16)
+        args = (k8.view(torch.uint8), v8.view(torch.uint8))
+    else:
+        args = (kc, vc)
+    q = _bf16(sum(ql), QH, D)
+    kl = torch.tensor(kv, dtype=torch.int32, device=DEV)
+    scale = D ** -0.5
+    out = ops.context_attention(q, *args, _cu(ql), kl, bt, scale, window)
+    ref = R.context_attention(q.cpu().float(), kc.cpu().float(),
+                              vc.cpu().float(), _cu(ql).cpu(), kl.cpu(),
+                              bt.cpu(), scale, window)
+    _check(out, ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,lens", [(1, [1, 64, 65]), (16, [200, 33]),
+                                    (5, [129, 128, 127])])
+def test_latent_prompts(H, lens):
+    """Split heads: 128 + 64 key dims, the 64 shared by the heads."""
+    torch.manual_seed(H)
+    T = sum(lens)
+    q = _bf16(T, H, 192)
+    q_pe, k_pe = _bf16(T, H, 64), _bf16(T, 64)
+    k = _bf16(T, H, 128)
+    v = _bf16(H, T, 128).transpose(0, 1)
+    scale = 192 ** -0.5
+    out = ops.mla_prefill_attention(q[..., :128], q_pe, k, k_pe, v,
+                                    _cu(lens), scale)
+    qf = torch.cat([q[..., :128], q_pe], -1)
+    kf = torch.cat([k, k_pe[:, None].expand(T, H, 64)], -1)
+    vf = torch.cat([v, torch.zeros_like(q_pe)], -1)
+    ref = R.prefill_attention(qf.cpu().float(), kf.cpu().float(),
+                              vf.cpu().float(), _cu(lens).cpu(), scale)
+    _check(out, ref[..., :128])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,G,D,V,mode", [
+    (4, 1, 128, 128, "cap"), (6, 2, 64, 32, "keep"), (4, 4, 256, 128, "sig"),
+    (4, 2, 128, 64, "bias"), (2, 1, 256, 256, "chunk"),
+    (8, 1, 64, 256, "gate"), (16, 1, 128, 256, "cap"),
+])
+def test_window_options(H, G, D, V, mode):
+    """Portions behind earlier tokens, every option of the paged window
+    attention, against its plain reference."""
+    torch.manual_seed(H + V)
+    kv, ql = [200, 64, 131], [130, 64, 33]
+    mb = -(-max(kv) // 16)
+    bt = torch.randperm(len(kv) * mb, device=DEV).int().view(len(kv), mb)
+    kc, vc = _bf16(len(kv) * mb, G, 16, D), _bf16(len(kv) * mb, G, 16, V)
+    T = sum(ql)
+    q = _bf16(T, H, D)
+    starts = [a - b for a, b in zip(kv, ql)]
+    seq = torch.repeat_interleave(torch.arange(3), torch.tensor(ql)).int()
+    pos = torch.cat([torch.arange(s, s + n) for s, n in zip(starts, ql)])
+    opt = dict(window=50)
+    vec = torch.rand(H, device=DEV)
+    if mode == "cap":
+        opt.update(softcap=4.0, r1=vec, r2=vec * 2)
+    elif mode == "keep":
+        opt.update(keep_first=35, sinks=vec)
+    elif mode == "sig":
+        opt.update(sigmoid_bias=vec - 4.0)
+    elif mode == "bias":
+        opt.update(dist_bias=torch.randn(H, 40, device=DEV), temp_coef=0.1,
+                   temp_every=16, window=0)
+    elif mode == "chunk":
+        opt.update(chunk=48)
+    else:
+        opt.update(gate=_bf16(T, H))
+    tiles = ops.build_query_tiles(ql, DEV, starts) + (
+        _cu(ql), torch.tensor(starts, dtype=torch.int32, device=DEV))
+    out = ops.window_attention(q, kc, vc, bt, seq.to(DEV), pos.to(DEV),
+                               D ** -0.5, tiles=tiles, **opt)
+    opt = {k: t.cpu().float() if torch.is_tensor(t) else t
+           for k, t in opt.items()}
+    ref = ops.window_attention(q.cpu().float(), kc.cpu().float(),
+                               vc.cpu().float(), bt.cpu(), seq, pos,
+                               D ** -0.5, **opt)
+    _check(out, ref)
