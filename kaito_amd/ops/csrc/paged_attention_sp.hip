@@ -1,392 +1,363 @@
-// Split-phase paged-attention DECODE kernel for gfx950 (MI355X).
+// Paged-attention DECODE kernel for gfx950: one query row per sequence, the
+// heads of a kv group in one pass over its K and V pages.
 //
-// Round-2 restructure of paged_attention.hip. The r01 kernel reached
-// 4.33 TB/s against a 6.0 TB/s read+dot diagnostic ceiling; the measured
-// gap was the per-chunk online-softmax serial chain (compare → exp →
-// rescale of the accumulator) riding INSIDE the K/V streaming loop at
-// 3 waves/SIMD (profiles/r01_decode_profile.md). This kernel removes
-// that chain from the memory loops entirely:
+// A wave walks a contiguous span of keys, 32 at a time, with the products on
+// v_mfma_f32_16x16x32_bf16, transposed as in flash_prefill.h (the group's
+// heads are the 16 columns, unused ones ride along):
+//   - S^T = K Q^T reads K straight from the pages into operand registers (a
+//     16-byte load per lane is 8 dims of one key);
+//   - the scores of one head sit in one column: maximum and rescale factor
+//     are per-lane scalars after two exchanges;
+//   - O^T += V^T P^T takes P from the score registers; V goes to wave-private
+//     LDS by 16-byte direct loads and comes back by transposing reads.
+// P enters as a bf16 value + remainder pair, which keeps 16 mantissa bits of
+// the f32 weight (the result is rounded to 8). fp8 (e4m3) pages are widened
+// to bf16, exactly, on the way. The waves of a workgroup, and with SPLIT the
+// workgroups of a (sequence, kv head), hold partial (max, sum, O) that are
+// folded at the end.
 //
-//   phase A  stream K only: dot + DC-lane DPP reduce + running MAX (one
-//            fmaxf — no exp, no rescale), raw scores parked in LDS.
-//   phase B  tiny throughput pass: one exp per (token, head) over the
-//            LDS scores with a wave-uniform max, probabilities written
-//            back in place.
-//   phase C  stream V only: vector LDS broadcast of the G
-//            probabilities + pure packed v_pk_fma_f32 accumulate.
+// What bounds it: bytes in flight. K and V of a tile (16 KB per wave at
+// D = 128) are all under way at once, while the arithmetic of a tile is
+// about 500 cycles (2 x 16 scores and weights on the vector unit took
+// 3000). Small steps are bound by the chain lengths -> table -> K -> V -> fold:
+// hence up to 16 waves per workgroup, so that each walks few tiles, and
+// workgroups per pair once those no longer fill the chip. Measured on one
+// MI355X against a kernel with 4 waves per pair, 16-byte K and V streams in
+// two phases and dot products by dot2 + DPP sums (before -> now; 8 kv heads
+// of 128, groups of 4):
+//   1 row, 217 keys: 11.3 -> 6.3 us;  16 rows, 2050-4100 fp8 keys: 225 -> 42;
+//   64 rows, 500-1000 keys: 77 -> 44;  250 rows, 200-400: 84 -> 65;
+//   2048 rows, 150-300: 453 -> 347 us (5.5 TB/s).
 //
-// Lane layout: DC = D/8 dim-lanes × TPC = 64/DC tokens per wave-step,
-// 8 dims (one short8, 16 B) per lane. For D=128 that is 16 dim-lanes ×
-// 4 tokens — each token's 16 lanes read 256 B CONTIGUOUS, and the
-// per-lane accumulator is acc[G][8] (32 VGPR at G=4), small enough that
-// the whole kernel fits the 128-VGPR 4-waves/SIMD occupancy bound with
-// no spill (the r01 kernel ran at 3 waves with acc[G][16]).
-//
-// Memory-level parallelism: each wave owns a CONTIGUOUS chunk span and
-// the streaming loops process one KV BLOCK (4 chunks = 16 tokens =
-// 4 KiB) per iteration — ONE block-table read per block (vs per-token),
-// no per-lane address clamp (a clamped block index keeps every
-// intra-block offset valid), and 4 independent 16 B loads in flight per
-// lane per iteration.
-//
-// Long histories are processed in SUPER-CHUNKS of SC chunks per wave;
-// carried (M, l, acc) state is rescaled once per super-chunk. All LDS
-// score regions are wave-private, so phases need no __syncthreads
-// (same-wave LDS RAW is ordered by the compiler's lgkmcnt).
-//
-// Cache layout: [num_blocks, KV_HEADS, BLOCK_SIZE, HEAD_DIM] bf16
-// (same as paged_attention.hip; replaces the vLLM decode attention the
-// reference delegates to — SURVEY.md §2.3).
-#include "common.h"
-#include <cstdlib>
+// Cache layout: [num_blocks, KV_HEADS, BLOCK_SIZE, HEAD_DIM] bf16 | e4m3.
+#include "flash_prefill.h"
 #include <torch/library.h>
 #include <ATen/ATen.h>
 #include <ATen/hip/HIPContext.h>
 
 namespace kaito {
 
-// OCC = target workgroups/CU (4 ⇒ 4 waves/SIMD at ≤128 VGPRs).
-// Measured (tools/bench_decode_attn.py --sweep-occ): OCC=3 == OCC=4
-// exactly and OCC=5 spills — the kernel is NOT wave-count-limited, so
-// at OCC=3 there are ~170 VGPRs of free headroom. UB (blocks per
-// streaming iteration) spends that headroom on memory-level
-// parallelism: UB=2 keeps 8 independent 16 B loads in flight per lane
-// (two KV blocks) instead of 4. Variants selectable at runtime via
-// KAITO_PA_SP_OCC / KAITO_PA_SP_UB for A/B on real hardware.
-template <int D, int G, int BS, bool FP8 = false, int OCC = (G <= 4 ? 4 : 3),
-          int UB = 1>
-__global__ __launch_bounds__(256, OCC)
-void paged_attention_sp_kernel(
-    short* __restrict__ out,             // [T, QH, D] bf16
-    const short* __restrict__ q,         // [T, QH, D] bf16
-    const void* __restrict__ k_cache,    // [B, KH, BS, D] bf16 | e4m3
-    const void* __restrict__ v_cache,
-    const int* __restrict__ block_tables,// [T, max_blocks]
-    const int* __restrict__ seq_lens,    // [T]
-    const float scale, const int KH, const int max_blocks,
-    const int64_t q_stride,
-    const int window,                    // 0 = full attention
-    const float* __restrict__ sinks) {   // [QH] or nullptr (gpt-oss)
-  constexpr int DC = D / 8;       // dim-chunk lanes (16 for D=128)
-  constexpr int TPC = 64 / DC;    // tokens per wave-step (4 for D=128)
-  constexpr int CPB = BS / TPC;   // chunks per KV block (4 for D=128)
-  constexpr int NW = 4;           // waves per workgroup
-  constexpr int G4 = G <= 2 ? 2 : (G <= 4 ? 4 : 8);  // padded score row
-  constexpr int SC = (G <= 4 ? 256 : 128) / TPC;  // chunks per super-chunk
-  static_assert(SC % CPB == 0, "super-chunk must align to KV blocks");
-  const int seq = blockIdx.x;
-  const int kvh = blockIdx.y;
-  const int wave = threadIdx.x >> 6;
+namespace {
+
+using flash::hbf16x8;
+using flash::LOG2E;
+
+constexpr int BS = 16;              // tokens per page
+constexpr int KT = 32;              // keys per wave step: two pages
+constexpr int64_t SPLIT_FILL = 256;  // workgroups that splits aim at
+constexpr int SPLIT_MIN = 2;        // tiles per wave that a split keeps
+
+struct DecodeArgs {
+  short* out;                       // [T, QH, D]
+  const short* q;
+  const void *k, *v;                // [NB, KH, BS, D] bf16 | e4m3
+  const int* block_tables;          // [T, max_blocks]
+  const int* seq_lens;              // [T]
+  float scale;
+  int KH, G, max_blocks;
+  int64_t q_stride;
+  int window;                       // 0 = all keys
+  const float* sinks;               // [QH] or nullptr
+  float* part;                      // SPLIT: [splits, T, QH, D + 2]
+};
+
+KAITO_DEV hbf16x8 widen8(const u8x8_t raw) {
+  float f[8];
+  fp8x8_to_f32(raw, f);
+  hbf16x8 w;
+#pragma unroll
+  for (int e = 0; e < 8; e++) w[e] = (__bf16)f[e];
+  return w;
+}
+
+// weights of the partial results of one head: exponent of each maximum
+// against the largest, summed with the sink's into the denominator
+KAITO_DEV float fold_weight(float m, float gm) {
+  return __builtin_amdgcn_exp2f(m - gm);
+}
+
+template <int D, bool FP8, int NW, bool SPLIT>
+__global__ __launch_bounds__(NW * 64, NW <= 4 ? 3 : (NW <= 8 ? 2 : 4))
+void paged_decode_kernel(const DecodeArgs a) {
+  constexpr int KK = D / 32;        // 16x16x32 steps over the dims
+  constexpr int DT = D / 16;        // 16-row tiles of O^T
+  constexpr int CV = D / 8;         // 16-byte chunks of a V row
+  constexpr int LV = KT * CV / 64;  // V chunks per lane and tile
+  __shared__ __attribute__((aligned(128))) short lds_v[NW][KT * D];
+  __shared__ float s_m[NW][16], s_l[NW][16];
+
+  const int seq = blockIdx.x / a.KH, kvh = blockIdx.x % a.KH;
   const int lane = threadIdx.x & 63;
-  const int tg = lane / DC;       // token slot in chunk (0..TPC-1)
-  const int dc = lane % DC;       // dim chunk (8 dims each)
-  const int seq_len = seq_lens[seq];
-  const int QH = KH * G;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lo = lane & 15, hi = lane >> 4;
+  const int seq_len = a.seq_lens[seq];
+  const int QH = a.KH * a.G;
+  const int* bt = a.block_tables + (int64_t)seq * a.max_blocks;
 
-  const int* bt = block_tables + (int64_t)seq * max_blocks;
+  // keys from the page that holds the window's first; a contiguous run of
+  // tiles per wave
+  const int start = a.window > 0 && seq_len > a.window ? seq_len - a.window : 0;
+  const int base = start / BS * BS;
+  const int tiles = (seq_len - base + KT - 1) / KT;
+  const int nsplit = SPLIT ? gridDim.y : 1, split = SPLIT ? blockIdx.y : 0;
+  // a split covers whole rounds of its workgroup's waves
+  const int per = (tiles + nsplit * NW - 1) / (nsplit * NW);
+  const int t0 = min(tiles, (split * NW + wave) * per);
+  const int t1 = min(tiles, t0 + per);
+  const int last_page = (seq_len - 1) / BS;
 
-  // scores/probabilities: wave-private [SC][TPC tokens][G4] f32
-  __shared__ float s_p[NW][SC][TPC][G4];
-
-  float M[G], lpart[G], acc[G][8];
+  hbf16x8 qf[KK];
+  {
+    const short* qp = a.q + (int64_t)seq * a.q_stride +
+        (int64_t)(kvh * a.G + min(lo, a.G - 1)) * D + hi * 8;
 #pragma unroll
-  for (int g = 0; g < G; g++) {
-    M[g] = -1e30f; lpart[g] = 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; j++) acc[g][j] = 0.f;
+    for (int kk = 0; kk < KK; kk++)
+      qf[kk] = *reinterpret_cast<const hbf16x8*>(qp + kk * 32);
   }
-
-  // sliding window: only tokens in [start, seq_len) are attended; the
-  // chunk range is aligned DOWN to the containing KV block (tokens
-  // before `start` in that block are masked by `valid`)
-  const int start = (window > 0 && seq_len > window) ? seq_len - window : 0;
-  const int c_lo = (start / BS) * CPB;
-  const int nchunks = (seq_len + TPC - 1) / TPC;
-  const int last_blk = (seq_len - 1) / BS;
-  // contiguous block-aligned chunk span per wave
-  const int total_c = nchunks - c_lo;
-  const int n_per = ((total_c + NW * CPB - 1) / (NW * CPB)) * CPB;
-  const int span0 = c_lo + wave * n_per;
-  const int n_i = max(0, min(nchunks, span0 + n_per) - span0);
-
-  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-
-  for (int s0 = 0; s0 < n_i; s0 += SC) {
-    const int n_ii = min(SC, n_i - s0);
-
-    // ---------------- phase A: stream K, raw scores to LDS -------------
-    // Q is (re)loaded per super-chunk so its registers die before
-    // phase C (Q and the accumulator never coexist). Lane dc holds dims
-    // dc*8..dc*8+8 — one contiguous 16B load per (head, lane). The fp8
-    // cache path pre-converts Q to f32 (the dot runs on fmaf over the
-    // hardware fp8→f32 pair converts instead of v_dot2 bf16).
-    short8_t qreg[G];
-    float qf[FP8 ? G : 1][FP8 ? 8 : 1];
+  float m = -1e30f, l = 0.f;
+  f32x4 o[DT];
 #pragma unroll
-    for (int g = 0; g < G; g++) {
-      qreg[g] = *reinterpret_cast<const short8_t*>(
-          q + (int64_t)seq * q_stride + (kvh * G + g) * D + dc * 8);
-      if constexpr (FP8) {
-#pragma unroll
-        for (int j = 0; j < 8; j++) qf[g][j] = bf16_to_f32(qreg[g][j]);
-      }
+  for (int dt = 0; dt < DT; dt++) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  short* vl = lds_v[wave];
+  const int vrow = 4 * hi + (lo >> 2), vc = (lo & 3) >> 1, ve = (lo & 1) * 4;
+  const float c = a.scale * LOG2E;
+
+  int pages = 0, pages_at = -64;    // lane i: page pages_at + i of the table
+  auto page_row = [&](const int p) {        // first cache row of page p
+    const int pc = min(p, last_page);
+    if (pc >= pages_at + 64) {              // uniform; spans move forward
+      pages_at = pc;
+      pages = bt[min(pc + lane, last_page)];
     }
-    float mloc[G];
+    const int page = __builtin_amdgcn_readlane(pages, pc - pages_at);
+    return ((int64_t)page * a.KH + kvh) * BS;
+  };
+  hbf16x8 kf[2][KK];
+  u8x8_t k8[FP8 ? 2 : 1][FP8 ? KK : 1];
+  auto load_k = [&](const int64_t r0, const int64_t r1) {
 #pragma unroll
-    for (int g = 0; g < G; g++) mloc[g] = -1e30f;
-    for (int ii0 = 0; ii0 < n_ii; ii0 += UB * CPB) {
-      const int c0 = span0 + s0 + ii0;           // multiple of CPB
-      // UB block bases; clamped indices keep every offset valid
-      int64_t gb[UB];
+    for (int i = 0; i < 2; i++) {
+      // uniform page address, 32-bit lane offset
+      const int64_t at = (i ? r1 : r0) * D;
+      const uint32_t off = lo * D + hi * 8;
 #pragma unroll
-      for (int b = 0; b < UB; b++) {
-        const int blk = bt[min(c0 / CPB + b, last_blk)];
-        gb[b] = (((int64_t)blk * KH + kvh) * BS + tg) * D + dc * 8;
-      }
-      short8_t kd[FP8 ? 1 : UB * CPB];
-      u8x8_t kd8[FP8 ? UB * CPB : 1];
-#pragma unroll
-      for (int u = 0; u < UB * CPB; u++) {
+      for (int kk = 0; kk < KK; kk++) {
         if constexpr (FP8)
-          kd8[u] = reinterpret_cast<const u8x8_t*>(k_cache)[
-              (gb[u / CPB] + (u % CPB) * (TPC * D)) / 8];
+          k8[i][kk] = *reinterpret_cast<const u8x8_t*>(
+              (const uint8_t*)a.k + at + (off + kk * 32));
         else
-          kd[u] = *reinterpret_cast<const short8_t*>(
-              (const short*)k_cache + gb[u / CPB] + (u % CPB) * (TPC * D));
-      }
-      const int nu = min(UB * CPB, n_ii - ii0);
-      // compile-time trip count: a runtime-bounded loop would make
-      // kd[u] a runtime-indexed register array → scratch (rule #20)
-#pragma unroll
-      for (int u = 0; u < UB * CPB; u++) {
-        if (u >= nu) break;
-        const int tok = (c0 + u) * TPC + tg;
-        const bool valid = tok >= start && tok < seq_len;
-        float s[G];
-        float kf[FP8 ? 8 : 1];
-        if constexpr (FP8) fp8x8_to_f32(kd8[u], kf);
-#pragma unroll
-        for (int g = 0; g < G; g++) {
-          float p = 0.f;
-          if constexpr (FP8) {
-#pragma unroll
-            for (int j = 0; j < 8; j++) p = fmaf(qf[g][j], kf[j], p);
-          } else {
-            const bf16x2_t* kp = reinterpret_cast<const bf16x2_t*>(&kd[u]);
-            const bf16x2_t* qp = reinterpret_cast<const bf16x2_t*>(&qreg[g]);
-#pragma unroll
-            for (int jj = 0; jj < 4; jj++)
-              p = __builtin_amdgcn_fdot2_f32_bf16(qp[jj], kp[jj], p, false);
-          }
-          p = group_reduce_sum<DC>(p) * scale;   // dot over DC dim-lanes
-          s[g] = valid ? p : -1e30f;
-          mloc[g] = fmaxf(mloc[g], s[g]);
-        }
-        // park raw scores: lane with dc<G writes s[dc] (static unroll —
-        // a runtime-indexed register array would spill to scratch)
-        if (dc < G) {
-          float sval = s[0];
-#pragma unroll
-          for (int g = 1; g < G; g++) if (dc == g) sval = s[g];
-          s_p[wave][ii0 + u][tg][dc] = sval;
-        }
+          kf[i][kk] = *reinterpret_cast<const hbf16x8*>(
+              (const short*)a.k + at + (off + kk * 32));
       }
     }
+  };
 
-    // ---- wave-uniform max; rescale carried state once per super ----
+  int64_t row0 = 0, row1 = 0;
+  if (t0 < t1) {
+    row0 = page_row(base / BS + t0 * 2);
+    row1 = page_row(base / BS + t0 * 2 + 1);
+    load_k(row0, row1);
+  }
+  for (int t = t0; t < t1; t++) {
+    // ---- V of this tile: slot j * 64 + lane is row s / CV, place s % CV
+    u8x8_t v8[FP8 ? LV : 1];
 #pragma unroll
-    for (int g = 0; g < G; g++) {
-      float gm = mloc[g];               // uniform over dc; varies over tg
+    for (int j = 0; j < LV; j++) {
+      const int row = j * (64 / CV) + lane / CV;
+      const int64_t at = (j * (64 / CV) < BS ? row0 : row1) * D;
+      const uint32_t off =
+          row % BS * D + flash::swz_v<D>(row, lane % CV) * 8;
+      if constexpr (FP8)
+        v8[j] = *reinterpret_cast<const u8x8_t*>(
+            (const uint8_t*)a.v + at + off);
+      else
+        flash::lds_copy16((const short*)a.v + at + off, vl + j * 512);
+    }
+    // ---- S^T: keys 16 i + 4 hi + r of head lo
+    f32x4 s[2];
 #pragma unroll
-      for (int off = DC; off < 64; off <<= 1)
-        gm = fmaxf(gm, __shfl_xor(gm, off, 64));
-      const float Mnew = fmaxf(M[g], gm);
-      if (Mnew > M[g]) {
-        const float corr = __expf(M[g] - Mnew);   // 0 on first super
-        lpart[g] *= corr;
-        float2_t* a2 = reinterpret_cast<float2_t*>(acc[g]);
+    for (int i = 0; i < 2; i++) {
+      s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < 4; j++) a2[j] *= corr;
-        M[g] = Mnew;
+      for (int kk = 0; kk < KK; kk++) {
+        if constexpr (FP8) kf[i][kk] = widen8(k8[i][kk]);
+        s[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[i][kk], qf[kk],
+                                                       s[i], 0, 0, 0);
       }
     }
-
-    // ---------------- phase B: exp over LDS scores (throughput) --------
-    const int entries = n_ii * TPC;     // (ii, tg) pairs
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-      for (int idx = lane; idx < entries; idx += 64) {
-        float* slot = &s_p[wave][0][0][0] + idx * G4 + g;
-        const float sv = *slot;
-        const float p = sv > -1e29f ? __expf(sv - M[g]) : 0.f;
-        lpart[g] += p;
-        *slot = p;
-      }
+    if (t + 1 < t1) {               // K of the next tile, under way with V
+      row0 = page_row(base / BS + t * 2 + 2);
+      row1 = page_row(base / BS + t * 2 + 3);
+      load_k(row0, row1);
     }
-
-    // ---------------- phase C: stream V, pure FMA accumulate -----------
-    for (int ii0 = 0; ii0 < n_ii; ii0 += UB * CPB) {
-      const int c0 = span0 + s0 + ii0;
-      int64_t gb[UB];
+    // ---- softmax
+    const int key0 = base + t * KT;
+    const bool whole = key0 >= start && key0 + KT <= seq_len;
+    float mx = -1e30f;
 #pragma unroll
-      for (int b = 0; b < UB; b++) {
-        const int blk = bt[min(c0 / CPB + b, last_blk)];
-        gb[b] = (((int64_t)blk * KH + kvh) * BS + tg) * D + dc * 8;
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int key = key0 + 16 * i + 4 * hi + r;
+        s[i][r] *= c;
+        if (!whole && (key < start || key >= seq_len)) s[i][r] = -1e30f;
+        mx = fmaxf(mx, s[i][r]);
       }
-      short8_t vd[FP8 ? 1 : UB * CPB];
-      u8x8_t vd8[FP8 ? UB * CPB : 1];
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if (__any(mx > m)) {
+      const float mn = fmaxf(m, mx);
+      const float corr = __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      l *= corr;
 #pragma unroll
-      for (int u = 0; u < UB * CPB; u++) {
-        if constexpr (FP8)
-          vd8[u] = reinterpret_cast<const u8x8_t*>(v_cache)[
-              (gb[u / CPB] + (u % CPB) * (TPC * D)) / 8];
-        else
-          vd[u] = *reinterpret_cast<const short8_t*>(
-              (const short*)v_cache + gb[u / CPB] + (u % CPB) * (TPC * D));
-      }
-      const int nu = min(UB * CPB, n_ii - ii0);
-#pragma unroll
-      for (int u = 0; u < UB * CPB; u++) {
-        if (u >= nu) break;
-        // G probabilities for this token: one vector LDS broadcast
-        float pg[G];
-        if constexpr (G4 == 2) {
-          float2_t pv = *reinterpret_cast<float2_t*>(
-              &s_p[wave][ii0 + u][tg][0]);
-#pragma unroll
-          for (int g = 0; g < G; g++) pg[g] = pv[g];
-        } else if constexpr (G4 == 4) {
-          float4_t pv = *reinterpret_cast<float4_t*>(
-              &s_p[wave][ii0 + u][tg][0]);
-#pragma unroll
-          for (int g = 0; g < G; g++) pg[g] = pv[g];
-        } else {
-          float4_t pv0 = *reinterpret_cast<float4_t*>(
-              &s_p[wave][ii0 + u][tg][0]);
-          float4_t pv1 = *reinterpret_cast<float4_t*>(
-              &s_p[wave][ii0 + u][tg][4]);
-#pragma unroll
-          for (int g = 0; g < G; g++) pg[g] = g < 4 ? pv0[g] : pv1[g - 4];
-        }
-        float vreg[8];
-        if constexpr (FP8) {
-          fp8x8_to_f32(vd8[u], vreg);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; j++) vreg[j] = bf16_to_f32(vd[u][j]);
-        }
-        const float2_t* v2 = reinterpret_cast<const float2_t*>(vreg);
-#pragma unroll
-        for (int g = 0; g < G; g++) {
-          float2_t* a2 = reinterpret_cast<float2_t*>(acc[g]);
-#pragma unroll
-          for (int j = 0; j < 4; j++) a2[j] += pg[g] * v2[j];
-        }
-      }
+      for (int dt = 0; dt < DT; dt++) o[dt] *= corr;
     }
+    hbf16x8 p, pl;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        // a masked key weighs nothing even where a lane saw no other yet
+        const float w = s[i][r] > -1e29f
+            ? __builtin_amdgcn_exp2f(s[i][r] - m) : 0.f;
+        l += w;
+        p[i * 4 + r] = (__bf16)w;
+        pl[i * 4 + r] = (__bf16)(w - (float)p[i * 4 + r]);
+      }
+    if constexpr (FP8) {
+#pragma unroll
+      for (int j = 0; j < LV; j++)
+        *reinterpret_cast<hbf16x8*>(vl + (j * 64 + lane) * 8) = widen8(v8[j]);
+    } else {
+      // the direct loads' data: this wave's own, so no barrier
+      __builtin_amdgcn_s_waitcnt(0x0f70);     // vmcnt(0)
+    }
+    __builtin_amdgcn_wave_barrier();
+    // ---- O^T: dims 16 dt + 4 hi + r of head lo
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++) {
+      const short* at = vl + vrow * D +
+          flash::swz_v<D>(vrow, dt * 2 + vc) * 8 + ve;
+      const short4_t a4 = flash::read_tr(at), b4 = flash::read_tr(at + 16 * D);
+      const hbf16x8 vf = __builtin_bit_cast(
+          hbf16x8, __builtin_shufflevector(a4, b4, 0, 1, 2, 3, 4, 5, 6, 7));
+      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p, o[dt], 0, 0, 0);
+      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl, o[dt], 0, 0, 0);
+    }
+    __builtin_amdgcn_wave_barrier();
   }
 
-  // ---- merge over the TPC token-group lanes (M already wave-uniform) --
+  // ---- fold the waves: O of the used heads through LDS (the V stage)
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  float* acc = reinterpret_cast<float*>(&lds_v[0][0]) + wave * a.G * D;
+  __syncthreads();
+  if (lo < a.G) {
 #pragma unroll
-  for (int g = 0; g < G; g++) {
-    lpart[g] = wave_reduce_sum(lpart[g]);
-#pragma unroll
-    for (int j = 0; j < 8; j++)
-#pragma unroll
-      for (int off = DC; off < 64; off <<= 1)
-        acc[g][j] += __shfl_xor(acc[g][j], off, 64);
-  }
-
-  // ---- cross-wave combine via LDS (same structure as the r01 kernel) --
-  __shared__ float s_acc[NW][G][D];
-  __shared__ float s_ml[NW][G][2];
-  if (tg == 0) {
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-#pragma unroll
-      for (int j = 0; j < 8; j++)
-        s_acc[wave][g][dc * 8 + j] = acc[g][j];
-      if (dc == 0) { s_ml[wave][g][0] = M[g]; s_ml[wave][g][1] = lpart[g]; }
-    }
+    for (int dt = 0; dt < DT; dt++)
+      *reinterpret_cast<f32x4*>(acc + lo * D + dt * 16 + hi * 4) = o[dt];
+    if (hi == 0) { s_m[wave][lo] = m; s_l[wave][lo] = l; }
   }
   __syncthreads();
-
-  for (int idx = threadIdx.x; idx < G * D; idx += 256) {
-    const int g = idx / D;
-    const int d = idx % D;
+  acc = reinterpret_cast<float*>(&lds_v[0][0]);
+  for (int idx = threadIdx.x; idx < a.G * D; idx += NW * 64) {
+    const int g = idx / D, d = idx % D, head = kvh * a.G + g;
     float gm = -1e30f;
 #pragma unroll
-    for (int w = 0; w < NW; w++) gm = fmaxf(gm, s_ml[w][g][0]);
+    for (int w = 0; w < NW; w++) gm = fmaxf(gm, s_m[w][g]);
+    const float sink = a.sinks && !SPLIT ? a.sinks[head] * LOG2E : -1e30f;
+    gm = fmaxf(gm, sink);
     float num = 0.f, den = 0.f;
-    float sink = sinks != nullptr ? sinks[kvh * G + g] : -1e30f;
-    gm = fmaxf(gm, sink);       // keep exp() bounded when sink dominates
 #pragma unroll
     for (int w = 0; w < NW; w++) {
-      const float e = __expf(s_ml[w][g][0] - gm);
-      num += e * s_acc[w][g][d];
-      den += e * s_ml[w][g][1];
+      const float e = fold_weight(s_m[w][g], gm);
+      num += e * acc[(w * a.G + g) * D + d];
+      den += e * s_l[w][g];
     }
-    if (sinks != nullptr)       // learned sink absorbs softmax mass
-      den += __expf(sink - gm);
-    out[((int64_t)seq * QH + kvh * G + g) * D + d] =
-        f32_to_bf16(num / fmaxf(den, 1e-20f));
+    if constexpr (SPLIT) {
+      const int64_t T = gridDim.x / a.KH;
+      float* row = a.part + ((split * T + seq) * QH + head) * (D + 2);
+      row[d] = num;
+      if (d == 0) { row[D] = gm; row[D + 1] = den; }
+    } else {
+      if (a.sinks) den += fold_weight(sink, gm);
+      a.out[((int64_t)seq * QH + head) * D + d] =
+          f32_to_bf16(num / fmaxf(den, 1e-20f));
+    }
   }
 }
 
-// KAITO_PA_SP_OCC=3|4|5 selects the occupancy variant (default: the
-// template default, i.e. 4 for G<=4). Only instantiated for bf16
-// caches; the fp8 path always uses the default.
-static int pa_sp_occ_env() {
-  static int occ = []() {
-    const char* e = getenv("KAITO_PA_SP_OCC");
-    return e ? atoi(e) : 0;
-  }();
-  return occ;
+// one workgroup per (sequence, head): folds the splits
+template <int D>
+__global__ void paged_fold_kernel(short* __restrict__ out,
+                                  const float* __restrict__ part,
+                                  const float* __restrict__ sinks,
+                                  const int QH, const int splits) {
+  const int64_t row = blockIdx.x, rows = gridDim.x;
+  const int d = threadIdx.x;
+  const float sink = sinks ? sinks[row % QH] * LOG2E : -1e30f;
+  float gm = sink;
+  for (int s = 0; s < splits; s++)
+    gm = fmaxf(gm, part[(s * rows + row) * (D + 2) + D]);
+  float num = 0.f, den = sinks ? fold_weight(sink, gm) : 0.f;
+  for (int s = 0; s < splits; s++) {
+    const float* p = part + (s * rows + row) * (D + 2);
+    const float e = fold_weight(p[D], gm);
+    num += e * p[d];
+    den += e * p[D + 1];
+  }
+  out[row * D + d] = f32_to_bf16(num / fmaxf(den, 1e-20f));
 }
 
-static int pa_sp_ub_env() {
-  static int ub = []() {
-    const char* e = getenv("KAITO_PA_SP_UB");
-    return e ? atoi(e) : 0;
-  }();
-  return ub;
+template <int D, bool FP8>
+void launch_decode(DecodeArgs a, const at::Tensor& out, int T) {
+  auto stream = at::hip::getCurrentHIPStream();
+  const int64_t pairs = (int64_t)T * a.KH;
+  // longest context that the table can hold: the lengths are on the device.
+  // Few pairs on long tables: splits until 256 workgroups, as long as every
+  // wave keeps two tiles (1 row of 16000 keys: 870 us in one workgroup per
+  // head before, 31 us in 32). Up to 256 pairs a workgroup has a CU to
+  // itself and takes 16 waves; above 512 pairs there are workgroups enough
+  // and 4 waves fold less (2048 rows of 300 keys run at 5.5 TB/s).
+  int64_t longest = (int64_t)a.max_blocks * BS;
+  if (a.window > 0) longest = std::min<int64_t>(longest, a.window + BS);
+  constexpr int WIDE = D <= 128 ? 16 : 8;   // waves whose V stage fits LDS
+#define PA_LAUNCH(NW_, SPLIT_, GRID_)                                         \
+  hipLaunchKernelGGL((paged_decode_kernel<D, FP8, NW_, SPLIT_>), GRID_,       \
+                     dim3(NW_ * 64), 0, stream, a)
+  const int64_t splits = std::min<int64_t>(
+      {(SPLIT_FILL + pairs - 1) / pairs, longest / (WIDE * KT * SPLIT_MIN), 64});
+  if (splits > 1) {
+    at::Tensor part = at::empty({splits, T, a.KH * a.G, D + 2},
+                                out.options().dtype(at::kFloat));
+    a.part = part.data_ptr<float>();
+    PA_LAUNCH(WIDE, true, dim3(pairs, splits));
+    hipLaunchKernelGGL((paged_fold_kernel<D>), dim3(T * a.KH * a.G), dim3(D),
+                       0, stream, a.out, a.part, a.sinks, a.KH * a.G,
+                       (int)splits);
+  } else if (pairs <= 256 && longest > 8 * KT) {
+    PA_LAUNCH(WIDE, false, dim3(pairs));
+  } else if (pairs <= 512 || D > 128) {
+    PA_LAUNCH(8, false, dim3(pairs));
+  } else {
+    PA_LAUNCH(4, false, dim3(pairs));
+  }
+#undef PA_LAUNCH
 }
 
-#define PA_SP_ARGS                                                            \
-  dim3(T, KH), dim3(256), 0, stream, (short*)out.data_ptr(),                  \
-      (const short*)query.data_ptr(), k_cache.data_ptr(),                     \
-      v_cache.data_ptr(), block_tables.data_ptr<int>(),                       \
-      seq_lens.data_ptr<int>(), (float)scale, KH, max_blocks,                 \
-      query.stride(0), (int)window, sink_ptr
-
-#define PA_SP_LAUNCH(D_, G_)                                                   \
-  do {                                                                        \
-    if (fp8)                                                                  \
-      hipLaunchKernelGGL((paged_attention_sp_kernel<D_, G_, 16, true>),        \
-          PA_SP_ARGS);                                                        \
-    else if (G_ <= 4 && pa_sp_ub_env() == 2)                                  \
-      hipLaunchKernelGGL((paged_attention_sp_kernel<D_, G_, 16, false, 3, 2>), \
-          PA_SP_ARGS);                                                        \
-    else if (G_ <= 4 && pa_sp_occ_env() == 5)                                 \
-      hipLaunchKernelGGL((paged_attention_sp_kernel<D_, G_, 16, false, 5>),    \
-          PA_SP_ARGS);                                                        \
-    else if (G_ <= 4 && pa_sp_occ_env() == 3)                                 \
-      hipLaunchKernelGGL((paged_attention_sp_kernel<D_, G_, 16, false, 3>),    \
-          PA_SP_ARGS);                                                        \
-    else                                                                      \
-      hipLaunchKernelGGL((paged_attention_sp_kernel<D_, G_, 16, false>),       \
-          PA_SP_ARGS);                                                        \
-  } while (0)
+}  // namespace
 
 void paged_attention_sp(at::Tensor out, at::Tensor query, at::Tensor k_cache,
                         at::Tensor v_cache, at::Tensor block_tables,
                         at::Tensor seq_lens, double scale, int64_t window,
                         at::Tensor sinks) {
-  const float* sink_ptr = nullptr;
+  DecodeArgs a{};
   if (sinks.numel() > 0) {
     TORCH_CHECK(sinks.dtype() == at::kFloat && sinks.is_cuda() &&
                 sinks.numel() == query.size(1));
-    sink_ptr = sinks.data_ptr<float>();
+    a.sinks = sinks.data_ptr<float>();
   }
   TORCH_CHECK(query.is_cuda() && query.dtype() == at::kBFloat16);
   TORCH_CHECK(out.is_contiguous());
@@ -395,46 +366,35 @@ void paged_attention_sp(at::Tensor out, at::Tensor query, at::Tensor k_cache,
   TORCH_CHECK(block_tables.dtype() == at::kInt && seq_lens.dtype() == at::kInt);
   const bool fp8 = k_cache.dtype() == at::kByte;   // OCP e4m3 KV cache
   const int T = query.size(0);
-  const int QH = query.size(1);
   const int D = query.size(2);
-  const int KH = k_cache.size(1);
-  const int BS = k_cache.size(2);
-  TORCH_CHECK(BS == 16, "block_size must be 16");
-  TORCH_CHECK(QH % KH == 0);
-  const int G = QH / KH;
-  const int max_blocks = block_tables.size(1);
-  auto stream = at::hip::getCurrentHIPStream();
+  a.KH = k_cache.size(1);
+  TORCH_CHECK(k_cache.size(2) == BS, "block_size must be 16");
+  TORCH_CHECK(query.size(1) % a.KH == 0);
+  a.G = query.size(1) / a.KH;
+  a.max_blocks = block_tables.size(1);
   if (T == 0) return;
-  if (D == 128) {
-    switch (G) {
-      case 1: PA_SP_LAUNCH(128, 1); break;
-      case 2: PA_SP_LAUNCH(128, 2); break;
-      case 3: PA_SP_LAUNCH(128, 3); break;
-      case 4: PA_SP_LAUNCH(128, 4); break;
-      case 5: PA_SP_LAUNCH(128, 5); break;
-      case 6: PA_SP_LAUNCH(128, 6); break;
-      case 7: PA_SP_LAUNCH(128, 7); break;
-      case 8: PA_SP_LAUNCH(128, 8); break;
-      default: TORCH_CHECK(false, "unsupported GQA group ", G);
-    }
-  } else if (D == 64) {
-    switch (G) {
-      case 1: PA_SP_LAUNCH(64, 1); break;
-      case 2: PA_SP_LAUNCH(64, 2); break;
-      case 4: PA_SP_LAUNCH(64, 4); break;
-      case 8: PA_SP_LAUNCH(64, 8); break;
-      default: TORCH_CHECK(false, "unsupported GQA group ", G);
-    }
-  } else if (D == 256) {   // gemma-3-4b class
-    switch (G) {
-      case 1: PA_SP_LAUNCH(256, 1); break;
-      case 2: PA_SP_LAUNCH(256, 2); break;
-      case 4: PA_SP_LAUNCH(256, 4); break;
-      default: TORCH_CHECK(false, "unsupported GQA group ", G);
-    }
-  } else {
-    TORCH_CHECK(false, "unsupported head_dim ", D);
+  const bool group_ok = D == 128 ? a.G >= 1 && a.G <= 8
+      : D == 64 ? a.G == 1 || a.G == 2 || a.G == 4 || a.G == 8
+                : a.G == 1 || a.G == 2 || a.G == 4;
+  TORCH_CHECK(D == 64 || D == 128 || D == 256, "unsupported head_dim ", D);
+  TORCH_CHECK(group_ok, "unsupported GQA group ", a.G);
+  a.out = (short*)out.data_ptr();
+  a.q = (const short*)query.data_ptr();
+  a.k = k_cache.data_ptr();
+  a.v = v_cache.data_ptr();
+  a.block_tables = block_tables.data_ptr<int>();
+  a.seq_lens = seq_lens.data_ptr<int>();
+  a.scale = (float)scale;
+  a.q_stride = query.stride(0);
+  a.window = (int)window;
+#define PA_DIM(D_)                                                            \
+  if (D == D_) {                                                              \
+    if (fp8) launch_decode<D_, true>(a, out, T);                              \
+    else launch_decode<D_, false>(a, out, T);                                 \
+    return;                                                                   \
   }
+  PA_DIM(64) PA_DIM(128) PA_DIM(256)
+#undef PA_DIM
 }
 
 }  // namespace kaito

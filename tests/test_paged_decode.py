@@ -1,0 +1,74 @@
+"""The MFMA decode attention (ops/csrc/paged_attention_sp.hip) at the edges
+of its 32-key tiles and of the rules that choose 4, 8 or 16 waves per
+workgroup and several workgroups per (sequence, kv head). Weights keep 16
+bits, so the outputs are off by their rounding to bf16 (2^-9) and f32 sums;
+the bound is four times that at the values' largest magnitude."""
+import pytest
+import torch
+
+from kaito_amd import ops
+from kaito_amd.ops import torch_ref as R
+
+DEV = "cuda"
+
+
+def _run(G, KH, D, lens, max_blocks=None, window=0, sink=False, fp8=False):
+    torch.manual_seed(G * D + len(lens))
+    mb = max(max_blocks or 0, -(-max(lens) // 16), 1)
+    used = [-(-n // 16) for n in lens]
+    perm = torch.randperm(sum(used) + 1)
+    bt = torch.zeros(len(lens), mb, dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(used):
+        bt[i, :n] = perm[at:at + n]
+        at += n
+    kc, vc = (torch.randn(sum(used) + 1, KH, 16, D).to(torch.bfloat16)
+              for _ in range(2))
+    args = (kc, vc)
+    if fp8:
+        args = tuple(t.to(torch.float8_e4m3fn) for t in args)
+        kc, vc = (t.to(torch.bfloat16) for t in args)
+        args = tuple(t.view(torch.uint8) for t in args)
+    # a strided query, as cut from a fused projection
+    q = torch.randn(len(lens), G * KH * D + 64).to(torch.bfloat16)
+    sl = torch.tensor(lens, dtype=torch.int32)
+    sinks = torch.randn(G * KH) if sink else None
+    q3 = q.to(DEV)[:, :G * KH * D].unflatten(-1, (-1, D))
+    out = ops.paged_attention(
+        q3, *(t.to(DEV) for t in args), bt.to(DEV), sl.to(DEV), D ** -0.5,
+        window, sinks.to(DEV) if sink else None).cpu().float()
+    live = [i for i, n in enumerate(lens) if n > 0]
+    ref = R.paged_attention(q3.cpu().float()[live], kc.float(), vc.float(),
+                            bt[live], sl[live], D ** -0.5, window, sinks)
+    assert torch.isfinite(out).all()
+    err = (out[live] - ref).abs()
+    assert (err <= 2.0 ** -7 * (ref.abs() + 0.1)).all(), err.max()
+    dead = [i for i, n in enumerate(lens) if n == 0]
+    assert (out[dead] == 0).all()
+
+
+EDGES = [1, 15, 16, 17, 31, 32, 33, 0, 64, 65, 127, 128, 129, 300]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("G,KH,D", [(1, 2, 64), (8, 1, 64), (1, 1, 128),
+                                    (3, 2, 128), (4, 2, 128), (7, 1, 128),
+                                    (8, 1, 128), (1, 2, 256), (4, 1, 256)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_edges(G, KH, D, fp8):
+    _run(G, KH, D, EDGES, fp8=fp8)
+    _run(G, KH, D, EDGES, max_blocks=17, window=40, sink=not fp8, fp8=fp8)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("KH,lens,max_blocks", [
+    (8, [40, 200, 7] * 11, 13),           # 264 pairs: 8 waves
+    (8, [64, 70, 90, 3] * 17, 6),         # 544 pairs: 4 waves
+    (2, [1900, 33, 0, 2047], 128),        # few pairs, long table: splits
+    (1, [5000], 700),
+    (8, [17], 4096),                      # splits that are all but one empty
+])
+@pytest.mark.parametrize("D,fp8", [(128, False), (128, True), (256, False)])
+def test_launch_rules(KH, lens, max_blocks, D, fp8):
+    _run(4, KH, D, lens, max_blocks, fp8=fp8)
+    _run(2, KH, D, lens, max_blocks, window=530, sink=True, fp8=fp8)
