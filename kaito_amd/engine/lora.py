@@ -27,6 +27,11 @@ def set_active(manager: Optional["LoRAManager"],
     _ACTIVE_IDS = ids
 
 
+def is_active() -> bool:
+    """Whether the running step carries adapters."""
+    return _ACTIVE_MANAGER is not None and _ACTIVE_IDS is not None
+
+
 def maybe_apply(module: torch.nn.Module, x: torch.Tensor,
                 y: torch.Tensor) -> torch.Tensor:
     """Called by parallel linear layers after the base GEMM."""

@@ -8,7 +8,6 @@ from typing import Dict, List, Optional
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from .. import ops
 from ..engine.config import ModelConfig
@@ -112,4 +111,4 @@ class HybridStackBase(nn.Module):
         """hidden: rows of the f32 residual stream → f32 logits."""
         h = ops.rms_norm_cast(hidden.contiguous(), self.norm,
                               self.cfg.rms_eps, self.cfg.dtype)
-        return F.linear(h, self.lm_head).float()
+        return ops.linear(h, self.lm_head).float()

@@ -216,7 +216,10 @@ class LlamaMLP(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if not self.cfg.gated_mlp:
             return self.down_proj(ops.gelu(self.up_proj(x)))
-        gu = self.gate_up_proj(x)
+        p = self.gate_up_proj
+        if self.cfg.hidden_act != "gelu_tanh" and p.is_plain():
+            return self.down_proj(ops.linear_swiglu(x, p.weight))
+        gu = p(x)
         act = ops.gelu_and_mul(gu) if self.cfg.hidden_act == "gelu_tanh" \
             else ops.silu_and_mul(gu)
         return self.down_proj(act)
@@ -427,7 +430,7 @@ class LlamaForCausalLM(nn.Module):
         if self.lm_head is not None:
             logits = self.lm_head(hidden)
         else:
-            logits = torch.nn.functional.linear(hidden, self.embed_tokens.weight)
+            logits = ops.linear(hidden, self.embed_tokens.weight)
         logits = tp_all_gather(logits, dim=-1)
         cap = self.cfg.final_logit_softcap
         if cap > 0:   # gemma-2 logit soft-capping

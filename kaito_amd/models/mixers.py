@@ -89,7 +89,7 @@ class GatedDeltaMixer(nn.Module):
     def forward(self, x, positions, cache, meta):
         s = self.spec
         T = x.size(0)
-        p = F.linear(x, self.in_proj)
+        p = ops.linear(x, self.in_proj)
         qkv = ops.causal_conv_update(
             p[:, :self.conv_ch], self.conv_weight, None, cache["conv"],
             meta.cu_seqlens, meta.state_slots, meta.seq_starts,
@@ -105,7 +105,7 @@ class GatedDeltaMixer(nn.Module):
             q, k, v, gate, a, b, self.a_log, self.dt_bias, self.out_norm,
             cache["ssm"], meta.cu_seqlens, meta.state_slots, meta.seq_starts,
             s.qk_eps, self.norm_eps)
-        return F.linear(o.reshape(T, self.n_v), self.o_proj)
+        return ops.linear(o.reshape(T, self.n_v), self.o_proj)
 
 
 class RGLRUMixer(nn.Module):
@@ -152,7 +152,7 @@ class RGLRUMixer(nn.Module):
     def forward(self, x, positions, cache, meta):
         s = self.spec
         T, w = x.size(0), s.width
-        p = F.linear(x, self.in_proj, self.in_bias)
+        p = ops.linear(x, self.in_proj, self.in_bias)
         u = ops.causal_conv_update(
             p[:, w:], self.conv_weight, self.conv_bias, cache["conv"],
             meta.cu_seqlens, meta.state_slots, meta.seq_starts,
@@ -162,7 +162,7 @@ class RGLRUMixer(nn.Module):
         o = ops.rglru_scan(u, gates, p[:, :w], self.decay_rate, cache["lru"],
                            meta.cu_seqlens, meta.state_slots, meta.seq_starts,
                            meta.token_seq)
-        return F.linear(o, self.o_proj)
+        return ops.linear(o, self.o_proj)
 
 
 class BiasedWindowAttention(nn.Module):
@@ -211,7 +211,7 @@ class BiasedWindowAttention(nn.Module):
     def forward(self, x, positions, cache, meta):
         s = self.spec
         T = x.size(0)
-        qkv = F.linear(x, self.qkv_proj)
+        qkv = ops.linear(x, self.qkv_proj)
         q = qkv[:, :self.q_size].unflatten(-1, (s.heads, s.dim))
         k = qkv[:, self.q_size:self.q_size + self.k_size].unflatten(
             -1, (s.kv_heads, s.dim))
@@ -228,7 +228,7 @@ class BiasedWindowAttention(nn.Module):
                                  meta.block_tables, meta.token_seq, positions,
                                  s.scale, s.softcap, self.r1, self.r2,
                                  s.window, tiles=tiles)
-        return F.linear(o.reshape(T, -1), self.o_proj)
+        return ops.linear(o.reshape(T, -1), self.o_proj)
 
 
 class RotaryWindowAttention(nn.Module):
@@ -328,7 +328,7 @@ class RotaryWindowAttention(nn.Module):
     def forward(self, x, positions, cache, meta):
         s = self.spec
         T = x.size(0)
-        p = F.linear(x, self.qkv_proj, self.qkv_bias)
+        p = ops.linear(x, self.qkv_proj, self.qkv_bias)
         qkv = p[:, :self.conv_ch]
         if s.conv_taps > 0:
             qkv = ops.causal_conv_update(
@@ -371,7 +371,7 @@ class RotaryWindowAttention(nn.Module):
         o = o.reshape(T, self.o_size)
         if s.gate:
             o = ops.sigmoid_mul(o, p[:, self.conv_ch:])
-        return F.linear(o, self.o_proj, self.o_bias)
+        return ops.linear(o, self.o_proj, self.o_bias)
 
 
 class MLSTMMixer(nn.Module):
@@ -408,8 +408,8 @@ class MLSTMMixer(nn.Module):
 
     def forward(self, x, positions, cache, meta):
         s = self.spec
-        p = F.linear(x, self.in_proj)
-        gates = F.linear(x.float(), self.gate_proj, self.gate_bias)
+        p = ops.linear(x, self.in_proj)
+        gates = ops.linear(x.float(), self.gate_proj, self.gate_bias)
         nq, nv = self.n_qk, self.n_v
         q = p[:, :nq].unflatten(-1, (s.heads, s.dim))
         k = p[:, nq:2 * nq].unflatten(-1, (s.heads, s.dim))
@@ -420,7 +420,7 @@ class MLSTMMixer(nn.Module):
             cache["c"], cache["n"], cache["m"], meta.cu_seqlens,
             meta.state_slots, meta.seq_starts, s.gate_cap, s.dim ** -0.5,
             self.norm_eps, s.denom_floor)
-        return F.linear(o, self.o_proj)
+        return ops.linear(o, self.o_proj)
 
 
 class SSDMixer(nn.Module):
@@ -468,8 +468,8 @@ class SSDMixer(nn.Module):
 
     def forward(self, x, positions, cache, meta):
         s = self.spec
-        p = F.linear(x, self.in_proj)
-        dt = F.linear(x.float(), self.dt_proj)
+        p = ops.linear(x, self.in_proj)
+        dt = ops.linear(x.float(), self.dt_proj)
         xbc = ops.causal_conv_update(
             p[:, self.inner:], self.conv_weight, self.conv_bias,
             cache["conv"], meta.cu_seqlens, meta.state_slots,
@@ -482,7 +482,7 @@ class SSDMixer(nn.Module):
                          self.dt_bias, self.d_skip, self.out_norm,
                          cache["ssm"], meta.cu_seqlens, meta.state_slots,
                          meta.seq_starts, s.norm_groups, self.norm_eps)
-        return F.linear(y, self.o_proj)
+        return ops.linear(y, self.o_proj)
 
 
 class ClampedGLU(nn.Module):
@@ -497,9 +497,9 @@ class ClampedGLU(nn.Module):
         self.down = _p(hidden, spec.ff, dtype=dtype)
 
     def forward(self, x):
-        a = ops.clamped_glu(F.linear(x, self.gate_up), self.spec.limit,
+        a = ops.clamped_glu(ops.linear(x, self.gate_up), self.spec.limit,
                             self.spec.alpha)
-        return F.linear(a, self.down)
+        return ops.linear(a, self.down)
 
 
 class LatentAttention(nn.Module):
@@ -593,11 +593,11 @@ class LatentAttention(nn.Module):
     def forward(self, x, positions, cache, meta):
         s = self.spec
         T, H, D = x.size(0), s.heads, s.dim
-        p = F.linear(x, self.in_proj)
+        p = ops.linear(x, self.in_proj)
         if s.q_rank > 0:
             cq = ops.rms_norm_cast(p[:, :s.q_rank], self.q_norm,
                                    self.norm_eps, self.dtype)
-            q = F.linear(cq, self.w_uq).unflatten(-1, (H, D + s.rot_dim))
+            q = ops.linear(cq, self.w_uq).unflatten(-1, (H, D + s.rot_dim))
         else:
             q = p[:, :self.q_size].unflatten(-1, (H, D + s.rot_dim))
         dkv = p[:, self.q_rows + self.g_size:self.in_rows] \
@@ -627,7 +627,7 @@ class LatentAttention(nn.Module):
         if self.g_size:
             o = ops.sigmoid_mul(o, p[:, self.q_rows:self.q_rows
                                      + self.g_size])
-        return F.linear(o, self.o_proj)
+        return ops.linear(o, self.o_proj)
 
     def _expanded(self, qr, kv, meta):
         """Prompt portions (bf16): per-head keys and values of the step's
@@ -641,8 +641,8 @@ class LatentAttention(nn.Module):
         lat, tables = ops.latent_gather(kv, meta.block_tables, meta.ctx_lens,
                                         first)
         k_s, v_s = ops.latent_expand(
-            F.linear(lat[:, :s.kv_rank], self.w_uk),
-            F.linear(lat[:, :s.kv_rank], self.w_uv), lat, H, D, V, s.kv_rank,
+            ops.linear(lat[:, :s.kv_rank], self.w_uk),
+            ops.linear(lat[:, :s.kv_rank], self.w_uv), lat, H, D, V, s.kv_rank,
             Dp, Vp, kv.size(1))
         o = ops.window_attention(
             qr, k_s, v_s, tables, meta.token_seq, None, s.scale,
@@ -664,7 +664,7 @@ class GatedFF(nn.Module):
         self.down = _p(hidden, spec.ff, dtype=dtype)
 
     def forward(self, x):
-        return F.linear(self.act(F.linear(x, self.gate_up)), self.down)
+        return ops.linear(self.act(ops.linear(x, self.gate_up)), self.down)
 
 
 class DiagDeltaMixer(nn.Module):
@@ -717,9 +717,9 @@ class DiagDeltaMixer(nn.Module):
     def forward(self, x, positions, cache, meta):
         s = self.spec
         n = self.n
-        p = F.linear(x, self.in_proj)
+        p = ops.linear(x, self.in_proj)
         gp = ops.linear_f32(x, self.gate_proj)               # [T, n + rank]
-        w_pre = F.linear(torch.tanh(gp[:, n:]), self.w2, self.w0)
+        w_pre = ops.linear(torch.tanh(gp[:, n:]), self.w2, self.w0)
         hd = (s.heads, s.dim)
         o = ops.diag_delta_rule(
             p[:, :n].unflatten(-1, hd), p[:, n:2 * n].unflatten(-1, hd),
@@ -727,7 +727,7 @@ class DiagDeltaMixer(nn.Module):
             p[:, 3 * n:].unflatten(-1, hd), self.out_norm, cache["ssm"],
             meta.cu_seqlens, meta.state_slots, meta.seq_starts,
             s.decay_rate, s.k_eps, self.norm_eps, a_bias=self.a_bias)
-        return F.linear(o, self.o_proj)
+        return ops.linear(o, self.o_proj)
 
 
 class HGRN2Mixer(nn.Module):
@@ -762,7 +762,7 @@ class HGRN2Mixer(nn.Module):
 
     def forward(self, x, positions, cache, meta):
         s = self.spec
-        p = F.linear(x, self.in_proj)
+        p = ops.linear(x, self.in_proj)
         f_pre = ops.linear_f32(x, self.f_proj)
         o = ops.hgrn2_scan(
             p[:, :self.n_q].unflatten(-1, (s.heads, s.dim)),
@@ -770,7 +770,7 @@ class HGRN2Mixer(nn.Module):
             self.lower, self.out_norm, cache["ssm"], meta.cu_seqlens,
             meta.state_slots, meta.seq_starts, self.norm_eps,
             f_bias=self.f_bias)
-        return F.linear(o, self.o_proj)
+        return ops.linear(o, self.o_proj)
 
 
 class GLAMixer(nn.Module):
@@ -820,7 +820,7 @@ class GLAMixer(nn.Module):
 
     def forward(self, x, positions, cache, meta):
         s = self.spec
-        p = F.linear(x, self.in_proj)
+        p = ops.linear(x, self.in_proj)
         low = ops.linear_f32(x, self.a1)
         nq, nv = self.n_q, self.n_v
         qk, vg = (s.heads, s.dim), (s.heads, s.vdim)
@@ -831,4 +831,4 @@ class GLAMixer(nn.Module):
             s.tau, s.dim ** -0.5, self.out_norm, cache["ssm"],
             meta.cu_seqlens, meta.state_slots, meta.seq_starts,
             self.norm_eps)
-        return F.linear(o, self.o_proj)
+        return ops.linear(o, self.o_proj)

@@ -124,7 +124,7 @@ class MLAAttention(nn.Module):
 
     def _project_q(self, x: torch.Tensor) -> torch.Tensor:
         if self.cfg.q_lora_rank > 0:
-            qa = torch.nn.functional.linear(x, self.q_a_proj)
+            qa = ops.linear(x, self.q_a_proj)
             qa = ops.rms_norm(qa, self.q_a_layernorm, self.cfg.rms_eps)
             q = self.q_b_proj(qa)
         else:
@@ -140,7 +140,7 @@ class MLAAttention(nn.Module):
         q_nope = q[..., :self.nope]
         q_pe = q[..., self.nope:].contiguous()          # [T, Hl, rope]
 
-        kv_a = torch.nn.functional.linear(x, self.kv_a_proj_with_mqa)
+        kv_a = ops.linear(x, self.kv_a_proj_with_mqa)
         c_kv = ops.rms_norm(kv_a[:, :self.r].contiguous(),
                             self.kv_a_layernorm, self.cfg.rms_eps)
         k_pe = kv_a[:, self.r:].contiguous()            # [T, rope]
@@ -232,7 +232,7 @@ class MLAAttention(nn.Module):
         tiles = None if meta.tile_seq is None else \
             (meta.tile_seq, meta.tile_qbase)
         # decompress: k_nope [T, Hl, nope], v [Hl, T, v]
-        k_nope = torch.nn.functional.linear(
+        k_nope = ops.linear(
             c_kv.to(self.w_kc.dtype), self.w_kc.view(Hl * self.nope, self.r)
         ).view(T, Hl, self.nope)
         v = torch.matmul(c_kv.to(self.w_vc.dtype).unsqueeze(0), self.w_vc)

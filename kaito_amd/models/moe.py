@@ -124,9 +124,9 @@ class MoEMLP(nn.Module):
         T = x.size(0)
         cfg = self.cfg
         if cfg.moe_router_fp32:
-            logits = torch.nn.functional.linear(x.float(), self.gate)
+            logits = ops.linear(x.float(), self.gate)
         else:
-            logits = torch.nn.functional.linear(x, self.gate)  # [T, E]
+            logits = ops.linear(x, self.gate)  # [T, E]
         if cfg.moe_routing in ("noaux_tc", "sigmoid_groups"):
             # deepseek-v3: sigmoid scores; SELECTION uses scores+bias with
             # group-limited top-k; WEIGHTS are the original sigmoid scores.
@@ -219,8 +219,8 @@ class MoEMLP(nn.Module):
         out = out32 if keep_f32 else out32.to(x.dtype)
         shared = None
         if self.w_shared_gate_up is not None:   # deepseek shared experts
-            h1 = torch.nn.functional.linear(x, self.w_shared_gate_up)
-            shared = torch.nn.functional.linear(
+            h1 = ops.linear(x, self.w_shared_gate_up)
+            shared = ops.linear(
                 ops.silu_and_mul(h1) if self.gated else ops.relu2(h1),
                 self.w_shared_down)
         if split_shared:
@@ -261,7 +261,7 @@ class MoEMLP(nn.Module):
                 continue
             rows = idx64[s:t]
             xs = x[rows]
-            h1 = torch.nn.functional.linear(
+            h1 = ops.linear(
                 xs, self.w_gate_up[le],
                 self.b_gate_up[le] if self.b_gate_up is not None else None)
             if self.act_mode == 2:
@@ -270,7 +270,7 @@ class MoEMLP(nn.Module):
                 act = ops.clamped_glu(h1, self.act_limit)
             else:
                 act = ops.silu_and_mul(h1.contiguous())
-            y = torch.nn.functional.linear(
+            y = ops.linear(
                 act, self.w_down[le],
                 self.b_down[le] if self.b_down is not None else None)
             # f32 accumulation over a token's experts, like the fused path

@@ -73,13 +73,8 @@ def repack_awq(qweight_awq: torch.Tensor, qzeros_awq: torch.Tensor,
 
 
 class QuantLinear(torch.nn.Module):
-    """W4A16 linear: HIP GEMV for decode-sized M, dequant + MFMA GEMM
-    (hipBLASLt) beyond. Drop-in for a bias-free nn.Linear."""
-
-    # measured crossover on MI355X (profiles/r01_decode_profile.md):
-    # GEMV wins to M=4 (10-24us vs ~38us dequant+GEMM); beyond, tile
-    # dequant into the MFMA GEMM path wins
-    GEMV_MAX_M = 4
+    """W4A16 linear: HIP kernels on the packed weights for decode-sized M,
+    dequant + MFMA GEMM (hipBLASLt) beyond. Drop-in for a bias-free nn.Linear."""
 
     def __init__(self, qweight, scales, zeros, group: int = 128):
         super().__init__()
@@ -97,7 +92,7 @@ class QuantLinear(torch.nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         shape = x.shape[:-1]
         x2 = x.reshape(-1, self.in_features)
-        if x2.size(0) <= self.GEMV_MAX_M:
+        if ops.w4a16_streams(x2, self.group):
             y = ops.w4a16_gemv(x2, self.qweight, self.scales, self.zeros,
                                self.group)
         elif x.is_cuda and self.out_features % 64 == 0 \

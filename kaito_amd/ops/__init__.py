@@ -24,7 +24,7 @@ _OP_GROUP = {}
 for _g, _names in {
     "core": ("rms_norm fused_add_rms_norm rotary_embedding silu_and_mul "
              "gelu_and_mul gelu layer_norm fused_add_layer_norm "
-             "reshape_and_cache topk"),
+             "reshape_and_cache topk skinny_linear skinny_swiglu"),
     "attn": ("paged_attention paged_attention_sp prefill_attention "
              "mla_prefill_attention context_attention mfma_tile_gemm paged_read_bw"),
     "mla": "mla_decode mla_cache_write",
@@ -137,6 +137,48 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
         _K.silu_and_mul(out, x)
         return out
     return torch_ref.silu_and_mul(x)
+
+
+SKINNY_MAX_M = 4
+
+
+def _skinny(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether x W^T runs on the row-streaming kernel: at most 4 rows of
+    bf16 on the GPU, 16-byte aligned rows, nothing to differentiate. At 8
+    llama-3.1-8b layers' sizes it reads W at 5 to 7 TB/s for one row and 3.7
+    to 5.7 for four, hipBLASLt's tuned choices at 2.2 to 4.8 for both; more
+    rows are bound by the vector unit and stay with the library."""
+    return (x.is_cuda and x.dim() == 2 and 1 <= x.size(0) <= SKINNY_MAX_M
+            and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+            and w.is_contiguous() and w.size(1) % 8 == 0 and w.numel() > 0
+            and x.stride(1) == 1
+            and (x.size(0) == 1 or x.stride(0) % 8 == 0)
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and not (torch.is_grad_enabled()
+                     and (x.requires_grad or w.requires_grad)))
+
+
+def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
+    """x W^T (+ bias): the row-streaming kernel for the smallest decode
+    steps, hipBLASLt otherwise."""
+    if _skinny(x, w) and (bias is None or (
+            bias.dtype == torch.bfloat16 and bias.is_contiguous()
+            and not (torch.is_grad_enabled() and bias.requires_grad))):
+        out = torch.empty(x.size(0), w.size(0), dtype=x.dtype,
+                          device=x.device)
+        _K.skinny_linear(out, x, w, _none(bias, x))
+        return out
+    return torch.nn.functional.linear(x, w, bias)
+
+
+def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu(x Wg^T) * (x Wu^T) for the stacked W = [Wg | Wu]."""
+    if _skinny(x, w):
+        out = torch.empty(x.size(0), w.size(0) // 2, dtype=x.dtype,
+                          device=x.device)
+        _K.skinny_swiglu(out, x, w)
+        return out
+    return silu_and_mul(torch.nn.functional.linear(x, w))
 
 
 def reshape_and_cache(k: torch.Tensor, v: torch.Tensor, k_cache: torch.Tensor,
@@ -385,11 +427,22 @@ def w4a16_gemv(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor,
     """Group-quantized W4A16 linear, small M (decode): out = x @ W^T with
     W dequantized on the fly inside the kernel."""
     if x.is_cuda:
+        x = x.contiguous()
         out = torch.empty(x.size(0), qweight.size(0), dtype=x.dtype,
                           device=x.device)
         _K.w4a16_gemv(out, x, qweight, scales, zeros, group)
         return out
     return torch_ref.w4a16_gemv(x, qweight, scales, zeros, group)
+
+
+def w4a16_streams(x: torch.Tensor, group: int) -> bool:
+    """Whether x [M, K] runs on the packed weights (w4a16_gemv) or on a
+    dequantized copy through the library's GEMM: M <= 4 always; up to 32
+    rows in the kernel's slices of 64 k (8 llama-3.1-8b layers' linears at M
+    = 16: 96 us a layer, of which 75 more for the copy alone)."""
+    return x.size(0) <= 4 or (
+        x.is_cuda and x.size(0) <= 32 and x.dtype == torch.bfloat16
+        and x.size(1) % 64 == 0 and group % 64 == 0)
 
 
 def w4a16_dequant(qweight: torch.Tensor, scales: torch.Tensor,

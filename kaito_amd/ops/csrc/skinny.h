@@ -1,0 +1,286 @@
+// Products of few rows with a large weight matrix, out[M, N] = x[M, K] W^T:
+// the linear layers of a decode step. They stream W once, so the designs are
+// about bytes in flight and the order of addresses; arithmetic is small.
+//
+// M <= 4: a wave streams whole rows, 1 KB of one row per load (full lines, in
+// address order, marked non-temporal), and multiplies on the vector unit
+// (dot2, f32 sums). On one MI355X, N = 28672, K = 4096, M = 1: 33.6 us, 7.0
+// TB/s; the same rows read as MFMA operands (64 B of 16 rows per load) 45.7
+// us, hipBLASLt's tuned choice 57.5 us.
+//
+// More rows of x, and experts with a few rows each: v_mfma_f32_16x16x32_bf16
+// with W read straight into operand registers (a lane's 16 bytes are 8 k of
+// one row); the waves of a workgroup take every NW-th slice of K and meet in
+// LDS, in f32.
+//
+// 4-bit weights run as integers: a word's nibbles j and j + 4 become the bf16
+// pair 128 + q by one shift and one and-or (x is permuted to match), and per
+// group of K, in f32,
+//     y += s (sum (128 + q) x) - (128 s + z) sum x
+// The offset costs 4 bits of the f32 partial sum's 24, out of a result
+// rounded to 8.
+#pragma once
+#include "common.h"
+
+namespace kaito {
+namespace skinny {
+
+typedef __bf16 hbf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+KAITO_DEV f32x4 mfma16(hbf16x8 a, hbf16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// streamed once: leave the caches to x
+template <typename V>
+KAITO_DEV V load_stream(const void* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const V*>(p));
+}
+
+KAITO_DEV hbf16x8 load_x(const short* p) {
+  return *reinterpret_cast<const hbf16x8*>(p);
+}
+
+// acc[mt][j] += x rows 16 mt.. times W rows of tile j, over the slices of
+// this wave. wp/xp: the lane's rows (l & 15) at k = 8 (l >> 4).
+template <int MT, int NT>
+KAITO_DEV void accumulate(f32x4 (&acc)[MT][NT], const short* const (&wp)[NT],
+                          const short* const (&xp)[MT], const int K,
+                          const int wave, const int nw) {
+  constexpr int STEPS = MT * NT <= 2 ? 8 : (MT * NT <= 4 ? 4 : 2);
+  constexpr int KC = STEPS * 32;
+  for (int k0 = wave * KC; k0 < K; k0 += nw * KC) {
+    if (k0 + KC <= K) {
+      hbf16x8 wf[NT][STEPS], xf[MT][STEPS];
+#pragma unroll
+      for (int s = 0; s < STEPS; s++)
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+          wf[j][s] = load_stream<hbf16x8>(wp[j] + k0 + s * 32);
+#pragma unroll
+      for (int s = 0; s < STEPS; s++)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+          xf[mt][s] = load_x(xp[mt] + k0 + s * 32);
+#pragma unroll
+      for (int s = 0; s < STEPS; s++)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+          for (int j = 0; j < NT; j++)
+            acc[mt][j] = mfma16(xf[mt][s], wf[j][s], acc[mt][j]);
+    } else {
+      for (int k = k0; k < K; k += 32)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+          for (int j = 0; j < NT; j++)
+            acc[mt][j] = mfma16(load_x(xp[mt] + k),
+                                load_stream<hbf16x8>(wp[j] + k), acc[mt][j]);
+    }
+  }
+}
+
+// the eight nibbles of a word as bf16 128 + q, in the order 0 4 1 5 2 6 3 7
+KAITO_DEV hbf16x8 nibbles(const unsigned int w) {
+  u32x4 r;
+#pragma unroll
+  for (int j = 0; j < 4; j++)
+    r[j] = ((w >> (4 * j)) & 0x000f000fu) | 0x43004300u;
+  return __builtin_bit_cast(hbf16x8, r);
+}
+
+// x in that order
+KAITO_DEV hbf16x8 nibble_order(const hbf16x8 x) {
+  return __builtin_shufflevector(x, x, 0, 4, 1, 5, 2, 6, 3, 7);
+}
+
+// 4-bit weights [N, K / 8]; WORDS words per lane and slice: a slice is
+// WORDS * 32 k and lies in one group (WORDS 4: groups of 128 n, 2: of 64 n).
+// A lane's k are 8 WORDS (l >> 4) onward; sc/ze: the lane's rows.
+template <int MT, int NT, int WORDS>
+KAITO_DEV void accumulate_w4(f32x4 (&acc)[MT][NT],
+                             const unsigned int* const (&wp)[NT],
+                             const float* const (&sc)[NT],
+                             const float* const (&ze)[NT],
+                             const short* const (&xp)[MT], const int K,
+                             const int group, const int wave, const int nw) {
+  constexpr int KC = WORDS * 32;
+  constexpr int U = MT * NT <= 2 ? 2 : 1;       // slices under way
+  typedef unsigned int wordv __attribute__((ext_vector_type(WORDS)));
+  const hbf16x8 ones = {1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f};
+  for (int k0 = wave * U * KC; k0 < K; k0 += nw * U * KC) {
+    wordv w[U][NT];
+    float s[U][NT], z[U][NT];
+    hbf16x8 xf[U][MT][WORDS];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int k = min(k0 + u * KC, K - KC);   // past the end: weighed zero
+      const float live = k0 + u * KC < K ? 1.f : 0.f;
+#pragma unroll
+      for (int j = 0; j < NT; j++) {
+        w[u][j] = load_stream<wordv>(wp[j] + k / 8);
+        s[u][j] = sc[j][k / group] * live;
+        z[u][j] = ze[j][k / group] * live;
+      }
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int i = 0; i < WORDS; i++)
+          xf[u][mt][i] = load_x(xp[mt] + k + i * 8);
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      f32x4 xs[MT], dot[MT][NT];
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++) {
+        xs[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < NT; j++) dot[mt][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll
+      for (int i = 0; i < WORDS; i++) {
+        hbf16x8 q[NT];
+#pragma unroll
+        for (int j = 0; j < NT; j++) q[j] = nibbles(w[u][j][i]);
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+          const hbf16x8 xv = nibble_order(xf[u][mt][i]);
+          xs[mt] = mfma16(xv, ones, xs[mt]);
+#pragma unroll
+          for (int j = 0; j < NT; j++)
+            dot[mt][j] = mfma16(xv, q[j], dot[mt][j]);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < NT; j++) {
+        const float zz = 128.f * s[u][j] + z[u][j];
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            acc[mt][j][r] += s[u][j] * dot[mt][j][r] - zz * xs[mt][r];
+      }
+    }
+  }
+}
+
+// Sums of the waves' tiles: thread (slot = tile * 64 + lane) gets its f32x4.
+// red: [NW][TILES * 64]
+template <int TILES, int NW>
+KAITO_DEV f32x4 fold(const f32x4* red, const int slot) {
+  f32x4 v = red[slot];
+#pragma unroll
+  for (int w = 1; w < NW; w++) v += red[w * TILES * 64 + slot];
+  return v;
+}
+
+// ---- M <= 4: rows streamed by a wave ---------------------------------------
+typedef __bf16 hbf16x2 __attribute__((ext_vector_type(2)));
+
+KAITO_DEV float dot8(const hbf16x8 a, const hbf16x8 b, float c) {
+  const hbf16x2* p = reinterpret_cast<const hbf16x2*>(&a);
+  const hbf16x2* q = reinterpret_cast<const hbf16x2*>(&b);
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    c = __builtin_amdgcn_fdot2_f32_bf16(p[i], q[i], c, false);
+  return c;
+}
+
+// acc[m][r] += x row m . W row r, this lane's k only. wp: row starts.
+template <int M, int R>
+KAITO_DEV void stream_rows(float (&acc)[M][R], const short* const (&wp)[R],
+                           const short* x, const int64_t x_stride,
+                           const int K, const int lane) {
+  constexpr int U = M * R <= 4 ? 4 : 2;
+  int k0 = 0;
+  for (; k0 + 512 * U <= K; k0 += 512 * U) {
+    hbf16x8 w[U][R], v[U][M];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int r = 0; r < R; r++)
+        w[u][r] = load_stream<hbf16x8>(wp[r] + k0 + u * 512 + lane * 8);
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int m = 0; m < M; m++)
+        v[u][m] = load_x(x + m * x_stride + k0 + u * 512 + lane * 8);
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int m = 0; m < M; m++)
+#pragma unroll
+        for (int r = 0; r < R; r++) acc[m][r] = dot8(w[u][r], v[u][m], acc[m][r]);
+  }
+  for (int k = k0 + lane * 8; k < K; k += 512) {
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const hbf16x8 w = load_stream<hbf16x8>(wp[r] + k);
+#pragma unroll
+      for (int m = 0; m < M; m++)
+        acc[m][r] = dot8(w, load_x(x + m * x_stride + k), acc[m][r]);
+    }
+  }
+}
+
+// the same for 4-bit rows: a lane's 16 bytes are 32 k of one group
+template <int M, int R>
+KAITO_DEV void stream_rows_w4(float (&acc)[M][R],
+                              const unsigned int* const (&wp)[R],
+                              const float* const (&sc)[R],
+                              const float* const (&ze)[R], const short* x,
+                              const int64_t x_stride, const int K,
+                              const int group, const int lane) {
+  const hbf16x8 ones = {1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f};
+  for (int k0 = lane * 32; k0 - lane * 32 < K; k0 += 2048) {
+    const int k = min(k0, K - 32);
+    const float live = k0 < K ? 1.f : 0.f;      // past the end: weighed zero
+    u32x4 w[R];
+    float s[R], z[R];
+    hbf16x8 xv[M][4];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      w[r] = load_stream<u32x4>(wp[r] + k / 8);
+      s[r] = sc[r][k / group] * live;
+      z[r] = ze[r][k / group] * live;
+    }
+#pragma unroll
+    for (int m = 0; m < M; m++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        xv[m][i] = load_x(x + m * x_stride + k + i * 8);
+    float dot[M][R], xs[M];
+#pragma unroll
+    for (int m = 0; m < M; m++) {
+      xs[m] = 0.f;
+#pragma unroll
+      for (int r = 0; r < R; r++) dot[m][r] = 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      hbf16x8 q[R];
+#pragma unroll
+      for (int r = 0; r < R; r++) q[r] = nibbles(w[r][i]);
+#pragma unroll
+      for (int m = 0; m < M; m++) {
+        const hbf16x8 v = nibble_order(xv[m][i]);
+        xs[m] = dot8(v, ones, xs[m]);
+#pragma unroll
+        for (int r = 0; r < R; r++) dot[m][r] = dot8(v, q[r], dot[m][r]);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const float zz = 128.f * s[r] + z[r];
+#pragma unroll
+      for (int m = 0; m < M; m++) acc[m][r] += s[r] * dot[m][r] - zz * xs[m];
+    }
+  }
+}
+
+KAITO_DEV float silu(float v) { return v / (1.f + __expf(-v)); }
+
+}  // namespace skinny
+}  // namespace kaito

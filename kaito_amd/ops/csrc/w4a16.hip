@@ -10,13 +10,11 @@
 // Two paths:
 //   w4a16_gemv    : M <= 32 decode shapes. Memory-bound on the 4-bit
 //                   weights (N*K/2 bytes vs 2*N*K for bf16 -> ~4x less
-//                   traffic than a bf16 GEMM at small M). One wave per
-//                   output row; lane takes 8-k packs round-robin so the
-//                   qweight reads coalesce per wave; x reads are short8.
+//                   traffic than a bf16 GEMM at small M); skinny.h.
 //   w4a16_dequant : tile dequant to bf16 scratch; large-M callers then run
 //                   the scratch through hipBLASLt MFMA (dequant is
 //                   O(N*K) against the GEMM's O(M*N*K) -> noise at M>=128).
-#include "common.h"
+#include "skinny.h"
 #include <torch/library.h>
 #include <ATen/ATen.h>
 #include <ATen/hip/HIPContext.h>
@@ -24,71 +22,90 @@
 namespace kaito {
 
 // ---------------------------------------------------------------- gemv
-// grid.x = N / ROWS, block = ROWS waves; each wave owns one output row.
-template <int M_TILE>
-__global__ __launch_bounds__(256, 4)
-void w4a16_gemv_kernel(short* __restrict__ out,          // [M, N] bf16
-                       const short* __restrict__ x,      // [M, K] bf16
-                       const uint32_t* __restrict__ qw,  // [N, K/8]
-                       const float* __restrict__ scales, // [N, K/G]
-                       const float* __restrict__ zeros,  // [N, K/G]
-                       int M, int N, int K, int group) {
-  // Each wave owns one output row n. A lane takes a CONTIGUOUS 8-word
-  // (64-k) slice per tile so its slice sits inside ONE quant group:
-  // scale/zero load once per slice (vs per word), q loads are uint4
-  // (16B), x loads are short8 (16B). Weight traffic is then the pure
-  // N*K/2 bytes and the kernel runs at HBM rate for small M.
-  const int wave = threadIdx.x >> 6;
+// M <= 4: a wave streams whole rows of packed weights, two or four of them
+// against the same x. One row of x: 15.1 us for N = 28672, K = 4096 (4.4
+// TB/s), 10.6 us for 4096 x 14336, 4.5 us for 4096 x 4096; with more rows the
+// vector unit is the bound (M = 2: 21.6, 17.2, 6.9 us). The linears of a
+// llama-3.1-8b layer at M = 2 took 124 us where a lane had 64 k of one row
+// and converted nibbles to f32 one by one.
+template <int M, int R>
+__global__ __launch_bounds__(256) void w4a16_stream_kernel(
+    short* __restrict__ out, const short* __restrict__ x,
+    const uint32_t* __restrict__ qw, const float* __restrict__ scales,
+    const float* __restrict__ zeros, int N, int K, int group) {
   const int lane = threadIdx.x & 63;
-  const int n = blockIdx.x * 4 + wave;
-  if (n >= N) return;
-  const int kw = K >> 3;                      // u32 words per row
-  const uint32_t* qrow = qw + (int64_t)n * kw;
-  const int gstride = K / group;
-  const float* srow = scales + (int64_t)n * gstride;
-  const float* zrow = zeros + (int64_t)n * gstride;
-
-  float acc[M_TILE];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = (blockIdx.x * 4 + wave) * R;
+  if (n0 >= N) return;
+  const uint32_t* wp[R];
+  const float *sc[R], *ze[R];
+  float acc[M][R];
 #pragma unroll
-  for (int m = 0; m < M_TILE; ++m) acc[m] = 0.f;
-
-  typedef uint32_t uint4_t __attribute__((ext_vector_type(4)));
-  for (int t = lane * 8; t < kw; t += 64 * 8) {  // 8 contiguous words/lane
-    const int k0 = t << 3;                       // 64 k per slice
-    const float s = srow[k0 / group];
-    const float z = zrow[k0 / group];
-    const uint4_t qa = *reinterpret_cast<const uint4_t*>(qrow + t);
-    const uint4_t qb = *reinterpret_cast<const uint4_t*>(qrow + t + 4);
-    float dotm[M_TILE], xsm[M_TILE];
+  for (int r = 0; r < R; r++) {
+    const int64_t n = min(n0 + r, N - 1);
+    wp[r] = qw + n * (K >> 3);
+    sc[r] = scales + n * (K / group);
+    ze[r] = zeros + n * (K / group);
 #pragma unroll
-    for (int m = 0; m < M_TILE; ++m) { dotm[m] = 0.f; xsm[m] = 0.f; }
+    for (int m = 0; m < M; m++) acc[m][r] = 0.f;
+  }
+  skinny::stream_rows_w4<M, R>(acc, wp, sc, ze, x, K, K, group, lane);
 #pragma unroll
-    for (int w = 0; w < 8; ++w) {
-      const uint32_t q = (w < 4) ? qa[w] : qb[w - 4];
-      float qv[8];
+  for (int m = 0; m < M; m++)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) qv[j] = (float)((q >> (4 * j)) & 0xF);
-#pragma unroll
-      for (int m = 0; m < M_TILE; ++m) {
-        if (m >= M) break;
-        const short8_t xv = *reinterpret_cast<const short8_t*>(
-            x + (int64_t)m * K + k0 + w * 8);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float xf = bf16_to_f32(xv[j]);
-          dotm[m] += xf * qv[j];
-          xsm[m] += xf;
-        }
-      }
+    for (int r = 0; r < R; r++) {
+      const float v = wave_reduce_sum(acc[m][r]);
+      if (lane == 0 && n0 + r < N) out[(int64_t)m * N + n0 + r] = f32_to_bf16(v);
     }
+}
+
+// 5 <= M <= 32: the same weights as MFMA operands, 16 rows per workgroup,
+// the waves over K
+template <int MT, int NT, int WORDS>
+__global__ __launch_bounds__(256) void w4a16_mfma_kernel(
+    short* __restrict__ out, const short* __restrict__ x,
+    const uint32_t* __restrict__ qw, const float* __restrict__ scales,
+    const float* __restrict__ zeros, int M, int N, int K, int group) {
+  constexpr int TILES = MT * NT, NW = 4;
+  __shared__ f32x4 red[NW * TILES * 64];
+  const int lane = threadIdx.x & 63, lo = lane & 15, hi = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = blockIdx.x * 16 * NT;
+  const uint32_t* wp[NT];
+  const float *sc[NT], *ze[NT];
+  const short* xp[MT];
 #pragma unroll
-    for (int m = 0; m < M_TILE; ++m) acc[m] += s * dotm[m] - z * xsm[m];
+  for (int j = 0; j < NT; j++) {
+    const int64_t n = min(n0 + j * 16 + lo, N - 1);
+    wp[j] = qw + n * (K >> 3) + hi * WORDS;
+    sc[j] = scales + n * (K / group);
+    ze[j] = zeros + n * (K / group);
   }
 #pragma unroll
-  for (int m = 0; m < M_TILE; ++m) {
-    if (m >= M) break;
-    const float r = wave_reduce_sum(acc[m]);
-    if (lane == 0) out[(int64_t)m * N + n] = f32_to_bf16(r);
+  for (int mt = 0; mt < MT; mt++)
+    xp[mt] = x + (int64_t)min(mt * 16 + lo, M - 1) * K + hi * 8 * WORDS;
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+    for (int j = 0; j < NT; j++) acc[mt][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  skinny::accumulate_w4<MT, NT, WORDS>(acc, wp, sc, ze, xp, K, group, wave,
+                                       NW);
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+      red[(wave * TILES + j * MT + mt) * 64 + lane] = acc[mt][j];
+  __syncthreads();
+  for (int slot = threadIdx.x; slot < TILES * 64; slot += NW * 64) {
+    const f32x4 v = skinny::fold<TILES, NW>(red, slot);
+    const int tile = slot / 64, l = slot % 64, mt = tile % MT;
+    const int n = n0 + tile / MT * 16 + (l & 15);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int m = mt * 16 + (l >> 4) * 4 + r;
+      if (m < M && n < N) out[(int64_t)m * N + n] = f32_to_bf16(v[r]);
+    }
   }
 }
 
@@ -255,19 +272,44 @@ void w4a16_gemv(at::Tensor out, at::Tensor x, at::Tensor qweight,
   TORCH_CHECK(M <= 32, "w4a16_gemv: M must be <= 32 (use dequant+GEMM)");
   TORCH_CHECK(K % 64 == 0 && group % 64 == 0 && K % group == 0,
               "w4a16_gemv: 64|K and 64|group required");
-  dim3 grid((N + 3) / 4), block(256);
+  TORCH_CHECK(x.is_contiguous() && out.is_contiguous());
+  if (M == 0 || N == 0) return;
   auto stream = at::hip::getCurrentHIPStream();
-  auto launch = [&](auto mt) {
-    w4a16_gemv_kernel<decltype(mt)::value><<<grid, block, 0, stream>>>(
-        (short*)out.data_ptr(), (const short*)x.data_ptr(),
-        (const uint32_t*)qweight.data_ptr(), scales.data_ptr<float>(),
-        zeros.data_ptr<float>(), M, N, K, (int)group);
-  };
-  if (M <= 1) launch(std::integral_constant<int, 1>{});
-  else if (M <= 4) launch(std::integral_constant<int, 4>{});
-  else if (M <= 8) launch(std::integral_constant<int, 8>{});
-  else if (M <= 16) launch(std::integral_constant<int, 16>{});
-  else launch(std::integral_constant<int, 32>{});
+#define W4_ARGS                                                               \
+  (short*)out.data_ptr(), (const short*)x.data_ptr(),                         \
+      (const uint32_t*)qweight.data_ptr(), scales.data_ptr<float>(),          \
+      zeros.data_ptr<float>()
+#define W4_STREAM(M_, R_)                                                     \
+  hipLaunchKernelGGL((w4a16_stream_kernel<M_, R_>),                           \
+                     dim3((N + 4 * R_ - 1) / (4 * R_)), dim3(256), 0, stream, \
+                     W4_ARGS, N, K, (int)group)
+  // four rows per wave share what they do with x once there are waves to
+  // spare (M = 4, N = 28672: 30.3 us against 38.6 with two; N = 6144: 12.8
+  // against 11.5)
+  const bool many = N >= 16384;
+  switch (M) {
+    case 1: W4_STREAM(1, 2); return;
+    case 2: if (many) W4_STREAM(2, 4); else W4_STREAM(2, 2); return;
+    case 3: if (many) W4_STREAM(3, 4); else W4_STREAM(3, 2); return;
+    case 4: if (many) W4_STREAM(4, 4); else W4_STREAM(4, 2); return;
+    default: break;
+  }
+#undef W4_STREAM
+#define W4_MFMA(MT_, NT_, WORDS_)                                             \
+  hipLaunchKernelGGL((w4a16_mfma_kernel<MT_, NT_, WORDS_>),                   \
+                     dim3((N + 16 * NT_ - 1) / (16 * NT_)), dim3(256), 0,     \
+                     stream, W4_ARGS, M, N, K, (int)group)
+  // two tiles per workgroup halve the x reads; only where rows are many
+  // enough to fill the chip all the same
+  const bool wide = N >= 16 * 2 * 256;
+  if (group % 128 == 0) {
+    if (M <= 16) { if (wide) W4_MFMA(1, 2, 4); else W4_MFMA(1, 1, 4); }
+    else { if (wide) W4_MFMA(2, 2, 4); else W4_MFMA(2, 1, 4); }
+  } else {
+    if (M <= 16) W4_MFMA(1, 1, 2); else W4_MFMA(2, 1, 2);
+  }
+#undef W4_MFMA
+#undef W4_ARGS
 }
 
 void w4a16_dequant(at::Tensor out, at::Tensor qweight, at::Tensor scales,

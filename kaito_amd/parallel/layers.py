@@ -2,7 +2,8 @@
 
 Column-parallel: weight split along output dim, no comm on forward.
 Row-parallel: weight split along input dim, all-reduce on forward.
-At tp=1 these are plain GEMMs (hipBLASLt via torch.nn.functional.linear).
+At tp=1 these are plain products (ops.linear: the row-streaming kernel for
+the smallest decode steps, hipBLASLt beyond).
 """
 from __future__ import annotations
 
@@ -10,6 +11,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from .. import ops
 from .state import get_state, tp_all_reduce
 from ..engine import lora as lora_mod
 
@@ -34,7 +36,6 @@ class _QuantMixin:
                              group: int = 128) -> None:
         """Install pre-packed 4-bit weights (native layout) — the AWQ
         checkpoint load path."""
-        from ..models.quant import QuantLinear
         dev = self.weight.device
         dtype = self.weight.dtype
         self.register_buffer("qweight", qweight.to(dev))
@@ -44,14 +45,12 @@ class _QuantMixin:
         self.weight = nn.Parameter(torch.empty(0, dtype=dtype, device=dev),
                                    requires_grad=False)  # drop bf16 copy
         self._quantized = True
-        self._gemv_max_m = QuantLinear.GEMV_MAX_M
 
     def _qmatmul(self, x: torch.Tensor) -> torch.Tensor:
-        from .. import ops
         shape = x.shape[:-1]
         x2 = x.reshape(-1, x.shape[-1])
-        if x2.size(0) <= self._gemv_max_m:
-            y = ops.w4a16_gemv(x2.contiguous(), self.qweight, self.scales,
+        if ops.w4a16_streams(x2, self.q_group):
+            y = ops.w4a16_gemv(x2, self.qweight, self.scales,
                                self.zeros, self.q_group)
         elif x.is_cuda and self.qweight.size(0) % 64 == 0 \
                 and x2.shape[-1] % 64 == 0 and ops.W4A16_FUSED_GEMM:
@@ -81,13 +80,19 @@ class ColumnParallelLinear(_QuantMixin, nn.Module):
             torch.empty(self.out_features_per_rank, dtype=dtype),
             requires_grad=False) if bias else None
 
+    def is_plain(self) -> bool:
+        """Nothing but the product with the weight: no bias, packed weight
+        or adapter."""
+        return self.bias is None and not self._quantized \
+            and not lora_mod.is_active()
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self._quantized:
             out = self._qmatmul(x)
             if self.bias is not None:
                 out = out + self.bias
         else:
-            out = F.linear(x, self.weight, self.bias)
+            out = ops.linear(x, self.weight, self.bias)
         return lora_mod.maybe_apply(self, x, out)
 
 
@@ -115,7 +120,8 @@ class RowParallelLinear(_QuantMixin, nn.Module):
             requires_grad=False) if bias else None
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        out = self._qmatmul(x) if self._quantized else F.linear(x, self.weight)
+        out = self._qmatmul(x) if self._quantized \
+            else ops.linear(x, self.weight)
         out = lora_mod.maybe_apply(self, x, out)
         if self.fuse_norm and self.bias is None and get_state().tp_size > 1:
             from . import one_shot

@@ -1,0 +1,67 @@
+"""Linear layers of small decode steps (ops/csrc/skinny.h): rows of x and of
+the weight, lengths of K around the steps of the loops, 4-bit groups. Sums
+are f32 (their error is far below), results bf16: half a unit of the 8 bits,
+and one unit where the sum cancels down to 1/16 of its typical size."""
+import pytest
+import torch
+
+from kaito_amd import ops
+from kaito_amd.models.quant import quantize_w4
+from kaito_amd.ops import torch_ref as R
+
+DEV = "cuda"
+
+
+def _close(out, ref):
+    assert out.dtype == torch.bfloat16 and torch.isfinite(out).all()
+    err = (out.double() - ref).abs()
+    rms = ref.square().mean().sqrt()
+    assert (err <= 2.0 ** -8 * ref.abs() + 2.0 ** -12 * rms).all(), err.max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("N,K", [(1, 8), (7, 64), (300, 520), (33, 2048),
+                                 (64, 2056), (129, 4608), (6, 14336)])
+def test_rows(M, N, K):
+    torch.manual_seed(M * N + K)
+    big = torch.randn(M, K + 16, device=DEV).to(torch.bfloat16)
+    x = big[:, 8:8 + K]                      # strided rows
+    w = torch.randn(2 * N, K, device=DEV).to(torch.bfloat16)
+    b = torch.randn(2 * N, device=DEV).to(torch.bfloat16)
+    ref = x.double() @ w.double().T
+    assert ops._skinny(x, w)
+    _close(ops.linear(x, w), ref)
+    _close(ops.linear(x, w, b), ref + b.double())
+    g, u = ref.chunk(2, -1)
+    _close(ops.linear_swiglu(x, w), g * torch.sigmoid(g) * u)
+
+
+@pytest.mark.gpu
+def test_other_forms_stay_with_the_library():
+    x = torch.randn(5, 64, device=DEV).to(torch.bfloat16)
+    w = torch.randn(32, 64, device=DEV).to(torch.bfloat16)
+    for a, b in [(x, w), (x[:2, :60], w[:, :60]), (x[:2, 1:57], w[:, :56].
+                 contiguous()), (x[:2].float(), w.float()), (x[:2, None], w),
+                 (x[:0], w), (x[:2], w.T.contiguous().T)]:
+        assert not ops._skinny(a, b)
+        assert torch.equal(ops.linear(a, b),
+                           torch.nn.functional.linear(a, b))
+    w.requires_grad_(True)
+    assert not ops._skinny(x[:2], w)
+    assert ops.linear(x[:2], w).requires_grad
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 16, 17, 32])
+@pytest.mark.parametrize("N,K,G", [(1, 64, 64), (40, 128, 128),
+                                   (33, 192, 192), (100, 4224, 128),
+                                   (17, 2112, 64), (8200, 384, 128),
+                                   (16390, 128, 128)])
+def test_packed_rows(M, N, K, G):
+    torch.manual_seed(M + K)
+    qw, s, z = (t.to(DEV) for t in quantize_w4(torch.randn(N, K), G))
+    x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    assert ops.w4a16_streams(x, G)
+    w = R.w4a16_unpack(qw.cpu(), s.cpu(), z.cpu(), G).to(DEV)
+    _close(ops.w4a16_gemv(x, qw, s, z, G), x.double() @ w.double().T)
