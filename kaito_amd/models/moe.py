@@ -117,72 +117,44 @@ class MoEMLP(nn.Module):
         else:
             self.w_shared_gate_up = None
 
-    def _route(self, x: torch.Tensor):
-        """Device-only top-k routing + expert sort. Returns
-        (sorted_tok int32 [TK], gates f32 [TK], offsets int32 [E+1],
-        weight f32 [T] on identity experts or None)."""
-        T = x.size(0)
+    def _choose(self, x: torch.Tensor):
+        """Top-k choice, device-only: (experts int32 [T, K], weights f32
+        [T, K], summed weight f32 [T] on identity experts)."""
         cfg = self.cfg
-        if cfg.moe_router_fp32:
-            logits = ops.linear(x.float(), self.gate)
-        else:
-            logits = ops.linear(x, self.gate)  # [T, E]
+        bias, groups, keep = None, 1, 1
+        renorm, scale = cfg.moe_norm_topk, cfg.routed_scaling_factor
         if cfg.moe_routing in ("noaux_tc", "sigmoid_groups"):
             # deepseek-v3: sigmoid scores; SELECTION uses scores+bias with
             # group-limited top-k; WEIGHTS are the original sigmoid scores.
             # "sigmoid_groups" is the same without a selection bias.
-            scores = torch.sigmoid(logits.float())
-            sel = scores + self.e_score_correction_bias \
-                if cfg.moe_routing == "noaux_tc" else scores
-            if cfg.n_group > 1:
-                gs = sel.view(T, cfg.n_group, -1)
-                group_score = gs.topk(min(2, gs.size(-1)), dim=-1)[0].sum(-1)
-                gi = group_score.topk(cfg.topk_group, dim=-1)[1]  # [T, kg]
-                mask = torch.zeros(T, cfg.n_group, device=x.device,
-                                   dtype=torch.bool)
-                mask.scatter_(1, gi, True)
-                sel = sel.masked_fill(
-                    ~mask.unsqueeze(-1).expand_as(gs).reshape(T, -1),
-                    float("-inf"))
-            topi = sel.topk(self.top_k, dim=-1)[1]             # [T, K]
-            topw = scores.gather(1, topi)
-            if cfg.moe_norm_topk:
-                topw = topw / (topw.sum(-1, keepdim=True) + 1e-20)
-            topw = topw * cfg.routed_scaling_factor
+            mode = "sigmoid"
+            groups, keep = cfg.n_group, cfg.topk_group
+            if cfg.moe_routing == "noaux_tc":
+                bias = self.e_score_correction_bias
         elif cfg.moe_routing == "softmax_bias":
             # softmax over all outputs; the choice adds the correction
             # (and is group-limited), the weights are the chosen scores
-            topi, topw, w_id = ops.moe_route(
-                logits.float(), self.e_score_correction_bias, self.top_k,
-                self.num_experts, cfg.n_group, cfg.topk_group,
-                cfg.moe_norm_topk, cfg.routed_scaling_factor)
-            # identity outputs sort behind every expert's rows
-            return ops.moe_sort(topi, topw, self.n_route) \
-                + (w_id if self.n_identity else None,)
+            mode = "softmax"
+            groups, keep = cfg.n_group, cfg.topk_group
+            bias = self.e_score_correction_bias
         elif cfg.moe_routing == "topk_softmax":
             # gpt-oss: top-k on raw logits, softmax over the selected k
-            topl, topi = torch.topk(logits.float(), self.top_k, dim=-1)
-            topw = torch.softmax(topl, dim=-1)
+            mode, renorm, scale = "logits", False, 1.0
         else:
-            probs = torch.softmax(logits.float(), dim=-1)
-            topw, topi = torch.topk(probs, self.top_k, dim=-1)  # [T, K]
-            if cfg.moe_norm_topk:
-                topw = topw / topw.sum(-1, keepdim=True)
-            topw = topw * cfg.routed_scaling_factor
-        flat_e = topi.reshape(-1)                              # [T*K]
-        flat_t = torch.arange(T, device=x.device,
-                              dtype=torch.int32).repeat_interleave(self.top_k)
-        order = torch.argsort(flat_e, stable=True)
-        sorted_tok = flat_t[order]
-        gates = topw.reshape(-1)[order].float()
-        counts = torch.zeros(self.num_experts, device=x.device,
-                             dtype=torch.int32)
-        counts.scatter_add_(0, flat_e,
-                            torch.ones_like(flat_e, dtype=torch.int32))
-        offsets = torch.zeros(self.num_experts + 1, device=x.device,
-                              dtype=torch.int32)
-        torch.cumsum(counts, 0, out=offsets[1:])
-        return sorted_tok, gates, offsets, None
+            mode = "softmax"
+        # f32 router: x is widened before the product
+        return ops.moe_gate_route(x, self.gate, bias, self.top_k,
+                                  self.num_experts, groups, keep, renorm,
+                                  scale, mode)
+
+    def _route(self, x: torch.Tensor):
+        """Device-only top-k routing + expert sort. Returns
+        (sorted_tok int32 [TK], gates f32 [TK], offsets int32 [E+1],
+        weight f32 [T] on identity experts or None)."""
+        topi, topw, w_id = self._choose(x)
+        # identity outputs sort behind every expert's rows
+        return ops.moe_sort(topi, topw, self.n_route) \
+            + (w_id if self.n_identity else None,)
 
     # fused kernels win at decode-sized batches (weight-streaming
     # bound, graph-capturable); per-expert hipBLASLt GEMMs win at

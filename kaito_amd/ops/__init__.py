@@ -29,7 +29,7 @@ for _g, _names in {
              "mla_prefill_attention context_attention mfma_tile_gemm paged_read_bw"),
     "mla": "mla_decode mla_cache_write",
     "moe": "moe_gate_silu moe_down_scatter",
-    "route": "moe_route moe_sort",
+    "route": "moe_route moe_gate_route moe_sort",
     "quant": "w4a16_gemv w4a16_dequant w4a16_gemm lora_shrink lora_expand",
     "comm": ("allreduce_rmsnorm one_shot_ar_rmsnorm ipc_handle ipc_open "
              "ipc_close"),
@@ -388,38 +388,81 @@ def moe_down_scatter(out: torch.Tensor, act: torch.Tensor,
 MOE_ROUTE_MAX = (1024, 64, 64)      # router outputs, chosen, groups
 
 
+ROUTE_MAX = 1024      # router outputs of the kernels; more run as torch ops
+ROUTE_MODES = {"softmax": 0, "sigmoid": 1, "logits": 2}
+
+
+def _route_out(T: int, top: int, device):
+    f32 = dict(dtype=torch.float32, device=device)
+    return (torch.empty(T, top, dtype=torch.int32, device=device),
+            torch.empty(T, top, **f32), torch.empty(T, **f32))
+
+
 def moe_route(logits, correction, top: int, n_real: int, groups: int = 1,
-              keep: int = 1, renorm: bool = False, scale: float = 1.0):
-    """Expert choice from f32 router logits [T, N]: scores s = softmax; the
-    choice adds `correction` [N] f32 (None: nothing); outputs form `groups` equal groups of
-    neighbours scored by their largest choice, of which the `keep` best
-    stay eligible; the `top` largest eligible choices are taken. Weights
-    are s (without the correction), over their sum + 1e-20 with `renorm`,
-    times scale. Returns (indices [T, top] int32, weights [T, top] f32,
-    summed weight [T] f32 of the taken outputs with index >= n_real)."""
-    if logits.is_cuda:
-        T = logits.size(0)
-        f32 = dict(dtype=torch.float32, device=logits.device)
-        topi = torch.empty(T, top, dtype=torch.int32, device=logits.device)
-        topw, w_id = torch.empty(T, top, **f32), torch.empty(T, **f32)
+              keep: int = 1, renorm: bool = False, scale: float = 1.0,
+              mode: str = "softmax"):
+    """Expert choice from f32 router logits [T, N]: scores s = softmax (or,
+    by `mode`, sigmoid); the choice adds `correction` [N] f32 (None:
+    nothing); outputs form `groups` equal groups of neighbours scored by
+    their largest choice (sigmoid: the sum of their two largest), of which
+    the `keep` best stay eligible; the `top` largest eligible choices are
+    taken. Weights are s (without the correction), over their sum + 1e-20
+    with `renorm`, times scale. Mode "logits" chooses by the logits and
+    weighs by a softmax over the taken ones. Returns (indices [T, top]
+    int32, weights [T, top] f32, summed weight [T] f32 of the taken outputs
+    with index >= n_real)."""
+    if logits.is_cuda and logits.size(1) <= ROUTE_MAX and top <= 64 \
+            and groups <= 64:
+        topi, topw, w_id = _route_out(logits.size(0), top, logits.device)
         _K.moe_route(topi, topw, w_id, logits, _none(correction, logits),
-                     n_real, groups, keep, renorm, scale)
+                     n_real, groups, keep, renorm, scale, ROUTE_MODES[mode])
         return topi, topw, w_id
     return torch_ref.moe_route(logits, correction, top, n_real, groups, keep,
-                               renorm, scale)
+                               renorm, scale, mode)
+
+
+def moe_gate_route(x, gate, correction, top: int, n_real: int,
+                   groups: int = 1, keep: int = 1, renorm: bool = False,
+                   scale: float = 1.0, mode: str = "softmax"):
+    """moe_route of the logits x gate^T, formed in f32. One launch up to 64
+    outputs and 512 rows of bf16; a workgroup per row reads the whole router
+    (64 KB at 8 x 2048 f32), so that longer steps (32 rows: 5 us; 8192 rows:
+    270 MB to 540 MB through the caches) leave the product to the library."""
+    T = x.size(0)
+    if x.is_cuda and x.dtype == torch.bfloat16 and T <= 512 \
+            and gate.size(0) <= 64 and gate.is_contiguous() \
+            and gate.dtype in (torch.bfloat16, torch.float32) \
+            and x.stride(1) == 1 and x.stride(0) % 8 == 0 \
+            and x.size(1) % 8 == 0 and x.data_ptr() % 16 == 0 \
+            and gate.data_ptr() % 16 == 0:
+        topi, topw, w_id = _route_out(T, top, x.device)
+        _K.moe_gate_route(topi, topw, w_id, x, gate, _none(correction, x),
+                          n_real, groups, keep, renorm, scale,
+                          ROUTE_MODES[mode])
+        return topi, topw, w_id
+    logits = torch.nn.functional.linear(x.to(gate.dtype), gate).float()
+    return moe_route(logits, correction, top, n_real, groups, keep, renorm,
+                     scale, mode)
+
+
+def moe_plan(topi, topw, n: int):
+    """moe_sort, and the sorted row of every pair ([TK] int32)."""
+    if topi.is_cuda and n <= ROUTE_MAX:
+        TK, dev = topi.numel(), topi.device
+        tok = torch.empty(TK, dtype=torch.int32, device=dev)
+        pos = torch.empty(TK, dtype=torch.int32, device=dev)
+        gates = torch.empty(TK, dtype=torch.float32, device=dev)
+        offsets = torch.empty(n + 1, dtype=torch.int32, device=dev)
+        _K.moe_sort(tok, gates, offsets, pos, topi, topw)
+        return tok, gates, offsets, pos
+    return torch_ref.moe_plan(topi, topw, n)
 
 
 def moe_sort(topi, topw, n: int):
-    """(token, expert) pairs ordered by expert: (token of each sorted row
-    [TK] int32, its weight [TK] f32, exclusive offsets [n + 1] int32)."""
-    if topi.is_cuda:
-        TK, dev = topi.numel(), topi.device
-        tok = torch.empty(TK, dtype=torch.int32, device=dev)
-        gates = torch.empty(TK, dtype=torch.float32, device=dev)
-        offsets = torch.empty(n + 1, dtype=torch.int32, device=dev)
-        _K.moe_sort(tok, gates, offsets, topi, topw)
-        return tok, gates, offsets
-    return torch_ref.moe_sort(topi, topw, n)
+    """(token, expert) pairs ordered by expert, stable: (token of each
+    sorted row [TK] int32, its weight [TK] f32, exclusive offsets [n + 1]
+    int32)."""
+    return moe_plan(topi, topw, n)[:3]
 
 
 def w4a16_gemv(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor,

@@ -1,17 +1,32 @@
 // Expert choice for routed feed-forwards, in two launches.
 //
-//   moe_route: one wave per token. s = softmax(logits); choice = s +
-//     correction (none given: s); the outputs form `groups` equal groups of neighbours, a
-//     group scores its largest choice, only the `keep` best groups stay
-//     eligible; the `top` largest eligible choices are taken (ties: lower
-//     index). Weights are the taken s (without the correction), divided by
-//     their sum + 1e-20 when `renorm`, times `scale`. Outputs with index >=
-//     n_real are identity experts: their weights are also summed per token.
-//   moe_sort: one workgroup. Counting sort of the (token, expert) pairs by
-//     expert: token and weight of every sorted row, exclusive offsets.
+//   moe_route: one wave per token, from f32 logits; moe_gate_route: one
+//     workgroup per token, which also forms the logits x W^T. Modes:
+//     SOFTMAX: s = softmax(logits), choice = s + correction (none given: s);
+//       a group of `groups` equal groups of neighbours scores its largest
+//       choice;
+//     SIGMOID: s = sigmoid(logits), choice alike; a group scores the sum of
+//       its two largest choices;
+//     LOGITS: the choice is the logit itself, the weights are a softmax over
+//       the taken logits.
+//     Only the `keep` best groups stay eligible; the `top` largest eligible
+//     choices are taken (ties: lower index). Weights are the taken s
+//     (without the correction), divided by their sum + 1e-20 when `renorm`,
+//     times `scale`. Outputs with index >= n_real are identity experts: their
+//     weights are also summed per token.
+//   moe_sort: one workgroup. Stable counting sort of the (token, expert)
+//     pairs by expert: token and weight of every sorted row, exclusive
+//     offsets, row of every pair. Ranks come from ballots over the distinct
+//     experts of 64 pairs, so the order does not depend on timing.
+//
+// A decode step's choice is launches and latency, not work: as torch ops
+// (product, cast, top-k, softmax, sort, gathers, scatter, scan) it was about
+// 25 launches, 130 us of a layer's 240 at 32 tokens and 8 experts; these
+// two take 5 and 5 us there.
 //
 // An output's place in the row lives in lane e % 64, register e / 64.
 #include "mix_common.h"
+#include "skinny.h"
 #include <type_traits>
 
 namespace kaito {
@@ -30,17 +45,23 @@ KAITO_DEV void wave_argmax(float& v, int& i) {
   }
 }
 
-template <int NPL>
-__global__ __launch_bounds__(256) void moe_route_kernel(
-    int* __restrict__ topi, float* __restrict__ topw,
-    float* __restrict__ w_id, const float* __restrict__ logits,
-    const float* __restrict__ correction, const int T, const int N,
-    const int n_real, const int top, const int groups, const int keep,
-    const bool renorm, const float scale) {
-  const int lane = threadIdx.x & 63;
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (t >= T) return;                       // whole waves; no barriers below
-  const float* row = logits + (int64_t)t * N;
+enum Mode { SOFTMAX = 0, SIGMOID = 1, LOGITS = 2 };
+
+struct RouteArgs {
+  int* topi;                        // [T, top]
+  float* topw;                      // [T, top]
+  float* w_id;                      // [T]
+  const float* correction;          // [N] or nullptr
+  int T, N, n_real, top, groups, keep;
+  bool renorm;
+  float scale;
+};
+
+// one wave: the choice of token t from its logits (row: N floats)
+template <int NPL, int MODE>
+KAITO_DEV void route_row(const RouteArgs& a, const float* row, const int64_t t,
+                         const int lane) {
+  const int N = a.N;
   float s[NPL], ch[NPL];
   float mx = -INFINITY;
 #pragma unroll
@@ -49,35 +70,66 @@ __global__ __launch_bounds__(256) void moe_route_kernel(
     s[r] = e < N ? row[e] : -INFINITY;
     mx = fmaxf(mx, s[r]);
   }
-  mx = wave_reduce_max(mx);
-  float sum = 0.f;
+  if constexpr (MODE == SIGMOID) {
 #pragma unroll
-  for (int r = 0; r < NPL; r++) {
-    s[r] = r * 64 + lane < N ? expf(s[r] - mx) : 0.f;
-    sum += s[r];
-  }
-  sum = wave_reduce_sum(sum);
+    for (int r = 0; r < NPL; r++) {
+      const int e = r * 64 + lane;
+      s[r] = sigmoid_f(s[r]);
+      ch[r] = e < N ? s[r] + (a.correction ? a.correction[e] : 0.f)
+                    : -INFINITY;
+    }
+  } else {
+    mx = wave_reduce_max(mx);
+    float sum = 0.f;
 #pragma unroll
-  for (int r = 0; r < NPL; r++) {
-    const int e = r * 64 + lane;
-    s[r] = s[r] / sum;
-    ch[r] = e < N ? s[r] + (correction ? correction[e] : 0.f) : -INFINITY;
-  }
-  if (groups > 1) {
-    const int n = N / groups;
-    float mine = -INFINITY;                 // lane g: group g's score
-    for (int g = 0; g < groups; g++) {
-      float m = -INFINITY;
+    for (int r = 0; r < NPL; r++) {
+      if constexpr (MODE == LOGITS) ch[r] = s[r];
+      s[r] = r * 64 + lane < N ? expf(s[r] - mx) : 0.f;
+      sum += s[r];
+    }
+    if constexpr (MODE == SOFTMAX) {
+      sum = wave_reduce_sum(sum);
 #pragma unroll
       for (int r = 0; r < NPL; r++) {
         const int e = r * 64 + lane;
-        if (e >= g * n && e < (g + 1) * n) m = fmaxf(m, ch[r]);
+        s[r] = s[r] / sum;
+        ch[r] = e < N ? s[r] + (a.correction ? a.correction[e] : 0.f)
+                      : -INFINITY;
       }
-      m = wave_reduce_max(m);
-      if (lane == g) mine = m;
+    }
+  }
+  if (a.groups > 1) {
+    const int n = N / a.groups;
+    float mine = -INFINITY;                 // lane g: group g's score
+    for (int g = 0; g < a.groups; g++) {
+      float m = -INFINITY;
+      int mi = N;
+#pragma unroll
+      for (int r = 0; r < NPL; r++) {
+        const int e = r * 64 + lane;
+        if (e >= g * n && e < (g + 1) * n && (ch[r] > m || mi == N)) {
+          m = ch[r];
+          mi = e;
+        }
+      }
+      float score;
+      if constexpr (MODE == SIGMOID) {
+        wave_argmax(m, mi);
+        score = m;
+        float m2 = -INFINITY;               // the second largest
+#pragma unroll
+        for (int r = 0; r < NPL; r++) {
+          const int e = r * 64 + lane;
+          if (e >= g * n && e < (g + 1) * n && e != mi) m2 = fmaxf(m2, ch[r]);
+        }
+        if (n > 1) score += wave_reduce_max(m2);
+      } else {
+        score = wave_reduce_max(m);
+      }
+      if (lane == g) mine = score;
     }
     unsigned long long kept = 0;
-    for (int k = 0; k < keep; k++) {
+    for (int k = 0; k < a.keep; k++) {
       float v = mine;
       int i = lane;
       wave_argmax(v, i);
@@ -92,7 +144,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(
   }
   float wsum = 0.f, mine = 0.f;             // lane k: k-th taken weight
   int mine_i = 0;
-  for (int k = 0; k < top; k++) {
+  for (int k = 0; k < a.top; k++) {
     float v = -INFINITY;
     int i = min(lane, N - 1);
 #pragma unroll
@@ -109,104 +161,277 @@ __global__ __launch_bounds__(256) void moe_route_kernel(
     wsum += sv;
     if (lane == k) { mine = sv; mine_i = i; }
   }
-  const float f = renorm ? scale / (wsum + 1e-20f) : scale;
-  mine *= f;
-  if (lane < top) {
-    topi[(int64_t)t * top + lane] = mine_i;
-    topw[(int64_t)t * top + lane] = mine;
+  if constexpr (MODE == LOGITS)
+    mine = mine / wsum * a.scale;
+  else
+    mine *= a.renorm ? a.scale / (wsum + 1e-20f) : a.scale;
+  if (lane < a.top) {
+    a.topi[t * a.top + lane] = mine_i;
+    a.topw[t * a.top + lane] = mine;
   }
-  const float idw = wave_reduce_sum(lane < top && mine_i >= n_real ? mine
-                                                                   : 0.f);
-  if (lane == 0) w_id[t] = idw;
+  const float idw = wave_reduce_sum(lane < a.top && mine_i >= a.n_real ? mine
+                                                                       : 0.f);
+  if (lane == 0) a.w_id[t] = idw;
+}
+
+template <int NPL, int MODE>
+__global__ __launch_bounds__(256) void moe_route_kernel(
+    const RouteArgs a, const float* __restrict__ logits) {
+  const int64_t t = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (t >= a.T) return;                     // whole waves; no barriers below
+  route_row<NPL, MODE>(a, logits + t * a.N, t, threadIdx.x & 63);
+}
+
+constexpr int GATE_MAX = 64;         // experts whose logits a workgroup forms
+
+KAITO_DEV float dot_gate(const skinny::hbf16x8 x, const short* w, float c) {
+  return skinny::dot8(x, skinny::load_x(w), c);
+}
+KAITO_DEV float dot_gate(const skinny::hbf16x8 x, const float* w, float c) {
+  const float4_t a = *reinterpret_cast<const float4_t*>(w);
+  const float4_t b = *reinterpret_cast<const float4_t*>(w + 4);
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    c = fmaf((float)x[i], a[i], c);
+    c = fmaf((float)x[i + 4], b[i], c);
+  }
+  return c;
+}
+
+// W: the router's element (bf16 or f32); H is a multiple of 8
+template <int MODE, typename W>
+__global__ __launch_bounds__(256) void moe_gate_route_kernel(
+    const RouteArgs a, const short* __restrict__ x, const int64_t x_stride,
+    const W* __restrict__ w, const int H) {
+  __shared__ float part[4][GATE_MAX];
+  const int64_t t = blockIdx.x;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const short* xr = x + t * x_stride;
+  for (int e0 = 0; e0 < a.N; e0 += 8) {
+    float acc[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) acc[i] = 0.f;
+    for (int k = threadIdx.x * 8; k < H; k += 2048) {
+      const skinny::hbf16x8 xv = skinny::load_x(xr + k);
+#pragma unroll
+      for (int i = 0; i < 8; i++)
+        acc[i] = dot_gate(xv, w + (int64_t)min(e0 + i, a.N - 1) * H + k,
+                          acc[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      acc[i] = wave_reduce_sum(acc[i]);
+      if (lane == 0 && e0 + i < a.N) part[wave][e0 + i] = acc[i];
+    }
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  if (lane < a.N)
+    part[0][lane] += part[1][lane] + part[2][lane] + part[3][lane];
+  __builtin_amdgcn_wave_barrier();
+  route_row<1, MODE>(a, part[0], t, lane);
+}
+
+// Pairs are cut into one contiguous run per wave. cnt[w][e]: first the pairs
+// of expert e in wave w's run, then the next row of such a pair.
+template <typename F>
+KAITO_DEV void each_expert(const int e, const F& f) {
+  unsigned long long todo = __ballot(e >= 0);
+  while (todo) {
+    const int src = __builtin_ctzll(todo);
+    const int ev = __builtin_amdgcn_readlane(e, src);
+    const unsigned long long same = __ballot(e == ev);
+    f(ev, same, src);
+    todo &= ~same;
+  }
 }
 
 __global__ __launch_bounds__(1024) void moe_sort_kernel(
     int* __restrict__ sorted_tok, float* __restrict__ gates,
-    int* __restrict__ offsets, const int* __restrict__ topi,
-    const float* __restrict__ topw, const int TK, const int top,
-    const int N) {
-  __shared__ int scan[ROUTE_MAX];
-  const int tid = threadIdx.x;
-  scan[tid] = 0;
+    int* __restrict__ offsets, int* __restrict__ pos,
+    const int* __restrict__ topi, const float* __restrict__ topw,
+    const int TK, const int top, const int N) {
+  extern __shared__ int cnt[];              // [waves][N]
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int nw = blockDim.x >> 6;
+  const int per = (TK + nw * 64 - 1) / (nw * 64) * 64;
+  const int first = min(TK, wave * per), last = min(TK, first + per);
+  int* mine = cnt + wave * N;
+  for (int i = tid; i < nw * N; i += blockDim.x) cnt[i] = 0;
   __syncthreads();
-  for (int i = tid; i < TK; i += 1024) atomicAdd(&scan[topi[i]], 1);
-  __syncthreads();
-  const int count = scan[tid];
-  for (int off = 1; off < N; off <<= 1) {   // inclusive scan
-    const int add = tid >= off ? scan[tid - off] : 0;
-    __syncthreads();
-    scan[tid] += add;
-    __syncthreads();
+  for (int base = first; base < last; base += 64) {
+    const int i = base + lane;
+    each_expert(i < last ? topi[i] : -1,
+                [&](int e, unsigned long long same, int src) {
+      if (lane == src) mine[e] += __builtin_popcountll(same);
+    });
   }
-  if (tid == 0) offsets[0] = 0;
-  if (tid < N) offsets[tid + 1] = scan[tid];
   __syncthreads();
-  scan[tid] -= count;                       // next free row of the expert
+  if (wave == 0) {                          // exclusive scan over the experts
+    const int chunk = (N + 63) / 64;
+    const int e0 = min(N, lane * chunk), e1 = min(N, e0 + chunk);
+    int sum = 0;
+    for (int e = e0; e < e1; e++)
+      for (int w = 0; w < nw; w++) sum += cnt[w * N + e];
+    int scan = sum;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int add = __shfl_up(scan, off, 64);
+      if (lane >= off) scan += add;
+    }
+    int next = scan - sum;
+    for (int e = e0; e < e1; e++) {
+      offsets[e] = next;
+      for (int w = 0; w < nw; w++) {
+        const int c = cnt[w * N + e];
+        cnt[w * N + e] = next;
+        next += c;
+      }
+    }
+    if (lane == 63) offsets[N] = TK;
+  }
   __syncthreads();
-  for (int i = tid; i < TK; i += 1024) {
-    const int at = atomicAdd(&scan[topi[i]], 1);
-    sorted_tok[at] = i / top;
-    gates[at] = topw[i];
+  for (int base = first; base < last; base += 64) {
+    const int i = base + lane;
+    int at = 0;
+    const int e = i < last ? topi[i] : -1;
+    each_expert(e, [&](int ev, unsigned long long same, int src) {
+      if (e == ev)
+        at = mine[ev] +
+            __builtin_popcountll(same & ((1ull << lane) - 1));
+      __builtin_amdgcn_wave_barrier();
+      if (lane == src) mine[ev] += __builtin_popcountll(same);
+      __builtin_amdgcn_wave_barrier();
+    });
+    if (e >= 0) {
+      sorted_tok[at] = i / top;
+      gates[at] = topw[i];
+      pos[i] = at;
+    }
   }
 }
 
 }  // namespace
 
-void moe_route(at::Tensor topi, at::Tensor topw, at::Tensor w_id,
-               at::Tensor logits, at::Tensor correction, int64_t n_real,
-               int64_t groups, int64_t keep, bool renorm, double scale) {
-  KAITO_CHECK_F32(logits);
+// checks shared by both entries
+static RouteArgs route_args(const at::Tensor& topi, const at::Tensor& topw,
+                            const at::Tensor& w_id,
+                            const at::Tensor& correction, int64_t T, int64_t N,
+                            int64_t n_real, int64_t groups, int64_t keep,
+                            bool renorm, double scale, int64_t mode) {
   const bool corr = correction.numel() > 0;
   if (corr) KAITO_CHECK_F32(correction);
   KAITO_CHECK_I32(topi); KAITO_CHECK_F32(topw); KAITO_CHECK_F32(w_id);
-  TORCH_CHECK(logits.dim() == 2 && topi.dim() == 2);
-  const int T = logits.size(0), N = logits.size(1), top = topi.size(1);
+  TORCH_CHECK(topi.dim() == 2);
+  const int64_t top = topi.size(1);
   TORCH_CHECK(topi.size(0) == T && topw.sizes() == topi.sizes() &&
               w_id.numel() == T && (!corr || correction.numel() == N));
   TORCH_CHECK(N >= 1 && N <= ROUTE_MAX && top >= 1 && top <= 64 && top <= N);
   TORCH_CHECK(groups >= 1 && groups <= 64 && N % groups == 0 && keep >= 1 &&
               keep <= groups);
+  TORCH_CHECK(mode >= 0 && mode <= 2 && !(mode == LOGITS && corr));
+  RouteArgs a{};
+  a.topi = topi.data_ptr<int>();
+  a.topw = topw.data_ptr<float>();
+  a.w_id = w_id.data_ptr<float>();
+  a.correction = corr ? correction.data_ptr<float>() : nullptr;
+  a.T = (int)T; a.N = (int)N; a.n_real = (int)n_real; a.top = (int)top;
+  a.groups = (int)groups; a.keep = (int)keep;
+  a.renorm = renorm; a.scale = (float)scale;
+  return a;
+}
+
+template <typename F>
+static void with_mode(int64_t mode, const F& f) {
+  if (mode == SOFTMAX) f(std::integral_constant<int, SOFTMAX>{});
+  else if (mode == SIGMOID) f(std::integral_constant<int, SIGMOID>{});
+  else f(std::integral_constant<int, LOGITS>{});
+}
+
+void moe_route(at::Tensor topi, at::Tensor topw, at::Tensor w_id,
+               at::Tensor logits, at::Tensor correction, int64_t n_real,
+               int64_t groups, int64_t keep, bool renorm, double scale,
+               int64_t mode) {
+  KAITO_CHECK_F32(logits);
+  TORCH_CHECK(logits.dim() == 2);
+  const int T = logits.size(0), N = logits.size(1);
+  const RouteArgs a = route_args(topi, topw, w_id, correction, T, N, n_real,
+                                 groups, keep, renorm, scale, mode);
   if (T == 0) return;
   auto stream = at::hip::getCurrentHIPStream();
-  auto launch = [&](auto npl) {
-    hipLaunchKernelGGL((moe_route_kernel<decltype(npl)::value>),
-        dim3((T + 3) / 4), dim3(256), 0, stream, topi.data_ptr<int>(),
-        topw.data_ptr<float>(), w_id.data_ptr<float>(),
-        logits.data_ptr<float>(),
-        corr ? correction.data_ptr<float>() : nullptr, T, N,
-        (int)n_real, top, (int)groups, (int)keep, renorm, (float)scale);
-  };
-  if (N <= 64) launch(std::integral_constant<int, 1>{});
-  else if (N <= 128) launch(std::integral_constant<int, 2>{});
-  else if (N <= 256) launch(std::integral_constant<int, 4>{});
-  else launch(std::integral_constant<int, 16>{});
+  with_mode(mode, [&](auto md) {
+    auto launch = [&](auto npl) {
+      hipLaunchKernelGGL(
+          (moe_route_kernel<decltype(npl)::value, decltype(md)::value>),
+          dim3((T + 3) / 4), dim3(256), 0, stream, a,
+          logits.data_ptr<float>());
+    };
+    if (N <= 64) launch(std::integral_constant<int, 1>{});
+    else if (N <= 128) launch(std::integral_constant<int, 2>{});
+    else if (N <= 256) launch(std::integral_constant<int, 4>{});
+    else launch(std::integral_constant<int, 16>{});
+  });
+}
+
+void moe_gate_route(at::Tensor topi, at::Tensor topw, at::Tensor w_id,
+                    at::Tensor x, at::Tensor gate, at::Tensor correction,
+                    int64_t n_real, int64_t groups, int64_t keep, bool renorm,
+                    double scale, int64_t mode) {
+  TORCH_CHECK(x.is_cuda() && x.dtype() == at::kBFloat16 && x.dim() == 2 &&
+              x.stride(1) == 1 && x.stride(0) % 8 == 0 &&
+              (uintptr_t)x.data_ptr() % 16 == 0);
+  TORCH_CHECK(gate.is_cuda() && gate.dim() == 2 && gate.is_contiguous() &&
+              gate.size(1) == x.size(1) && x.size(1) % 8 == 0 &&
+              (uintptr_t)gate.data_ptr() % 16 == 0);
+  const int T = x.size(0), N = gate.size(0), H = x.size(1);
+  TORCH_CHECK(N <= GATE_MAX);
+  const RouteArgs a = route_args(topi, topw, w_id, correction, T, N, n_real,
+                                 groups, keep, renorm, scale, mode);
+  if (T == 0) return;
+  auto stream = at::hip::getCurrentHIPStream();
+  with_mode(mode, [&](auto md) {
+    if (gate.dtype() == at::kFloat) {
+      hipLaunchKernelGGL((moe_gate_route_kernel<decltype(md)::value, float>),
+          dim3(T), dim3(256), 0, stream, a, (const short*)x.data_ptr(),
+          x.stride(0), gate.data_ptr<float>(), H);
+    } else {
+      TORCH_CHECK(gate.dtype() == at::kBFloat16);
+      hipLaunchKernelGGL((moe_gate_route_kernel<decltype(md)::value, short>),
+          dim3(T), dim3(256), 0, stream, a, (const short*)x.data_ptr(),
+          x.stride(0), (const short*)gate.data_ptr(), H);
+    }
+  });
 }
 
 void moe_sort(at::Tensor sorted_tok, at::Tensor gates, at::Tensor offsets,
-              at::Tensor topi, at::Tensor topw) {
-  KAITO_CHECK_I32(topi); KAITO_CHECK_F32(topw);
+              at::Tensor pos, at::Tensor topi, at::Tensor topw) {
+  KAITO_CHECK_I32(topi); KAITO_CHECK_F32(topw); KAITO_CHECK_I32(pos);
   KAITO_CHECK_I32(sorted_tok); KAITO_CHECK_F32(gates);
   KAITO_CHECK_I32(offsets);
   TORCH_CHECK(topi.dim() == 2 && topw.sizes() == topi.sizes());
-  TORCH_CHECK(topi.numel() < (1ll << 31));
+  TORCH_CHECK(topi.numel() < (1ll << 31) - (1 << 20));
   const int TK = topi.numel(), top = topi.size(1);
   const int N = offsets.numel() - 1;
-  TORCH_CHECK(sorted_tok.numel() == TK && gates.numel() == TK && N >= 1 &&
-              N <= ROUTE_MAX);
+  TORCH_CHECK(sorted_tok.numel() == TK && gates.numel() == TK &&
+              pos.numel() == TK && N >= 1 && N <= ROUTE_MAX);
+  // waves by the number of 64-pair rounds; their counters fit 64 KB
+  const int nw = TK <= 256 ? 4 : 16;
   auto stream = at::hip::getCurrentHIPStream();
-  hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, stream,
-      sorted_tok.data_ptr<int>(), gates.data_ptr<float>(),
-      offsets.data_ptr<int>(), topi.data_ptr<int>(), topw.data_ptr<float>(),
-      TK, top, N);
+  hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(nw * 64),
+      (size_t)nw * N * 4, stream, sorted_tok.data_ptr<int>(),
+      gates.data_ptr<float>(), offsets.data_ptr<int>(), pos.data_ptr<int>(),
+      topi.data_ptr<int>(), topw.data_ptr<float>(), TK, top, N);
 }
 
 }  // namespace kaito
 
 TORCH_LIBRARY_FRAGMENT(kaito, m) {
-  m.def("moe_route(Tensor(a!) topi, Tensor(b!) topw, Tensor(c!) w_id, Tensor logits, Tensor correction, int n_real, int groups, int keep, bool renorm, float scale) -> ()");
-  m.def("moe_sort(Tensor(a!) sorted_tok, Tensor(b!) gates, Tensor(c!) offsets, Tensor topi, Tensor topw) -> ()");
+  m.def("moe_route(Tensor(a!) topi, Tensor(b!) topw, Tensor(c!) w_id, Tensor logits, Tensor correction, int n_real, int groups, int keep, bool renorm, float scale, int mode) -> ()");
+  m.def("moe_gate_route(Tensor(a!) topi, Tensor(b!) topw, Tensor(c!) w_id, Tensor x, Tensor gate, Tensor correction, int n_real, int groups, int keep, bool renorm, float scale, int mode) -> ()");
+  m.def("moe_sort(Tensor(a!) sorted_tok, Tensor(b!) gates, Tensor(c!) offsets, Tensor(d!) pos, Tensor topi, Tensor topw) -> ()");
 }
 TORCH_LIBRARY_IMPL(kaito, CUDA, m) {
   m.impl("moe_route", &kaito::moe_route);
+  m.impl("moe_gate_route", &kaito::moe_gate_route);
   m.impl("moe_sort", &kaito::moe_sort);
 }

@@ -796,37 +796,51 @@ def hgrn2_scan(q, v, f_pre, lower, norm_w, state, cu_seqlens, state_slots,
 
 
 def moe_route(logits, correction, top: int, n_real: int, groups: int,
-              keep: int, renorm: bool, scale: float):
-    """Softmax scores; choice by score + correction among the `keep` groups
-    with the largest choice; weights are the scores. Returns (indices
-    [T, top] int32, weights [T, top] f32, weight [T] on outputs >=
-    n_real)."""
+              keep: int, renorm: bool, scale: float, mode: str = "softmax"):
+    """Softmax or sigmoid scores; choice by score + correction among the
+    `keep` groups with the largest choice (sigmoid: sum of the two largest);
+    weights are the scores. "logits": choice by logit, weights a softmax
+    over the taken ones. Returns (indices [T, top] int32, weights [T, top]
+    f32, weight [T] on outputs >= n_real)."""
     T, N = logits.shape
-    s = torch.softmax(logits.float(), -1)
-    choice = s if correction is None else s + correction.float()
+    z = logits.float()
+    if mode == "logits":
+        s = choice = z
+    else:
+        s = torch.softmax(z, -1) if mode == "softmax" else torch.sigmoid(z)
+        choice = s if correction is None else s + correction.float()
     if groups > 1:
-        best = choice.view(T, groups, -1).amax(-1).topk(keep, -1)[1]
+        by_group = choice.view(T, groups, -1)
+        score = by_group.topk(min(2, by_group.size(-1)), -1)[0].sum(-1) \
+            if mode == "sigmoid" else by_group.amax(-1)
+        best = score.topk(keep, -1)[1]
         ok = torch.zeros(T, groups, dtype=torch.bool, device=logits.device)
         ok.scatter_(1, best, True)
         choice = choice.masked_fill(
             ~ok.repeat_interleave(N // groups, 1), float("-inf"))
     topi = choice.topk(top, -1)[1]
     w = s.gather(1, topi)
-    if renorm:
+    if mode == "logits":
+        w = torch.softmax(w, -1)
+    elif renorm:
         w = w / (w.sum(-1, keepdim=True) + 1e-20)
     w = w * scale
     return topi.to(torch.int32), w, (w * (topi >= n_real)).sum(-1)
 
 
-def moe_sort(topi, topw, n: int):
+def moe_plan(topi, topw, n: int):
     """Stable sort of the (token, expert) pairs by expert: (token, weight,
-    exclusive offsets [n + 1])."""
+    exclusive offsets [n + 1], sorted row of every pair)."""
     flat = topi.reshape(-1).long()
     order = torch.argsort(flat, stable=True)
     offsets = torch.zeros(n + 1, dtype=torch.int32, device=topi.device)
-    offsets[1:] = torch.cumsum(torch.bincount(flat, minlength=n), 0)
+    counts = torch.zeros(n, dtype=torch.long, device=topi.device)
+    counts.scatter_add_(0, flat, torch.ones_like(flat))
+    offsets[1:] = torch.cumsum(counts, 0)
+    pos = torch.empty_like(order)
+    pos[order] = torch.arange(order.numel(), device=topi.device)
     return ((order // topi.size(1)).to(torch.int32),
-            topw.reshape(-1)[order].float(), offsets)
+            topw.reshape(-1)[order].float(), offsets, pos.to(torch.int32))
 
 
 def _stream_norm(u, w, eps: float, out_dtype):
