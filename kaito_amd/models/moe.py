@@ -5,8 +5,9 @@ catalog (gpt-oss-120b / Qwen MoE presets in
 supported_models.yaml).
 
 Round 2: the GPU path is FUSED and host-sync-free — tokens are sorted by
-expert on the device and two HIP grouped-GEMM kernels (ops/csrc/moe.hip)
-consume (sorted_ids, offsets) directly: gather→gate/up GEMM→silu·mul,
+expert on the device and two HIP grouped-GEMM kernels (ops/csrc/moe.hip for
+decode-sized steps, moe_gemm.hip for prompts) consume (sorted_ids, offsets)
+directly: gather→gate/up GEMM→silu·mul,
 then down GEMM→weighted scatter-add. Worst-case tile grids make every
 shape static, so MoE decode steps capture into hipGraphs (the round-1
 per-expert torch loop read expert counts on the host each layer, forcing
@@ -156,16 +157,30 @@ class MoEMLP(nn.Module):
         return ops.moe_sort(topi, topw, self.n_route) \
             + (w_id if self.n_identity else None,)
 
-    # fused kernels win at decode-sized batches (weight-streaming
-    # bound, graph-capturable); per-expert hipBLASLt GEMMs win at
-    # prefill sizes (compute-bound, Tensile ~2x our 2-barrier tile —
-    # tools/bench_moe_kernels.py: TK=16384 fused 5.8ms vs loop 3.0ms).
-    # Prefill steps run eagerly, so the loop's host-side segment reads
-    # are harmless there. KAITO_MOE_FUSED_MAX overrides (high-top-k MoE
-    # like deepseek k=6 crosses TK=4096 at decode bs>682, where losing
-    # hipGraph capture costs more than the tile-efficiency gap).
+    # Pairs up to which the weight-streaming kernels run, beyond it the tiled
+    # grouped GEMMs: 64 rows per expert, where 8 experts of 2048 x 2048 take
+    # 81 us tiled and 93 streamed, 8 of 4096 x 14336 741 and 998, 64 of 2048 x
+    # 1408 (48 rows) still 284 and 260. KAITO_MOE_FUSED_MAX overrides.
     import os as _os
-    FUSED_MAX_TOKENS = int(_os.environ.get("KAITO_MOE_FUSED_MAX", "4096"))
+    _most = _os.environ.get("KAITO_MOE_FUSED_MAX")
+    FUSED_MAX_TOKENS = None if _most is None else int(_most)
+
+    def _kernels_for(self, x: torch.Tensor) -> str:
+        """"streamed", "tiled" (both free of host reads) or "loop": one
+        library GEMM per expert, for f32, odd widths, and where an expert's
+        rows and width keep the library's tiles full (1024 rows or more of
+        4096 x 14336: 5.68 ms a step of 8192 tokens against 5.99 tiled)."""
+        E, H, TK = self.num_experts, x.size(1), x.size(0) * self.top_k
+        if not (x.is_cuda and x.dtype == torch.bfloat16 and H % 64 == 0
+                and self.ie_local % 64 == 0):
+            return "loop"
+        most = self.FUSED_MAX_TOKENS
+        if TK <= (64 * E if most is None else most):
+            return "streamed"
+        if TK >= 1024 * E and H >= 4096 and self.ie_local >= 4096 \
+                and not torch.cuda.is_current_stream_capturing():
+            return "loop"
+        return "tiled"
 
     def forward(self, x: torch.Tensor, keep_f32: bool = False,
                 split_shared: bool = False):
@@ -173,35 +188,66 @@ class MoEMLP(nn.Module):
         split_shared: returns (routed sum, the shared expert's output or
         None) for a caller that adds them itself."""
         T, H = x.shape
-        sorted_tok, gates, offsets, w_id = self._route(x)
-        # the routed sum starts from the identity experts' share
-        out32 = torch.zeros(T, H, dtype=torch.float32, device=x.device) \
-            if w_id is None else x * w_id[:, None]
-        fused_shapes = (x.is_cuda and x.dtype == torch.bfloat16
-                        and H % 64 == 0 and self.ie_local % 64 == 0)
-        # under hipGraph capture the fused kernels are mandatory (the
-        # per-expert loop reads segment sizes on the host): deepseek k=6
-        # crosses TK=4096 at decode bs>682 and measured 30.9k vs timeout
-        # at bs=768 (profiles/r02_perf_notes.md)
-        if fused_shapes and (T * self.top_k <= self.FUSED_MAX_TOKENS
-                             or torch.cuda.is_current_stream_capturing()):
-            self._forward_fused(x, sorted_tok, gates, offsets, out32)
-        else:
-            self._forward_loop(x, sorted_tok, gates, offsets, out32)
-        out = out32 if keep_f32 else out32.to(x.dtype)
+        topi, topw, w_id = self._choose(x)
+        # identity outputs sort behind every expert's rows
+        sorted_tok, gates, offsets, pos = ops.moe_plan(topi, topw,
+                                                       self.n_route)
+        if not self.n_identity:
+            w_id = None
         shared = None
         if self.w_shared_gate_up is not None:   # deepseek shared experts
-            h1 = ops.linear(x, self.w_shared_gate_up)
-            shared = ops.linear(
-                ops.silu_and_mul(h1) if self.gated else ops.relu2(h1),
-                self.w_shared_down)
+            h1 = ops.linear_swiglu(x, self.w_shared_gate_up) if self.gated \
+                else ops.relu2(ops.linear(x, self.w_shared_gate_up))
+            shared = ops.linear(h1, self.w_shared_down)
+        added = None if split_shared else shared
+        kernels = self._kernels_for(x)
+        if kernels == "tiled":
+            out = self._forward_grouped(
+                x.contiguous(), topi, topw, w_id, sorted_tok, offsets, pos,
+                added, keep_f32)
+            added = None
+        else:
+            out = self._routed_start(x, w_id)
+            run = self._forward_fused if kernels == "streamed" \
+                else self._forward_loop
+            run(x, sorted_tok, gates, offsets, out)
+            out = out if keep_f32 else out.to(x.dtype)
         if split_shared:
             assert get_state().tp_size == 1
             return out, shared
-        if shared is not None:
-            out = out + shared
+        if added is not None:
+            out = out + added
         if get_state().tp_size > 1:
             out = tp_all_reduce(out)
+        return out
+
+    @staticmethod
+    def _routed_start(x, w_id):
+        """The routed sum starts from the identity experts' share."""
+        return torch.zeros(x.shape, dtype=torch.float32, device=x.device) \
+            if w_id is None else x * w_id[:, None]
+
+    def _forward_grouped(self, x, topi, topw, w_id, sorted_tok, offsets, pos,
+                         shared, keep_f32):
+        """Tiled grouped GEMMs over the sorted rows, then one pass per token
+        that sums its experts (static shapes, no host read)."""
+        TK, H = topi.numel(), x.size(1)
+        act = torch.empty(TK, self.ie_local, dtype=x.dtype, device=x.device)
+        ops.moe_grouped_up(act, x, self.w_gate_up, sorted_tok, offsets,
+                           self.e_base, self.b_gate_up, self.act_mode,
+                           self.act_limit)
+        # rows keep f32 until their sum where they always did: in steps of
+        # up to 4096 pairs and in captured ones
+        y = torch.empty(TK, H, device=x.device, dtype=torch.float32
+                        if TK <= 4096
+                        or torch.cuda.is_current_stream_capturing()
+                        else x.dtype)
+        ops.moe_grouped_down(y, act, self.w_down, offsets, self.e_base,
+                             self.b_down)
+        out = torch.empty(x.shape, dtype=torch.float32 if keep_f32
+                          else x.dtype, device=x.device)
+        ops.moe_combine(out, y, pos, topi, topw, self.e_base, self.e_local,
+                        x, w_id, shared)
         return out
 
     def _forward_fused(self, x, sorted_tok, gates, offsets, out32):
@@ -222,8 +268,8 @@ class MoEMLP(nn.Module):
                              self.b_down)
 
     def _forward_loop(self, x, sorted_tok, gates, offsets, out):
-        """Per-expert torch GEMMs (CPU tests / odd shapes). Host sync on
-        the segment sizes — never used on the GPU hot path."""
+        """Per-expert torch GEMMs (_kernels_for). Host sync on the segment
+        sizes."""
         off = offsets.tolist()
         idx64 = sorted_tok.long()
         for le in range(self.e_local):

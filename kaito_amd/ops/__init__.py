@@ -28,7 +28,8 @@ for _g, _names in {
     "attn": ("paged_attention paged_attention_sp prefill_attention "
              "mla_prefill_attention context_attention mfma_tile_gemm paged_read_bw"),
     "mla": "mla_decode mla_cache_write",
-    "moe": "moe_gate_silu moe_down_scatter",
+    "moe": ("moe_gate_silu moe_down_scatter moe_grouped_up "
+            "moe_grouped_down moe_combine"),
     "route": "moe_route moe_gate_route moe_sort",
     "quant": "w4a16_gemv w4a16_dequant w4a16_gemm lora_shrink lora_expand",
     "comm": ("allreduce_rmsnorm one_shot_ar_rmsnorm ipc_handle ipc_open "
@@ -386,6 +387,28 @@ def moe_down_scatter(out: torch.Tensor, act: torch.Tensor,
 
 
 MOE_ROUTE_MAX = (1024, 64, 64)      # router outputs, chosen, groups
+
+
+def moe_grouped_up(act, x, w, sorted_ids, offsets, e_base: int, bias=None,
+                   act_mode: int = 0, act_limit: float = 7.0) -> None:
+    """moe_gate_silu for prompt-sized steps (GPU, bf16): `act` [TK, IE]
+    exactly, widths multiples of 64, every tile bound read on the device."""
+    _K.moe_grouped_up(act, x, w, sorted_ids, offsets, _none(bias, x),
+                      act_mode, e_base, act_limit)
+
+
+def moe_grouped_down(y, act, w, offsets, e_base: int, bias=None) -> None:
+    """y[s] = act[s] w[e]^T (+ bias) of the sorted rows (GPU, bf16; y bf16
+    or f32)."""
+    _K.moe_grouped_down(y, act, w, offsets, _none(bias, act), e_base)
+
+
+def moe_combine(out, y, pos, topi, topw, e_base: int, e_local: int, x=None,
+                w_id=None, shared=None) -> None:
+    """out[t] = sum over t's choices of topw * y[pos] (experts e_base ..
+    e_base + e_local) + w_id x + shared, summed in f32; out bf16 or f32."""
+    _K.moe_combine(out, y, pos, topi, topw, out if w_id is None else x,
+                   _none(w_id, y), _none(shared, y), e_base, e_local)
 
 
 ROUTE_MAX = 1024      # router outputs of the kernels; more run as torch ops

@@ -33,7 +33,7 @@ GROUPS: Dict[str, List[str]] = {
              "paged_attention_sp.hip", "prefill_attention.hip",
              "context_attention.hip", "diag.hip", "mfma_probe.hip"],
     "mla": ["bind_mla.cpp", "mla_attention.hip"],
-    "moe": ["bind_moe.cpp", "moe.hip"],
+    "moe": ["bind_moe.cpp", "moe.hip", "moe_gemm.hip"],
     # expert choice (softmax, correction, groups, top-k) and expert sort
     "route": ["moe_route.hip"],
     "quant": ["bind_quant.cpp", "w4a16.hip", "lora.hip"],

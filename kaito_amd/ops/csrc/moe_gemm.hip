@@ -1,0 +1,440 @@
+// Grouped GEMMs of prompt-sized MoE steps: rows sorted by expert, one launch
+// per projection, tile bounds from the device's offsets (no host read).
+//
+//   moe_grouped_up    act[s] = act(x[tok_s] Wg[e]^T, x[tok_s] Wu[e]^T)
+//   moe_grouped_down  y[s] = act[s] Wd[e]^T (+ bias), bf16 or f32
+//   moe_combine       out[t] = sum over t's pairs of weight * y[row], f32
+//                     sums in the order of the choice, plus identity and
+//                     shared experts
+//
+// A workgroup of 8 waves (2 over rows x 4 over weight rows) computes BM rows
+// x 256 weight rows (up: 128 gate rows beside their 128 up rows, 32 + 32 per
+// wave, so a lane holds both of a pair) in K steps of 64 on
+// v_mfma_f32_32x32x16_bf16, transposed (C^T = W X^T: a lane owns one token row
+// and 4 neighbouring outputs at a time, stored as 8 bytes). Both operands
+// arrive by 16-byte global_load_lds one K step ahead (two buffers, one
+// barrier per step; 16-byte chunk c of row r at c ^ (r & 7)). At BM = 256 a
+// step is 32 MFMA per wave, 2048 cycles of a SIMD's two waves, against 192 KB
+// of LDS reads (1536 cycles) and 64 KB of staging per CU.
+//
+// Tiles are numbered expert by expert, in blocks of 4 column tiles x all row
+// tiles, and every XCD takes one contiguous eighth of them: the 32 tiles in
+// flight behind one L2 share rows and weights. Measured on one MI355X, 8
+// experts of 2048 x 2048, top 2: 8192 tokens 347 + 200 + 17 us (790 and 690
+// TFLOP/s) where a library GEMM per expert with its gathers, casts and
+// index_add took 973 us behind a host read; 1024 tokens 141 us against 179
+// for the streaming kernels of moe.hip. 8 of 4096 x 14336: 990 TFLOP/s.
+#include "flash_prefill.h"
+#include <torch/library.h>
+#include <ATen/ATen.h>
+#include <ATen/hip/HIPContext.h>
+
+namespace kaito {
+
+namespace {
+
+using flash::f32x16;
+using flash::hbf16x8;
+using flash::lds_copy16;
+using flash::mfma32;
+
+constexpr int BK = 64;              // K step
+constexpr int BN = 256;             // weight rows per tile
+constexpr int NG = 4;               // column tiles that share row tiles
+
+struct GemmArgs {
+  short* out;                       // [TK, N]
+  float* out32;                     // the same in f32 (DOWN), or nullptr
+  const short* x;                   // up: [T, K]; down: [TK, K]
+  const short* w;                   // [E, rows, K]
+  const short* bias;                // [E, rows] or nullptr
+  const int* rows;                  // up: token of a sorted row; down: none
+  const int* offsets;               // [.., E + 1]
+  int e_base, E, N, K;
+  int act_mode;                     // 0 SwiGLU, 1 clamped, 2 squared relu
+  float limit;
+};
+
+enum Kind { UP_GATED, UP_PLAIN, DOWN };
+
+KAITO_DEV float silu_of(float v) { return v / (1.f + __expf(-v)); }
+
+// act_mode 1: min(g, limit) sigmoid(1.702 min(g, limit)) (clamp(u) + 1)
+KAITO_DEV float gated(int mode, float g, float u, float limit) {
+  if (mode == 1) {
+    g = fminf(g, limit);
+    u = fminf(fmaxf(u, -limit), limit);
+    return (u + 1.f) * (g / (1.f + __expf(-1.702f * g)));
+  }
+  return silu_of(g) * u;
+}
+
+template <int BM, int KIND>
+__global__ __launch_bounds__(512, 2) void moe_grouped_kernel(const GemmArgs a) {
+  constexpr int MT = BM / 64;       // 32-row tiles of a wave
+  constexpr int COLS = KIND == UP_GATED ? BN / 2 : BN;   // outputs per tile
+  constexpr int LX = BM * BK / 8 / 512, LW = BN * BK / 8 / 512;
+  __shared__ __attribute__((aligned(128))) short lds[2][(BM + BN) * BK];
+
+  const int lane = threadIdx.x & 63, lr = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 2, wn = wave & 3;
+  const int ntiles = (a.N + COLS - 1) / COLS;
+
+  // ---- this workgroup's tile: every wave scans the experts, 64 at a time
+  int total = 0;
+  for (int e0 = 0; e0 < a.E; e0 += 64) {
+    const int e = a.e_base + e0 + lane;
+    int n = e0 + lane < a.E
+        ? (a.offsets[e + 1] - a.offsets[e] + BM - 1) / BM : 0;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+    total += n;
+  }
+  total *= ntiles;
+  const int share = (total + 7) / 8;
+  const int in_share = blockIdx.x / 8;
+  int t = (blockIdx.x % 8) * share + in_share;
+  if (in_share >= share || t >= total) return;
+  int expert = -1, mtiles = 0, row0 = 0, row_end = 0;
+  for (int e0 = 0; e0 < a.E && expert < 0; e0 += 64) {
+    const int e = a.e_base + e0 + lane;
+    const int o0 = e0 + lane < a.E ? a.offsets[e] : 0;
+    const int o1 = e0 + lane < a.E ? a.offsets[e + 1] : 0;
+    const int n = (o1 - o0 + BM - 1) / BM;
+    int scan = n;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int add = __shfl_up(scan, off, 64);
+      if (lane >= off) scan += add;
+    }
+    const unsigned long long hit = __ballot(scan * ntiles > t);
+    if (hit) {
+      const int src = __builtin_ctzll(hit);
+      expert = a.e_base + e0 + src;
+      mtiles = __builtin_amdgcn_readlane(n, src);
+      t -= (__builtin_amdgcn_readlane(scan, src) - mtiles) * ntiles;
+      row0 = __builtin_amdgcn_readlane(o0, src);
+      row_end = __builtin_amdgcn_readlane(o1, src);
+    } else {
+      t -= __builtin_amdgcn_readlane(scan, 63) * ntiles;
+    }
+  }
+  // blocks of NG column tiles, column fastest
+  const int blk = t / (NG * mtiles);
+  const int wide = min(NG, ntiles - blk * NG);
+  const int in_blk = t - blk * NG * mtiles;
+  const int nt = blk * NG + in_blk % wide, mt0 = in_blk / wide;
+  const int m0 = row0 + mt0 * BM, n0 = nt * COLS;
+
+  // ---- staging slots: slot s (16 bytes) is row s / 8, place s % 8
+  const short* xs[LX];
+  const short* ws[LW];
+#pragma unroll
+  for (int j = 0; j < LX; j++) {
+    const int s = j * 512 + threadIdx.x, row = s / 8;
+    const int c = (s % 8) ^ (row & 7);
+    const int m = min(m0 + row, row_end - 1);
+    const int64_t src = KIND == DOWN ? m : a.rows[m];
+    xs[j] = a.x + src * a.K + c * 8;
+  }
+  const int wrows = KIND == UP_GATED ? 2 * a.N : a.N;
+  const short* we = a.w + (int64_t)expert * wrows * a.K;
+#pragma unroll
+  for (int j = 0; j < LW; j++) {
+    const int s = j * 512 + threadIdx.x, row = s / 8;
+    const int c = (s % 8) ^ (row & 7);
+    // gated: every 64 tile rows are 32 gate rows, then their up rows
+    const int n = KIND == UP_GATED
+        ? min(n0 + (row / 64) * 32 + row % 32, a.N - 1) +
+              (row % 64 >= 32 ? a.N : 0)
+        : min(n0 + row, a.N - 1);
+    ws[j] = we + (int64_t)n * a.K + c * 8;
+  }
+  auto stage = [&](const int k, short* buf) {
+#pragma unroll
+    for (int j = 0; j < LX; j++)
+      lds_copy16(xs[j] + k, buf + (j * 512 + wave * 64) * 8);
+#pragma unroll
+    for (int j = 0; j < LW; j++)
+      lds_copy16(ws[j] + k, buf + BM * BK + (j * 512 + wave * 64) * 8);
+  };
+
+  f32x16 acc[2][MT];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < MT; j++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
+
+  stage(0, lds[0]);
+  __syncthreads();
+  int cur = 0;
+  for (int k = 0; k < a.K; k += BK) {
+    if (k + BK < a.K) stage(k + BK, lds[cur ^ 1]);
+    const short* xb = lds[cur] + (wm * (BM / 2) + lr) * BK;
+    const short* wb = lds[cur] + BM * BK + (wn * 64 + lr) * BK;
+#pragma unroll
+    for (int kk = 0; kk < BK / 16; kk++) {
+      const int c = ((kk * 2 + h) ^ (lr & 7)) * 8;
+      hbf16x8 wf[2], xf[MT];
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+        wf[i] = *reinterpret_cast<const hbf16x8*>(wb + i * 32 * BK + c);
+#pragma unroll
+      for (int j = 0; j < MT; j++)
+        xf[j] = *reinterpret_cast<const hbf16x8*>(xb + j * 32 * BK + c);
+#pragma unroll
+      for (int j = 0; j < MT; j++)
+#pragma unroll
+        for (int i = 0; i < 2; i++) acc[i][j] = mfma32(wf[i], xf[j], acc[i][j]);
+    }
+    __syncthreads();
+    cur ^= 1;
+  }
+
+  // ---- outputs n = 8 b + 4 h + e of 32-row tile i, token row lr of tile j
+  const short* be = a.bias ? a.bias + (int64_t)expert * wrows : nullptr;
+#pragma unroll
+  for (int j = 0; j < MT; j++) {
+    const int m = m0 + wm * (BM / 2) + j * 32 + lr;
+    if (m >= row_end) continue;
+    short* orow = a.out + (int64_t)m * a.N;
+#pragma unroll
+    for (int i = 0; i < (KIND == UP_GATED ? 1 : 2); i++)
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        const int n = n0 + (KIND == UP_GATED ? wn * 32 : wn * 64 + i * 32) +
+            8 * b + 4 * h;
+        if (n >= a.N) continue;               // N is a multiple of 64
+        short4_t o;
+        float4_t o32;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          float v = acc[i][j][b * 4 + e];
+          if constexpr (KIND == UP_GATED) {
+            float u = acc[1][j][b * 4 + e];
+            if (be) {
+              v += bf16_to_f32(be[n + e]);
+              u += bf16_to_f32(be[a.N + n + e]);
+            }
+            v = gated(a.act_mode, v, u, a.limit);
+          } else if constexpr (KIND == UP_PLAIN) {
+            v = fmaxf(v, 0.f);
+            v *= v;
+          } else {
+            if (be) v += bf16_to_f32(be[n + e]);
+          }
+          o[e] = f32_to_bf16(v);
+          o32[e] = v;
+        }
+        if (KIND == DOWN && a.out32)
+          *reinterpret_cast<float4_t*>(a.out32 + (int64_t)m * a.N + n) = o32;
+        else
+          *reinterpret_cast<short4_t*>(orow + n) = o;
+      }
+  }
+}
+
+// one workgroup per token, 8 outputs per thread and pass
+template <typename O, typename Y>
+__global__ __launch_bounds__(256) void moe_combine_kernel(
+    O* __restrict__ out, const Y* __restrict__ y,
+    const int* __restrict__ pos, const int* __restrict__ topi,
+    const float* __restrict__ topw, const short* __restrict__ x,
+    const float* __restrict__ w_id, const short* __restrict__ shared,
+    const int K, const int H, const int e_lo, const int e_hi) {
+  const int64_t t = blockIdx.x;
+  for (int c = threadIdx.x * 8; c < H; c += 2048) {
+    float acc[8];
+    auto add = [&](const auto* p, const float w) {
+      if constexpr (sizeof(*p) == 4) {
+        const float4_t* v = reinterpret_cast<const float4_t*>(p + c);
+        const float4_t lo = v[0], hi = v[1];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          acc[e] += w * lo[e];
+          acc[e + 4] += w * hi[e];
+        }
+      } else {
+        const short8_t v = *reinterpret_cast<const short8_t*>(p + c);
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc[e] += w * bf16_to_f32(v[e]);
+      }
+    };
+#pragma unroll
+    for (int e = 0; e < 8; e++) acc[e] = 0.f;
+    if (w_id) add(x + t * H, w_id[t]);
+    for (int k = 0; k < K; k++) {
+      const int e = topi[t * K + k];
+      if (e >= e_lo && e < e_hi)              // experts of this rank
+        add(y + (int64_t)pos[t * K + k] * H, topw[t * K + k]);
+    }
+    if (shared) add(shared + t * H, 1.0f);
+    if constexpr (sizeof(O) == 4) {
+      float4_t* o = reinterpret_cast<float4_t*>(out + t * H + c);
+      o[0] = float4_t{acc[0], acc[1], acc[2], acc[3]};
+      o[1] = float4_t{acc[4], acc[5], acc[6], acc[7]};
+    } else {
+      short8_t o;
+#pragma unroll
+      for (int e = 0; e < 8; e++) o[e] = f32_to_bf16(acc[e]);
+      *reinterpret_cast<short8_t*>(out + t * H + c) = o;
+    }
+  }
+}
+
+template <int KIND>
+void launch_grouped(const GemmArgs& a, int64_t TK) {
+  constexpr int COLS = KIND == UP_GATED ? BN / 2 : BN;
+  const int64_t ntiles = (a.N + COLS - 1) / COLS;
+  auto stream = at::hip::getCurrentHIPStream();
+  auto launch = [&](auto bm) {
+    constexpr int BM = decltype(bm)::value;
+    // most row tiles that TK rows in E groups can make
+    const int64_t most = TK / BM + std::min<int64_t>(a.E, TK);
+    hipLaunchKernelGGL((moe_grouped_kernel<BM, KIND>),
+        dim3((most * ntiles + 7) / 8 * 8), dim3(512), 0, stream, a);
+  };
+  // half tiles where an expert's rows would leave most of a whole one empty
+  if (TK >= 192 * (int64_t)a.E) launch(std::integral_constant<int, 256>{});
+  else launch(std::integral_constant<int, 128>{});
+}
+
+void check16(const at::Tensor& t) {
+  TORCH_CHECK(t.is_cuda() && t.is_contiguous() &&
+              t.dtype() == at::kBFloat16 &&
+              (uintptr_t)t.data_ptr() % 16 == 0);
+}
+void check_int(const at::Tensor& t) {
+  TORCH_CHECK(t.is_cuda() && t.is_contiguous() && t.dtype() == at::kInt);
+}
+
+}  // namespace
+
+void moe_grouped_up(at::Tensor act, at::Tensor x, at::Tensor w,
+                    at::Tensor sorted_ids, at::Tensor offsets, at::Tensor bias,
+                    int64_t act_mode, int64_t e_base, double act_limit) {
+  check16(act); check16(x); check16(w);
+  check_int(sorted_ids); check_int(offsets);
+  const bool plain = act_mode == 2;
+  TORCH_CHECK(act.dim() == 2 && x.dim() == 2 && w.dim() == 3);
+  GemmArgs a{};
+  a.E = (int)w.size(0); a.N = (int)act.size(1); a.K = (int)x.size(1);
+  a.e_base = (int)e_base;
+  TORCH_CHECK(w.size(1) == (plain ? 1 : 2) * (int64_t)a.N &&
+              w.size(2) == a.K && a.K % BK == 0 && a.N % 64 == 0 && a.K > 0);
+  TORCH_CHECK(e_base >= 0 && offsets.numel() > e_base + a.E &&
+              sorted_ids.numel() == act.size(0));
+  TORCH_CHECK(act_mode >= 0 && act_mode <= 2);
+  if (bias.numel() > 0) {
+    check16(bias);
+    TORCH_CHECK(!plain && bias.numel() == (int64_t)a.E * 2 * a.N);
+    a.bias = (const short*)bias.data_ptr();
+  }
+  a.out = (short*)act.data_ptr();
+  a.x = (const short*)x.data_ptr();
+  // expert indices count from e_base in the offsets, from 0 in the weights
+  a.w = (const short*)w.data_ptr() - e_base * w.stride(0);
+  if (a.bias) a.bias -= e_base * 2 * a.N;
+  a.rows = sorted_ids.data_ptr<int>();
+  a.offsets = offsets.data_ptr<int>();
+  a.act_mode = (int)act_mode;
+  a.limit = (float)act_limit;
+  if (act.size(0) == 0 || a.E == 0 || a.N == 0) return;
+  if (plain) launch_grouped<UP_PLAIN>(a, act.size(0));
+  else launch_grouped<UP_GATED>(a, act.size(0));
+}
+
+void moe_grouped_down(at::Tensor y, at::Tensor act, at::Tensor w,
+                      at::Tensor offsets, at::Tensor bias, int64_t e_base) {
+  const bool wide = y.dtype() == at::kFloat;
+  if (wide) {
+    TORCH_CHECK(y.is_cuda() && y.is_contiguous() &&
+                (uintptr_t)y.data_ptr() % 16 == 0);
+  } else {
+    check16(y);
+  }
+  check16(act); check16(w); check_int(offsets);
+  TORCH_CHECK(y.dim() == 2 && act.dim() == 2 && w.dim() == 3 &&
+              y.size(0) == act.size(0));
+  GemmArgs a{};
+  a.E = (int)w.size(0); a.N = (int)y.size(1); a.K = (int)act.size(1);
+  a.e_base = (int)e_base;
+  TORCH_CHECK(w.size(1) == a.N && w.size(2) == a.K && a.K % BK == 0 &&
+              a.N % 64 == 0 && a.K > 0);
+  TORCH_CHECK(e_base >= 0 && offsets.numel() > e_base + a.E);
+  if (bias.numel() > 0) {
+    check16(bias);
+    TORCH_CHECK(bias.numel() == (int64_t)a.E * a.N);
+    a.bias = (const short*)bias.data_ptr() - e_base * a.N;
+  }
+  if (wide) a.out32 = y.data_ptr<float>();
+  else a.out = (short*)y.data_ptr();
+  a.x = (const short*)act.data_ptr();
+  a.w = (const short*)w.data_ptr() - e_base * w.stride(0);
+  a.offsets = offsets.data_ptr<int>();
+  if (y.size(0) == 0 || a.E == 0 || a.N == 0) return;
+  launch_grouped<DOWN>(a, y.size(0));
+}
+
+void moe_combine(at::Tensor out, at::Tensor y, at::Tensor pos, at::Tensor topi,
+                 at::Tensor topw, at::Tensor x, at::Tensor w_id,
+                 at::Tensor shared, int64_t e_base, int64_t e_local) {
+  const bool wide = y.dtype() == at::kFloat;
+  if (wide) {
+    TORCH_CHECK(y.is_cuda() && y.is_contiguous() &&
+                (uintptr_t)y.data_ptr() % 16 == 0);
+  } else {
+    check16(y);
+  }
+  check_int(pos); check_int(topi);
+  TORCH_CHECK(out.is_cuda() && out.is_contiguous() && out.dim() == 2 &&
+              (out.dtype() == at::kFloat || out.dtype() == at::kBFloat16) &&
+              (uintptr_t)out.data_ptr() % 16 == 0);
+  TORCH_CHECK(topw.is_cuda() && topw.is_contiguous() &&
+              topw.dtype() == at::kFloat && topi.dim() == 2 &&
+              topw.sizes() == topi.sizes() && pos.numel() == topi.numel());
+  const int64_t T = out.size(0), H = out.size(1), K = topi.size(1);
+  TORCH_CHECK(H % 8 == 0 && topi.size(0) == T && y.size(0) == T * K &&
+              y.size(1) == H);
+  const bool ids = w_id.numel() > 0, sh = shared.numel() > 0;
+  if (ids) {
+    check16(x);
+    TORCH_CHECK(x.size(0) == T && x.size(1) == H && w_id.numel() == T &&
+                w_id.dtype() == at::kFloat && w_id.is_contiguous());
+  }
+  if (sh) {
+    check16(shared);
+    TORCH_CHECK(shared.sizes() == out.sizes());
+  }
+  if (T == 0 || H == 0) return;
+#define MC_LAUNCH(O_, Y_)                                                     \
+  hipLaunchKernelGGL((moe_combine_kernel<O_, Y_>), dim3(T), dim3(256), 0,     \
+      at::hip::getCurrentHIPStream(), (O_*)out.data_ptr(),                    \
+      (const Y_*)y.data_ptr(), pos.data_ptr<int>(), topi.data_ptr<int>(),     \
+      topw.data_ptr<float>(), ids ? (const short*)x.data_ptr() : nullptr,     \
+      ids ? w_id.data_ptr<float>() : nullptr,                                 \
+      sh ? (const short*)shared.data_ptr() : nullptr, (int)K, (int)H,         \
+      (int)e_base, (int)(e_base + e_local))
+  if (out.dtype() == at::kFloat) {
+    if (wide) MC_LAUNCH(float, float); else MC_LAUNCH(float, short);
+  } else {
+    if (wide) MC_LAUNCH(short, float); else MC_LAUNCH(short, short);
+  }
+#undef MC_LAUNCH
+}
+
+}  // namespace kaito
+
+TORCH_LIBRARY_FRAGMENT(kaito, m) {
+  m.def("moe_grouped_up(Tensor(a!) act, Tensor x, Tensor w, Tensor sorted_ids, Tensor offsets, Tensor bias, int act_mode, int e_base, float act_limit) -> ()");
+  m.def("moe_grouped_down(Tensor(a!) y, Tensor act, Tensor w, Tensor offsets, Tensor bias, int e_base) -> ()");
+  m.def("moe_combine(Tensor(a!) out, Tensor y, Tensor pos, Tensor topi, Tensor topw, Tensor x, Tensor w_id, Tensor shared, int e_base, int e_local) -> ()");
+}
+TORCH_LIBRARY_IMPL(kaito, CUDA, m) {
+  m.impl("moe_grouped_up", &kaito::moe_grouped_up);
+  m.impl("moe_grouped_down", &kaito::moe_grouped_down);
+  m.impl("moe_combine", &kaito::moe_combine);
+}

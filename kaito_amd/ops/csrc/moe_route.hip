@@ -14,10 +14,12 @@
 //     (without the correction), divided by their sum + 1e-20 when `renorm`,
 //     times `scale`. Outputs with index >= n_real are identity experts: their
 //     weights are also summed per token.
-//   moe_sort: one workgroup. Stable counting sort of the (token, expert)
-//     pairs by expert: token and weight of every sorted row, exclusive
-//     offsets, row of every pair. Ranks come from ballots over the distinct
-//     experts of 64 pairs, so the order does not depend on timing.
+//   moe_sort: stable counting sort of the (token, expert) pairs by expert:
+//     token and weight of every sorted row, exclusive offsets, row of every
+//     pair. Ranks come from ballots over the distinct experts of 64 pairs,
+//     so the order does not depend on timing. One workgroup up to 2048
+//     pairs; beyond, one per 1024 pairs behind a counting launch (16384 pairs
+//     took 46 us in one workgroup).
 //
 // A decode step's choice is launches and latency, not work: as torch ops
 // (product, cast, top-k, softmax, sort, gathers, scatter, scan) it was about
@@ -246,16 +248,39 @@ KAITO_DEV void each_expert(const int e, const F& f) {
   }
 }
 
+constexpr int SORT_BLOCK = 1024;     // pairs of a workgroup when several sort
+
+// hist[b][e]: pairs of expert e in block b
+__global__ __launch_bounds__(1024) void moe_count_kernel(
+    int* __restrict__ hist, const int* __restrict__ topi, const int TK,
+    const int N) {
+  extern __shared__ int cnt[];              // [N]
+  const int tid = threadIdx.x, lane = tid & 63;
+  for (int i = tid; i < N; i += SORT_BLOCK) cnt[i] = 0;
+  __syncthreads();
+  const int i = blockIdx.x * SORT_BLOCK + tid;
+  each_expert(i < TK ? topi[i] : -1,
+              [&](int e, unsigned long long same, int src) {
+    if (lane == src) atomicAdd(&cnt[e], __builtin_popcountll(same));
+  });
+  __syncthreads();
+  for (int e = tid; e < N; e += SORT_BLOCK)
+    hist[(int64_t)blockIdx.x * N + e] = cnt[e];
+}
+
+// hist: counts of SORT_BLOCK pairs each, or nullptr for one workgroup
 __global__ __launch_bounds__(1024) void moe_sort_kernel(
     int* __restrict__ sorted_tok, float* __restrict__ gates,
     int* __restrict__ offsets, int* __restrict__ pos,
     const int* __restrict__ topi, const float* __restrict__ topw,
-    const int TK, const int top, const int N) {
+    const int* __restrict__ hist, const int TK, const int top, const int N) {
   extern __shared__ int cnt[];              // [waves][N]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nw = blockDim.x >> 6;
-  const int per = (TK + nw * 64 - 1) / (nw * 64) * 64;
-  const int first = min(TK, wave * per), last = min(TK, first + per);
+  const int begin = hist ? blockIdx.x * SORT_BLOCK : 0;
+  const int end = hist ? min(TK, begin + SORT_BLOCK) : TK;
+  const int per = (end - begin + nw * 64 - 1) / (nw * 64) * 64;
+  const int first = min(end, begin + wave * per), last = min(end, first + per);
   int* mine = cnt + wave * N;
   for (int i = tid; i < nw * N; i += blockDim.x) cnt[i] = 0;
   __syncthreads();
@@ -270,25 +295,37 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(
   if (wave == 0) {                          // exclusive scan over the experts
     const int chunk = (N + 63) / 64;
     const int e0 = min(N, lane * chunk), e1 = min(N, e0 + chunk);
+    auto all_of = [&](const int e) {
+      int n = 0;
+      if (hist)
+        for (unsigned b = 0; b < gridDim.x; b++) n += hist[(int64_t)b * N + e];
+      else
+        for (int w = 0; w < nw; w++) n += cnt[w * N + e];
+      return n;
+    };
     int sum = 0;
-    for (int e = e0; e < e1; e++)
-      for (int w = 0; w < nw; w++) sum += cnt[w * N + e];
+    for (int e = e0; e < e1; e++) sum += all_of(e);
     int scan = sum;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
       const int add = __shfl_up(scan, off, 64);
       if (lane >= off) scan += add;
     }
-    int next = scan - sum;
+    int start = scan - sum;
     for (int e = e0; e < e1; e++) {
-      offsets[e] = next;
+      if (blockIdx.x == 0) offsets[e] = start;
+      int next = start;
+      if (hist)                             // rows of the blocks before
+        for (unsigned b = 0; b < blockIdx.x; b++)
+          next += hist[(int64_t)b * N + e];
+      start += all_of(e);
       for (int w = 0; w < nw; w++) {
         const int c = cnt[w * N + e];
         cnt[w * N + e] = next;
         next += c;
       }
     }
-    if (lane == 63) offsets[N] = TK;
+    if (blockIdx.x == 0 && lane == 63) offsets[N] = TK;
   }
   __syncthreads();
   for (int base = first; base < last; base += 64) {
@@ -414,13 +451,22 @@ void moe_sort(at::Tensor sorted_tok, at::Tensor gates, at::Tensor offsets,
   const int N = offsets.numel() - 1;
   TORCH_CHECK(sorted_tok.numel() == TK && gates.numel() == TK &&
               pos.numel() == TK && N >= 1 && N <= ROUTE_MAX);
+  auto stream = at::hip::getCurrentHIPStream();
   // waves by the number of 64-pair rounds; their counters fit 64 KB
   const int nw = TK <= 256 ? 4 : 16;
-  auto stream = at::hip::getCurrentHIPStream();
-  hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(nw * 64),
+  const int blocks = TK <= 2048 ? 1 : (TK + SORT_BLOCK - 1) / SORT_BLOCK;
+  at::Tensor hist;
+  if (blocks > 1) {
+    hist = at::empty({blocks, N}, topi.options());
+    hipLaunchKernelGGL(moe_count_kernel, dim3(blocks), dim3(SORT_BLOCK),
+        (size_t)N * 4, stream, hist.data_ptr<int>(), topi.data_ptr<int>(), TK,
+        N);
+  }
+  hipLaunchKernelGGL(moe_sort_kernel, dim3(blocks), dim3(nw * 64),
       (size_t)nw * N * 4, stream, sorted_tok.data_ptr<int>(),
       gates.data_ptr<float>(), offsets.data_ptr<int>(), pos.data_ptr<int>(),
-      topi.data_ptr<int>(), topw.data_ptr<float>(), TK, top, N);
+      topi.data_ptr<int>(), topw.data_ptr<float>(),
+      blocks > 1 ? hist.data_ptr<int>() : nullptr, TK, top, N);
 }
 
 }  // namespace kaito

@@ -1,0 +1,96 @@
+"""Grouped GEMMs of prompt-sized MoE steps (ops/csrc/moe_gemm.hip): expert
+row counts around the 128- and 256-row tiles, empty experts, widths that end
+inside a 256-column tile, ranks that hold part of the experts, activations,
+biases, identity and shared experts. Activations and rows are bf16 between
+the products (2^-8 each, f32 sums)."""
+import pytest
+import torch
+
+from kaito_amd import ops
+
+DEV = "cuda"
+
+
+def _rand(*shape, std=1.0):
+    return (std * torch.randn(*shape, device=DEV)).to(torch.bfloat16)
+
+
+def _act(mode, h, n):
+    if mode == 2:
+        return h.relu().square()
+    g, u = h[:, :n], h[:, n:]
+    if mode == 1:
+        g, u = g.clamp(max=7.0), u.clamp(-7.0, 7.0)
+        return (u + 1) * g * torch.sigmoid(1.702 * g)
+    return g * torch.sigmoid(g) * u
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("counts,H,IE,mode,bias,part", [
+    ([1], 64, 64, 0, False, None),
+    ([127, 0, 129, 1], 128, 192, 0, True, None),
+    ([0, 128, 300, 0, 77], 192, 64, 2, False, None),
+    ([255, 257, 256], 128, 320, 1, True, None),
+    ([900, 12], 320, 128, 0, False, None),
+    ([64, 200, 3, 131], 128, 128, 0, False, (1, 2)),
+    ([5] * 70, 64, 128, 1, False, None),           # more experts than lanes
+])
+@pytest.mark.parametrize("f32", [False, True])
+def test_grouped_step(counts, H, IE, mode, bias, part, f32):
+    torch.manual_seed(sum(counts))
+    E, top = len(counts), 1
+    T = sum(counts)
+    lo, n = part or (0, E)
+    topi = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    topi = topi[torch.randperm(T)].to(DEV).int()[:, None]
+    topw = torch.rand(T, top, device=DEV) + 0.5
+    x, shared = _rand(T, H), _rand(T, H)
+    rows = 1 if mode == 2 else 2
+    wu = _rand(E, rows * IE, H, std=H ** -0.5)
+    wd = _rand(E, H, IE, std=IE ** -0.5)
+    bu = _rand(E, 2 * IE) if bias else None
+    bd = _rand(E, H) if bias else None
+    w_id = torch.rand(T, device=DEV)
+    tok, gates, off, pos = ops.moe_plan(topi, topw, E)
+    act = torch.full((T, IE), float("nan"), device=DEV).to(torch.bfloat16)
+    y = torch.full((T, H), float("nan"), device=DEV)
+    y = y if f32 else y.to(torch.bfloat16)
+    cut = slice(lo, lo + n)
+    ops.moe_grouped_up(act, x, wu[cut].contiguous(), tok, off, lo,
+                       bu[cut].contiguous() if bias else None, mode, 7.0)
+    ops.moe_grouped_down(y, act, wd[cut].contiguous(), off, lo,
+                         bd[cut].contiguous() if bias else None)
+    out = torch.empty(T, H, device=DEV, dtype=torch.float32 if f32
+                      else torch.bfloat16)
+    ops.moe_combine(out, y, pos, topi, topw, lo, n, x, w_id, shared)
+    ref = x.double() * w_id[:, None].double() + shared.double()
+    for e in range(lo, lo + n):
+        t = torch.nonzero(topi[:, 0] == e)[:, 0]
+        h = x[t].double() @ wu[e].double().T
+        if bias:
+            h = h + bu[e].double()
+        v = _act(mode, h, IE) @ wd[e].double().T
+        if bias:
+            v = v + bd[e].double()
+        ref[t] += v * topw[t].double()
+    assert torch.isfinite(out).all()
+    err = (out.double() - ref).abs()
+    rms = ref.square().mean().sqrt()
+    # act and y rounded once each, out once: a few 2^-9 of the row's size
+    assert err.max() <= 2.0 ** -5 * rms, err.max() / rms
+    assert err.square().mean().sqrt() <= 2.0 ** -7.5 * rms
+
+
+@pytest.mark.gpu
+def test_several_choices_sum():
+    torch.manual_seed(3)
+    T, H, K = 50, 2056, 6
+    y = _rand(T * K, H)
+    topi = torch.randint(0, 9, (T, K), device=DEV).int()
+    topw = torch.rand(T, K, device=DEV)
+    pos = torch.randperm(T * K, device=DEV).int()
+    out = torch.empty(T, H, device=DEV)
+    ops.moe_combine(out, y, pos, topi, topw, 2, 5)
+    live = ((topi >= 2) & (topi < 7)).double() * topw.double()
+    ref = (y[pos.long()].view(T, K, H).double() * live[..., None]).sum(1)
+    assert torch.allclose(out.double(), ref, atol=1e-5)
