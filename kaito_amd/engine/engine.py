@@ -559,7 +559,7 @@ class LLMEngine:
             seq = Sequence(seq_id, [], SamplingParams(max_tokens=0))
             self.seqs[seq_id] = seq
             self.scheduler.add(seq)
-        seq.prompt_token_ids.extend(int(t) for t in tokens)
+        seq.prompt_token_ids.extend(map(int, tokens))
         if seq.num_tokens > self.runner.max_model_len:
             raise ValueError(
                 f"request {seq_id} exceeds max_model_len="

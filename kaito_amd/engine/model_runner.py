@@ -14,6 +14,7 @@ import logging
 from pathlib import Path
 from typing import Dict, List, Optional, Tuple
 
+import numpy as np
 import torch
 
 # hipBLASLt algo selections tuned offline on MI355X (torch TunableOp);
@@ -177,11 +178,6 @@ class ModelRunner:
                     n_slots, n_slots * slot_bytes / (1 << 30))
         return n_blocks
 
-    # ------------------------------------------------------------- helpers
-    def _slot(self, seq: Sequence, pos: int) -> int:
-        bs = self.cfg.block_size
-        return seq.block_table[pos // bs] * bs + pos % bs
-
     # ------------------------------------------------------------- prefill
     @torch.no_grad()
     def execute_prefill(self, chunks, rows=None) -> torch.Tensor:
@@ -192,56 +188,74 @@ class ModelRunner:
         in chunk order (aligned with batch.sampling_seqs) — or, with
         `rows` (indices into the concatenated chunk rows), of exactly
         those rows."""
-        ids, pos, slots, cu = [], [], [], [0]
         fresh = (not self.stateful
                  and all(c.start == 0 and c.completes for c in chunks))
-        for c in chunks:
-            toks = c.seq.context_token_ids[c.start:c.start + c.length]
-            ids.extend(toks)
-            pos.extend(range(c.start, c.start + c.length))
-            slots.extend(self._slot(c.seq, p)
-                         for p in range(c.start, c.start + c.length))
-            cu.append(cu[-1] + c.length)
-        dev = self.device
-        input_ids = torch.tensor(ids, dtype=torch.long, device=dev)
-        positions = torch.tensor(pos, dtype=torch.long, device=dev)
-        kv_lens = None
-        block_tables = None
+        dev, bs = self.device, self.cfg.block_size
+        lens = np.array([c.length for c in chunks], dtype=np.int64)
+        starts = np.array([c.start for c in chunks], dtype=np.int64)
+        cu = np.concatenate([[0], np.cumsum(lens)])
+        T = int(cu[-1])
+        # everything the step's kernels read about its rows goes to the
+        # device in two copies: [ids | positions | slots | wanted rows] and
+        # the small per-chunk int32 arrays
+        last = [int(cu[i + 1]) - 1 for i, c in enumerate(chunks)
+                if c.completes] if rows is None else list(rows)
+        wide = np.empty(3 * T + len(last), dtype=np.int64)
+        ids, pos, slots = wide[:T], wide[T:2 * T], wide[2 * T:3 * T]
+        wide[3 * T:] = last
+        for i, c in enumerate(chunks):
+            a, b = cu[i], cu[i + 1]
+            ids[a:b] = c.seq.context_token_ids[c.start:c.start + c.length]
+            p = np.arange(c.start, c.start + c.length)
+            pos[a:b] = p
+            table = np.array(c.seq.block_table, dtype=np.int64)
+            slots[a:b] = table[p // bs] * bs + p % bs
+        wide = torch.from_numpy(wide).to(dev)
+        input_ids, positions, slot_mapping = (
+            wide[i * T:(i + 1) * T] for i in range(3))
+        narrow = {"cu": cu}
         if not fresh:
-            import numpy as np
             mb = max(len(c.seq.block_table) for c in chunks)
             flat = np.zeros((len(chunks), mb), dtype=np.int32)
             for i, c in enumerate(chunks):
                 flat[i, :len(c.seq.block_table)] = c.seq.block_table
-            block_tables = torch.from_numpy(flat).to(dev)
-            kv_lens = torch.tensor([c.start + c.length for c in chunks],
-                                   dtype=torch.int32, device=dev)
-        meta = AttnMetadata(
-            is_prefill=True,
-            slot_mapping=torch.tensor(slots, dtype=torch.long, device=dev),
-            cu_seqlens=torch.tensor(cu, dtype=torch.int32, device=dev),
-            max_seqlen=max(c.length for c in chunks),
-            block_tables=block_tables,
-            kv_lens=kv_lens)
+            narrow["block_tables"] = flat
+            narrow["kv_lens"] = starts + lens
         if self.stateful:
-            seq_of = []
-            for i, c in enumerate(chunks):
-                seq_of.extend([i] * c.length)
-            meta.state_slots = torch.tensor(
-                [c.seq.state_slot for c in chunks], dtype=torch.int32,
-                device=dev)
-            meta.seq_starts = torch.tensor(
-                [c.start for c in chunks], dtype=torch.int32, device=dev)
-            meta.token_seq = torch.tensor(seq_of, dtype=torch.int32,
-                                          device=dev)
-            meta.ctx_lens = [c.start + c.length for c in chunks]
-            meta.ctx_starts = [c.start for c in chunks]
-            if self.is_gpu and meta.max_seqlen >= 8:
-                # prompt portions: tile the chunks for the MFMA attention
-                # kernel (a step of single tokens keeps the decode kernel)
-                from .. import ops
-                meta.tile_seq, meta.tile_qbase = ops.build_query_tiles(
-                    [c.length for c in chunks], dev, meta.ctx_starts)
+            narrow["state_slots"] = [c.seq.state_slot for c in chunks]
+            narrow["seq_starts"] = starts
+            narrow["token_seq"] = np.repeat(np.arange(len(chunks)), lens)
+        max_seqlen = int(lens.max())
+        if self.is_gpu and (not self.stateful or max_seqlen >= 8):
+            # query tiles of the prompt attention (a stateful step of single
+            # tokens keeps the decode kernel)
+            from .. import ops
+            narrow["tile_seq"], narrow["tile_qbase"] = ops.query_tiles(
+                lens, starts)
+        narrow = {k: np.ascontiguousarray(v, dtype=np.int32)
+                  for k, v in narrow.items()}
+        # 16-byte aligned pieces of one buffer
+        at, places = 0, {}
+        for k, v in narrow.items():
+            places[k] = at
+            at += -(-v.size // 4) * 4
+        buf = np.zeros(at, dtype=np.int32)
+        for k, v in narrow.items():
+            buf[places[k]:places[k] + v.size] = v.reshape(-1)
+        buf = torch.from_numpy(buf).to(dev)
+        d = {k: buf[places[k]:places[k] + v.size].view(v.shape)
+             for k, v in narrow.items()}
+        meta = AttnMetadata(
+            is_prefill=True, slot_mapping=slot_mapping,
+            cu_seqlens=d["cu"], max_seqlen=max_seqlen,
+            block_tables=d.get("block_tables"), kv_lens=d.get("kv_lens"),
+            tile_seq=d.get("tile_seq"), tile_qbase=d.get("tile_qbase"))
+        if self.stateful:
+            meta.state_slots = d["state_slots"]
+            meta.seq_starts = d["seq_starts"]
+            meta.token_seq = d["token_seq"]
+            meta.ctx_lens = (starts + lens).tolist()
+            meta.ctx_starts = starts.tolist()
         if self.lora_manager is not None:
             tok_ids = []
             for c in chunks:
@@ -253,11 +267,9 @@ class ModelRunner:
             lora_mod.set_active(None, None)
         if hidden is None:
             return None  # intermediate PP stage
-        last = [cu[i + 1] - 1 for i, c in enumerate(chunks) if c.completes] \
-            if rows is None else list(rows)
         if not last:
             return hidden[:0]
-        return hidden[torch.tensor(last, device=dev)]
+        return hidden[wide[3 * T:]]
 
     # ------------------------------------------------------------- decode
     def _init_decode_buffers(self):
@@ -265,22 +277,24 @@ class ModelRunner:
         max_bs = max(max(cfg.graph_batch_sizes), cfg.max_num_seqs)
         mb = cfg.max_blocks_per_seq(self.max_model_len)
         dev = self.device
+        # the per-row inputs are rows of two blocks, so that a rebuilt batch
+        # arrives in one copy each
+        self._wide = torch.zeros(3, max_bs, dtype=torch.long, device=dev)
+        self._narrow = torch.zeros(4, max_bs, dtype=torch.int32, device=dev)
+        self._wide[2].fill_(-1)
+        self._narrow[1:3].fill_(-1)
         self._buf = {
-            "input_ids": torch.zeros(max_bs, dtype=torch.long, device=dev),
-            "positions": torch.zeros(max_bs, dtype=torch.long, device=dev),
-            "slot_mapping": torch.full((max_bs,), -1, dtype=torch.long, device=dev),
+            "input_ids": self._wide[0], "positions": self._wide[1],
+            "slot_mapping": self._wide[2],
+            "seq_lens": self._narrow[0], "lora_ids": self._narrow[1],
             "block_tables": torch.zeros(max_bs, mb, dtype=torch.int32, device=dev),
-            "seq_lens": torch.zeros(max_bs, dtype=torch.int32, device=dev),
-            "lora_ids": torch.full((max_bs,), -1, dtype=torch.int32, device=dev),
         }
         if self.stateful:
             # decode = chunks of one token: static layout tensors, plus
             # the per-sequence slot (-1 pads) and start position
             self._buf.update({
-                "state_slots": torch.full((max_bs,), -1, dtype=torch.int32,
-                                          device=dev),
-                "seq_starts": torch.zeros(max_bs, dtype=torch.int32,
-                                          device=dev),
+                "state_slots": self._narrow[2],
+                "seq_starts": self._narrow[3],
                 "cu_seqlens": torch.arange(max_bs + 1, dtype=torch.int32,
                                            device=dev),
                 "token_seq": torch.arange(max_bs, dtype=torch.int32,
@@ -484,57 +498,47 @@ class ModelRunner:
                 blk * self.cfg.block_size + pos % self.cfg.block_size)
         else:
             ptoks, pmap = pending_map if pending_map is not None else (None, {})
-            ids, dst, src = [], [], []
+            wide = np.zeros(self._wide.shape, dtype=np.int64)
+            narrow = np.zeros(self._narrow.shape, dtype=np.int32)
+            wide[2] = -1                   # padding rows do no work
+            narrow[1:3] = -1
+            dst, src = [], []
+            lens = [s.sched_tokens for s in seqs]
+            bsz = self.cfg.block_size
+            flat = np.zeros((bs, self._max_blocks), dtype=np.int32)
             for i, s in enumerate(seqs):
                 j = pmap.get(s.seq_id)
-                if j is not None and s.sched_tokens > s.num_tokens:
-                    ids.append(0)
+                if j is not None and lens[i] > s.num_tokens:
                     dst.append(i)
                     src.append(j)
                 else:
-                    ids.append(s.last_token_id)
-            pos = [s.sched_tokens - 1 for s in seqs]
-            slots = [self._slot(s, p) for s, p in zip(seqs, pos)]
-            lens = [s.sched_tokens for s in seqs]
-            b["input_ids"][:bs].copy_(
-                torch.tensor(ids, dtype=torch.long), non_blocking=True)
-            if dst:
-                didx = torch.tensor(dst, dtype=torch.long, device=self.device)
-                sidx = torch.tensor(src, dtype=torch.long, device=self.device)
-                b["input_ids"][:bs].index_copy_(0, didx, ptoks[sidx])
-            b["positions"][:bs].copy_(
-                torch.tensor(pos, dtype=torch.long), non_blocking=True)
-            b["slot_mapping"][:bs].copy_(
-                torch.tensor(slots, dtype=torch.long), non_blocking=True)
-            b["seq_lens"][:bs].copy_(
-                torch.tensor(lens, dtype=torch.int32), non_blocking=True)
-            if self.stateful:
-                b["state_slots"][:bs].copy_(torch.tensor(
-                    [s.state_slot for s in seqs], dtype=torch.int32),
-                    non_blocking=True)
-                b["seq_starts"][:bs].copy_(
-                    torch.tensor(pos, dtype=torch.int32), non_blocking=True)
-            import numpy as np
-            flat = np.zeros((bs, self._max_blocks), dtype=np.int32)
-            for i, s in enumerate(seqs):
-                flat[i, :len(s.block_table)] = s.block_table
+                    wide[0, i] = s.last_token_id
+                table = s.block_table
+                flat[i, :len(table)] = table
+                wide[2, i] = table[(lens[i] - 1) // bsz]
                 s._bt_dirty = False
+            narrow[0, :bs] = lens
+            pos = narrow[0, :bs].astype(np.int64) - 1
+            wide[1, :bs] = pos
+            wide[2, :bs] = wide[2, :bs] * bsz + pos % bsz
+            if self.lora_manager is not None:
+                narrow[1, :bs] = [s.lora_id for s in seqs]
+            if self.stateful:
+                narrow[2, :bs] = [s.state_slot for s in seqs]
+                narrow[3, :bs] = pos
+            self._wide.copy_(torch.from_numpy(wide), non_blocking=True)
+            self._narrow.copy_(torch.from_numpy(narrow), non_blocking=True)
             b["block_tables"][:bs].copy_(
                 torch.from_numpy(flat), non_blocking=True)
-            if self.lora_manager is not None:
-                b["lora_ids"][:bs].copy_(torch.tensor(
-                    [s.lora_id for s in seqs], dtype=torch.int32),
-                    non_blocking=True)
+            if dst:
+                at = torch.tensor([dst, src], dtype=torch.long,
+                                  device=self.device)
+                b["input_ids"].index_copy_(0, at[0], ptoks[at[1]])
         self._last_ids = ids_now
 
         bucket = self._graph_bucket(bs) if self._graphs else None
         if bucket is not None:
-            # zero the padded tail so padded rows do no work
-            if bucket > bs:
-                b["seq_lens"][bs:bucket].zero_()
-                b["slot_mapping"][bs:bucket].fill_(-1)
-                if self.stateful:
-                    b["state_slots"][bs:bucket].fill_(-1)
+            # rows behind the batch were made padding when it was built
             g, out = self._graphs[bucket]
             g.replay()
             return out[:bs]

@@ -12,6 +12,7 @@ time one of its ops is called.
 """
 from __future__ import annotations
 
+import numpy as np
 import torch
 
 from . import torch_ref
@@ -700,17 +701,24 @@ def window_attention(q, k_cache, v_cache, block_tables, token_seq, positions,
                                       temp_coef, temp_every)
 
 
+def query_tiles(chunk_lens, starts=None):
+    """64-row query tiles of a step's chunks, as numpy arrays (chunk of a
+    tile, its first row). Tiles with the most keys ahead of them (`starts`:
+    the chunks' first positions) come first, so that a causal launch does
+    not end on its longest workgroups."""
+    lens = np.asarray(chunk_lens, dtype=np.int64)
+    n = -(-lens // QTILE)
+    seq = np.repeat(np.arange(len(lens)), n)
+    base = (np.arange(int(n.sum())) - np.repeat(np.cumsum(n) - n, n)) * QTILE
+    ahead = base if starts is None else base + np.asarray(starts)[seq]
+    order = np.argsort(-ahead, kind="stable")
+    return seq[order].astype(np.int32), base[order].astype(np.int32)
+
+
 def build_query_tiles(chunk_lens, device, starts=None):
-    """Host-side tiling of a step's chunks into 64-row query tiles:
-    (tile_seq, tile_qbase) int32 tensors. Tiles with the most keys ahead
-    of them (`starts`: the chunks' first positions) come first, so that a
-    causal launch does not end on its longest workgroups."""
-    tiles = [(i, q0) for i, n in enumerate(chunk_lens)
-             for q0 in range(0, n, QTILE)]
-    tiles.sort(key=lambda t: -(t[1] + (starts[t[0]] if starts else 0)))
-    seqs, bases = [t[0] for t in tiles], [t[1] for t in tiles]
-    return (torch.tensor(seqs, dtype=torch.int32, device=device),
-            torch.tensor(bases, dtype=torch.int32, device=device))
+    """query_tiles as int32 tensors (tile_seq, tile_qbase)."""
+    return tuple(torch.from_numpy(t).to(device)
+                 for t in query_tiles(chunk_lens, starts))
 
 
 def post_norm_residual(x32, y, w, eps: float, out_dtype, y2=None, w_y=None,
