@@ -158,9 +158,10 @@ class MoEMLP(nn.Module):
             + (w_id if self.n_identity else None,)
 
     # Pairs up to which the weight-streaming kernels run, beyond it the tiled
-    # grouped GEMMs: 64 rows per expert, where 8 experts of 2048 x 2048 take
-    # 81 us tiled and 93 streamed, 8 of 4096 x 14336 741 and 998, 64 of 2048 x
-    # 1408 (48 rows) still 284 and 260. KAITO_MOE_FUSED_MAX overrides.
+    # grouped GEMMs: 16 rows per expert. Streamed and tiled, in us: 8 experts
+    # of 2048 x 2048 at 16 rows 59 and 79, at 32 99 and 82; 8 of 4096 x 14336
+    # 600 and 692, 1034 and 701; 64 of 2048 x 1408 at 12 rows 251 and 263, at
+    # 24 308 and 266. KAITO_MOE_FUSED_MAX overrides.
     import os as _os
     _most = _os.environ.get("KAITO_MOE_FUSED_MAX")
     FUSED_MAX_TOKENS = None if _most is None else int(_most)
@@ -175,7 +176,7 @@ class MoEMLP(nn.Module):
                 and self.ie_local % 64 == 0):
             return "loop"
         most = self.FUSED_MAX_TOKENS
-        if TK <= (64 * E if most is None else most):
+        if TK <= (16 * E if most is None else most):
             return "streamed"
         if TK >= 1024 * E and H >= 4096 and self.ie_local >= 4096 \
                 and not torch.cuda.is_current_stream_capturing():
@@ -201,17 +202,22 @@ class MoEMLP(nn.Module):
             shared = ops.linear(h1, self.w_shared_down)
         added = None if split_shared else shared
         kernels = self._kernels_for(x)
-        if kernels == "tiled":
-            out = self._forward_grouped(
-                x.contiguous(), topi, topw, w_id, sorted_tok, offsets, pos,
-                added, keep_f32)
-            added = None
-        else:
+        if kernels == "loop":
             out = self._routed_start(x, w_id)
-            run = self._forward_fused if kernels == "streamed" \
-                else self._forward_loop
-            run(x, sorted_tok, gates, offsets, out)
+            self._forward_loop(x, sorted_tok, gates, offsets, out)
             out = out if keep_f32 else out.to(x.dtype)
+        else:
+            x = x.contiguous()
+            if x.data_ptr() % 16:
+                x = x.clone()
+            y = self._rows_streamed(x, sorted_tok, offsets) \
+                if kernels == "streamed" \
+                else self._rows_tiled(x, sorted_tok, offsets)
+            out = torch.empty(T, H, device=x.device, dtype=torch.float32
+                              if keep_f32 else x.dtype)
+            ops.moe_combine(out, y, pos, topi, topw, self.e_base,
+                            self.e_local, x, w_id, added)
+            added = None
         if split_shared:
             assert get_state().tp_size == 1
             return out, shared
@@ -227,11 +233,10 @@ class MoEMLP(nn.Module):
         return torch.zeros(x.shape, dtype=torch.float32, device=x.device) \
             if w_id is None else x * w_id[:, None]
 
-    def _forward_grouped(self, x, topi, topw, w_id, sorted_tok, offsets, pos,
-                         shared, keep_f32):
-        """Tiled grouped GEMMs over the sorted rows, then one pass per token
-        that sums its experts (static shapes, no host read)."""
-        TK, H = topi.numel(), x.size(1)
+    # Both return the experts' outputs of the sorted rows, to be summed per
+    # token by moe_combine; static shapes, no host read.
+    def _rows_tiled(self, x, sorted_tok, offsets):
+        TK, H = sorted_tok.numel(), x.size(1)
         act = torch.empty(TK, self.ie_local, dtype=x.dtype, device=x.device)
         ops.moe_grouped_up(act, x, self.w_gate_up, sorted_tok, offsets,
                            self.e_base, self.b_gate_up, self.act_mode,
@@ -244,25 +249,27 @@ class MoEMLP(nn.Module):
                         else x.dtype)
         ops.moe_grouped_down(y, act, self.w_down, offsets, self.e_base,
                              self.b_down)
-        out = torch.empty(x.shape, dtype=torch.float32 if keep_f32
-                          else x.dtype, device=x.device)
-        ops.moe_combine(out, y, pos, topi, topw, self.e_base, self.e_local,
-                        x, w_id, shared)
-        return out
+        return y
 
-    def _forward_fused(self, x, sorted_tok, gates, offsets, out32):
-        """Static-shape HIP grouped GEMMs (graph-capturable), added into
-        out32."""
-        T, H = x.shape
-        TK = T * self.top_k
-        # staging reads WHOLE 64-row tiles from unaligned expert offsets:
-        # a tile may start at row TK-1 and read through TK+62, so pad a
-        # full extra tile beyond the round-up
-        pad = (TK + 63) // 64 * 64 + 64
-        act = torch.empty(pad, self.ie_local, dtype=x.dtype, device=x.device)
+    def _gated_rows(self, x, sorted_tok, offsets):
+        act = torch.empty(sorted_tok.numel(), self.ie_local, dtype=x.dtype,
+                          device=x.device)
         ops.moe_gate_silu(act, x, self.w_gate_up, sorted_tok, offsets,
                           self.e_base, self.e_local, self.b_gate_up,
                           self.act_mode, self.act_limit)
+        return act
+
+    def _rows_streamed(self, x, sorted_tok, offsets):
+        act = self._gated_rows(x, sorted_tok, offsets)
+        y = torch.empty(sorted_tok.numel(), x.size(1), dtype=torch.float32,
+                        device=x.device)
+        ops.moe_down_rows(y, act, self.w_down, offsets, self.e_base,
+                          self.e_local, self.b_down)
+        return y
+
+    def _forward_fused(self, x, sorted_tok, gates, offsets, out32):
+        """The streaming kernels with the weighted rows added into out32."""
+        act = self._gated_rows(x, sorted_tok, offsets)
         ops.moe_down_scatter(out32, act, self.w_down, sorted_tok, gates,
                              offsets, self.e_base, self.e_local,
                              self.b_down)

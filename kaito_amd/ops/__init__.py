@@ -29,7 +29,7 @@ for _g, _names in {
     "attn": ("paged_attention paged_attention_sp prefill_attention "
              "mla_prefill_attention context_attention mfma_tile_gemm paged_read_bw"),
     "mla": "mla_decode mla_cache_write",
-    "moe": ("moe_gate_silu moe_down_scatter moe_grouped_up "
+    "moe": ("moe_gate_silu moe_down_rows moe_down_scatter moe_grouped_up "
             "moe_grouped_down moe_combine"),
     "route": "moe_route moe_gate_route moe_sort",
     "quant": "w4a16_gemv w4a16_dequant w4a16_gemm lora_shrink lora_expand",
@@ -141,28 +141,42 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
     return torch_ref.silu_and_mul(x)
 
 
-SKINNY_MAX_M = 4
+def _skinny(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
+    """Whether x W^T runs on the weight-streaming kernels: a few rows of
+    bf16 on the GPU, 16-byte aligned rows, nothing to differentiate.
 
-
-def _skinny(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether x W^T runs on the row-streaming kernel: at most 4 rows of
-    bf16 on the GPU, 16-byte aligned rows, nothing to differentiate. At 8
-    llama-3.1-8b layers' sizes it reads W at 5 to 7 TB/s for one row and 3.7
-    to 5.7 for four, hipBLASLt's tuned choices at 2.2 to 4.8 for both; more
-    rows are bound by the vector unit and stay with the library."""
-    return (x.is_cuda and x.dim() == 2 and 1 <= x.size(0) <= SKINNY_MAX_M
+    Up to 4 rows always: at 8 llama-3.1-8b layers' sizes W is read at 5 to 7
+    TB/s for one row and 3.6 to 4.9 for four, by hipBLASLt's tuned choices at
+    2.2 to 4.8 for both. Beyond, x comes through the caches once per 16 rows
+    of W, and the library is ahead from where that costs more (us, streamed
+    and library): 8 rows win but for the longest K (28672 x 4096: 44.5, 53.0;
+    4096 x 14336: 25.9, 25.1); 16 rows up to 4096 x 4096 (11.2, 15.4; 6144 x
+    4096: 15.9, 14.4) and in a SwiGLU pair; 32 rows up to 3072 x 2048 (7.9,
+    11.4; 6144 x 2048: 13.3, 12.4)."""
+    if not (x.is_cuda and x.dim() == 2 and 1 <= x.size(0) <= 32
             and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and w.is_contiguous() and w.size(1) % 8 == 0 and w.numel() > 0
             and x.stride(1) == 1
             and (x.size(0) == 1 or x.stride(0) % 8 == 0)
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
             and not (torch.is_grad_enabled()
-                     and (x.requires_grad or w.requires_grad)))
+                     and (x.requires_grad or w.requires_grad))):
+        return False
+    M, (N, K) = x.size(0), w.shape
+    if M <= 4:
+        return True
+    if K % 64 or N % 16:
+        return False
+    if M <= 8:
+        return K <= 8192
+    if M <= 16:
+        return N * K <= 4096 * 4096 or (glu and K <= 8192)
+    return N * K <= 3072 * 2048
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
-    """x W^T (+ bias): the row-streaming kernel for the smallest decode
-    steps, hipBLASLt otherwise."""
+    """x W^T (+ bias): the weight-streaming kernels for small decode steps,
+    hipBLASLt otherwise."""
     if _skinny(x, w) and (bias is None or (
             bias.dtype == torch.bfloat16 and bias.is_contiguous()
             and not (torch.is_grad_enabled() and bias.requires_grad))):
@@ -175,7 +189,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
 
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x Wg^T) * (x Wu^T) for the stacked W = [Wg | Wu]."""
-    if _skinny(x, w):
+    if _skinny(x, w, True):
         out = torch.empty(x.size(0), w.size(0) // 2, dtype=x.dtype,
                           device=x.device)
         _K.skinny_swiglu(out, x, w)
@@ -373,6 +387,14 @@ def moe_gate_silu(act: torch.Tensor, x: torch.Tensor,
     b = bias if bias is not None else         torch.empty(0, dtype=x.dtype, device=x.device)
     _K.moe_gate_silu(act, x, w_gate_up, sorted_ids, offsets, b, act_mode,
                      e_base, n_local_experts, act_limit)
+
+
+def moe_down_rows(y, act, w_down, offsets, e_base: int, n_local_experts: int,
+                  bias=None) -> None:
+    """Stage 2 of decode-sized steps (GPU only): y [TK, H] f32, the down
+    product (+ optional [E, H] bias) of every sorted row."""
+    _K.moe_down_rows(y, act, w_down, offsets, _none(bias, act), e_base,
+                     n_local_experts)
 
 
 def moe_down_scatter(out: torch.Tensor, act: torch.Tensor,

@@ -8,10 +8,12 @@
 // TB/s; the same rows read as MFMA operands (64 B of 16 rows per load) 45.7
 // us, hipBLASLt's tuned choice 57.5 us.
 //
-// More rows of x, and experts with a few rows each: v_mfma_f32_16x16x32_bf16
-// with W read straight into operand registers (a lane's 16 bytes are 8 k of
-// one row); the waves of a workgroup take every NW-th slice of K and meet in
-// LDS, in f32.
+// Up to 32 rows of x, and experts with a few rows each: the same streams
+// through LDS into v_mfma_f32_16x16x32_bf16 (stream_tile). A workgroup owns
+// 16 rows of W; its waves take every fourth slice of K and meet in LDS, in
+// f32. 28672 x 4096: 44.5 us at M = 8 (library 53.0), 50.5 at 16 (53.8), 74.6 at
+// 32 (53.2): x comes through the caches once per workgroup, so the gain ends
+// where its rows cost what those of W do.
 //
 // 4-bit weights run as integers: a word's nibbles j and j + 4 become the bf16
 // pair 128 + q by one shift and one and-or (x is permuted to match), and per
@@ -42,43 +44,85 @@ KAITO_DEV hbf16x8 load_x(const short* p) {
   return *reinterpret_cast<const hbf16x8*>(p);
 }
 
-// acc[mt][j] += x rows 16 mt.. times W rows of tile j, over the slices of
-// this wave. wp/xp: the lane's rows (l & 15) at k = 8 (l >> 4).
-template <int MT, int NT>
-KAITO_DEV void accumulate(f32x4 (&acc)[MT][NT], const short* const (&wp)[NT],
-                          const short* const (&xp)[MT], const int K,
-                          const int wave, const int nw) {
-  constexpr int STEPS = MT * NT <= 2 ? 8 : (MT * NT <= 4 ? 4 : 2);
-  constexpr int KC = STEPS * 32;
-  for (int k0 = wave * KC; k0 < K; k0 += nw * KC) {
-    if (k0 + KC <= K) {
-      hbf16x8 wf[NT][STEPS], xf[MT][STEPS];
+// ---- up to 32 rows of x: 16 rows of W per workgroup through LDS -------------
+// A stage is 16 rows x KS k, copied by 16-byte direct loads in pieces of KS *
+// 2 contiguous bytes (whole lines), 16-byte chunk c of row r at c ^ (r & 7).
+// Two stages per wave: the next one, and the x operands beside it, are under
+// way while the present one is multiplied. Nothing is shared between waves, so
+// the waits are counts of this wave's own loads and there are no barriers.
+constexpr int TILE_NW = 4;          // waves per workgroup, over K
+
+// direct loads per lane and stage of 16 rows x KS k
+template <int KS>
+constexpr int tile_loads() { return 16 * KS / 512; }
+
+// row of the 16 that load j of this lane copies, and the element offset of
+// its piece inside the row's stage
+template <int KS>
+KAITO_DEV int tile_row(const int j, const int lane) {
+  return j * (512 / KS) + lane / (KS / 8);
+}
+template <int KS>
+KAITO_DEV int tile_col(const int j, const int lane) {
+  return ((lane % (KS / 8)) ^ (tile_row<KS>(j, lane) & 7)) * 8;
+}
+
+template <int N>
+KAITO_DEV void wait_loads() {       // until N of this wave's loads are left
+  __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
+  asm volatile("" ::: "memory");
+}
+
+// acc[mt] += x rows 16 mt.. times the 16 rows of W. src[j]: source of load j
+// (tile_row, tile_col); xp[mt]: the lane's x row (lane & 15) at 8 (lane >> 4);
+// ring: [2][16 * KS] of this wave. K is a multiple of KS.
+template <int MT, int KS>
+KAITO_DEV void stream_tile(f32x4 (&acc)[MT],
+                           const short* const (&src)[tile_loads<KS>()],
+                           const short* const (&xp)[MT], short* ring,
+                           const int K, const int wave, const int lane) {
+  constexpr int NI = tile_loads<KS>(), STEPS = KS / 32;
+  const int n = K / KS, lo = lane & 15, hi = lane >> 4;
+  hbf16x8 xf[2][MT][STEPS];
+  auto fetch = [&](const int s, const int b) {
 #pragma unroll
-      for (int s = 0; s < STEPS; s++)
+    for (int mt = 0; mt < MT; mt++)
 #pragma unroll
-        for (int j = 0; j < NT; j++)
-          wf[j][s] = load_stream<hbf16x8>(wp[j] + k0 + s * 32);
+      for (int i = 0; i < STEPS; i++)
+        xf[b][mt][i] = load_x(xp[mt] + s * KS + i * 32);
 #pragma unroll
-      for (int s = 0; s < STEPS; s++)
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++)
-          xf[mt][s] = load_x(xp[mt] + k0 + s * 32);
-#pragma unroll
-      for (int s = 0; s < STEPS; s++)
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-          for (int j = 0; j < NT; j++)
-            acc[mt][j] = mfma16(xf[mt][s], wf[j][s], acc[mt][j]);
+    for (int j = 0; j < NI; j++)
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) unsigned int*)(src[j] +
+                                                                  s * KS),
+          (__attribute__((address_space(3))) unsigned int*)(
+              ring + b * 16 * KS + j * 512),
+          16, 0, 2 /* non-temporal */);
+  };
+  auto step = [&](const int s, const int b) {
+    // the other stage's reads are done before it is overwritten
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    asm volatile("" ::: "memory");
+    if (s + TILE_NW < n) {
+      fetch(s + TILE_NW, b ^ 1);
+      wait_loads<MT * STEPS + NI>();
     } else {
-      for (int k = k0; k < K; k += 32)
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-          for (int j = 0; j < NT; j++)
-            acc[mt][j] = mfma16(load_x(xp[mt] + k),
-                                load_stream<hbf16x8>(wp[j] + k), acc[mt][j]);
+      wait_loads<0>();
     }
+    const short* w = ring + b * 16 * KS + lo * KS;
+#pragma unroll
+    for (int i = 0; i < STEPS; i++) {
+      const hbf16x8 wf =
+          load_x(w + (((i * 4 + hi) ^ (lo & 7)) * 8));
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++)
+        acc[mt] = mfma16(xf[b][mt][i], wf, acc[mt]);
+    }
+  };
+  if (wave < n) fetch(wave, 0);
+  for (int s = wave; s < n; s += 2 * TILE_NW) {
+    step(s, 0);
+    if (s + TILE_NW < n) step(s + TILE_NW, 1);
   }
 }
 

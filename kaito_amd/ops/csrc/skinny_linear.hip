@@ -1,4 +1,4 @@
-// Linear layers of the smallest decode steps (skinny.h), M <= 4 rows:
+// Linear layers of decode steps (skinny.h), M <= 32 rows:
 //   skinny_linear  out = x W^T (+ bias)
 //   skinny_swiglu  out = silu(x Wg^T) * (x Wu^T), W = [Wg | Wu] stacked
 #include "skinny.h"
@@ -49,17 +49,74 @@ __global__ __launch_bounds__(NW * 64) void skinny_linear_kernel(
   }
 }
 
+// M <= 16 MT rows; N is a multiple of 16 (GLU: of 8, the workgroup's 16 rows
+// are 8 gate rows and their up rows, N apart), K of the stage
+template <int MT, int KS, bool GLU>
+__global__ __launch_bounds__(256, 2) void skinny_tile_kernel(
+    short* __restrict__ out, const short* __restrict__ x,
+    const int64_t x_stride, const short* __restrict__ w,
+    const short* __restrict__ bias, const int M, const int N, const int K) {
+  constexpr int NI = skinny::tile_loads<KS>();
+  __shared__ __attribute__((aligned(128))) short ring[4][2][16 * KS];
+  static_assert(sizeof(ring) >= 4 * MT * 64 * sizeof(f32x4), "fold");
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = blockIdx.x * (GLU ? 8 : 16);
+  const short *src[NI], *xp[MT];
+#pragma unroll
+  for (int j = 0; j < NI; j++) {
+    const int r = skinny::tile_row<KS>(j, lane);
+    const int64_t n = GLU ? n0 + r % 8 + (r >= 8 ? N : 0) : n0 + r;
+    src[j] = w + n * K + skinny::tile_col<KS>(j, lane);
+  }
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++)
+    xp[mt] = x + min(mt * 16 + (lane & 15), M - 1) * x_stride +
+        (lane >> 4) * 8;
+  f32x4 acc[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  skinny::stream_tile<MT, KS>(acc, src, xp, ring[wave][0], K, wave, lane);
+  __syncthreads();                  // every wave is done with its stages
+  f32x4* red = reinterpret_cast<f32x4*>(&ring[0][0][0]);
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++) red[(wave * MT + mt) * 64 + lane] = acc[mt];
+  __syncthreads();
+  // slot: tile mt, lane l: rows 16 mt + 4 (l >> 4) .. of column l & 15
+  if (threadIdx.x >= MT * 64) return;
+  const int slot = threadIdx.x, l = slot & 63, c = l & 15;
+  if (GLU && c >= 8) return;
+  f32x4 v = skinny::fold<MT, 4>(red, slot);
+  if constexpr (GLU) {
+    const f32x4 u = skinny::fold<MT, 4>(red, slot + 8);
+#pragma unroll
+    for (int r = 0; r < 4; r++) v[r] = skinny::silu(v[r]) * u[r];
+  } else if (bias) {
+    v += bf16_to_f32(bias[n0 + c]);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int m = (slot >> 6) * 16 + (l >> 4) * 4 + r;
+    if (m < M) out[(int64_t)m * N + n0 + c] = f32_to_bf16(v[r]);
+  }
+}
+
+constexpr int MAX_M = 32;
+
 void check(const at::Tensor& out, const at::Tensor& x, const at::Tensor& w,
-           int64_t N) {
+           int64_t N, int64_t cols) {
   for (const auto& t : {out, x, w})
     TORCH_CHECK(t.is_cuda() && t.dtype() == at::kBFloat16 && t.dim() == 2 &&
                 t.stride(1) == 1 && (uintptr_t)t.data_ptr() % 16 == 0);
   TORCH_CHECK(w.is_contiguous() && out.is_contiguous() &&
               x.size(1) == w.size(1) && out.size(0) == x.size(0) &&
               out.size(1) == N);
-  TORCH_CHECK(x.size(0) >= 1 && x.size(0) <= 4 && w.size(1) % 8 == 0 &&
-              w.size(1) > 0 && (x.size(0) == 1 || x.stride(0) % 8 == 0) &&
-              w.size(0) < (1ll << 31) && w.size(1) < (1ll << 31));
+  const int64_t M = x.size(0), K = w.size(1);
+  TORCH_CHECK(M >= 1 && M <= MAX_M && K % 8 == 0 && K > 0 &&
+              (M == 1 || x.stride(0) % 8 == 0) && w.size(0) < (1ll << 31) &&
+              K < (1ll << 31));
+  TORCH_CHECK(M <= 4 || (K % 64 == 0 && N % cols == 0),
+              "more than 4 rows: K in whole stages, N in whole tiles");
 }
 
 }  // namespace
@@ -67,7 +124,7 @@ void check(const at::Tensor& out, const at::Tensor& x, const at::Tensor& w,
 void skinny_linear(at::Tensor out, at::Tensor x, at::Tensor w,
                    at::Tensor bias) {
   const int64_t N = w.size(0);
-  check(out, x, w, N);
+  check(out, x, w, N, 16);
   const bool has_bias = bias.numel() > 0;
   TORCH_CHECK(!has_bias || (bias.is_cuda() && bias.is_contiguous() &&
                             bias.dtype() == at::kBFloat16 &&
@@ -83,7 +140,22 @@ void skinny_linear(at::Tensor out, at::Tensor x, at::Tensor w,
       (const short*)x.data_ptr(), x.stride(0), (const short*)w.data_ptr(),    \
       has_bias ? (const short*)bias.data_ptr() : nullptr, (int)N,             \
       (int)w.size(1))
-  switch (x.size(0)) {
+  const int M = x.size(0);
+#define SLT_LAUNCH(MT_, KS_)                                                  \
+  hipLaunchKernelGGL((skinny_tile_kernel<MT_, KS_, false>), dim3(N / 16),         \
+      dim3(256), 0, at::hip::getCurrentHIPStream(), (short*)out.data_ptr(),   \
+      (const short*)x.data_ptr(), x.stride(0), (const short*)w.data_ptr(),    \
+      has_bias ? (const short*)bias.data_ptr() : nullptr, M, (int)N, (int)w.size(1))
+  if (M > 4) {
+    if (w.size(1) % 256 == 0) {
+      if (M > 16) SLT_LAUNCH(2, 256); else SLT_LAUNCH(1, 256);
+    } else {
+      if (M > 16) SLT_LAUNCH(2, 64); else SLT_LAUNCH(1, 64);
+    }
+    return;
+  }
+#undef SLT_LAUNCH
+  switch (M) {
     case 1: SL_LAUNCH(1, 1); break;
     case 2: SL_LAUNCH(2, 2); break;
     case 3: SL_LAUNCH(3, 2); break;
@@ -95,15 +167,30 @@ void skinny_linear(at::Tensor out, at::Tensor x, at::Tensor w,
 void skinny_swiglu(at::Tensor out, at::Tensor x, at::Tensor w) {
   TORCH_CHECK(w.size(0) % 2 == 0);
   const int64_t N = w.size(0) / 2;
-  check(out, x, w, N);
+  check(out, x, w, N, 8);
   if (N == 0) return;
+  const int M = x.size(0);
+#define SGT_LAUNCH(MT_, KS_)                                                  \
+  hipLaunchKernelGGL((skinny_tile_kernel<MT_, KS_, true>), dim3(N / 8),         \
+      dim3(256), 0, at::hip::getCurrentHIPStream(), (short*)out.data_ptr(),   \
+      (const short*)x.data_ptr(), x.stride(0), (const short*)w.data_ptr(),    \
+      nullptr, M, (int)N, (int)w.size(1))
+  if (M > 4) {
+    if (w.size(1) % 256 == 0) {
+      if (M > 16) SGT_LAUNCH(2, 256); else SGT_LAUNCH(1, 256);
+    } else {
+      if (M > 16) SGT_LAUNCH(2, 64); else SGT_LAUNCH(1, 64);
+    }
+    return;
+  }
+#undef SGT_LAUNCH
 #define SG_LAUNCH(M_)                                                         \
   hipLaunchKernelGGL((skinny_linear_kernel<M_, 2, true>),                     \
       dim3((N + NW - 1) / NW), dim3(NW * 64), 0,                              \
       at::hip::getCurrentHIPStream(), (short*)out.data_ptr(),                 \
       (const short*)x.data_ptr(), x.stride(0), (const short*)w.data_ptr(),    \
       nullptr, (int)N, (int)w.size(1))
-  switch (x.size(0)) {
+  switch (M) {
     case 1: SG_LAUNCH(1); break;
     case 2: SG_LAUNCH(2); break;
     case 3: SG_LAUNCH(3); break;

@@ -82,6 +82,59 @@ def test_grouped_step(counts, H, IE, mode, bias, part, f32):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("counts,H,IE,mode,bias,part", [
+    ([1], 64, 64, 0, False, None),
+    ([3, 0, 16, 17, 1], 256, 192, 0, True, None),
+    ([0, 15, 33], 192, 512, 2, False, None),
+    ([70, 2], 512, 64, 1, True, None),
+    ([9, 20, 3, 12], 128, 128, 0, True, (1, 2)),
+    ([2] * 70, 64, 256, 1, False, None),
+])
+def test_streamed_step(counts, H, IE, mode, bias, part):
+    """The decode-sized kernels (ops/csrc/moe.hip): passes of 16 and 32 rows
+    per expert, K in stages of 256 and 64; the two ways to add the rows."""
+    torch.manual_seed(sum(counts))
+    E, T = len(counts), sum(counts)
+    lo, n = part or (0, E)
+    topi = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    topi = topi[torch.randperm(T)].to(DEV).int()[:, None]
+    topw = torch.rand(T, 1, device=DEV) + 0.5
+    x = _rand(T, H)
+    wu = _rand(E, (1 if mode == 2 else 2) * IE, H, std=H ** -0.5)
+    wd = _rand(E, H, IE, std=IE ** -0.5)
+    bu = _rand(E, 2 * IE) if bias and mode != 2 else None
+    bd = _rand(E, H) if bias else None
+    tok, gates, off, pos = ops.moe_plan(topi, topw, E)
+    cut = slice(lo, lo + n)
+    act = torch.full((T, IE), float("nan"), device=DEV).to(torch.bfloat16)
+    y = torch.full((T, H), float("nan"), device=DEV)
+    out, added = torch.empty(T, H, device=DEV), torch.zeros(T, H, device=DEV)
+    ops.moe_gate_silu(act, x, wu[cut].contiguous(), tok, off, lo, n,
+                      bu[cut].contiguous() if bu is not None else None, mode,
+                      7.0)
+    b = bd[cut].contiguous() if bias else None
+    ops.moe_down_rows(y, act, wd[cut].contiguous(), off, lo, n, b)
+    ops.moe_combine(out, y, pos, topi, topw, lo, n)
+    ops.moe_down_scatter(added, act, wd[cut].contiguous(), tok, gates, off,
+                         lo, n, b)
+    ref = torch.zeros(T, H, dtype=torch.float64, device=DEV)
+    for e in range(lo, lo + n):
+        t = torch.nonzero(topi[:, 0] == e)[:, 0]
+        h = x[t].double() @ wu[e].double().T
+        if bu is not None:
+            h = h + bu[e].double()
+        v = _act(mode, h, IE) @ wd[e].double().T
+        if bias:
+            v = v + bd[e].double()
+        ref[t] = v * topw[t].double()
+    rms = ref.square().mean().sqrt()
+    for got in (out, added):        # act rounded to bf16 once
+        err = (got.double() - ref).abs()
+        assert err.max() <= 2.0 ** -5.5 * rms, err.max() / rms
+        assert err.square().mean().sqrt() <= 2.0 ** -8 * rms
+
+
+@pytest.mark.gpu
 def test_several_choices_sum():
     torch.manual_seed(3)
     T, H, K = 50, 2056, 6

@@ -38,12 +38,31 @@ def test_rows(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [5, 8, 9, 16, 17, 31, 32])
+@pytest.mark.parametrize("N,K", [(16, 64), (48, 192), (64, 256), (112, 1792),
+                                 (32, 2048), (16, 2368)])
+def test_tiles(M, N, K):
+    torch.manual_seed(M * N + K)
+    x = torch.randn(M, K + 16, device=DEV).to(torch.bfloat16)[:, 8:8 + K]
+    w = torch.randn(2 * N, K, device=DEV).to(torch.bfloat16)
+    b = torch.randn(2 * N, device=DEV).to(torch.bfloat16)
+    ref = x.double() @ w.double().T
+    assert ops._skinny(x, w)
+    _close(ops.linear(x, w), ref)
+    _close(ops.linear(x, w, b), ref + b.double())
+    g, u = ref.chunk(2, -1)
+    _close(ops.linear_swiglu(x, w), g * torch.sigmoid(g) * u)
+
+
+@pytest.mark.gpu
 def test_other_forms_stay_with_the_library():
-    x = torch.randn(5, 64, device=DEV).to(torch.bfloat16)
+    x = torch.randn(33, 64, device=DEV).to(torch.bfloat16)
     w = torch.randn(32, 64, device=DEV).to(torch.bfloat16)
     for a, b in [(x, w), (x[:2, :60], w[:, :60]), (x[:2, 1:57], w[:, :56].
                  contiguous()), (x[:2].float(), w.float()), (x[:2, None], w),
-                 (x[:0], w), (x[:2], w.T.contiguous().T)]:
+                 (x[:0], w), (x[:2], w.T.contiguous().T),
+                 (x[:5, :56].contiguous(), w[:, :56].contiguous()),
+                 (x[:5], w[:24])]:
         assert not ops._skinny(a, b)
         assert torch.equal(ops.linear(a, b),
                            torch.nn.functional.linear(a, b))
