@@ -138,33 +138,18 @@ class MLAAttention(nn.Module):
         T = x.size(0)
         q = self._project_q(x)                          # [T, Hl, nope+rope]
         q_nope = q[..., :self.nope]
-        q_pe = q[..., self.nope:].contiguous()          # [T, Hl, rope]
-
+        q_pe = q[..., self.nope:]                       # [T, Hl, rope]
         kv_a = ops.linear(x, self.kv_a_proj_with_mqa)
-        c_kv = ops.rms_norm(kv_a[:, :self.r].contiguous(),
-                            self.kv_a_layernorm, self.cfg.rms_eps)
-        k_pe = kv_a[:, self.r:].contiguous()            # [T, rope]
-
-        q_pe, k_pe = ops.rotary_embedding(
-            positions, q_pe.view(T, -1), k_pe, self.rope, cos_sin)
-        q_pe = q_pe.view(T, self.num_heads, self.rope)
-
-        if kv_cache is not None:
-            cache = kv_cache[0]                    # [NB+1, BS, r+rope]
-            if cache.is_cuda:
-                # one fused scatter (skips -1 padding slots in-kernel);
-                # replaces a where+cat+index_copy_ chain that cost ~7%
-                # of a serving run (profiles/r02_mla_kernels.md)
-                ops.mla_cache_write(cache, c_kv, k_pe, meta.slot_mapping)
-            else:
-                rows = cache.view(-1, cache.size(-1))
-                slots = meta.slot_mapping
-                slots = torch.where(
-                    slots < 0, torch.full_like(slots, rows.size(0) - 1),
-                    slots)
-                rows.index_copy_(
-                    0, slots,
-                    torch.cat([c_kv, k_pe], dim=-1).to(cache.dtype))
+        if x.is_cuda and x.dtype == torch.bfloat16 \
+                and (self.r, self.rope, cos_sin.size(1)) == (512, 64, 64) \
+                and self.nope % 8 == 0 and q.data_ptr() % 16 == 0:
+            q_pe, c_kv, k_pe = ops.mla_prepare(
+                q_pe, kv_a, self.kv_a_layernorm, self.cfg.rms_eps, positions,
+                cos_sin, None if kv_cache is None else kv_cache[0],
+                None if kv_cache is None else meta.slot_mapping)
+        else:
+            q_pe, c_kv, k_pe = self._prepare(q_pe, kv_a, positions, cos_sin,
+                                             kv_cache, meta)
 
         if meta.is_prefill:
             if meta.kv_lens is not None:
@@ -177,17 +162,38 @@ class MLAAttention(nn.Module):
             out = self._decode(q_nope, q_pe, kv_cache[0], meta)
         return self.o_proj(out.reshape(T, -1))
 
+    def _prepare(self, q_pe, kv_a, positions, cos_sin, kv_cache, meta):
+        """ops.mla_prepare by single operations, for other sizes."""
+        T = q_pe.size(0)
+        c_kv = ops.rms_norm(kv_a[:, :self.r].contiguous(),
+                            self.kv_a_layernorm, self.cfg.rms_eps)
+        k_pe = kv_a[:, self.r:].contiguous()            # [T, rope]
+        q_pe, k_pe = ops.rotary_embedding(
+            positions, q_pe.contiguous().view(T, -1), k_pe, self.rope,
+            cos_sin)
+        if kv_cache is not None:
+            cache = kv_cache[0]                    # [NB+1, BS, r+rope]
+            if cache.is_cuda:
+                ops.mla_cache_write(cache, c_kv, k_pe, meta.slot_mapping)
+            else:
+                rows = cache.view(-1, cache.size(-1))
+                slots = meta.slot_mapping
+                slots = torch.where(
+                    slots < 0, torch.full_like(slots, rows.size(0) - 1),
+                    slots)
+                rows.index_copy_(
+                    0, slots,
+                    torch.cat([c_kv, k_pe], dim=-1).to(cache.dtype))
+        return q_pe.view(T, self.num_heads, self.rope), c_kv, k_pe
+
     # ---- absorbed decode over the latent cache --------------------------
     def _decode(self, q_nope, q_pe, cache, meta) -> torch.Tensor:
         T = q_nope.size(0)
-        # q_c[h] = q_nope[h] @ w_kc[h]: [Hl, T, nope] x [Hl, nope, r].
-        # strided views feed hipBLASLt batched GEMM directly (no
-        # .contiguous() copies — profiles/r02_mla_kernels.md overhead)
+        # q_c[h] = q_nope[h] @ w_kc[h]: [Hl, T, nope] x [Hl, nope, r], read
+        # by the kernel where the product leaves it
         q_c = torch.bmm(q_nope.transpose(0, 1), self.w_kc)
-        q_full = torch.cat(
-            [q_c.transpose(0, 1), q_pe], dim=-1).contiguous()  # [T,Hl,r+rope]
-        out_c = ops.mla_decode(q_full, cache, meta.block_tables,
-                               meta.seq_lens, self.scale, self.r)
+        out_c = ops.mla_decode(q_c.transpose(0, 1), cache, meta.block_tables,
+                               meta.seq_lens, self.scale, self.r, q_pe)
         # latent -> per-head v: [Hl, T, r] x [Hl, r, v]
         o = torch.bmm(out_c.transpose(0, 1), self.w_vc)
         return o.transpose(0, 1).reshape(T, -1)         # one copy at most

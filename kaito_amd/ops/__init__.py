@@ -28,7 +28,7 @@ for _g, _names in {
              "reshape_and_cache topk skinny_linear skinny_swiglu"),
     "attn": ("paged_attention paged_attention_sp prefill_attention "
              "mla_prefill_attention context_attention mfma_tile_gemm paged_read_bw"),
-    "mla": "mla_decode mla_cache_write",
+    "mla": "mla_decode mla_prepare mla_cache_write",
     "moe": ("moe_gate_silu moe_down_rows moe_down_scatter moe_grouped_up "
             "moe_grouped_down moe_combine"),
     "route": "moe_route moe_gate_route moe_sort",
@@ -244,16 +244,37 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
 
 def mla_decode(q: torch.Tensor, cache: torch.Tensor,
                block_tables: torch.Tensor, seq_lens: torch.Tensor,
-               scale: float, r: int) -> torch.Tensor:
+               scale: float, r: int,
+               q_rope: torch.Tensor | None = None) -> torch.Tensor:
     """Absorbed MLA decode over the compressed latent cache (DeepSeek).
-    q: [T, H, r+rope]; cache: [NB, BS, r+rope] bf16. Returns [T, H, r]."""
+    q: [T, H, r+rope], or [T, H, r] with q_rope [T, H, rope], of any token
+    and head strides; cache: [NB, BS, r+rope] bf16. Returns [T, H, r]."""
     if q.is_cuda:
+        if q_rope is None:
+            assert q.is_contiguous()
+            q, q_rope = q[..., :r], q[..., r:]
         out = torch.empty(q.size(0), q.size(1), r, dtype=q.dtype,
                           device=q.device)
-        _K.mla_decode(out, q, cache, block_tables, seq_lens,
-                                   scale)
+        _K.mla_decode(out, q, q_rope, cache, block_tables, seq_lens, scale)
         return out
+    if q_rope is not None:
+        q = torch.cat([q, q_rope], -1)
     return torch_ref.mla_decode(q, cache, block_tables, seq_lens, scale, r)
+
+
+def mla_prepare(q: torch.Tensor, kv_a: torch.Tensor, w: torch.Tensor,
+                eps: float, positions: torch.Tensor, cos_sin: torch.Tensor,
+                cache: torch.Tensor | None, slots: torch.Tensor | None):
+    """GPU only: rotated q [T, H, 64] (any token and head strides), the
+    normed latent and the rotated key part of kv_a [T, 512 + 64], both
+    scattered into the cache, if one is given, as by mla_cache_write."""
+    T, H, P = q.shape
+    q_out = torch.empty(T, H, P, dtype=q.dtype, device=q.device)
+    c = torch.empty(T, w.numel(), dtype=q.dtype, device=q.device)
+    k = torch.empty(T, P, dtype=q.dtype, device=q.device)
+    _K.mla_prepare(q_out, c, k, _none(cache, q), q, kv_a, w, eps, positions,
+                   cos_sin, positions if slots is None else slots)
+    return q_out, c, k
 
 
 def mla_cache_write(cache: torch.Tensor, c_kv: torch.Tensor,

@@ -4,18 +4,24 @@
 #include <ATen/ATen.h>
 
 namespace kaito {
-void mla_decode(at::Tensor out, at::Tensor q, at::Tensor cache,
+void mla_decode(at::Tensor out, at::Tensor qc, at::Tensor qr, at::Tensor cache,
                 at::Tensor block_tables, at::Tensor seq_lens, double scale);
+void mla_prepare(at::Tensor q_out, at::Tensor c_out, at::Tensor k_out,
+                 at::Tensor cache, at::Tensor q, at::Tensor kv_a, at::Tensor w,
+                 double eps, at::Tensor positions, at::Tensor cos_sin,
+                 at::Tensor slots);
 void mla_cache_write(at::Tensor cache, at::Tensor c_kv, at::Tensor k_pe,
                      at::Tensor slots);
 }  // namespace kaito
 
 TORCH_LIBRARY_FRAGMENT(kaito, m) {
-  m.def("mla_decode(Tensor(a!) out, Tensor q, Tensor cache, Tensor block_tables, Tensor seq_lens, float scale) -> ()");
+  m.def("mla_decode(Tensor(a!) out, Tensor qc, Tensor qr, Tensor cache, Tensor block_tables, Tensor seq_lens, float scale) -> ()");
+  m.def("mla_prepare(Tensor(a!) q_out, Tensor(b!) c_out, Tensor(c!) k_out, Tensor(d!) cache, Tensor q, Tensor kv_a, Tensor w, float eps, Tensor positions, Tensor cos_sin, Tensor slots) -> ()");
   m.def("mla_cache_write(Tensor(a!) cache, Tensor c_kv, Tensor k_pe, Tensor slots) -> ()");
 }
 
 TORCH_LIBRARY_IMPL(kaito, CUDA, m) {
   m.impl("mla_decode", &kaito::mla_decode);
+  m.impl("mla_prepare", &kaito::mla_prepare);
   m.impl("mla_cache_write", &kaito::mla_cache_write);
 }

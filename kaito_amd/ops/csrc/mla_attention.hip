@@ -1,609 +1,519 @@
-// MLA (multi-head latent attention) DECODE kernel for gfx950 (MI355X).
+// MLA (multi-head latent attention) for gfx950: DECODE over the paged cache
+// and what precedes attention in a layer.
 //
-// DeepSeek V2/V3/R1 absorbed decode (models/mla.py): one compressed
-// latent row per cached token — c_kv[R=512] ‖ k_rope[P=64], 576 bf16 —
-// shared by EVERY head. Replaces the vLLM MLA backend the reference
-// delegates to for the deepseek presets (SURVEY.md §2.3,
-// supported_models.yaml deepseek-v3-0324 / deepseek-r1-0528).
+// Absorbed decode of DeepSeek V2/V3/R1 (models/mla.py): one latent row per
+// cached token, c_kv[R = 512] | k_rope[P = 64], shared by every head. With
+// q_c = W_uk^T q_nope, scores[h][t] = (q_c | q_rope)[h] . row[t] and
+// out[h] = sum_t softmax * row[t][0:R]. Stands for the vLLM MLA backend that
+// the reference hands the deepseek presets to (supported_models.yaml:
+// deepseek-v3-0324, deepseek-r1-0528).
 //
-// Shape: scores[h][t] = q_latent[h]·cache[t] (the full 576-dot — rope
-// term included by construction), out[h] = Σ_t softmax·c_kv[t][0:512].
-// Compared with GQA decode (paged_attention_sp.hip) the arithmetic
-// intensity is ~16 heads × 2 dots per byte, so the kernel is organized
-// around HBM-byte REUSE, not pure streaming:
+// mla_decode_kernel: a workgroup of 1 to 4 waves per (sequence, 16 heads, split of
+// the keys); 16 heads fill the columns of v_mfma_f32_16x16x32_bf16. Every
+// wave walks its own keys, 32 at a time, without a barrier:
+//   - two pages (18 KB each, contiguous) go to the wave's LDS by 16-byte
+//     direct loads, the chunk order of a row exclusive-ored with its number,
+//     so that both ways to read it spread over the banks;
+//   - S^T = C Q^T reads 16-byte chunks of rows; a head's scores sit in one
+//     column, so maximum and rescale are per-lane scalars;
+//   - O^T += C^T P^T takes P (bf16) from the score registers and reads the
+//     same rows again, transposed, as columns: the cache row serves as key
+//     and as value from one load.
+// The waves' (max, sum, O) are folded through LDS, the splits' by
+// mla_fold_kernel.
 //
-//   * grid (seq, head-tile of 16); each 256-thread workgroup stages one
-//     16-token KV block (18 KB) into LDS cooperatively, then all 16
-//     heads consume it — every HBM byte is read ONCE per tile. At
-//     deepseek-v3 TP=8 each rank holds exactly 16 heads = one tile;
-//     V2-Lite (16 heads) is one tile at TP=1.
-//   * score phase: lane = (head&3)<<4 | slice, 4 heads per wave; each
-//     lane dots a 36-dim slice (9 × b64 LDS reads, bf16 v_dot2) and the
-//     16 slice-lanes shfl-reduce. The 4 same-slice lanes read the same
-//     LDS address → broadcast, conflict-free.
-//   * online softmax per block: per-head running (M, l) and the
-//     accumulator rescale, amortized over 16 heads × 512 dims (the
-//     per-block rescale is ~6% of the accumulate FLOPs — cheap here,
-//     unlike the GQA kernel where it forced the split-phase design).
-//   * accumulate phase: thread (head = tid>>4, dim-slice = tid&15)
-//     carries 32 f32 accumulator registers; p broadcasts from LDS.
-//   * all LDS handoffs except the staging barrier are intra-wave
-//     (score→exp→accumulate stay inside the head's own wave), so each
-//     block iteration needs only TWO __syncthreads.
+// What bounds it: bytes in flight. A tile costs a CU 68 KB of LDS reads (550
+// cycles) and 70 matrix instructions on one of four SIMDs for 36 KB of cache,
+// far less than HBM takes for it (2900 cycles at 13 B per CU and cycle), so
+// LDS is spent on loads under way: 4 x 36 KB per CU. Measured on one MI355X
+// against 16-token blocks staged by 256 threads through registers behind two
+// barriers, with V transposed by scalar LDS stores (before -> now, 16 heads):
+//   1 sequence of 512 tokens: 28 -> 14 us;  32 of 1800: 65 -> 26;
+//   256 of 400: 77 -> 30;  2048 of 300: 351 -> 160 (4.4 TB/s);
+//   128 heads, 250 of 300: 352 -> 82 us.
 //
-// Cache layout: [num_blocks, BLOCK_SIZE=16, R+P] bf16 (the aliased
-// (c, c) pair from model_runner.profile_and_allocate_kv).
-//
-// Known limit: grid = T × ceil(H/16) — below ~512 concurrent sequences
-// the launch underfills 256 CUs; a flash-decoding token-split tier is
-// the designated fix (docs/ROADMAP.md).
-#include "common.h"
+// Cache layout: [num_blocks, 16, R + P] bf16.
+#include "flash_prefill.h"
 #include <algorithm>
-#include <cstdlib>
 #include <torch/library.h>
 #include <ATen/ATen.h>
 #include <ATen/hip/HIPContext.h>
 
 namespace kaito {
 
-typedef short short4_t __attribute__((ext_vector_type(4)));
+namespace {
 
-// OCC: workgroups/CU. LDS (19.3 KB/wg) allows 8; VGPRs decide the
-// real bound — selectable via KAITO_MLA_OCC for A/B on hardware.
-// DB: software double-buffer THROUGH REGISTERS — the next block's
-// global loads (5 x b128 per thread) issue before the current block's
-// compute, hiding the HBM latency the single-buffer stage exposes at
-// every __syncthreads; LDS footprint unchanged (KAITO_MLA_DB).
-// PH: diagnostic phase mask (1 = stage only, 2 = +scores, 3 = full) —
-// timing ablation via KAITO_MLA_PH; output is garbage for PH<3.
-// MF: MFMA score phase — C[16h x 16t] via mfma_f32_16x16x32_bf16 with
-// the 18 K-steps split 4/5/4/5 across the 4 waves (partials reduced
-// through LDS), Q K-range PRELOADED per wave (Q is block-invariant),
-// s_kv rows padded +16 B so B-fragment b128 reads hit the 2-cycle
-// LDS minimum instead of a 16-way bank conflict (KAITO_MLA_MF).
-// MV: MFMA V-accumulate — out[16h x 512d] += P[16h x 16t(+16 zero-pad
-// k)] @ C_kv[16t x 512d] via 8 d-tiles per wave; V staged TRANSPOSED
-// (s_vt[dim][token]) during the cooperative copy so B-fragments are
-// contiguous b128 reads (same trick as prefill_attention); requires MF.
-// SP: flash-decoding token-split — blockIdx.z picks a contiguous
-// partition of the KV blocks; each split writes UN-normalized partials
-// (acc, M, l) to scratch and mla_merge_kernel combines them. Fills the
-// 256-CU chip when T x head-tiles alone can't (docs/ROADMAP.md).
-template <int R, int P, int BS, int OCC = 4, bool DB = false, int PH = 3,
-          bool MF = false, bool MV = false, bool SP = false>
-__global__ __launch_bounds__(256, OCC)
-void mla_decode_kernel(
-    short* __restrict__ out,            // [T, H, R] bf16
-    const short* __restrict__ q,        // [T, H, R+P] bf16
-    const short* __restrict__ cache,    // [NB, BS, R+P] bf16
-    const int* __restrict__ block_tables,  // [T, max_blocks]
-    const int* __restrict__ seq_lens,   // [T]
-    const float scale, const int H, const int max_blocks,
-    float* __restrict__ part_acc = nullptr,   // [T, S, 16, R]
-    float* __restrict__ part_ml = nullptr,    // [T, S, 16, 2]
-    const int S = 1) {
-  constexpr int DT = R + P;             // 576
-  constexpr int SL = DT / 16;           // 36 dims per score slice
-  constexpr int AD = R / 16;            // 32 dims per accum slice
-  constexpr int HT = 16;                // heads per workgroup
-  static_assert(DT % 16 == 0 && R % 16 == 0 && SL % 12 == 0
-                && AD % 8 == 0);
+using flash::hbf16x8;
+using flash::LOG2E;
 
-  const int seq = blockIdx.x;
-  const int h0 = blockIdx.y * HT;
-  const int split = SP ? blockIdx.z : 0;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int seq_len = seq_lens[seq];
-  const int nb_all = (seq_len + BS - 1) / BS;
-  const int b_lo = SP ? (nb_all * split) / S : 0;
-  const int nblocks = SP ? (nb_all * (split + 1)) / S : nb_all;
-  const int* bt = block_tables + (int64_t)seq * max_blocks;
+constexpr int R = 512, P = 64, DT = R + P;
+constexpr int BS = 16;              // tokens per page
+constexpr int KT = 32;              // keys per wave step: two pages
+constexpr int WIDE = 4;             // waves whose rows fill the LDS
+constexpr int HT = 16;              // heads per workgroup
+constexpr int RS = R + 4;           // floats per head in the fold
 
-  // score-phase role: 4 heads per wave, 16 dim-slices per head
-  const int sc_head = wave * 4 + (lane >> 4);     // 0..15 == tid>>4
-  const int slice = lane & 15;
-  // accum/exp-phase role (same head): dim/token slice
-  const int ac_h = tid >> 4;                      // == sc_head
-  const int ac_s = tid & 15;
+struct MlaArgs {
+  short* out;                       // [T, H, R]
+  const short* qc;                  // q in the latent space: t, h strides
+  const short* qr;                  // its rotated part
+  int64_t qc_ts, qc_hs, qr_ts, qr_hs;
+  const short* cache;
+  const int* block_tables;          // [T, max_blocks]
+  const int* seq_lens;              // [T]
+  float scale;
+  int T, H, max_blocks;
+  float* part;                      // splits: [splits, T, H, R]
+  float* ml;                        // splits: [splits, T, H, 2] max, sum
+};
 
-  constexpr int RS = MF ? DT + 8 : DT;   // padded row (bank spread)
-  constexpr int TP = 20;                 // s_vt token stride (16+4 pad)
-  __shared__ short s_kv[BS * RS];                 // staged block
-  __shared__ float s_p[BS][HT];                   // scores→probs
-  __shared__ float s_part[MF ? 4 : 1][HT][HT];    // per-wave C partials
-  __shared__ short s_vt[MV ? R * TP : 1];         // V transposed (20.5KB)
-  __shared__ short s_pb[MV ? HT : 1][TP];         // P row-major bf16
-  __shared__ float s_corr[HT], s_l[HT];
-  __shared__ float s_M2[SP ? HT : 1];             // running max (splits)
+// Workgroup id -> (sequence, head tile). Ids go round the 8 dies, each with
+// its own L2: the tiles of a sequence, which read the same rows, share one.
+KAITO_DEV int seq_of(int id, int tiles) {
+  return id / (8 * tiles) * 8 + id % 8;
+}
 
-  // per-head online-softmax state, held REDUNDANTLY in registers by all
-  // 16 lanes of the head's thread group (every lane derives identical
-  // values from the same shfl reductions) — no cross-lane LDS handoff
-  float M = -1e30f, l = 0.f;
+template <int NW, bool SPLIT>
+__global__ __launch_bounds__(NW * 64)
+__attribute__((amdgpu_waves_per_eu(1, 1)))
+void mla_decode_kernel(const MlaArgs a) {
+  constexpr int LP = BS * DT / 8 / 64;      // loads per lane and page: 18
+  constexpr int KK = DT / 32, OT = R / 16, KB = 3;
+  __shared__ __attribute__((aligned(128))) short lds[NW][KT * DT];
+  __shared__ float s_m[NW][HT], s_l[NW][HT];
+  static_assert(sizeof(lds) >= NW * HT * RS * sizeof(float), "fold");
+  const int tiles_h = (a.H + HT - 1) / HT;
+  const int seq = seq_of(blockIdx.x, tiles_h);
+  const int h0 = blockIdx.x / 8 % tiles_h * HT;
+  if (seq >= a.T) return;           // the last 8 sequences may be fewer
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lo = lane & 15, hi = lane >> 4;
+  const int seq_len = a.seq_lens[seq];
+  const int* bt = a.block_tables + (int64_t)seq * a.max_blocks;
 
-  constexpr int KSTEPS = DT / 32;                 // MFMA K-chunks (18)
-  constexpr int KW = (KSTEPS + 3) / 4 + 1;        // per-wave upper bound
-  const int kb0 = (KSTEPS * wave) / 4;            // ragged 4/5/4/5 split
-  const int kb1 = (KSTEPS * (wave + 1)) / 4;
-  const int hi = lane >> 4;
-
-  // q for the score phase; zero for padded heads so their scores stay
-  // finite (their output is never written). Rows are CLAMPED (not just
-  // the value) so an if-converted load can't read past the q tensor.
-  short4_t qv[MF ? 1 : SL / 4];
-  bf16x8 af[MF ? KW : 1];
-  if constexpr (MF) {
-    // A-fragment rows: head = lane&15; k = kc*32 + (lane>>4)*8 + [0..7]
-    const bool ok = h0 + (lane & 15) < H;
-    const int hq = min(h0 + (lane & 15), H - 1);
-    const short* qp = q + ((int64_t)seq * H + hq) * DT;
-#pragma unroll
-    for (int j = 0; j < KW; j++) {
-      if (kb0 + j >= kb1) break;
-      af[j] = *reinterpret_cast<const bf16x8*>(
-          qp + (kb0 + j) * 32 + hi * 8);
-      if (!ok) af[j] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-    }
-  } else {
-    const bool head_ok = h0 + sc_head < H;
-    const int hq = min(h0 + sc_head, H - 1);
-    const short* qp = q + ((int64_t)seq * H + hq) * DT + slice * SL;
-#pragma unroll
-    for (int j = 0; j < SL / 4; j++) {
-      qv[j] = *reinterpret_cast<const short4_t*>(qp + j * 4);
-      if (!head_ok) qv[j] = short4_t{0, 0, 0, 0};
+  const int tiles = (seq_len + KT - 1) / KT;
+  const int nsplit = SPLIT ? gridDim.y : 1, split = SPLIT ? blockIdx.y : 0;
+  const int per = (tiles + nsplit * NW - 1) / (nsplit * NW);
+  const int t0 = min(tiles, (split * NW + wave) * per);
+  const int t1 = min(tiles, t0 + per);
+  const int last_page = (seq_len - 1) / BS;
+  if constexpr (SPLIT) {
+    if (split * NW * per >= tiles) {        // nothing for any of the waves
+      if (threadIdx.x < HT && h0 + (int)threadIdx.x < a.H) {
+        float* ml = a.ml +
+            (((int64_t)split * a.T + seq) * a.H + h0 + threadIdx.x) * 2;
+        ml[0] = -1e30f;
+        ml[1] = 0.f;
+      }
+      return;
     }
   }
 
-  float acc[MV ? 1 : AD];
-  f32x4 accv[MV ? 8 : 1];
-  if constexpr (MV) {
+  hbf16x8 qf[KK];
+  {
+    const int h = min(h0 + lo, a.H - 1);
+    const short* qc = a.qc + seq * a.qc_ts + h * a.qc_hs + hi * 8;
+    const short* qr = a.qr + seq * a.qr_ts + h * a.qr_hs + hi * 8;
 #pragma unroll
-    for (int j = 0; j < 8; j++) accv[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  } else {
+    for (int kk = 0; kk < KK; kk++)
+      qf[kk] = *reinterpret_cast<const hbf16x8*>(
+          kk < R / 32 ? qc + kk * 32 : qr + (kk - R / 32) * 32);
+  }
+  float m = -1e30f, l = 0.f;
+  f32x4 o[OT];
 #pragma unroll
-    for (int j = 0; j < AD; j++) acc[j] = 0.f;
+  for (int i = 0; i < OT; i++) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  short* const st = lds[wave];
+  // chunk c of row r lies at place c ^ (r / 2 % 8); 72 chunks a row, so the
+  // low three bits stay in the row
+  uint32_t off[LP / 2];             // the other 8 rows of a page: off ^ 32
+#pragma unroll
+  for (int j = 0; j < LP / 2; j++) {
+    const uint32_t s = j * 64 + lane;
+    off[j] = (s ^ (s / (DT / 8) >> 1 & 7)) * 8;
+  }
+  const short* kp[2];                       // even and odd 32-dim steps
+#pragma unroll
+  for (int e = 0; e < 2; e++)
+    kp[e] = st + lo * DT + ((e * 4 + hi) ^ (lo >> 1 & 7)) * 8;
+  const int vrow = 4 * hi + (lo >> 2), vc = (lo & 3) >> 1, ve = (lo & 1) * 4;
+  const short* vp[4];
+#pragma unroll
+  for (int e = 0; e < 4; e++)
+    vp[e] = st + vrow * DT + ((e * 2 + vc) ^ (vrow >> 1 & 7)) * 8 + ve;
+  const float c = a.scale * LOG2E;
+
+  int pages = 0, pages_at = -64;    // lane i: page pages_at + i of the table
+  for (int t = t0; t < t1; t++) {
+    // the pages of a tile are even and odd: one test serves both
+    if (t * 2 >= pages_at + 64) {           // uniform; spans move forward
+      pages_at = t * 2;
+      pages = bt[min(t * 2 + lane, last_page)];
+    }
+    const short* src[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+      src[i] = a.cache + (int64_t)__builtin_amdgcn_readlane(
+          pages, t * 2 + i - pages_at) * BS * DT;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < LP; j++)
+        flash::lds_copy16(
+            src[i] + (j < LP / 2 ? off[j] : (off[j - LP / 2] ^ 32) + 8 * DT),
+            st + (i * LP + j) * 512);
+    __builtin_amdgcn_s_waitcnt(0x0f70);     // vmcnt(0): this wave's own rows
+    __builtin_amdgcn_wave_barrier();
+    // ---- S^T: keys 16 i + 4 hi + r of head lo
+    f32x4 s[2][2];
+    hbf16x8 kf[2][KB][2];           // a batch of steps and the next one's
+    auto read_k = [&](const int b) {
+#pragma unroll
+      for (int kk = 0; kk < KB; kk++)
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+          kf[b & 1][kk][i] = *reinterpret_cast<const hbf16x8*>(
+              kp[(b * KB + kk) & 1] + i * BS * DT + (b * KB + kk) / 2 * 64);
+      __builtin_amdgcn_sched_barrier(0);    // all under way before products
+    };
+    read_k(0);
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+      s[i][0] = s[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int b = 0; b < KK / KB; b++) {
+      if (b + 1 < KK / KB) read_k(b + 1);
+#pragma unroll
+      for (int kk = 0; kk < KB; kk++)
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+          s[i][kk & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              kf[b & 1][kk][i], qf[b * KB + kk], s[i][kk & 1], 0, 0, 0);
+    }
+    s[0][0] += s[0][1];
+    s[1][0] += s[1][1];
+    // ---- softmax
+    const int key0 = t * KT;
+    const bool whole = key0 + KT <= seq_len;
+    float mx = -1e30f;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        s[i][0][r] *= c;
+        if (!whole && key0 + 16 * i + 4 * hi + r >= seq_len)
+          s[i][0][r] = -1e30f;
+        mx = fmaxf(mx, s[i][0][r]);
+      }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if (__any(mx > m)) {
+      const float mn = fmaxf(m, mx);
+      const float corr = __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      l *= corr;
+#pragma unroll
+      for (int i = 0; i < OT; i++) o[i] *= corr;
+    }
+    hbf16x8 p;
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const float w = s[i][0][r] > -1e29f
+            ? __builtin_amdgcn_exp2f(s[i][0][r] - m) : 0.f;
+        l += w;
+        p[i * 4 + r] = (__bf16)w;
+      }
+    // ---- O^T: dims 16 i + 4 hi + r of head lo
+#pragma unroll
+    for (int i = 0; i < OT; i++) {
+      const short* at = vp[i & 3] + i / 4 * 64;
+      const short4_t a4 = flash::read_tr(at), b4 = flash::read_tr(at + BS * DT);
+      const hbf16x8 vf = __builtin_bit_cast(
+          hbf16x8, __builtin_shufflevector(a4, b4, 0, 1, 2, 3, 4, 5, 6, 7));
+      o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p, o[i], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x100, 16, 1);
+#pragma unroll
+    for (int i = 0; i < OT - 8; i++) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 1);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, 8, 1);
+    __builtin_amdgcn_wave_barrier();        // rows read before the next ones
   }
 
-  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-
-  constexpr int NCH = (BS * DT / 8 + 255) / 256;   // b128 chunks/thread
-  short8_t pf[DB ? NCH : 1];
-  if constexpr (DB) {   // prologue: first block's loads in flight
-    const short8_t* src = reinterpret_cast<const short8_t*>(
-        cache + (int64_t)bt[b_lo] * (BS * DT));
+  // ---- fold the waves through LDS
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  float* const acc = reinterpret_cast<float*>(&lds[0][0]);
+  __syncthreads();                  // every wave is done with its rows
 #pragma unroll
-    for (int c = 0; c < NCH; c++) {
-      const int idx = c * 256 + tid;
-      if (idx < BS * DT / 8) pf[c] = src[idx];
-    }
-  }
-
-  for (int b = b_lo; b < nblocks; b++) {
-    // ---- stage one KV block: 1152 x b128, 256 threads ----
-    if constexpr (DB) {
-#pragma unroll
-      for (int c = 0; c < NCH; c++) {
-        const int idx = c * 256 + tid;
-        if (idx < BS * DT / 8) {
-          *reinterpret_cast<short8_t*>(
-              s_kv + (idx / (DT / 8)) * RS + (idx % (DT / 8)) * 8) = pf[c];
-          if constexpr (MV) {
-            const int tok = idx / (DT / 8);
-            const int d0 = (idx % (DT / 8)) * 8;
-            if (d0 < R) {
-#pragma unroll
-              for (int j = 0; j < 8; j++)
-                s_vt[(d0 + j) * TP + tok] = pf[c][j];
-            }
-          }
-        }
-      }
-    } else {
-      const short8_t* src = reinterpret_cast<const short8_t*>(
-          cache + (int64_t)bt[b] * (BS * DT));
-#pragma unroll
-      for (int c = 0; c < NCH; c++) {
-        const int idx = c * 256 + tid;
-        if (idx < BS * DT / 8)
-          *reinterpret_cast<short8_t*>(
-              s_kv + (idx / (DT / 8)) * RS + (idx % (DT / 8)) * 8) =
-              src[idx];
-      }
-    }
-    __syncthreads();
-    if constexpr (DB) {   // issue NEXT block's loads before computing
-      if (b + 1 < nblocks) {
-        const short8_t* src = reinterpret_cast<const short8_t*>(
-            cache + (int64_t)bt[b + 1] * (BS * DT));
-#pragma unroll
-        for (int c = 0; c < NCH; c++) {
-          const int idx = c * 256 + tid;
-          if (idx < BS * DT / 8) pf[c] = src[idx];
-        }
-      }
-    }
-
-    // ---- scores for the 16 tokens (intra-wave handoff to exp) ----
-    // 3 independent dot accumulators per token + 2-token unroll: the
-    // naive single-accumulator form is an 18-deep serial v_dot2 chain
-    // (~170 dependent cycles/token) that stalls the SIMD
-    if constexpr (MF) {
-      f32x4 cp = {0.f, 0.f, 0.f, 0.f};
-      const int tcol = lane & 15;
-#pragma unroll
-      for (int j = 0; j < KW; j++) {
-        if (kb0 + j >= kb1) break;
-        const bf16x8 bfr = *reinterpret_cast<const bf16x8*>(
-            s_kv + tcol * RS + (kb0 + j) * 32 + hi * 8);
-        cp = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[j], bfr, cp,
-                                                     0, 0, 0);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; r++)
-        s_part[wave][hi * 4 + r][tcol] = cp[r];
-      __syncthreads();                 // cross-wave partial handoff
-    } else if constexpr (PH >= 2) {
+  for (int i = 0; i < OT; i++)
+    *reinterpret_cast<f32x4*>(acc + (wave * HT + lo) * RS + i * 16 + hi * 4) =
+        o[i];
+  if (hi == 0) { s_m[wave][lo] = m; s_l[wave][lo] = l; }
+  __syncthreads();
 #pragma unroll 2
-    for (int t = 0; t < BS; t++) {
-      const short* kp = s_kv + t * RS + slice * SL;
-      float p0 = 0.f, p1 = 0.f, p2 = 0.f;
+  for (int idx = threadIdx.x; idx < HT * R / 4; idx += NW * 64) {
+    const int g = idx / (R / 4), d = idx % (R / 4) * 4;
+    if (h0 + g >= a.H) break;
+    float gm = -1e30f, den = 0.f;
 #pragma unroll
-      for (int j = 0; j < SL / 12; j++) {
-        const short4_t a = *reinterpret_cast<const short4_t*>(kp + j * 12);
-        const short4_t bq = *reinterpret_cast<const short4_t*>(
-            kp + j * 12 + 4);
-        const short4_t c = *reinterpret_cast<const short4_t*>(
-            kp + j * 12 + 8);
-        const bf16x2_t* ka = reinterpret_cast<const bf16x2_t*>(&a);
-        const bf16x2_t* kb = reinterpret_cast<const bf16x2_t*>(&bq);
-        const bf16x2_t* kc = reinterpret_cast<const bf16x2_t*>(&c);
-        const bf16x2_t* qa = reinterpret_cast<const bf16x2_t*>(
-            &qv[j * 3]);
-        const bf16x2_t* qb = reinterpret_cast<const bf16x2_t*>(
-            &qv[j * 3 + 1]);
-        const bf16x2_t* qc = reinterpret_cast<const bf16x2_t*>(
-            &qv[j * 3 + 2]);
-        p0 = __builtin_amdgcn_fdot2_f32_bf16(qa[0], ka[0], p0, false);
-        p1 = __builtin_amdgcn_fdot2_f32_bf16(qb[0], kb[0], p1, false);
-        p2 = __builtin_amdgcn_fdot2_f32_bf16(qc[0], kc[0], p2, false);
-        p0 = __builtin_amdgcn_fdot2_f32_bf16(qa[1], ka[1], p0, false);
-        p1 = __builtin_amdgcn_fdot2_f32_bf16(qb[1], kb[1], p1, false);
-        p2 = __builtin_amdgcn_fdot2_f32_bf16(qc[1], kc[1], p2, false);
-      }
-      float part = (p0 + p1) + p2;
+    for (int w = 0; w < NW; w++) gm = fmaxf(gm, s_m[w][g]);
+    f32x4 num{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int off = 1; off < 16; off <<= 1)
-        part += __shfl_xor(part, off, 64);
-      if (slice == 0) {
-        const bool valid = b * BS + t < seq_len;
-        s_p[t][sc_head] = valid ? part * scale : -1e30f;
-      }
+    for (int w = 0; w < NW; w++) {
+      const float e = __builtin_amdgcn_exp2f(s_m[w][g] - gm);
+      num += e * *reinterpret_cast<const f32x4*>(acc + (w * HT + g) * RS + d);
+      den += e * s_l[w][g];
     }
+    const int64_t row = ((int64_t)split * a.T + seq) * a.H + h0 + g;
+    if constexpr (SPLIT) {
+      *reinterpret_cast<f32x4*>(a.part + row * R + d) = num;
+      if (d == 0) { a.ml[row * 2] = gm; a.ml[row * 2 + 1] = den; }
+    } else {
+      const float inv = 1.f / fmaxf(den, 1e-20f);
+      short4_t v;
+#pragma unroll
+      for (int r = 0; r < 4; r++) v[r] = f32_to_bf16(num[r] * inv);
+      *reinterpret_cast<short4_t*>(a.out + row * R + d) = v;
     }
-
-    // ---- online softmax update (thread (h, t); state in registers) ----
-    float corr = 1.f;
-    if constexpr (PH >= 3) {
-      const int t = ac_s;
-      float s;
-      if constexpr (MF) {
-        s = ((s_part[0][ac_h][t] + s_part[1][ac_h][t])
-             + (s_part[2][ac_h][t] + s_part[3][ac_h][t])) * scale;
-        if (b * BS + t >= seq_len) s = -1e30f;
-      } else {
-        s = s_p[t][ac_h];
-      }
-      float bm = s;
-#pragma unroll
-      for (int off = 1; off < 16; off <<= 1)
-        bm = fmaxf(bm, __shfl_xor(bm, off, 64));
-      const float Mnew = fmaxf(M, bm);
-      const float p = s > -1e29f ? __expf(s - Mnew) : 0.f;
-      float bsum = p;
-#pragma unroll
-      for (int off = 1; off < 16; off <<= 1)
-        bsum += __shfl_xor(bsum, off, 64);
-      s_p[t][ac_h] = p;
-      corr = Mnew > M ? __expf(M - Mnew) : 1.f;
-      l = l * corr + bsum;
-      M = Mnew;
-      if constexpr (MV) {
-        s_pb[ac_h][t] = f32_to_bf16(p);
-        if (t == 0) {
-          s_corr[ac_h] = corr;
-          s_l[ac_h] = l;
-          if constexpr (SP) s_M2[ac_h] = M;
-        }
-      }
-    }
-    if constexpr (MV) __syncthreads();   // s_pb/s_corr to all waves
-
-    // ---- accumulate c_kv into the latent-space output ----
-    if constexpr (MV) {
-      // rescale C fragments: row hi*4+r is head hi*4+r
-      float cr[4];
-#pragma unroll
-      for (int r = 0; r < 4; r++) cr[r] = s_corr[hi * 4 + r];
-#pragma unroll
-      for (int j = 0; j < 8; j++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) accv[j][r] *= cr[r];
-      const int tok0 = (hi & 1) * 8;    // hi>=2: A is zero, B ignored
-      const bf16x8 pa = hi < 2
-          ? *reinterpret_cast<const bf16x8*>(&s_pb[lane & 15][hi * 8])
-          : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-      for (int j = 0; j < 8; j++) {     // 8 dim-tiles per wave
-        const int dim = (wave * 8 + j) * 16 + (lane & 15);
-        const bf16x8 vb = *reinterpret_cast<const bf16x8*>(
-            &s_vt[dim * TP + tok0]);
-        accv[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, vb, accv[j],
-                                                          0, 0, 0);
-      }
-    } else if constexpr (PH >= 3) {
-      float2_t* a2 = reinterpret_cast<float2_t*>(acc);
-      const float2_t corr2 = {corr, corr};
-#pragma unroll
-      for (int j = 0; j < AD / 2; j++) a2[j] *= corr2;
-      for (int t = 0; t < BS; t++) {
-        const float p = s_p[t][ac_h];
-        const float2_t p2 = {p, p};
-        const short* vp = s_kv + t * RS + ac_s * AD;
-#pragma unroll
-        for (int c = 0; c < AD / 8; c++) {
-          const short8_t v8 = *reinterpret_cast<const short8_t*>(vp + c * 8);
-          float vreg[8];
-#pragma unroll
-          for (int j = 0; j < 8; j++) vreg[j] = bf16_to_f32(v8[j]);
-          const float2_t* v2 = reinterpret_cast<const float2_t*>(vreg);
-#pragma unroll
-          for (int k = 0; k < 4; k++) a2[c * 4 + k] += p2 * v2[k];
-        }
-      }
-    }
-    __syncthreads();   // s_kv free for the next block's staging
-  }
-
-  if constexpr (PH < 3) {
-    // ablation variants: fake consumer keeps the staging/score stores
-    // alive (never taken at runtime — seq_len >= 1)
-    if (seq_len < 0)
-      out[tid] = s_kv[tid] + (short)s_p[tid & 15][tid >> 4];
-    return;
-  }
-
-  if constexpr (SP) {
-    // split partials: UN-normalized latent acc + (M, l) per head; the
-    // merge kernel rescales across splits. Empty split (b_lo >=
-    // nblocks, short sequences) contributes exp(-1e30)=0.
-    const bool empty = b_lo >= nblocks;
-    const int HTOT = gridDim.y * HT;     // scratch covers ALL head tiles
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const int dim = (wave * 8 + j) * 16 + (lane & 15);
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int h = hi * 4 + r;
-        part_acc[(((int64_t)seq * S + split) * HTOT + h0 + h) * R + dim] =
-            accv[j][r];
-      }
-    }
-    if (wave == 0 && (lane & 15) == 0) {
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int h = hi * 4 + r;
-        float* ml = part_ml
-            + (((int64_t)seq * S + split) * HTOT + h0 + h) * 2;
-        ml[0] = empty ? -1e30f : s_M2[h];
-        ml[1] = empty ? 0.f : s_l[h];
-      }
-    }
-    return;
-  }
-
-  // ---- epilogue: normalize + write [T, H, R] ----
-  if constexpr (MV) {
-    // C-fragment layout: row hi*4+r = head, col = dim-within-tile
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const int dim = (wave * 8 + j) * 16 + (lane & 15);
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int h = hi * 4 + r;
-        if (h0 + h < H)
-          out[((int64_t)seq * H + (h0 + h)) * R + dim] =
-              f32_to_bf16(accv[j][r] / fmaxf(s_l[h], 1e-20f));
-      }
-    }
-    return;
-  }
-  if (h0 + ac_h < H) {
-    const float inv = 1.f / fmaxf(l, 1e-20f);
-    short* op = out + ((int64_t)seq * H + (h0 + ac_h)) * R + ac_s * AD;
-#pragma unroll
-    for (int j = 0; j < AD; j++) op[j] = f32_to_bf16(acc[j] * inv);
   }
 }
 
-// Combine flash-decoding split partials: out[h] = sum_s w_s*acc_s /
-// sum_s w_s*l_s with w_s = exp(M_s - max M). Thread (head = tid>>4,
-// dim-slice = tid&15) mirrors the main kernel's accum layout.
-template <int R>
-__global__ __launch_bounds__(256, 8)
-void mla_merge_kernel(short* __restrict__ out,
-                      const float* __restrict__ part_acc,
-                      const float* __restrict__ part_ml,
-                      const int H, const int S) {
-  constexpr int HT = 16;
-  constexpr int AD = R / 16;
-  const int seq = blockIdx.x;
-  const int h = (int)(threadIdx.x >> 4) + blockIdx.y * HT;
-  const int ds = threadIdx.x & 15;
-  if (h >= H) return;
-  const int HTOT = gridDim.y * HT;
-  const int64_t base = (int64_t)seq * S;
-  float gm = -1e30f;
-  for (int sp = 0; sp < S; sp++)
-    gm = fmaxf(gm, part_ml[((base + sp) * HTOT + h) * 2]);
-  float den = 0.f;
-  float num[AD];
-#pragma unroll
-  for (int j = 0; j < AD; j++) num[j] = 0.f;
-  for (int sp = 0; sp < S; sp++) {
-    const float* ml = part_ml + ((base + sp) * HTOT + h) * 2;
-    const float w = __expf(ml[0] - gm);
-    den += w * ml[1];
-    const float* pa = part_acc + ((base + sp) * HTOT + h) * R + ds * AD;
-#pragma unroll
-    for (int j = 0; j < AD; j++) num[j] += w * pa[j];
+// One workgroup per (sequence, head) folds the splits, up to 64; empty ones
+// (no key) hold a maximum and no row. A chain of loads, so short ones: lane s
+// of every wave has split s's weight, 4 groups of 2 waves take every 4th row.
+__global__ __launch_bounds__(R)
+void mla_fold_kernel(short* __restrict__ out, const float* __restrict__ part,
+                     const float* __restrict__ ml, const int splits) {
+  __shared__ f32x4 red[4][R / 4];
+  const int64_t row = blockIdx.x, rows = gridDim.x;
+  const int lane = threadIdx.x & 63;
+  const int group = __builtin_amdgcn_readfirstlane(threadIdx.x / (R / 4));
+  const int col = threadIdx.x % (R / 4);
+  float m = -1e30f, l = 0.f;
+  if (lane < splits) {
+    const float2 v = reinterpret_cast<const float2*>(ml)[lane * rows + row];
+    m = v.x;
+    l = v.y;
   }
+  float gm = m;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) gm = fmaxf(gm, __shfl_xor(gm, d, 64));
+  const float e = m > -1e29f ? __builtin_amdgcn_exp2f(m - gm) : 0.f;
+  float den = e * l;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) den += __shfl_xor(den, d, 64);
+  f32x4 num{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int s = group; s < splits; s += 4) {
+    const float w = __builtin_bit_cast(
+        float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, e), s));
+    if (w == 0.f) continue;
+    num += w * *reinterpret_cast<const f32x4*>(part + (s * rows + row) * R +
+                                               col * 4);
+  }
+  red[group][col] = num;
+  __syncthreads();
+  if (group > 0) return;
+  num += red[1][col] + red[2][col] + red[3][col];
   const float inv = 1.f / fmaxf(den, 1e-20f);
-  short* op = out + ((int64_t)seq * H + h) * R + ds * AD;
+  short4_t v;
 #pragma unroll
-  for (int j = 0; j < AD; j++) op[j] = f32_to_bf16(num[j] * inv);
+  for (int r = 0; r < 4; r++) v[r] = f32_to_bf16(num[r] * inv);
+  *reinterpret_cast<short4_t*>(out + row * R + col * 4) = v;
 }
 
-void mla_decode(at::Tensor out, at::Tensor q, at::Tensor cache,
+}  // namespace
+
+// qc [T, H, R] and qr [T, H, P] of any token and head stride
+void mla_decode(at::Tensor out, at::Tensor qc, at::Tensor qr, at::Tensor cache,
                 at::Tensor block_tables, at::Tensor seq_lens, double scale) {
-  TORCH_CHECK(q.is_cuda() && q.dtype() == at::kBFloat16 && q.is_contiguous());
+  auto ok = [](const at::Tensor& t) {
+    return t.is_cuda() && t.dtype() == at::kBFloat16 && t.stride(-1) == 1;
+  };
+  TORCH_CHECK(ok(qc) && ok(qr) && qc.dim() == 3 && qr.dim() == 3);
   TORCH_CHECK(cache.dtype() == at::kBFloat16 && cache.is_contiguous());
   TORCH_CHECK(out.is_contiguous() && out.dtype() == at::kBFloat16);
   TORCH_CHECK(block_tables.dtype() == at::kInt
               && seq_lens.dtype() == at::kInt);
-  const int T = q.size(0);
-  const int H = q.size(1);
-  const int DT = q.size(2);
-  const int BS = cache.size(1);
-  const int R = out.size(2);
-  TORCH_CHECK(cache.size(2) == DT && out.size(0) == T && out.size(1) == H);
-  TORCH_CHECK(BS == 16, "block_size must be 16");
-  const int max_blocks = block_tables.size(1);
+  const int T = qc.size(0), H = qc.size(1);
+  TORCH_CHECK(qc.size(2) == R && qr.size(2) == P && out.size(2) == R &&
+              cache.size(2) == DT, "unsupported MLA dims r=", out.size(2),
+              " r+rope=", cache.size(2), " (deepseek family is 512/576)");
+  TORCH_CHECK(qr.size(0) == T && qr.size(1) == H && out.size(0) == T &&
+              out.size(1) == H);
+  TORCH_CHECK(cache.size(1) == BS, "block_size must be 16");
+  if (T == 0 || H == 0) return;
+  MlaArgs a{};
+  a.out = (short*)out.data_ptr();
+  a.qc = (const short*)qc.data_ptr();
+  a.qr = (const short*)qr.data_ptr();
+  a.qc_ts = qc.stride(0); a.qc_hs = qc.stride(1);
+  a.qr_ts = qr.stride(0); a.qr_hs = qr.stride(1);
+  a.cache = (const short*)cache.data_ptr();
+  a.block_tables = block_tables.data_ptr<int>();
+  a.seq_lens = seq_lens.data_ptr<int>();
+  a.scale = (float)scale;
+  a.T = T; a.H = H;
+  a.max_blocks = block_tables.size(1);
   auto stream = at::hip::getCurrentHIPStream();
-  if (T == 0) return;
-  const dim3 grid(T, (H + 15) / 16);
-  static const int occ_env = []() {
-    const char* e = getenv("KAITO_MLA_OCC");
-    return e ? atoi(e) : 0;
-  }();
-  // register double-buffer measured faster at every shape (247.9 vs
-  // 258.8 us bs=768, 183.5 vs 209.7 bs=256) — default ON
-  static const bool db_env = []() {
-    const char* e = getenv("KAITO_MLA_DB");
-    return e == nullptr || atoi(e) != 0;
-  }();
-  if (R == 512 && DT == 576) {
-#define MLA_LAUNCH(OCC_, DB_)                                                 \
-    hipLaunchKernelGGL((mla_decode_kernel<512, 64, 16, OCC_, DB_>), grid,      \
-                       dim3(256), 0, stream, (short*)out.data_ptr(),          \
-                       (const short*)q.data_ptr(),                            \
-                       (const short*)cache.data_ptr(),                        \
-                       block_tables.data_ptr<int>(),                          \
-                       seq_lens.data_ptr<int>(), (float)scale, H, max_blocks)
-    static const int ph_env = []() {
-      const char* e = getenv("KAITO_MLA_PH");
-      return e ? atoi(e) : 3;
-    }();
-    // MFMA scores measured 159 vs 245 us (bs=768), 86 vs 176 (bs=256),
-    // 184 vs 295 (bs=1024) — default ON (KAITO_MLA_MF=0 reverts)
-    static const bool mf_env = []() {
-      const char* e = getenv("KAITO_MLA_MF");
-      return e == nullptr || atoi(e) != 0;
-    }();
-    // MFMA V-accumulate: 139.8 vs 158.7 us (bs=768), equal at bs=1024
-    // — default ON (KAITO_MLA_MV=0 reverts)
-    static const bool mv_env = []() {
-      const char* e = getenv("KAITO_MLA_MV");
-      return e == nullptr || atoi(e) != 0;
-    }();
-    if (ph_env == 1) {
-      hipLaunchKernelGGL((mla_decode_kernel<512, 64, 16, 4, true, 1>), grid,
-                         dim3(256), 0, stream, (short*)out.data_ptr(),
-                         (const short*)q.data_ptr(),
-                         (const short*)cache.data_ptr(),
-                         block_tables.data_ptr<int>(),
-                         seq_lens.data_ptr<int>(), (float)scale, H,
-                         max_blocks);
-    } else if (ph_env == 2) {
-      hipLaunchKernelGGL((mla_decode_kernel<512, 64, 16, 4, true, 2>), grid,
-                         dim3(256), 0, stream, (short*)out.data_ptr(),
-                         (const short*)q.data_ptr(),
-                         (const short*)cache.data_ptr(),
-                         block_tables.data_ptr<int>(),
-                         seq_lens.data_ptr<int>(), (float)scale, H,
-                         max_blocks);
-    } else if (mf_env && mv_env) {
-      // flash-decoding token-split when the plain grid underfills the
-      // 256-CU chip (KAITO_MLA_SPLIT overrides; 0 disables)
-      const int tiles = (H + 15) / 16;
-      int S = 1;
-      const char* se = getenv("KAITO_MLA_SPLIT");
-      if (se != nullptr) {
-        S = atoi(se);
-      } else if (T * tiles < 320) {
-        S = std::min<int>(8, std::max<int>(2, 512 / std::max(T * tiles, 1)));
-      }
-      if (S > 1) {
-        auto opts = at::TensorOptions()
-            .dtype(at::kFloat).device(q.device());
-        at::Tensor pacc = at::empty(
-            {(int64_t)T * S * tiles * 16 * 512}, opts);
-        at::Tensor pml = at::empty({(int64_t)T * S * tiles * 16 * 2}, opts);
-        hipLaunchKernelGGL(
-            (mla_decode_kernel<512, 64, 16, 4, true, 3, true, true, true>),
-            dim3(T, tiles, S), dim3(256), 0, stream,
-            (short*)out.data_ptr(), (const short*)q.data_ptr(),
-            (const short*)cache.data_ptr(), block_tables.data_ptr<int>(),
-            seq_lens.data_ptr<int>(), (float)scale, H, max_blocks,
-            pacc.data_ptr<float>(), pml.data_ptr<float>(), S);
-        hipLaunchKernelGGL((mla_merge_kernel<512>), dim3(T, tiles),
-                           dim3(256), 0, stream, (short*)out.data_ptr(),
-                           pacc.data_ptr<float>(), pml.data_ptr<float>(),
-                           H, S);
-      } else {
-        hipLaunchKernelGGL(
-            (mla_decode_kernel<512, 64, 16, 4, true, 3, true, true>), grid,
-            dim3(256), 0, stream, (short*)out.data_ptr(),
-            (const short*)q.data_ptr(), (const short*)cache.data_ptr(),
-            block_tables.data_ptr<int>(), seq_lens.data_ptr<int>(),
-            (float)scale, H, max_blocks);
-      }
-    } else if (mf_env) {
-      hipLaunchKernelGGL(
-          (mla_decode_kernel<512, 64, 16, 4, true, 3, true>), grid,
-          dim3(256), 0, stream, (short*)out.data_ptr(),
-          (const short*)q.data_ptr(), (const short*)cache.data_ptr(),
-          block_tables.data_ptr<int>(), seq_lens.data_ptr<int>(),
-          (float)scale, H, max_blocks);
-    } else if (db_env) {
-      switch (occ_env) {
-        case 5: MLA_LAUNCH(5, true); break;
-        case 6: MLA_LAUNCH(6, true); break;
-        default: MLA_LAUNCH(4, true); break;
-      }
-    } else {
-      switch (occ_env) {
-        case 5: MLA_LAUNCH(5, false); break;
-        case 6: MLA_LAUNCH(6, false); break;
-        case 8: MLA_LAUNCH(8, false); break;
-        default: MLA_LAUNCH(4, false); break;
-      }
-    }
-#undef MLA_LAUNCH
+  // 4 waves have a CU to themselves: splits until 256 workgroups, as long as
+  // every wave keeps a tile of the longest context that the table can hold
+  // (the lengths are on the device). With more workgroups than CUs, smaller
+  // ones start and fold behind the others' loads: 768 sequences of 300
+  // tokens 72 us with 4 waves, 68 with 2; 2048 193, 169 and 160 with 1.
+  const int tiles_h = (H + HT - 1) / HT;
+  const int64_t grid = (int64_t)(T + 7) / 8 * 8 * tiles_h;
+  const int64_t splits = std::min<int64_t>(
+      {(256 + (int64_t)T * tiles_h - 1) / ((int64_t)T * tiles_h),
+       (int64_t)a.max_blocks * BS / (WIDE * KT), 64});
+  if (splits > 1) {
+    auto opts = out.options().dtype(at::kFloat);
+    at::Tensor part = at::empty({splits, T, H, R}, opts);
+    at::Tensor ml = at::empty({splits, T, H, 2}, opts);
+    a.part = part.data_ptr<float>();
+    a.ml = ml.data_ptr<float>();
+    hipLaunchKernelGGL((mla_decode_kernel<WIDE, true>), dim3(grid, splits),
+                       dim3(WIDE * 64), 0, stream, a);
+    hipLaunchKernelGGL(mla_fold_kernel, dim3(T * H), dim3(R), 0, stream,
+                       a.out, a.part, a.ml, (int)splits);
+  } else if ((int64_t)T * tiles_h <= 512) {
+    hipLaunchKernelGGL((mla_decode_kernel<WIDE, false>), dim3(grid),
+                       dim3(WIDE * 64), 0, stream, a);
+  } else if ((int64_t)T * tiles_h > 1024) {
+    hipLaunchKernelGGL((mla_decode_kernel<1, false>), dim3(grid),
+                       dim3(64), 0, stream, a);
   } else {
-    TORCH_CHECK(false, "unsupported MLA dims r=", R, " r+rope=", DT,
-                " (deepseek family is 512/576)");
+    hipLaunchKernelGGL((mla_decode_kernel<WIDE / 2, false>), dim3(grid),
+                       dim3(WIDE / 2 * 64), 0, stream, a);
   }
 }
 
-// Fused MLA cache write: latent row (c_kv ‖ k_rope) scattered to the
-// paged cache in ONE kernel. Replaces a torch where + cat + index_copy_
-// chain that showed up at ~7% of a v2-lite serving run
-// (profiles/r02_mla_kernels.md). One wave per token: 64 lanes x 16 B
-// covers the 512-dim c_kv; lanes 0-7 append the 64 rope dims.
-template <int R, int P>
+namespace {
+
+// What a layer needs before attention, in one launch per step instead of
+// seven (three copies of strided parts, norm, rotation, cache write; about
+// 4 us each): RMS norm of the latent, rotation of the shared key part and of
+// the queries' rotated parts, scatter into the cache. Bound by the launch for
+// decode steps. Wave 0 of a token's workgroup has the latent (8 dims a lane),
+// the others rotate 8 pairs a lane; norm and rotation round as the single
+// kernels do.
+__global__ __launch_bounds__(256)
+void mla_prepare_kernel(
+    short* __restrict__ q_out,              // [T, H, P]
+    short* __restrict__ c_out,              // [T, R]
+    short* __restrict__ k_out,              // [T, P]
+    short* __restrict__ cache,              // [NB, BS, DT] or nullptr
+    const short* __restrict__ q, const int64_t q_ts, const int64_t q_hs,
+    const short* __restrict__ kv_a, const int64_t kv_ts,
+    const short* __restrict__ w, const float eps,
+    const int64_t* __restrict__ positions,
+    const float* __restrict__ cos_sin,      // [max_pos, P]
+    const int64_t* __restrict__ slots, const int H) {
+  const int64_t t = blockIdx.x;
+  const int tid = threadIdx.x;
+  const int64_t slot = cache ? slots[t] : -1;
+  if (tid < 64) {
+    const short8_t v =
+        *reinterpret_cast<const short8_t*>(kv_a + t * kv_ts + tid * 8);
+    const short8_t g = *reinterpret_cast<const short8_t*>(w + tid * 8);
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const float f = bf16_to_f32(v[j]);
+      ss += f * f;
+    }
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) ss += __shfl_xor(ss, d, 64);
+    const float inv = rsqrtf(ss / (float)R + eps);
+    short8_t o;
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      o[j] = f32_to_bf16(bf16_to_f32(v[j]) * inv * bf16_to_f32(g[j]));
+    *reinterpret_cast<short8_t*>(c_out + t * R + tid * 8) = o;
+    if (slot >= 0)
+      *reinterpret_cast<short8_t*>(cache + slot * DT + tid * 8) = o;
+    return;
+  }
+  const float* cs = cos_sin + positions[t] * P;
+  // (head, 8 pairs); head H is the key
+  for (int i = tid - 64; i < (H + 1) * (P / 16); i += 192) {
+    const int h = i / (P / 16), d = i % (P / 16) * 8;
+    const short* src = h < H ? q + t * q_ts + h * q_hs
+                             : kv_a + t * kv_ts + R;
+    short* dst = h < H ? q_out + (t * H + h) * P : k_out + t * P;
+    const short8_t xa = *reinterpret_cast<const short8_t*>(src + d);
+    const short8_t xb = *reinterpret_cast<const short8_t*>(src + P / 2 + d);
+    short8_t oa, ob;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const float co = cs[d + j], si = cs[P / 2 + d + j];
+      const float x = bf16_to_f32(xa[j]), y = bf16_to_f32(xb[j]);
+      oa[j] = f32_to_bf16(x * co - y * si);
+      ob[j] = f32_to_bf16(y * co + x * si);
+    }
+    *reinterpret_cast<short8_t*>(dst + d) = oa;
+    *reinterpret_cast<short8_t*>(dst + P / 2 + d) = ob;
+    if (h == H && slot >= 0) {
+      short* row = cache + slot * DT + R;
+      *reinterpret_cast<short8_t*>(row + d) = oa;
+      *reinterpret_cast<short8_t*>(row + P / 2 + d) = ob;
+    }
+  }
+}
+
+}  // namespace
+
+// q [T, H, P] of any token and head stride; an empty cache: nothing cached
+void mla_prepare(at::Tensor q_out, at::Tensor c_out, at::Tensor k_out,
+                 at::Tensor cache, at::Tensor q, at::Tensor kv_a, at::Tensor w,
+                 double eps, at::Tensor positions, at::Tensor cos_sin,
+                 at::Tensor slots) {
+  auto ok = [](const at::Tensor& t) {
+    bool fine = t.is_cuda() && t.dtype() == at::kBFloat16 &&
+                t.stride(-1) == 1 && (uintptr_t)t.data_ptr() % 16 == 0;
+    for (int i = 0; i + 1 < t.dim(); i++)
+      fine = fine && (t.size(i) == 1 || t.stride(i) % 8 == 0);
+    return fine;
+  };
+  const int64_t T = q.size(0), H = q.size(1);
+  TORCH_CHECK(ok(q) && ok(kv_a) && ok(w) && q.dim() == 3 && kv_a.dim() == 2);
+  TORCH_CHECK(q.size(2) == P && kv_a.size(0) == T && kv_a.size(1) == DT &&
+              w.numel() == R);
+  TORCH_CHECK(ok(q_out) && ok(c_out) && ok(k_out) && q_out.is_contiguous() &&
+              c_out.is_contiguous() && k_out.is_contiguous() &&
+              q_out.numel() == T * H * P && c_out.numel() == T * R &&
+              k_out.numel() == T * P);
+  TORCH_CHECK(positions.dtype() == at::kLong && positions.numel() >= T &&
+              positions.is_contiguous() && cos_sin.dtype() == at::kFloat &&
+              cos_sin.size(1) == P && cos_sin.is_contiguous());
+  const bool cached = cache.numel() > 0;
+  if (cached) {
+    TORCH_CHECK(cache.dtype() == at::kBFloat16 && cache.is_contiguous() &&
+                cache.size(2) == DT && slots.dtype() == at::kLong &&
+                slots.numel() == T && slots.is_contiguous());
+  }
+  if (T == 0) return;
+  hipLaunchKernelGGL(mla_prepare_kernel, dim3(T), dim3(256), 0,
+                     at::hip::getCurrentHIPStream(), (short*)q_out.data_ptr(),
+                     (short*)c_out.data_ptr(), (short*)k_out.data_ptr(),
+                     cached ? (short*)cache.data_ptr() : nullptr,
+                     (const short*)q.data_ptr(), q.stride(0), q.stride(1),
+                     (const short*)kv_a.data_ptr(), kv_a.stride(0),
+                     (const short*)w.data_ptr(), (float)eps,
+                     positions.data_ptr<int64_t>(), cos_sin.data_ptr<float>(),
+                     cached ? slots.data_ptr<int64_t>() : nullptr, (int)H);
+}
+
+// MLA cache write alone: latent row (c_kv ‖ k_rope) scattered to the paged
+// cache. One wave per token: 64 lanes x 16 B covers the 512-dim c_kv; lanes
+// 0-7 append the 64 rope dims.
 __global__ __launch_bounds__(64, 8)
 void mla_cache_write_kernel(
     short* __restrict__ cache,          // [NB, BS, R+P] bf16
@@ -611,7 +521,6 @@ void mla_cache_write_kernel(
     const short* __restrict__ k_pe,     // [T, P] (row stride pe_stride)
     const int64_t* __restrict__ slots,  // [T]; <0 = skip (padding)
     const int64_t pe_stride) {
-  constexpr int DT = R + P;
   const int t = blockIdx.x;
   const int lane = threadIdx.x;
   const int64_t slot = slots[t];
@@ -633,21 +542,16 @@ void mla_cache_write(at::Tensor cache, at::Tensor c_kv, at::Tensor k_pe,
   TORCH_CHECK(k_pe.stride(-1) == 1 && k_pe.dtype() == at::kBFloat16);
   TORCH_CHECK(slots.dtype() == at::kLong);
   const int T = c_kv.size(0);
-  const int R = c_kv.size(1);
-  const int P = k_pe.size(1);
-  TORCH_CHECK(cache.size(2) == R + P && k_pe.size(0) == T
+  TORCH_CHECK(c_kv.size(1) == R && k_pe.size(1) == P,
+              "unsupported MLA cache dims ", c_kv.size(1), "+", k_pe.size(1));
+  TORCH_CHECK(cache.size(2) == DT && k_pe.size(0) == T
               && slots.size(0) == T);
   auto stream = at::hip::getCurrentHIPStream();
   if (T == 0) return;
-  if (R == 512 && P == 64) {
-    hipLaunchKernelGGL((mla_cache_write_kernel<512, 64>), dim3(T), dim3(64),
-                       0, stream, (short*)cache.data_ptr(),
-                       (const short*)c_kv.data_ptr(),
-                       (const short*)k_pe.data_ptr(),
-                       slots.data_ptr<int64_t>(), k_pe.stride(0));
-  } else {
-    TORCH_CHECK(false, "unsupported MLA cache dims ", R, "+", P);
-  }
+  hipLaunchKernelGGL((mla_cache_write_kernel), dim3(T), dim3(64), 0, stream,
+                     (short*)cache.data_ptr(), (const short*)c_kv.data_ptr(),
+                     (const short*)k_pe.data_ptr(),
+                     slots.data_ptr<int64_t>(), k_pe.stride(0));
 }
 
 }  // namespace kaito

@@ -1,7 +1,6 @@
 #!/usr/bin/env python3
-"""MLA decode kernel microbench (+ occupancy sweep via KAITO_MLA_OCC)."""
+"""MLA decode kernel microbench, checked against the plain reference."""
 import os
-import subprocess
 import sys
 
 sys.path.insert(0, os.path.join(os.path.dirname(__file__), ".."))
@@ -10,21 +9,15 @@ SHAPES = [(768, 300), (256, 400), (1024, 300)]   # (batch, kv_len)
 H, R_, P_, BS = 16, 512, 64, 16
 
 
-def run_one():
+def run():
     import torch
     from kaito_amd import ops
     from kaito_amd.ops import torch_ref as TR
 
     torch.manual_seed(0)
     dev = "cuda"
-    tag = os.environ.get("KAITO_MLA_OCC", "dflt") + \
-        ("+db" if os.environ.get("KAITO_MLA_DB") else "") + \
-        ("+ph" + os.environ.get("KAITO_MLA_PH")
-         if os.environ.get("KAITO_MLA_PH") else "") + \
-        ("+mf" if os.environ.get("KAITO_MLA_MF") else "") + \
-        ("+mv" if os.environ.get("KAITO_MLA_MV") else "")
     DT = R_ + P_
-    first = os.environ.get("KAITO_MLA_PH", "3") == "3"
+    first = True
     for bs, L in SHAPES:
         bps = (L + BS - 1) // BS
         nblocks = bs * bps + 1
@@ -34,7 +27,7 @@ def run_one():
                           device=dev).reshape(bs, bps)
         sl = torch.full((bs,), L, dtype=torch.int32, device=dev)
         scale = 192 ** -0.5
-        if first:   # one numerics check per variant
+        if first:   # one numerics check
             got = ops.mla_decode(q, cache, bt, sl, scale, R_)
             want = TR.mla_decode(q.float(), cache.float(), bt, sl, scale, R_)
             err = (got.float() - want).abs().max().item()
@@ -52,23 +45,9 @@ def run_one():
         torch.cuda.synchronize()
         us = s.elapsed_time(e) / iters * 1000
         rd = bs * L * DT * 2
-        print(f"[occ={tag:>4}] bs={bs:4d} L={L:4d}: {us:7.1f} us  "
+        print(f"bs={bs:4d} L={L:4d}: {us:7.1f} us  "
               f"{rd / us / 1e6:.2f} TB/s cache-read", flush=True)
 
 
-def main():
-    if "--sweep" not in sys.argv:
-        run_one()
-        return
-    # default (MF+MV) vs regression references
-    variants = [{}, {"KAITO_MLA_MV": "0"},
-                {"KAITO_MLA_MF": "0", "KAITO_MLA_MV": "0"}]
-    for v in variants:
-        env = {k: val for k, val in os.environ.items()
-               if not k.startswith("KAITO_MLA")}
-        env.update(v)
-        subprocess.run([sys.executable, __file__], env=env, check=True)
-
-
 if __name__ == "__main__":
-    main()
+    run()
