@@ -179,6 +179,12 @@ __global__ void delta_recurrence_kernel(
 // current tile is consumed and parked in LDS afterwards. k and q rows are
 // zero-padded to DP * PARTS in LDS so the inner loops read unconditional
 // float4s; the dot products run on four independent accumulators.
+//
+// The loop is a chain state -> sums over lanes -> u -> state of about 900
+// cycles a token; what else waits in it costs as much. With loads that
+// nothing converts or tests before they are parked, and stores behind them:
+// 4 prompts of 2048 tokens, 16 heads of 128 x 128, 948 -> 839 us; one 794 ->
+// 627; 4 of 512 tokens, 4 heads of 256 x 64, 235 -> 191.
 template <typename T, int DP, int PARTS>
 __global__ __launch_bounds__(64) void delta_recurrence_wave_kernel(
     float* __restrict__ o,                                 // [T, H, V]
@@ -223,49 +229,51 @@ __global__ __launch_bounds__(64) void delta_recurrence_wave_kernel(
     S[i] = (carried && live && d < D) ? sp[(int64_t)d * V] : 0.0f;
   }
 
+  // Loads of a tile: unconditional, from a row of the chunk and a dim that
+  // exist, and kept as read, so that nothing waits for them before they are
+  // parked; dims that do not exist are zeroed there, rows past the chunk are
+  // not used.
   float4_t rk[KQ4], rq[KQ4];
-  float rv[VN], rdb = 0.f;
-  auto fetch = [&](int t0) {
-    const int nt = min(TT, r1 - t0);
+  T rv[VN];
+  float rdb;
+  auto fetch = [&](const int t0) {
 #pragma unroll
     for (int i = 0; i < KQ4; i++) {
       const int e = tid + i * 64;
-      const int tt = e / (DPAD / 4), d = (e % (DPAD / 4)) * 4;
-      const bool ok = tt < nt && d < D;
-      const int64_t src = ((int64_t)(t0 + tt) * G + g) * D + d;
-      rk[i] = ok ? *reinterpret_cast<const float4_t*>(kn + src)
-                 : float4_t{0.f, 0.f, 0.f, 0.f};
-      rq[i] = ok ? *reinterpret_cast<const float4_t*>(qn + src)
-                 : float4_t{0.f, 0.f, 0.f, 0.f};
+      const int64_t t = min(t0 + e / (DPAD / 4), r1 - 1);
+      const int64_t src = (t * G + g) * D + min(e % (DPAD / 4) * 4, D - 4);
+      rk[i] = *reinterpret_cast<const float4_t*>(kn + src);
+      rq[i] = *reinterpret_cast<const float4_t*>(qn + src);
     }
 #pragma unroll
     for (int i = 0; i < VN; i++) {
       const int e = tid + i * 64;
-      const int tt = e / VB, c = blockIdx.z * VB + e % VB;
-      rv[i] = (e < TT * VB && tt < nt && c < V)
-          ? act_ld(v + (int64_t)(t0 + tt) * v_s0 + (int64_t)h * v_s1 + c)
-          : 0.f;
+      const int64_t t = min(t0 + e / VB % TT, r1 - 1);
+      const int c = min((int)blockIdx.z * VB + e % VB, V - 1);
+      rv[i] = v[t * v_s0 + (int64_t)h * v_s1 + c];
     }
-    if (tid < 3 * TT) {
-      const int tt = tid / 3, which = tid % 3;
-      if (tt >= nt) rdb = 0.f;
-      else if (which == 2) rdb = kq[(int64_t)(t0 + tt) * G + g];
-      else rdb = (which ? beta : decay)[(int64_t)(t0 + tt) * H + h];
-    }
+    const int which = tid % 3;
+    const int64_t t = min(t0 + tid / 3 % TT, r1 - 1);
+    rdb = which == 2 ? kq[t * G + g]
+                     : (which ? beta : decay)[t * H + h];
   };
   auto park = [&](float* buf) {
+    const float4_t none{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < KQ4; i++) {
       const int e = tid + i * 64;
       const int tt = e / (DPAD / 4), d = (e % (DPAD / 4)) * 4;
       const int dd = (d / DP) * DPS + d % DP;
-      *reinterpret_cast<float4_t*>(buf + tt * ROW + dd) = rk[i];
-      *reinterpret_cast<float4_t*>(buf + tt * ROW + KROW + dd) = rq[i];
+      *reinterpret_cast<float4_t*>(buf + tt * ROW + dd) =
+          d < D ? rk[i] : none;
+      *reinterpret_cast<float4_t*>(buf + tt * ROW + KROW + dd) =
+          d < D ? rq[i] : none;
     }
 #pragma unroll
     for (int i = 0; i < VN; i++) {
       const int e = tid + i * 64;
-      if (e < TT * VB) buf[(e / VB) * ROW + 2 * KROW + e % VB] = rv[i];
+      if (e < TT * VB)
+        buf[(e / VB) * ROW + 2 * KROW + e % VB] = act_ld(&rv[i]);
     }
     if (tid < 3 * TT) buf[(tid / 3) * ROW + 2 * KROW + VB + tid % 3] = rdb;
   };
@@ -279,6 +287,7 @@ __global__ __launch_bounds__(64) void delta_recurrence_wave_kernel(
     const bool more = t0 + TT < r1;
     if (more) fetch(t0 + TT);
     const float* buf = lds[cur];
+    float keep[(TT + PARTS - 1) / PARTS];   // row n PARTS + part of column j
     for (int tt = 0; tt < nt; tt++) {
       const float* lk = buf + tt * ROW + part * DPS;
       const float* lq = lk + KROW;
@@ -313,10 +322,16 @@ __global__ __launch_bounds__(64) void delta_recurrence_wave_kernel(
         S[i + 2] = dec * S[i + 2] + k4[2] * u;
         S[i + 3] = dec * S[i + 3] + k4[3] * u;
       }
-      if (live && part == 0)
-        o[((int64_t)(t0 + tt) * H + h) * V + j] = oj;
+#pragma unroll
+      for (int n = 0; n < (TT + PARTS - 1) / PARTS; n++)
+        if (tt == n * PARTS + part) keep[n] = oj;
     }
     if (more) park(lds[cur ^ 1]);
+    // behind the wait for the tile's loads, so that it is not for stores
+#pragma unroll
+    for (int n = 0; n < (TT + PARTS - 1) / PARTS; n++)
+      if (live && n * PARTS + part < nt)
+        o[((int64_t)(t0 + n * PARTS + part) * H + h) * V + j] = keep[n];
     __syncthreads();
     cur ^= 1;
   }

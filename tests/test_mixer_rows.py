@@ -1,0 +1,158 @@
+"""Row kernels of the stateful mixers at the edges of their tiles: convolution
+(16 rows of 16-byte channels), linear recurrent unit (segments of 64 rows, 8
+at a time), delta rule (4 tokens at once), post-norm (rows in registers)."""
+import pytest
+import torch
+
+from kaito_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+I32 = dict(dtype=torch.int32, device=DEV)
+
+
+def _layout(lens, starts, slots, pad=0):
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    ts = [b for b, n in enumerate(lens) for _ in range(n)] + [-1] * pad
+    t = lambda v: torch.tensor(v, **I32)
+    return t(cu), t(slots), t(starts), t(ts)
+
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("taps", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("C", [8, 1544, 44])
+@pytest.mark.parametrize("lens", [[1, 1, 1], [2, 37, 1, 16], [64]])
+def test_causal_conv(lens, C, taps, dt):
+    torch.manual_seed(C + taps)
+    T = sum(lens)
+    starts = [5 * (i % 2) for i in range(len(lens))]
+    slots = [2 * i + 1 for i in range(len(lens))]
+    if len(lens) > 3:
+        slots[1] = -1
+    x = torch.randn(T, 2 * C, device=DEV).to(dt)[:, C:]
+    w, b = torch.randn(C, taps, device=DEV), torch.randn(C, device=DEV)
+    state = torch.randn(2 * len(lens), max(taps - 1, 1), C, device=DEV).to(dt)
+    want = state.double().clone()
+    lay = _layout(lens, starts, slots)
+    out = ops.causal_conv_update(x, w, b, state, *lay, act=1)
+    at = 0
+    for n, st, slot in zip(lens, starts, slots):
+        rows = x[at:at + n].double()
+        if slot >= 0:
+            old = want[slot] if st else torch.zeros_like(want[slot])
+            seq = torch.cat([old[:taps - 1], rows])
+            acc = b.double() + sum(seq[j:j + n] * w[:, j].double()
+                                   for j in range(taps))
+            mag = b.double().abs() + sum(
+                (seq[j:j + n] * w[:, j].double()).abs() for j in range(taps))
+            ref = acc * torch.sigmoid(acc)
+            eps = 2.0 ** -8 if dt == torch.bfloat16 else 0.0
+            err = (out[at:at + n].double() - ref).abs()
+            assert (err <= eps * ref.abs() + 2.0 ** -20 * mag + 1e-30).all()
+            if taps > 1:
+                want[slot][:taps - 1] = seq[n:]
+        at += n
+    assert torch.equal(state.double(), want)
+
+
+@pytest.mark.parametrize("lens,pad", [([130], 0), ([64, 64, 1, 70], 0),
+                                      ([7, 200, 9], 5), ([513], 0)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_rglru_segments(lens, pad, dt):
+    torch.manual_seed(len(lens))
+    W, NB, T = 320, 5, sum(lens) + pad
+    bw = W // NB
+    starts = [3 * (i % 2) for i in range(len(lens))]
+    slots = list(range(len(lens), 0, -1))
+    u, y = (torch.randn(T, W, device=DEV).to(dt) for _ in range(2))
+    gates = torch.randn(NB, T, 2 * bw, device=DEV) * 3
+    gates[0, :3, :2], gates[1, 5, 3] = -200.0, 200.0
+    rate = torch.rand(W, device=DEV)
+    rate[::7] = 1e-6                      # states that hardly decay
+    state = torch.randn(len(lens) + 1, W, device=DEV)
+    S0 = state.double()
+    cu, sl, st, ts = _layout(lens, starts, slots, pad)
+    out = ops.rglru_scan(u, gates, y, rate, state, cu, sl, st, ts)
+    g = gates.double().permute(1, 0, 2)
+    r = torch.sigmoid(g[..., :bw]).reshape(T, W)
+    i = torch.sigmoid(g[..., bw:]).reshape(T, W)
+    la = -r * rate.double()
+    a, drive = la.exp(), (-torch.expm1(2 * la)).sqrt() * i * u.double()
+    tol = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -18
+    at = 0
+    for n, s, slot in zip(lens, starts, slots):
+        S = S0[slot] if s else torch.zeros_like(S0[slot])
+        for t in range(at, at + n):
+            S = a[t] * S + drive[t]
+            ref = S * torch.nn.functional.gelu(y[t].double(),
+                                               approximate="tanh")
+            err = (out[t].double() - ref).abs()
+            assert (err <= tol * ref.abs() + 1e-5 * y[t].double().abs()).all()
+        assert ((state[slot].double() - S).abs() <= 1e-5 * (1 + S.abs())).all()
+        at += n
+
+
+@pytest.mark.parametrize("lens", [[1, 2, 3, 4, 5, 9], [31], [8, 64]])
+@pytest.mark.parametrize("D,V,a0", [(128, 128, -2.0), (64, 20, 3.0),
+                                    (256, 8, -6.0), (12, 12, 0.0)])
+def test_delta_rule_steps(lens, D, V, a0):
+    """Chunks that four tokens do not divide; slow to very fast decay."""
+    torch.manual_seed(D)
+    T, G, H, n_seq = sum(lens), 2, 4, len(lens)
+    r = lambda *s: torch.randn(*s, device=DEV)
+    q, k, v, gate = r(T, G, D), r(T, G, D), r(T, H, V), r(T, H, V)
+    a, b = r(T, H), r(T, H)
+    a_log, dt_bias, nw = r(H) * 0.5 + a0, r(H), r(V)
+    starts = [i % 2 for i in range(n_seq)]
+    state = r(n_seq, H, D, V)
+    S0 = state.double()
+    cu, sl, st, _ = _layout(lens, starts, list(range(n_seq)))
+    out = ops.gated_delta_rule(q, k, v, gate, a, b, a_log, dt_bias, nw, state,
+                               cu, sl, st, 1e-6, 1e-5)
+    qd, kd = q.double(), k.double()
+    qd = qd / (qd.square().sum(-1, True) + 1e-6).sqrt() / D ** 0.5
+    kd = kd / (kd.square().sum(-1, True) + 1e-6).sqrt()
+    qd, kd = (x.repeat_interleave(H // G, 1) for x in (qd, kd))
+    dec = torch.exp(-a_log.double().exp() * torch.nn.functional.softplus(
+        a.double() + dt_bias.double()))
+    beta, vd, gd = torch.sigmoid(b.double()), v.double(), gate.double()
+    at = 0
+    for i, n in enumerate(lens):
+        S = S0[i] if starts[i] else torch.zeros_like(S0[i])
+        for t in range(at, at + n):
+            S = S * dec[t][:, None, None]
+            u = beta[t][:, None] * (vd[t] - (S * kd[t][:, :, None]).sum(1))
+            S = S + kd[t][:, :, None] * u[:, None]
+            o = (S * qd[t][:, :, None]).sum(1)
+            rms = (o.square().mean(-1, True) + 1e-5).sqrt()
+            ref = o / rms * nw.double() * gd[t] * torch.sigmoid(gd[t])
+            err = (out[t].view(H, V).double() - ref).abs()
+            # f32 sums of D terms, relative to the row's rms
+            lim = 2e-5 * (nw.double() * gd[t]).abs() / rms.clamp(min=1e-2) \
+                * S.abs().amax().clamp(min=1) + 1e-6
+            assert (err <= lim).all(), (t, (err / lim).max())
+        assert ((state[i].double() - S).abs() <= 1e-5 * (1 + S.abs())).all()
+        at += n
+
+
+@pytest.mark.parametrize("H", [8, 520, 2048, 2056, 4096, 8192, 8200, 100])
+@pytest.mark.parametrize("pair", [False, True])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_post_norm(H, pair, dt):
+    torch.manual_seed(H)
+    T = 3
+    x32 = torch.randn(T, H, device=DEV)
+    y = torch.randn(T, H + 8, device=DEV).to(dt)[:, :H]
+    y2 = torch.randn(T, H, device=DEV).to(dt)
+    w, wa, wb = (torch.rand(H, device=DEV) + 0.5 for _ in range(3))
+    X, Y, Y2 = x32.double(), y.double(), y2.double()
+    kw = dict(y2=y2, w_y=wa, w_y2=wb) if pair else {}
+    xa = ops.post_norm_residual(x32, y, w, 1e-5, torch.bfloat16, **kw)
+    n = lambda t: t / (t.square().mean(-1, True) + 1e-5).sqrt()
+    m = (n(Y) * wa.double() + n(Y2) * wb.double()) / 2 if pair else Y
+    ref = X + n(m) * w.double()
+    assert ((x32.double() - ref).abs() <= 2e-6 * (1 + ref.abs())).all()
+    assert torch.equal(xa, x32.to(torch.bfloat16))
