@@ -11,19 +11,21 @@
 // x 256 weight rows (up: 128 gate rows beside their 128 up rows, 32 + 32 per
 // wave, so a lane holds both of a pair) in K steps of 64 on
 // v_mfma_f32_32x32x16_bf16, transposed (C^T = W X^T: a lane owns one token row
-// and 4 neighbouring outputs at a time, stored as 8 bytes). Both operands
-// arrive by 16-byte global_load_lds one K step ahead (two buffers, one
-// barrier per step; 16-byte chunk c of row r at c ^ (r & 7)). At BM = 256 a
-// step is 32 MFMA per wave, 2048 cycles of a SIMD's two waves, against 192 KB
-// of LDS reads (1536 cycles) and 64 KB of staging per CU.
+// and 4 neighbouring outputs at a time). Both operands arrive by 16-byte
+// loads straight to LDS one K step ahead (two buffers, one barrier per step;
+// 16-byte chunk c of row r at c ^ (r & 7)); as buffer loads, behind which the
+// compiler can count LDS reads (behind the global form it waits for all).
+// At BM = 256 a step is 32 MFMA per wave, 2048 cycles of a SIMD's two waves,
+// against 192 KB of LDS reads (1536 cycles) and 64 KB of staging per CU: both
+// have to overlap, so fragments are read one step of 16 dims ahead.
 //
 // Tiles are numbered expert by expert, in blocks of 4 column tiles x all row
 // tiles, and every XCD takes one contiguous eighth of them: the 32 tiles in
 // flight behind one L2 share rows and weights. Measured on one MI355X, 8
-// experts of 2048 x 2048, top 2: 8192 tokens 347 + 200 + 17 us (790 and 690
-// TFLOP/s) where a library GEMM per expert with its gathers, casts and
-// index_add took 973 us behind a host read; 1024 tokens 141 us against 179
-// for the streaming kernels of moe.hip. 8 of 4096 x 14336: 990 TFLOP/s.
+// experts of 2048 x 2048, top 2, 8192 tokens: 309 + 166 + 17 us (890 and 829
+// TFLOP/s; 333 + 201 with the reads beside their products and 8-byte stores)
+// where a library GEMM per expert with its gathers, casts and index_add took
+// 958 us behind a host read. 8 of 4096 x 14336: 1141 and 1027 TFLOP/s.
 #include "flash_prefill.h"
 #include <torch/library.h>
 #include <ATen/ATen.h>
@@ -35,7 +37,6 @@ namespace {
 
 using flash::f32x16;
 using flash::hbf16x8;
-using flash::lds_copy16;
 using flash::mfma32;
 
 constexpr int BK = 64;              // K step
@@ -48,7 +49,7 @@ struct GemmArgs {
   const short* x;                   // up: [T, K]; down: [TK, K]
   const short* w;                   // [E, rows, K]
   const short* bias;                // [E, rows] or nullptr
-  const int* rows;                  // up: token of a sorted row; down: none
+  const int* rows;                  // x row of a sorted row; none: the same
   const int* offsets;               // [.., E + 1]
   int e_base, E, N, K;
   int act_mode;                     // 0 SwiGLU, 1 clamped, 2 squared relu
@@ -56,6 +57,13 @@ struct GemmArgs {
 };
 
 enum Kind { UP_GATED, UP_PLAIN, DOWN };
+
+// 16 bytes per lane from r + lane offset + uniform offset to dst + 16 * lane
+KAITO_DEV void buffer_copy16(__amdgpu_buffer_rsrc_t r, short* dst,
+                             const uint32_t lane_off, const int off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(
+      r, (__attribute__((address_space(3))) void*)dst, 16, lane_off, off, 0, 0);
+}
 
 KAITO_DEV float silu_of(float v) { return v / (1.f + __expf(-v)); }
 
@@ -91,7 +99,7 @@ __global__ __launch_bounds__(512, 2) void moe_grouped_kernel(const GemmArgs a) {
     for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
     total += n;
   }
-  total *= ntiles;
+  total = __builtin_amdgcn_readfirstlane(total) * ntiles;
   const int share = (total + 7) / 8;
   const int in_share = blockIdx.x / 8;
   int t = (blockIdx.x % 8) * share + in_share;
@@ -127,37 +135,44 @@ __global__ __launch_bounds__(512, 2) void moe_grouped_kernel(const GemmArgs a) {
   const int nt = blk * NG + in_blk % wide, mt0 = in_blk / wide;
   const int m0 = row0 + mt0 * BM, n0 = nt * COLS;
 
-  // ---- staging slots: slot s (16 bytes) is row s / 8, place s % 8
-  const short* xs[LX];
-  const short* ws[LW];
+  // ---- staging slots: slot s (16 bytes) is row s / 8, place s % 8; byte
+  // offsets from the tile's first row (gathered rows: from x, which the caller
+  // keeps below 4 GB)
+  const int wrows = KIND == UP_GATED ? 2 * a.N : a.N;
+  const short* we = a.w + ((int64_t)expert * wrows + n0) * a.K;
+  const short* xe = a.rows ? a.x : a.x + (int64_t)m0 * a.K;
+  const auto xr = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<short*>(xe), 0, 0xffffffff, 0x27000);
+  const auto wr = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<short*>(we), 0, 0xffffffff, 0x27000);
+  uint32_t xs[LX], ws[LW];
 #pragma unroll
   for (int j = 0; j < LX; j++) {
     const int s = j * 512 + threadIdx.x, row = s / 8;
     const int c = (s % 8) ^ (row & 7);
     const int m = min(m0 + row, row_end - 1);
-    const int64_t src = KIND == DOWN ? m : a.rows[m];
-    xs[j] = a.x + src * a.K + c * 8;
+    const uint32_t src = a.rows ? a.rows[m] : m - m0;
+    xs[j] = (src * a.K + c * 8) * 2;
   }
-  const int wrows = KIND == UP_GATED ? 2 * a.N : a.N;
-  const short* we = a.w + (int64_t)expert * wrows * a.K;
 #pragma unroll
   for (int j = 0; j < LW; j++) {
     const int s = j * 512 + threadIdx.x, row = s / 8;
     const int c = (s % 8) ^ (row & 7);
     // gated: every 64 tile rows are 32 gate rows, then their up rows
-    const int n = KIND == UP_GATED
-        ? min(n0 + (row / 64) * 32 + row % 32, a.N - 1) +
+    const uint32_t n = KIND == UP_GATED
+        ? min((row / 64) * 32 + row % 32, a.N - 1 - n0) +
               (row % 64 >= 32 ? a.N : 0)
-        : min(n0 + row, a.N - 1);
-    ws[j] = we + (int64_t)n * a.K + c * 8;
+        : min(row, a.N - 1 - n0);
+    ws[j] = (n * a.K + c * 8) * 2;
   }
   auto stage = [&](const int k, short* buf) {
 #pragma unroll
     for (int j = 0; j < LX; j++)
-      lds_copy16(xs[j] + k, buf + (j * 512 + wave * 64) * 8);
+      buffer_copy16(xr, buf + (j * 512 + wave * 64) * 8, xs[j], k * 2);
 #pragma unroll
     for (int j = 0; j < LW; j++)
-      lds_copy16(ws[j] + k, buf + BM * BK + (j * 512 + wave * 64) * 8);
+      buffer_copy16(wr, buf + BM * BK + (j * 512 + wave * 64) * 8, ws[j],
+                    k * 2);
   };
 
   f32x16 acc[2][MT];
@@ -168,72 +183,123 @@ __global__ __launch_bounds__(512, 2) void moe_grouped_kernel(const GemmArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
 
-  stage(0, lds[0]);
-  __syncthreads();
-  int cur = 0;
-  for (int k = 0; k < a.K; k += BK) {
-    if (k + BK < a.K) stage(k + BK, lds[cur ^ 1]);
-    const short* xb = lds[cur] + (wm * (BM / 2) + lr) * BK;
-    const short* wb = lds[cur] + BM * BK + (wn * 64 + lr) * BK;
+  // Fragments of 16 dims of K are read one step ahead of their products, the
+  // first of the next tile beside the last products of this one: the barrier
+  // that frees this tile stands between its last read and its last products.
+  hbf16x8 wf[2][2], xf[2][MT];
+  auto read = [&](const short* buf, const int kk) {
+    const int c = ((kk * 2 + h) ^ (lr & 7)) * 8, f = kk & 1;
+    const short* xb = buf + (wm * (BM / 2) + lr) * BK + c;
+    const short* wb = buf + BM * BK + (wn * 64 + lr) * BK + c;
 #pragma unroll
-    for (int kk = 0; kk < BK / 16; kk++) {
-      const int c = ((kk * 2 + h) ^ (lr & 7)) * 8;
-      hbf16x8 wf[2], xf[MT];
+    for (int i = 0; i < 2; i++)
+      wf[f][i] = *reinterpret_cast<const hbf16x8*>(wb + i * 32 * BK);
+#pragma unroll
+    for (int j = 0; j < MT; j++)
+      xf[f][j] = *reinterpret_cast<const hbf16x8*>(xb + j * 32 * BK);
+  };
+  auto multiply = [&](const int kk) {
+    const int f = kk & 1;
+    __builtin_amdgcn_sched_barrier(0);      // the next reads are under way
+#pragma unroll
+    for (int j = 0; j < MT; j++)
 #pragma unroll
       for (int i = 0; i < 2; i++)
-        wf[i] = *reinterpret_cast<const hbf16x8*>(wb + i * 32 * BK + c);
+        acc[i][j] = mfma32(wf[f][i], xf[f][j], acc[i][j]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto meet = [&]() {               // own loads landed and reads done: all's
+    __builtin_amdgcn_s_waitcnt(0x0070);     // vmcnt(0) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  constexpr int LAST = BK / 16 - 1;
+
+  stage(0, lds[0]);
+  meet();
+  if (BK < a.K) stage(BK, lds[1]);
+  read(lds[0], 0);
+  int cur = 0;
+  for (int k = 0; k < a.K; k += BK) {
 #pragma unroll
-      for (int j = 0; j < MT; j++)
-        xf[j] = *reinterpret_cast<const hbf16x8*>(xb + j * 32 * BK + c);
-#pragma unroll
-      for (int j = 0; j < MT; j++)
-#pragma unroll
-        for (int i = 0; i < 2; i++) acc[i][j] = mfma32(wf[i], xf[j], acc[i][j]);
+    for (int kk = 0; kk < LAST; kk++) {
+      read(lds[cur], kk + 1);
+      multiply(kk);
     }
-    __syncthreads();
+    meet();
+    if (k + 2 * BK < a.K) stage(k + 2 * BK, lds[cur]);
+    if (k + BK < a.K) read(lds[cur ^ 1], 0);
+    multiply(LAST);
     cur ^= 1;
   }
 
   // ---- outputs n = 8 b + 4 h + e of 32-row tile i, token row lr of tile j
-  const short* be = a.bias ? a.bias + (int64_t)expert * wrows : nullptr;
+  constexpr int NI = KIND == UP_GATED ? 1 : 2;
+  constexpr int WC = NI * 32;       // columns of a wave: all exist or none
+  const int c0 = n0 + wn * WC;
+  if (c0 >= a.N) return;            // N is a multiple of 64; no barrier below
+  if (a.bias) {
+    const short* be = a.bias + (int64_t)expert * wrows + c0;
 #pragma unroll
-  for (int j = 0; j < MT; j++) {
-    const int m = m0 + wm * (BM / 2) + j * 32 + lr;
-    if (m >= row_end) continue;
-    short* orow = a.out + (int64_t)m * a.N;
-#pragma unroll
-    for (int i = 0; i < (KIND == UP_GATED ? 1 : 2); i++)
+    for (int i = 0; i < 2; i++)
 #pragma unroll
       for (int b = 0; b < 4; b++) {
-        const int n = n0 + (KIND == UP_GATED ? wn * 32 : wn * 64 + i * 32) +
-            8 * b + 4 * h;
-        if (n >= a.N) continue;               // N is a multiple of 64
-        short4_t o;
-        float4_t o32;
+        const short4_t v = *reinterpret_cast<const short4_t*>(
+            be + (KIND == UP_GATED ? i * a.N : i * 32) + 8 * b + 4 * h);
+#pragma unroll
+        for (int j = 0; j < MT; j++)
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+            acc[i][j][b * 4 + e] += bf16_to_f32(v[e]);
+      }
+  }
+  // bf16 rows pass through the wave's part of LDS (every wave is done with
+  // its tiles) and leave as 16 bytes a lane
+  constexpr int PITCH = WC + 8, LANES = WC / 8;
+  short* slab = &lds[0][0] + wave * 32 * PITCH;
+#pragma unroll
+  for (int j = 0; j < MT; j++) {
+    const int mj = m0 + wm * (BM / 2) + j * 32;
+#pragma unroll
+    for (int i = 0; i < NI; i++)
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        float4_t v;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-          float v = acc[i][j][b * 4 + e];
+          v[e] = acc[i][j][b * 4 + e];
           if constexpr (KIND == UP_GATED) {
-            float u = acc[1][j][b * 4 + e];
-            if (be) {
-              v += bf16_to_f32(be[n + e]);
-              u += bf16_to_f32(be[a.N + n + e]);
-            }
-            v = gated(a.act_mode, v, u, a.limit);
+            v[e] = gated(a.act_mode, v[e], acc[1][j][b * 4 + e], a.limit);
           } else if constexpr (KIND == UP_PLAIN) {
-            v = fmaxf(v, 0.f);
-            v *= v;
-          } else {
-            if (be) v += bf16_to_f32(be[n + e]);
+            v[e] = fmaxf(v[e], 0.f);
+            v[e] *= v[e];
           }
-          o[e] = f32_to_bf16(v);
-          o32[e] = v;
         }
-        if (KIND == DOWN && a.out32)
-          *reinterpret_cast<float4_t*>(a.out32 + (int64_t)m * a.N + n) = o32;
-        else
-          *reinterpret_cast<short4_t*>(orow + n) = o;
+        const int n = i * 32 + 8 * b + 4 * h;
+        if (KIND == DOWN && a.out32) {
+          if (mj + lr < row_end)
+            *reinterpret_cast<float4_t*>(
+                a.out32 + (int64_t)(mj + lr) * a.N + c0 + n) = v;
+        } else {
+          *reinterpret_cast<short4_t*>(slab + lr * PITCH + n) =
+              short4_t{f32_to_bf16(v[0]), f32_to_bf16(v[1]),
+                       f32_to_bf16(v[2]), f32_to_bf16(v[3])};
+        }
       }
+    if (KIND == DOWN && a.out32) continue;
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int r = 0; r < 32; r += 64 / LANES) {
+      const int row = r + lane / LANES, n = lane % LANES * 8;
+      const short8_t v =
+          *reinterpret_cast<const short8_t*>(slab + row * PITCH + n);
+      if (mj + row < row_end)
+        *reinterpret_cast<short8_t*>(a.out + (int64_t)(mj + row) * a.N + c0 +
+                                     n) = v;
+    }
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
   }
 }
 
@@ -339,6 +405,12 @@ void moe_grouped_up(at::Tensor act, at::Tensor x, at::Tensor w,
   a.w = (const short*)w.data_ptr() - e_base * w.stride(0);
   if (a.bias) a.bias -= e_base * 2 * a.N;
   a.rows = sorted_ids.data_ptr<int>();
+  at::Tensor gathered;
+  if (x.numel() >= 1LL << 31) {     // beyond 32-bit byte offsets
+    gathered = x.index_select(0, sorted_ids);
+    a.x = (const short*)gathered.data_ptr();
+    a.rows = nullptr;
+  }
   a.offsets = offsets.data_ptr<int>();
   a.act_mode = (int)act_mode;
   a.limit = (float)act_limit;
