@@ -150,25 +150,27 @@ class LlamaAttention(nn.Module):
             k = ops.rms_norm(
                 k.reshape(-1, self.head_dim).contiguous(), self.k_norm,
                 self.cfg.rms_eps).reshape(k.shape[0], -1)
-            # k is now a fresh contiguous tensor; reshape_and_cache needs
-            # k/v with EQUAL row strides, so v must match
+            # k is now a fresh contiguous tensor; where rope_and_cache goes
+            # by reshape_and_cache, k and v need EQUAL row strides
             v = v.contiguous()
         cs = cos_sin_local if self.local_rope else cos_sin
-        q, k = ops.rotary_embedding(positions, q, k, self.head_dim, cs)
+        if kv_cache is not None:
+            q, k = ops.rope_and_cache(positions, q, k, v, self.head_dim, cs,
+                                      kv_cache[0], kv_cache[1],
+                                      meta.slot_mapping)
+        else:
+            q, k = ops.rotary_embedding(positions, q, k, self.head_dim, cs)
         T = x.size(0)
         qh = q.unflatten(-1, (self.num_heads, self.head_dim))
         kh = k.unflatten(-1, (self.num_kv_heads, self.head_dim))
         vh = v.unflatten(-1, (self.num_kv_heads, self.head_dim))
-        if kv_cache is not None:
-            ops.reshape_and_cache(kh, vh, kv_cache[0], kv_cache[1],
-                                  meta.slot_mapping)
         sinks = getattr(self, "sinks", None)
         if meta.is_prefill:
             tiles = None if meta.tile_seq is None else \
                 (meta.tile_seq, meta.tile_qbase)
             if meta.kv_lens is not None:
                 # suffix-query attention over the paged cache (the suffix
-                # K/V was just written by reshape_and_cache above)
+                # K/V was just written by rope_and_cache above)
                 out = ops.context_attention(qh, kv_cache[0], kv_cache[1],
                                             meta.cu_seqlens, meta.kv_lens,
                                             meta.block_tables, self.scale,

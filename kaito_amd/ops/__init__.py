@@ -25,7 +25,7 @@ _OP_GROUP = {}
 for _g, _names in {
     "core": ("rms_norm fused_add_rms_norm rotary_embedding silu_and_mul "
              "gelu_and_mul gelu layer_norm fused_add_layer_norm "
-             "reshape_and_cache topk skinny_linear skinny_swiglu"),
+             "rope_and_cache reshape_and_cache topk skinny_linear skinny_swiglu"),
     "attn": ("paged_attention paged_attention_sp prefill_attention "
              "mla_prefill_attention context_attention mfma_tile_gemm paged_read_bw"),
     "mla": "mla_decode mla_prepare mla_cache_write",
@@ -152,7 +152,7 @@ def _skinny(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
     and library): 8 rows win but for the longest K (28672 x 4096: 44.5, 53.0;
     4096 x 14336: 25.9, 25.1); 16 rows up to 4096 x 4096 (11.2, 15.4; 6144 x
     4096: 15.9, 14.4) and in a SwiGLU pair; 32 rows up to 3072 x 2048 (7.9,
-    11.4; 6144 x 2048: 13.3, 12.4)."""
+    11.4; 6144 x 2048: 13.3, 12.4, where a SwiGLU pair saves its launch)."""
     if not (x.is_cuda and x.dim() == 2 and 1 <= x.size(0) <= 32
             and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and w.is_contiguous() and w.size(1) % 8 == 0 and w.numel() > 0
@@ -171,7 +171,7 @@ def _skinny(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
         return K <= 8192
     if M <= 16:
         return N * K <= 4096 * 4096 or (glu and K <= 8192)
-    return N * K <= 3072 * 2048
+    return N * K <= (6144 if glu else 3072) * 2048
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
@@ -204,6 +204,34 @@ def reshape_and_cache(k: torch.Tensor, v: torch.Tensor, k_cache: torch.Tensor,
         _K.reshape_and_cache(k, v, k_cache, v_cache, slot_mapping)
         return
     torch_ref.reshape_and_cache(k, v, k_cache, v_cache, slot_mapping)
+
+
+def rope_and_cache(positions: torch.Tensor, q: torch.Tensor, k: torch.Tensor,
+                   v: torch.Tensor, head_dim: int, cos_sin: torch.Tensor,
+                   k_cache: torch.Tensor, v_cache: torch.Tensor,
+                   slot_mapping: torch.Tensor):
+    """rotary_embedding of q and k [T, heads * head_dim], then
+    reshape_and_cache of k and v. Returns (q, k). One launch for rows of
+    whole 16-byte chunks."""
+    rows = (q, k, v)
+    if q.is_cuda and all(
+            t.dim() == 2 and t.dtype == torch.bfloat16 and t.stride(1) == 1
+            and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
+            for t in rows) \
+            and cos_sin.size(1) % 16 == 0 and cos_sin.size(1) <= head_dim \
+            and cos_sin.is_contiguous() and positions.is_contiguous() \
+            and head_dim % 8 == 0 and k_cache.size(3) == head_dim \
+            and k.size(1) == v.size(1) == k_cache.size(1) * head_dim \
+            and slot_mapping.is_contiguous() \
+            and positions.numel() == slot_mapping.numel() == q.size(0):
+        _K.rope_and_cache(positions, q, k, v, cos_sin, k_cache, v_cache,
+                          slot_mapping)
+        return q, k
+    q, k = rotary_embedding(positions, q, k, head_dim, cos_sin)
+    reshape_and_cache(k.unflatten(-1, (-1, head_dim)),
+                      v.unflatten(-1, (-1, head_dim)), k_cache, v_cache,
+                      slot_mapping)
+    return q, k
 
 
 # decode-attention implementation: "sp" = split-phase (r02, K-stream →

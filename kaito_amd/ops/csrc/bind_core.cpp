@@ -17,6 +17,9 @@ void layer_norm(at::Tensor out, at::Tensor input, at::Tensor weight,
 void fused_add_layer_norm(at::Tensor out, at::Tensor input,
                           at::Tensor residual, at::Tensor weight,
                           at::Tensor bias, double eps);
+void rope_and_cache(at::Tensor positions, at::Tensor q, at::Tensor k,
+                    at::Tensor v, at::Tensor cos_sin, at::Tensor k_cache,
+                    at::Tensor v_cache, at::Tensor slots);
 void reshape_and_cache(at::Tensor k, at::Tensor v, at::Tensor k_cache,
                        at::Tensor v_cache, at::Tensor slot_mapping);
 void topk(at::Tensor out_vals, at::Tensor out_idx, at::Tensor scores,
@@ -32,6 +35,7 @@ TORCH_LIBRARY_FRAGMENT(kaito, m) {
   m.def("gelu(Tensor(a!) out, Tensor x) -> ()");
   m.def("layer_norm(Tensor(a!) out, Tensor input, Tensor weight, Tensor bias, float eps) -> ()");
   m.def("fused_add_layer_norm(Tensor(a!) out, Tensor input, Tensor(b!) residual, Tensor weight, Tensor bias, float eps) -> ()");
+  m.def("rope_and_cache(Tensor positions, Tensor(a!) q, Tensor(b!) k, Tensor v, Tensor cos_sin, Tensor(c!) k_cache, Tensor(d!) v_cache, Tensor slots) -> ()");
   m.def("reshape_and_cache(Tensor k, Tensor v, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor slot_mapping) -> ()");
   m.def("topk(Tensor(a!) out_vals, Tensor(b!) out_idx, Tensor scores, int k) -> ()");
 }
@@ -45,6 +49,7 @@ TORCH_LIBRARY_IMPL(kaito, CUDA, m) {
   m.impl("gelu", &kaito::gelu);
   m.impl("layer_norm", &kaito::layer_norm);
   m.impl("fused_add_layer_norm", &kaito::fused_add_layer_norm);
+  m.impl("rope_and_cache", &kaito::rope_and_cache);
   m.impl("reshape_and_cache", &kaito::reshape_and_cache);
   m.impl("topk", &kaito::topk);
 }
