@@ -189,14 +189,13 @@ class MLAAttention(nn.Module):
     # ---- absorbed decode over the latent cache --------------------------
     def _decode(self, q_nope, q_pe, cache, meta) -> torch.Tensor:
         T = q_nope.size(0)
-        # q_c[h] = q_nope[h] @ w_kc[h]: [Hl, T, nope] x [Hl, nope, r], read
-        # by the kernel where the product leaves it
-        q_c = torch.bmm(q_nope.transpose(0, 1), self.w_kc)
-        out_c = ops.mla_decode(q_c.transpose(0, 1), cache, meta.block_tables,
-                               meta.seq_lens, self.scale, self.r, q_pe)
-        # latent -> per-head v: [Hl, T, r] x [Hl, r, v]
-        o = torch.bmm(out_c.transpose(0, 1), self.w_vc)
-        return o.transpose(0, 1).reshape(T, -1)         # one copy at most
+        # q_c[h] = q_nope[h] @ w_kc[h], read by the kernel where the product
+        # leaves it
+        q_c = ops.head_rows(q_nope, self.w_kc)          # [T, Hl, r]
+        out_c = ops.mla_decode(q_c, cache, meta.block_tables, meta.seq_lens,
+                               self.scale, self.r, q_pe)
+        # latent -> per-head v
+        return ops.head_rows(out_c, self.w_vc).reshape(T, -1)
 
     # ---- absorbed suffix attention over the paged latent cache ----------
     def _context(self, q_nope, q_pe, cache, meta) -> torch.Tensor:

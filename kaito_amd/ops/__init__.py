@@ -28,7 +28,7 @@ for _g, _names in {
              "rope_and_cache reshape_and_cache topk skinny_linear skinny_swiglu"),
     "attn": ("paged_attention paged_attention_sp prefill_attention "
              "mla_prefill_attention context_attention mfma_tile_gemm paged_read_bw"),
-    "mla": "mla_decode mla_prepare mla_cache_write",
+    "mla": "mla_decode mla_prepare head_rows mla_cache_write",
     "moe": ("moe_gate_silu moe_down_rows moe_down_scatter moe_grouped_up "
             "moe_grouped_down moe_combine"),
     "route": "moe_route moe_gate_route moe_sort",
@@ -303,6 +303,22 @@ def mla_prepare(q: torch.Tensor, kv_a: torch.Tensor, w: torch.Tensor,
     _K.mla_prepare(q_out, c, k, _none(cache, q), q, kv_a, w, eps, positions,
                    cos_sin, positions if slots is None else slots)
     return q_out, c, k
+
+
+def head_rows(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x [T, H, K] (any token and head strides) times w [H, K, N] per head:
+    [T, H, N]. One launch for up to 32 rows, a batched library product and
+    its transposition beyond: W is read once per 32 rows."""
+    T, H, K = x.shape
+    if x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and T <= 32 \
+            and K % 64 == 0 and 0 < K <= 512 and w.size(2) % 32 == 0 \
+            and w.is_contiguous() and w.data_ptr() % 16 == 0 \
+            and x.stride(2) == 1 and x.stride(0) % 4 == 0 \
+            and x.stride(1) % 4 == 0 and x.data_ptr() % 8 == 0:
+        y = torch.empty(T, H, w.size(2), dtype=x.dtype, device=x.device)
+        _K.head_rows(y, x, w)
+        return y
+    return torch.bmm(x.transpose(0, 1), w).transpose(0, 1)
 
 
 def mla_cache_write(cache: torch.Tensor, c_kv: torch.Tensor,

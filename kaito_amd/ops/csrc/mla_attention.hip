@@ -511,6 +511,107 @@ void mla_prepare(at::Tensor q_out, at::Tensor c_out, at::Tensor k_out,
                      cached ? slots.data_ptr<int64_t>() : nullptr, (int)H);
 }
 
+namespace {
+
+// y[t, h] = x[t, h] W[h] for the two small products around absorbed decode
+// (W_uk [nope, R] and W_uv [R, v] per head), up to 32 rows: a workgroup per
+// (32 columns, head) holds its [K, 32] of W in LDS, every byte on its way at
+// once, and reads it transposed (C^T = W^T X^T); two waves per 16 columns take
+// half of K each. Bound by the chain launch -> load -> products; the batched
+// library products took 12.3 (K = 128) and 4.7 us (K = 512) of which the
+// second needed a copy of 4.7 us to transpose its result, these
+// 5.9 each (32 rows of 16 heads, with the launch).
+template <int MT>
+__global__ __launch_bounds__(256)
+void head_rows_kernel(short* __restrict__ y, const short* __restrict__ x,
+                      const int64_t x_ts, const int64_t x_hs,
+                      const short* __restrict__ w, const int T, const int K,
+                      const int N) {
+  extern __shared__ __attribute__((aligned(128))) short wt[];   // [K][32]
+  __shared__ f32x4 red[2][MT][64];
+  const int n0 = blockIdx.x * 32, head = blockIdx.y, H = gridDim.y;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lo = lane & 15, hi = lane >> 4;
+  const int half = wave >> 1, col = (wave & 1) * 16;
+  const short* wh = w + (int64_t)head * K * N + n0;
+  // slot s (16 bytes) is row s / 4, place s % 4
+  for (int j = 0; j < K / 64; j++) {
+    const int s = j * 256 + threadIdx.x, row = s / 4;
+    const int c = s % 4 ^ (row >> 2 & 1) << 1;
+    flash::lds_copy16(wh + (int64_t)row * N + c * 8,
+                      wt + (j * 256 + wave * 64) * 8);
+  }
+  const short* xp[MT];
+#pragma unroll
+  for (int m = 0; m < MT; m++)
+    xp[m] = x + min(m * 16 + lo, T - 1) * x_ts + head * x_hs + hi * 4;
+  f32x4 acc[MT];
+#pragma unroll
+  for (int m = 0; m < MT; m++) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  __syncthreads();
+  // rows k + 4 hi + j and k + 16 + 4 hi + j: the order of a transposed read
+  const int row = 4 * hi + (lo >> 2);
+  const short* wp = wt + row * 32 +
+      ((col / 8 + ((lo & 3) >> 1)) ^ (row >> 2 & 1) << 1) * 8 + (lo & 1) * 4;
+#pragma unroll 4
+  for (int k = half * (K / 2); k < (half + 1) * (K / 2); k += 32) {
+    const short4_t a4 = flash::read_tr(wp + k * 32);
+    const short4_t b4 = flash::read_tr(wp + (k + 16) * 32);
+    const hbf16x8 wf = __builtin_bit_cast(
+        hbf16x8, __builtin_shufflevector(a4, b4, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+    for (int m = 0; m < MT; m++) {
+      const short4_t u = *reinterpret_cast<const short4_t*>(xp[m] + k);
+      const short4_t v = *reinterpret_cast<const short4_t*>(xp[m] + k + 16);
+      const hbf16x8 xf = __builtin_bit_cast(
+          hbf16x8, __builtin_shufflevector(u, v, 0, 1, 2, 3, 4, 5, 6, 7));
+      acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xf, acc[m], 0, 0, 0);
+    }
+  }
+  if (half) {
+#pragma unroll
+    for (int m = 0; m < MT; m++) red[wave & 1][m][lane] = acc[m];
+  }
+  __syncthreads();
+  if (half) return;
+#pragma unroll
+  for (int m = 0; m < MT; m++) {
+    const int t = m * 16 + lo;
+    if (t >= T) break;
+    const f32x4 v = acc[m] + red[wave & 1][m][lane];
+    *reinterpret_cast<short4_t*>(
+        y + ((int64_t)t * H + head) * N + n0 + col + hi * 4) =
+        short4_t{f32_to_bf16(v[0]), f32_to_bf16(v[1]), f32_to_bf16(v[2]),
+                 f32_to_bf16(v[3])};
+  }
+}
+
+}  // namespace
+
+// y [T, H, N], x [T, H, K] of any token and head stride, w [H, K, N]
+void head_rows(at::Tensor y, at::Tensor x, at::Tensor w) {
+  for (const at::Tensor* t : {&y, &x, &w})
+    TORCH_CHECK(t->is_cuda() && t->dtype() == at::kBFloat16 && t->dim() == 3);
+  const int64_t T = x.size(0), H = x.size(1), K = x.size(2), N = w.size(2);
+  TORCH_CHECK(y.is_contiguous() && w.is_contiguous() && x.stride(2) == 1 &&
+              y.size(0) == T && y.size(1) == H && y.size(2) == N &&
+              w.size(0) == H && w.size(1) == K);
+  TORCH_CHECK(T <= 32 && K % 64 == 0 && K > 0 && K <= 512 && N % 32 == 0 &&
+              x.stride(0) % 4 == 0 && x.stride(1) % 4 == 0 &&
+              (uintptr_t)x.data_ptr() % 8 == 0 &&
+              (uintptr_t)w.data_ptr() % 16 == 0);
+  if (T == 0 || H == 0 || N == 0) return;
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(N / 32, H), dim3(256), K * 64,
+        at::hip::getCurrentHIPStream(), (short*)y.data_ptr(),
+        (const short*)x.data_ptr(), x.stride(0), x.stride(1),
+        (const short*)w.data_ptr(), (int)T, (int)K, (int)N);
+  };
+  if (T <= 16) launch(&head_rows_kernel<1>);
+  else launch(&head_rows_kernel<2>);
+}
+
 // MLA cache write alone: latent row (c_kv ‖ k_rope) scattered to the paged
 // cache. One wave per token: 64 lanes x 16 B covers the 512-dim c_kv; lanes
 // 0-7 append the 64 rope dims.

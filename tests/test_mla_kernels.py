@@ -83,6 +83,21 @@ def test_prepare(T, H, cached):
     assert torch.equal(cache, want)
 
 
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 32, 33])
+@pytest.mark.parametrize("H,K,N", [(1, 64, 32), (16, 128, 512),
+                                   (3, 512, 128), (2, 192, 96)])
+def test_head_rows(T, H, K, N):
+    """One and two row tiles, halves of K, and the library beyond."""
+    torch.manual_seed(T + K)
+    x = _bf16(T, H, K + 64)[..., 32:32 + K]
+    w = _bf16(H, K, N, scale=K ** -0.5)
+    y = ops.head_rows(x, w)
+    ref = torch.einsum("thk,hkn->thn", x.double(), w.double())
+    mag = torch.einsum("thk,hkn->thn", x.double().abs(), w.double().abs())
+    err = (y.double() - ref).abs()
+    assert (err <= 2.0 ** -8 * ref.abs() + 2.0 ** -18 * mag).all()
+
+
 def test_single_operations_agree():
     """mla_decode of the plain reference, CPU side of both argument forms."""
     q = torch.randn(2, 3, 576)
