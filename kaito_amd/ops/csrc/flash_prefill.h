@@ -188,8 +188,11 @@ void flash_prefill_kernel(const Args a) {
   const float hr2 = EXT && a.r1 ? a.r2[head] : 0.f;
   const float hpb = SIG ? a.pb[head] : 0.f;
 
-  // running maximum (log2 domain) and this lane's share of the sum
-  float m = a.sinks ? a.sinks[head] * LOG2E : -1e30f;
+  // running maximum (log2 domain) and this lane's share of the sum. It is
+  // finite from the start (a sink may be -inf) and masked scores are -inf, at
+  // any scale: a tile in which a row sees nothing neither moves the maximum
+  // nor weighs anything.
+  float m = a.sinks ? fmaxf(a.sinks[head] * LOG2E, -1e30f) : -1e30f;
   float l = (a.sinks || SIG) && h == 0 ? 1.0f : 0.f;
   f32x16 o[DT];
 #pragma unroll
@@ -386,7 +389,7 @@ void flash_prefill_kernel(const Args a) {
           bool dead = dist < 0 || (a.window > 0 && dist >= a.window &&
                                    !(EXT && key < a.keep_first));
           if (EXT) dead = dead || key < low;
-          if (dead) s[kt][i] = -1e30f;
+          if (dead) s[kt][i] = -INFINITY;
         }
     }
     if constexpr (SIG) {

@@ -89,6 +89,101 @@ def test_suffixes_over_pages(QH, KH, D, pairs, window, fp8):
     _check(out, ref)
 
 
+SCALES = [None, 0.1, 0.22, 1 / 16, 1 / 12]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,window", [(64, 32), (64, 100), (96, 40),
+                                      (128, 100), (128, 1024), (256, 32),
+                                      (256, 1024)])
+@pytest.mark.parametrize("G", [1, 2, 4])
+@pytest.mark.parametrize("scale", SCALES)
+def test_rows_past_a_window(D, window, G, scale):
+    """Rows that see nothing of the first key tile which their workgroup
+    reads: 128 / G positions from multiples of that number, behind a window
+    that starts inside a tile, with no sink to bound the maximum."""
+    torch.manual_seed(D + window + G)
+    lens = [window + 201, 1]
+    T = sum(lens)
+    q, k, v = _bf16(T, 2 * G, D), _bf16(T, 2, D), _bf16(T, 2, D)
+    s = scale or D ** -0.5
+    k = (k.float() * D ** -0.5 / s).to(torch.bfloat16)   # scores of order 1
+    out = ops.prefill_attention(q, k, v, _cu(lens), s, window=window)
+    ref = R.prefill_attention(q.float(), k.float(), v.float(), _cu(lens), s,
+                              window)
+    _check(out, ref.cpu())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,G", [(64, 1), (64, 2), (128, 4), (256, 1),
+                                 (256, 2)])
+@pytest.mark.parametrize("window", [32, 100, 1024])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_suffix_rows_past_a_window(D, G, window, fp8):
+    """The same over pages, the suffix starting anywhere in a tile."""
+    torch.manual_seed(D + window)
+    kv, ql = [window + 333, window + 140], [201, 129]
+    mb = -(-max(kv) // 16)
+    bt = torch.randperm(2 * mb, device=DEV).int().view(2, mb)
+    kc, vc = (_bf16(2 * mb, 2, 16, D) for _ in range(2))
+    args = kc, vc
+    if fp8:
+        args = tuple(t.to(torch.float8_e4m3fn) for t in args)
+        kc, vc = (t.to(torch.bfloat16) for t in args)
+        args = tuple(t.view(torch.uint8) for t in args)
+    q = _bf16(sum(ql), 2 * G, D)
+    kl = torch.tensor(kv, dtype=torch.int32, device=DEV)
+    out = ops.context_attention(q, *args, _cu(ql), kl, bt, D ** -0.5, window)
+    ref = R.context_attention(q.float(), kc.float(), vc.float(), _cu(ql), kl,
+                              bt, D ** -0.5, window)
+    _check(out, ref.cpu())
+
+
+@pytest.mark.gpu
+def test_sinks_without_weight():
+    """A sink of -inf absorbs nothing, also behind a masked first tile."""
+    torch.manual_seed(5)
+    T, QH, D = 300, 4, 64
+    q, k, v = _bf16(T, QH, D), _bf16(T, QH, D), _bf16(T, QH, D)
+    sinks = torch.tensor([float("-inf"), 0.5, -2e30, 3.0], device=DEV)
+    out = ops.prefill_attention(q, k, v, _cu([T]), D ** -0.5, window=40,
+                                sinks=sinks)
+    ref = R.prefill_attention(q.float(), k.float(), v.float(), _cu([T]),
+                              D ** -0.5, 40, sinks)
+    _check(out, ref.cpu())
+
+
+@pytest.mark.gpu
+def test_long_prompt_of_a_windowed_model():
+    """Windowed layers of 64-dim heads (window 32), prompts past the first
+    masked tile: logits of the engine on the GPU and on the CPU."""
+    from kaito_amd.engine import EngineConfig, LLMEngine
+    from kaito_amd.models import get_model_config
+    from kaito_amd.parallel.state import init_parallel
+    init_parallel(1)
+    n, state, logits = 300, None, []
+    for dev in ("cpu", DEV):
+        torch.manual_seed(11)
+        eng = LLMEngine(EngineConfig(
+            model=get_model_config("tiny-gemma3-test"), device=dev,
+            max_num_seqs=2, max_model_len=512, num_gpu_blocks=64,
+            enforce_eager=True))
+        model = eng.runner.model
+        if state is None:
+            state = {k: t.clone() for k, t in model.state_dict().items()}
+        model.load_state_dict(state)
+        eng.extend_request(0, [(7 * i + 3) % 500 for i in range(n)])
+        # whole, and as a suffix behind cached tokens
+        logits.append(eng.step_explicit([(0, 200)],
+                                        [(0, i) for i in range(200)]).cpu())
+        logits.append(eng.step_explicit([(0, n - 200)],
+                                        [(0, i) for i in range(n - 200)]).cpu())
+    for ref, out in zip(logits[:2], logits[2:]):
+        assert torch.isfinite(out).all()
+        # bf16 activations through 4 layers, as in the CPU engine's
+        assert (out - ref).norm() < 0.05 * ref.norm()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,lens", [(1, [1, 64, 65]), (16, [200, 33]),
                                     (5, [129, 128, 127])])
