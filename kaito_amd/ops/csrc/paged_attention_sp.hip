@@ -10,9 +10,9 @@
 //     are per-lane scalars after two exchanges;
 //   - O^T += V^T P^T takes P from the score registers; V goes to wave-private
 //     LDS by 16-byte direct loads and comes back by transposing reads.
-// P enters as a bf16 value + remainder pair, which keeps 16 mantissa bits of
-// the f32 weight (the result is rounded to 8). fp8 (e4m3) pages are widened
-// to bf16, exactly, on the way. The waves of a workgroup, and with SPLIT the
+// P enters as the sum of three bf16 terms, which hold every bit of the f32
+// weight (two of them 16 of its 24). fp8 (e4m3) pages are widened to bf16,
+// exactly, on the way. The waves of a workgroup, and with SPLIT the
 // workgroups of a (sequence, kv head), hold partial (max, sum, O) that are
 // folded at the end.
 //
@@ -25,9 +25,9 @@
 // MI355X against a kernel with 4 waves per pair, 16-byte K and V streams in
 // two phases and dot products by dot2 + DPP sums (before -> now; 8 kv heads
 // of 128, groups of 4):
-//   1 row, 217 keys: 11.3 -> 6.3 us;  16 rows, 2050-4100 fp8 keys: 225 -> 42;
-//   64 rows, 500-1000 keys: 77 -> 44;  250 rows, 200-400: 84 -> 65;
-//   2048 rows, 150-300: 453 -> 347 us (5.5 TB/s).
+//   1 row, 217 keys: 11.0 -> 6.2 us;  16 rows of 4000: 176 -> 51 (two terms
+//   of P: 45);  of 4000 fp8 keys: 179 -> 38 (35);  64 rows of 800: 48 -> 35;
+//   250 of 300: 72 -> 56;  2048 of 220: 428 -> 333 us (5.5 TB/s).
 //
 // Cache layout: [num_blocks, KV_HEADS, BLOCK_SIZE, HEAD_DIM] bf16 | e4m3.
 #include "flash_prefill.h"
@@ -214,17 +214,20 @@ void paged_decode_kernel(const DecodeArgs a) {
 #pragma unroll
       for (int dt = 0; dt < DT; dt++) o[dt] *= corr;
     }
-    hbf16x8 p, pl;
+    hbf16x8 p[3];                   // the weight's leading bits, the rest
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         // a masked key weighs nothing even where a lane saw no other yet
-        const float w = s[i][r] > -1e29f
+        float w = s[i][r] > -1e29f
             ? __builtin_amdgcn_exp2f(s[i][r] - m) : 0.f;
         l += w;
-        p[i * 4 + r] = (__bf16)w;
-        pl[i * 4 + r] = (__bf16)(w - (float)p[i * 4 + r]);
+#pragma unroll
+        for (int n = 0; n < 3; n++) {
+          p[n][i * 4 + r] = (__bf16)w;
+          w -= (float)p[n][i * 4 + r];
+        }
       }
     if constexpr (FP8) {
 #pragma unroll
@@ -243,8 +246,10 @@ void paged_decode_kernel(const DecodeArgs a) {
       const short4_t a4 = flash::read_tr(at), b4 = flash::read_tr(at + 16 * D);
       const hbf16x8 vf = __builtin_bit_cast(
           hbf16x8, __builtin_shufflevector(a4, b4, 0, 1, 2, 3, 4, 5, 6, 7));
-      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p, o[dt], 0, 0, 0);
-      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl, o[dt], 0, 0, 0);
+#pragma unroll
+      for (int n = 2; n >= 0; n--)
+        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p[n], o[dt], 0, 0,
+                                                        0);
     }
     __builtin_amdgcn_wave_barrier();
   }

@@ -1,8 +1,8 @@
 """The MFMA decode attention (ops/csrc/paged_attention_sp.hip) at the edges
 of its 32-key tiles and of the rules that choose 4, 8 or 16 waves per
-workgroup and several workgroups per (sequence, kv head). Weights keep 16
-bits, so the outputs are off by their rounding to bf16 (2^-9) and f32 sums;
-the bound is four times that at the values' largest magnitude."""
+workgroup and several workgroups per (sequence, kv head). Weights are f32, so
+the outputs are off by their rounding to bf16 (2^-9) and f32 sums; the bound
+is four times that at the values' largest magnitude."""
 import pytest
 import torch
 
@@ -72,3 +72,47 @@ def test_edges(G, KH, D, fp8):
 def test_launch_rules(KH, lens, max_blocks, D, fp8):
     _run(4, KH, D, lens, max_blocks, fp8=fp8)
     _run(2, KH, D, lens, max_blocks, window=530, sink=True, fp8=fp8)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,KH,gap,max_blocks", [
+    (128, 8, 2, 1), (128, 1, 40, 4), (64, 8, 20, 2), (256, 2, 700, 60),
+    (128, 2, 5000, 400),              # other tiles, waves and splits
+])
+def test_weights_keep_f32(D, KH, gap, max_blocks):
+    """One key of weight w = exp(-s) and value -1 against keys of weight 1
+    whose values sum to w up to 2^-14: what is left shows w's error 2^14
+    times larger. f32 weights and sums are off by a few 2^-24, so what is
+    left by 2^-8 and its rounding, 2^-9; 16-bit weights by up to 2^-3."""
+    torch.manual_seed(D + gap)
+    T, nb = 64, max_blocks * 64 + 1
+    bt = torch.arange(1, nb, dtype=torch.int32).view(T, -1)
+    n = gap + 3                       # keys: two of weight 1, filler, w
+    kc, vc = (torch.zeros(nb, KH, 16, D).to(torch.bfloat16)
+              for _ in range(2))
+    kc[..., 0] = -4096.0              # filler weighs nothing
+    x = (torch.rand(T, KH) * 0.9 + 0.05) * D ** 0.5
+    x = x.to(torch.bfloat16).double()
+    w = torch.exp(-x * torch.tensor(D ** -0.5, dtype=torch.float32).double())
+    target = w * (1 + 2.0 ** -14)
+    v1 = target.to(torch.bfloat16).double()
+    v2 = (target - v1).to(torch.bfloat16).double()
+
+    def row(t, key):
+        return int(bt[t, key // 16]), key % 16
+    for t in range(T):
+        b, o = row(t, n - 1)
+        kc[b, :, o, 0] = -x[t].to(torch.bfloat16)
+        vc[b, :, o] = -1.0
+        for key, v in ((0, v1), (1, v2)):
+            b, o = row(t, key)
+            kc[b, :, o, 0] = 0.0
+            vc[b, :, o] = v[t].to(torch.bfloat16)[:, None]
+    q = torch.zeros(T, KH, D).to(torch.bfloat16)
+    q[..., 0] = 1.0
+    sl = torch.full((T,), n, dtype=torch.int32)
+    out = ops.paged_attention(*(t.to(DEV) for t in (q, kc, vc, bt, sl)),
+                              D ** -0.5).cpu().double()
+    ref = (v1 + v2 - w) / (2 + w)
+    err = ((out - ref[..., None]) / ref[..., None]).abs()
+    assert err.max() < 2.0 ** -6, err.max()
