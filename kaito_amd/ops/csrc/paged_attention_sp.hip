@@ -76,6 +76,24 @@ KAITO_DEV float fold_weight(float m, float gm) {
   return __builtin_amdgcn_exp2f(m - gm);
 }
 
+// how a sequence's keys are shared out: 32-key tiles from the page that
+// holds the window's first key on, a contiguous run of `per` for every wave.
+// A split is the share of a workgroup's waves, so that with `used` == 1 the
+// first one has every key and writes the result itself.
+struct Spans {
+  int start, base, tiles, per, used;
+};
+KAITO_DEV Spans spans_of(const int seq_len, const int window, const int nsplit,
+                         const int nw) {
+  Spans p;
+  p.start = window > 0 && seq_len > window ? seq_len - window : 0;
+  p.base = p.start / BS * BS;
+  p.tiles = (seq_len - p.base + KT - 1) / KT;
+  p.per = (p.tiles + nsplit * nw - 1) / (nsplit * nw);
+  p.used = p.per > 0 ? (p.tiles + p.per * nw - 1) / (p.per * nw) : 1;
+  return p;
+}
+
 template <int D, bool FP8, int NW, bool SPLIT>
 __global__ __launch_bounds__(NW * 64, NW <= 4 ? 3 : (NW <= 8 ? 2 : 4))
 void paged_decode_kernel(const DecodeArgs a) {
@@ -94,16 +112,13 @@ void paged_decode_kernel(const DecodeArgs a) {
   const int QH = a.KH * a.G;
   const int* bt = a.block_tables + (int64_t)seq * a.max_blocks;
 
-  // keys from the page that holds the window's first; a contiguous run of
-  // tiles per wave
-  const int start = a.window > 0 && seq_len > a.window ? seq_len - a.window : 0;
-  const int base = start / BS * BS;
-  const int tiles = (seq_len - base + KT - 1) / KT;
   const int nsplit = SPLIT ? gridDim.y : 1, split = SPLIT ? blockIdx.y : 0;
-  // a split covers whole rounds of its workgroup's waves
-  const int per = (tiles + nsplit * NW - 1) / (nsplit * NW);
-  const int t0 = min(tiles, (split * NW + wave) * per);
-  const int t1 = min(tiles, t0 + per);
+  const Spans sp = spans_of(seq_len, a.window, nsplit, NW);
+  if (split >= sp.used) return;     // no keys: the fold does not look here
+  const bool partial = SPLIT && sp.used > 1;
+  const int start = sp.start, base = sp.base;
+  const int t0 = min(sp.tiles, (split * NW + wave) * sp.per);
+  const int t1 = min(sp.tiles, t0 + sp.per);
   const int last_page = (seq_len - 1) / BS;
 
   hbf16x8 qf[KK];
@@ -272,7 +287,8 @@ void paged_decode_kernel(const DecodeArgs a) {
     float gm = -1e30f;
 #pragma unroll
     for (int w = 0; w < NW; w++) gm = fmaxf(gm, s_m[w][g]);
-    const float sink = a.sinks && !SPLIT ? a.sinks[head] * LOG2E : -1e30f;
+    const float sink =
+        a.sinks && !partial ? a.sinks[head] * LOG2E : -1e30f;
     gm = fmaxf(gm, sink);
     float num = 0.f, den = 0.f;
 #pragma unroll
@@ -281,7 +297,7 @@ void paged_decode_kernel(const DecodeArgs a) {
       num += e * acc[(w * a.G + g) * D + d];
       den += e * s_l[w][g];
     }
-    if constexpr (SPLIT) {
+    if (partial) {
       const int64_t T = gridDim.x / a.KH;
       float* row = a.part + ((split * T + seq) * QH + head) * (D + 2);
       row[d] = num;
@@ -294,26 +310,35 @@ void paged_decode_kernel(const DecodeArgs a) {
   }
 }
 
-// one workgroup per (sequence, head): folds the splits
-template <int D>
-__global__ void paged_fold_kernel(short* __restrict__ out,
-                                  const float* __restrict__ part,
-                                  const float* __restrict__ sinks,
-                                  const int QH, const int splits) {
+// One workgroup per (sequence, head) folds the splits that had keys, unless
+// the first had them all. A chain of loads, so a short one: lane s of every
+// wave has split s's weight.
+template <int D, int NW>
+__global__ __launch_bounds__(D)
+void paged_fold_kernel(const DecodeArgs a, const int QH, const int splits) {
   const int64_t row = blockIdx.x, rows = gridDim.x;
-  const int d = threadIdx.x;
-  const float sink = sinks ? sinks[row % QH] * LOG2E : -1e30f;
-  float gm = sink;
-  for (int s = 0; s < splits; s++)
-    gm = fmaxf(gm, part[(s * rows + row) * (D + 2) + D]);
-  float num = 0.f, den = sinks ? fold_weight(sink, gm) : 0.f;
-  for (int s = 0; s < splits; s++) {
-    const float* p = part + (s * rows + row) * (D + 2);
-    const float e = fold_weight(p[D], gm);
-    num += e * p[d];
-    den += e * p[D + 1];
+  const int used =
+      spans_of(a.seq_lens[row / QH], a.window, splits, NW).used;
+  if (used == 1) return;
+  const int d = threadIdx.x, lane = d & 63;
+  const float sink = a.sinks ? a.sinks[row % QH] * LOG2E : -1e30f;
+  float m = -1e30f, l = 0.f;
+  if (lane < used) {
+    const float* p = a.part + (lane * rows + row) * (D + 2) + D;
+    m = p[0];
+    l = p[1];
   }
-  out[row * D + d] = f32_to_bf16(num / fmaxf(den, 1e-20f));
+  const float gm = fmaxf(wave_reduce_max(m), sink);
+  const float e = lane < used ? fold_weight(m, gm) : 0.f;
+  float den = wave_reduce_sum(e * l);
+  if (a.sinks) den += fold_weight(sink, gm);
+  float num = 0.f;
+#pragma unroll 4
+  for (int s = 0; s < used; s++)
+    num += __builtin_bit_cast(float, __builtin_amdgcn_readlane(
+               __builtin_bit_cast(int, e), s)) *
+        a.part[(s * rows + row) * (D + 2) + d];
+  a.out[row * D + d] = f32_to_bf16(num / fmaxf(den, 1e-20f));
 }
 
 template <int D, bool FP8>
@@ -323,7 +348,10 @@ void launch_decode(DecodeArgs a, const at::Tensor& out, int T) {
   // longest context that the table can hold: the lengths are on the device.
   // Few pairs on long tables: splits until 256 workgroups, as long as every
   // wave keeps two tiles (1 row of 16000 keys: 870 us in one workgroup per
-  // head before, 31 us in 32). Up to 256 pairs a workgroup has a CU to
+  // head before, 31 us in 32). Short contexts under such a table cost the
+  // fold's launch, whatever the table's width: 1 row of 217 keys 6.2 us under
+  // a table of its size and 10.1 under any wider one (11.0 in one workgroup of
+  // 4 waves; 27.4 where empty splits still stored and folded zeros). Up to 256 pairs a workgroup has a CU to
   // itself and takes 16 waves; above 512 pairs there are workgroups enough
   // and 4 waves fold less (2048 rows of 300 keys run at 5.5 TB/s).
   int64_t longest = (int64_t)a.max_blocks * BS;
@@ -339,9 +367,8 @@ void launch_decode(DecodeArgs a, const at::Tensor& out, int T) {
                                 out.options().dtype(at::kFloat));
     a.part = part.data_ptr<float>();
     PA_LAUNCH(WIDE, true, dim3(pairs, splits));
-    hipLaunchKernelGGL((paged_fold_kernel<D>), dim3(T * a.KH * a.G), dim3(D),
-                       0, stream, a.out, a.part, a.sinks, a.KH * a.G,
-                       (int)splits);
+    hipLaunchKernelGGL((paged_fold_kernel<D, WIDE>), dim3(T * a.KH * a.G),
+                       dim3(D), 0, stream, a, a.KH * a.G, (int)splits);
   } else if (pairs <= 256 && longest > 8 * KT) {
     PA_LAUNCH(WIDE, false, dim3(pairs));
   } else if (pairs <= 512 || D > 128) {

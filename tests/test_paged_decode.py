@@ -75,6 +75,16 @@ def test_launch_rules(KH, lens, max_blocks, D, fp8):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("window,sink", [(0, False), (0, True), (700, True)])
+def test_split_edges(D, window, sink):
+    """Under a table that asks for splits: sequences whose keys the first
+    workgroup has alone (16 tiles, 8 for wide heads) and one key more."""
+    _run(4, 2, D, [0, 1, 256, 257, 512, 513, 1024, 1025, 2048, 6000], 4096,
+         window, sink)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("D,KH,gap,max_blocks", [
     (128, 8, 2, 1), (128, 1, 40, 4), (64, 8, 20, 2), (256, 2, 700, 60),
     (128, 2, 5000, 400),              # other tiles, waves and splits
