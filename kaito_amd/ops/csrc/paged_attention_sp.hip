@@ -252,6 +252,17 @@ void paged_decode_kernel(const DecodeArgs a) {
       // the direct loads' data: this wave's own, so no barrier
       __builtin_amdgcn_s_waitcnt(0x0f70);     // vmcnt(0)
     }
+    if (!whole) {
+      // slots outside the sequence hold what their last user left, and a
+      // weight of zero does not silence an infinity
+#pragma unroll
+      for (int j = 0; j < LV; j++) {
+        const int key = key0 + j * (64 / CV) + lane / CV;
+        if (key < start || key >= seq_len)
+          *reinterpret_cast<short8_t*>(vl + (j * 64 + lane) * 8) =
+              short8_t{0, 0, 0, 0, 0, 0, 0, 0};
+      }
+    }
     __builtin_amdgcn_wave_barrier();
     // ---- O^T: dims 16 dt + 4 hi + r of head lo
 #pragma unroll

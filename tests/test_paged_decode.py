@@ -85,6 +85,40 @@ def test_split_edges(D, window, sink):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("window", [0, 20])
+def test_slots_outside_the_sequence(D, fp8, window):
+    """What a page's last user left behind the sequence's end, or before its
+    window, has no say, not even a NaN."""
+    lens = [1, 4, 8, 15, 16, 17, 28, 32, 36, 52]
+    bt = torch.arange(4 * len(lens), dtype=torch.int32).view(-1, 4)
+    kc, vc = (torch.randn(bt.numel(), 2, 16, D).to(torch.bfloat16)
+              for _ in range(2))
+    if fp8:
+        kc, vc = (t.to(torch.float8_e4m3fn).to(torch.bfloat16)
+                  for t in (kc, vc))
+    dead_k, dead_v = kc.clone(), vc.clone()
+    for i, n in enumerate(lens):
+        key = torch.arange(64).view(4, 16)
+        out = (key >= n) | (key < n - window if window else key < 0)
+        for t in (dead_k, dead_v):
+            t[bt[i].long()] = torch.where(
+                out[:, None, :, None], float("nan"), t[bt[i].long()].float()
+            ).to(torch.bfloat16)
+    q = torch.randn(len(lens), 4, D).to(torch.bfloat16)
+    sl = torch.tensor(lens, dtype=torch.int32)
+    got = []
+    for c in ((dead_k, dead_v), (kc, vc)):
+        if fp8:
+            c = tuple(t.to(torch.float8_e4m3fn).view(torch.uint8) for t in c)
+        got.append(ops.paged_attention(
+            q.to(DEV), *(t.to(DEV) for t in c), bt.to(DEV), sl.to(DEV),
+            D ** -0.5, window).cpu())
+    assert torch.equal(*got)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("D,KH,gap,max_blocks", [
     (128, 8, 2, 1), (128, 1, 40, 4), (64, 8, 20, 2), (256, 2, 700, 60),
     (128, 2, 5000, 400),              # other tiles, waves and splits
