@@ -15,12 +15,11 @@
 // 32 (53.2): x comes through the caches once per workgroup, so the gain ends
 // where its rows cost what those of W do.
 //
-// 4-bit weights run as integers: a word's nibbles j and j + 4 become the bf16
-// pair 128 + q by one shift and one and-or (x is permuted to match), and per
-// group of K, in f32,
-//     y += s (sum (128 + q) x) - (128 s + z) sum x
-// The offset costs 4 bits of the f32 partial sum's 24, out of a result
-// rounded to 8.
+// 4-bit weights run as integers. Read as fp8 (e4m3, subnormals and the first
+// binade), a byte of 0 to 15 is exactly q / 512: two masks and four packed
+// conversions turn a word's nibbles into bf16 (x is permuted to match), and
+// per group of K, in f32,
+//     y += 512 s (sum (q / 512) x) - z sum x
 #pragma once
 #include "common.h"
 
@@ -28,6 +27,7 @@ namespace kaito {
 namespace skinny {
 
 typedef __bf16 hbf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 hbf16x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 KAITO_DEV f32x4 mfma16(hbf16x8 a, hbf16x8 b, f32x4 c) {
@@ -126,18 +126,20 @@ KAITO_DEV void stream_tile(f32x4 (&acc)[MT],
   }
 }
 
-// the eight nibbles of a word as bf16 128 + q, in the order 0 4 1 5 2 6 3 7
+// the eight nibbles of a word as bf16 q / 512, in the order 0 2 4 6 1 3 5 7
 KAITO_DEV hbf16x8 nibbles(const unsigned int w) {
-  u32x4 r;
-#pragma unroll
-  for (int j = 0; j < 4; j++)
-    r[j] = ((w >> (4 * j)) & 0x000f000fu) | 0x43004300u;
-  return __builtin_bit_cast(hbf16x8, r);
+  const unsigned int even = w & 0x0f0f0f0fu, odd = (w >> 4) & 0x0f0f0f0fu;
+  const hbf16x2 a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 1.f, false);
+  const hbf16x2 b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 1.f, true);
+  const hbf16x2 c = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 1.f, false);
+  const hbf16x2 d = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 1.f, true);
+  return hbf16x8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
+constexpr float NIBBLE = 512.f;     // q over its bf16 form
 
 // x in that order
 KAITO_DEV hbf16x8 nibble_order(const hbf16x8 x) {
-  return __builtin_shufflevector(x, x, 0, 4, 1, 5, 2, 6, 3, 7);
+  return __builtin_shufflevector(x, x, 0, 2, 4, 6, 1, 3, 5, 7);
 }
 
 // 4-bit weights [N, K / 8]; WORDS words per lane and slice: a slice is
@@ -165,7 +167,7 @@ KAITO_DEV void accumulate_w4(f32x4 (&acc)[MT][NT],
 #pragma unroll
       for (int j = 0; j < NT; j++) {
         w[u][j] = load_stream<wordv>(wp[j] + k / 8);
-        s[u][j] = sc[j][k / group] * live;
+        s[u][j] = sc[j][k / group] * (live * NIBBLE);
         z[u][j] = ze[j][k / group] * live;
       }
 #pragma unroll
@@ -199,12 +201,11 @@ KAITO_DEV void accumulate_w4(f32x4 (&acc)[MT][NT],
       }
 #pragma unroll
       for (int j = 0; j < NT; j++) {
-        const float zz = 128.f * s[u][j] + z[u][j];
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
 #pragma unroll
           for (int r = 0; r < 4; r++)
-            acc[mt][j][r] += s[u][j] * dot[mt][j][r] - zz * xs[mt][r];
+            acc[mt][j][r] += s[u][j] * dot[mt][j][r] - z[u][j] * xs[mt][r];
       }
     }
   }
@@ -221,7 +222,6 @@ KAITO_DEV f32x4 fold(const f32x4* red, const int slot) {
 }
 
 // ---- M <= 4: rows streamed by a wave ---------------------------------------
-typedef __bf16 hbf16x2 __attribute__((ext_vector_type(2)));
 
 KAITO_DEV float dot8(const hbf16x8 a, const hbf16x8 b, float c) {
   const hbf16x2* p = reinterpret_cast<const hbf16x2*>(&a);
@@ -287,7 +287,7 @@ KAITO_DEV void stream_rows_w4(float (&acc)[M][R],
 #pragma unroll
     for (int r = 0; r < R; r++) {
       w[r] = load_stream<u32x4>(wp[r] + k / 8);
-      s[r] = sc[r][k / group] * live;
+      s[r] = sc[r][k / group] * (live * NIBBLE);
       z[r] = ze[r][k / group] * live;
     }
 #pragma unroll
@@ -317,9 +317,9 @@ KAITO_DEV void stream_rows_w4(float (&acc)[M][R],
     }
 #pragma unroll
     for (int r = 0; r < R; r++) {
-      const float zz = 128.f * s[r] + z[r];
 #pragma unroll
-      for (int m = 0; m < M; m++) acc[m][r] += s[r] * dot[m][r] - zz * xs[m];
+      for (int m = 0; m < M; m++)
+        acc[m][r] += s[r] * dot[m][r] - z[r] * xs[m];
     }
   }
 }

@@ -23,11 +23,12 @@ namespace kaito {
 
 // ---------------------------------------------------------------- gemv
 // M <= 4: a wave streams whole rows of packed weights, two or four of them
-// against the same x. One row of x: 15.1 us for N = 28672, K = 4096 (4.4
-// TB/s), 10.6 us for 4096 x 14336, 4.5 us for 4096 x 4096; with more rows the
-// vector unit is the bound (M = 2: 21.6, 17.2, 6.9 us). The linears of a
-// llama-3.1-8b layer at M = 2 took 124 us where a lane had 64 k of one row
-// and converted nibbles to f32 one by one.
+// against the same x. One row of x: 14.9 us for N = 28672, K = 4096 (66 MB
+// with the scales: 4.4 TB/s), 10.6 for 4096 x 14336, 4.3 for 4096 x 4096; with
+// more rows the vector unit is the bound (M = 2: 18.9, 13.2, 5.5 us). Lanes
+// with 64 k of one row that turned nibbles into f32 one by one took 36.2,
+// 19.1, 6.6 and 62.6, 32.0, 10.3 us; nibbles as bf16 128 + q, which cost the
+// sums 4 bits, 16.3, 11.3, 4.5 and 25.0, 16.6, 6.3.
 template <int M, int R>
 __global__ __launch_bounds__(256) void w4a16_stream_kernel(
     short* __restrict__ out, const short* __restrict__ x,
@@ -284,8 +285,8 @@ void w4a16_gemv(at::Tensor out, at::Tensor x, at::Tensor qweight,
                      dim3((N + 4 * R_ - 1) / (4 * R_)), dim3(256), 0, stream, \
                      W4_ARGS, N, K, (int)group)
   // four rows per wave share what they do with x once there are waves to
-  // spare (M = 4, N = 28672: 30.3 us against 38.6 with two; N = 6144: 12.8
-  // against 11.5)
+  // spare (M = 4, N = 28672: 32.3 us against 36.4 with two; N = 6144: 13.0
+  // against 10.3)
   const bool many = N >= 16384;
   switch (M) {
     case 1: W4_STREAM(1, 2); return;

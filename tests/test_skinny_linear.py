@@ -84,3 +84,30 @@ def test_packed_rows(M, N, K, G):
     assert ops.w4a16_streams(x, G)
     w = R.w4a16_unpack(qw.cpu(), s.cpu(), z.cpu(), G).to(DEV)
     _close(ops.w4a16_gemv(x, qw, s, z, G), x.double() @ w.double().T)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 16, 17, 32])
+@pytest.mark.parametrize("N,K,G", [(40, 2048, 128), (40, 1088, 64)])
+def test_packed_sums_keep_f32(M, N, K, G):
+    """Integers throughout, small ones beside one pair of +-2^20 in every
+    group that cancels. Sums of q x stay below 2^24 and are exact in f32 in
+    any order; so is the result up to its rounding to bf16. Sums of terms
+    larger than q x are not: at 143 times 2^20 the last 4 bits are lost."""
+    torch.manual_seed(M + G)
+    q = torch.randint(0, 16, (N, K))
+    x = torch.randint(-8, 9, (M, K)).float()
+    for g in range(0, K, G):
+        at = g + 16 * int(torch.randint(0, G // 16, ()))
+        i, j = at + int(torch.randint(0, 8, ())), at + int(
+            torch.randint(8, 16, ()))
+        x[:, i], x[:, j] = 2.0 ** 20, -2.0 ** 20
+        q[:, j] = q[:, i]             # cancels
+    words = (q.view(N, K // 8, 8) << (4 * torch.arange(8))).sum(-1)
+    words = torch.where(words >= 2 ** 31, words - 2 ** 32, words).int()
+    s = torch.ones(N, K // G)
+    z = torch.full((N, K // G), 8.0)
+    xd = x.to(torch.bfloat16).to(DEV)
+    out = ops.w4a16_gemv(xd, words.to(DEV), s.to(DEV), z.to(DEV), G).cpu()
+    ref = x.double() @ (q.double() - 8).T
+    assert torch.equal(out, ref.to(torch.bfloat16))
