@@ -35,7 +35,8 @@
 //   one prompt of 8192, 32/8 heads of 128: 140 -> 762 TFLOP/s;
 //   latent prompts 4 x 2048, 16 heads: 2307 us (padded to 256) -> 113 us;
 //   8192 suffix rows over 20000 paged keys: 140 -> 825 TFLOP/s;
-//   paged window 1024 with cap and penalty, 4 x 2048, 16/4 heads: 583 -> 155.
+//   paged window 1024 with cap and penalty, 4 x 2048, 16/4 heads: 583 -> 176
+//   (with the bare hardware reciprocal in cap and sigmoid 161).
 #pragma once
 #include "common.h"
 
@@ -107,6 +108,13 @@ KAITO_DEV void lds_copy16(const short* src, short* dst) {
 
 KAITO_DEV f32x16 mfma32(hbf16x8 a, hbf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// 1 / d for d >= 1, to a division's precision: one Newton step on the
+// hardware's reciprocal, which gives 0 by itself where the step would not end
+KAITO_DEV float recip(const float d) {
+  const float r = __builtin_amdgcn_rcpf(d);
+  return d > 0x1p125f ? r : fmaf(fmaf(-d, r, 1.0f), r, r);
 }
 
 // 4 rows x 16 columns per 16 lanes -> lane i: column i of the 4 rows
@@ -349,7 +357,7 @@ void flash_prefill_kernel(const Args a) {
       for (int kt = 0; kt < NK; kt++)
 #pragma unroll
         for (int i = 0; i < 16; i++)          // cap * tanh(s / cap), via exp
-          s[kt][i] = c2 - 2.0f * c2 * __builtin_amdgcn_rcpf(
+          s[kt][i] = c2 - 2.0f * c2 * recip(
               __builtin_amdgcn_exp2f(s[kt][i] * g2) + 1.0f);
     } else if (!fold) {
       const float c = qs * LOG2E;
@@ -397,7 +405,7 @@ void flash_prefill_kernel(const Args a) {
       for (int kt = 0; kt < NK; kt++)
 #pragma unroll
         for (int i = 0; i < 16; i++)          // a masked score weighs zero
-          s[kt][i] = __builtin_amdgcn_rcpf(
+          s[kt][i] = recip(
               1.0f + __builtin_amdgcn_exp2f(-s[kt][i] - hpb * LOG2E));
     } else {
       float mx = s[0][0];
