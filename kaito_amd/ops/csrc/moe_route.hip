@@ -10,7 +10,9 @@
 //     LOGITS: the choice is the logit itself, the weights are a softmax over
 //       the taken logits.
 //     Only the `keep` best groups stay eligible; the `top` largest eligible
-//     choices are taken (ties: lower index). Weights are the taken s
+//     choices are taken (ties: lower index; a NaN counts as larger than every
+//     number, and where fewer than `top` are above -inf the lowest indices
+//     among the others fill up). Weights are the taken s
 //     (without the correction), divided by their sum + 1e-20 when `renorm`,
 //     times `scale`. Outputs with index >= n_real are identity experts: their
 //     weights are also summed per token.
@@ -46,6 +48,8 @@ KAITO_DEV void wave_argmax(float& v, int& i) {
     if (ov > v || (ov == v && oi < i)) { v = ov; i = oi; }
   }
 }
+
+constexpr int NONE = 1 << 30;        // a lane without a candidate
 
 enum Mode { SOFTMAX = 0, SIGMOID = 1, LOGITS = 2 };
 
@@ -100,6 +104,10 @@ KAITO_DEV void route_row(const RouteArgs& a, const float* row, const int64_t t,
       }
     }
   }
+  // as in a sort, a NaN is larger than every number
+  auto rank = [](const float v) { return v == v ? v : INFINITY; };
+#pragma unroll
+  for (int r = 0; r < NPL; r++) ch[r] = rank(ch[r]);
   if (a.groups > 1) {
     const int n = N / a.groups;
     float mine = -INFINITY;                 // lane g: group g's score
@@ -128,15 +136,15 @@ KAITO_DEV void route_row(const RouteArgs& a, const float* row, const int64_t t,
       } else {
         score = wave_reduce_max(m);
       }
-      if (lane == g) mine = score;
+      if (lane == g) mine = rank(score);
     }
     unsigned long long kept = 0;
     for (int k = 0; k < a.keep; k++) {
-      float v = mine;
-      int i = lane;
+      const bool open = lane < a.groups && !((kept >> lane) & 1);
+      float v = open ? mine : -INFINITY;
+      int i = open ? lane : NONE;
       wave_argmax(v, i);
       kept |= 1ull << i;
-      if (lane == i) mine = -INFINITY;
     }
 #pragma unroll
     for (int r = 0; r < NPL; r++) {
@@ -146,19 +154,26 @@ KAITO_DEV void route_row(const RouteArgs& a, const float* row, const int64_t t,
   }
   float wsum = 0.f, mine = 0.f;             // lane k: k-th taken weight
   int mine_i = 0;
-  for (int k = 0; k < a.top; k++) {
+  unsigned open = 0;                        // outputs of this lane not taken
+#pragma unroll
+  for (int r = 0; r < NPL; r++)
+    if (r * 64 + lane < N) open |= 1u << r;
+  for (int k = 0; k < a.top; k++) {         // top <= N: one is always open
     float v = -INFINITY;
-    int i = min(lane, N - 1);
+    int i = NONE;
 #pragma unroll
     for (int r = 0; r < NPL; r++)
-      if (ch[r] > v) { v = ch[r]; i = r * 64 + lane; }
+      if ((open >> r & 1) && (ch[r] > v || i == NONE)) {
+        v = ch[r];
+        i = r * 64 + lane;
+      }
     wave_argmax(v, i);
     float sv = 0.f;
 #pragma unroll
     for (int r = 0; r < NPL; r++) {
       const float b = __shfl(s[r], i & 63, 64);
       if (r == (i >> 6)) sv = b;
-      if (r * 64 + lane == i) ch[r] = -INFINITY;
+      if (r * 64 + lane == i) open &= ~(1u << r);
     }
     wsum += sv;
     if (lane == k) { mine = sv; mine_i = i; }

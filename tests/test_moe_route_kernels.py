@@ -65,3 +65,51 @@ def test_sort_is_stable(T, top, n):
     topw = torch.rand(T, top, device=DEV)
     for a, b in zip(ops.moe_plan(topi, topw, n), R.moe_plan(topi, topw, n)):
         assert a.dtype == b.dtype and torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["softmax", "sigmoid", "logits"])
+@pytest.mark.parametrize("N,groups,keep,top,why", [
+    (16, 8, 1, 4, "groups"), (130, 10, 1, 20, "groups"), (8, 1, 1, 3, "-inf"),
+    (100, 4, 2, 6, "-inf"), (6, 3, 3, 6, "-inf")])
+def test_more_choices_than_eligible_outputs(mode, N, groups, keep, top, why):
+    """Outputs are taken once each: eligible ones first, then others at
+    their own score, as a sort leaves them."""
+    torch.manual_seed(N)
+    z, corr = torch.randn(5, N, device=DEV), None
+    if mode == "logits":
+        if why == "groups":
+            return                    # this mode has none
+        z[:, 1:] = float("-inf")
+        groups = keep = 1
+    elif why == "-inf":
+        corr = torch.full((N,), float("-inf"), device=DEV)
+        corr[N // 2:N // 2 + 2] = 0.5
+    a = (top, N, groups, keep, False, 1.0, mode)
+    gi, gw, _ = ops.moe_route(z, corr, *a)
+    wi, ww, _ = R.moe_route(z, corr, *a)
+    gi, wi = gi.long(), wi.long()
+    assert all(len(set(r)) == top for r in gi.tolist())
+    s = {"softmax": torch.softmax(z, -1), "sigmoid": torch.sigmoid(z),
+         "logits": torch.softmax(z, -1)}[mode]
+    assert torch.allclose(gw, s.gather(1, gi), atol=2e-6)
+    sure = 2 if why == "-inf" and mode != "logits" else \
+        1 if why == "-inf" else N // groups
+    assert torch.equal(gi[:, :sure], wi[:, :sure])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["softmax", "sigmoid", "logits"])
+@pytest.mark.parametrize("N,groups,keep", [(8, 1, 1), (70, 1, 1), (64, 8, 2)])
+def test_a_nan_is_not_passed_over(mode, N, groups, keep):
+    """A router that forms a NaN for one output shows it in the weights."""
+    torch.manual_seed(N)
+    z = torch.randn(6, N, device=DEV)
+    z[torch.arange(6), torch.arange(6) * (N // 6)] = float("nan")
+    if mode == "logits":
+        groups = keep = 1
+    a = (2, N, groups, keep, True, 1.0, mode)
+    got, want = ops.moe_route(z, None, *a), R.moe_route(z, None, *a)
+    assert torch.isnan(want[1]).any(1).all()
+    assert torch.isnan(got[1]).any(1).all()
+    assert all(len(set(r)) == 2 for r in got[0].tolist())
