@@ -532,6 +532,17 @@ def moe_route(logits, correction, top: int, n_real: int, groups: int = 1,
                                renorm, scale, mode)
 
 
+def _router_logits(x: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
+    """x gate^T in f32, whatever the operands and the number of rows: a
+    token's experts do not hang on the length of the step it came in. (bf16
+    logits, widened afterwards, take a launch more: 8192 rows of 2048 to 8
+    outputs 11.1 us, f32 ones 9.0; 32 rows of 7168 to 256 outputs 12.6 and
+    10.7.)"""
+    if x.is_cuda and x.dtype == gate.dtype == torch.bfloat16:
+        return torch.mm(x, gate.t(), out_dtype=torch.float32)
+    return torch.nn.functional.linear(x.float(), gate.float())
+
+
 def moe_gate_route(x, gate, correction, top: int, n_real: int,
                    groups: int = 1, keep: int = 1, renorm: bool = False,
                    scale: float = 1.0, mode: str = "softmax"):
@@ -551,8 +562,7 @@ def moe_gate_route(x, gate, correction, top: int, n_real: int,
                           n_real, groups, keep, renorm, scale,
                           ROUTE_MODES[mode])
         return topi, topw, w_id
-    logits = torch.nn.functional.linear(x.to(gate.dtype), gate).float()
-    return moe_route(logits, correction, top, n_real, groups, keep, renorm,
+    return moe_route(_router_logits(x, gate), correction, top, n_real, groups, keep, renorm,
                      scale, mode)
 
 

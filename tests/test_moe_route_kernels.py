@@ -113,3 +113,29 @@ def test_a_nan_is_not_passed_over(mode, N, groups, keep):
     assert torch.isnan(want[1]).any(1).all()
     assert torch.isnan(got[1]).any(1).all()
     assert all(len(set(r)) == 2 for r in got[0].tolist())
+
+
+@pytest.mark.parametrize("device", [
+    "cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("N", [8, 40, 130])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_choice_does_not_hang_on_the_step(device, N, dtype):
+    """Two outputs 2^-10 apart: the same experts and weights for a token
+    alone, in a short step and in a long one. Logits rounded to bf16 (2^-9)
+    would tie."""
+    torch.manual_seed(N)
+    H = 256
+    x = torch.ones(600, H).to(torch.bfloat16)
+    x[:, 1] = 2.0 ** -10
+    gate = torch.zeros(N, H)
+    gate[2, 0], gate[2, 1] = 1.0, -1.0    # 1 - 2^-10
+    gate[5, 0] = 1.0                      # 1
+    gate[7, 0], gate[7, 1] = 1.0, 1.0     # 1 + 2^-10
+    x, gate = x.to(device), gate.to(dtype).to(device)
+    w = None
+    for T in (1, 32, 512, 600):
+        i, topw, _ = ops.moe_gate_route(x[:T], gate, None, 3, N, renorm=True,
+                                        mode="logits")
+        assert (i.cpu() == torch.tensor([7, 5, 2])).all()
+        w = topw[:1].cpu() if w is None else w
+        assert torch.allclose(topw.cpu(), w, atol=1e-6)
