@@ -546,13 +546,18 @@ def _router_logits(x: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
 def moe_gate_route(x, gate, correction, top: int, n_real: int,
                    groups: int = 1, keep: int = 1, renorm: bool = False,
                    scale: float = 1.0, mode: str = "softmax"):
-    """moe_route of the logits x gate^T, formed in f32. One launch up to 64
-    outputs and 512 rows of bf16; a workgroup per row reads the whole router
-    (64 KB at 8 x 2048 f32), so that longer steps (32 rows: 5 us; 8192 rows:
-    270 MB to 540 MB through the caches) leave the product to the library."""
+    """moe_route of the logits x gate^T, formed in f32. One launch for short
+    steps and narrow routers: a workgroup per row reads the whole router, 8
+    outputs after one another, so that wider ones and longer steps leave the
+    product to the library (us, one launch and two; rows of 2048 and 7168, bf16
+    router: 8 outputs 5.1, 9.4 and 6.1, 13.2 at 32 rows, 5.7, 9.5 and 7.0, 11.4
+    at 512; 32 outputs 9.2, 9.6 and 12.2, 13.7 at 32 rows, 9.6, 9.6 and 13.3,
+    13.7 at 256, 10.3, 9.7 and 16.0, 13.9 at 512; 48 outputs 12.0, 9.5 and
+    16.5, 13.6 at 32)."""
     T = x.size(0)
     if x.is_cuda and x.dtype == torch.bfloat16 and T <= 512 \
-            and gate.size(0) <= 64 and gate.is_contiguous() \
+            and gate.size(0) <= 32 and T * gate.size(0) <= 8192 \
+            and gate.is_contiguous() \
             and gate.dtype in (torch.bfloat16, torch.float32) \
             and x.stride(1) == 1 and x.stride(0) % 8 == 0 \
             and x.size(1) % 8 == 0 and x.data_ptr() % 16 == 0 \

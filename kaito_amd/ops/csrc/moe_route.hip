@@ -25,8 +25,9 @@
 //
 // A decode step's choice is launches and latency, not work: as torch ops
 // (product, cast, top-k, softmax, sort, gathers, scatter, scan) it was about
-// 25 launches, 130 us of a layer's 240 at 32 tokens and 8 experts; these
-// two take 5 and 5 us there.
+// 25 launches, 130 us of a layer's 240 at 32 tokens and 8 experts. Now it is
+// 5.1 us for logits and choice (rows of 2048, one launch behind another; 9.5
+// where the row before has to arrive from its norm) and 4.8 for the sort.
 //
 // An output's place in the row lives in lane e % 64, register e / 64.
 #include "mix_common.h"
@@ -199,7 +200,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(
   route_row<NPL, MODE>(a, logits + t * a.N, t, threadIdx.x & 63);
 }
 
-constexpr int GATE_MAX = 64;         // experts whose logits a workgroup forms
+constexpr int GATE_MAX = 32;         // outputs whose logits a workgroup forms
 
 KAITO_DEV float dot_gate(const skinny::hbf16x8 x, const short* w, float c) {
   return skinny::dot8(x, skinny::load_x(w), c);

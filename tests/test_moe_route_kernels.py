@@ -139,3 +139,16 @@ def test_choice_does_not_hang_on_the_step(device, N, dtype):
         assert (i.cpu() == torch.tensor([7, 5, 2])).all()
         w = topw[:1].cpu() if w is None else w
         assert torch.allclose(topw.cpu(), w, atol=1e-6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,N", [(1, 32), (256, 32), (257, 32), (341, 24),
+                                 (342, 24), (512, 16), (513, 16), (1, 33)])
+def test_choice_on_both_sides_of_the_rule(T, N):
+    torch.manual_seed(T)
+    x = torch.randn(T, 64, device=DEV).to(torch.bfloat16)
+    gate = torch.randn(N, 64, device=DEV).to(torch.bfloat16) / 4
+    z = (x.double() @ gate.double().T).float()
+    a = (2, N, 1, 1, True, 1.0, "softmax")
+    _check(ops.moe_gate_route(x, gate, None, *a),
+           R.moe_route(z, None, *a), N)
