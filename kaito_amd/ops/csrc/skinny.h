@@ -11,9 +11,10 @@
 // Up to 32 rows of x, and experts with a few rows each: the same streams
 // through LDS into v_mfma_f32_16x16x32_bf16 (stream_tile). A workgroup owns
 // 16 rows of W; its waves take every fourth slice of K and meet in LDS, in
-// f32. 28672 x 4096: 44.5 us at M = 8 (library 53.0), 50.5 at 16 (53.8), 74.6 at
-// 32 (53.2): x comes through the caches once per workgroup, so the gain ends
-// where its rows cost what those of W do.
+// f32. 28672 x 4096: 44.4 us at M = 8 (library 56.8), 50.9 at 16 (57.4), 72.8 at
+// 32 (48.6): x comes through the caches once per workgroup, so the gain ends
+// where its rows cost what those of W do. K in stages of 64, 2880 x 2880: 6.5
+// at 8 (16.3), 6.8 at 16 (16.4).
 //
 // 4-bit weights run as integers. Read as fp8 (e4m3, subnormals and the first
 // binade), a byte of 0 to 15 is exactly q / 512: two masks and four packed
@@ -69,6 +70,7 @@ KAITO_DEV int tile_col(const int j, const int lane) {
 
 template <int N>
 KAITO_DEV void wait_loads() {       // until N of this wave's loads are left
+  __builtin_amdgcn_sched_barrier(0);        // every one of them is issued
   __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14));
   asm volatile("" ::: "memory");
 }
@@ -99,16 +101,7 @@ KAITO_DEV void stream_tile(f32x4 (&acc)[MT],
               ring + b * 16 * KS + j * 512),
           16, 0, 2 /* non-temporal */);
   };
-  auto step = [&](const int s, const int b) {
-    // the other stage's reads are done before it is overwritten
-    __builtin_amdgcn_s_waitcnt(0xc07f);
-    asm volatile("" ::: "memory");
-    if (s + TILE_NW < n) {
-      fetch(s + TILE_NW, b ^ 1);
-      wait_loads<MT * STEPS + NI>();
-    } else {
-      wait_loads<0>();
-    }
+  auto multiply = [&](const int b) {
     const short* w = ring + b * 16 * KS + lo * KS;
 #pragma unroll
     for (int i = 0; i < STEPS; i++) {
@@ -119,10 +112,32 @@ KAITO_DEV void stream_tile(f32x4 (&acc)[MT],
         acc[mt] = mfma16(xf[b][mt][i], wf, acc[mt]);
     }
   };
-  if (wave < n) fetch(wave, 0);
-  for (int s = wave; s < n; s += 2 * TILE_NW) {
+  // Every step fetches or none does: where the two met in one product, the
+  // compiler could no longer count the loads and waited for all of them.
+  auto step = [&](const int s, const int b) {
+    // the other stage's reads are done before it is overwritten
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    asm volatile("" ::: "memory");
+    fetch(s + TILE_NW, b ^ 1);
+    wait_loads<MT * STEPS + NI>();
+    multiply(b);
+  };
+  auto last = [&](const int b) {
+    wait_loads<0>();
+    multiply(b);
+  };
+  if (wave >= n) return;
+  fetch(wave, 0);
+  int s = wave;
+  for (; s + 2 * TILE_NW < n; s += 2 * TILE_NW) {
     step(s, 0);
-    if (s + TILE_NW < n) step(s + TILE_NW, 1);
+    step(s + TILE_NW, 1);
+  }
+  if (s + TILE_NW < n) {
+    step(s, 0);
+    last(1);
+  } else {
+    last(0);
   }
 }
 
