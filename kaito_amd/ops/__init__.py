@@ -145,14 +145,24 @@ def _skinny(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
     """Whether x W^T runs on the weight-streaming kernels: a few rows of
     bf16 on the GPU, 16-byte aligned rows, nothing to differentiate.
 
-    Up to 4 rows always: at 8 llama-3.1-8b layers' sizes W is read at 5 to 7
-    TB/s for one row and 3.6 to 4.9 for four, by hipBLASLt's tuned choices at
-    2.2 to 4.8 for both. Beyond, x comes through the caches once per 16 rows
-    of W, and the library is ahead from where that costs more (us, streamed
-    and library): 8 rows win but for the longest K (28672 x 4096: 44.5, 53.0;
-    4096 x 14336: 25.9, 25.1); 16 rows up to 4096 x 4096 (11.2, 15.4; 6144 x
-    4096: 15.9, 14.4) and in a SwiGLU pair; 32 rows up to 3072 x 2048 (7.9,
-    11.4; 6144 x 2048: 13.3, 12.4, where a SwiGLU pair saves its launch)."""
+    The lines, with us on both sides (streamed, library; weights out of the
+    caches): beyond 4 rows x comes through the caches once per 16 rows of W,
+    and the library is ahead from where that costs more.
+    Up to 4 rows always (28672 x 4096: 34.6, 56.3 for one row and 41.1, 55.9
+    for four; 4096 x 4096: 7.2, 15.3 and 9.2, 15.5; a tie or 6 % behind at
+    576 x 7168 and 2560 x 10240 for four).
+    Up to 8: all but few rows of W with a long K (576 x 7168: 9.5, 8.2 at 8)
+    and counts of rows that go unevenly on the CUs (5120 x 5120: 15.7, 14.5;
+    as a SwiGLU pair 15.8, 16.9).
+    Up to 16: to 4096 x 4096 (10.7, 15.5; 6144 x 4096: 16.3, 14.4) and K of
+    7168 (2112 x 7168: 12.7, 12.6; 2048 x 8192: 14.6, 13.1); SwiGLU pairs,
+    which save a launch, to 8192 (28672 x 4096: 50.3, 60.5), uneven ones
+    excepted (5120 x 5120: 19.1, 17.9).
+    Up to 32: to 3072 x 2048 (7.4, 11.5; 6144 x 2048: 13.0, 12.6, as a pair
+    12.5, 15.0) and K of 4096 (1024 x 4096: 10.1, 11.3 at 24), where beyond 24
+    rows the library has another kernel for few rows of W and K of 2560 and
+    more (1024 x 2560: 8.0, 6.9; 2048 x 2816: 8.8, 9.5; 1024 x 2816 as a pair
+    9.0, 9.5)."""
     if not (x.is_cuda and x.dim() == 2 and 1 <= x.size(0) <= 32
             and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and w.is_contiguous() and w.size(1) % 8 == 0 and w.numel() > 0
@@ -167,11 +177,16 @@ def _skinny(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
         return True
     if K % 64 or N % 16:
         return False
+    if M <= 16 and N < 1024 and K > 5120 and not glu:
+        return False
+    uneven = 4096 < N < 7168 and K > 4096
     if M <= 8:
-        return K <= 8192
+        return (K <= 8192 or N >= 4096) and (glu or not uneven)
     if M <= 16:
-        return N * K <= 4096 * 4096 or (glu and K <= 8192)
-    return N * K <= (6144 if glu else 3072) * 2048
+        return K <= 8192 and not uneven if glu \
+            else N * K <= 4096 * 4096 and K <= 7168
+    return N * K <= (6144 if glu else 3072) * 2048 and K <= 4096 and (
+        M <= 24 or K < 2560 or N >= 2048 or glu)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:

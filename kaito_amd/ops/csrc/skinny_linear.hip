@@ -103,6 +103,16 @@ __global__ __launch_bounds__(256, 2) void skinny_tile_kernel(
 
 constexpr int MAX_M = 32;
 
+// Rows of W streamed whole, or tiles of 16 through LDS? Beyond 4 rows of x
+// tiles. 3 and 4 rows are about even while W is small and tile counts go
+// unevenly on 256 CUs (5120 x 5120 at 4 rows: 13.6 us, 14.5 in tiles; 4096 x
+// 4096 9.2, 8.7); beyond 2^25 weights the row kernel's sums are the bound
+// (28672 x 4096: 49.4, 41.7; 128256 x 4096: 217, 164).
+bool in_tiles(int64_t M, int64_t N, int64_t K, int64_t cols, int64_t weights) {
+  return M > 4 || (M > 2 && weights > (1ll << 25) && K % 64 == 0 &&
+                   N % cols == 0);
+}
+
 void check(const at::Tensor& out, const at::Tensor& x, const at::Tensor& w,
            int64_t N, int64_t cols) {
   for (const auto& t : {out, x, w})
@@ -146,7 +156,7 @@ void skinny_linear(at::Tensor out, at::Tensor x, at::Tensor w,
       dim3(256), 0, at::hip::getCurrentHIPStream(), (short*)out.data_ptr(),   \
       (const short*)x.data_ptr(), x.stride(0), (const short*)w.data_ptr(),    \
       has_bias ? (const short*)bias.data_ptr() : nullptr, M, (int)N, (int)w.size(1))
-  if (M > 4) {
+  if (in_tiles(M, N, w.size(1), 16, w.numel())) {
     if (w.size(1) % 256 == 0) {
       if (M > 16) SLT_LAUNCH(2, 256); else SLT_LAUNCH(1, 256);
     } else {
@@ -175,7 +185,7 @@ void skinny_swiglu(at::Tensor out, at::Tensor x, at::Tensor w) {
       dim3(256), 0, at::hip::getCurrentHIPStream(), (short*)out.data_ptr(),   \
       (const short*)x.data_ptr(), x.stride(0), (const short*)w.data_ptr(),    \
       nullptr, M, (int)N, (int)w.size(1))
-  if (M > 4) {
+  if (in_tiles(M, N, w.size(1), 8, w.numel())) {
     if (w.size(1) % 256 == 0) {
       if (M > 16) SGT_LAUNCH(2, 256); else SGT_LAUNCH(1, 256);
     } else {

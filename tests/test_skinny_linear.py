@@ -55,6 +55,21 @@ def test_tiles(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [2, 3, 4])
+@pytest.mark.parametrize("N,K", [(4096, 8192), (4128, 8192), (4104, 8192),
+                                 (4128, 8200)])
+def test_large_weights(M, N, K):
+    """3 and 4 rows on both sides of 2^25 weights, in whole tiles or not."""
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    w = torch.randn(N, K, device=DEV).to(torch.bfloat16)
+    ref = x.double() @ w.double().T
+    _close(ops.linear(x, w), ref)
+    g, u = ref.chunk(2, -1)
+    _close(ops.linear_swiglu(x, w), g * torch.sigmoid(g) * u)
+
+
+@pytest.mark.gpu
 def test_other_forms_stay_with_the_library():
     x = torch.randn(33, 64, device=DEV).to(torch.bfloat16)
     w = torch.randn(32, 64, device=DEV).to(torch.bfloat16)
