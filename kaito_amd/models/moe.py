@@ -143,6 +143,8 @@ class MoEMLP(nn.Module):
             mode, renorm, scale = "logits", False, 1.0
         else:
             mode = "softmax"
+        if groups <= 1:             # no limit, whatever the number kept says
+            groups = keep = 1
         # f32 router: x is widened before the product
         return ops.moe_gate_route(x, self.gate, bias, self.top_k,
                                   self.num_experts, groups, keep, renorm,

@@ -152,3 +152,30 @@ def test_choice_on_both_sides_of_the_rule(T, N):
     a = (2, N, 1, 1, True, 1.0, "softmax")
     _check(ops.moe_gate_route(x, gate, None, *a),
            R.moe_route(z, None, *a), N)
+
+
+@pytest.mark.parametrize("device", [
+    "cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("n_group,topk_group", [(1, 1), (1, 4), (0, 0),
+                                                (1, 0), (4, 4)])
+@pytest.mark.parametrize("routing", ["noaux_tc", "sigmoid_groups"])
+def test_layers_without_a_group_limit(device, n_group, topk_group, routing):
+    """Counts of kept groups mean nothing where there is one group or none."""
+    from kaito_amd.engine.config import ModelConfig
+    from kaito_amd.models.moe import MoEMLP
+    from kaito_amd.parallel.state import init_parallel
+    init_parallel(1)
+    torch.manual_seed(2)
+    m = MoEMLP(ModelConfig(
+        name="t", hidden_size=64, num_experts=8, num_experts_per_tok=3,
+        moe_intermediate_size=64, moe_routing=routing, n_group=n_group,
+        topk_group=topk_group)).requires_grad_(False)
+    for p in m.parameters():
+        p.normal_(0, 0.2)
+    x = torch.randn(9, 64).to(torch.bfloat16)
+    s = torch.sigmoid(x.float() @ m.gate.float().T)
+    sel = s + m.e_score_correction_bias if routing == "noaux_tc" else s
+    want = sel.topk(3, -1)[1]
+    got = m.to(device)._choose(x.to(device))[0].cpu()
+    assert torch.equal(got.long().sort(-1)[0], want.sort(-1)[0])
+    assert torch.isfinite(m(x.to(device)).float()).all()
