@@ -4,14 +4,13 @@ Replaces vLLM's fused-MoE CUDA path for the MoE presets in the reference
 catalog (gpt-oss-120b / Qwen MoE presets in
 supported_models.yaml).
 
-Round 2: the GPU path is FUSED and host-sync-free — tokens are sorted by
-expert on the device and two HIP grouped-GEMM kernels (ops/csrc/moe.hip for
-decode-sized steps, moe_gemm.hip for prompts) consume (sorted_ids, offsets)
-directly: gather→gate/up GEMM→silu·mul,
-then down GEMM→weighted scatter-add. Worst-case tile grids make every
-shape static, so MoE decode steps capture into hipGraphs (the round-1
-per-expert torch loop read expert counts on the host each layer, forcing
-eager decode — docs/ROADMAP.md #3).
+The GPU path needs no host read: two launches choose the experts and sort
+the (token, expert) pairs by expert (ops/csrc/moe_route.hip), grouped products
+gather the rows, apply the activation and go down again behind the device's
+offsets (ops/csrc/moe.hip for decode-sized steps, moe_gemm.hip for prompts),
+and one launch sums every token's rows with their weights, the identity
+experts' share and the shared expert. Worst-case tile grids make every shape
+static, so MoE decode steps capture into hipGraphs.
 
 Parallelism at tp>1:
   * EP (expert parallel) when num_experts % tp == 0: each rank owns
@@ -150,15 +149,6 @@ class MoEMLP(nn.Module):
                                   self.num_experts, groups, keep, renorm,
                                   scale, mode)
 
-    def _route(self, x: torch.Tensor):
-        """Device-only top-k routing + expert sort. Returns
-        (sorted_tok int32 [TK], gates f32 [TK], offsets int32 [E+1],
-        weight f32 [T] on identity experts or None)."""
-        topi, topw, w_id = self._choose(x)
-        # identity outputs sort behind every expert's rows
-        return ops.moe_sort(topi, topw, self.n_route) \
-            + (w_id if self.n_identity else None,)
-
     # Pairs up to which the weight-streaming kernels run, beyond it the tiled
     # grouped GEMMs: 16 rows per expert. Streamed and tiled, in us: 8 experts
     # of 2048 x 2048 at 16 rows 59 and 79, at 32 99 and 82; 8 of 4096 x 14336
@@ -250,28 +240,17 @@ class MoEMLP(nn.Module):
                              self.b_down)
         return y
 
-    def _gated_rows(self, x, sorted_tok, offsets):
+    def _rows_streamed(self, x, sorted_tok, offsets):
         act = torch.empty(sorted_tok.numel(), self.ie_local, dtype=x.dtype,
                           device=x.device)
         ops.moe_gate_silu(act, x, self.w_gate_up, sorted_tok, offsets,
                           self.e_base, self.e_local, self.b_gate_up,
                           self.act_mode, self.act_limit)
-        return act
-
-    def _rows_streamed(self, x, sorted_tok, offsets):
-        act = self._gated_rows(x, sorted_tok, offsets)
         y = torch.empty(sorted_tok.numel(), x.size(1), dtype=torch.float32,
                         device=x.device)
         ops.moe_down_rows(y, act, self.w_down, offsets, self.e_base,
                           self.e_local, self.b_down)
         return y
-
-    def _forward_fused(self, x, sorted_tok, gates, offsets, out32):
-        """The streaming kernels with the weighted rows added into out32."""
-        act = self._gated_rows(x, sorted_tok, offsets)
-        ops.moe_down_scatter(out32, act, self.w_down, sorted_tok, gates,
-                             offsets, self.e_base, self.e_local,
-                             self.b_down)
 
     def _forward_loop(self, x, sorted_tok, gates, offsets, out):
         """Per-expert torch GEMMs (_kernels_for). Host sync on the segment

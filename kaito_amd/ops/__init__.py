@@ -29,7 +29,7 @@ for _g, _names in {
     "attn": ("paged_attention paged_attention_sp prefill_attention "
              "mla_prefill_attention context_attention mfma_tile_gemm paged_read_bw"),
     "mla": "mla_decode mla_prepare head_rows mla_cache_write",
-    "moe": ("moe_gate_silu moe_down_rows moe_down_scatter moe_grouped_up "
+    "moe": ("moe_gate_silu moe_down_rows moe_grouped_up "
             "moe_grouped_down moe_combine"),
     "route": "moe_route moe_gate_route moe_sort",
     "quant": "w4a16_gemv w4a16_dequant w4a16_gemm lora_shrink lora_expand",
@@ -475,21 +475,6 @@ def moe_down_rows(y, act, w_down, offsets, e_base: int, n_local_experts: int,
     product (+ optional [E, H] bias) of every sorted row."""
     _K.moe_down_rows(y, act, w_down, offsets, _none(bias, act), e_base,
                      n_local_experts)
-
-
-def moe_down_scatter(out: torch.Tensor, act: torch.Tensor,
-                     w_down: torch.Tensor, sorted_ids: torch.Tensor,
-                     gates: torch.Tensor, offsets: torch.Tensor,
-                     e_base: int, n_local_experts: int,
-                     bias: torch.Tensor | None = None) -> None:
-    """Fused MoE stage 2 (GPU only): down grouped GEMM (+ optional
-    [E, H] bias) + gated f32 atomic scatter into `out`."""
-    b = bias if bias is not None else         torch.empty(0, dtype=act.dtype, device=act.device)
-    _K.moe_down_scatter(out, act, w_down, sorted_ids, gates,
-                                     offsets, b, e_base, n_local_experts)
-
-
-MOE_ROUTE_MAX = (1024, 64, 64)      # router outputs, chosen, groups
 
 
 def moe_grouped_up(act, x, w, sorted_ids, offsets, e_base: int, bias=None,

@@ -10,8 +10,7 @@
 //     gathered through sorted_ids (ungated experts, act_mode 2: relu(.)^2). A
 //     workgroup's 16 weight rows are 8 gate rows and their 8 up rows;
 //   * moe_down_rows: y[s] = act[s] Wd^T in f32, summed per token by
-//     moe_combine; moe_down_scatter: out[tok] += gate * the same by f32
-//     atomics.
+//     moe_combine.
 //
 // One workgroup per (16 weight rows, expert); an expert with more rows than 16
 // MT is walked in passes, whose weights come back from the caches. Measured
@@ -35,16 +34,15 @@ struct StreamArgs {
   const short* w;                   // [E local, rows, K]
   const short* bias;                // [E local, rows] or nullptr
   const int* rows;                  // token of a sorted row
-  const float* gates;               // SCATTER: weight of a sorted row
   const int* offsets;               // [global E + 1]
   int e_base, N, K;
   int act_mode;
   float limit;
   short* act;                       // up: [TK, N]
-  float* y;                         // down: [TK, N], SCATTER: [T, N]
+  float* y;                         // down: [TK, N]
 };
 
-enum Kind { UP_GATED, UP_PLAIN, DOWN, SCATTER };
+enum Kind { UP_GATED, UP_PLAIN, DOWN };
 
 // act_mode 1: clamped swiglu — gate=min(g,limit), up=clamp(u,±limit),
 // (up+1) * gate*sigmoid(1.702*gate); gpt-oss uses limit 7
@@ -87,7 +85,7 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const StreamArgs a) 
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
       const int m = min(m0 + mt * 16 + (lane & 15), end - 1);
-      const int64_t row = KIND == UP_GATED || KIND == UP_PLAIN ? a.rows[m] : m;
+      const int64_t row = KIND == DOWN ? m : a.rows[m];
       xp[mt] = a.x + row * a.K + (lane >> 4) * 8;
     }
     f32x4 acc[MT];
@@ -116,11 +114,8 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const StreamArgs a) 
         } else if constexpr (KIND == UP_PLAIN) {
           const float p = fmaxf(v[r], 0.f);
           a.act[(int64_t)m * a.N + n0 + c] = f32_to_bf16(p * p);
-        } else if constexpr (KIND == DOWN) {
-          a.y[(int64_t)m * a.N + n0 + c] = v[r];
         } else {
-          atomicAdd(&a.y[(int64_t)a.rows[m] * a.N + n0 + c],
-                    a.gates[m] * v[r]);
+          a.y[(int64_t)m * a.N + n0 + c] = v[r];
         }
       }
     }
@@ -150,32 +145,6 @@ void launch_stream(const StreamArgs& a, int64_t E_local, int64_t pairs,
 void check16(const at::Tensor& t) {
   TORCH_CHECK(t.is_cuda() && t.dtype() == at::kBFloat16 &&
               t.is_contiguous() && (uintptr_t)t.data_ptr() % 16 == 0);
-}
-
-StreamArgs down_args(const at::Tensor& out, const at::Tensor& act,
-                     const at::Tensor& w_down, const at::Tensor& offsets,
-                     const at::Tensor& bias, int64_t e_base,
-                     int64_t n_local_experts) {
-  TORCH_CHECK(out.is_cuda() && out.dtype() == at::kFloat &&
-              out.is_contiguous() && offsets.dtype() == at::kInt);
-  check16(act); check16(w_down);
-  StreamArgs a{};
-  a.N = out.size(1); a.K = act.size(1);
-  TORCH_CHECK(a.N % 64 == 0 && a.K % 64 == 0);
-  TORCH_CHECK(w_down.size(1) == a.N && w_down.size(2) == a.K &&
-              w_down.size(0) >= n_local_experts &&
-              offsets.numel() > e_base + n_local_experts);
-  if (bias.numel() > 0) {
-    TORCH_CHECK(bias.dtype() == at::kBFloat16 && bias.is_contiguous() &&
-                bias.numel() == w_down.size(0) * a.N);
-    a.bias = (const short*)bias.data_ptr();
-  }
-  a.x = (const short*)act.data_ptr();
-  a.w = (const short*)w_down.data_ptr();
-  a.offsets = offsets.data_ptr<int>();
-  a.e_base = (int)e_base;
-  a.y = out.data_ptr<float>();
-  return a;
 }
 
 }  // namespace
@@ -220,27 +189,28 @@ void moe_gate_silu(at::Tensor act, at::Tensor x, at::Tensor w_gate_up,
 void moe_down_rows(at::Tensor y, at::Tensor act, at::Tensor w_down,
                    at::Tensor offsets, at::Tensor bias, int64_t e_base,
                    int64_t n_local_experts) {
-  const StreamArgs a = down_args(y, act, w_down, offsets, bias, e_base,
-                                 n_local_experts);
-  TORCH_CHECK(act.size(0) >= y.size(0));
+  TORCH_CHECK(y.is_cuda() && y.dtype() == at::kFloat && y.is_contiguous() &&
+              offsets.dtype() == at::kInt);
+  check16(act); check16(w_down);
+  StreamArgs a{};
+  a.N = y.size(1); a.K = act.size(1);
+  TORCH_CHECK(a.N % 64 == 0 && a.K % 64 == 0);
+  TORCH_CHECK(w_down.size(1) == a.N && w_down.size(2) == a.K &&
+              w_down.size(0) >= n_local_experts &&
+              offsets.numel() > e_base + n_local_experts &&
+              act.size(0) >= y.size(0));
+  if (bias.numel() > 0) {
+    TORCH_CHECK(bias.dtype() == at::kBFloat16 && bias.is_contiguous() &&
+                bias.numel() == w_down.size(0) * a.N);
+    a.bias = (const short*)bias.data_ptr();
+  }
   if (y.size(0) == 0 || n_local_experts == 0 || a.N == 0) return;
+  a.x = (const short*)act.data_ptr();
+  a.w = (const short*)w_down.data_ptr();
+  a.offsets = offsets.data_ptr<int>();
+  a.e_base = (int)e_base;
+  a.y = y.data_ptr<float>();
   launch_stream<DOWN>(a, n_local_experts, y.size(0), offsets.numel() - 1);
-}
-
-void moe_down_scatter(at::Tensor out, at::Tensor act, at::Tensor w_down,
-                      at::Tensor sorted_ids, at::Tensor gates,
-                      at::Tensor offsets, at::Tensor bias, int64_t e_base,
-                      int64_t n_local_experts) {
-  StreamArgs a = down_args(out, act, w_down, offsets, bias, e_base,
-                           n_local_experts);
-  TORCH_CHECK(gates.dtype() == at::kFloat && sorted_ids.dtype() == at::kInt &&
-              gates.numel() == sorted_ids.numel() &&
-              act.size(0) >= sorted_ids.numel());
-  if (sorted_ids.numel() == 0 || n_local_experts == 0 || a.N == 0) return;
-  a.rows = sorted_ids.data_ptr<int>();
-  a.gates = gates.data_ptr<float>();
-  launch_stream<SCATTER>(a, n_local_experts, sorted_ids.numel(),
-                         offsets.numel() - 1);
 }
 
 }  // namespace kaito

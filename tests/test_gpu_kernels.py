@@ -678,8 +678,9 @@ def test_engine_gpu_mixed_overlap_matches_classic():
     (64, 256, 1024, 4, 4),     # wide intermediate, top-4
 ])
 def test_moe_fused_grouped_gemms(T, H, IE, E, K):
-    """The host-sync-free MoE path (sorted ids + offsets → gather GEMM →
-    silu·mul → down GEMM → gated scatter) vs an fp32 per-expert loop."""
+    """The host-sync-free MoE layer (sorted ids + offsets → gather GEMM →
+    silu·mul → down GEMM → weighted sum per token), streamed and tiled, vs
+    an fp32 per-expert loop."""
     from kaito_amd.models.moe import MoEMLP
     from kaito_amd.engine.config import ModelConfig
     from kaito_amd.parallel.state import init_parallel
@@ -692,9 +693,12 @@ def test_moe_fused_grouped_gemms(T, H, IE, E, K):
         for p in m.parameters():
             p.normal_(0, 0.05)
     x = _bf16(T, H, scale=0.5)
-    sorted_tok, gates, offsets, _ = m._route(x)
-    out_fused = torch.zeros(T, H, dtype=torch.float32, device=DEV)
-    m._forward_fused(x, sorted_tok, gates, offsets, out_fused)
+    sorted_tok, gates, offsets, _ = ops.moe_plan(*m._choose(x)[:2], E)
+    outs = []
+    for most, kernels in ((T * K, "streamed"), (0, "tiled")):
+        m.FUSED_MAX_TOKENS = most
+        assert m._kernels_for(x) == kernels
+        outs.append(m(x, keep_f32=True))
     # fp32 oracle on the same routing
     off = offsets.tolist()
     expect = torch.zeros(T, H, dtype=torch.float32, device=DEV)
@@ -709,7 +713,8 @@ def test_moe_fused_grouped_gemms(T, H, IE, E, K):
         act = torch.nn.functional.silu(g) * u
         y = act @ m.w_down[e].float().T
         expect.index_add_(0, idx[s:t], y * gates[s:t, None])
-    _close(out_fused, expect, atol=5e-2, rtol=5e-2)
+    for out in outs:
+        _close(out, expect, atol=5e-2, rtol=5e-2)
 
 
 def test_moe_engine_decode_uses_graphs_on_gpu():

@@ -17,14 +17,12 @@ wd = (torch.randn(E, H, IE, device=dev) * 0.02).to(torch.bfloat16)
 flat_e = torch.arange(TK, device=dev) % E
 order = torch.argsort(flat_e)
 sorted_tok = (torch.arange(TK, device=dev) // K_TOP).int()[order]
-gates = torch.full((TK,), 0.5, device=dev)
 counts = torch.bincount(flat_e, minlength=E).int()
 offsets = torch.zeros(E + 1, dtype=torch.int32, device=dev)
 torch.cumsum(counts, 0, out=offsets[1:].long()) if False else None
 offsets[1:] = torch.cumsum(counts, 0)
-pad = (TK + 63) // 64 * 64 + 64
-act = torch.empty(pad, IE, dtype=torch.bfloat16, device=dev)
-out32 = torch.zeros(T, H, dtype=torch.float32, device=dev)
+act = torch.empty(TK, IE, dtype=torch.bfloat16, device=dev)
+rows = torch.empty(TK, H, dtype=torch.float32, device=dev)
 
 def t(f, n=50):
     for _ in range(10): f()
@@ -33,11 +31,11 @@ def t(f, n=50):
     torch.cuda.synchronize(); return (time.perf_counter() - t0) / n * 1e6
 
 us_a = t(lambda: ops.moe_gate_silu(act, x, wgu, sorted_tok, offsets, 0, E))
-us_b = t(lambda: ops.moe_down_scatter(out32, act, wd, sorted_tok, gates, offsets, 0, E))
+us_b = t(lambda: ops.moe_down_rows(rows, act, wd, offsets, 0, E))
 gb_a = E * 2 * IE * H * 2 / 1e9
 gb_b = E * H * IE * 2 / 1e9
 print(f"gate_silu: {us_a:.1f} us  weightBW={gb_a/us_a*1e6:.2f} TB/s (floor ~{gb_a/6.0*1e3:.0f} us)")
-print(f"down_scat: {us_b:.1f} us  weightBW={gb_b/us_b*1e6:.2f} TB/s (floor ~{gb_b/6.0*1e3:.0f} us)")
+print(f"down_rows: {us_b:.1f} us  weightBW={gb_b/us_b*1e6:.2f} TB/s (floor ~{gb_b/6.0*1e3:.0f} us)")
 # reference: hipBLASLt per-expert GEMMs on the same shapes
 xs = x[sorted_tok.long()]
 def blaslt():
