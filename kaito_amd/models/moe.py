@@ -150,10 +150,14 @@ class MoEMLP(nn.Module):
                                   scale, mode)
 
     # Pairs up to which the weight-streaming kernels run, beyond it the tiled
-    # grouped GEMMs: 16 rows per expert. Streamed and tiled, in us: 8 experts
-    # of 2048 x 2048 at 16 rows 59 and 79, at 32 99 and 82; 8 of 4096 x 14336
-    # 600 and 692, 1034 and 701; 64 of 2048 x 1408 at 12 rows 251 and 263, at
-    # 24 308 and 266. KAITO_MOE_FUSED_MAX overrides.
+    # grouped GEMMs: 16 rows per expert, 12 with many experts. A layer streamed
+    # and tiled, in us, at 8, 16 and 32 rows per expert: 8 experts of 2048 x
+    # 2048 58 and 73, 70 and 72, 101 and 74; 8 of 4096 x 14336 469 and 650, 615
+    # and 641, 1102 and 660; 32 of 2880 x 2880 293 and 373, 375 and 373, 627
+    # and 384; 128 of 2048 x 768 280 and 293, 352 and 309, 538 and 318; 64 of
+    # 2048 x 1408 at 12 rows 270 and 272, at 16 288 and 271. (Beyond 4096 pairs
+    # tiled rows are bf16, hence 16 for more than 256 experts.)
+    # KAITO_MOE_FUSED_MAX overrides.
     import os as _os
     _most = _os.environ.get("KAITO_MOE_FUSED_MAX")
     FUSED_MAX_TOKENS = None if _most is None else int(_most)
@@ -168,9 +172,9 @@ class MoEMLP(nn.Module):
                 and self.ie_local % 64 == 0):
             return "loop"
         most = self.FUSED_MAX_TOKENS
-        if TK <= (16 * E if most is None else most):
-            return "streamed"
-        return "tiled"
+        if most is None:
+            most = E * (12 if 32 < E <= 256 else 16)
+        return "streamed" if TK <= most else "tiled"
 
     def forward(self, x: torch.Tensor, keep_f32: bool = False,
                 split_shared: bool = False):

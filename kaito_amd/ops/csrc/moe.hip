@@ -16,7 +16,9 @@
 // MT is walked in passes, whose weights come back from the caches. Measured
 // on one MI355X (32 tokens, 8 experts of 2048 x 2048, top 2) against 64 x 128
 // tiles with both operands staged behind barriers, on 128 workgroups:
-// 89 us for both products, now 47 (201 MB of weights: 4.3 TB/s).
+// 89 us for both products, now 47 (201 MB of weights: 4.3 TB/s). 32 experts
+// of 2880 x 2880 (K in stages of 64), top 4, whole layer: 8 tokens 491 -> 178,
+// 64 tokens 440 -> 297.
 //
 // Expert parallelism: callers pass `e_base` and the LOCAL weights; TP shards
 // the expert intermediate dim. Both use these kernels unchanged.
