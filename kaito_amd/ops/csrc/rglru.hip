@@ -30,8 +30,8 @@ KAITO_DEV float recip_f(float d) {
   const float r = __builtin_amdgcn_rcpf(d);
   return fmaf(fmaf(-d, r, 1.0f), r, r);
 }
-KAITO_DEV float logistic_f(float x) {   // below -80 as at -80: 2e-35
-  return recip_f(1.0f + expf(x < -80.0f ? 80.0f : -x));
+KAITO_DEV float logistic_f(float x) {   // 0 below -80: 2e-35
+  return x < -80.0f ? 0.0f : recip_f(1.0f + expf(-x));
 }
 // z / 2 (1 + tanh u) = z logistic(2 u)
 KAITO_DEV float gelu_f(float z) {

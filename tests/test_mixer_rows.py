@@ -95,6 +95,19 @@ def test_rglru_segments(lens, pad, dt):
         at += n
 
 
+@pytest.mark.parametrize("z", [-20.0, -1e4, -1e20, -1e36])
+def test_rglru_closed_output_gate(z):
+    """gelu of a large negative value is 0, however large."""
+    T, W = 256, 64
+    u, y = torch.randn(T, W, device=DEV), torch.full((T, W), z, device=DEV)
+    gates = torch.randn(1, T, 2 * W, device=DEV)
+    state = torch.zeros(2, W, device=DEV)
+    cu, sl, st, ts = _layout([T], [0], [1], 0)
+    out = ops.rglru_scan(u, gates, y, torch.rand(W, device=DEV), state, cu,
+                         sl, st, ts)
+    assert out.abs().max().item() < 1e-30
+
+
 @pytest.mark.parametrize("lens", [[1, 2, 3, 4, 5, 9], [31], [8, 64]])
 @pytest.mark.parametrize("D,V,a0", [(128, 128, -2.0), (64, 20, 3.0),
                                     (256, 8, -6.0), (12, 12, 0.0)])
