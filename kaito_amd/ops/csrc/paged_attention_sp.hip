@@ -25,9 +25,10 @@
 // MI355X against a kernel with 4 waves per pair, 16-byte K and V streams in
 // two phases and dot products by dot2 + DPP sums (before -> now; 8 kv heads
 // of 128, groups of 4):
-//   1 row, 217 keys: 11.0 -> 6.2 us;  16 rows of 4000: 176 -> 51 (two terms
-//   of P: 45);  of 4000 fp8 keys: 179 -> 38 (35);  64 rows of 800: 48 -> 35;
-//   250 of 300: 72 -> 56;  2048 of 220: 428 -> 333 us (5.5 TB/s).
+//   1 row, 217 keys: 11.0 -> 6.4 us;  16 rows of 4000: 176 -> 46, of 4000 fp8
+//   keys 179 -> 34;  64 rows of 800: 48 -> 35;  250 of 300: 72 -> 56;  2048 of
+//   220: 428 -> 332 us (5.5 TB/s).
+// Two terms of P would take 0.1 to 2 % off the long ones.
 //
 // Cache layout: [num_blocks, KV_HEADS, BLOCK_SIZE, HEAD_DIM] bf16 | e4m3.
 #include "flash_prefill.h"
@@ -103,6 +104,11 @@ void paged_decode_kernel(const DecodeArgs a) {
   constexpr int LV = KT * CV / 64;  // V chunks per lane and tile
   __shared__ __attribute__((aligned(128))) short lds_v[NW][KT * D];
   __shared__ float s_m[NW][16], s_l[NW][16];
+  // 16 waves leave a wave 128 registers: the queries wait in LDS, 16-byte
+  // chunk c of row r at c ^ (r & 7) (16 rows of 4000 keys 53 -> 47 us; fp8 pages
+  // spill either way, 34.4 without and 37.8 with it)
+  constexpr bool QLDS = NW > 8 && !FP8;
+  __shared__ __attribute__((aligned(128))) short lds_q[QLDS ? 16 * D : 8];
 
   const int seq = blockIdx.x / a.KH, kvh = blockIdx.x % a.KH;
   const int lane = threadIdx.x & 63;
@@ -124,10 +130,21 @@ void paged_decode_kernel(const DecodeArgs a) {
   hbf16x8 qf[KK];
   {
     const short* qp = a.q + (int64_t)seq * a.q_stride +
-        (int64_t)(kvh * a.G + min(lo, a.G - 1)) * D + hi * 8;
+        (int64_t)(kvh * a.G) * D;
+    if constexpr (QLDS) {
+      static_assert(16 * CV <= NW * 64);
+      const int row = threadIdx.x / CV, ch = threadIdx.x % CV;
+      if (row < 16)
+        *reinterpret_cast<hbf16x8*>(lds_q + row * D + (ch ^ (row & 7)) * 8) =
+            *reinterpret_cast<const hbf16x8*>(qp + min(row, a.G - 1) * D +
+                                              ch * 8);
+      __syncthreads();
+    } else {
 #pragma unroll
-    for (int kk = 0; kk < KK; kk++)
-      qf[kk] = *reinterpret_cast<const hbf16x8*>(qp + kk * 32);
+      for (int kk = 0; kk < KK; kk++)
+        qf[kk] = *reinterpret_cast<const hbf16x8*>(
+            qp + min(lo, a.G - 1) * D + hi * 8 + kk * 32);
+    }
   }
   float m = -1e30f, l = 0.f;
   f32x4 o[DT];
@@ -175,6 +192,12 @@ void paged_decode_kernel(const DecodeArgs a) {
     load_k(row0, row1);
   }
   for (int t = t0; t < t1; t++) {
+    if constexpr (QLDS) {
+#pragma unroll
+      for (int kk = 0; kk < KK; kk++)
+        qf[kk] = *reinterpret_cast<const hbf16x8*>(
+            lds_q + lo * D + ((kk * 4 + hi) ^ (lo & 7)) * 8);
+    }
     // ---- V of this tile: slot j * 64 + lane is row s / CV, place s % CV
     u8x8_t v8[FP8 ? LV : 1];
 #pragma unroll
@@ -266,16 +289,23 @@ void paged_decode_kernel(const DecodeArgs a) {
     __builtin_amdgcn_wave_barrier();
     // ---- O^T: dims 16 dt + 4 hi + r of head lo
 #pragma unroll
-    for (int dt = 0; dt < DT; dt++) {
-      const short* at = vl + vrow * D +
-          flash::swz_v<D>(vrow, dt * 2 + vc) * 8 + ve;
-      const short4_t a4 = flash::read_tr(at), b4 = flash::read_tr(at + 16 * D);
-      const hbf16x8 vf = __builtin_bit_cast(
-          hbf16x8, __builtin_shufflevector(a4, b4, 0, 1, 2, 3, 4, 5, 6, 7));
+    for (int dt = 0; dt < DT; dt += 2) {    // two at a time: 47 -> 46 us there
+      hbf16x8 vf[2];
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const short* at = vl + vrow * D +
+            flash::swz_v<D>(vrow, (dt + u) * 2 + vc) * 8 + ve;
+        const short4_t a4 = flash::read_tr(at);
+        const short4_t b4 = flash::read_tr(at + 16 * D);
+        vf[u] = __builtin_bit_cast(
+            hbf16x8, __builtin_shufflevector(a4, b4, 0, 1, 2, 3, 4, 5, 6, 7));
+      }
 #pragma unroll
       for (int n = 2; n >= 0; n--)
-        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p[n], o[dt], 0, 0,
-                                                        0);
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+          o[dt + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              vf[u], p[n], o[dt + u], 0, 0, 0);
     }
     __builtin_amdgcn_wave_barrier();
   }
