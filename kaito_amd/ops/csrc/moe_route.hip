@@ -18,10 +18,11 @@
 //     weights are also summed per token.
 //   moe_sort: stable counting sort of the (token, expert) pairs by expert:
 //     token and weight of every sorted row, exclusive offsets, row of every
-//     pair. Ranks come from ballots over the distinct experts of 64 pairs,
-//     so the order does not depend on timing. One workgroup up to 2048
-//     pairs; beyond, one per 1024 pairs behind a counting launch (16384 pairs
-//     took 46 us in one workgroup).
+//     pair. Ranks among 64 pairs come from a ballot per bit of the expert's
+//     number, so the order does not depend on timing and the time not on how
+//     many experts there are. One workgroup up to 2048 pairs; beyond, one per
+//     1024 pairs behind a counting launch (16384 pairs took 46 us in one
+//     workgroup).
 //
 // A decode step's choice is launches and latency, not work: as torch ops
 // (product, cast, top-k, softmax, sort, gathers, scatter, scan) it was about
@@ -250,18 +251,16 @@ __global__ __launch_bounds__(256) void moe_gate_route_kernel(
   route_row<1, MODE>(a, part[0], t, lane);
 }
 
-// Pairs are cut into one contiguous run per wave. cnt[w][e]: first the pairs
-// of expert e in wave w's run, then the next row of such a pair.
-template <typename F>
-KAITO_DEV void each_expert(const int e, const F& f) {
-  unsigned long long todo = __ballot(e >= 0);
-  while (todo) {
-    const int src = __builtin_ctzll(todo);
-    const int ev = __builtin_amdgcn_readlane(e, src);
-    const unsigned long long same = __ballot(e == ev);
-    f(ev, same, src);
-    todo &= ~same;
+// lanes of the wave with this lane's expert e (< 2^bits; any lane with -1 is
+// in no group): a ballot per bit, however many experts there are
+KAITO_DEV unsigned long long same_expert(const int e, const int bits) {
+  unsigned long long m = __ballot(e >= 0);
+  for (int b = 0; b < bits; b++) {
+    const bool one = (e >> b) & 1;
+    const unsigned long long ones = __ballot(one);
+    m &= one ? ones : ~ones;
   }
+  return m;
 }
 
 constexpr int SORT_BLOCK = 1024;     // pairs of a workgroup when several sort
@@ -271,26 +270,27 @@ __global__ __launch_bounds__(1024) void moe_count_kernel(
     int* __restrict__ hist, const int* __restrict__ topi, const int TK,
     const int N) {
   extern __shared__ int cnt[];              // [N]
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x;
   for (int i = tid; i < N; i += SORT_BLOCK) cnt[i] = 0;
   __syncthreads();
   const int i = blockIdx.x * SORT_BLOCK + tid;
-  each_expert(i < TK ? topi[i] : -1,
-              [&](int e, unsigned long long same, int src) {
-    if (lane == src) atomicAdd(&cnt[e], __builtin_popcountll(same));
-  });
+  if (i < TK) atomicAdd(&cnt[topi[i]], 1);
   __syncthreads();
   for (int e = tid; e < N; e += SORT_BLOCK)
     hist[(int64_t)blockIdx.x * N + e] = cnt[e];
 }
 
-// hist: counts of SORT_BLOCK pairs each, or nullptr for one workgroup
+// Pairs are cut into one contiguous run per wave. cnt[w][e]: first the pairs
+// of expert e in wave w's run, then the next row of such a pair; row w = waves
+// is the experts' starts. hist: counts of SORT_BLOCK pairs each, or nullptr
+// for one workgroup
 __global__ __launch_bounds__(1024) void moe_sort_kernel(
     int* __restrict__ sorted_tok, float* __restrict__ gates,
     int* __restrict__ offsets, int* __restrict__ pos,
     const int* __restrict__ topi, const float* __restrict__ topw,
-    const int* __restrict__ hist, const int TK, const int top, const int N) {
-  extern __shared__ int cnt[];              // [waves][N]
+    const int* __restrict__ hist, const int TK, const int top, const int N,
+    const int bits) {
+  extern __shared__ int cnt[];              // [waves + 1][N]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nw = blockDim.x >> 6;
   const int begin = hist ? blockIdx.x * SORT_BLOCK : 0;
@@ -298,69 +298,61 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(
   const int per = (end - begin + nw * 64 - 1) / (nw * 64) * 64;
   const int first = min(end, begin + wave * per), last = min(end, first + per);
   int* mine = cnt + wave * N;
+  int* start = cnt + nw * N;
   for (int i = tid; i < nw * N; i += blockDim.x) cnt[i] = 0;
   __syncthreads();
-  for (int base = first; base < last; base += 64) {
-    const int i = base + lane;
-    each_expert(i < last ? topi[i] : -1,
-                [&](int e, unsigned long long same, int src) {
-      if (lane == src) mine[e] += __builtin_popcountll(same);
-    });
+  for (int i = first + lane; i < last; i += 64) atomicAdd(&mine[topi[i]], 1);
+  __syncthreads();
+  // a thread per expert: its pairs, and those before each wave's in this block
+  for (int e = tid; e < N; e += blockDim.x) {
+    int here = 0, before = 0, all = 0;
+    if (hist)
+      for (unsigned b = 0; b < gridDim.x; b++) {
+        const int n = hist[(int64_t)b * N + e];
+        if (b < blockIdx.x) before += n;
+        all += n;
+      }
+    for (int w = 0; w < nw; w++) {
+      const int c = cnt[w * N + e];
+      cnt[w * N + e] = before + here;
+      here += c;
+    }
+    start[e] = hist ? all : here;
   }
   __syncthreads();
   if (wave == 0) {                          // exclusive scan over the experts
-    const int chunk = (N + 63) / 64;
-    const int e0 = min(N, lane * chunk), e1 = min(N, e0 + chunk);
-    auto all_of = [&](const int e) {
-      int n = 0;
-      if (hist)
-        for (unsigned b = 0; b < gridDim.x; b++) n += hist[(int64_t)b * N + e];
-      else
-        for (int w = 0; w < nw; w++) n += cnt[w * N + e];
-      return n;
-    };
-    int sum = 0;
-    for (int e = e0; e < e1; e++) sum += all_of(e);
-    int scan = sum;
+    int base = 0;
+    for (int e0 = 0; e0 < N; e0 += 64) {
+      const int e = e0 + lane, n = e < N ? start[e] : 0;
+      int scan = n;
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int add = __shfl_up(scan, off, 64);
-      if (lane >= off) scan += add;
-    }
-    int start = scan - sum;
-    for (int e = e0; e < e1; e++) {
-      if (blockIdx.x == 0) offsets[e] = start;
-      int next = start;
-      if (hist)                             // rows of the blocks before
-        for (unsigned b = 0; b < blockIdx.x; b++)
-          next += hist[(int64_t)b * N + e];
-      start += all_of(e);
-      for (int w = 0; w < nw; w++) {
-        const int c = cnt[w * N + e];
-        cnt[w * N + e] = next;
-        next += c;
+      for (int off = 1; off < 64; off <<= 1) {
+        const int add = __shfl_up(scan, off, 64);
+        if (lane >= off) scan += add;
       }
+      if (e < N) {
+        start[e] = base + scan - n;
+        if (blockIdx.x == 0) offsets[e] = base + scan - n;
+      }
+      base += __shfl(scan, 63, 64);
     }
-    if (blockIdx.x == 0 && lane == 63) offsets[N] = TK;
+    if (blockIdx.x == 0 && lane == 0) offsets[N] = TK;
   }
   __syncthreads();
-  for (int base = first; base < last; base += 64) {
-    const int i = base + lane;
-    int at = 0;
+  for (int i0 = first; i0 < last; i0 += 64) {
+    const int i = i0 + lane;
     const int e = i < last ? topi[i] : -1;
-    each_expert(e, [&](int ev, unsigned long long same, int src) {
-      if (e == ev)
-        at = mine[ev] +
-            __builtin_popcountll(same & ((1ull << lane) - 1));
-      __builtin_amdgcn_wave_barrier();
-      if (lane == src) mine[ev] += __builtin_popcountll(same);
-      __builtin_amdgcn_wave_barrier();
-    });
+    const unsigned long long same = same_expert(e, bits);
+    const int rank = __builtin_popcountll(same & ((1ull << lane) - 1));
     if (e >= 0) {
+      const int at = start[e] + mine[e] + rank;
       sorted_tok[at] = i / top;
       gates[at] = topw[i];
       pos[i] = at;
     }
+    __builtin_amdgcn_wave_barrier();        // all have read mine
+    if (e >= 0 && rank == 0) mine[e] += __builtin_popcountll(same);
+    __builtin_amdgcn_wave_barrier();
   }
 }
 
@@ -469,7 +461,7 @@ void moe_sort(at::Tensor sorted_tok, at::Tensor gates, at::Tensor offsets,
               pos.numel() == TK && N >= 1 && N <= ROUTE_MAX);
   auto stream = at::hip::getCurrentHIPStream();
   // waves by the number of 64-pair rounds; their counters fit 64 KB
-  const int nw = TK <= 256 ? 4 : 16;
+  const int nw = TK <= 256 ? 4 : (N <= 960 ? 16 : 8);
   const int blocks = TK <= 2048 ? 1 : (TK + SORT_BLOCK - 1) / SORT_BLOCK;
   at::Tensor hist;
   if (blocks > 1) {
@@ -478,11 +470,13 @@ void moe_sort(at::Tensor sorted_tok, at::Tensor gates, at::Tensor offsets,
         (size_t)N * 4, stream, hist.data_ptr<int>(), topi.data_ptr<int>(), TK,
         N);
   }
+  int bits = 0;
+  while ((1 << bits) < N) bits++;
   hipLaunchKernelGGL(moe_sort_kernel, dim3(blocks), dim3(nw * 64),
-      (size_t)nw * N * 4, stream, sorted_tok.data_ptr<int>(),
+      (size_t)(nw + 1) * N * 4, stream, sorted_tok.data_ptr<int>(),
       gates.data_ptr<float>(), offsets.data_ptr<int>(), pos.data_ptr<int>(),
       topi.data_ptr<int>(), topw.data_ptr<float>(),
-      blocks > 1 ? hist.data_ptr<int>() : nullptr, TK, top, N);
+      blocks > 1 ? hist.data_ptr<int>() : nullptr, TK, top, N, bits);
 }
 
 }  // namespace kaito

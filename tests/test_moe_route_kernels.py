@@ -179,3 +179,20 @@ def test_layers_without_a_group_limit(device, n_group, topk_group, routing):
     got = m.to(device)._choose(x.to(device))[0].cpu()
     assert torch.equal(got.long().sort(-1)[0], want.sort(-1)[0])
     assert torch.isfinite(m(x.to(device)).float()).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,top,n", [(300, 8, 256), (2048, 1, 961),
+                                     (2049, 1, 961), (700, 3, 960),
+                                     (3000, 1, 1024), (513, 4, 1000),
+                                     (4096, 8, 65), (257, 1, 2)])
+@pytest.mark.parametrize("spread", ["all", "one", "last"])
+def test_sort_of_many_experts(T, top, n, spread):
+    torch.manual_seed(T)
+    topi = {"all": torch.randint(0, n, (T, top)),
+            "one": torch.full((T, top), n // 2),
+            "last": (n - 1 - torch.arange(T * top) // 64 % n).view(T, top)}
+    topi = topi[spread].to(DEV).int()
+    topw = torch.rand(T, top, device=DEV)
+    for a, b in zip(ops.moe_plan(topi, topw, n), R.moe_plan(topi, topw, n)):
+        assert a.dtype == b.dtype and torch.equal(a, b)
