@@ -15,8 +15,8 @@
 //     (8192 rows of 2048 channels, 4 taps: 136 us with one thread per output
 //     and 2-byte loads, 35 now);
 //   - decode steps: a sequence's row, then its tail, in one launch.
-// Channels that 16 bytes do not divide, or more than 4 taps: one thread per
-// (row, channel).
+// Channels that 16 bytes do not divide, more than 4 taps, and prompts too small
+// to hide a workgroup's walk of 16 rows: one thread per (row, channel).
 #include "mix_common.h"
 
 namespace kaito {
@@ -219,13 +219,19 @@ void causal_conv_update(at::Tensor out, at::Tensor x, at::Tensor weight,
     return (uintptr_t)t.data_ptr() % 16 == 0;
   };
   const int vec = 16 / x.element_size();
+  const bool whole = T <= B;        // a row per sequence: one launch
+  // The walk takes 19 us (bf16) or 12 (f32) however short the prompt, a thread
+  // per output 6 us and more with its size (4 taps; 200 x 2048 bf16: 18.9, 6.9;
+  // 500 x 6144: 19.7, 22.6; 2000 x 1024: 18.9, 14.5; 2000 x 2048: 21.1, 31.4; f32,
+  // 500 x 2048: 13.0, 10.3; 1000 x 2048: 14.0, 17.1).
+  const int64_t least = x.element_size() == 2 ? 11ll << 18 : 3ll << 19;
   const bool rows = C % vec == 0 && x.stride(0) % vec == 0 && taps <= 4 &&
-      wide(x) && wide(out) && wide(conv_state);
+      wide(x) && wide(out) && wide(conv_state) &&
+      (whole || (int64_t)T * C >= least);
   if (rows) {
-    // threads for the channels there are; a row per sequence: one launch
+    // threads for the channels there are
     const int lanes = C / vec;
     const int block = lanes >= 256 ? 256 : (lanes + 63) / 64 * 64;
-    const bool whole = T <= B;
     const dim3 grid(whole ? B : (T + CONV_ROWS - 1) / CONV_ROWS,
                     (lanes + block - 1) / block);
 #define CONV_ROWS_LAUNCH(TAPS_, WHOLE_)                                       \

@@ -58,6 +58,16 @@ def test_causal_conv(lens, C, taps, dt):
     assert torch.equal(state.double(), want)
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("taps", [1, 2, 3, 4])
+@pytest.mark.parametrize("C", [6144, 6152])
+@pytest.mark.parametrize("lens", [[2, 301, 1, 200], [16, 17, 15, 456]])
+def test_causal_conv_of_long_prompts(lens, C, taps, dt):
+    """Sizes at which a workgroup walks 16 rows, chunks that begin anywhere
+    in them."""
+    test_causal_conv(lens, C, taps, dt)
+
+
 @pytest.mark.parametrize("lens,pad", [([130], 0), ([64, 64, 1, 70], 0),
                                       ([7, 200, 9], 5), ([513], 0)])
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
