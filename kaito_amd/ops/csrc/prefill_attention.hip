@@ -41,6 +41,14 @@ void prefill_attention(at::Tensor out, at::Tensor q, at::Tensor k, at::Tensor v,
   a.KH = k.size(1);
   TORCH_CHECK(a.QH % a.KH == 0);
   if (ntiles == 0) return;
+  // keys and values go straight to LDS in 16-byte pieces of their rows
+  auto aligned = [](const at::Tensor& t) {
+    return (uintptr_t)t.data_ptr() % 16 == 0 && t.stride(0) % 8 == 0;
+  };
+  if (!aligned(k) || !aligned(v)) {
+    k = k.clone(at::MemoryFormat::Contiguous);
+    v = v.clone(at::MemoryFormat::Contiguous);
+  }
   a.out = (short*)out.data_ptr();
   a.q = (const short*)q.data_ptr();
   a.k = k.data_ptr();

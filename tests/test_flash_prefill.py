@@ -60,6 +60,24 @@ def test_whole_prompts(QH, KH, D, lens, window, sink, scale_sign):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("shift,pad", [(1, 0), (0, 4), (3, 5)])
+def test_rows_off_16_bytes(shift, pad):
+    """Rows and strides that 16 bytes do not divide: those of a copy."""
+    torch.manual_seed(shift)
+    KH, D, T = 2, 64, 150
+    wide = _bf16(T, 2 * KH * D + pad + 8).view(-1)
+
+    def rows(at):
+        return wide.as_strided((T, KH, D), (2 * KH * D + pad + 8, D, 1), at)
+
+    q = _bf16(T, 4, D)
+    k, v = rows(shift), rows(shift + KH * D)
+    out = ops.prefill_attention(q, k, v, _cu([T]), D ** -0.5)
+    ref = ops.prefill_attention(q, k.clone(), v.clone(), _cu([T]), D ** -0.5)
+    assert torch.equal(out, ref)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("QH,KH,D,pairs,window", [
     (4, 1, 128, [(64, 64), (65, 1), (191, 33)], 0),
     (8, 8, 128, [(300, 129), (128, 128)], 0),
