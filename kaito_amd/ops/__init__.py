@@ -14,6 +14,7 @@ from __future__ import annotations
 
 import numpy as np
 import torch
+import torch.autograd.forward_ad as _fwd_ad
 
 from . import torch_ref
 from ._build import GROUPS, SO_PATH, so_path
@@ -141,6 +142,16 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
     return torch_ref.silu_and_mul(x)
 
 
+def _transformed() -> bool:
+    """Whether torch does more with a call than run it: forward-mode
+    derivatives, vmap and the like, tracing, autocast. They know torch's
+    operations and none of ours."""
+    return _fwd_ad._current_level >= 0 \
+        or torch._C._functorch.peek_interpreter_stack() is not None \
+        or torch._C._len_torch_dispatch_stack() > 0 \
+        or torch.is_autocast_enabled("cuda")
+
+
 def _skinny(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
     """Whether x W^T runs on the weight-streaming kernels: a few rows of
     bf16 on the GPU, 16-byte aligned rows, nothing to differentiate.
@@ -163,8 +174,9 @@ def _skinny(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
     rows the library has another kernel for few rows of W and K of 2560 and
     more (1024 x 2560: 8.0, 6.9; 2048 x 2816: 8.8, 9.5; 1024 x 2816 as a pair
     9.0, 9.5)."""
-    if not (x.is_cuda and x.dim() == 2 and 1 <= x.size(0) <= 32
+    if not (x.is_cuda and x.dim() == w.dim() == 2 and 1 <= x.size(0) <= 32
             and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+            and x.device == w.device and not _transformed()
             and w.is_contiguous() and w.size(1) % 8 == 0 and w.numel() > 0
             and x.stride(1) == 1
             and (x.size(0) == 1 or x.stride(0) % 8 == 0)
@@ -194,6 +206,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
     hipBLASLt otherwise."""
     if _skinny(x, w) and (bias is None or (
             bias.dtype == torch.bfloat16 and bias.is_contiguous()
+            and bias.shape == w.shape[:1] and bias.device == w.device
             and not (torch.is_grad_enabled() and bias.requires_grad))):
         out = torch.empty(x.size(0), w.size(0), dtype=x.dtype,
                           device=x.device)

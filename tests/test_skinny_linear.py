@@ -4,6 +4,8 @@ are f32 (their error is far below), results bf16: half a unit of the 8 bits,
 and one unit where the sum cancels down to 1/16 of its typical size."""
 import pytest
 import torch
+import torch.autograd.forward_ad as fwAD
+from torch.fx.experimental.proxy_tensor import make_fx
 
 from kaito_amd import ops
 from kaito_amd.models.quant import quantize_w4
@@ -84,6 +86,42 @@ def test_other_forms_stay_with_the_library():
     w.requires_grad_(True)
     assert not ops._skinny(x[:2], w)
     assert ops.linear(x[:2], w).requires_grad
+
+
+@pytest.mark.gpu
+def test_calls_that_torch_transforms_stay_with_the_library():
+    x = torch.randn(2, 64, device=DEV).to(torch.bfloat16)
+    w = torch.randn(32, 64, device=DEV).to(torch.bfloat16)
+    with fwAD.dual_level():
+        y = ops.linear(fwAD.make_dual(x, 2 * x), w)
+        tangent = fwAD.unpack_dual(y).tangent
+    assert torch.equal(tangent, torch.nn.functional.linear(2 * x, w))
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert ops.linear(x, w).dtype == torch.float16
+    # biases other than one value per row of W
+    one = torch.ones(1, device=DEV, dtype=torch.bfloat16)
+    assert torch.equal(ops.linear(x, w, one),
+                       torch.nn.functional.linear(x, w, one))
+    with pytest.raises(RuntimeError):
+        ops.linear(x, w, one[:0])
+
+
+def test_transformed_calls_are_seen():
+    seen = []
+
+    def look(t):
+        seen.append(ops._transformed())
+        return t * 2
+
+    x = torch.randn(2, 3)
+    look(x)
+    torch.func.vmap(look)(x)
+    torch.func.jvp(look, (x,), (x,))
+    make_fx(look)(x)
+    with fwAD.dual_level():
+        look(fwAD.make_dual(x, x))
+    look(x)
+    assert seen == [False, True, True, True, True, False]
 
 
 @pytest.mark.gpu
