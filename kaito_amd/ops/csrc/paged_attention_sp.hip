@@ -20,15 +20,15 @@
 // D = 128) are all under way at once, while the arithmetic of a tile is
 // about 500 cycles (2 x 16 scores and weights on the vector unit took
 // 3000). Small steps are bound by the chain lengths -> table -> K -> V -> fold:
-// hence up to 16 waves per workgroup, so that each walks few tiles, and
-// workgroups per pair once those no longer fill the chip. Measured on one
-// MI355X against a kernel with 4 waves per pair, 16-byte K and V streams in
-// two phases and dot products by dot2 + DPP sums (before -> now; 8 kv heads
-// of 128, groups of 4):
-//   1 row, 217 keys: 11.0 -> 6.4 us;  16 rows of 4000: 176 -> 46, of 4000 fp8
-//   keys 179 -> 34;  64 rows of 800: 48 -> 35;  250 of 300: 72 -> 56;  2048 of
-//   220: 428 -> 332 us (5.5 TB/s).
-// Two terms of P would take 0.1 to 2 % off the long ones.
+// hence 8 waves per workgroup, so that each walks few tiles, and workgroups per
+// pair while those do not fill the chip; fewer waves where there are pairs
+// enough (launch_decode). Measured on one MI355X against a kernel with 4 waves
+// per pair, 16-byte K and V streams in two phases and dot products by dot2 +
+// DPP sums (before -> now; 8 kv heads of 128, groups of 4):
+//   1 row, 217 keys: 11.0 -> 6.4 us (8.0 where the table is wide enough for
+//   splits);  16 rows of 4000: 194 -> 43, of 4000 fp8 keys 180 -> 28;  64 rows
+//   of 800: 47 -> 34;  250 of 300: 68 -> 55;  2048 of 220: 429 -> 335 us.
+// Two terms of P would take 0.1 to 5 % off.
 //
 // Cache layout: [num_blocks, KV_HEADS, BLOCK_SIZE, HEAD_DIM] bf16 | e4m3.
 #include "flash_prefill.h"
@@ -45,6 +45,7 @@ using flash::LOG2E;
 
 constexpr int BS = 16;              // tokens per page
 constexpr int KT = 32;              // keys per wave step: two pages
+constexpr int WIDE = 8;             // waves per workgroup while pairs are few
 constexpr int64_t SPLIT_FILL = 256;  // workgroups that splits aim at
 constexpr int SPLIT_MIN = 2;        // tiles per wave that a split keeps
 
@@ -96,7 +97,7 @@ KAITO_DEV Spans spans_of(const int seq_len, const int window, const int nsplit,
 }
 
 template <int D, bool FP8, int NW, bool SPLIT>
-__global__ __launch_bounds__(NW * 64, NW <= 4 ? 3 : (NW <= 8 ? 2 : 4))
+__global__ __launch_bounds__(NW * 64, NW <= 4 && D <= 128 ? 3 : 2)
 void paged_decode_kernel(const DecodeArgs a) {
   constexpr int KK = D / 32;        // 16x16x32 steps over the dims
   constexpr int DT = D / 16;        // 16-row tiles of O^T
@@ -104,11 +105,6 @@ void paged_decode_kernel(const DecodeArgs a) {
   constexpr int LV = KT * CV / 64;  // V chunks per lane and tile
   __shared__ __attribute__((aligned(128))) short lds_v[NW][KT * D];
   __shared__ float s_m[NW][16], s_l[NW][16];
-  // 16 waves leave a wave 128 registers: the queries wait in LDS, 16-byte
-  // chunk c of row r at c ^ (r & 7) (16 rows of 4000 keys 53 -> 47 us; fp8 pages
-  // spill either way, 34.4 without and 37.8 with it)
-  constexpr bool QLDS = NW > 8 && !FP8;
-  __shared__ __attribute__((aligned(128))) short lds_q[QLDS ? 16 * D : 8];
 
   const int seq = blockIdx.x / a.KH, kvh = blockIdx.x % a.KH;
   const int lane = threadIdx.x & 63;
@@ -131,20 +127,10 @@ void paged_decode_kernel(const DecodeArgs a) {
   {
     const short* qp = a.q + (int64_t)seq * a.q_stride +
         (int64_t)(kvh * a.G) * D;
-    if constexpr (QLDS) {
-      static_assert(16 * CV <= NW * 64);
-      const int row = threadIdx.x / CV, ch = threadIdx.x % CV;
-      if (row < 16)
-        *reinterpret_cast<hbf16x8*>(lds_q + row * D + (ch ^ (row & 7)) * 8) =
-            *reinterpret_cast<const hbf16x8*>(qp + min(row, a.G - 1) * D +
-                                              ch * 8);
-      __syncthreads();
-    } else {
 #pragma unroll
-      for (int kk = 0; kk < KK; kk++)
-        qf[kk] = *reinterpret_cast<const hbf16x8*>(
-            qp + min(lo, a.G - 1) * D + hi * 8 + kk * 32);
-    }
+    for (int kk = 0; kk < KK; kk++)
+      qf[kk] = *reinterpret_cast<const hbf16x8*>(
+          qp + min(lo, a.G - 1) * D + hi * 8 + kk * 32);
   }
   float m = -1e30f, l = 0.f;
   f32x4 o[DT];
@@ -192,12 +178,6 @@ void paged_decode_kernel(const DecodeArgs a) {
     load_k(row0, row1);
   }
   for (int t = t0; t < t1; t++) {
-    if constexpr (QLDS) {
-#pragma unroll
-      for (int kk = 0; kk < KK; kk++)
-        qf[kk] = *reinterpret_cast<const hbf16x8*>(
-            lds_q + lo * D + ((kk * 4 + hi) ^ (lo & 7)) * 8);
-    }
     // ---- V of this tile: slot j * 64 + lane is row s / CV, place s % CV
     u8x8_t v8[FP8 ? LV : 1];
 #pragma unroll
@@ -289,7 +269,7 @@ void paged_decode_kernel(const DecodeArgs a) {
     __builtin_amdgcn_wave_barrier();
     // ---- O^T: dims 16 dt + 4 hi + r of head lo
 #pragma unroll
-    for (int dt = 0; dt < DT; dt += 2) {    // two at a time: 47 -> 46 us there
+    for (int dt = 0; dt < DT; dt += 2) {    // in pairs: neither waits for itself
       hbf16x8 vf[2];
 #pragma unroll
       for (int u = 0; u < 2; u++) {
@@ -354,12 +334,12 @@ void paged_decode_kernel(const DecodeArgs a) {
 // One workgroup per (sequence, head) folds the splits that had keys, unless
 // the first had them all. A chain of loads, so a short one: lane s of every
 // wave has split s's weight.
-template <int D, int NW>
+template <int D>
 __global__ __launch_bounds__(D)
 void paged_fold_kernel(const DecodeArgs a, const int QH, const int splits) {
   const int64_t row = blockIdx.x, rows = gridDim.x;
   const int used =
-      spans_of(a.seq_lens[row / QH], a.window, splits, NW).used;
+      spans_of(a.seq_lens[row / QH], a.window, splits, WIDE).used;
   if (used == 1) return;
   const int d = threadIdx.x, lane = d & 63;
   const float sink = a.sinks ? a.sinks[row % QH] * LOG2E : -1e30f;
@@ -386,34 +366,44 @@ template <int D, bool FP8>
 void launch_decode(DecodeArgs a, const at::Tensor& out, int T) {
   auto stream = at::hip::getCurrentHIPStream();
   const int64_t pairs = (int64_t)T * a.KH;
-  // longest context that the table can hold: the lengths are on the device.
-  // Few pairs on long tables: splits until 256 workgroups, as long as every
-  // wave keeps two tiles (1 row of 16000 keys: 870 us in one workgroup per
-  // head before, 31 us in 32). Short contexts under such a table cost the
-  // fold's launch, whatever the table's width: 1 row of 217 keys 6.2 us under
-  // a table of its size and 10.1 under any wider one (11.0 in one workgroup of
-  // 4 waves; 27.4 where empty splits still stored and folded zeros). Up to 256 pairs a workgroup has a CU to
-  // itself and takes 16 waves; above 512 pairs there are workgroups enough
-  // and 4 waves fold less (2048 rows of 300 keys run at 5.5 TB/s).
+  // Waves per workgroup and workgroups per pair, by the number of pairs and the
+  // longest context that the table can hold (the lengths are on the device).
+  // Times in us, bf16 / fp8 pages, 4 heads per pair of 128 unless stated.
+  //   Splits up to 128 pairs, two or more workgroups each until 256, as long as
+  // every wave keeps two tiles: 1 row of 16000 keys 24.5 / 21.8, 142 / 140 in one
+  // workgroup per pair, 16 of 4000 43.6 / 28.3 and 44.3 / 40.7; 24 rows, which
+  // would get one and a third, 84 / 49 and 69 / 41. 16 waves in each: 4 of 4000
+  // 20.5 / 21.9, with 8 18.2 / 15.5. Short contexts under a wide table pay
+  // for the fold's launch: 1 row of 40 keys 6.6, 5.0 under a table of 64 (6.0 in
+  // one workgroup of 4 waves before; with one head per pair 6.1, 4.6 and 4.0).
+  //   8 waves while a workgroup has a CU to itself: 32 of 1000 23 / 16, with 16
+  // 24 / 19. Then 4: 64 of 200 12 / 9, with 8 15 / 13; heads of 64 are small
+  // enough for two of 8 (48 of 4000: 71 / 38, with 4 83 / 45).
+  //   2 waves where one round of the chip then takes the pairs that would need
+  // two rounds of 4 (ROUND2 workgroups fit: 128 of 64 keys 7.6 / 7.2, with 4 9.8
+  // / 8.6; of 2000 176 / 94, 186 / 108), and from 4096 pairs on, whose many rounds
+  // cost by the wave (1024 of 40 keys 36 / 32, with 4 51 / 50, with 8 129 / 133; of
+  // 300 233 / 129 and 224 / 142; heads of 256 and 2 per pair, 1024 of 40: 36 / 33,
+  // 49 / 48 and 89 / 93).
   int64_t longest = (int64_t)a.max_blocks * BS;
   if (a.window > 0) longest = std::min<int64_t>(longest, a.window + BS);
-  constexpr int WIDE = D <= 128 ? 16 : 8;   // waves whose V stage fits LDS
 #define PA_LAUNCH(NW_, SPLIT_, GRID_)                                         \
   hipLaunchKernelGGL((paged_decode_kernel<D, FP8, NW_, SPLIT_>), GRID_,       \
                      dim3(NW_ * 64), 0, stream, a)
   const int64_t splits = std::min<int64_t>(
-      {(SPLIT_FILL + pairs - 1) / pairs, longest / (WIDE * KT * SPLIT_MIN), 64});
+      {SPLIT_FILL / pairs, longest / (WIDE * KT * SPLIT_MIN), 64});
+  constexpr int64_t ROUND2 = D <= 64 ? 2048 : D <= 128 ? 1536 : 1024;
   if (splits > 1) {
     at::Tensor part = at::empty({splits, T, a.KH * a.G, D + 2},
                                 out.options().dtype(at::kFloat));
     a.part = part.data_ptr<float>();
     PA_LAUNCH(WIDE, true, dim3(pairs, splits));
-    hipLaunchKernelGGL((paged_fold_kernel<D, WIDE>), dim3(T * a.KH * a.G),
+    hipLaunchKernelGGL((paged_fold_kernel<D>), dim3(T * a.KH * a.G),
                        dim3(D), 0, stream, a, a.KH * a.G, (int)splits);
-  } else if (pairs <= 256 && longest > 8 * KT) {
+  } else if (pairs <= (D <= 64 ? 512 : 256)) {
     PA_LAUNCH(WIDE, false, dim3(pairs));
-  } else if (pairs <= 512 || D > 128) {
-    PA_LAUNCH(8, false, dim3(pairs));
+  } else if ((pairs > ROUND2 / 2 && pairs <= ROUND2) || pairs >= 4096) {
+    PA_LAUNCH(2, false, dim3(pairs));
   } else {
     PA_LAUNCH(4, false, dim3(pairs));
   }

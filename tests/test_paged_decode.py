@@ -1,5 +1,5 @@
 """The MFMA decode attention (ops/csrc/paged_attention_sp.hip) at the edges
-of its 32-key tiles and of the rules that choose 4, 8 or 16 waves per
+of its 32-key tiles and of the rules that choose 2, 4 or 8 waves per
 workgroup and several workgroups per (sequence, kv head). Weights are f32, so
 the outputs are off by their rounding to bf16 (2^-9) and f32 sums; the bound
 is four times that at the values' largest magnitude."""
@@ -62,8 +62,8 @@ def test_edges(G, KH, D, fp8):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("KH,lens,max_blocks", [
-    (8, [40, 200, 7] * 11, 13),           # 264 pairs: 8 waves
-    (8, [64, 70, 90, 3] * 17, 6),         # 544 pairs: 4 waves
+    (8, [40, 200, 7] * 11, 13),           # 264 pairs
+    (8, [64, 70, 90, 3] * 17, 6),         # 544 pairs
     (2, [1900, 33, 0, 2047], 128),        # few pairs, long table: splits
     (1, [5000], 700),
     (8, [17], 4096),                      # splits that are all but one empty
@@ -75,11 +75,28 @@ def test_launch_rules(KH, lens, max_blocks, D, fp8):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("D,pairs,max_blocks", [
+    (128, 128, 64), (128, 129, 64),           # splits or none
+    (64, 512, 8), (64, 513, 8), (128, 256, 8), (128, 257, 8),   # 8 | 4 waves
+    (64, 1024, 8), (64, 1025, 8), (64, 2048, 8), (64, 2049, 8),  # 4 | 2 | 4
+    (128, 768, 8), (128, 769, 8), (128, 1536, 8), (128, 1537, 8),
+    (256, 512, 8), (256, 513, 8), (256, 1024, 8), (256, 1025, 8),
+    (64, 4095, 8), (64, 4096, 8), (256, 4096, 8),                # 4 | 2
+])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_pair_lines(D, pairs, max_blocks, fp8):
+    """Both sides of the lines between numbers of waves."""
+    lens = [(i * 37) % 97 for i in range(pairs)]
+    _run(2, 1, D, lens, max_blocks, sink=fp8, fp8=fp8)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("D", [64, 128, 256])
 @pytest.mark.parametrize("window,sink", [(0, False), (0, True), (700, True)])
 def test_split_edges(D, window, sink):
     """Under a table that asks for splits: sequences whose keys the first
-    workgroup has alone (16 tiles, 8 for wide heads) and one key more."""
+    workgroup has alone (8 tiles) and one key more, and twice to four times
+    as many."""
     _run(4, 2, D, [0, 1, 256, 257, 512, 513, 1024, 1025, 2048, 6000], 4096,
          window, sink)
 
