@@ -91,12 +91,19 @@ __global__ void rglru_scan_kernel(
 //      away), walk again, write the outputs, and park the state at every
 //      chunk's last row;
 //   3. the parked states go to the slots, whose old ones 2 still reads.
+// The fold costs every segment a walk over those before it, unless they have
+// decayed away. Beyond FOLD_FROM segments that is more than one walk over all
+// of them in a launch of its own (2048 channels: 131072 rows without decay 3090
+// us and 1567, with fast decay 1501 and 1569; 65536 rows in walks 1128 and 762,
+// 65600 with the launch 801 and 798).
 // Rows are loaded 8 ahead of the walk. Measured on one MI355X, 4 prompts of
 // 2048 tokens, 2048 channels: 230 us with the fold and the last segments'
 // walk in launches of their own, one row's loads at a time, 126 now.
 constexpr int SEG = 64;
 constexpr int AHEAD = 8;
+constexpr int FOLD_FROM = 1024;
 
+// PHASE 1, 2: see above. 3: 2 with the carry already in seg_e
 template <typename T, int PHASE>
 __global__ __launch_bounds__(256)
 void rglru_segment_kernel(
@@ -116,6 +123,7 @@ void rglru_segment_kernel(
   const float* gp = gates + ((int64_t)blk * T_total) * (2 * bw) + cc;
   const int t0 = s * SEG, t1 = min(T_total, t0 + SEG);
   float S = 0.0f, P = 1.0f;
+  if (PHASE == 3) S = seg_e[(int64_t)s * W + c];
   if (PHASE == 2) {
     for (int e = s - 1; e >= 0 && P != 0.0f; e -= AHEAD) {
       float p[AHEAD], v[AHEAD];
@@ -141,7 +149,7 @@ void rglru_segment_kernel(
       rg[i] = gp[t * (2 * bw)];
       ig[i] = gp[t * (2 * bw) + bw];
       uv[i] = act_ld(u + t * u_s0 + c);
-      if (PHASE == 2) yv[i] = act_ld(y + t * y_s0 + c);
+      if (PHASE > 1) yv[i] = act_ld(y + t * y_s0 + c);
     }
 #pragma unroll
     for (int i = 0; i < AHEAD; i++) {
@@ -173,6 +181,38 @@ void rglru_segment_kernel(
   if (PHASE == 1) {
     seg_p[(int64_t)s * W + c] = P;
     seg_e[(int64_t)s * W + c] = S;
+  }
+}
+
+// seg_e[s]: the state at segment s's end from a zero carry -> its carry
+__global__ __launch_bounds__(64) void rglru_fold_kernel(
+    const float* __restrict__ seg_p, float* __restrict__ seg_e, const int nseg,
+    const int W) {
+  const int c = blockIdx.x * 64 + threadIdx.x;
+  if (c >= W) return;
+  constexpr int N = 32;             // a batch, and the next one under way
+  float p[2][N], v[2][N], S = 0.0f;
+  auto fetch = [&](const int s, const int b) {
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      const int64_t at = (int64_t)min(s + i, nseg - 1) * W + c;
+      p[b][i] = seg_p[at];
+      v[b][i] = seg_e[at];
+    }
+  };
+  auto fold = [&](const int s, const int b) {
+    fetch(s + N, b ^ 1);            // ahead of the stores, which are to other rows
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      if (s + i < nseg) seg_e[(int64_t)(s + i) * W + c] = S;
+      // a product of 0: a chunk starts here
+      S = p[b][i] == 0.0f ? v[b][i] : p[b][i] * S + v[b][i];
+    }
+  };
+  fetch(0, 0);
+  for (int s = 0; s < nseg; s += 2 * N) {
+    fold(s, 0);
+    fold(s + N, 1);
   }
 }
 
@@ -210,7 +250,13 @@ void run_rglru_segments(hipStream_t stream, at::Tensor& out,
       slots.data_ptr<int>(), starts.data_ptr<int>(),                         \
       token_seq.data_ptr<int>(), T_total, W, bw)
   KAITO_RGLRU_SEG(1);
-  KAITO_RGLRU_SEG(2);
+  if (nseg <= FOLD_FROM) {
+    KAITO_RGLRU_SEG(2);
+  } else {
+    hipLaunchKernelGGL(rglru_fold_kernel, dim3((W + 63) / 64), dim3(64), 0,
+        stream, seg_p.data_ptr<float>(), seg_e.data_ptr<float>(), nseg, W);
+    KAITO_RGLRU_SEG(3);
+  }
 #undef KAITO_RGLRU_SEG
   hipLaunchKernelGGL(rglru_store_kernel, dim3(B, cblocks), dim3(threads), 0,
       stream, state.data_ptr<float>(), last.data_ptr<float>(),

@@ -105,6 +105,35 @@ def test_rglru_segments(lens, pad, dt):
         at += n
 
 
+@pytest.mark.parametrize("T", [65536, 65537, 65600, 70000])
+def test_rglru_very_long_steps(T):
+    """Both sides of the line from which the carries have a launch of their
+    own: the same rows in steps on the short side of it. Sums in another
+    order, of states that hardly decay: f32's 2^-24 by the depth of the sums
+    (64 rows, 1100 segments)."""
+    torch.manual_seed(T)
+    W = 64
+    lens = [T // 3, 5, T - T // 3 - 5]
+    u, y = torch.randn(T, W, device=DEV), torch.randn(T, W, device=DEV)
+    gates = torch.randn(1, T, 2 * W, device=DEV)
+    rate = torch.rand(W, device=DEV)
+    rate[::3] = 1e-6
+    state = torch.randn(4, W, device=DEV)
+    one, parts = state.clone(), state.clone()
+    cu, sl, st, ts = _layout(lens, [0, 3, 0], [1, 2, 3], 0)
+    out = ops.rglru_scan(u, gates, y, rate, one, cu, sl, st, ts)
+    at = 0
+    for n, s, slot in zip(lens, [0, 3, 0], [1, 2, 3]):
+        cut = slice(at, at + n)
+        cu, sl, st, ts = _layout([n], [s], [slot], 0)
+        ref = ops.rglru_scan(u[cut], gates[:, cut].contiguous(), y[cut], rate,
+                             parts, cu, sl, st, ts)
+        err = (out[cut] - ref).abs()
+        assert (err <= 2.0 ** -14 * (ref.abs() + y[cut].abs())).all()
+        at += n
+    assert ((one - parts).abs() <= 2.0 ** -14 * (1 + parts.abs())).all()
+
+
 @pytest.mark.parametrize("z", [-20.0, -1e4, -1e20, -1e36])
 def test_rglru_closed_output_gate(z):
     """gelu of a large negative value is 0, however large."""
