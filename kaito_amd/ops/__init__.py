@@ -370,7 +370,8 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         tile_seq, tile_qbase = tiles or _build_tiles(cu_seqlens)
         _K.prefill_attention(out, q, k, v, tile_seq, tile_qbase,
                                           cu_seqlens, scale, window,
-                                          _sinks_arg(sinks, q.device))
+                                          _sinks_arg(sinks, q.device),
+                                          max_seqlen or 0)
         return out
     return torch_ref.prefill_attention(q, k, v, cu_seqlens, scale, window,
                                        sinks)

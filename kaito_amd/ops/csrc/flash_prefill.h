@@ -7,6 +7,7 @@
 // that a group of 4 heads takes 32 positions per workgroup: every K/V tile
 // is staged once for the whole group and little of the causal diagonal is
 // computed for nothing. Groups that are no power of two run head by head.
+// Prompts of up to 32 rows take one wave per head and half as many keys.
 //
 // Products are transposed, S^T = K Q^T and O^T = V^T P^T on
 // v_mfma_f32_32x32x16_bf16:
@@ -47,7 +48,6 @@ typedef __bf16 hbf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 hbf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int ROWS = 128;           // flattened query rows per workgroup
 constexpr int TILE = 64;            // granularity of the caller's tile list
 constexpr float LOG2E = 1.4426950408889634f;
 
@@ -127,21 +127,22 @@ KAITO_DEV short4_t read_tr(const short* p) {
 template <int D, int DV>
 constexpr int kvt() { return D + DV <= 320 ? 64 : 32; }
 
-// D1: dims of q and k that come from q/k; the others come from q2/k2.
+// D1: dims of q and k that come from q/k; the others come from q2/k2. KVT: keys
+// per tile; NW: waves of 32 rows.
 // EXT: capping, penalty, kept first keys, chunked mask, head gate, and
 // softmax weights that enter P.V as a bf16 value + remainder pair.
 template <int D, int DV, int SRC, bool EXT, bool SIG = false, bool DB = false,
-          int D1 = D>
-__global__ __launch_bounds__(256, (D + DV > 384 ? 1 : 2))
+          int D1 = D, int KVT = kvt<D, DV>(), int NW = 4>
+__global__ __launch_bounds__(NW * 64, (D + DV > 384 ? 1 : 2))
 void flash_prefill_kernel(const Args a) {
-  constexpr int KVT = kvt<D, DV>();
   constexpr int NK = KVT / 32, KK = D / 16, NS = KVT / 16, DT = DV / 32;
   constexpr int CK = D / 8, CV = DV / 8;          // 16-byte chunks of a row
-  constexpr int LK = KVT * CK / 256, LV = KVT * CV / 256;
+  constexpr int NT = NW * 64, ROWS = NW * 32;     // threads, query rows
+  constexpr int LK = KVT * CK / NT, LV = KVT * CV / NT;
   // with nothing but a positive factor between product and exponent, it
   // rides in the exponent's multiply-add
   const bool fold = !EXT && !SIG && !DB && a.scale > 0.f;
-  static_assert(KVT * CK % 256 == 0 && KVT * CV % 256 == 0 && DV % 32 == 0);
+  static_assert(KVT * CK % NT == 0 && KVT * CV % NT == 0 && DV % 32 == 0);
 
   const int HG = a.QH >> a.gs;                    // head groups
   const int hg = blockIdx.x % HG;
@@ -221,17 +222,17 @@ void flash_prefill_kernel(const Args a) {
   };
 
   // ---- staging. Slot s of a tile (16 bytes of LDS) is row s / C, place
-  // s % C; thread tid fills slots j * 256 + tid.
+  // s % C; thread tid fills slots j * NT + tid.
   int pk[SRC == ROWS_BF16 ? 1 : LK], pv[SRC == ROWS_BF16 ? 1 : LV];
   auto fetch_pages = [&](const int kv0) {       // pages of the tile at kv0
     if constexpr (SRC != ROWS_BF16) {
 #pragma unroll
       for (int j = 0; j < LK; j++)
-        pk[j] = bt[min(kv0 + (j * 256 + tid) / CK, kv_len - 1) / a.BS];
+        pk[j] = bt[min(kv0 + (j * NT + tid) / CK, kv_len - 1) / a.BS];
       if constexpr (CV != CK) {
 #pragma unroll
         for (int j = 0; j < LV; j++)
-          pv[j] = bt[min(kv0 + (j * 256 + tid) / CV, kv_len - 1) / a.BS];
+          pv[j] = bt[min(kv0 + (j * NT + tid) / CV, kv_len - 1) / a.BS];
       }
     }
   };
@@ -239,7 +240,7 @@ void flash_prefill_kernel(const Args a) {
   auto stage = [&](const int kv0, short* buf) {
 #pragma unroll
     for (int j = 0; j < LK; j++) {
-      const int s = j * 256 + tid, row = s / CK;
+      const int s = j * NT + tid, row = s / CK;
       const int col = swz_k<D>(row, s % CK) * 8;
       const int key = min(kv0 + row, kv_len - 1);
       if constexpr (SRC == ROWS_BF16) {
@@ -247,7 +248,7 @@ void flash_prefill_kernel(const Args a) {
         const short* p = col < D1
             ? (const short*)a.k + tok * a.k_ts + kvh * a.k_hs + col
             : a.k2 + tok * a.k2_ts + col - D1;
-        lds_copy16(p, buf + (j * 256 + wave * 64) * 8);
+        lds_copy16(p, buf + (j * NT + wave * 64) * 8);
       } else {
         const int64_t at =
             (((int64_t)pk[j] * a.KH + kvh) * a.BS + key % a.BS) * D + col;
@@ -255,19 +256,19 @@ void flash_prefill_kernel(const Args a) {
           rk[j] = *reinterpret_cast<const u8x8_t*>((const uint8_t*)a.k + at);
         else
           lds_copy16((const short*)a.k + at,
-                     buf + (j * 256 + wave * 64) * 8);
+                     buf + (j * NT + wave * 64) * 8);
       }
     }
     short* vbuf = buf + KVT * D;
 #pragma unroll
     for (int j = 0; j < LV; j++) {
-      const int s = j * 256 + tid, row = s / CV;
+      const int s = j * NT + tid, row = s / CV;
       const int col = swz_v<DV>(row, s % CV) * 8;
       const int key = min(kv0 + row, kv_len - 1);
       if constexpr (SRC == ROWS_BF16) {
         lds_copy16((const short*)a.v + (int64_t)(tok0 + key) * a.v_ts +
                        kvh * a.v_hs + col,
-                   vbuf + (j * 256 + wave * 64) * 8);
+                   vbuf + (j * NT + wave * 64) * 8);
       } else {
         const int64_t page = CV == CK ? pk[j] : pv[j];
         const int64_t at =
@@ -276,7 +277,7 @@ void flash_prefill_kernel(const Args a) {
           rv[j] = *reinterpret_cast<const u8x8_t*>((const uint8_t*)a.v + at);
         else
           lds_copy16((const short*)a.v + at,
-                     vbuf + (j * 256 + wave * 64) * 8);
+                     vbuf + (j * NT + wave * 64) * 8);
       }
     }
   };
@@ -292,10 +293,10 @@ void flash_prefill_kernel(const Args a) {
         *reinterpret_cast<hbf16x8*>(dst) = w;
       };
 #pragma unroll
-      for (int j = 0; j < LK; j++) put(rk[j], buf + (j * 256 + tid) * 8);
+      for (int j = 0; j < LK; j++) put(rk[j], buf + (j * NT + tid) * 8);
 #pragma unroll
       for (int j = 0; j < LV; j++)
-        put(rv[j], buf + KVT * D + (j * 256 + tid) * 8);
+        put(rv[j], buf + KVT * D + (j * NT + tid) * 8);
     }
   };
   // the tile's bias by (position of the row) - key + KVT - 1
@@ -494,9 +495,9 @@ inline int group_shift(int QH, int KH) {
   return 0;
 }
 
-// workgroups of a launch over `tiles` 64-row tiles
-inline int64_t grid_size(const Args& a, int64_t tiles) {
-  const int QP = ROWS >> a.gs;
+// workgroups of `waves` waves over `tiles` 64-row tiles
+inline int64_t grid_size(const Args& a, int64_t tiles, int waves = 4) {
+  const int QP = waves * 32 >> a.gs;
   return tiles * (QP < TILE ? TILE / QP : 1) * (a.QH >> a.gs);
 }
 

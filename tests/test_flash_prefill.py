@@ -60,6 +60,29 @@ def test_whole_prompts(QH, KH, D, lens, window, sink, scale_sign):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("QH,KH,D", [(4, 1, 128), (3, 1, 128), (4, 2, 96),
+                                     (4, 4, 96), (8, 1, 64), (4, 4, 64),
+                                     (4, 2, 256)])
+@pytest.mark.parametrize("lens", [[1], [31, 1, 32, 7], [32] * 40, [33, 5],
+                                  [64, 40, 63] * 60, [65, 3]])
+@pytest.mark.parametrize("window,sink,scale", [(0, False, 1.0), (0, True, 0.1),
+                                               (9, False, -0.2)])
+def test_short_prompts(QH, KH, D, lens, window, sink, scale):
+    """Up to 32 rows, one wave per head, up to 64, two, and one row more; with
+    the longest prompt given and without."""
+    torch.manual_seed(D + len(lens))
+    T, cu = sum(lens), _cu(lens)
+    q, k, v = _bf16(T, QH, D), _bf16(T, KH, D), _bf16(T, KH, D)
+    sinks = torch.randn(QH, device=DEV) if sink else None
+    ref = R.prefill_attention(q.cpu().float(), k.cpu().float(),
+                              v.cpu().float(), cu.cpu(), scale, window,
+                              sinks.cpu() if sink else None)
+    for longest in (max(lens), None):
+        _check(ops.prefill_attention(q, k, v, cu, scale, longest, window,
+                                     sinks), ref)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("shift,pad", [(1, 0), (0, 4), (3, 5)])
 def test_rows_off_16_bytes(shift, pad):
     """Rows and strides that 16 bytes do not divide: those of a copy."""
