@@ -262,9 +262,9 @@ def rope_and_cache(positions: torch.Tensor, q: torch.Tensor, k: torch.Tensor,
     return q, k
 
 
-# decode-attention implementation: "sp" = split-phase (r02, K-stream →
-# exp pass → V-stream, no softmax chain in the memory loops), "fused" =
-# the r01 single-pass online-softmax kernel. Overridable for A/B runs.
+# decode-attention implementation: "sp" = the matrix-core kernel
+# (paged_attention_sp.hip), "fused" = the earlier single-pass one with 4
+# waves per pair (paged_attention.hip). Overridable for A/B runs.
 import os as _os
 _PA_IMPL = _os.environ.get("KAITO_PA_IMPL", "sp")
 # fused W4A16 GEMM for M>4: measured slower than dequant+hipBLASLt on
@@ -286,7 +286,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         out = torch.empty_like(q)
         if _PA_IMPL == "sp" or window > 0 or sinks is not None \
                 or k_cache.dtype == torch.uint8:
-            # window/sink support lives in the split-phase kernel only
+            # windows, sinks and fp8 pages: the matrix-core kernel only
             _K.paged_attention_sp(
                 out, q, k_cache, v_cache, block_tables, seq_lens, scale,
                 window, _sinks_arg(sinks, q.device))
