@@ -382,9 +382,11 @@ void launch_decode(DecodeArgs a, const at::Tensor& out, int T) {
   //   2 waves where one round of the chip then takes the pairs that would need
   // two rounds of 4 (ROUND2 workgroups fit: 128 of 64 keys 7.6 / 7.2, with 4 9.8
   // / 8.6; of 2000 176 / 94, 186 / 108), and from 4096 pairs on, whose many rounds
-  // cost by the wave (1024 of 40 keys 36 / 32, with 4 51 / 50, with 8 129 / 133; of
-  // 300 233 / 129 and 224 / 142; heads of 256 and 2 per pair, 1024 of 40: 36 / 33,
-  // 49 / 48 and 89 / 93).
+  // cost by the wave (1024 of 64 keys 44 / 31, with 4 55 / 47; heads of 256 44 / 33,
+  // 51 / 45, with 8 twice that), except bf16 pages of grouped heads, where the
+  // contexts to be expected there want 4 (1024 of 300 keys 232 / 130, 223 / 143;
+  // 2048 of 400 594 / 318, 573 / 344) unless windows keep them to a few tiles (2048
+  // of 220 in a window of 128, heads of 64: 124, 141).
   int64_t longest = (int64_t)a.max_blocks * BS;
   if (a.window > 0) longest = std::min<int64_t>(longest, a.window + BS);
 #define PA_LAUNCH(NW_, SPLIT_, GRID_)                                         \
@@ -402,7 +404,9 @@ void launch_decode(DecodeArgs a, const at::Tensor& out, int T) {
                        dim3(D), 0, stream, a, a.KH * a.G, (int)splits);
   } else if (pairs <= (D <= 64 ? 512 : 256)) {
     PA_LAUNCH(WIDE, false, dim3(pairs));
-  } else if ((pairs > ROUND2 / 2 && pairs <= ROUND2) || pairs >= 4096) {
+  } else if ((pairs > ROUND2 / 2 && pairs <= ROUND2) ||
+             (pairs >= 4096 &&
+              (FP8 || D > 128 || a.G == 1 || longest <= 5 * KT))) {
     PA_LAUNCH(2, false, dim3(pairs));
   } else {
     PA_LAUNCH(4, false, dim3(pairs));

@@ -81,7 +81,7 @@ def test_launch_rules(KH, lens, max_blocks, D, fp8):
     (64, 1024, 8), (64, 1025, 8), (64, 2048, 8), (64, 2049, 8),  # 4 | 2 | 4
     (128, 768, 8), (128, 769, 8), (128, 1536, 8), (128, 1537, 8),
     (256, 512, 8), (256, 513, 8), (256, 1024, 8), (256, 1025, 8),
-    (64, 4095, 8), (64, 4096, 8), (256, 4096, 8),                # 4 | 2
+    (64, 4095, 8), (64, 4096, 8), (256, 4096, 8), (128, 4096, 16),  # 4 | 2 | 4
 ])
 @pytest.mark.parametrize("fp8", [False, True])
 def test_pair_lines(D, pairs, max_blocks, fp8):
