@@ -13,6 +13,7 @@
 //
 // Three launches:
 //   1. prep (token-parallel): unit-norm q/k, decay and beta → f32 scratch
+// Long chunks take delta_chunks.h for 1 and 2. Otherwise:
 //   2. recurrence: thread (j, part) owns rows [part*DP, part*DP+DP) of
 //      column j of S in registers; tokens are staged through LDS eight at
 //      a time, so the token loop itself has no barrier and the only
@@ -22,7 +23,7 @@
 //   3. epilogue (token-parallel): RMS norm, weight, silu gate, store
 // A chunk that starts at position 0 starts from S = 0 whatever its slot
 // held; slots < 0 are padding and skipped.
-#include "mix_common.h"
+#include "delta_chunks.h"
 #include <cstdlib>
 
 namespace kaito {
@@ -363,6 +364,31 @@ __global__ void delta_epilogue_kernel(
     act_st(dst + j, orow[j] * inv * norm_w[j] * silu_f(act_ld(gr + j)));
 }
 
+// the same, LANES = V / 4 lanes per head, four values each. 8192 tokens of 16
+// heads of 128: 51.2 us with one wave per head and 2-byte stores, 26.5 now.
+template <typename T, int LANES>
+__global__ __launch_bounds__(256) void delta_epilogue_vec_kernel(
+    T* __restrict__ out, const float* __restrict__ o,
+    const T* __restrict__ gate, const int64_t g_s0, const int64_t g_s1,
+    const float* __restrict__ norm_w, const int64_t rows, const int H,
+    const float eps) {
+  constexpr int V = LANES * 4;
+  const int64_t row = ((int64_t)blockIdx.x * 256 + threadIdx.x) / LANES;
+  const int c = threadIdx.x % LANES * 4;
+  if (row >= rows) return;          // whole groups of LANES
+  const float4_t x = *reinterpret_cast<const float4_t*>(o + row * V + c);
+  const float4_t g =
+      act_ld4(gate + row / H * g_s0 + row % H * g_s1 + c);
+  const float4_t w = *reinterpret_cast<const float4_t*>(norm_w + c);
+  const float ss = group_reduce_sum<LANES>(
+      (x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3]));
+  const float inv = 1.0f / sqrtf(ss / (float)V + eps);
+  float4_t y;
+#pragma unroll
+  for (int e = 0; e < 4; e++) y[e] = x[e] * inv * w[e] * silu_f(g[e]);
+  act_st4(out + row * V + c, y);
+}
+
 template <typename T, int DP, int PARTS>
 void launch_recurrence(int B, int H, int threads, size_t lds_bytes,
                        hipStream_t stream, float* o, const float* qn,
@@ -385,6 +411,77 @@ void launch_recurrence(int B, int H, int threads, size_t lds_bytes,
         state_slots.data_ptr<int>(), seq_starts.data_ptr<int>(), G, D, V);   \
   }
 
+// delta_chunks.h's path, or false where its forms do not fit. Whole op, us,
+// heads of 128 x 128, token loop / one wave / four waves per 16 columns:
+//   4 prompts of 2048 tokens, 16 heads    785 / 536 / 296
+//   1 of 8192                            2390 / 1847 / 657
+//   8 of 1024 (1024 groups of columns)    711 / 352 / 282
+//   16 of 512 (2048)                      537 / 235 / 279
+//   32 of 230                             354 / 240 / 285
+//   32 of 32                               61 / 59 / 67
+//   4 of 24, 1 of 16              23.4, 22.7 / 25.3, 22.6 / 23.6, 22.1
+// hence from 32 tokens per sequence on, four waves up to 1024 groups. 2-norm
+// error against f64, relative, f32 inputs of 300 tokens, loop and chunks:
+// read-out 1.62e-7 and 1.58e-7, state 1.11e-7 and 1.16e-7 (decays around 0.9);
+// 4.87e-7 and 4.45e-7, 1.14e-6 and 1.13e-6 (0.998).
+template <typename T>
+bool run_chunks(hipStream_t stream, const at::Tensor& q, const at::Tensor& k,
+                const at::Tensor& v, const at::Tensor& a, const at::Tensor& b,
+                const at::Tensor& a_log, const at::Tensor& dt_bias,
+                at::Tensor& state, const at::Tensor& cu_seqlens,
+                const at::Tensor& state_slots, const at::Tensor& seq_starts,
+                at::Tensor& qn, at::Tensor& kn, at::Tensor& o, float qk_eps) {
+  namespace dc = delta_chunks;
+  const int64_t T_ = q.size(0);
+  const int G = q.size(1), D = q.size(2), H = v.size(1), V = v.size(2);
+  const int B = state_slots.size(0);
+  auto fours = [](const at::Tensor& t) {        // loads of four elements
+    return t.stride(0) % 4 == 0 && t.stride(1) % 4 == 0 &&
+           (uintptr_t)t.data_ptr() % (4 * t.element_size()) == 0;
+  };
+  // a sequence, its last chunk filled up, within 32-bit byte offsets
+  auto reach = [&](int64_t row) {
+    return row >= 0 && (T_ + dc::C) * row < 1LL << 31;
+  };
+  // KAITO_DELTA_WAVES=1|4 pins the waves, 0 the token loop (A/B runs, tests)
+  const char* pin = getenv("KAITO_DELTA_WAVES");
+  if ((D != 64 && D != 128) || V % 16 || T_ < 32 * (int64_t)B ||
+      !fours(q) || !fours(k) || !reach(G * (int64_t)D * 4) ||
+      !reach(H * (int64_t)V * 4) || !reach(v.stride(0) * v.element_size()) ||
+      (pin && atoi(pin) == 0) ||
+      getenv("KAITO_DELTA_ROWS_PER_LANE"))
+    return false;
+  const int64_t chunks = T_ / dc::C + B;
+  at::Tensor rec = at::empty({chunks, H, dc::REC}, qn.options());
+  const int64_t groups = (int64_t)B * H * (V / 16);
+  const int nw = pin ? atoi(pin) : groups > 1024 ? 1 : 4;
+#define KAITO_DELTA_CHUNKS(NJ_, NW_)                                         \
+  if (nw == NW_)                                                             \
+    hipLaunchKernelGGL((dc::delta_chunk_kernel<T, NJ_, NW_>),                \
+        dim3(B, H, V / 16), dim3(64 * NW_), 0, stream, o.data_ptr<float>(),  \
+        qn.data_ptr<float>(), kn.data_ptr<float>(), rec.data_ptr<float>(),   \
+        (const T*)v.data_ptr(), v.stride(0), v.stride(1),                    \
+        state.data_ptr<float>(), cu_seqlens.data_ptr<int>(),                 \
+        state_slots.data_ptr<int>(), seq_starts.data_ptr<int>(), G, H, V)
+#define KAITO_DELTA_DIM(NJ_)                                                 \
+  if (D == 16 * NJ_) {                                                       \
+    hipLaunchKernelGGL((dc::delta_chunk_prep_kernel<T, NJ_>),                \
+        dim3(chunks, G), dim3(64), 0, stream, qn.data_ptr<float>(),          \
+        kn.data_ptr<float>(), rec.data_ptr<float>(), (const T*)q.data_ptr(), \
+        q.stride(0), q.stride(1), (const T*)k.data_ptr(), k.stride(0),       \
+        k.stride(1), (const T*)a.data_ptr(), a.stride(0),                    \
+        (const T*)b.data_ptr(), b.stride(0), a_log.data_ptr<float>(),        \
+        dt_bias.data_ptr<float>(), cu_seqlens.data_ptr<int>(),               \
+        state_slots.data_ptr<int>(), B, G, H, qk_eps);                       \
+    KAITO_DELTA_CHUNKS(NJ_, 1);                                              \
+    KAITO_DELTA_CHUNKS(NJ_, 4);                                              \
+  }
+  KAITO_DELTA_DIM(4) KAITO_DELTA_DIM(8)
+#undef KAITO_DELTA_DIM
+#undef KAITO_DELTA_CHUNKS
+  return true;
+}
+
 template <typename T>
 void run_delta(hipStream_t stream, at::Tensor& out, const at::Tensor& q,
                const at::Tensor& k, const at::Tensor& v,
@@ -400,6 +497,34 @@ void run_delta(hipStream_t stream, at::Tensor& out, const at::Tensor& q,
   const int T_ = q.size(0), G = q.size(1), D = q.size(2);
   const int H = v.size(1), V = v.size(2);
   const int B = state_slots.size(0);
+  auto epilogue = [&]() {
+    const size_t four = 4 * gate.element_size();
+    const bool fours = gate.stride(0) % 4 == 0 && gate.stride(1) % 4 == 0 &&
+        (uintptr_t)gate.data_ptr() % four == 0 &&
+        (uintptr_t)out.data_ptr() % four == 0 &&
+        (uintptr_t)norm_w.data_ptr() % 16 == 0;
+    const int64_t rows = (int64_t)T_ * H;
+#define KAITO_DELTA_EPILOGUE(LANES_)                                         \
+    if (fours && V == 4 * LANES_) {                                          \
+      hipLaunchKernelGGL((delta_epilogue_vec_kernel<T, LANES_>),             \
+          dim3((rows * LANES_ + 255) / 256), dim3(256), 0, stream,           \
+          (T*)out.data_ptr(), o.data_ptr<float>(),                           \
+          (const T*)gate.data_ptr(), gate.stride(0), gate.stride(1),         \
+          norm_w.data_ptr<float>(), rows, H, norm_eps);                      \
+      return;                                                                \
+    }
+    KAITO_DELTA_EPILOGUE(16) KAITO_DELTA_EPILOGUE(32) KAITO_DELTA_EPILOGUE(64)
+#undef KAITO_DELTA_EPILOGUE
+    hipLaunchKernelGGL((delta_epilogue_kernel<T>), dim3(T_, H), dim3(64), 0,
+        stream, (T*)out.data_ptr(), o.data_ptr<float>(),
+        (const T*)gate.data_ptr(), gate.stride(0), gate.stride(1),
+        norm_w.data_ptr<float>(), H, V, norm_eps);
+  };
+  if (run_chunks<T>(stream, q, k, v, a, b, a_log, dt_bias, state, cu_seqlens,
+                    state_slots, seq_starts, qn, kn, o, qk_eps)) {
+    epilogue();
+    return;
+  }
   hipLaunchKernelGGL((delta_prep_kernel<T>), dim3(T_, G), dim3(64), 0,
       stream, qn.data_ptr<float>(), kn.data_ptr<float>(),
       kq.data_ptr<float>(), decay.data_ptr<float>(), beta.data_ptr<float>(),
@@ -443,10 +568,7 @@ void run_delta(hipStream_t stream, at::Tensor& out, const at::Tensor& q,
     KAITO_DELTA_CASE(32, 8) KAITO_DELTA_CASE(64, 1) KAITO_DELTA_CASE(64, 2)
     KAITO_DELTA_CASE(64, 4) KAITO_DELTA_CASE(64, 8)
   }
-  hipLaunchKernelGGL((delta_epilogue_kernel<T>), dim3(T_, H), dim3(64), 0,
-      stream, (T*)out.data_ptr(), o.data_ptr<float>(),
-      (const T*)gate.data_ptr(), gate.stride(0), gate.stride(1),
-      norm_w.data_ptr<float>(), H, V, norm_eps);
+  epilogue();
 }
 #undef KAITO_DELTA_CASE
 

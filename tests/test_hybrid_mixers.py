@@ -122,6 +122,52 @@ def test_delta_rule_portions(mode, G, H, D, V, rows_per_lane, monkeypatch):
     assert torch.all(state[0] == 3.0)        # the other slot is untouched
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("G,H,D,V", [(1, 3, 64, 16), (2, 10, 128, 48)])
+@pytest.mark.parametrize("waves", ["1", "4"])
+def test_delta_rule_chunks(dt, G, H, D, V, waves, monkeypatch):
+    """The form that takes 16 tokens at a time: whole and partial chunks, a
+    state that is carried in, several sequences, and a value that is not
+    finite, which no token before it may see."""
+    monkeypatch.setenv("KAITO_DELTA_WAVES", waves)
+    dev = "cuda"
+    lens = [114, 33, 97]
+    r = lambda n, *s: torch.randn(n, *s).to(dt)
+    seqs = [(r(n, G, D), r(n, G, D), r(n, H, V), r(n, H, V), r(n, H),
+             r(n, H)) for n in lens]
+    a_log = torch.randn(H) * 0.5 - 2.0
+    dt_bias, norm_w = torch.randn(H), torch.randn(V)
+    dw = [t.to(dev) for t in (a_log, dt_bias, norm_w)]
+    want = [plain_delta(*(t.double() for t in (*s, a_log, dt_bias, norm_w)),
+                        1e-5) for s in seqs]
+    state = torch.full((5, H, D, V), 3.0, device=dev)
+    cu, sl, st, _, _ = layout(dev, lens, [0, 0, 0], [3, 0, 2])
+
+    def run(xs, cu, sl, st):
+        return ops.gated_delta_rule(*(t.to(dev) for t in xs), *dw, state, cu,
+                                    sl, st, 1e-6, 1e-5)
+    both = [torch.cat(t) for t in zip(*seqs)]
+    close(run(both, cu, sl, st), torch.cat(want), dt)
+    whole = state.clone()
+    assert torch.all(state[1] == 3.0) and torch.all(state[4] == 3.0)
+    outs = []
+    for start, n in split_runs(lens[0], [48, 81]):
+        c1, s1, t1, _, _ = layout(dev, [n], [start], [4])
+        outs.append(run([t[start:start + n] for t in seqs[0]], c1, s1, t1))
+    close(torch.cat(outs), want[0], dt)
+    # f32 states of the same tokens in chunks of another cut
+    assert (state[4] - whole[3]).norm() <= 3e-6 * whole[3].norm()
+    clean = run(both, cu, sl, st)
+    both[2][40, 0, 3] = float("nan")
+    bad = run(both, cu, sl, st)
+    cut = slice(lens[0], None)
+    assert torch.equal(bad[:40], clean[:40])
+    assert torch.equal(bad[cut], clean[cut])
+    assert bad[40:lens[0], :V].isnan().all()
+    assert torch.equal(bad[:, V:], clean[:, V:])
+
+
 # ------------------------------------------------------------------ RG-LRU
 
 @pytest.mark.parametrize("mode", MODES)
