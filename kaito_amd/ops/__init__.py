@@ -169,6 +169,9 @@ def _skinny(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
     7168 (2112 x 7168: 12.7, 12.6; 2048 x 8192: 14.6, 13.1); SwiGLU pairs,
     which save a launch, to 8192 (28672 x 4096: 50.3, 60.5), uneven ones
     excepted (5120 x 5120: 19.1, 17.9).
+    Many rows of W whose x fits the registers, K of 2048 up to 32 rows and of
+    4096 up to 16, always (12288 x 2048: 13.6, 16.6 at 16, 15.9, 16.9 at 32;
+    32000 x 2048 29.7, 31.8 at 32; 128256 x 4096 168, 186 at 16).
     Up to 32: to 3072 x 2048 (7.4, 11.5; 6144 x 2048: 13.0, 12.6, as a pair
     12.5, 15.0) and K of 4096 (1024 x 4096: 10.1, 11.3 at 24), where beyond 24
     rows the library has another kernel for few rows of W and K of 2560 and
@@ -189,6 +192,10 @@ def _skinny(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
         return True
     if K % 64 or N % 16:
         return False
+    # x stays in registers while W streams
+    if N >= 12288 and N * K < 1 << 31 and (
+            K == 2048 or (K == 4096 and M <= 16)):
+        return True
     if M <= 16 and N < 1024 and K > 5120 and not glu:
         return False
     uneven = 4096 < N < 7168 and K > 4096

@@ -12,11 +12,13 @@
 //   * moe_down_rows: y[s] = act[s] Wd^T in f32, summed per token by
 //     moe_combine.
 //
-// One workgroup per (16 weight rows, expert); an expert with more rows than 16
-// MT is walked in passes, whose weights come back from the caches. Measured
+// One workgroup per (16 weight rows, expert), or with K = 2048 about one per CU
+// that goes from tile to tile; an expert with more rows than 16 MT is walked in
+// passes, whose weights come back from the caches. Measured
 // on one MI355X (32 tokens, 8 experts of 2048 x 2048, top 2) against 64 x 128
 // tiles with both operands staged behind barriers, on 128 workgroups:
-// 89 us for both products, now 47 (201 MB of weights: 4.3 TB/s). 32 experts
+// 89 us for both products, 47 in tiles of their own, now 38.5 (201 MB of
+// weights: 5.2 TB/s, launches included). 32 experts
 // of 2880 x 2880 (K in stages of 64), top 4, whole layer: 8 tokens 491 -> 178,
 // 64 tokens 440 -> 297.
 //
@@ -26,6 +28,8 @@
 #include <torch/library.h>
 #include <ATen/ATen.h>
 #include <ATen/hip/HIPContext.h>
+#include <algorithm>
+#include <cmath>
 
 namespace kaito {
 
@@ -56,6 +60,26 @@ KAITO_DEV float moe_act_f(int mode, float g, float u, float limit) {
     return (u + 1.f) * glu;
   }
   return skinny::silu(g) * u;
+}
+
+// column n of rows m .. m + 3 below end: v, or gate v and up u
+template <int KIND>
+KAITO_DEV void store_rows(const StreamArgs& a, const f32x4 v, const f32x4 u,
+                          const int m0, const int end, const int n) {
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int m = m0 + r;
+    if (m >= end) break;
+    if constexpr (KIND == UP_GATED) {
+      a.act[(int64_t)m * a.N + n] =
+          f32_to_bf16(moe_act_f(a.act_mode, v[r], u[r], a.limit));
+    } else if constexpr (KIND == UP_PLAIN) {
+      const float p = fmaxf(v[r], 0.f);
+      a.act[(int64_t)m * a.N + n] = f32_to_bf16(p * p);
+    } else {
+      a.y[(int64_t)m * a.N + n] = v[r];
+    }
+  }
 }
 
 template <int MT, int KS, int KIND>
@@ -106,22 +130,77 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const StreamArgs a) 
         v += bf16_to_f32(be[0]);
         if constexpr (GATED) u += bf16_to_f32(be[a.N]);
       }
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int m = m0 + (slot >> 6) * 16 + (l >> 4) * 4 + r;
-        if (m >= end) break;
-        if constexpr (KIND == UP_GATED) {
-          a.act[(int64_t)m * a.N + n0 + c] =
-              f32_to_bf16(moe_act_f(a.act_mode, v[r], u[r], a.limit));
-        } else if constexpr (KIND == UP_PLAIN) {
-          const float p = fmaxf(v[r], 0.f);
-          a.act[(int64_t)m * a.N + n0 + c] = f32_to_bf16(p * p);
-        } else {
-          a.y[(int64_t)m * a.N + n0 + c] = v[r];
-        }
-      }
+      store_rows<KIND>(a, v, u, m0 + (slot >> 6) * 16 + (l >> 4) * 4, end,
+                       n0 + c);
     }
     __syncthreads();                // sums read before the next pass's stages
+  }
+}
+
+// K = 1024 S: see skinny::stream_tiles. gridDim.x workgroups share an expert's
+// ntiles tiles; MT row tiles of 16 in a pass.
+template <int MT, int S, int KIND>
+KAITO_DEV void stream_pass(const StreamArgs& a, const int le, const int ntiles,
+                           const int m0, const int end, short* ring,
+                           f32x4* red, const int wave, const int lane) {
+  constexpr int KS = skinny::TILES_KS, NW = skinny::TILE_NW;
+  constexpr bool GATED = KIND == UP_GATED;
+  constexpr int COLS = GATED ? 8 : 16;
+  const int64_t wrows = GATED ? 2 * a.N : a.N;
+  const int slot = threadIdx.x, l = slot & 63, c = l & 15;
+  const bool mine = slot < MT * 64 && !(GATED && c >= 8);
+  skinny::stream_tiles<MT, S>(
+      a.w + le * wrows * a.K,
+      [&](const int j) {
+        const int r = skinny::tile_row<KS>(j, lane);
+        const uint32_t n = GATED ? r % 8 + (r >= 8 ? a.N : 0) : r;
+        return (n * a.K + skinny::tile_col<KS>(j, lane)) * 2;
+      },
+      COLS * a.K * 2, blockIdx.x, gridDim.x, ntiles,
+      [&](const short* (&xp)[MT]) {
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+          const int m = min(m0 + mt * 16 + (lane & 15), end - 1);
+          const int64_t row = KIND == DOWN ? m : a.rows[m];
+          xp[mt] = a.x + row * a.K + (lane >> 4) * 8;
+        }
+      },
+      ring, red, wave, lane,
+      [&](const int t, const f32x4* sums) {
+        if (!mine) return;
+        const int n = t * COLS + c;
+        f32x4 v = skinny::fold<MT, NW>(sums, slot), u{0.f, 0.f, 0.f, 0.f};
+        if constexpr (GATED) u = skinny::fold<MT, NW>(sums, slot + 8);
+        if (a.bias) {
+          const short* be = a.bias + le * wrows + n;
+          v += bf16_to_f32(be[0]);
+          if constexpr (GATED) u += bf16_to_f32(be[a.N]);
+        }
+        store_rows<KIND>(a, v, u, m0 + (slot >> 6) * 16 + (l >> 4) * 4, end,
+                         n);
+      });
+  __syncthreads();                  // sums read before the next pass's
+}
+
+template <int S, int KIND>
+__global__ __launch_bounds__(256, 2) void moe_tiles_kernel(const StreamArgs a,
+                                                           const int ntiles) {
+  constexpr int KS = skinny::TILES_KS, NW = skinny::TILE_NW;
+  __shared__ __attribute__((aligned(128))) short ring[NW][2][16 * KS];
+  __shared__ f32x4 red[2][NW][2 * 64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int le = blockIdx.y;
+  const int begin = a.offsets[a.e_base + le], end = a.offsets[a.e_base + le + 1];
+  // An expert that many tokens share would hold up its workgroups for a second
+  // pass: as many row tiles as it has.
+  for (int m0 = begin; m0 < end; m0 += 32) {
+    if (end - m0 > 16)
+      stream_pass<2, S, KIND>(a, le, ntiles, m0, end, ring[wave][0],
+                              &red[0][0][0], wave, lane);
+    else
+      stream_pass<1, S, KIND>(a, le, ntiles, m0, end, ring[wave][0],
+                              &red[0][0][0], wave, lane);
   }
 }
 
@@ -133,6 +212,29 @@ void launch_stream(const StreamArgs& a, int64_t E_local, int64_t pairs,
   auto stream = at::hip::getCurrentHIPStream();
   // two row tiles once most experts have more than one
   const bool two = pairs > 12 * E;
+  // With K = 2048 and up to 32 experts, workgroups that stay
+  // (skinny::stream_tiles), from three tiles per CU on of the experts that are
+  // likely hit. us, per tile and staying: 8 experts of 2048 x 2048, up 17.6 and
+  // 16.1, 26.1 and 24.2, 28.4 and 24.4, 35.7 and 25.7 at 4, 16, 32 and 64
+  // tokens of two experts; down 16.1 and 14.0, 16.9 and 14.2, 21.5 and 16.0 at
+  // 16 to 64, 10.7 and 11.4 at 4 (672 tiles); one token 8.4 and 10.7, 7.2 and
+  // 8.4. 32 of 2048 x 768, top 8, up 28.1 and 26.5 at 4, 51.9 and 37.4 at 64;
+  // 64 of 2048 x 1408, top 6, 39.5 and 53.8 at 4, 99 and 105 at 16: an equal
+  // share per expert leaves CUs idle when some of many are not hit, and equal
+  // runs over those that are cost more to find than they give (26.0 and 15.5
+  // for the 32 tokens). Wider K streams as fast in tiles of their own: 8 of
+  // 28672 x 4096, 16 tokens, 275 and 282.
+  const double hit =
+      E_local * (1.0 - std::pow(1.0 - 1.0 / E, (double)pairs));
+  if (a.K == 2048 && E_local <= 32 && hit * grid.x >= 768) {
+    // never more than the CUs: a CU with two of them ends late (264
+    // workgroups for the 32 tokens: 31.2 and 18.4)
+    const int most = (int)std::min<int64_t>(E_local, pairs);
+    const int per = std::max(1, std::min<int>(grid.x, 256 / most));
+    hipLaunchKernelGGL((moe_tiles_kernel<2, KIND>), dim3(per, E_local), block,
+                       0, stream, a, (int)grid.x);
+    return;
+  }
 #define MS_LAUNCH(MT_, KS_)                                                   \
   hipLaunchKernelGGL((moe_stream_kernel<MT_, KS_, KIND>), grid, block, 0,     \
                      stream, a)

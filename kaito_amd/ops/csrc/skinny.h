@@ -13,7 +13,8 @@
 // 16 rows of W; its waves take every fourth slice of K and meet in LDS, in
 // f32. 28672 x 4096: 44.4 us at M = 8 (library 56.8), 50.9 at 16 (57.4), 72.8 at
 // 32 (48.6): x comes through the caches once per workgroup, so the gain ends
-// where its rows cost what those of W do. K in stages of 64, 2880 x 2880: 6.5
+// where its rows cost what those of W do. Where x fits the registers,
+// workgroups stay for many tiles (stream_tiles): 40.1 at 8, 41.8 at 16. K in stages of 64, 2880 x 2880: 6.5
 // at 8 (16.3), 6.8 at 16 (16.4).
 //
 // 4-bit weights run as integers. Read as fp8 (e4m3, subnormals and the first
@@ -139,6 +140,103 @@ KAITO_DEV void stream_tile(f32x4 (&acc)[MT],
   } else {
     last(0);
   }
+}
+
+// ---- the same over many tiles ----------------------------------------------
+// Where K is 4 S stages of 256, a wave's slices of x fit its registers: they
+// are read once, and the workgroup goes from tile to tile with the next stage
+// always under way, also across the sum over its waves. Tiles of their own
+// workgroups (stream_tile) spend as long on offsets, x and the sum as on 64 KB
+// of weights, and no more than two of them fit a CU.
+constexpr int TILES_KS = 256;
+
+// Sums of the 16 rows of W of tiles first, first + step .. < n. rows(j): byte
+// offset of load j's piece from the start of tile 0, which lies at w; tile:
+// bytes from a tile to the next; xp: as for stream_tile, asked for once the
+// first weights are under way. ring: [2][16 * 256] of this wave, red:
+// [2][4][MT * 64] of the workgroup. out(tile, sums): on every thread, the sums
+// of the waves for fold().
+template <int MT, int S, typename Rows, typename X, typename Out>
+KAITO_DEV void stream_tiles(const void* w, const Rows& rows,
+                            const uint32_t tile, const int first,
+                            const int step, const int n, const X& x,
+                            short* ring, f32x4* red, const int wave,
+                            const int lane, const Out& out) {
+  constexpr int KS = TILES_KS, NI = tile_loads<KS>(), STEPS = KS / 32;
+  static_assert(S % 2 == 0, "a tile starts in ring 0");
+  if (first >= n) return;           // uniform
+  const auto wb = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<void*>(w), 0, 0xffffffff, 0x27000);
+  // past the last tile: loads of nothing, so that the waits stay counts
+  const auto none = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<void*>(w), 0, 0, 0x27000);
+  uint32_t off[NI];
+#pragma unroll
+  for (int j = 0; j < NI; j++) off[j] = rows(j);
+  auto fetch = [&](const int t, const int s) {
+    const auto r = t < n ? wb : none;
+    const uint32_t at =
+        __builtin_amdgcn_readfirstlane(t * tile + (wave + s * TILE_NW) * KS * 2);
+#pragma unroll
+    for (int j = 0; j < NI; j++)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          r,
+          (__attribute__((address_space(3))) void*)(ring + (s & 1) * 16 * KS +
+                                                    j * 512),
+          16, off[j], at, 0, 2 /* non-temporal */);
+  };
+  fetch(first, 0);
+  fetch(first, 1);
+  hbf16x8 xf[S][MT][STEPS];
+  {
+    const short* xp[MT];
+    x(xp);
+#pragma unroll
+    for (int s = 0; s < S; s++)
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+        for (int i = 0; i < STEPS; i++)
+          xf[s][mt][i] =
+              load_x(xp[mt] + (wave + s * TILE_NW) * KS + i * 32);
+  }
+  wait_loads<0>();                  // none of x is left for the loop's counts
+  const int lo = lane & 15, hi = lane >> 4;
+  int par = 0;
+  for (int t = first; t < n; t += step) {
+    f32x4 acc[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < S; s++) {
+      wait_loads<NI>();             // this stage's; the next is under way
+      const short* p = ring + (s & 1) * 16 * KS + lo * KS;
+#pragma unroll
+      for (int i = 0; i < STEPS; i++) {
+        const hbf16x8 wf = load_x(p + (((i * 4 + hi) ^ (lo & 7)) * 8));
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+          acc[mt] = mfma16(xf[s][mt][i], wf, acc[mt]);
+      }
+      // its reads are done before it is overwritten
+      __builtin_amdgcn_s_waitcnt(0xc07f);
+      asm volatile("" ::: "memory");
+      if (s + 2 < S) fetch(t, s + 2);
+      else fetch(t + step, s + 2 - S);
+    }
+    f32x4* sums = red + par * TILE_NW * MT * 64;
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+      sums[(wave * MT + mt) * 64 + lane] = acc[mt];
+    // own sums written, the next weights still under way; the other half of
+    // red is free once all are here
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    out(t, sums);
+    par ^= 1;
+  }
+  wait_loads<0>();                  // no copy to LDS outlives the workgroup's
 }
 
 // the eight nibbles of a word as bf16 q / 512, in the order 0 2 4 6 1 3 5 7

@@ -101,6 +101,54 @@ __global__ __launch_bounds__(256, 2) void skinny_tile_kernel(
   }
 }
 
+// K = 1024 S: see skinny::stream_tiles. gridDim.x workgroups share the tiles.
+template <int MT, int S, bool GLU>
+__global__ __launch_bounds__(256, 2) void skinny_tiles_kernel(
+    short* __restrict__ out, const short* __restrict__ x,
+    const int64_t x_stride, const short* __restrict__ w,
+    const short* __restrict__ bias, const int M, const int N, const int K) {
+  constexpr int KS = skinny::TILES_KS, TW = skinny::TILE_NW;
+  constexpr int COLS = GLU ? 8 : 16;
+  __shared__ __attribute__((aligned(128))) short ring[TW][2][16 * KS];
+  __shared__ f32x4 red[2][TW][MT * 64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int slot = threadIdx.x, l = slot & 63, c = l & 15;
+  const bool mine = slot < MT * 64 && !(GLU && c >= 8);
+  skinny::stream_tiles<MT, S>(
+      w,
+      [&](const int j) {
+        const int r = skinny::tile_row<KS>(j, lane);
+        const uint32_t n = GLU ? r % 8 + (r >= 8 ? N : 0) : r;
+        return (n * K + skinny::tile_col<KS>(j, lane)) * 2;
+      },
+      COLS * K * 2, blockIdx.x, gridDim.x, N / COLS,
+      [&](const short* (&xp)[MT]) {
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+          xp[mt] = x + min(mt * 16 + (lane & 15), M - 1) * x_stride +
+              (lane >> 4) * 8;
+      },
+      ring[wave][0], &red[0][0][0], wave, lane,
+      [&](const int t, const f32x4* sums) {
+        if (!mine) return;
+        const int n = t * COLS + c;
+        f32x4 v = skinny::fold<MT, TW>(sums, slot);
+        if constexpr (GLU) {
+          const f32x4 u = skinny::fold<MT, TW>(sums, slot + 8);
+#pragma unroll
+          for (int r = 0; r < 4; r++) v[r] = skinny::silu(v[r]) * u[r];
+        } else if (bias) {
+          v += bf16_to_f32(bias[n]);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int m = (slot >> 6) * 16 + (l >> 4) * 4 + r;
+          if (m < M) out[(int64_t)m * N + n] = f32_to_bf16(v[r]);
+        }
+      });
+}
+
 constexpr int MAX_M = 32;
 
 // Rows of W streamed whole, or tiles of 16 through LDS? Beyond 4 rows of x
@@ -111,6 +159,19 @@ constexpr int MAX_M = 32;
 bool in_tiles(int64_t M, int64_t N, int64_t K, int64_t cols, int64_t weights) {
   return M > 4 || (M > 2 && weights > (1ll << 25) && K % 64 == 0 &&
                    N % cols == 0);
+}
+
+// Tiles handed to workgroups that stay, a CU each, or to one workgroup per tile?
+// From three tiles per CU on (us, per tile and staying; 2048 columns: 448 tiles
+// 8.9 and 9.2, 512 of a pair 8.9 and 9.5, 768 13.1 and 12.6 at M = 5, 15.5 and
+// 13.6 at 16, 19.4 and 15.9 at 32, 2000 44.1 and 29.6 at 32; 4096 columns: 384
+// 13.8 and 14.0, 1792 of a pair 40.2 and 39.3 at 5, 48.5 and 41.8 at 16, 8016
+// 209 and 168 at 16). Two workgroups per CU are no faster (1792 of a pair 42.8).
+constexpr int WORKGROUPS = 256;
+
+bool many_tiles(int M, int64_t tiles, const at::Tensor& w) {
+  return tiles >= 3 * WORKGROUPS && w.numel() < (1ll << 31) &&
+         (w.size(1) == 2048 || (w.size(1) == 4096 && M <= 16));
 }
 
 void check(const at::Tensor& out, const at::Tensor& x, const at::Tensor& w,
@@ -156,7 +217,19 @@ void skinny_linear(at::Tensor out, at::Tensor x, at::Tensor w,
       dim3(256), 0, at::hip::getCurrentHIPStream(), (short*)out.data_ptr(),   \
       (const short*)x.data_ptr(), x.stride(0), (const short*)w.data_ptr(),    \
       has_bias ? (const short*)bias.data_ptr() : nullptr, M, (int)N, (int)w.size(1))
+#define SLTS_LAUNCH(MT_, S_)                                                  \
+  hipLaunchKernelGGL((skinny_tiles_kernel<MT_, S_, false>),                    \
+      dim3(WORKGROUPS), dim3(256), 0, at::hip::getCurrentHIPStream(),         \
+      (short*)out.data_ptr(), (const short*)x.data_ptr(), x.stride(0),        \
+      (const short*)w.data_ptr(),                                             \
+      has_bias ? (const short*)bias.data_ptr() : nullptr, M, (int)N, (int)w.size(1))
   if (in_tiles(M, N, w.size(1), 16, w.numel())) {
+    if (many_tiles(M, N / 16, w)) {
+      if (w.size(1) == 4096) SLTS_LAUNCH(1, 4);
+      else if (M > 16) SLTS_LAUNCH(2, 2);
+      else SLTS_LAUNCH(1, 2);
+      return;
+    }
     if (w.size(1) % 256 == 0) {
       if (M > 16) SLT_LAUNCH(2, 256); else SLT_LAUNCH(1, 256);
     } else {
@@ -165,6 +238,7 @@ void skinny_linear(at::Tensor out, at::Tensor x, at::Tensor w,
     return;
   }
 #undef SLT_LAUNCH
+#undef SLTS_LAUNCH
   switch (M) {
     case 1: SL_LAUNCH(1, 1); break;
     case 2: SL_LAUNCH(2, 2); break;
@@ -185,7 +259,19 @@ void skinny_swiglu(at::Tensor out, at::Tensor x, at::Tensor w) {
       dim3(256), 0, at::hip::getCurrentHIPStream(), (short*)out.data_ptr(),   \
       (const short*)x.data_ptr(), x.stride(0), (const short*)w.data_ptr(),    \
       nullptr, M, (int)N, (int)w.size(1))
+#define SGTS_LAUNCH(MT_, S_)                                                  \
+  hipLaunchKernelGGL((skinny_tiles_kernel<MT_, S_, true>),                    \
+      dim3(WORKGROUPS), dim3(256), 0, at::hip::getCurrentHIPStream(),         \
+      (short*)out.data_ptr(), (const short*)x.data_ptr(), x.stride(0),        \
+      (const short*)w.data_ptr(),                                             \
+      nullptr, M, (int)N, (int)w.size(1))
   if (in_tiles(M, N, w.size(1), 8, w.numel())) {
+    if (many_tiles(M, N / 8, w)) {
+      if (w.size(1) == 4096) SGTS_LAUNCH(1, 4);
+      else if (M > 16) SGTS_LAUNCH(2, 2);
+      else SGTS_LAUNCH(1, 2);
+      return;
+    }
     if (w.size(1) % 256 == 0) {
       if (M > 16) SGT_LAUNCH(2, 256); else SGT_LAUNCH(1, 256);
     } else {
@@ -194,6 +280,7 @@ void skinny_swiglu(at::Tensor out, at::Tensor x, at::Tensor w) {
     return;
   }
 #undef SGT_LAUNCH
+#undef SGTS_LAUNCH
 #define SG_LAUNCH(M_)                                                         \
   hipLaunchKernelGGL((skinny_linear_kernel<M_, 2, true>),                     \
       dim3((N + NW - 1) / NW), dim3(NW * 64), 0,                              \

@@ -132,6 +132,17 @@ def test_streamed_step(counts, H, IE, mode, bias, part):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("counts,IE,mode,bias,part", [
+    ([5, 0, 16, 17, 1, 40, 3, 33], 2048, 0, True, None),
+    ([2, 1, 3, 0, 1, 1, 2, 2], 2048, 2, False, None),
+    ([16, 9, 1, 30, 2, 8, 7], 1600, 1, True, (1, 5)),
+])
+def test_streamed_step_staying(counts, IE, mode, bias, part):
+    """K = 2048 and enough tiles: workgroups that go from tile to tile."""
+    test_streamed_step(counts, 2048, IE, mode, bias, part)
+
+
+@pytest.mark.gpu
 def test_several_choices_sum():
     torch.manual_seed(3)
     T, H, K = 50, 2056, 6
