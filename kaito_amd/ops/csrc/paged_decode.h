@@ -1,0 +1,486 @@
+// Paged-attention DECODE kernel for gfx950: one query row per sequence, the
+// heads of a kv group in one pass over its K and V pages.
+//
+// A wave walks a contiguous span of keys, 32 at a time, with the products on
+// v_mfma_f32_16x16x32_bf16, transposed as in flash_prefill.h (the group's
+// heads are the 16 columns, unused ones ride along):
+//   - S^T = K Q^T reads K straight from the pages into operand registers (a
+//     16-byte load per lane is 8 dims of one key);
+//   - the scores of one head sit in one column: maximum and rescale factor
+//     are per-lane scalars after two exchanges;
+//   - O^T += V^T P^T takes P from the score registers; V goes to wave-private
+//     LDS by 16-byte direct loads and comes back by transposing reads.
+// P enters as the sum of three bf16 terms, which hold every bit of the f32
+// weight (two of them 16 of its 24). fp8 (e4m3) pages are widened to bf16,
+// exactly, on the way. The waves of a workgroup, and with SPLIT the
+// workgroups of a (sequence, kv head), hold partial (max, sum, O) that are
+// folded at the end.
+//
+// What bounds it: bytes in flight. K and V of a tile (16 KB per wave at
+// D = 128) are all under way at once, while the arithmetic of a tile is
+// about 500 cycles (2 x 16 scores and weights on the vector unit took
+// 3000). Small steps are bound by the chain lengths -> table -> K -> V -> fold:
+// hence 8 waves per workgroup, so that each walks few tiles, and workgroups per
+// pair while those do not fill the chip; fewer waves where there are pairs
+// enough (launch_paged_decode). Measured on one MI355X against a kernel with 4
+// waves per pair, 16-byte K and V streams in two phases and dot products by dot2 +
+// DPP sums (before -> now; 8 kv heads of 128, groups of 4):
+//   1 row, 217 keys: 11.0 -> 6.4 us (8.0 where the table is wide enough for
+//   splits);  16 rows of 4000: 194 -> 43, of 4000 fp8 keys 180 -> 28;  64 rows
+//   of 800: 47 -> 34;  250 of 300: 68 -> 55;  2048 of 220: 429 -> 335 us.
+// Two terms of P would take 0.1 to 5 % off.
+//
+// BIASED is the form of the hybrid stacks' windowed layers
+// (window_attention.hip): scores with a tanh cap and a distance penalty, the
+// mask on keys and not on values. log1pf in place of the penalty's logf took 5
+// us of 25 (32 rows of a 1024-key window); the argument's rounding, 6e-8, is
+// that of the score it is taken from.
+//
+// Cache layout: [num_blocks, KV_HEADS, BLOCK_SIZE, HEAD_DIM] bf16 | e4m3.
+#pragma once
+#include "flash_prefill.h"
+#include <ATen/ATen.h>
+#include <ATen/hip/HIPContext.h>
+
+namespace kaito {
+
+namespace {
+
+using flash::hbf16x8;
+using flash::LOG2E;
+
+constexpr int BS = 16;              // tokens per page
+constexpr int KT = 32;              // keys per wave step: two pages
+constexpr int WIDE = 8;             // waves per workgroup while pairs are few
+constexpr int64_t SPLIT_FILL = 256;  // workgroups that splits aim at
+constexpr int SPLIT_MIN = 2;        // tiles per wave that a split keeps
+
+struct DecodeArgs {
+  short* out;                       // [T, QH, D]
+  const short* q;
+  const void *k, *v;                // [NB, KH, BS, D] bf16 | e4m3
+  const int* block_tables;          // [T, max_blocks]
+  const int* seq_lens;              // [T]
+  float scale;
+  int KH, G, max_blocks;
+  int64_t q_stride;
+  int window;                       // 0 = all keys
+  const float* sinks;               // [QH] or nullptr
+  float* part;                      // SPLIT: [splits, T, QH, D + 2]
+  // BIASED: rows of any sequence, at positions of their own, scores in natural
+  // units cap * tanh(scale q.k / cap) - r1 ln(1 + r2 distance)
+  const int* token_seq;             // [T]: row of block_tables, < 0: none
+  const int64_t* positions;         // [T], in place of seq_lens - 1
+  float cap;                        // 0 = none
+  const float *r1, *r2;             // [QH] or nullptr
+  const short* gate;                // [T, ..]: sigmoid of it times the output
+  int64_t gate_stride;
+
+  template <bool BIASED> KAITO_DEV int len(const int64_t row) const {
+    return BIASED ? (int)positions[row] + 1 : seq_lens[row];
+  }
+};
+
+KAITO_DEV hbf16x8 widen8(const u8x8_t raw) {
+  float f[8];
+  fp8x8_to_f32(raw, f);
+  hbf16x8 w;
+#pragma unroll
+  for (int e = 0; e < 8; e++) w[e] = (__bf16)f[e];
+  return w;
+}
+
+// weights of the partial results of one head: exponent of each maximum
+// against the largest, summed with the sink's into the denominator
+template <bool BIASED>
+KAITO_DEV float fold_weight(float m, float gm) {
+  return __builtin_amdgcn_exp2f(BIASED ? (m - gm) * LOG2E : m - gm);
+}
+
+template <bool BIASED>
+KAITO_DEV void store_head(const DecodeArgs& a, const int64_t row, const int QH,
+                          const int head, const int D, const int d,
+                          const float num, const float den) {
+  float v;
+  if constexpr (BIASED) {
+    v = num / den;
+    if (a.gate)
+      v /= 1.f + expf(-bf16_to_f32(a.gate[row * a.gate_stride + head]));
+  } else {
+    v = num / fmaxf(den, 1e-20f);
+  }
+  a.out[(row * QH + head) * D + d] = f32_to_bf16(v);
+}
+
+// how a sequence's keys are shared out: 32-key tiles from the page that
+// holds the window's first key on, a contiguous run of `per` for every wave.
+// A split is the share of a workgroup's waves, so that with `used` == 1 the
+// first one has every key and writes the result itself.
+struct Spans {
+  int start, base, tiles, per, used;
+};
+KAITO_DEV Spans spans_of(const int seq_len, const int window, const int nsplit,
+                         const int nw) {
+  Spans p;
+  p.start = window > 0 && seq_len > window ? seq_len - window : 0;
+  p.base = p.start / BS * BS;
+  p.tiles = (seq_len - p.base + KT - 1) / KT;
+  p.per = (p.tiles + nsplit * nw - 1) / (nsplit * nw);
+  p.used = p.per > 0 ? (p.tiles + p.per * nw - 1) / (p.per * nw) : 1;
+  return p;
+}
+
+template <int D, bool FP8, int NW, bool SPLIT, bool BIASED>
+__global__ __launch_bounds__(NW * 64, NW <= 4 && D <= 128 ? 3 : 2)
+void paged_decode_kernel(const DecodeArgs a) {
+  constexpr int KK = D / 32;        // 16x16x32 steps over the dims
+  constexpr int DT = D / 16;        // 16-row tiles of O^T
+  constexpr int CV = D / 8;         // 16-byte chunks of a V row
+  constexpr int LV = KT * CV / 64;  // V chunks per lane and tile
+  __shared__ __attribute__((aligned(128))) short lds_v[NW][KT * D];
+  __shared__ float s_m[NW][16], s_l[NW][16];
+
+  const int seq = blockIdx.x / a.KH, kvh = blockIdx.x % a.KH;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lo = lane & 15, hi = lane >> 4;
+  const int QH = a.KH * a.G;
+  const int table = BIASED ? a.token_seq[seq] : seq;
+  if (BIASED && table < 0) {        // a padding row
+    if (!SPLIT || blockIdx.y == 0)
+      for (int i = threadIdx.x; i < a.G * D; i += NW * 64)
+        a.out[((int64_t)seq * QH + kvh * a.G) * D + i] = 0;
+    return;
+  }
+  const int seq_len = a.len<BIASED>(seq);
+  const int* bt = a.block_tables + (int64_t)table * a.max_blocks;
+
+  const int nsplit = SPLIT ? gridDim.y : 1, split = SPLIT ? blockIdx.y : 0;
+  const Spans sp = spans_of(seq_len, a.window, nsplit, NW);
+  if (split >= sp.used) return;     // no keys: the fold does not look here
+  const bool partial = SPLIT && sp.used > 1;
+  const int start = sp.start, base = sp.base;
+  const int t0 = min(sp.tiles, (split * NW + wave) * sp.per);
+  const int t1 = min(sp.tiles, t0 + sp.per);
+  const int last_page = (seq_len - 1) / BS;
+
+  hbf16x8 qf[KK];
+  {
+    const short* qp = a.q + (int64_t)seq * a.q_stride +
+        (int64_t)(kvh * a.G) * D;
+#pragma unroll
+    for (int kk = 0; kk < KK; kk++)
+      qf[kk] = *reinterpret_cast<const hbf16x8*>(
+          qp + min(lo, a.G - 1) * D + hi * 8 + kk * 32);
+  }
+  constexpr float NONE = BIASED ? -INFINITY : -1e30f;
+  float m = NONE, l = 0.f;
+  float r1 = 0.f, r2 = 0.f;
+  if (BIASED && a.r1) {
+    r1 = a.r1[kvh * a.G + min(lo, a.G - 1)];
+    r2 = a.r2[kvh * a.G + min(lo, a.G - 1)];
+  }
+  f32x4 o[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; dt++) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  short* vl = lds_v[wave];
+  const int vrow = 4 * hi + (lo >> 2), vc = (lo & 3) >> 1, ve = (lo & 1) * 4;
+  const float c = a.scale * LOG2E;
+
+  int pages = 0, pages_at = -64;    // lane i: page pages_at + i of the table
+  auto page_row = [&](const int p) {        // first cache row of page p
+    const int pc = min(p, last_page);
+    if (pc >= pages_at + 64) {              // uniform; spans move forward
+      pages_at = pc;
+      pages = bt[min(pc + lane, last_page)];
+    }
+    const int page = __builtin_amdgcn_readlane(pages, pc - pages_at);
+    return ((int64_t)page * a.KH + kvh) * BS;
+  };
+  hbf16x8 kf[2][KK];
+  u8x8_t k8[FP8 ? 2 : 1][FP8 ? KK : 1];
+  auto load_k = [&](const int64_t r0, const int64_t r1) {
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      // uniform page address, 32-bit lane offset
+      const int64_t at = (i ? r1 : r0) * D;
+      const uint32_t off = lo * D + hi * 8;
+#pragma unroll
+      for (int kk = 0; kk < KK; kk++) {
+        if constexpr (FP8)
+          k8[i][kk] = *reinterpret_cast<const u8x8_t*>(
+              (const uint8_t*)a.k + at + (off + kk * 32));
+        else
+          kf[i][kk] = *reinterpret_cast<const hbf16x8*>(
+              (const short*)a.k + at + (off + kk * 32));
+      }
+    }
+  };
+
+  int64_t row0 = 0, row1 = 0;
+  if (t0 < t1) {
+    row0 = page_row(base / BS + t0 * 2);
+    row1 = page_row(base / BS + t0 * 2 + 1);
+    load_k(row0, row1);
+  }
+  for (int t = t0; t < t1; t++) {
+    // ---- V of this tile: slot j * 64 + lane is row s / CV, place s % CV
+    u8x8_t v8[FP8 ? LV : 1];
+#pragma unroll
+    for (int j = 0; j < LV; j++) {
+      const int row = j * (64 / CV) + lane / CV;
+      const int64_t at = (j * (64 / CV) < BS ? row0 : row1) * D;
+      const uint32_t off =
+          row % BS * D + flash::swz_v<D>(row, lane % CV) * 8;
+      if constexpr (FP8)
+        v8[j] = *reinterpret_cast<const u8x8_t*>(
+            (const uint8_t*)a.v + at + off);
+      else
+        flash::lds_copy16((const short*)a.v + at + off, vl + j * 512);
+    }
+    // ---- S^T: keys 16 i + 4 hi + r of head lo
+    f32x4 s[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kk = 0; kk < KK; kk++) {
+        if constexpr (FP8) kf[i][kk] = widen8(k8[i][kk]);
+        s[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[i][kk], qf[kk],
+                                                       s[i], 0, 0, 0);
+      }
+    }
+    if (t + 1 < t1) {               // K of the next tile, under way with V
+      row0 = page_row(base / BS + t * 2 + 2);
+      row1 = page_row(base / BS + t * 2 + 3);
+      load_k(row0, row1);
+    }
+    // ---- softmax
+    const int key0 = base + t * KT;
+    const bool whole = key0 >= start && key0 + KT <= seq_len;
+    float mx = NONE;
+    if constexpr (BIASED) {
+#pragma unroll
+      for (int i = 0; i < 2; i++) s[i] *= a.scale;
+      if (a.cap > 0.f)
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+          s[i / 4][i % 4] = a.cap * tanhf(s[i / 4][i % 4] / a.cap);
+      if (a.r1)
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+          const int key = key0 + 16 * (i / 4) + 4 * hi + i % 4;
+          s[i / 4][i % 4] -=
+              r1 * logf(fmaf(r2, (float)(seq_len - 1 - key), 1.f));
+        }
+    }
+    auto seen = [&](const int i, const int r) {
+      const int key = key0 + 16 * i + 4 * hi + r;
+      return whole || (key >= start && key < seq_len);
+    };
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        if (!BIASED) s[i][r] *= c;
+        if (!seen(i, r)) s[i][r] = NONE;
+        mx = fmaxf(mx, s[i][r]);
+      }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if (__any(mx > m)) {
+      const float mn = fmaxf(m, mx);
+      const float corr = BIASED && m == mn ? 1.f : fold_weight<BIASED>(m, mn);
+      m = mn;
+      l *= corr;
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++) o[dt] *= corr;
+    }
+    hbf16x8 p[3];                   // the weight's leading bits, the rest
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        // a masked key weighs nothing even where a lane saw no other yet
+        const bool live = BIASED ? seen(i, r) : s[i][r] > -1e29f;
+        float w = live ? fold_weight<BIASED>(s[i][r], m) : 0.f;
+        l += w;
+#pragma unroll
+        for (int n = 0; n < 3; n++) {
+          p[n][i * 4 + r] = (__bf16)w;
+          w -= (float)p[n][i * 4 + r];
+        }
+      }
+    if constexpr (FP8) {
+#pragma unroll
+      for (int j = 0; j < LV; j++)
+        *reinterpret_cast<hbf16x8*>(vl + (j * 64 + lane) * 8) = widen8(v8[j]);
+    } else {
+      // the direct loads' data: this wave's own, so no barrier
+      __builtin_amdgcn_s_waitcnt(0x0f70);     // vmcnt(0)
+    }
+    if (!whole) {
+      // slots outside the sequence hold what their last user left, and a
+      // weight of zero does not silence an infinity
+#pragma unroll
+      for (int j = 0; j < LV; j++) {
+        const int key = key0 + j * (64 / CV) + lane / CV;
+        if (key < start || key >= seq_len)
+          *reinterpret_cast<short8_t*>(vl + (j * 64 + lane) * 8) =
+              short8_t{0, 0, 0, 0, 0, 0, 0, 0};
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+    // ---- O^T: dims 16 dt + 4 hi + r of head lo
+#pragma unroll
+    for (int dt = 0; dt < DT; dt += 2) {    // in pairs: neither waits for itself
+      hbf16x8 vf[2];
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const short* at = vl + vrow * D +
+            flash::swz_v<D>(vrow, (dt + u) * 2 + vc) * 8 + ve;
+        const short4_t a4 = flash::read_tr(at);
+        const short4_t b4 = flash::read_tr(at + 16 * D);
+        vf[u] = __builtin_bit_cast(
+            hbf16x8, __builtin_shufflevector(a4, b4, 0, 1, 2, 3, 4, 5, 6, 7));
+      }
+#pragma unroll
+      for (int n = 2; n >= 0; n--)
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+          o[dt + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              vf[u], p[n], o[dt + u], 0, 0, 0);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+
+  // ---- fold the waves: O of the used heads through LDS (the V stage)
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  float* acc = reinterpret_cast<float*>(&lds_v[0][0]) + wave * a.G * D;
+  __syncthreads();
+  if (lo < a.G) {
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++)
+      *reinterpret_cast<f32x4*>(acc + lo * D + dt * 16 + hi * 4) = o[dt];
+    if (hi == 0) { s_m[wave][lo] = m; s_l[wave][lo] = l; }
+  }
+  __syncthreads();
+  acc = reinterpret_cast<float*>(&lds_v[0][0]);
+  for (int idx = threadIdx.x; idx < a.G * D; idx += NW * 64) {
+    const int g = idx / D, d = idx % D, head = kvh * a.G + g;
+    float gm = NONE;
+#pragma unroll
+    for (int w = 0; w < NW; w++) gm = fmaxf(gm, s_m[w][g]);
+    const float sink = a.sinks && !partial
+        ? a.sinks[head] * (BIASED ? 1.f : LOG2E) : NONE;
+    gm = fmaxf(gm, sink);
+    float num = 0.f, den = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      const float e = fold_weight<BIASED>(s_m[w][g], gm);
+      num += e * acc[(w * a.G + g) * D + d];
+      den += e * s_l[w][g];
+    }
+    if (partial) {
+      const int64_t T = gridDim.x / a.KH;
+      float* row = a.part + ((split * T + seq) * QH + head) * (D + 2);
+      row[d] = num;
+      if (d == 0) { row[D] = gm; row[D + 1] = den; }
+    } else {
+      if (a.sinks) den += fold_weight<BIASED>(sink, gm);
+      store_head<BIASED>(a, seq, QH, head, D, d, num, den);
+    }
+  }
+}
+
+// One workgroup per (sequence, head) folds the splits that had keys, unless
+// the first had them all. A chain of loads, so a short one: lane s of every
+// wave has split s's weight.
+template <int D, bool BIASED>
+__global__ __launch_bounds__(D)
+void paged_fold_kernel(const DecodeArgs a, const int QH, const int splits) {
+  const int64_t row = blockIdx.x, rows = gridDim.x;
+  if (BIASED && a.token_seq[row / QH] < 0) return;
+  const int used =
+      spans_of(a.len<BIASED>(row / QH), a.window, splits, WIDE).used;
+  if (used == 1) return;
+  constexpr float NONE = BIASED ? -INFINITY : -1e30f;
+  const int d = threadIdx.x, lane = d & 63;
+  const float sink =
+      a.sinks ? a.sinks[row % QH] * (BIASED ? 1.f : LOG2E) : NONE;
+  float m = NONE, l = 0.f;
+  if (lane < used) {
+    const float* p = a.part + (lane * rows + row) * (D + 2) + D;
+    m = p[0];
+    l = p[1];
+  }
+  const float gm = fmaxf(wave_reduce_max(m), sink);
+  const float e = lane < used ? fold_weight<BIASED>(m, gm) : 0.f;
+  float den = wave_reduce_sum(e * l);
+  if (a.sinks) den += fold_weight<BIASED>(sink, gm);
+  float num = 0.f;
+#pragma unroll 4
+  for (int s = 0; s < used; s++)
+    num += __builtin_bit_cast(float, __builtin_amdgcn_readlane(
+               __builtin_bit_cast(int, e), s)) *
+        a.part[(s * rows + row) * (D + 2) + d];
+  store_head<BIASED>(a, row / QH, QH, (int)(row % QH), D, d, num, den);
+}
+
+template <int D, bool FP8, bool BIASED>
+void launch_paged_decode(DecodeArgs a, const at::Tensor& out, int T) {
+  auto stream = at::hip::getCurrentHIPStream();
+  const int64_t pairs = (int64_t)T * a.KH;
+  // Waves per workgroup and workgroups per pair, by the number of pairs and the
+  // longest context that the table can hold (the lengths are on the device).
+  // Times in us, bf16 / fp8 pages, 4 heads per pair of 128 unless stated.
+  //   Splits up to 128 pairs, two or more workgroups each until 256, as long as
+  // every wave keeps two tiles: 1 row of 16000 keys 24.5 / 21.8, 142 / 140 in one
+  // workgroup per pair, 16 of 4000 43.6 / 28.3 and 44.3 / 40.7; 24 rows, which
+  // would get one and a third, 84 / 49 and 69 / 41. 16 waves in each: 4 of 4000
+  // 20.5 / 21.9, with 8 18.2 / 15.5. Short contexts under a wide table pay
+  // for the fold's launch: 1 row of 40 keys 6.6, 5.0 under a table of 64 (6.0 in
+  // one workgroup of 4 waves before; with one head per pair 6.1, 4.6 and 4.0).
+  //   8 waves while a workgroup has a CU to itself: 32 of 1000 23 / 16, with 16
+  // 24 / 19. Then 4: 64 of 200 12 / 9, with 8 15 / 13; heads of 64 are small
+  // enough for two of 8 (48 of 4000: 71 / 38, with 4 83 / 45).
+  //   2 waves where one round of the chip then takes the pairs that would need
+  // two rounds of 4 (ROUND2 workgroups fit: 128 of 64 keys 7.6 / 7.2, with 4 9.8
+  // / 8.6; of 2000 176 / 94, 186 / 108), and from 4096 pairs on, whose many rounds
+  // cost by the wave (1024 of 64 keys 44 / 31, with 4 55 / 47; heads of 256 44 / 33,
+  // 51 / 45, with 8 twice that), except bf16 pages of grouped heads, where the
+  // contexts to be expected there want 4 (1024 of 300 keys 232 / 130, 223 / 143;
+  // 2048 of 400 594 / 318, 573 / 344) unless windows keep them to a few tiles (2048
+  // of 220 in a window of 128, heads of 64: 124, 141).
+  int64_t longest = (int64_t)a.max_blocks * BS;
+  if (a.window > 0) longest = std::min<int64_t>(longest, a.window + BS);
+#define PA_LAUNCH(NW_, SPLIT_, GRID_)                                         \
+  hipLaunchKernelGGL((paged_decode_kernel<D, FP8, NW_, SPLIT_, BIASED>), GRID_,      \
+                     dim3(NW_ * 64), 0, stream, a)
+  const int64_t splits = std::min<int64_t>(
+      {SPLIT_FILL / pairs, longest / (WIDE * KT * SPLIT_MIN), 64});
+  constexpr int64_t ROUND2 = D <= 64 ? 2048 : D <= 128 ? 1536 : 1024;
+  if (splits > 1) {
+    at::Tensor part = at::empty({splits, T, a.KH * a.G, D + 2},
+                                out.options().dtype(at::kFloat));
+    a.part = part.data_ptr<float>();
+    PA_LAUNCH(WIDE, true, dim3(pairs, splits));
+    hipLaunchKernelGGL((paged_fold_kernel<D, BIASED>), dim3(T * a.KH * a.G),
+                       dim3(D), 0, stream, a, a.KH * a.G, (int)splits);
+  } else if (pairs <= (D <= 64 ? 512 : 256)) {
+    PA_LAUNCH(WIDE, false, dim3(pairs));
+  } else if ((pairs > ROUND2 / 2 && pairs <= ROUND2) ||
+             (pairs >= 4096 &&
+              (FP8 || D > 128 || a.G == 1 || longest <= 5 * KT))) {
+    PA_LAUNCH(2, false, dim3(pairs));
+  } else {
+    PA_LAUNCH(4, false, dim3(pairs));
+  }
+#undef PA_LAUNCH
+}
+
+}  // namespace
+
+}  // namespace kaito

@@ -31,10 +31,12 @@
 // [blocks, G, block_size, D|V] in the activation dtype. Scores, softmax
 // weights and the output accumulation are f32.
 //
-// Three kernels share these semantics:
+// Four kernels share these semantics:
 //   flash_prefill_kernel           bf16 prompt portions, 64-row query tiles
 //                                  (flash_prefill.h)
-//   window_attention_decode_kernel single rows (and f32 portions), the
+//   paged_decode_kernel            bf16 single rows with plain softmax masks
+//                                  (paged_decode.h)
+//   window_attention_decode_kernel other single rows (and f32 portions), the
 //                                  heads of a kv group in one pass
 //   window_attention_kernel        any sizes: one workgroup per (row, head),
 //                                  one thread scores one key, the tile's
@@ -42,8 +44,8 @@
 //                                  thread-per-value-dim
 // All fold key tiles with the running-max (online softmax) recurrence, so
 // any window length works.
-#include "flash_prefill.h"
 #include "mix_common.h"
+#include "paged_decode.h"
 
 namespace kaito {
 
@@ -865,6 +867,44 @@ void window_attention(at::Tensor out, at::Tensor q, at::Tensor k_cache,
   TORCH_CHECK((int64_t)k_cache.size(0) * G * BS < (1ll << 31));
   if (T == 0) return;
   auto stream0 = at::hip::getCurrentHIPStream();
+  // Matrix-core decode (paged_decode.h): softmax over bf16 pages of 16 with any
+  // window, cap, penalty, sinks and head gates. us, decode kernel below and
+  // now, 16 heads of 128 on 4 kv heads, window 1024: 32 rows of 2049 keys 39.7
+  // and 19.6, 8 of up to 2000 31.5 and 17.1, 96 of 600 69 and 23, 500 of 250 136
+  // and 44, one of 300 14.3 and 8.7; where it gains least, one head per kv
+  // head: 96 of 600, 8 heads of 128, 40.8 and 38.9, 4 of 256 41.9 and 40.7.
+  const int rep = H / G;
+  if (q.dtype() == at::kBFloat16 && D == V && BS == 16 &&
+      (D == 64 || D == 128 || D == 256) && rep <= (D == 256 ? 4 : 8) &&
+      kf == 0 && chunk == 0 && pb == nullptr && db == nullptr &&
+      temp_coef == 0 && (uintptr_t)q.data_ptr() % 16 == 0 &&
+      (uintptr_t)k_cache.data_ptr() % 16 == 0 &&
+      (uintptr_t)v_cache.data_ptr() % 16 == 0) {
+    DecodeArgs a{};
+    a.out = (short*)out.data_ptr();
+    a.q = (const short*)q.data_ptr();
+    a.k = k_cache.data_ptr();
+    a.v = v_cache.data_ptr();
+    a.block_tables = block_tables.data_ptr<int>();
+    a.max_blocks = (int)block_tables.size(1);
+    a.scale = (float)scale;
+    a.KH = G;
+    a.G = rep;
+    a.q_stride = (int64_t)H * D;
+    a.window = window > 0 ? (int)window : 0;
+    a.sinks = has_sinks ? sinks.data_ptr<float>() : nullptr;
+    a.token_seq = token_seq.data_ptr<int>();
+    a.positions = positions.data_ptr<int64_t>();
+    a.cap = (float)softcap;
+    a.r1 = bias ? r1.data_ptr<float>() : nullptr;
+    a.r2 = bias ? r2.data_ptr<float>() : nullptr;
+    a.gate = gated ? (const short*)gate.data_ptr() : nullptr;
+    a.gate_stride = gated ? gate.stride(0) : 0;
+    if (D == 64) launch_paged_decode<64, false, true>(a, out, T);
+    else if (D == 128) launch_paged_decode<128, false, true>(a, out, T);
+    else launch_paged_decode<256, false, true>(a, out, T);
+    return;
+  }
   if (decode_kernel_fits(D, V, (int)q.element_size())) {
     const int R = H / G;
     // heads per workgroup: share K/V reads across the group when the step

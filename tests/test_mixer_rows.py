@@ -147,6 +147,66 @@ def test_rglru_closed_output_gate(z):
     assert out.abs().max().item() < 1e-30
 
 
+@pytest.mark.parametrize("D,H,G", [(64, 3, 3), (128, 8, 1), (128, 6, 2),
+                                   (256, 8, 2)])
+@pytest.mark.parametrize("window,cap,bias,sink,gated",
+                         [(100, 20.0, True, False, False),
+                          (0, 0.0, True, True, True),
+                          (33, 0.0, False, False, False)])
+def test_window_decode_rows(D, H, G, window, cap, bias, sink, gated):
+    """Single rows on the matrix cores: lengths around pages, tiles and
+    splits, a padding row, slots past a row that hold NaN."""
+    torch.manual_seed(D + H)
+    lens = [1, 15, 16, 17, 32, 33, 100, 1, 131, 1040]
+    T, BS = len(lens), 16
+    pages = [-(-n // BS) for n in lens]
+    kc = torch.randn(sum(pages), G, BS, D, device=DEV).to(torch.bfloat16)
+    vc = torch.randn(sum(pages), G, BS, D, device=DEV).to(torch.bfloat16)
+    table = torch.zeros(T, max(pages), dtype=torch.int32)
+    at = 0
+    for b, n in enumerate(lens):
+        table[b, :pages[b]] = torch.arange(at, at + pages[b])
+        at += pages[b]
+        if n % BS:
+            kc[at - 1, :, n % BS:] = float("nan")
+            vc[at - 1, :, n % BS:] = float("nan")
+    q = 2 * torch.randn(T, H, D, device=DEV).to(torch.bfloat16)
+    r1 = torch.rand(H, device=DEV) if bias else None
+    r2 = torch.rand(H, device=DEV) if bias else None
+    sinks = torch.randn(H, device=DEV) if sink else None
+    gate = torch.randn(T, H, device=DEV).to(torch.bfloat16) if gated else None
+    seq = torch.arange(T, dtype=torch.int32, device=DEV)
+    seq[7] = -1
+    pos = torch.tensor(lens, device=DEV) - 1
+    out = ops.window_attention(q, kc, vc, table.to(DEV), seq, pos, D ** -0.5,
+                               cap, r1, r2, window, sinks=sinks, gate=gate)
+    assert (out[7] == 0).all()
+    for t, n in enumerate(lens):
+        if t == 7:
+            continue
+        lo = max(0, n - window) if window else 0
+        rows = table[t, :pages[t]].long()
+        k, v = (c[rows].transpose(1, 2).reshape(-1, G, D)[lo:n].double()
+                .repeat_interleave(H // G, 1) for c in (kc, vc))
+        s = (k * q[t].double()).sum(-1).T * D ** -0.5          # [H, keys]
+        if cap:
+            s = cap * torch.tanh(s / cap)
+        if bias:
+            dist = torch.arange(n - 1 - lo, -1, -1, device=DEV).double()
+            s = s - r1.double()[:, None] * torch.log1p(
+                r2.double()[:, None] * dist)
+        if sink:
+            s = torch.cat([s, sinks.double()[:, None]], 1)
+        p = s.softmax(-1)[:, :n - lo]
+        ref = (p.T[:, :, None] * v).sum(0)
+        if gated:
+            ref = ref * torch.sigmoid(gate[t].double())[:, None]
+        # rounded once to bf16, half a unit of 8 bits; f32 scores and sums are
+        # far below
+        err = (out[t].double() - ref).abs()
+        assert (err <= 2.0 ** -8 * ref.abs() + 2e-5).all(), (t, n)
+
+
 @pytest.mark.parametrize("lens", [[1, 2, 3, 4, 5, 9], [31], [8, 64]])
 @pytest.mark.parametrize("D,V,a0", [(128, 128, -2.0), (64, 20, 3.0),
                                     (256, 8, -6.0), (12, 12, 0.0)])
