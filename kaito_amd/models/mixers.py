@@ -127,7 +127,7 @@ class RGLRUMixer(nn.Module):
         self.conv_weight = _p(w, spec.conv_taps, dtype=torch.float32)
         self.conv_bias = _p(w, dtype=torch.float32)
         # per block, rows [recurrence gate | input gate], stored
-        # transposed ([in, out]) for the batched product; f32: the gates
+        # transposed ([in, out]) for the product; f32: the gates
         # enter the recurrence
         self.gate_w = _p(nb, self.bw, 2 * self.bw, dtype=torch.float32)
         self.gate_b = _p(nb, 1, 2 * self.bw, dtype=torch.float32)
@@ -157,8 +157,7 @@ class RGLRUMixer(nn.Module):
             p[:, w:], self.conv_weight, self.conv_bias, cache["conv"],
             meta.cu_seqlens, meta.state_slots, meta.seq_starts,
             meta.token_seq, act=0)
-        ub = u.float().view(T, s.blocks, self.bw).transpose(0, 1)
-        gates = torch.baddbmm(self.gate_b, ub, self.gate_w)   # [B, T, 2bw]
+        gates = ops.rglru_gates(u, self.gate_w, self.gate_b)  # [B, T, 2bw]
         o = ops.rglru_scan(u, gates, p[:, :w], self.decay_rate, cache["lru"],
                            meta.cu_seqlens, meta.state_slots, meta.seq_starts,
                            meta.token_seq)

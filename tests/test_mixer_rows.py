@@ -134,6 +134,31 @@ def test_rglru_very_long_steps(T):
     assert ((one - parts).abs() <= 2.0 ** -14 * (1 + parts.abs())).all()
 
 
+@pytest.mark.parametrize("T", [1, 31, 32, 33, 1100])
+@pytest.mark.parametrize("B,bw", [(1, 64), (3, 128), (16, 128), (2, 32)])
+def test_rglru_gates(T, B, bw):
+    """Rows around the 32 of a tile, several tiles per workgroup; sizes of the
+    batched product."""
+    torch.manual_seed(T + bw)
+    big = torch.randn(T, B * bw + 24, device=DEV).to(torch.bfloat16)
+    u = big[:, 8:8 + B * bw]
+    w = torch.randn(B, bw, 2 * bw, device=DEV)
+    b = torch.randn(B, 1, 2 * bw, device=DEV)
+    if T > 1:
+        u[T // 2, 3], u[0, 5], u[1, 9] = float("inf"), -float("inf"), \
+            float("nan")
+    ub = u.reshape(T, B, bw).transpose(0, 1).contiguous()
+    ref = torch.baddbmm(b.double(), ub.double(), w.double())
+    out = ops.rglru_gates(u, w, b)
+    fine = ref.isfinite()
+    assert torch.equal(out.isnan(), ref.isnan())
+    assert torch.equal(out.double()[ref.isinf()], ref[ref.isinf()])
+    # an f32 sum of 3 bw products, every rounding at its worst
+    size = torch.baddbmm(b.abs(), ub.float().abs(), w.abs()).double()
+    err = (out.double() - ref).abs()
+    assert (err[fine] <= 3 * bw * 2.0 ** -24 * size[fine]).all()
+
+
 @pytest.mark.parametrize("z", [-20.0, -1e4, -1e20, -1e36])
 def test_rglru_closed_output_gate(z):
     """gelu of a large negative value is 0, however large."""
