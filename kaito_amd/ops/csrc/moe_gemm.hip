@@ -12,24 +12,33 @@
 // wave, so a lane holds both of a pair) in K steps of 64 on
 // v_mfma_f32_32x32x16_bf16, transposed (C^T = W X^T: a lane owns one token row
 // and 4 neighbouring outputs at a time). Both operands arrive by 16-byte
-// loads straight to LDS one K step ahead (two buffers, one barrier per step;
-// 16-byte chunk c of row r at c ^ (r & 7)); as buffer loads, behind which the
-// compiler can count LDS reads (behind the global form it waits for all).
-// At BM = 256 a step is 32 MFMA per wave, 2048 cycles of a SIMD's two waves,
-// against 192 KB of LDS reads (1536 cycles) and 64 KB of staging per CU: both
-// have to overlap, so fragments are read one step of 16 dims ahead.
+// loads straight to LDS (16-byte chunk c of row r at c ^ (r & 7)); as buffer
+// loads, behind which the compiler can count LDS reads (behind the global form
+// it waits for all). At BM = 256 a step is 32 MFMA per wave, 2048 cycles of a
+// SIMD's two waves, against 192 KB of LDS reads (1536 cycles) and 64 KB of
+// staging per CU: all have to overlap, so fragments are read one step of 16 dims
+// ahead and the loads go out a few at a time. The bound is the way from the
+// caches to LDS: without the products the loads alone take nine tenths of the
+// time, without the loads the rest takes four fifths. (K steps of 32 in four or
+// five buffers, whose rows are half lines: a tenth slower; waves of a SIMD taking
+// turns behind barriers, other starts in K per tile: no change.)
 //
 // Tiles are numbered expert by expert, in blocks of 4 column tiles x all row
 // tiles, and every XCD takes one contiguous eighth of them: the 32 tiles in
-// flight behind one L2 share rows and weights. Measured on one MI355X, 8
-// experts of 2048 x 2048, top 2, 8192 tokens: 309 + 166 + 17 us (890 and 829
-// TFLOP/s; 333 + 201 with the reads beside their products and 8-byte stores)
-// where a library GEMM per expert with its gathers, casts and index_add took
-// 958 us behind a host read. 8 of 4096 x 14336: 1141 and 1027 TFLOP/s.
+// flight behind one L2 share rows and weights. A last round of up to 8 tiles for
+// an XCD's 32 CUs is cut in quarters, 128 x 128, one per CU; so is a small step's
+// only round of up to 16. Measured on one MI355X, 8 experts of 2048 x 2048, top
+// 2, rows as drawn from 16 kinds of tokens, us, two buffers and whole tiles, now:
+// 8192 tokens 317 and 278 (990 TFLOP/s), down 165 and 139; 4096 174 and 149, 106
+// and 86; 2048 114 and 90; 1000 down 60 and 49. 8 of 4096 x 14336, 8192 tokens:
+// 3419 and 3262 (1180 TFLOP/s), 1875 and 1676. 8-byte stores cost a tenth more. A
+// library GEMM per expert with its gathers, casts and index_add took 958 us behind
+// a host read at the first of these.
 #include "flash_prefill.h"
 #include <torch/library.h>
 #include <ATen/ATen.h>
 #include <ATen/hip/HIPContext.h>
+#include <type_traits>
 
 namespace kaito {
 
@@ -42,6 +51,12 @@ using flash::mfma32;
 constexpr int BK = 64;              // K step
 constexpr int BN = 256;             // weight rows per tile
 constexpr int NG = 4;               // column tiles that share row tiles
+constexpr int XCD_CUS = 32;
+// A quarter takes about two fifths of a tile's time, and the last round runs on
+// caches of its own: 17 to 24 tiles in three rounds of quarters lost (2880 x 2880,
+// 4096 tokens, down: 341 and 352 us), 9 to 16 in two broke even or lost 1 %, except
+// where they are the whole step (58 and 50).
+constexpr int QUARTER_REST = XCD_CUS / 4;
 
 struct GemmArgs {
   short* out;                       // [TK, N]
@@ -77,63 +92,22 @@ KAITO_DEV float gated(int mode, float g, float u, float limit) {
   return silu_of(g) * u;
 }
 
-template <int BM, int KIND>
-__global__ __launch_bounds__(512, 2) void moe_grouped_kernel(const GemmArgs a) {
-  constexpr int MT = BM / 64;       // 32-row tiles of a wave
-  constexpr int COLS = KIND == UP_GATED ? BN / 2 : BN;   // outputs per tile
-  constexpr int LX = BM * BK / 8 / 512, LW = BN * BK / 8 / 512;
-  __shared__ __attribute__((aligned(128))) short lds[2][(BM + BN) * BK];
+// elements of LDS: two and a half K steps of a whole tile, five of a quarter
+constexpr int LDS = 5 * 256 * BK;
 
+// BM rows x BW weight rows of one expert by 8 waves, WM of them over the rows;
+// NST K steps in LDS, or 0: five slots of BM = BW rows. m0: first row, n0: first
+// output.
+template <int BM, int BW, int WM, int NST, int KIND>
+KAITO_DEV void grouped_tile(const GemmArgs& a, short* lds, const int expert,
+                            const int m0, const int row_end, const int n0) {
+  constexpr int WN = 8 / WM, MT = BM / WM / 32;   // 32-row tiles of a wave
+  constexpr int LX = BM * BK / 8 / 512, LW = BW * BK / 8 / 512;
+  constexpr int STEP = (BM + BW) * BK;
+  static_assert(WN * 64 == BW && NST * STEP <= LDS, "tile");
   const int lane = threadIdx.x & 63, lr = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = wave >> 2, wn = wave & 3;
-  const int ntiles = (a.N + COLS - 1) / COLS;
-
-  // ---- this workgroup's tile: every wave scans the experts, 64 at a time
-  int total = 0;
-  for (int e0 = 0; e0 < a.E; e0 += 64) {
-    const int e = a.e_base + e0 + lane;
-    int n = e0 + lane < a.E
-        ? (a.offsets[e + 1] - a.offsets[e] + BM - 1) / BM : 0;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
-    total += n;
-  }
-  total = __builtin_amdgcn_readfirstlane(total) * ntiles;
-  const int share = (total + 7) / 8;
-  const int in_share = blockIdx.x / 8;
-  int t = (blockIdx.x % 8) * share + in_share;
-  if (in_share >= share || t >= total) return;
-  int expert = -1, mtiles = 0, row0 = 0, row_end = 0;
-  for (int e0 = 0; e0 < a.E && expert < 0; e0 += 64) {
-    const int e = a.e_base + e0 + lane;
-    const int o0 = e0 + lane < a.E ? a.offsets[e] : 0;
-    const int o1 = e0 + lane < a.E ? a.offsets[e + 1] : 0;
-    const int n = (o1 - o0 + BM - 1) / BM;
-    int scan = n;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int add = __shfl_up(scan, off, 64);
-      if (lane >= off) scan += add;
-    }
-    const unsigned long long hit = __ballot(scan * ntiles > t);
-    if (hit) {
-      const int src = __builtin_ctzll(hit);
-      expert = a.e_base + e0 + src;
-      mtiles = __builtin_amdgcn_readlane(n, src);
-      t -= (__builtin_amdgcn_readlane(scan, src) - mtiles) * ntiles;
-      row0 = __builtin_amdgcn_readlane(o0, src);
-      row_end = __builtin_amdgcn_readlane(o1, src);
-    } else {
-      t -= __builtin_amdgcn_readlane(scan, 63) * ntiles;
-    }
-  }
-  // blocks of NG column tiles, column fastest
-  const int blk = t / (NG * mtiles);
-  const int wide = min(NG, ntiles - blk * NG);
-  const int in_blk = t - blk * NG * mtiles;
-  const int nt = blk * NG + in_blk % wide, mt0 = in_blk / wide;
-  const int m0 = row0 + mt0 * BM, n0 = nt * COLS;
+  const int wm = wave / WN, wn = wave % WN;
 
   // ---- staging slots: slot s (16 bytes) is row s / 8, place s % 8; byte
   // offsets from the tile's first row (gathered rows: from x, which the caller
@@ -145,19 +119,26 @@ __global__ __launch_bounds__(512, 2) void moe_grouped_kernel(const GemmArgs a) {
       const_cast<short*>(xe), 0, 0xffffffff, 0x27000);
   const auto wr = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<short*>(we), 0, 0xffffffff, 0x27000);
+  constexpr int CH = BK / 8;        // 16-byte chunks of a row
+  auto place = [](const int row, const int c) { return c ^ (row & 7); };
   uint32_t xs[LX], ws[LW];
+  int src[LX];                      // one wait for all of them
+#pragma unroll
+  for (int j = 0; j < LX; j++)
+    src[j] = min((int)(j * 512 + threadIdx.x) / CH, row_end - 1 - m0);
+  if (a.rows) {
+#pragma unroll
+    for (int j = 0; j < LX; j++) src[j] = a.rows[m0 + src[j]];
+  }
 #pragma unroll
   for (int j = 0; j < LX; j++) {
-    const int s = j * 512 + threadIdx.x, row = s / 8;
-    const int c = (s % 8) ^ (row & 7);
-    const int m = min(m0 + row, row_end - 1);
-    const uint32_t src = a.rows ? a.rows[m] : m - m0;
-    xs[j] = (src * a.K + c * 8) * 2;
+    const int s = j * 512 + threadIdx.x;
+    xs[j] = ((uint32_t)src[j] * a.K + place(s / CH, s % CH) * 8) * 2;
   }
 #pragma unroll
   for (int j = 0; j < LW; j++) {
-    const int s = j * 512 + threadIdx.x, row = s / 8;
-    const int c = (s % 8) ^ (row & 7);
+    const int s = j * 512 + threadIdx.x, row = s / CH;
+    const int c = place(row, s % CH);
     // gated: every 64 tile rows are 32 gate rows, then their up rows
     const uint32_t n = KIND == UP_GATED
         ? min((row / 64) * 32 + row % 32, a.N - 1 - n0) +
@@ -165,14 +146,16 @@ __global__ __launch_bounds__(512, 2) void moe_grouped_kernel(const GemmArgs a) {
         : min(row, a.N - 1 - n0);
     ws[j] = (n * a.K + c * 8) * 2;
   }
-  auto stage = [&](const int k, short* buf) {
+  auto stage_x = [&](const int k, short* buf, const int j0, const int j1) {
 #pragma unroll
     for (int j = 0; j < LX; j++)
-      buffer_copy16(xr, buf + (j * 512 + wave * 64) * 8, xs[j], k * 2);
+      if (j >= j0 && j < j1)
+        buffer_copy16(xr, buf + (j * 512 + wave * 64) * 8, xs[j], k * 2);
+  };
+  auto stage_w = [&](const int k, short* buf) {
 #pragma unroll
     for (int j = 0; j < LW; j++)
-      buffer_copy16(wr, buf + BM * BK + (j * 512 + wave * 64) * 8, ws[j],
-                    k * 2);
+      buffer_copy16(wr, buf + (j * 512 + wave * 64) * 8, ws[j], k * 2);
   };
 
   f32x16 acc[2][MT];
@@ -187,10 +170,10 @@ __global__ __launch_bounds__(512, 2) void moe_grouped_kernel(const GemmArgs a) {
   // first of the next tile beside the last products of this one: the barrier
   // that frees this tile stands between its last read and its last products.
   hbf16x8 wf[2][2], xf[2][MT];
-  auto read = [&](const short* buf, const int kk) {
-    const int c = ((kk * 2 + h) ^ (lr & 7)) * 8, f = kk & 1;
-    const short* xb = buf + (wm * (BM / 2) + lr) * BK + c;
-    const short* wb = buf + BM * BK + (wn * 64 + lr) * BK + c;
+  auto read = [&](const short* xbuf, const short* wbuf, const int kk) {
+    const int c = place(lr, kk * 2 + h) * 8, f = kk & 1;
+    const short* xb = xbuf + (wm * (BM / WM) + lr) * BK + c;
+    const short* wb = wbuf + (wn * 64 + lr) * BK + c;
 #pragma unroll
     for (int i = 0; i < 2; i++)
       wf[f][i] = *reinterpret_cast<const hbf16x8*>(wb + i * 32 * BK);
@@ -208,29 +191,80 @@ __global__ __launch_bounds__(512, 2) void moe_grouped_kernel(const GemmArgs a) {
         acc[i][j] = mfma32(wf[f][i], xf[f][j], acc[i][j]);
     __builtin_amdgcn_sched_barrier(0);
   };
-  auto meet = [&]() {               // own loads landed and reads done: all's
-    __builtin_amdgcn_s_waitcnt(0x0070);     // vmcnt(0) lgkmcnt(0)
+  // own reads done and own loads landed but for the newest LATER: all's
+  auto meet = [&](auto newest, const bool later) {
+    constexpr int N = decltype(newest)::value;
+    if (N > 0 && later)
+      __builtin_amdgcn_s_waitcnt(0x0070 | (N & 15) | ((N >> 4) << 14));
+    else
+      __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  constexpr int LAST = BK / 16 - 1;
 
-  stage(0, lds[0]);
-  meet();
-  if (BK < a.K) stage(BK, lds[1]);
-  read(lds[0], 0);
-  int cur = 0;
-  for (int k = 0; k < a.K; k += BK) {
-#pragma unroll
-    for (int kk = 0; kk < LAST; kk++) {
-      read(lds[cur], kk + 1);
-      multiply(kk);
+  if constexpr (NST == 0) {
+    // x and w by turns through five slots: x(s), w(s) and x(s + 1) are there
+    // when step s begins, w(s + 1) and x(s + 2) are asked for in its course.
+    // All of a step's loads at once, for the next but one, kept the caches busy
+    // in bursts: 514 cycles from request to data where 360 are now.
+    constexpr int SLOT = BM * BK;
+    static_assert(BM == BW && 5 * SLOT <= LDS && BK == 64, "slots");
+    constexpr std::integral_constant<int, LX> newest;
+    stage_w(0, lds + SLOT);
+    stage_x(0, lds, 0, LX);
+    if (BK < a.K) stage_x(BK, lds + 2 * SLOT, 0, LX);
+    meet(newest, BK < a.K);
+    int slot = 0;                   // of x(s); w(s), x(s + 1) .. follow
+    auto nth = [&](const int i) {
+      return lds + (slot + i < 5 ? slot + i : slot + i - 5) * SLOT;
+    };
+    read(nth(0), nth(1), 0);
+    for (int k = 0; k < a.K; k += BK) {
+      const bool more = k + BK < a.K, more2 = k + 2 * BK < a.K;
+      read(nth(0), nth(1), 1);
+      if (more) stage_w(k + BK, nth(3));
+      multiply(0);
+      read(nth(0), nth(1), 2);
+      if (more2) stage_x(k + 2 * BK, nth(4), 0, LX / 2);
+      multiply(1);
+      read(nth(0), nth(1), 3);
+      if (more2) stage_x(k + 2 * BK, nth(4), LX / 2, LX);
+      multiply(2);
+      meet(newest, more2);
+      slot = slot < 3 ? slot + 2 : slot - 3;
+      if (more) read(nth(0), nth(1), 0);
+      multiply(3);
     }
-    meet();
-    if (k + 2 * BK < a.K) stage(k + 2 * BK, lds[cur]);
-    if (k + BK < a.K) read(lds[cur ^ 1], 0);
-    multiply(LAST);
-    cur ^= 1;
+  } else {
+    constexpr int STEPS = BK / 16;
+    constexpr std::integral_constant<int, (NST - 2) * (LX + LW)> newest;
+    auto stage = [&](const int k, const int at) {
+      stage_x(k, lds + at * STEP, 0, LX);
+      stage_w(k, lds + at * STEP + BM * BK);
+    };
+    auto next = [&](const int at, const int kk) {
+      read(lds + at * STEP, lds + at * STEP + BM * BK, kk);
+    };
+    stage(0, 0);
+#pragma unroll
+    for (int i = 1; i < NST - 1; i++)
+      if (i * BK < a.K) stage(i * BK, i);
+    meet(newest, (NST - 2) * BK < a.K);
+    if ((NST - 1) * BK < a.K) stage((NST - 1) * BK, NST - 1);
+    next(0, 0);
+    int cur = 0;
+    for (int k = 0; k < a.K; k += BK) {
+#pragma unroll
+      for (int kk = 0; kk < STEPS - 1; kk++) {
+        next(cur, kk + 1);
+        multiply(kk);
+      }
+      meet(newest, k + (NST - 1) * BK < a.K);
+      if (k + NST * BK < a.K) stage(k + NST * BK, cur);
+      cur = cur == NST - 1 ? 0 : cur + 1;
+      if (k + BK < a.K) next(cur, 0);
+      multiply(STEPS - 1);
+    }
   }
 
   // ---- outputs n = 8 b + 4 h + e of 32-row tile i, token row lr of tile j
@@ -256,10 +290,10 @@ __global__ __launch_bounds__(512, 2) void moe_grouped_kernel(const GemmArgs a) {
   // bf16 rows pass through the wave's part of LDS (every wave is done with
   // its tiles) and leave as 16 bytes a lane
   constexpr int PITCH = WC + 8, LANES = WC / 8;
-  short* slab = &lds[0][0] + wave * 32 * PITCH;
+  short* slab = lds + wave * 32 * PITCH;
 #pragma unroll
   for (int j = 0; j < MT; j++) {
-    const int mj = m0 + wm * (BM / 2) + j * 32;
+    const int mj = m0 + wm * (BM / WM) + j * 32;
 #pragma unroll
     for (int i = 0; i < NI; i++)
 #pragma unroll
@@ -301,6 +335,83 @@ __global__ __launch_bounds__(512, 2) void moe_grouped_kernel(const GemmArgs a) {
     __builtin_amdgcn_wave_barrier();
     asm volatile("" ::: "memory");
   }
+}
+
+template <int BM, int KIND>
+__global__ __launch_bounds__(512, 2) void moe_grouped_kernel(const GemmArgs a) {
+  constexpr int COLS = KIND == UP_GATED ? BN / 2 : BN;   // outputs per tile
+  constexpr bool QUARTERS = BM == 256;
+  __shared__ __attribute__((aligned(128)))
+  short lds[BM == 256 ? LDS : 2 * (BM + BN) * BK];
+  const int lane = threadIdx.x & 63;
+  const int ntiles = (a.N + COLS - 1) / COLS;
+
+  // ---- this workgroup's tile: every wave scans the experts, 64 at a time
+  int total = 0;
+  for (int e0 = 0; e0 < a.E; e0 += 64) {
+    const int e = a.e_base + e0 + lane;
+    int n = e0 + lane < a.E
+        ? (a.offsets[e + 1] - a.offsets[e] + BM - 1) / BM : 0;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+    total += n;
+  }
+  total = __builtin_amdgcn_readfirstlane(total) * ntiles;
+  const int share = (total + 7) / 8, at = (blockIdx.x % 8) * share;
+  const int here = min(share, total - at);  // tiles of this XCD
+  int rest = here % XCD_CUS;        // of its last round
+  if (!QUARTERS || rest > (here < XCD_CUS ? 2 : 1) * QUARTER_REST) rest = 0;
+  int in_share = blockIdx.x / 8, quarter = -1;
+  if (in_share >= here - rest) {
+    const int p = in_share - (here - rest);
+    if (p >= 4 * rest) return;
+    in_share = here - rest + p / 4;
+    quarter = p % 4;
+  }
+  int t = at + in_share;
+  int expert = -1, mtiles = 0, row0 = 0, row_end = 0;
+  for (int e0 = 0; e0 < a.E && expert < 0; e0 += 64) {
+    const int e = a.e_base + e0 + lane;
+    const int o0 = e0 + lane < a.E ? a.offsets[e] : 0;
+    const int o1 = e0 + lane < a.E ? a.offsets[e + 1] : 0;
+    const int n = (o1 - o0 + BM - 1) / BM;
+    int scan = n;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int add = __shfl_up(scan, off, 64);
+      if (lane >= off) scan += add;
+    }
+    const unsigned long long hit = __ballot(scan * ntiles > t);
+    if (hit) {
+      const int src = __builtin_ctzll(hit);
+      expert = a.e_base + e0 + src;
+      mtiles = __builtin_amdgcn_readlane(n, src);
+      t -= (__builtin_amdgcn_readlane(scan, src) - mtiles) * ntiles;
+      row0 = __builtin_amdgcn_readlane(o0, src);
+      row_end = __builtin_amdgcn_readlane(o1, src);
+    } else {
+      t -= __builtin_amdgcn_readlane(scan, 63) * ntiles;
+    }
+  }
+  // blocks of NG column tiles, column fastest
+  const int blk = t / (NG * mtiles);
+  const int wide = min(NG, ntiles - blk * NG);
+  const int in_blk = t - blk * NG * mtiles;
+  const int nt = blk * NG + in_blk % wide, mt0 = in_blk / wide;
+
+  const int m0 = row0 + mt0 * BM, n0 = nt * COLS;
+  if constexpr (QUARTERS) {
+    if (quarter >= 0) {
+      const int m = m0 + quarter / 2 * (BM / 2);
+      const int n = n0 + quarter % 2 * (COLS / 2);
+      if (m < row_end && n < a.N)
+        grouped_tile<BM / 2, BN / 2, 4, 5, KIND>(a, lds, expert, m, row_end,
+                                                 n);
+      return;
+    }
+  }
+  grouped_tile<BM, BN, 2, BM == 256 ? 0 : 2, KIND>(a, lds, expert, m0, row_end,
+                                                   n0);
 }
 
 // one workgroup per token, 8 outputs per thread and pass
@@ -360,8 +471,11 @@ void launch_grouped(const GemmArgs& a, int64_t TK) {
     constexpr int BM = decltype(bm)::value;
     // most row tiles that TK rows in E groups can make
     const int64_t most = TK / BM + std::min<int64_t>(a.E, TK);
+    // per XCD, a rest's quarters in place of its tiles
+    const int64_t quarters = BM == 256 ? 3 * 2 * QUARTER_REST : 0;
     hipLaunchKernelGGL((moe_grouped_kernel<BM, KIND>),
-        dim3((most * ntiles + 7) / 8 * 8), dim3(512), 0, stream, a);
+        dim3(((most * ntiles + 7) / 8 + quarters) * 8), dim3(512), 0, stream,
+        a);
   };
   // half tiles where an expert's rows would leave most of a whole one empty
   if (TK >= 192 * (int64_t)a.E) launch(std::integral_constant<int, 256>{});

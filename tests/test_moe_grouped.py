@@ -82,6 +82,17 @@ def test_grouped_step(counts, H, IE, mode, bias, part, f32):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("counts,H,IE,mode,bias", [
+    ([5000, 0, 130, 500], 1600, 1600, 0, True),    # 38 and 21 tiles per XCD
+    ([700, 3201], 64, 1088, 2, False),             # 10 and 2; a K of 64
+    ([4097, 1100], 192, 2176, 1, False),
+])
+def test_grouped_rounds(counts, H, IE, mode, bias):
+    """Whole rounds of tiles, last ones in quarters or not, few steps of K."""
+    test_grouped_step(counts, H, IE, mode, bias, None, False)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("counts,H,IE,mode,bias,part", [
     ([1], 64, 64, 0, False, None),
     ([3, 0, 16, 17, 1], 256, 192, 0, True, None),
