@@ -29,7 +29,7 @@ from ..engine.config import ModelConfig
 from .hybrid_base import HybridStackBase, MixerLayerBase
 from .hybrid_config import LayerSpec, layer_moe_config
 from .mixers import BiasedWindowAttention, GatedDeltaMixer, RGLRUMixer
-from .moe import MoEMLP
+from .moe import MoEMLP, MoERows
 
 
 def _vec(n):
@@ -76,8 +76,10 @@ class HybridLayer(MixerLayerBase):
                                         w_y=self.attn_out_norm,
                                         w_y2=self.rglru_out_norm)
         if self.mlp is not None:
-            f = self.mlp(xa)
-            xa = ops.post_norm_residual(x32, f, self.norm2, eps, dt)
+            f = self.mlp(xa, defer=True)
+            xa = f.post_norm(x32, self.norm2, eps, dt) \
+                if isinstance(f, MoERows) \
+                else ops.post_norm_residual(x32, f, self.norm2, eps, dt)
         return xa
 
 

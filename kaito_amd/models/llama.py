@@ -236,7 +236,10 @@ def _tp_fused_add_rms_norm(hidden, residual, weight, eps: float,
     interface.go:439-446). Falls back to the already-reduced plain fused
     norm when no group is active or the batch exceeds the staging
     window (the RowParallel layer makes the same `defer` decision, so
-    the paths always agree)."""
+    the paths always agree). Rows of experts (models/moe.py MoERows) are
+    summed on the way."""
+    if hasattr(hidden, "add_rms_norm"):
+        return hidden.add_rms_norm(residual, weight, eps)
     if deferred_producer and get_state().tp_size > 1:
         from ..parallel import one_shot
         grp = one_shot.defer(hidden.reshape(-1, hidden.shape[-1]).shape[0])
@@ -255,7 +258,8 @@ class LlamaDecoderLayer(nn.Module):
         else:
             self.self_attn = LlamaAttention(cfg, layer_idx)
         # deepseek: the first k layers are dense even in MoE models
-        if cfg.num_experts > 0 and layer_idx >= cfg.first_k_dense:
+        self.routed = cfg.num_experts > 0 and layer_idx >= cfg.first_k_dense
+        if self.routed:
             from .moe import MoEMLP
             self.mlp = MoEMLP(cfg)
         else:
@@ -284,7 +288,9 @@ class LlamaDecoderLayer(nn.Module):
         return ops.rms_norm(x, w, self.cfg.rms_eps)
 
     def forward(self, hidden, residual, positions, kv_cache, meta, cos_sin,
-                cos_sin_local=None):
+                cos_sin_local=None, defer: bool = False):
+        """defer: the first result may be MoERows, for the next layer's norm
+        (RMS norms, one rank)."""
         cfg = self.cfg
         if cfg.parallel_block:
             # phi-2/falcon: one shared norm; attn and mlp read the same
@@ -330,6 +336,10 @@ class LlamaDecoderLayer(nn.Module):
             hidden, residual = ops.fused_add_layer_norm(
                 hidden, residual, self.post_attention_layernorm,
                 self.post_attention_layernorm_bias, cfg.rms_eps)
+        elif defer and self.routed:
+            return self.mlp.forward_add_norm(
+                hidden, residual, self.post_attention_layernorm, cfg.rms_eps,
+                defer=True)
         else:
             hidden, residual = _tp_fused_add_rms_norm(
                 hidden, residual, self.post_attention_layernorm, cfg.rms_eps,
@@ -407,11 +417,17 @@ class LlamaForCausalLM(nn.Module):
             assert hidden_in is not None, "non-first PP stage needs hidden_in"
             hidden = hidden_in
             residual = None
+        cfg = self.cfg
+        # a layer's experts are summed by the norm behind it
+        defer = cfg.norm_type != "layernorm" and not cfg.parallel_block \
+            and not cfg.sandwich_norms and get_state().tp_size == 1
+        last = len(self.layers) - 1
         for i, layer in enumerate(self.layers):
             kv = kv_caches[i] if kv_caches is not None else None
             hidden, residual = layer(hidden, residual, positions, kv, meta,
                                      self.cos_sin_cache,
-                                     self.cos_sin_cache_local)
+                                     self.cos_sin_cache_local,
+                                     defer and (i < last or self.is_last))
         if self.is_last:
             if self.cfg.norm_type == "layernorm":
                 hidden, _ = ops.fused_add_layer_norm(

@@ -4,9 +4,9 @@ Replaces vLLM's fused-MoE CUDA path for the MoE presets in the reference
 catalog (gpt-oss-120b / Qwen MoE presets in
 supported_models.yaml).
 
-The GPU path needs no host read: two launches choose the experts and sort
-the (token, expert) pairs by expert (ops/csrc/moe_route.hip), grouped products
-gather the rows, apply the activation and go down again behind the device's
+The GPU path needs no host read: two launches choose the experts and, beyond
+decode sizes, sort the (token, expert) pairs by expert (ops/csrc/moe_route.hip),
+grouped products gather the rows, apply the activation and go down again behind the device's
 offsets (ops/csrc/moe.hip for decode-sized steps, moe_gemm.hip for prompts),
 and one launch sums every token's rows with their weights, the identity
 experts' share and the shared expert. Worst-case tile grids make every shape
@@ -27,6 +27,41 @@ import torch.nn as nn
 from .. import ops
 from ..engine.config import ModelConfig
 from ..parallel.state import get_state, tp_all_reduce
+
+
+class MoERows:
+    """A layer's output before its sum over the experts: whoever normalises
+    it next sums it in the same launch."""
+
+    def __init__(self, shape, dtype, *sum_args):
+        self.shape, self.dtype, self.sum_args = shape, dtype, sum_args
+
+    def tensor(self) -> torch.Tensor:
+        y = self.sum_args[0]
+        out = torch.empty(self.shape, device=y.device, dtype=self.dtype)
+        ops.moe_combine(out, *self.sum_args)
+        return out
+
+    def _fits(self, residual, weight) -> bool:
+        return self.dtype == torch.bfloat16 and self.shape[1] <= 8192 \
+            and residual.dtype == weight.dtype \
+            and all(t.is_contiguous() and t.data_ptr() % 16 == 0
+                    for t in (residual, weight))
+
+    def add_rms_norm(self, residual, weight, eps: float):
+        """ops.fused_add_rms_norm of it."""
+        if residual.dtype == torch.bfloat16 and self._fits(residual, weight):
+            return ops.moe_combine_norm(residual, weight, eps,
+                                        *self.sum_args), residual
+        return ops.fused_add_rms_norm(self.tensor(), residual, weight, eps)
+
+    def post_norm(self, x32, weight, eps: float, out_dtype):
+        """ops.post_norm_residual of it."""
+        if out_dtype == torch.bfloat16 and x32.dtype == torch.float32 \
+                and self._fits(x32, weight):
+            return ops.moe_combine_norm(x32, weight, eps, *self.sum_args)
+        return ops.post_norm_residual(x32, self.tensor(), weight, eps,
+                                      out_dtype)
 
 
 class MoEMLP(nn.Module):
@@ -117,9 +152,8 @@ class MoEMLP(nn.Module):
         else:
             self.w_shared_gate_up = None
 
-    def _choose(self, x: torch.Tensor):
-        """Top-k choice, device-only: (experts int32 [T, K], weights f32
-        [T, K], summed weight f32 [T] on identity experts)."""
+    def _choice(self):
+        """The router's arguments behind the rows it reads."""
         cfg = self.cfg
         bias, groups, keep = None, 1, 1
         renorm, scale = cfg.moe_norm_topk, cfg.routed_scaling_factor
@@ -145,9 +179,13 @@ class MoEMLP(nn.Module):
         if groups <= 1:             # no limit, whatever the number kept says
             groups = keep = 1
         # f32 router: x is widened before the product
-        return ops.moe_gate_route(x, self.gate, bias, self.top_k,
-                                  self.num_experts, groups, keep, renorm,
-                                  scale, mode)
+        return (self.gate, bias, self.top_k, self.num_experts, groups, keep,
+                renorm, scale, mode)
+
+    def _choose(self, x: torch.Tensor):
+        """Top-k choice, device-only: (experts int32 [T, K], weights f32
+        [T, K], summed weight f32 [T] on identity experts)."""
+        return ops.moe_gate_route(x, *self._choice())
 
     # Pairs up to which the weight-streaming kernels run, beyond it the tiled
     # grouped GEMMs: 16 rows per expert, 12 with many experts. A layer streamed
@@ -176,16 +214,31 @@ class MoEMLP(nn.Module):
             most = E * (12 if 32 < E <= 256 else 16)
         return "streamed" if TK <= most else "tiled"
 
+    def forward_add_norm(self, x, residual, weight, eps: float,
+                         defer: bool = False):
+        """fused_add_rms_norm(x, residual, weight), then forward of its rows:
+        (output, residual)."""
+        xn, residual, *chosen = ops.moe_norm_gate_route(
+            x, residual, weight, eps, *self._choice())
+        return self(xn, defer=defer, chosen=chosen), residual
+
     def forward(self, x: torch.Tensor, keep_f32: bool = False,
-                split_shared: bool = False):
+                split_shared: bool = False, defer: bool = False,
+                chosen=None):
         """keep_f32: the routed sum is returned as accumulated, in f32.
         split_shared: returns (routed sum, the shared expert's output or
-        None) for a caller that adds them itself."""
+        None) for a caller that adds them itself. defer: the output may be
+        MoERows. chosen: the result of _choose, if it is there already."""
         T, H = x.shape
-        topi, topw, w_id = self._choose(x)
-        # identity outputs sort behind every expert's rows
-        sorted_tok, gates, offsets, pos = ops.moe_plan(topi, topw,
-                                                       self.n_route)
+        topi, topw, w_id = chosen if chosen is not None else self._choose(x)
+        kernels = self._kernels_for(x)
+        # decode-sized steps: every expert finds its rows by itself
+        pairs = kernels == "streamed" and topi.numel() <= ops.PAIRS_MAX
+        pos = None
+        if not pairs:
+            # identity outputs sort behind every expert's rows
+            sorted_tok, gates, offsets, pos = ops.moe_plan(topi, topw,
+                                                           self.n_route)
         if not self.n_identity:
             w_id = None
         shared = None
@@ -194,7 +247,6 @@ class MoEMLP(nn.Module):
                 else ops.relu2(ops.linear(x, self.w_shared_gate_up))
             shared = ops.linear(h1, self.w_shared_down)
         added = None if split_shared else shared
-        kernels = self._kernels_for(x)
         if kernels == "loop":
             out = self._routed_start(x, w_id)
             self._forward_loop(x, sorted_tok, gates, offsets, out)
@@ -203,13 +255,19 @@ class MoEMLP(nn.Module):
             x = x.contiguous()
             if x.data_ptr() % 16:
                 x = x.clone()
-            y = self._rows_streamed(x, sorted_tok, offsets) \
-                if kernels == "streamed" \
-                else self._rows_tiled(x, sorted_tok, offsets)
-            out = torch.empty(T, H, device=x.device, dtype=torch.float32
-                              if keep_f32 else x.dtype)
-            ops.moe_combine(out, y, pos, topi, topw, self.e_base,
-                            self.e_local, x, w_id, added)
+            if pairs:
+                y = self._rows_pairs(x, topi)
+            elif kernels == "streamed":
+                y = self._rows_streamed(x, sorted_tok, offsets)
+            else:
+                y = self._rows_tiled(x, sorted_tok, offsets)
+            rows = MoERows((T, H), torch.float32 if keep_f32 else x.dtype, y,
+                           pos, topi, topw, self.e_base, self.e_local, x,
+                           w_id, added)
+            if defer and get_state().tp_size == 1:
+                assert not split_shared
+                return rows
+            out = rows.tensor()
             added = None
         if split_shared:
             assert get_state().tp_size == 1
@@ -226,8 +284,20 @@ class MoEMLP(nn.Module):
         return torch.zeros(x.shape, dtype=torch.float32, device=x.device) \
             if w_id is None else x * w_id[:, None]
 
-    # Both return the experts' outputs of the sorted rows, to be summed per
-    # token by moe_combine; static shapes, no host read.
+    # All return the experts' outputs of the sorted rows (or of the pairs), to be
+    # summed per token by moe_combine; static shapes, no host read.
+    def _rows_pairs(self, x, topi):
+        act = torch.empty(topi.numel(), self.ie_local, dtype=x.dtype,
+                          device=x.device)
+        ops.moe_up_pairs(act, x, self.w_gate_up, topi, self.n_route,
+                         self.e_base, self.e_local, self.b_gate_up,
+                         self.act_mode, self.act_limit)
+        y = torch.empty(topi.numel(), x.size(1), dtype=torch.float32,
+                        device=x.device)
+        ops.moe_down_pairs(y, act, self.w_down, topi, self.n_route,
+                           self.e_base, self.e_local, self.b_down)
+        return y
+
     def _rows_tiled(self, x, sorted_tok, offsets):
         TK, H = sorted_tok.numel(), x.size(1)
         act = torch.empty(TK, self.ie_local, dtype=x.dtype, device=x.device)

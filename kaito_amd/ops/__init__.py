@@ -30,9 +30,9 @@ for _g, _names in {
     "attn": ("paged_attention paged_attention_sp prefill_attention "
              "mla_prefill_attention context_attention mfma_tile_gemm paged_read_bw"),
     "mla": "mla_decode mla_prepare head_rows mla_cache_write",
-    "moe": ("moe_gate_silu moe_down_rows moe_grouped_up "
-            "moe_grouped_down moe_combine"),
-    "route": "moe_route moe_gate_route moe_sort",
+    "moe": ("moe_gate_silu moe_down_rows moe_up_pairs moe_down_pairs "
+            "moe_grouped_up moe_grouped_down moe_combine moe_combine_norm"),
+    "route": "moe_route moe_gate_route moe_norm_gate_route moe_sort",
     "quant": "w4a16_gemv w4a16_dequant w4a16_gemm lora_shrink lora_expand",
     "comm": ("allreduce_rmsnorm one_shot_ar_rmsnorm ipc_handle ipc_open "
              "ipc_close"),
@@ -500,6 +500,25 @@ def moe_down_rows(y, act, w_down, offsets, e_base: int, n_local_experts: int,
                      n_local_experts)
 
 
+PAIRS_MAX = 256       # pairs of a step whose experts find their own rows
+
+
+def moe_up_pairs(act, x, w_gate_up, topi, n_experts: int, e_base: int,
+                 n_local_experts: int, bias=None, act_mode: int = 0,
+                 act_limit: float = 7.0) -> None:
+    """moe_gate_silu with the rows of `act` in the order of the pairs of
+    `topi` [T, top] int32, up to PAIRS_MAX of them: no sort (GPU only)."""
+    _K.moe_up_pairs(act, x, w_gate_up, topi, _none(bias, x), act_mode,
+                    n_experts, e_base, n_local_experts, act_limit)
+
+
+def moe_down_pairs(y, act, w_down, topi, n_experts: int, e_base: int,
+                   n_local_experts: int, bias=None) -> None:
+    """moe_down_rows with rows in the order of the pairs (GPU only)."""
+    _K.moe_down_pairs(y, act, w_down, topi, _none(bias, act), n_experts,
+                      e_base, n_local_experts)
+
+
 def moe_grouped_up(act, x, w, sorted_ids, offsets, e_base: int, bias=None,
                    act_mode: int = 0, act_limit: float = 7.0) -> None:
     """moe_gate_silu for prompt-sized steps (GPU, bf16): `act` [TK, IE]
@@ -517,9 +536,25 @@ def moe_grouped_down(y, act, w, offsets, e_base: int, bias=None) -> None:
 def moe_combine(out, y, pos, topi, topw, e_base: int, e_local: int, x=None,
                 w_id=None, shared=None) -> None:
     """out[t] = sum over t's choices of topw * y[pos] (experts e_base ..
-    e_base + e_local) + w_id x + shared, summed in f32; out bf16 or f32."""
-    _K.moe_combine(out, y, pos, topi, topw, out if w_id is None else x,
-                   _none(w_id, y), _none(shared, y), e_base, e_local)
+    e_base + e_local) + w_id x + shared, summed in f32; out bf16 or f32. pos
+    None: rows of y in the order of the pairs."""
+    _K.moe_combine(out, y, _none(pos, y), topi, topw,
+                   out if w_id is None else x, _none(w_id, y),
+                   _none(shared, y), e_base, e_local)
+
+
+def moe_combine_norm(residual, weight, eps: float, y, pos, topi, topw,
+                     e_base: int, e_local: int, x=None, w_id=None,
+                     shared=None):
+    """moe_combine rounded to bf16, then (GPU, rows up to 8192) with a bf16
+    residual fused_add_rms_norm, with an f32 one post_norm_residual, in
+    place. Returns the bf16 rows of those."""
+    out = torch.empty(residual.shape, dtype=torch.bfloat16,
+                      device=residual.device)
+    _K.moe_combine_norm(out, residual, y, _none(pos, y), topi, topw,
+                        out if w_id is None else x, _none(w_id, y),
+                        _none(shared, y), weight, eps, e_base, e_local)
+    return out
 
 
 ROUTE_MAX = 1024      # router outputs of the kernels; more run as torch ops
@@ -566,6 +601,40 @@ def _router_logits(x: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
     return torch.nn.functional.linear(x.float(), gate.float())
 
 
+def _gate_in_route(x, gate) -> bool:
+    T = x.size(0)
+    return (x.is_cuda and x.dtype == torch.bfloat16 and T <= 512
+            and gate.size(0) <= 32 and T * gate.size(0) <= 8192
+            and gate.is_contiguous()
+            and gate.dtype in (torch.bfloat16, torch.float32)
+            and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and x.size(1) % 8 == 0 and x.data_ptr() % 16 == 0
+            and gate.data_ptr() % 16 == 0)
+
+
+def moe_norm_gate_route(x, residual, norm_w, eps: float, gate, correction,
+                        top: int, n_real: int, groups: int = 1, keep: int = 1,
+                        renorm: bool = False, scale: float = 1.0,
+                        mode: str = "softmax"):
+    """fused_add_rms_norm, then moe_gate_route of its rows: (rows, residual,
+    indices, weights, identity weight); one launch where the choice is."""
+    def aligned(t):
+        return t.dtype == torch.bfloat16 and t.is_contiguous() \
+            and t.data_ptr() % 16 == 0
+    if _gate_in_route(x, gate) and aligned(x) and aligned(residual) \
+            and aligned(norm_w) and residual.shape == x.shape \
+            and x.size(1) <= 8192:
+        topi, topw, w_id = _route_out(x.size(0), top, x.device)
+        xn = torch.empty_like(x)
+        _K.moe_norm_gate_route(topi, topw, w_id, xn, residual, x, norm_w, eps,
+                               gate, _none(correction, x), n_real, groups,
+                               keep, renorm, scale, ROUTE_MODES[mode])
+        return xn, residual, topi, topw, w_id
+    xn, residual = fused_add_rms_norm(x, residual, norm_w, eps)
+    return (xn, residual) + moe_gate_route(
+        xn, gate, correction, top, n_real, groups, keep, renorm, scale, mode)
+
+
 def moe_gate_route(x, gate, correction, top: int, n_real: int,
                    groups: int = 1, keep: int = 1, renorm: bool = False,
                    scale: float = 1.0, mode: str = "softmax"):
@@ -578,13 +647,7 @@ def moe_gate_route(x, gate, correction, top: int, n_real: int,
     13.7 at 256, 10.3, 9.7 and 16.0, 13.9 at 512; 48 outputs 12.0, 9.5 and
     16.5, 13.6 at 32)."""
     T = x.size(0)
-    if x.is_cuda and x.dtype == torch.bfloat16 and T <= 512 \
-            and gate.size(0) <= 32 and T * gate.size(0) <= 8192 \
-            and gate.is_contiguous() \
-            and gate.dtype in (torch.bfloat16, torch.float32) \
-            and x.stride(1) == 1 and x.stride(0) % 8 == 0 \
-            and x.size(1) % 8 == 0 and x.data_ptr() % 16 == 0 \
-            and gate.data_ptr() % 16 == 0:
+    if _gate_in_route(x, gate):
         topi, topw, w_id = _route_out(T, top, x.device)
         _K.moe_gate_route(topi, topw, w_id, x, gate, _none(correction, x),
                           n_real, groups, keep, renorm, scale,

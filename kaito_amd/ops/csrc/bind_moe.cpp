@@ -11,14 +11,25 @@ void moe_gate_silu(at::Tensor act, at::Tensor x, at::Tensor w_gate_up,
 void moe_down_rows(at::Tensor y, at::Tensor act, at::Tensor w_down,
                    at::Tensor offsets, at::Tensor bias, int64_t e_base,
                    int64_t n_local_experts);
+void moe_up_pairs(at::Tensor act, at::Tensor x, at::Tensor w_gate_up,
+                  at::Tensor topi, at::Tensor bias, int64_t act_mode,
+                  int64_t n_experts, int64_t e_base, int64_t n_local_experts,
+                  double act_limit);
+void moe_down_pairs(at::Tensor y, at::Tensor act, at::Tensor w_down,
+                    at::Tensor topi, at::Tensor bias, int64_t n_experts,
+                    int64_t e_base, int64_t n_local_experts);
 }  // namespace kaito
 
 TORCH_LIBRARY_FRAGMENT(kaito, m) {
   m.def("moe_gate_silu(Tensor(a!) act, Tensor x, Tensor w_gate_up, Tensor sorted_ids, Tensor offsets, Tensor bias, int act_mode, int e_base, int n_local_experts, float act_limit) -> ()");
   m.def("moe_down_rows(Tensor(a!) y, Tensor act, Tensor w_down, Tensor offsets, Tensor bias, int e_base, int n_local_experts) -> ()");
+  m.def("moe_up_pairs(Tensor(a!) act, Tensor x, Tensor w_gate_up, Tensor topi, Tensor bias, int act_mode, int n_experts, int e_base, int n_local_experts, float act_limit) -> ()");
+  m.def("moe_down_pairs(Tensor(a!) y, Tensor act, Tensor w_down, Tensor topi, Tensor bias, int n_experts, int e_base, int n_local_experts) -> ()");
 }
 
 TORCH_LIBRARY_IMPL(kaito, CUDA, m) {
   m.impl("moe_gate_silu", &kaito::moe_gate_silu);
   m.impl("moe_down_rows", &kaito::moe_down_rows);
+  m.impl("moe_up_pairs", &kaito::moe_up_pairs);
+  m.impl("moe_down_pairs", &kaito::moe_down_pairs);
 }

@@ -41,6 +41,9 @@ struct StreamArgs {
   const short* bias;                // [E local, rows] or nullptr
   const int* rows;                  // token of a sorted row
   const int* offsets;               // [global E + 1]
+  // or, in place of both, rows in the order of the pairs themselves:
+  const int* topi;                  // [pairs] expert of a pair
+  int pairs, top;                   // top pairs per token
   int e_base, N, K;
   int act_mode;
   float limit;
@@ -62,14 +65,50 @@ KAITO_DEV float moe_act_f(int mode, float g, float u, float limit) {
   return skinny::silu(g) * u;
 }
 
-// column n of rows m .. m + 3 below end: v, or gate v and up u
+// The rows begin .. end - 1 of an expert: sorted ones, or the pairs that chose it,
+// found by every wave for itself, 64 at a time, and listed in LDS. The sort's
+// launch is 4.3 us of a decode step's layer; the scan takes the place of the
+// loads of offsets and rows, one after the other.
+constexpr int PAIRS_MAX = 256;
+
+struct Rows {
+  int begin, end;
+  const unsigned short* list;       // or nullptr
+
+  // row of act and y
+  KAITO_DEV int at(const int m) const { return list ? list[m] : m; }
+};
+
+KAITO_DEV Rows rows_of(const StreamArgs& a, const int expert,
+                       unsigned short* list, const int lane) {
+  if (!a.topi) return {a.offsets[expert], a.offsets[expert + 1], nullptr};
+  int n = 0, e[PAIRS_MAX / 64];
+#pragma unroll
+  for (int i = 0; i < PAIRS_MAX / 64; i++) {
+    const int p = i * 64 + lane;
+    e[i] = p < a.pairs ? a.topi[p] : -1;
+  }
+#pragma unroll
+  for (int i = 0; i < PAIRS_MAX / 64; i++) {
+    if (i * 64 >= a.pairs) break;
+    const unsigned long long hit = __ballot(e[i] == expert);
+    if (e[i] == expert)
+      list[n + __builtin_popcountll(hit & ((1ull << lane) - 1))] =
+          i * 64 + lane;
+    n += __builtin_popcountll(hit);
+  }
+  __builtin_amdgcn_wave_barrier();
+  return {0, n, list};
+}
+
+// column n of rows m .. m + 3 below the end: v, or gate v and up u
 template <int KIND>
 KAITO_DEV void store_rows(const StreamArgs& a, const f32x4 v, const f32x4 u,
-                          const int m0, const int end, const int n) {
+                          const int m0, const Rows& rows, const int n) {
 #pragma unroll
   for (int r = 0; r < 4; r++) {
-    const int m = m0 + r;
-    if (m >= end) break;
+    if (m0 + r >= rows.end) break;
+    const int m = rows.at(m0 + r);
     if constexpr (KIND == UP_GATED) {
       a.act[(int64_t)m * a.N + n] =
           f32_to_bf16(moe_act_f(a.act_mode, v[r], u[r], a.limit));
@@ -82,17 +121,28 @@ KAITO_DEV void store_rows(const StreamArgs& a, const f32x4 v, const f32x4 u,
   }
 }
 
+// x of row m, the last one's past the end
+template <int KIND>
+KAITO_DEV const short* x_row(const StreamArgs& a, const Rows& rows,
+                             const int m) {
+  const int r = rows.at(min(m, rows.end - 1));
+  const int64_t row = KIND == DOWN ? r : rows.list ? r / a.top : a.rows[r];
+  return a.x + row * a.K;
+}
+
 template <int MT, int KS, int KIND>
 __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const StreamArgs a) {
   constexpr int NI = skinny::tile_loads<KS>();
   constexpr bool GATED = KIND == UP_GATED;
   __shared__ __attribute__((aligned(128))) short ring[4][2][16 * KS];
   static_assert(sizeof(ring) >= 4 * MT * 64 * sizeof(f32x4), "fold");
+  __shared__ unsigned short list[4][PAIRS_MAX];
   const int le = blockIdx.y;
-  const int begin = a.offsets[a.e_base + le], end = a.offsets[a.e_base + le + 1];
-  if (begin >= end) return;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const Rows rows = rows_of(a, a.e_base + le, list[wave], lane);
+  const int begin = rows.begin, end = rows.end;
+  if (begin >= end) return;
   const int n0 = blockIdx.x * (GATED ? 8 : 16);
   const int64_t wrows = GATED ? 2 * a.N : a.N;
   const short* src[NI];
@@ -110,9 +160,8 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const StreamArgs a) 
     const short* xp[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
-      const int m = min(m0 + mt * 16 + (lane & 15), end - 1);
-      const int64_t row = KIND == DOWN ? m : a.rows[m];
-      xp[mt] = a.x + row * a.K + (lane >> 4) * 8;
+      xp[mt] = x_row<KIND>(a, rows, m0 + mt * 16 + (lane & 15)) +
+          (lane >> 4) * 8;
     }
     f32x4 acc[MT];
 #pragma unroll
@@ -130,7 +179,7 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const StreamArgs a) 
         v += bf16_to_f32(be[0]);
         if constexpr (GATED) u += bf16_to_f32(be[a.N]);
       }
-      store_rows<KIND>(a, v, u, m0 + (slot >> 6) * 16 + (l >> 4) * 4, end,
+      store_rows<KIND>(a, v, u, m0 + (slot >> 6) * 16 + (l >> 4) * 4, rows,
                        n0 + c);
     }
     __syncthreads();                // sums read before the next pass's stages
@@ -141,7 +190,7 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const StreamArgs a) 
 // ntiles tiles; MT row tiles of 16 in a pass.
 template <int MT, int S, int KIND>
 KAITO_DEV void stream_pass(const StreamArgs& a, const int le, const int ntiles,
-                           const int m0, const int end, short* ring,
+                           const int m0, const Rows& rows, short* ring,
                            f32x4* red, const int wave, const int lane) {
   constexpr int KS = skinny::TILES_KS, NW = skinny::TILE_NW;
   constexpr bool GATED = KIND == UP_GATED;
@@ -159,11 +208,9 @@ KAITO_DEV void stream_pass(const StreamArgs& a, const int le, const int ntiles,
       COLS * a.K * 2, blockIdx.x, gridDim.x, ntiles,
       [&](const short* (&xp)[MT]) {
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-          const int m = min(m0 + mt * 16 + (lane & 15), end - 1);
-          const int64_t row = KIND == DOWN ? m : a.rows[m];
-          xp[mt] = a.x + row * a.K + (lane >> 4) * 8;
-        }
+        for (int mt = 0; mt < MT; mt++)
+          xp[mt] = x_row<KIND>(a, rows, m0 + mt * 16 + (lane & 15)) +
+              (lane >> 4) * 8;
       },
       ring, red, wave, lane,
       [&](const int t, const f32x4* sums) {
@@ -176,7 +223,7 @@ KAITO_DEV void stream_pass(const StreamArgs& a, const int le, const int ntiles,
           v += bf16_to_f32(be[0]);
           if constexpr (GATED) u += bf16_to_f32(be[a.N]);
         }
-        store_rows<KIND>(a, v, u, m0 + (slot >> 6) * 16 + (l >> 4) * 4, end,
+        store_rows<KIND>(a, v, u, m0 + (slot >> 6) * 16 + (l >> 4) * 4, rows,
                          n);
       });
   __syncthreads();                  // sums read before the next pass's
@@ -190,16 +237,17 @@ __global__ __launch_bounds__(256, 2) void moe_tiles_kernel(const StreamArgs a,
   __shared__ f32x4 red[2][NW][2 * 64];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  __shared__ unsigned short list[NW][PAIRS_MAX];
   const int le = blockIdx.y;
-  const int begin = a.offsets[a.e_base + le], end = a.offsets[a.e_base + le + 1];
+  const Rows rows = rows_of(a, a.e_base + le, list[wave], lane);
   // An expert that many tokens share would hold up its workgroups for a second
   // pass: as many row tiles as it has.
-  for (int m0 = begin; m0 < end; m0 += 32) {
-    if (end - m0 > 16)
-      stream_pass<2, S, KIND>(a, le, ntiles, m0, end, ring[wave][0],
+  for (int m0 = rows.begin; m0 < rows.end; m0 += 32) {
+    if (rows.end - m0 > 16)
+      stream_pass<2, S, KIND>(a, le, ntiles, m0, rows, ring[wave][0],
                               &red[0][0][0], wave, lane);
     else
-      stream_pass<1, S, KIND>(a, le, ntiles, m0, end, ring[wave][0],
+      stream_pass<1, S, KIND>(a, le, ntiles, m0, rows, ring[wave][0],
                               &red[0][0][0], wave, lane);
   }
 }
@@ -253,68 +301,122 @@ void check16(const at::Tensor& t) {
 
 }  // namespace
 
-void moe_gate_silu(at::Tensor act, at::Tensor x, at::Tensor w_gate_up,
-                   at::Tensor sorted_ids, at::Tensor offsets,
-                   at::Tensor bias, int64_t act_mode,
-                   int64_t e_base, int64_t n_local_experts,
-                   double act_limit) {
+namespace {
+
+// rows of `act`/`y` by sorted rows (offsets, ids) or by pairs (topi [T, top])
+struct RowArgs {
+  at::Tensor offsets, ids, topi;
+  int64_t pairs, E;                 // of all experts
+};
+
+void set_rows(StreamArgs& a, const RowArgs& r, int64_t e_base, int64_t n_local,
+              const at::Tensor& w) {
+  TORCH_CHECK(e_base >= 0 && n_local >= 0 && w.size(0) >= n_local);
+  a.e_base = (int)e_base;
+  if (r.topi.defined()) {
+    TORCH_CHECK(r.topi.is_cuda() && r.topi.is_contiguous() &&
+                r.topi.dim() == 2 && r.topi.dtype() == at::kInt &&
+                r.pairs <= PAIRS_MAX);
+    a.topi = r.topi.data_ptr<int>();
+    a.pairs = (int)r.pairs;
+    a.top = (int)r.topi.size(1);
+  } else {
+    TORCH_CHECK(r.offsets.dtype() == at::kInt &&
+                r.offsets.numel() > e_base + n_local);
+    a.offsets = r.offsets.data_ptr<int>();
+    if (r.ids.defined()) {
+      TORCH_CHECK(r.ids.dtype() == at::kInt);
+      a.rows = r.ids.data_ptr<int>();
+    }
+  }
+}
+
+void up_rows(at::Tensor& act, const at::Tensor& x, const at::Tensor& w_gate_up,
+             const RowArgs& rows, const at::Tensor& bias, int64_t act_mode,
+             int64_t e_base, int64_t n_local, double act_limit) {
   check16(act); check16(x); check16(w_gate_up);
-  TORCH_CHECK(sorted_ids.dtype() == at::kInt && offsets.dtype() == at::kInt);
   const bool gated = act_mode != 2;
   StreamArgs a{};
   a.N = act.size(1); a.K = x.size(1);
   TORCH_CHECK(a.K % 64 == 0 && a.N % 64 == 0,
               "H/IE must be multiples of 64 for the fused MoE path");
   TORCH_CHECK(w_gate_up.size(1) == (gated ? 2 : 1) * (int64_t)a.N &&
-              w_gate_up.size(2) == a.K &&
-              w_gate_up.size(0) >= n_local_experts &&
-              offsets.numel() > e_base + n_local_experts &&
-              act.size(0) >= sorted_ids.numel());
+              w_gate_up.size(2) == a.K && act.size(0) >= rows.pairs);
   if (bias.numel() > 0) {
     TORCH_CHECK(bias.dtype() == at::kBFloat16 && bias.is_contiguous() &&
                 bias.numel() == w_gate_up.size(0) * 2 * a.N);
     a.bias = (const short*)bias.data_ptr();
   }
   TORCH_CHECK(gated || a.bias == nullptr, "ungated experts take no bias");
-  if (sorted_ids.numel() == 0 || n_local_experts == 0 || a.N == 0) return;
+  set_rows(a, rows, e_base, n_local, w_gate_up);
+  if (rows.pairs == 0 || n_local == 0 || a.N == 0) return;
   a.x = (const short*)x.data_ptr();
   a.w = (const short*)w_gate_up.data_ptr();
-  a.rows = sorted_ids.data_ptr<int>();
-  a.offsets = offsets.data_ptr<int>();
-  a.e_base = (int)e_base;
   a.act_mode = (int)act_mode;
   a.limit = (float)act_limit;
   a.act = (short*)act.data_ptr();
-  const int64_t pairs = sorted_ids.numel(), E = offsets.numel() - 1;
-  if (gated) launch_stream<UP_GATED>(a, n_local_experts, pairs, E);
-  else launch_stream<UP_PLAIN>(a, n_local_experts, pairs, E);
+  if (gated) launch_stream<UP_GATED>(a, n_local, rows.pairs, rows.E);
+  else launch_stream<UP_PLAIN>(a, n_local, rows.pairs, rows.E);
 }
 
-void moe_down_rows(at::Tensor y, at::Tensor act, at::Tensor w_down,
-                   at::Tensor offsets, at::Tensor bias, int64_t e_base,
-                   int64_t n_local_experts) {
-  TORCH_CHECK(y.is_cuda() && y.dtype() == at::kFloat && y.is_contiguous() &&
-              offsets.dtype() == at::kInt);
+void down_rows(at::Tensor& y, const at::Tensor& act, const at::Tensor& w_down,
+               const RowArgs& rows, const at::Tensor& bias, int64_t e_base,
+               int64_t n_local) {
+  TORCH_CHECK(y.is_cuda() && y.dtype() == at::kFloat && y.is_contiguous());
   check16(act); check16(w_down);
   StreamArgs a{};
   a.N = y.size(1); a.K = act.size(1);
   TORCH_CHECK(a.N % 64 == 0 && a.K % 64 == 0);
   TORCH_CHECK(w_down.size(1) == a.N && w_down.size(2) == a.K &&
-              w_down.size(0) >= n_local_experts &&
-              offsets.numel() > e_base + n_local_experts &&
               act.size(0) >= y.size(0));
   if (bias.numel() > 0) {
     TORCH_CHECK(bias.dtype() == at::kBFloat16 && bias.is_contiguous() &&
                 bias.numel() == w_down.size(0) * a.N);
     a.bias = (const short*)bias.data_ptr();
   }
-  if (y.size(0) == 0 || n_local_experts == 0 || a.N == 0) return;
+  set_rows(a, rows, e_base, n_local, w_down);
+  if (y.size(0) == 0 || n_local == 0 || a.N == 0) return;
   a.x = (const short*)act.data_ptr();
   a.w = (const short*)w_down.data_ptr();
-  a.offsets = offsets.data_ptr<int>();
-  a.e_base = (int)e_base;
   a.y = y.data_ptr<float>();
-  launch_stream<DOWN>(a, n_local_experts, y.size(0), offsets.numel() - 1);
+  launch_stream<DOWN>(a, n_local, rows.pairs, rows.E);
+}
+
+}  // namespace
+
+void moe_gate_silu(at::Tensor act, at::Tensor x, at::Tensor w_gate_up,
+                   at::Tensor sorted_ids, at::Tensor offsets,
+                   at::Tensor bias, int64_t act_mode,
+                   int64_t e_base, int64_t n_local_experts,
+                   double act_limit) {
+  up_rows(act, x, w_gate_up,
+          {offsets, sorted_ids, {}, sorted_ids.numel(), offsets.numel() - 1},
+          bias, act_mode, e_base, n_local_experts, act_limit);
+}
+
+void moe_down_rows(at::Tensor y, at::Tensor act, at::Tensor w_down,
+                   at::Tensor offsets, at::Tensor bias, int64_t e_base,
+                   int64_t n_local_experts) {
+  down_rows(y, act, w_down,
+            {offsets, {}, {}, y.size(0), offsets.numel() - 1}, bias, e_base,
+            n_local_experts);
+}
+
+void moe_up_pairs(at::Tensor act, at::Tensor x, at::Tensor w_gate_up,
+                  at::Tensor topi, at::Tensor bias, int64_t act_mode,
+                  int64_t n_experts, int64_t e_base, int64_t n_local_experts,
+                  double act_limit) {
+  TORCH_CHECK(x.size(0) == topi.size(0));
+  up_rows(act, x, w_gate_up, {{}, {}, topi, topi.numel(), n_experts}, bias,
+          act_mode, e_base, n_local_experts, act_limit);
+}
+
+void moe_down_pairs(at::Tensor y, at::Tensor act, at::Tensor w_down,
+                    at::Tensor topi, at::Tensor bias, int64_t n_experts,
+                    int64_t e_base, int64_t n_local_experts) {
+  TORCH_CHECK(y.size(0) == topi.numel());
+  down_rows(y, act, w_down, {{}, {}, topi, topi.numel(), n_experts}, bias,
+            e_base, n_local_experts);
 }
 
 }  // namespace kaito

@@ -251,6 +251,77 @@ __global__ __launch_bounds__(256) void moe_gate_route_kernel(
   route_row<1, MODE>(a, part[0], t, lane);
 }
 
+// The residual norm ahead of the router in the same launch: residual += x, xn =
+// rms(residual) * w, logits of xn as rounded to bf16. A thread keeps its 8 * ITER
+// elements. 32 rows of 2048 with 8 outputs: 4.6 + 5.3 us -> 5.7.
+template <int MODE, typename W, int ITER>
+__global__ __launch_bounds__(256) void moe_norm_gate_route_kernel(
+    const RouteArgs a, short* __restrict__ xn, short* __restrict__ residual,
+    const short* __restrict__ x, const short* __restrict__ nw,
+    const float eps, const W* __restrict__ w, const int H) {
+  __shared__ float part[4][GATE_MAX], red[4];
+  const int64_t t = blockIdx.x;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  short8_t v[ITER], g[ITER];
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < ITER; i++) {
+    const int k = i * 2048 + threadIdx.x * 8;
+    if (k >= H) break;
+    const short8_t xv = *reinterpret_cast<const short8_t*>(x + t * H + k);
+    const short8_t rv =
+        *reinterpret_cast<const short8_t*>(residual + t * H + k);
+    g[i] = *reinterpret_cast<const short8_t*>(nw + k);
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      v[i][e] = f32_to_bf16(bf16_to_f32(xv[e]) + bf16_to_f32(rv[e]));
+      const float f = bf16_to_f32(v[i][e]);
+      ss += f * f;
+    }
+    *reinterpret_cast<short8_t*>(residual + t * H + k) = v[i];
+  }
+  ss = wave_reduce_sum(ss);
+  if (lane == 0) red[wave] = ss;
+  __syncthreads();
+  ss = (red[0] + red[1]) + (red[2] + red[3]);
+  const float inv = rsqrtf(ss / (float)H + eps);
+#pragma unroll
+  for (int i = 0; i < ITER; i++) {
+    const int k = i * 2048 + threadIdx.x * 8;
+    if (k >= H) break;
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+      v[i][e] = f32_to_bf16(bf16_to_f32(v[i][e]) * inv * bf16_to_f32(g[i][e]));
+    *reinterpret_cast<short8_t*>(xn + t * H + k) = v[i];
+  }
+  for (int e0 = 0; e0 < a.N; e0 += 8) {
+    float acc[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) acc[i] = 0.f;
+#pragma unroll
+    for (int j = 0; j < ITER; j++) {
+      const int k = j * 2048 + threadIdx.x * 8;
+      if (k >= H) break;
+      const auto xv = __builtin_bit_cast(skinny::hbf16x8, v[j]);
+#pragma unroll
+      for (int i = 0; i < 8; i++)
+        acc[i] = dot_gate(xv, w + (int64_t)min(e0 + i, a.N - 1) * H + k,
+                          acc[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      acc[i] = wave_reduce_sum(acc[i]);
+      if (lane == 0 && e0 + i < a.N) part[wave][e0 + i] = acc[i];
+    }
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  if (lane < a.N)
+    part[0][lane] += part[1][lane] + part[2][lane] + part[3][lane];
+  __builtin_amdgcn_wave_barrier();
+  route_row<1, MODE>(a, part[0], t, lane);
+}
+
 // lanes of the wave with this lane's expert e (< 2^bits; any lane with -1 is
 // in no group): a ballot per bit, however many experts there are
 KAITO_DEV unsigned long long same_expert(const int e, const int bits) {
@@ -448,6 +519,48 @@ void moe_gate_route(at::Tensor topi, at::Tensor topw, at::Tensor w_id,
   });
 }
 
+void moe_norm_gate_route(at::Tensor topi, at::Tensor topw, at::Tensor w_id,
+                         at::Tensor xn, at::Tensor residual, at::Tensor x,
+                         at::Tensor norm_w, double eps, at::Tensor gate,
+                         at::Tensor correction, int64_t n_real, int64_t groups,
+                         int64_t keep, bool renorm, double scale,
+                         int64_t mode) {
+  for (const auto& t : {xn, residual, x, norm_w})
+    TORCH_CHECK(t.is_cuda() && t.dtype() == at::kBFloat16 &&
+                t.is_contiguous() && (uintptr_t)t.data_ptr() % 16 == 0);
+  TORCH_CHECK(x.dim() == 2 && xn.sizes() == x.sizes() &&
+              residual.sizes() == x.sizes() && norm_w.numel() == x.size(1));
+  TORCH_CHECK(gate.is_cuda() && gate.dim() == 2 && gate.is_contiguous() &&
+              gate.size(1) == x.size(1) && x.size(1) % 8 == 0 &&
+              (uintptr_t)gate.data_ptr() % 16 == 0);
+  const int T = x.size(0), N = gate.size(0), H = x.size(1);
+  TORCH_CHECK(N <= GATE_MAX && H <= 8192);
+  const RouteArgs a = route_args(topi, topw, w_id, correction, T, N, n_real,
+                                 groups, keep, renorm, scale, mode);
+  if (T == 0) return;
+  const bool f32 = gate.dtype() == at::kFloat;
+  TORCH_CHECK(f32 || gate.dtype() == at::kBFloat16);
+  auto stream = at::hip::getCurrentHIPStream();
+  with_mode(mode, [&](auto md) {
+    auto launch = [&](auto it, auto wt) {
+      using W = decltype(wt);
+      hipLaunchKernelGGL(
+          (moe_norm_gate_route_kernel<decltype(md)::value, W,
+                                      decltype(it)::value>),
+          dim3(T), dim3(256), 0, stream, a, (short*)xn.data_ptr(),
+          (short*)residual.data_ptr(), (const short*)x.data_ptr(),
+          (const short*)norm_w.data_ptr(), (float)eps,
+          (const W*)gate.data_ptr(), H);
+    };
+    auto sized = [&](auto wt) {
+      if (H <= 2048) launch(std::integral_constant<int, 1>{}, wt);
+      else if (H <= 4096) launch(std::integral_constant<int, 2>{}, wt);
+      else launch(std::integral_constant<int, 4>{}, wt);
+    };
+    if (f32) sized(0.f); else sized((short)0);
+  });
+}
+
 void moe_sort(at::Tensor sorted_tok, at::Tensor gates, at::Tensor offsets,
               at::Tensor pos, at::Tensor topi, at::Tensor topw) {
   KAITO_CHECK_I32(topi); KAITO_CHECK_F32(topw); KAITO_CHECK_I32(pos);
@@ -484,10 +597,12 @@ void moe_sort(at::Tensor sorted_tok, at::Tensor gates, at::Tensor offsets,
 TORCH_LIBRARY_FRAGMENT(kaito, m) {
   m.def("moe_route(Tensor(a!) topi, Tensor(b!) topw, Tensor(c!) w_id, Tensor logits, Tensor correction, int n_real, int groups, int keep, bool renorm, float scale, int mode) -> ()");
   m.def("moe_gate_route(Tensor(a!) topi, Tensor(b!) topw, Tensor(c!) w_id, Tensor x, Tensor gate, Tensor correction, int n_real, int groups, int keep, bool renorm, float scale, int mode) -> ()");
+  m.def("moe_norm_gate_route(Tensor(a!) topi, Tensor(b!) topw, Tensor(c!) w_id, Tensor(d!) xn, Tensor(e!) residual, Tensor x, Tensor norm_w, float eps, Tensor gate, Tensor correction, int n_real, int groups, int keep, bool renorm, float scale, int mode) -> ()");
   m.def("moe_sort(Tensor(a!) sorted_tok, Tensor(b!) gates, Tensor(c!) offsets, Tensor(d!) pos, Tensor topi, Tensor topw) -> ()");
 }
 TORCH_LIBRARY_IMPL(kaito, CUDA, m) {
   m.impl("moe_route", &kaito::moe_route);
   m.impl("moe_gate_route", &kaito::moe_gate_route);
+  m.impl("moe_norm_gate_route", &kaito::moe_norm_gate_route);
   m.impl("moe_sort", &kaito::moe_sort);
 }

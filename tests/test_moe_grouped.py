@@ -166,3 +166,92 @@ def test_several_choices_sum():
     live = ((topi >= 2) & (topi < 7)).double() * topw.double()
     ref = (y[pos.long()].view(T, K, H).double() * live[..., None]).sum(1)
     assert torch.allclose(out.double(), ref, atol=1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,E,top,H,IE,mode,ident,part", [
+    (1, 4, 1, 64, 64, 0, 0, None),
+    (33, 5, 3, 256, 128, 1, 0, (1, 3)),
+    (64, 9, 4, 128, 192, 2, 2, None),           # 256 pairs, identity experts
+    (32, 8, 2, 2048, 2048, 0, 0, None),         # workgroups that stay
+    (100, 8, 2, 2048, 1536, 0, 1, (2, 6)),
+])
+def test_rows_of_pairs(T, E, top, H, IE, mode, ident, part):
+    """Experts that find their own rows write what sorted ones hold."""
+    torch.manual_seed(T + E)
+    lo, n = part or (0, E)
+    topi = torch.stack([torch.randperm(E + ident, device=DEV)[:top]
+                        for _ in range(T)]).int()
+    topw = torch.rand(T, top, device=DEV)
+    x = _rand(T, H)
+    wu = _rand(n, (1 if mode == 2 else 2) * IE, H, std=H ** -0.5)
+    wd = _rand(n, H, IE, std=IE ** -0.5)
+    bd = _rand(n, H)
+    tok, _, off, pos = ops.moe_plan(topi, topw, E + ident)
+    act = torch.zeros(T * top, IE, device=DEV, dtype=torch.bfloat16)
+    y = torch.zeros(T * top, H, device=DEV)
+    act2, y2 = act.clone(), y.clone()
+    ops.moe_gate_silu(act, x, wu, tok, off, lo, n, None, mode)
+    ops.moe_down_rows(y, act, wd, off, lo, n, bd)
+    ops.moe_up_pairs(act2, x, wu, topi, E + ident, lo, n, None, mode)
+    ops.moe_down_pairs(y2, act2, wd, topi, E + ident, lo, n, bd)
+    assert torch.equal(act2, act[pos.long()])
+    assert torch.equal(y2, y[pos.long()])
+    a, b = (torch.empty(T, H, device=DEV) for _ in range(2))
+    w_id = torch.rand(T, device=DEV)
+    ops.moe_combine(a, y, pos, topi, topw, lo, n, x, w_id, x)
+    ops.moe_combine(b, y2, None, topi, topw, lo, n, x, w_id, x)
+    assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,H", [(1, 8), (3, 2048), (5, 2056), (2, 4104),
+                                 (2, 8192)])
+@pytest.mark.parametrize("wide", [True, False])
+@pytest.mark.parametrize("post", [True, False])
+def test_sum_and_norm(T, H, wide, post):
+    """The sum over the experts inside the residual norm behind it."""
+    torch.manual_seed(H)
+    topi = torch.randint(0, 4, (T, 2), device=DEV).int()
+    topw = torch.rand(T, 2, device=DEV)
+    y = torch.randn(2 * T, H, device=DEV)
+    y = y if wide else y.to(torch.bfloat16)
+    shared = _rand(T, H)
+    args = (y, None, topi, topw, 1, 3, None, None, shared)
+    s = torch.empty(T, H, device=DEV, dtype=torch.bfloat16)
+    ops.moe_combine(s, *args)
+    if post:
+        res, w = torch.randn(T, H, device=DEV), torch.rand(H, device=DEV)
+        r2 = res.clone()
+        ref = ops.post_norm_residual(res, s, w, 1e-5, torch.bfloat16)
+    else:
+        res, w = _rand(T, H), _rand(H)
+        r2 = res.clone()
+        ref, res = ops.fused_add_rms_norm(s, res, w, 1e-5)
+    out = ops.moe_combine_norm(r2, w, 1e-5, *args)
+    # sums of squares in another order: 2^-20 of the factor, then one rounding
+    assert ((r2 - res).abs() <= 2.0 ** -20 * (1 + res.abs())).all() if post \
+        else torch.equal(r2, res)
+    assert ((out.float() - ref.float()).abs()
+            <= 2.0 ** -7 * ref.float().abs()).all()
+    assert (out != ref).float().mean() < 0.02
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,H,N,f32", [(1, 8, 2, False), (32, 2048, 8, False),
+                                       (3, 2056, 32, True),
+                                       (300, 8192, 20, False)])
+def test_norm_and_choice(T, H, N, f32):
+    """The residual norm inside the router's launch."""
+    torch.manual_seed(H + N)
+    x, res, w = _rand(T, H), _rand(T, H), _rand(H)
+    gate = torch.randn(N, H, device=DEV).to(torch.float32 if f32
+                                            else torch.bfloat16)
+    ref, r1 = ops.fused_add_rms_norm(x, res.clone(), w, 1e-5)
+    xn, r2, *chosen = ops.moe_norm_gate_route(x, res, w, 1e-5, gate, None, 2, N)
+    assert torch.equal(r1, r2)
+    assert ((xn.float() - ref.float()).abs()
+            <= 2.0 ** -7 * ref.float().abs()).all()
+    assert (xn != ref).float().mean() < 0.02
+    for a, b in zip(chosen, ops.moe_gate_route(xn, gate, None, 2, N)):
+        assert torch.equal(a, b)
