@@ -169,11 +169,12 @@ def _skinny(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
     7168 (2112 x 7168: 12.7, 12.6; 2048 x 8192: 14.6, 13.1); SwiGLU pairs,
     which save a launch, to 8192 (28672 x 4096: 50.3, 60.5), uneven ones
     excepted (5120 x 5120: 19.1, 17.9).
-    Many rows of W whose x fits the registers, K of 2048 up to 32 rows and of
-    4096 up to 16, always (12288 x 2048: 13.6, 16.6 at 16, 15.9, 16.9 at 32;
-    32000 x 2048 29.7, 31.8 at 32; 128256 x 4096 168, 186 at 16).
-    Up to 32: to 3072 x 2048 (7.4, 11.5; 6144 x 2048: 13.0, 12.6, as a pair
-    12.5, 15.0) and K of 4096 (1024 x 4096: 10.1, 11.3 at 24), where beyond 24
+    K of 2048, where x fits the registers, always (7168 x 2048: 10.5, 13.9 at
+    16; 12288 13.6, 16.6; at 32 4096 x 2048: 8.9, 11.9; 5152 11.4, 12.6; 8192
+    12.8, 14.0; 12288 15.9, 16.9; 32000 29.7, 31.8), and K of 4096 with many
+    rows of W up to 16 (128256 x 4096 168, 186).
+    Up to 32: to 3072 x 2048 (7.4, 11.5; as a pair to 6144 x 2048 12.5, 15.0)
+    and K of 4096 (1024 x 4096: 10.1, 11.3 at 24), where beyond 24
     rows the library has another kernel for few rows of W and K of 2560 and
     more (1024 x 2560: 8.0, 6.9; 2048 x 2816: 8.8, 9.5; 1024 x 2816 as a pair
     9.0, 9.5)."""
@@ -193,8 +194,8 @@ def _skinny(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
     if K % 64 or N % 16:
         return False
     # x stays in registers while W streams
-    if N >= 12288 and N * K < 1 << 31 and (
-            K == 2048 or (K == 4096 and M <= 16)):
+    if N * K < 1 << 31 and (
+            K == 2048 or (K == 4096 and M <= 16 and N >= 12288)):
         return True
     if M <= 16 and N < 1024 and K > 5120 and not glu:
         return False

@@ -166,11 +166,15 @@ bool in_tiles(int64_t M, int64_t N, int64_t K, int64_t cols, int64_t weights) {
 // 8.9 and 9.2, 512 of a pair 8.9 and 9.5, 768 13.1 and 12.6 at M = 5, 15.5 and
 // 13.6 at 16, 19.4 and 15.9 at 32, 2000 44.1 and 29.6 at 32; 4096 columns: 384
 // 13.8 and 14.0, 1792 of a pair 40.2 and 39.3 at 5, 48.5 and 41.8 at 16, 8016
-// 209 and 168 at 16). Two workgroups per CU are no faster (1792 of a pair 42.8).
+// 209 and 168 at 16). Beyond 16 rows, whose x costs twice as much to bring, as
+// soon as a tile per CU is not enough (M = 32: 256 tiles 8.9 and 9.6, 322 13.3
+// and 11.4, 384 13.6 and 11.9, 512 14.5 and 12.8; M = 17: 322 11.0 and 10.4). Two
+// workgroups per CU are no faster (1792 of a pair 42.8).
 constexpr int WORKGROUPS = 256;
 
 bool many_tiles(int M, int64_t tiles, const at::Tensor& w) {
-  return tiles >= 3 * WORKGROUPS && w.numel() < (1ll << 31) &&
+  return tiles >= (M > 16 ? WORKGROUPS + 64 : 3 * WORKGROUPS) &&
+         w.numel() < (1ll << 31) &&
          (w.size(1) == 2048 || (w.size(1) == 4096 && M <= 16));
 }
 

@@ -59,9 +59,9 @@ def test_tiles(M, N, K):
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [3, 5, 16, 17, 32])
 @pytest.mark.parametrize("N,K", [(6144, 2048), (6168, 2048), (6144, 4096),
-                                 (7336, 4096)])
+                                 (7336, 4096), (2560, 2048), (2568, 2048)])
 def test_staying_workgroups(M, N, K):
-    """Tiles that workgroups share evenly or not."""
+    """Tiles that workgroups share evenly or not, just enough of them."""
     if M > 16 and K == 4096:
         pytest.skip("the library's")
     test_tiles(M, N, K)
