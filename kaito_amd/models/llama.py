@@ -221,6 +221,10 @@ class LlamaMLP(nn.Module):
         p = self.gate_up_proj
         if self.cfg.hidden_act != "gelu_tanh" and p.is_plain():
             return self.down_proj(ops.linear_swiglu(x, p.weight))
+        if self.cfg.hidden_act != "gelu_tanh":
+            act = p.quantized_swiglu(x)
+            if act is not None:
+                return self.down_proj(act)
         gu = p(x)
         act = ops.gelu_and_mul(gu) if self.cfg.hidden_act == "gelu_tanh" \
             else ops.silu_and_mul(gu)

@@ -33,7 +33,8 @@ for _g, _names in {
     "moe": ("moe_gate_silu moe_down_rows moe_up_pairs moe_down_pairs "
             "moe_grouped_up moe_grouped_down moe_combine moe_combine_norm"),
     "route": "moe_route moe_gate_route moe_norm_gate_route moe_sort",
-    "quant": "w4a16_gemv w4a16_dequant w4a16_gemm lora_shrink lora_expand",
+    "quant": ("w4a16_gemv w4a16_dequant w4a16_gemm w4a16_swiglu "
+              "w4a16_swiglu_fits lora_shrink lora_expand"),
     "comm": ("allreduce_rmsnorm one_shot_ar_rmsnorm ipc_handle ipc_open "
              "ipc_close"),
     "mix": ("causal_conv_update "
@@ -689,6 +690,21 @@ def w4a16_gemv(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor,
         _K.w4a16_gemv(out, x, qweight, scales, zeros, group)
         return out
     return torch_ref.w4a16_gemv(x, qweight, scales, zeros, group)
+
+
+def w4a16_swiglu(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor,
+                 zeros: torch.Tensor, group: int):
+    """silu(x Wg^T) * (x Wu^T) of the packed W = [Wg | Wu] in one launch, for
+    a few rows x [M, K]; None for other sizes."""
+    N, K = qweight.size(0) // 2, x.size(1)
+    if not (x.is_cuda and x.dtype == torch.bfloat16 and x.size(0) <= 16
+            and qweight.size(0) % 2 == 0 and x.data_ptr() % 16 == 0
+            and qweight.data_ptr() % 16 == 0
+            and _K.w4a16_swiglu_fits(x.size(0), N, K, group)):
+        return None
+    out = torch.empty(x.size(0), N, dtype=x.dtype, device=x.device)
+    _K.w4a16_swiglu(out, x.contiguous(), qweight, scales, zeros, group)
+    return out
 
 
 def w4a16_streams(x: torch.Tensor, group: int) -> bool:

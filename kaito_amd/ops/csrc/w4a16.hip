@@ -18,6 +18,7 @@
 #include <torch/library.h>
 #include <ATen/ATen.h>
 #include <ATen/hip/HIPContext.h>
+#include <algorithm>
 
 namespace kaito {
 
@@ -109,6 +110,233 @@ __global__ __launch_bounds__(256) void w4a16_mfma_kernel(
     }
   }
 }
+
+// ---------------------------------------------------------------- tiles
+// Few rows of x, kept in LDS: a workgroup per CU that goes from tile to tile of
+// 16 rows of W, its eight waves over K, each with a ring of its own through which
+// 512 k of a tile (4 KB of nibbles, 256 contiguous bytes of a row, and the rows'
+// scales and zeros) arrive by direct loads, up to DEPTH stages under way. A lane's
+// 16 bytes are 32 k of one group, four operands of v_mfma_f32_16x16x32_bf16, so
+// that a nibble is unpacked once and multiplied with every row of x on the matrix
+// unit. x lies in the unpacked nibbles' order, beside its sums over the groups.
+// Bound by the unpacking, about 270 instructions per stage and 2 x 8 waves: the
+// time hardly grows with the rows. us, rows streamed (5 rows and more: MFMA from
+// global memory) and now, at 1, 2, 3, 4, 8 rows: 28672 x 4096 15.8 19.7 23.6 33.2
+// 37.7 and 16.7 17.4 17.4 17.5 18.3; 4096 x 14336 11.4 13.8 and 11.7 11.7 (more rows
+// do not fit); 4096 x 4096 4.6 5.7 7.9 8.8 8.7 and 5.9 6.1 6.6 7.0 7.9. Four waves:
+// 20.5 at 2 rows; sums of two tiles at a time: no change.
+namespace {
+
+constexpr int W4_K = 512;           // k of a stage
+constexpr int W4_STAGE = 16 * W4_K / 2 + 2 * 256;
+constexpr int W4_LDS = 160 * 1024;
+constexpr int W4_WAVES = 8;
+
+// bytes behind the rings: sums over the waves (twice), sums of x, x
+__host__ __device__ constexpr int w4_red(int mr) {
+  return W4_WAVES * mr * 4 * 16;
+}
+inline int64_t w4_lds(int depth, int mr, int64_t M, int64_t K) {
+  return W4_WAVES * depth * W4_STAGE + 2 * w4_red(mr) + K / 128 * mr * 4 +
+         M * (K * 2 + 16);
+}
+
+KAITO_DEV __amdgpu_buffer_rsrc_t w4_buffer(const void* p,
+                                           const uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes,
+                                           0x27000);
+}
+
+// MR: rows of x that have a place (4 or 16); GLU: N gate rows, then N up rows
+template <int MR, int DEPTH, bool GLU>
+__global__ __launch_bounds__(64 * W4_WAVES) void w4a16_tiles_kernel(
+    short* __restrict__ out, const short* __restrict__ x,
+    const uint32_t* __restrict__ qw, const float* __restrict__ scales,
+    const float* __restrict__ zeros, const int M, const int N, const int K) {
+  using skinny::hbf16x8;
+  typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+  constexpr int COLS = GLU ? 8 : 16, LOADS = 6, USED = MR * 4;
+  __shared__ __attribute__((aligned(128))) char lds[W4_LDS];
+  const int lane = threadIdx.x & 63, lo = lane & 15, hi = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  char* ring = lds + wave * DEPTH * W4_STAGE;
+  f32x4* red = reinterpret_cast<f32x4*>(lds + W4_WAVES * DEPTH * W4_STAGE);
+  float* xs = reinterpret_cast<float*>(
+      lds + W4_WAVES * DEPTH * W4_STAGE + 2 * w4_red(MR));     // [K / 128][MR]
+  short* xl = reinterpret_cast<short*>(xs + K / 128 * MR);  // [M][K + 8]
+  const int ntiles = N / COLS, nst = K / W4_K;
+  const int spt = (nst + W4_WAVES - 1) / W4_WAVES;  // stages of a wave and tile
+  if ((int)blockIdx.x >= ntiles) return;
+
+  auto n_of = [&](const int r) {    // row of W of row r of tile 0
+    return (uint32_t)(GLU ? r % 8 + (r >= 8 ? N : 0) : r);
+  };
+  uint32_t wo[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const int r = j * 4 + lane / 16;
+    wo[j] = n_of(r) * (K / 2) + ((lane % 16) ^ r) * 16;
+  }
+  const uint32_t so = n_of(lane / 4) * (K / 128) * 4 + lane % 4 * 4;
+  int ft = blockIdx.x, fs = 0;      // the next stage to ask for
+  auto fetch = [&](const int slot) {
+    // past the last stage: loads of nothing, so that the waits stay counts
+    const uint32_t all = __builtin_amdgcn_readfirstlane(
+        ft < ntiles && fs * W4_WAVES + wave < nst ? 0xffffffff : 0);
+    const auto wr = w4_buffer(qw, all), sr = w4_buffer(scales, all),
+               zr = w4_buffer(zeros, all);
+    const int k = (fs * W4_WAVES + wave) * W4_K;
+    const uint32_t row = ft * COLS;
+    const uint32_t at = __builtin_amdgcn_readfirstlane(row * (K / 2) + k / 2);
+    const uint32_t sat =
+        __builtin_amdgcn_readfirstlane(row * (K / 128) * 4 + k / 128 * 4);
+    char* p = ring + slot * W4_STAGE;
+#define W4_COPY(R_, P_, SIZE_, OFF_, AT_, AUX_)                               \
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(                                 \
+        R_, (__attribute__((address_space(3))) void*)(P_), SIZE_, OFF_, AT_,  \
+        0, AUX_)
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      W4_COPY(wr, p + j * 1024, 16, wo[j], at, 2 /* non-temporal */);
+    W4_COPY(sr, p + 4096, 4, so, sat, 0);
+    W4_COPY(zr, p + 4352, 4, so, sat, 0);
+#undef W4_COPY
+    if (++fs == spt) {
+      fs = 0;
+      ft += gridDim.x;
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < DEPTH; i++) fetch(i);
+
+  // ---- x and its sums over the groups; 16 threads have a group
+  for (int c = threadIdx.x; c < M * K / 8; c += 64 * W4_WAVES) {
+    const int m = c / (K / 8), k = c % (K / 8) * 8;
+    const hbf16x8 v = skinny::load_x(x + (int64_t)m * K + k);
+    float sum = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; e++) sum += (float)v[e];
+    sum = group_reduce_sum<16>(sum);
+    *reinterpret_cast<hbf16x8*>(xl + m * (K + 8) + k) =
+        skinny::nibble_order(v);
+    if (c % 16 == 0) xs[k / 128 * MR + m] = sum;
+  }
+  skinny::wait_loads<0>();
+  __syncthreads();
+
+  const short* xr = xl + min(lo, M - 1) * (K + 8) + hi * 32;
+  // rows past M of a lane's four are not stored
+  const float* xsr = xs + (MR == 16 ? 4 * hi : 0);
+  int slot = 0, par = 0;
+  for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
+    f32x4 acc{0.f, 0.f, 0.f, 0.f};
+    for (int st = 0; st < spt; st++) {
+      skinny::wait_loads<(DEPTH - 1) * LOADS>();
+      const int k = (st * W4_WAVES + wave) * W4_K;
+      if (k < K) {
+        const char* p = ring + slot * W4_STAGE;
+        const f32x4 sc = *reinterpret_cast<const f32x4*>(p + 4096 + lo * 16);
+        const f32x4 ze = *reinterpret_cast<const f32x4*>(p + 4352 + lo * 16);
+        u32x4 w[4];
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+          w[g] = *reinterpret_cast<const u32x4*>(
+              p + lo * 256 + ((g * 4 + hi) ^ lo) * 16);
+        f32x4 dot[4];
+#pragma unroll
+        for (int g = 0; g < 4; g++) dot[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+          for (int g = 0; g < 4; g++)
+            dot[g] = skinny::mfma16(
+                skinny::load_x(xr + k + g * 128 + j * 8),
+                skinny::nibbles(w[g][j]), dot[g]);
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+          const f32x4 s =
+              *reinterpret_cast<const f32x4*>(xsr + (k / 128 + g) * MR);
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            acc[r] += sc[g] * skinny::NIBBLE * dot[g][r] - ze[g] * s[r];
+        }
+      }
+      // its reads are done before it is overwritten
+      __builtin_amdgcn_s_waitcnt(0xc07f);
+      asm volatile("" ::: "memory");
+      fetch(slot);
+      slot = slot == DEPTH - 1 ? 0 : slot + 1;
+    }
+    f32x4* sums = red + par * W4_WAVES * USED;
+    if (lane < USED) sums[wave * USED + lane] = acc;
+    // own sums written, the next weights still under way; the other half of
+    // red is free once all are here
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (wave == 0 && lane < USED && !(GLU && lo >= 8)) {
+      f32x4 v = sums[lane];
+#pragma unroll
+      for (int w = 1; w < W4_WAVES; w++) v += sums[w * USED + lane];
+      if constexpr (GLU) {
+        f32x4 u = sums[lane + 8];
+#pragma unroll
+        for (int w = 1; w < W4_WAVES; w++) u += sums[w * USED + lane + 8];
+#pragma unroll
+        for (int r = 0; r < 4; r++) v[r] = skinny::silu(v[r]) * u[r];
+      }
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int m = 4 * hi + r;
+        if (m < M) out[(int64_t)m * N + t * COLS + lo] = f32_to_bf16(v[r]);
+      }
+    }
+    par ^= 1;
+  }
+  skinny::wait_loads<0>();          // no copy to LDS outlives the workgroup's
+}
+
+// 0, or the stages of a ring with which the sizes fit
+int w4_tiles_depth(int64_t M, int64_t N, int64_t K, int64_t group, int cols) {
+  if (M < 1 || M > 16 || group != 128 || K % W4_K || N % cols ||
+      (N * 2) * (K / 2) >= 1LL << 32)
+    return 0;
+  const int mr = M <= 4 ? 4 : 16;
+  return w4_lds(3, mr, M, K) <= W4_LDS ? 3
+      : w4_lds(2, mr, M, K) <= W4_LDS ? 2 : 0;
+}
+
+template <bool GLU>
+bool launch_w4_tiles(at::Tensor& out, const at::Tensor& x,
+                     const at::Tensor& qweight, const at::Tensor& scales,
+                     const at::Tensor& zeros, int64_t group) {
+  const int M = x.size(0), K = x.size(1);
+  const int N = qweight.size(0) / (GLU ? 2 : 1);
+  const int depth = w4_tiles_depth(M, N, K, group, GLU ? 8 : 16);
+  // alone, two rows pay from 48 M weights on (4096 x 14336 13.8 and 11.7 us; 4096
+  // x 8192 9.1 and 9.4, 12288 x 2048 7.1 and 8.1), one row never; the pair saves
+  // a launch of 4.6
+  if (!GLU && (M < 2 || (M == 2 && (int64_t)N * K < 48 << 20))) return false;
+  if (!depth || (uintptr_t)x.data_ptr() % 16 ||
+      (uintptr_t)qweight.data_ptr() % 16)
+    return false;
+  const dim3 grid(std::min(256, N / (GLU ? 8 : 16)));
+#define W4T_LAUNCH(MR_, D_)                                                   \
+  hipLaunchKernelGGL((w4a16_tiles_kernel<MR_, D_, GLU>), grid,                \
+      dim3(64 * W4_WAVES), 0,                                                 \
+      at::hip::getCurrentHIPStream(), (short*)out.data_ptr(),                 \
+      (const short*)x.data_ptr(), (const uint32_t*)qweight.data_ptr(),        \
+      scales.data_ptr<float>(), zeros.data_ptr<float>(), M, N, K)
+  if (M <= 4) {
+    if (depth == 3) W4T_LAUNCH(4, 3); else W4T_LAUNCH(4, 2);
+  } else {
+    if (depth == 3) W4T_LAUNCH(16, 3); else W4T_LAUNCH(16, 2);
+  }
+#undef W4T_LAUNCH
+  return true;
+}
+
+}  // namespace
 
 // ---------------------------------------------------------------- dequant
 // out[N, K] bf16 <- dequantized weights. Elementwise, one u32 pack per
@@ -275,6 +503,7 @@ void w4a16_gemv(at::Tensor out, at::Tensor x, at::Tensor qweight,
               "w4a16_gemv: 64|K and 64|group required");
   TORCH_CHECK(x.is_contiguous() && out.is_contiguous());
   if (M == 0 || N == 0) return;
+  if (launch_w4_tiles<false>(out, x, qweight, scales, zeros, group)) return;
   auto stream = at::hip::getCurrentHIPStream();
 #define W4_ARGS                                                               \
   (short*)out.data_ptr(), (const short*)x.data_ptr(),                         \
@@ -311,6 +540,25 @@ void w4a16_gemv(at::Tensor out, at::Tensor x, at::Tensor qweight,
   }
 #undef W4_MFMA
 #undef W4_ARGS
+}
+
+// silu(x Wg^T) * (x Wu^T) of the stacked W = [Wg | Wu], where the tiles take it
+// (w4a16_swiglu_fits)
+bool w4a16_swiglu_fits(int64_t M, int64_t N, int64_t K, int64_t group) {
+  return w4_tiles_depth(M, N, K, group, 8) > 0;
+}
+
+void w4a16_swiglu(at::Tensor out, at::Tensor x, at::Tensor qweight,
+                  at::Tensor scales, at::Tensor zeros, int64_t group) {
+  TORCH_CHECK(x.is_contiguous() && out.is_contiguous() &&
+              x.dtype() == at::kBFloat16 && out.dtype() == at::kBFloat16 &&
+              qweight.is_contiguous() && scales.is_contiguous() &&
+              zeros.is_contiguous());
+  TORCH_CHECK(qweight.size(0) % 2 == 0 && qweight.size(1) * 8 == x.size(1) &&
+              out.size(0) == x.size(0) &&
+              out.size(1) * 2 == qweight.size(0));
+  TORCH_CHECK(launch_w4_tiles<true>(out, x, qweight, scales, zeros, group),
+              "w4a16_swiglu: sizes of the tiles");
 }
 
 void w4a16_dequant(at::Tensor out, at::Tensor qweight, at::Tensor scales,

@@ -86,6 +86,15 @@ class ColumnParallelLinear(_QuantMixin, nn.Module):
         return self.bias is None and not self._quantized \
             and not lora_mod.is_active()
 
+    def quantized_swiglu(self, x: torch.Tensor):
+        """silu(gate) * up of this layer's packed [gate | up] rows, or None
+        where that is not one launch."""
+        if not self._quantized or self.bias is not None \
+                or lora_mod.is_active() or x.dim() != 2:
+            return None
+        return ops.w4a16_swiglu(x, self.qweight, self.scales, self.zeros,
+                                self.q_group)
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self._quantized:
             out = self._qmatmul(x)

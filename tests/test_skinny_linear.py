@@ -136,6 +136,26 @@ def test_transformed_calls_are_seen():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8, 14, 16])
+@pytest.mark.parametrize("N,K", [(8, 512), (24, 4608), (2056, 1536),
+                                 (2080, 2048), (16, 14336)])
+def test_w4_tiles(M, N, K):
+    """x in LDS: fewer tiles than workgroups and several each, waves without a
+    stage, rings of two and three stages, sizes that do not fit."""
+    torch.manual_seed(M * N + K)
+    x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    qw, s, z = (t.to(DEV) for t in quantize_w4(torch.randn(2 * N, K), 128))
+    w = R.w4a16_unpack(qw.cpu(), s.cpu(), z.cpu(), 128).to(DEV)
+    ref = x.double() @ w.double().T
+    _close(ops.w4a16_gemv(x, qw, s, z, 128), ref)
+    out = ops.w4a16_swiglu(x, qw, s, z, 128)
+    assert out is not None or M * K > 34000      # LDS
+    if out is not None:
+        g, u = ref.chunk(2, -1)
+        _close(out, g * torch.sigmoid(g) * u)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 16, 17, 32])
 @pytest.mark.parametrize("N,K,G", [(1, 64, 64), (40, 128, 128),
                                    (33, 192, 192), (100, 4224, 128),
