@@ -603,10 +603,13 @@ def _router_logits(x: torch.Tensor, gate: torch.Tensor) -> torch.Tensor:
     return torch.nn.functional.linear(x.float(), gate.float())
 
 
-def _gate_in_route(x, gate) -> bool:
+def _gate_short(x, gate) -> bool:
     T = x.size(0)
-    return (x.is_cuda and x.dtype == torch.bfloat16 and T <= 512
-            and gate.size(0) <= 32 and T * gate.size(0) <= 8192
+    return T <= 512 and T * gate.size(0) <= 8192
+
+
+def _gate_in_route(x, gate) -> bool:
+    return (x.is_cuda and x.dtype == torch.bfloat16 and gate.size(0) <= 32
             and gate.is_contiguous()
             and gate.dtype in (torch.bfloat16, torch.float32)
             and x.stride(1) == 1 and x.stride(0) % 8 == 0
@@ -623,7 +626,8 @@ def moe_norm_gate_route(x, residual, norm_w, eps: float, gate, correction,
     def aligned(t):
         return t.dtype == torch.bfloat16 and t.is_contiguous() \
             and t.data_ptr() % 16 == 0
-    if _gate_in_route(x, gate) and aligned(x) and aligned(residual) \
+    if _gate_short(x, gate) and _gate_in_route(x, gate) \
+            and aligned(x) and aligned(residual) \
             and aligned(norm_w) and residual.shape == x.shape \
             and x.size(1) <= 8192:
         topi, topw, w_id = _route_out(x.size(0), top, x.device)
@@ -642,14 +646,20 @@ def moe_gate_route(x, gate, correction, top: int, n_real: int,
                    scale: float = 1.0, mode: str = "softmax"):
     """moe_route of the logits x gate^T, formed in f32. One launch for short
     steps and narrow routers: a workgroup per row reads the whole router, 8
-    outputs after one another, so that wider ones and longer steps leave the
-    product to the library (us, one launch and two; rows of 2048 and 7168, bf16
+    outputs after one another, so that wider ones and longer steps take tiles of
+    16 rows or leave the product to the library (us, one launch and two; rows of 2048 and 7168, bf16
     router: 8 outputs 5.1, 9.4 and 6.1, 13.2 at 32 rows, 5.7, 9.5 and 7.0, 11.4
     at 512; 32 outputs 9.2, 9.6 and 12.2, 13.7 at 32 rows, 9.6, 9.6 and 13.3,
     13.7 at 256, 10.3, 9.7 and 16.0, 13.9 at 512; 48 outputs 12.0, 9.5 and
-    16.5, 13.6 at 32)."""
+    16.5, 13.6 at 32). Tiles up to 32 outputs: an f32 router saves the cast of
+    the rows (8192 rows, 8 outputs: 16.3, 38.0 and 38.2, 103; 32 outputs 27.7,
+    38.3), a bf16 one has to be narrow (8 outputs 11.7, 15.5 and 27.4, 26.4; 32
+    outputs 16.0, 15.7; 1024 rows of 7168 to 32 outputs 23.0, 14.6)."""
     T = x.size(0)
-    if _gate_in_route(x, gate):
+    H = x.size(1)
+    long = H % 32 == 0 and (gate.dtype == torch.float32
+                            or gate.size(0) <= 16 and H <= 4096)
+    if (long or _gate_short(x, gate)) and _gate_in_route(x, gate):
         topi, topw, w_id = _route_out(T, top, x.device)
         _K.moe_gate_route(topi, topw, w_id, x, gate, _none(correction, x),
                           n_real, groups, keep, renorm, scale,

@@ -1,7 +1,8 @@
 // Expert choice for routed feed-forwards, in two launches.
 //
 //   moe_route: one wave per token, from f32 logits; moe_gate_route: one
-//     workgroup per token, which also forms the logits x W^T. Modes:
+//     workgroup per token (of long steps per 16 tokens), which also forms the
+//     logits x W^T. Modes:
 //     SOFTMAX: s = softmax(logits), choice = s + correction (none given: s);
 //       a group of `groups` equal groups of neighbours scores its largest
 //       choice;
@@ -249,6 +250,114 @@ __global__ __launch_bounds__(256) void moe_gate_route_kernel(
     part[0][lane] += part[1][lane] + part[2][lane] + part[3][lane];
   __builtin_amdgcn_wave_barrier();
   route_row<1, MODE>(a, part[0], t, lane);
+}
+
+// Prompts: 16 rows per workgroup, products on v_mfma_f32_16x16x32_bf16. A wave
+// takes the dims 128 w .. of every 2048 and, once the 16 partial sums are added,
+// the choice of one row: logits never leave the workgroup. An f32 router is three
+// bf16 terms to the last bit, so three products have the exact terms of an f32 one
+// and rows need no cast. Bound by latency up to 2048 rows, behind them by reading
+// rows and router through L2; a workgroup per row reads the router 16 times as
+// often (us, product by the library and choice -> here, rows of 2048, 8 outputs:
+// bf16 router 9.7 -> 7.6 at 600 rows, 15.5 -> 11.7 at 8192 (row by row 20.4); f32
+// 16.3 -> 9.5 and 38.0 -> 16.3 (27.2)). Loads of a round's router ahead of its
+// products cost f32 routers half their waves: 19.3. Error of the weights against
+// f64 logits at 8192 rows: 1.8e-7, of the library's 3.0e-7 and 6.6e-7.
+constexpr int GATE_ROWS = 16, GATE_STEPS = 4;
+
+// the terms of 8 elements of the router, largest first
+KAITO_DEV void gate_terms(const short* w, skinny::hbf16x8 (&b)[1]) {
+  b[0] = skinny::load_x(w);
+}
+KAITO_DEV void gate_terms(const float* w, skinny::hbf16x8 (&b)[3]) {
+  const float4_t lo = *reinterpret_cast<const float4_t*>(w);
+  const float4_t hi = *reinterpret_cast<const float4_t*>(w + 4);
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    float v = i < 4 ? lo[i & 3] : hi[i & 3];
+#pragma unroll
+    for (int n = 0; n < 3; n++) {
+      b[n][i] = (__bf16)v;
+      v -= (float)b[n][i];
+      if (!(fabsf(v) < INFINITY)) v = 0.f;  // behind an infinity, a NaN
+    }
+  }
+}
+
+// NT: 16 outputs each; H is a multiple of 32
+template <int MODE, typename W, int NT>
+__global__ __launch_bounds__(1024) void moe_gate_route_tiles_kernel(
+    const RouteArgs a, const short* __restrict__ x, const int64_t x_stride,
+    const W* __restrict__ w, const int H) {
+  constexpr int TERMS = sizeof(W) == 4 ? 3 : 1, COLS = NT * 16 + 1;
+  __shared__ float part[16][GATE_ROWS][COLS], logit[GATE_ROWS][COLS];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c = lane & 15, q = lane >> 4;
+  const int64_t t0 = (int64_t)blockIdx.x * GATE_ROWS;
+  const short* xr = x + min(t0 + c, (int64_t)a.T - 1) * x_stride + q * 8;
+  float4_t acc[NT][TERMS > 1 ? 2 : 1];      // the largest terms, the rest
+#pragma unroll
+  for (int n = 0; n < NT; n++)
+    for (auto& v : acc[n]) v = float4_t{0.f, 0.f, 0.f, 0.f};
+  for (int k0 = wave * 32 * GATE_STEPS; k0 < H; k0 += 512 * GATE_STEPS) {
+    skinny::hbf16x8 xv[GATE_STEPS];
+#pragma unroll
+    for (int i = 0; i < GATE_STEPS; i++)
+      xv[i] = skinny::load_x(xr + min(k0 + 32 * i, H - 32));
+#pragma unroll
+    for (int i = 0; i < GATE_STEPS; i++) {
+      const int k = k0 + 32 * i;
+      if (k >= H) break;
+      bool wild = false;                    // an infinity or a NaN in x
+      if constexpr (TERMS > 1) {
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+          wild |= !(fabsf((float)xv[i][e]) < INFINITY);
+        wild = __any(wild);
+      }
+#pragma unroll
+      for (int n = 0; n < NT; n++) {
+        skinny::hbf16x8 b[TERMS];
+        gate_terms(w + (int64_t)min(n * 16 + c, a.N - 1) * H + k + q * 8, b);
+        acc[n][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xv[i], b[0],
+                                                            acc[n][0], 0, 0, 0);
+        if constexpr (TERMS > 1) {
+          // an infinity is multiplied once: its product with a smaller term
+          // could have the other sign, or be 0 times it
+          auto xs = xv[i];
+          if (wild) {
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+              if (!(fabsf((float)xs[e]) < INFINITY)) xs[e] = (__bf16)0.f;
+          }
+#pragma unroll
+          for (int j = TERMS - 1; j > 0; j--)
+            acc[n][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                xs, b[j], acc[n][1], 0, 0, 0);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < NT; n++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      float v = acc[n][0][r];
+      if constexpr (TERMS > 1) v += acc[n][1][r];
+      part[wave][q * 4 + r][n * 16 + c] = v;
+    }
+  __syncthreads();
+  // wave r: row r. Lane: output lane % 16 (% 32), and a share of the sums
+  constexpr int SHARE = 64 / (NT * 16), EACH = 16 / SHARE;
+  const int col = lane % (NT * 16), first = lane / (NT * 16) * EACH;
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < EACH; i++) sum += part[first + i][wave][col];
+#pragma unroll
+  for (int off = NT * 16; off < 64; off <<= 1) sum += __shfl_xor(sum, off, 64);
+  if (lane < NT * 16) logit[wave][lane] = sum;
+  __builtin_amdgcn_wave_barrier();
+  if (t0 + wave < a.T) route_row<1, MODE>(a, logit[wave], t0 + wave, lane);
 }
 
 // The residual norm ahead of the router in the same launch: residual += x, xn =
@@ -505,13 +614,34 @@ void moe_gate_route(at::Tensor topi, at::Tensor topw, at::Tensor w_id,
                                  groups, keep, renorm, scale, mode);
   if (T == 0) return;
   auto stream = at::hip::getCurrentHIPStream();
+  const bool f32 = gate.dtype() == at::kFloat;
+  TORCH_CHECK(f32 || gate.dtype() == at::kBFloat16);
+  // short steps go row by row: 512 rows of 2048, 8 outputs, 6.5 us and 7.6
+  if (H % 32 == 0 && (T > 512 || (int64_t)T * N > 8192)) {
+    const int blocks = (T + GATE_ROWS - 1) / GATE_ROWS;
+    with_mode(mode, [&](auto md) {
+      auto launch = [&](auto nt, auto wt) {
+        using W = decltype(wt);
+        hipLaunchKernelGGL(
+            (moe_gate_route_tiles_kernel<decltype(md)::value, W,
+                                         decltype(nt)::value>),
+            dim3(blocks), dim3(1024), 0, stream, a, (const short*)x.data_ptr(),
+            x.stride(0), (const W*)gate.data_ptr(), H);
+      };
+      auto sized = [&](auto wt) {
+        if (N <= 16) launch(std::integral_constant<int, 1>{}, wt);
+        else launch(std::integral_constant<int, 2>{}, wt);
+      };
+      if (f32) sized(0.f); else sized((short)0);
+    });
+    return;
+  }
   with_mode(mode, [&](auto md) {
-    if (gate.dtype() == at::kFloat) {
+    if (f32) {
       hipLaunchKernelGGL((moe_gate_route_kernel<decltype(md)::value, float>),
           dim3(T), dim3(256), 0, stream, a, (const short*)x.data_ptr(),
           x.stride(0), gate.data_ptr<float>(), H);
     } else {
-      TORCH_CHECK(gate.dtype() == at::kBFloat16);
       hipLaunchKernelGGL((moe_gate_route_kernel<decltype(md)::value, short>),
           dim3(T), dim3(256), 0, stream, a, (const short*)x.data_ptr(),
           x.stride(0), (const short*)gate.data_ptr(), H);

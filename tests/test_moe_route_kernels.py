@@ -196,3 +196,37 @@ def test_sort_of_many_experts(T, top, n, spread):
     topw = torch.rand(T, top, device=DEV)
     for a, b in zip(ops.moe_plan(topi, topw, n), R.moe_plan(topi, topw, n)):
         assert a.dtype == b.dtype and torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,N,H,mode", [
+    (513, 16, 64, "softmax"), (600, 1, 32, "softmax"), (529, 9, 2080, "logits"),
+    (257, 32, 2176, "sigmoid"), (4099, 17, 96, "sigmoid")])
+def test_choice_of_16_rows(dtype, T, N, H, mode):
+    torch.manual_seed(T + N)
+    x = torch.randn(T, H + 8, device=DEV).to(torch.bfloat16)[:, :H]
+    gate = torch.randn(N, H, device=DEV).to(dtype) * 3 / H ** 0.5
+    z = (x.double() @ gate.double().T).float()
+    a = (min(2, N), N, 1, 1, True, 1.0, mode)
+    _check(ops.moe_gate_route(x, gate, None, *a),
+           R.moe_route(z, None, *a), N)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_choice_of_16_rows_not_finite(dtype):
+    """Infinities and NaN of rows and router reach the choice as in the
+    product of short steps."""
+    torch.manual_seed(3)
+    x = torch.randn(600, 256, device=DEV).to(torch.bfloat16)
+    gate = (torch.randn(8, 256, device=DEV) / 16).to(dtype)
+    gate[5, 7] = float("inf")
+    x[3, 9], x[4, 9], x[40, 11] = float("inf"), -float("inf"), float("nan")
+    a = (3, 8, 1, 1, False, 1.0, "logits")
+    long = ops.moe_gate_route(x, gate, None, *a)
+    short = ops.moe_gate_route(x[:512], gate, None, *a)
+    assert torch.equal(long[0][:512], short[0])
+    # weights: logits of unit size, sums of 256 products in another order
+    torch.testing.assert_close(long[1][:512], short[1], rtol=1e-5, atol=1e-6,
+                               equal_nan=True)
