@@ -35,11 +35,13 @@
 //   whole prompts 4 x 2048, 16/4 heads of 128, window 1024: 447 -> 89 us;
 //   one prompt of 8192, 32/8 heads of 128: 140 -> 762 TFLOP/s;
 //   latent prompts 4 x 2048, 16 heads: 2307 us (padded to 256) -> 113 us;
-//   8192 suffix rows over 20000 paged keys: 140 -> 825 TFLOP/s;
+//   8192 suffix rows over 20000 paged keys: 140 -> 825 TFLOP/s (997 over 16384
+//   with the pages' addresses as scalars);
 //   paged window 1024 with cap and penalty, 4 x 2048, 16/4 heads: 583 -> 176
 //   (with the bare hardware reciprocal in cap and sigmoid 161).
 #pragma once
 #include "common.h"
+#include <type_traits>
 
 namespace kaito {
 namespace flash {
@@ -143,6 +145,7 @@ void flash_prefill_kernel(const Args a) {
   // rides in the exponent's multiply-add
   const bool fold = !EXT && !SIG && !DB && a.scale > 0.f;
   static_assert(KVT * CK % NT == 0 && KVT * CV % NT == 0 && DV % 32 == 0);
+  static_assert(SRC != PAGED_FP8 || !EXT);
 
   const int HG = a.QH >> a.gs;                    // head groups
   const int hg = blockIdx.x % HG;
@@ -223,21 +226,87 @@ void flash_prefill_kernel(const Args a) {
 
   // ---- staging. Slot s of a tile (16 bytes of LDS) is row s / C, place
   // s % C; thread tid fills slots j * NT + tid.
-  int pk[SRC == ROWS_BF16 ? 1 : LK], pv[SRC == ROWS_BF16 ? 1 : LV];
+  // Pages of 16 keys: a wave's instruction reads rows of one page, so that page
+  // numbers and addresses are scalars and a lane's offset does not change. With a
+  // page, a quotient and a 64-bit address per lane and copy, the vector unit
+  // had more to do than the matrix cores (before -> now): 8192 suffix rows over
+  // 8192 keys, 32/8 heads of 128, 883 -> 999 TFLOP/s; 3627 over 16384 810 ->
+  // 932; fp8 cache, 4096 over 4096, 757 -> 893; heads of 64 and 256, 2048 over
+  // 2048, 78 -> 65 and 297 -> 244 us; window 1024 with key size 128, value
+  // size 256, 118 -> 107 us. The same for rows of the step gave 3 % at 8192 and
+  // took 2 % at 4 x 2048.
+  static_assert(SRC == ROWS_BF16 || (64 % CK == 0 && 64 % CV == 0));
+  constexpr bool PAGED = SRC != ROWS_BF16;
+  const bool by16 = PAGED && (!EXT || a.BS == 16);
+  int pages_k = 0, pages_v = 0;     // lane j: page of this wave's j-th copy
+  int pk[PAGED && EXT ? LK : 1], pv[PAGED && EXT ? LV : 1];
   auto fetch_pages = [&](const int kv0) {       // pages of the tile at kv0
-    if constexpr (SRC != ROWS_BF16) {
+    if constexpr (PAGED) {
+      if (by16) {
+        auto number = [&](const int chunks, const int copies) {
+          const int key = kv0 + min(lane, copies - 1) * (NT / chunks) +
+              wave * (64 / chunks);
+          return bt[min(key, kv_len - 1) >> 4];
+        };
+        pages_k = number(CK, LK);
+        if constexpr (CV != CK) pages_v = number(CV, LV);
+      } else if constexpr (EXT) {
 #pragma unroll
-      for (int j = 0; j < LK; j++)
-        pk[j] = bt[min(kv0 + (j * NT + tid) / CK, kv_len - 1) / a.BS];
-      if constexpr (CV != CK) {
+        for (int j = 0; j < LK; j++)
+          pk[j] = bt[min(kv0 + (j * NT + tid) / CK, kv_len - 1) / a.BS];
+        if constexpr (CV != CK) {
 #pragma unroll
-        for (int j = 0; j < LV; j++)
-          pv[j] = bt[min(kv0 + (j * NT + tid) / CV, kv_len - 1) / a.BS];
+          for (int j = 0; j < LV; j++)
+            pv[j] = bt[min(kv0 + (j * NT + tid) / CV, kv_len - 1) / a.BS];
+        }
       }
     }
   };
   u8x8_t rk[SRC == PAGED_FP8 ? LK : 1], rv[SRC == PAGED_FP8 ? LV : 1];
+  auto stage_pages = [&](const int kv0, short* buf, auto whole) {
+    auto at = [&](const int pages, const int j, const int chunks) {
+      const int64_t page = __builtin_amdgcn_readlane(pages, j);
+      return (page * a.KH + kvh) * 16 * (chunks * 8);
+    };
+    // row of its page; behind the last key that one again
+    auto place = [&](const int j, const int chunks) {
+      const int row = tid / chunks, step = j * (NT / chunks);
+      if (decltype(whole)::value) return (row & 15) + (step & 15);
+      return min(kv0 + step + row, kv_len - 1) & 15;
+    };
+#pragma unroll
+    for (int j = 0; j < LK; j++) {
+      const int s = j * NT + tid;
+      const int off = place(j, CK) * D + swz_k<D>(s / CK, s % CK) * 8;
+      if constexpr (SRC == PAGED_FP8)
+        rk[j] = *reinterpret_cast<const u8x8_t*>(
+            (const uint8_t*)a.k + at(pages_k, j, CK) + (uint32_t)off);
+      else
+        lds_copy16((const short*)a.k + at(pages_k, j, CK) + (uint32_t)off,
+                   buf + (j * NT + wave * 64) * 8);
+    }
+#pragma unroll
+    for (int j = 0; j < LV; j++) {
+      const int s = j * NT + tid;
+      const int off = place(j, CV) * DV + swz_v<DV>(s / CV, s % CV) * 8;
+      const int64_t page = at(CV == CK ? pages_k : pages_v, j, CV);
+      if constexpr (SRC == PAGED_FP8)
+        rv[j] = *reinterpret_cast<const u8x8_t*>((const uint8_t*)a.v + page +
+                                                 (uint32_t)off);
+      else
+        lds_copy16((const short*)a.v + page + (uint32_t)off,
+                   buf + KVT * D + (j * NT + wave * 64) * 8);
+    }
+  };
   auto stage = [&](const int kv0, short* buf) {
+    if constexpr (PAGED) {
+      if (by16) {
+        if (kv0 + KVT <= kv_len) stage_pages(kv0, buf, std::true_type{});
+        else stage_pages(kv0, buf, std::false_type{});
+        return;
+      }
+      if constexpr (!EXT) return;
+    }
 #pragma unroll
     for (int j = 0; j < LK; j++) {
       const int s = j * NT + tid, row = s / CK;
@@ -249,14 +318,11 @@ void flash_prefill_kernel(const Args a) {
             ? (const short*)a.k + tok * a.k_ts + kvh * a.k_hs + col
             : a.k2 + tok * a.k2_ts + col - D1;
         lds_copy16(p, buf + (j * NT + wave * 64) * 8);
-      } else {
-        const int64_t at =
-            (((int64_t)pk[j] * a.KH + kvh) * a.BS + key % a.BS) * D + col;
-        if constexpr (SRC == PAGED_FP8)
-          rk[j] = *reinterpret_cast<const u8x8_t*>((const uint8_t*)a.k + at);
-        else
-          lds_copy16((const short*)a.k + at,
-                     buf + (j * NT + wave * 64) * 8);
+      } else if constexpr (EXT) {
+        lds_copy16((const short*)a.k +
+                       (((int64_t)pk[j] * a.KH + kvh) * a.BS + key % a.BS) * D +
+                       col,
+                   buf + (j * NT + wave * 64) * 8);
       }
     }
     short* vbuf = buf + KVT * D;
@@ -269,15 +335,11 @@ void flash_prefill_kernel(const Args a) {
         lds_copy16((const short*)a.v + (int64_t)(tok0 + key) * a.v_ts +
                        kvh * a.v_hs + col,
                    vbuf + (j * NT + wave * 64) * 8);
-      } else {
+      } else if constexpr (EXT) {
         const int64_t page = CV == CK ? pk[j] : pv[j];
-        const int64_t at =
-            ((page * a.KH + kvh) * a.BS + key % a.BS) * DV + col;
-        if constexpr (SRC == PAGED_FP8)
-          rv[j] = *reinterpret_cast<const u8x8_t*>((const uint8_t*)a.v + at);
-        else
-          lds_copy16((const short*)a.v + at,
-                     vbuf + (j * NT + wave * 64) * 8);
+        lds_copy16((const short*)a.v +
+                       ((page * a.KH + kvh) * a.BS + key % a.BS) * DV + col,
+                   vbuf + (j * NT + wave * 64) * 8);
       }
     }
   };

@@ -291,3 +291,62 @@ def test_window_options(H, G, D, V, mode):
                                vc.cpu().float(), bt.cpu(), seq, pos,
                                D ** -0.5, **opt)
     _check(out, ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_page_rows_behind_the_last_key(D, fp8):
+    """What the last page holds behind a sequence has no say, in tiles read
+    whole (64 and 128 keys) and in those read in part."""
+    torch.manual_seed(D)
+    kv, ql = [64, 79, 128, 17, 129, 1], [64, 40, 3, 17, 65, 1]
+    mb = 9
+    bt = torch.randperm(len(kv) * mb, device=DEV).int().view(len(kv), mb)
+    kc, vc = (_bf16(len(kv) * mb, 2, 16, D) for _ in range(2))
+    for b, n in enumerate(kv):          # everything behind the keys is NaN
+        for i in range(mb):
+            kc[bt[b, i].long(), :, max(0, min(16, n - 16 * i)):] = math.nan
+            vc[bt[b, i].long(), :, max(0, min(16, n - 16 * i)):] = math.nan
+    args = kc, vc
+    if fp8:
+        args = tuple(t.to(torch.float8_e4m3fn) for t in args)
+        kc, vc = (t.to(torch.bfloat16) for t in args)
+        args = tuple(t.view(torch.uint8) for t in args)
+    q = _bf16(sum(ql), 4, D)
+    kl = torch.tensor(kv, dtype=torch.int32, device=DEV)
+    out = ops.context_attention(q, *args, _cu(ql), kl, bt, D ** -0.5)
+    ref = R.context_attention(q.float(), kc.float(), vc.float(), _cu(ql), kl,
+                              bt, D ** -0.5)
+    _check(out, ref.cpu())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,V", [(64, 64), (64, 256), (128, 32), (128, 128),
+                                 (256, 64), (256, 256)])
+@pytest.mark.parametrize("window,keep", [(0, 0), (100, 0), (70, 5)])
+def test_pages_of_16_keys_and_others(D, V, window, keep):
+    """Pages of 16 keys have copies of their own: the same keys in pages of 8
+    and 32 give the same bits."""
+    torch.manual_seed(D + V)
+    starts, ql, mb = [130, 0, 33], [129, 70, 31], 20
+    q, n = _bf16(sum(ql), 4, D), len(ql)
+    k, v = _bf16(n, mb * 16, 2, D), _bf16(n, mb * 16, 2, V)
+    st = torch.tensor(starts, dtype=torch.int32, device=DEV)
+    tiles = ops.build_query_tiles(ql, DEV) + (_cu(ql), st)
+    outs = []
+    for bs in (16, 8, 32):
+        pages = mb * 16 // bs
+        bt = torch.randperm(n * pages, device=DEV).int().view(n, pages)
+        caches = []
+        for rows in (k, v):
+            c = torch.empty(n * pages, 2, bs, rows.size(3), device=DEV,
+                            dtype=torch.bfloat16)
+            c[bt.view(-1).long()] = rows.view(n * pages, bs, 2, -1) \
+                .transpose(1, 2)
+            caches.append(c)
+        outs.append(ops.window_attention(
+            q, *caches, bt, None, None, D ** -0.5, window=window, tiles=tiles,
+            keep_first=keep))
+    assert torch.isfinite(outs[0]).all()
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
