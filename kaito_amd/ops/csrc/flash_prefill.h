@@ -298,6 +298,30 @@ void flash_prefill_kernel(const Args a) {
                    buf + KVT * D + (j * NT + wave * 64) * 8);
     }
   };
+  // Split keys: a lane's copies of a tile come from either part, those PERIOD
+  // apart from the same dims; their places move on by one tile at a time. One
+  // prompt of 8192, 16 heads, 601 -> 562 us; 4 x 2048 132 -> 125; 128 heads, 16 x
+  // 128, 79 -> 73 to 78.
+  constexpr bool SPLIT_K = !PAGED && D1 < D;
+  constexpr int PERIOD = SPLIT_K ? 3 : 1, AHEAD = PERIOD * NT / CK;
+  static_assert(!SPLIT_K || (LK % PERIOD == 0 && PERIOD * NT % CK == 0 &&
+                             AHEAD % 8 == 0 && KVT == LK / PERIOD * AHEAD));
+  const short* k_lane[PERIOD];
+  const short* v_lane = nullptr;
+  if constexpr (SPLIT_K) {
+    const int64_t tok = tok0 + kv_first;
+#pragma unroll
+    for (int j = 0; j < PERIOD; j++) {
+      const int s = j * NT + tid, row = s / CK;
+      const int col = swz_k<D>(row, s % CK) * 8;
+      k_lane[j] = col < D1
+          ? (const short*)a.k + (tok + row) * a.k_ts + kvh * a.k_hs + col
+          : a.k2 + (tok + row) * a.k2_ts + col - D1;
+    }
+    v_lane = (const short*)a.v + (tok + tid / CV) * a.v_ts + kvh * a.v_hs +
+        swz_v<DV>(tid / CV, tid % CV) * 8;
+    static_assert(NT / CV % 8 == 0);
+  }
   auto stage = [&](const int kv0, short* buf) {
     if constexpr (PAGED) {
       if (by16) {
@@ -306,6 +330,24 @@ void flash_prefill_kernel(const Args a) {
         return;
       }
       if constexpr (!EXT) return;
+    }
+    if constexpr (SPLIT_K) {
+      if (kv0 + KVT <= kv_len) {    // no row to stand for another
+#pragma unroll
+        for (int j = 0; j < LK; j++) {
+          const short*& p = k_lane[j % PERIOD];
+          lds_copy16(p, buf + (j * NT + wave * 64) * 8);
+          const int s = j % PERIOD * NT + tid;
+          const bool first = swz_k<D>(s / CK, s % CK) * 8 < D1;
+          p += AHEAD * (first ? a.k_ts : a.k2_ts);
+        }
+#pragma unroll
+        for (int j = 0; j < LV; j++)
+          lds_copy16(v_lane + j * (NT / CV) * a.v_ts,
+                     buf + KVT * D + (j * NT + wave * 64) * 8);
+        v_lane += KVT * a.v_ts;
+        return;
+      }
     }
 #pragma unroll
     for (int j = 0; j < LK; j++) {
