@@ -1,6 +1,6 @@
 #!/usr/bin/env python3
 """Kernel microbenchmarks on MI355X: prints achieved bandwidth/time for the
-hot kernels at bench-like shapes. Run under gpurun."""
+hot kernels at bench-like shapes. Run on an MI355X."""
 import argparse
 import math
 import os
