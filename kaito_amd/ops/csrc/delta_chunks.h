@@ -160,9 +160,9 @@ __global__ __launch_bounds__(64) void delta_chunk_prep_kernel(
       double s = i == lo ? 1. : 0.;
 #pragma unroll
       for (int m = 0; m < i; m++) s -= A[hi][i][m] * x[m];
-      // what stands above the diagonal is 0 also where A is not finite
+      // what stands above the diagonal is 0 also where A or beta is not finite
       x[i] = i < lo ? 0. : s;
-      if (live) out[i * C + lo] = (float)(x[i] * beta);
+      if (live) out[i * C + lo] = i < lo ? 0.f : (float)(x[i] * beta);
     }
     __syncthreads();
   }

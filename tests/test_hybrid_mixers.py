@@ -168,6 +168,50 @@ def test_delta_rule_chunks(dt, G, H, D, V, waves, monkeypatch):
     assert torch.equal(bad[:, V:], clean[:, V:])
 
 
+def _chunk_inputs(lens, G, H, D, V, dt, dev="cuda"):
+    T = sum(lens)
+    r = lambda *s: torch.randn(*s).to(dt).to(dev)
+    x = [r(T, G, D), r(T, G, D), r(T, H, V), r(T, H, V), r(T, H), r(T, H)]
+    w = [t.to(dev) for t in (torch.randn(H) * 0.5 - 2.0, torch.randn(H),
+                             torch.randn(V))]
+    lay = layout(dev, lens, [0] * len(lens), list(range(len(lens))))[:3]
+    return x, w, lay
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("waves", ["1", "4"])
+@pytest.mark.parametrize("what", ["q", "k", "v", "a", "b", "token"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), -float("inf")])
+def test_delta_chunks_are_causal(what, value, waves, monkeypatch):
+    """A value that is not finite, wherever it enters, leaves the tokens before
+    it, other sequences and, in a head's own inputs, other heads alone."""
+    monkeypatch.setenv("KAITO_DELTA_WAVES", waves)
+    lens, at = [50, 100, 40], 50 + 37            # inside a chunk
+    G, H, D, V = 2, 4, 64, 32
+    x, w, lay = _chunk_inputs(lens, G, H, D, V, torch.float32)
+
+    def run():
+        state = torch.zeros(3, H, D, V, device="cuda")
+        o = ops.gated_delta_rule(*x, *w, state, *lay, 1e-6, 1e-5)
+        return o.view(-1, H, V), state
+    clean, state = run()
+    for i, name in enumerate(("q", "k", "v", "gate", "a", "b")):
+        if what == "token":
+            x[i][at] = value
+        elif what == name:
+            x[i][at, 0] = value                 # head 0, or heads 0 and 1
+    bad, bad_state = run()
+    end = lens[0] + lens[1]
+    assert torch.equal(bad[:at], clean[:at])
+    assert torch.equal(bad[end:], clean[end:])
+    assert torch.equal(bad_state[::2], state[::2])
+    if what != "token":
+        assert torch.equal(bad[:, 2:], clean[:, 2:])
+    if what == "q":                             # read by its own token only
+        assert torch.equal(bad[at + 1:], clean[at + 1:])
+        assert torch.equal(bad_state, state)
+
+
 # ------------------------------------------------------------------ RG-LRU
 
 @pytest.mark.parametrize("mode", MODES)
