@@ -93,20 +93,22 @@ __global__ __launch_bounds__(64) void delta_chunk_prep_kernel(
   }
   const float iq = (1.0f / sqrtf(sq + qk_eps)) * (1.0f / sqrtf((float)D));
   const float ik = 1.0f / sqrtf(sk + qk_eps);
-  // sums in trees of one instruction's, for their rounding
+  // k.k of the unit vectors, as the state has them; q.k of the rows, rounded last.
+  // Sums in trees of one instruction's, for their rounding.
   const f32x4 zero{0.f, 0.f, 0.f, 0.f};
   f32x4 ck[NJ], cq[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; j++) {
     const int64_t at = (t * G + g) * D + 16 * j + 4 * hi;
+    const float4_t ku = kv[j] * ik;
     if (lo < n) {
-      *reinterpret_cast<float4_t*>(kn + at) = kv[j] * ik;
+      *reinterpret_cast<float4_t*>(kn + at) = ku;
       *reinterpret_cast<float4_t*>(qn + at) = qv[j] * iq;
     }
     f32x4 pk[4], pq[4];
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      pk[e] = mfma4(kv[j][e], kv[j][e], zero);
+      pk[e] = mfma4(ku[e], ku[e], zero);
       pq[e] = mfma4(qv[j][e], kv[j][e], zero);
     }
     ck[j] = (pk[0] + pk[1]) + (pk[2] + pk[3]);
@@ -121,8 +123,10 @@ __global__ __launch_bounds__(64) void delta_chunk_prep_kernel(
     }
 #pragma unroll
   for (int r = 0; r < 4; r++) {
-    kk[4 * hi + r][lo] = ck[0][r] * (__shfl(ik, 4 * hi + r, 64) * ik);
-    qk[4 * hi + r][lo] = cq[0][r] * (__shfl(iq, 4 * hi + r, 64) * ik);
+    kk[4 * hi + r][lo] = ck[0][r];
+    // a row whose square is beyond f32 has a unit vector of 0
+    const float ir = __shfl(iq, 4 * hi + r, 64);
+    qk[4 * hi + r][lo] = ir == 0.f || ik == 0.f ? 0.f : cq[0][r] * ir * ik;
   }
 
   // four heads at a time, a quarter wave each

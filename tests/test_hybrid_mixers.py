@@ -212,6 +212,24 @@ def test_delta_chunks_are_causal(what, value, waves, monkeypatch):
         assert torch.equal(bad_state, state)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("waves", ["0", "1", "4"])
+@pytest.mark.parametrize("name", ["q", "k"])
+def test_delta_rule_long_vectors(name, waves, monkeypatch):
+    """Vectors whose squared length is beyond f32 have a unit vector of 0: two
+    such keys write nothing, such a query reads nothing."""
+    monkeypatch.setenv("KAITO_DELTA_WAVES", waves)
+    G, H, D, V = 1, 2, 64, 32
+    x, w, lay = _chunk_inputs([50], G, H, D, V, torch.bfloat16)
+    state = torch.zeros(2, 1, H, D, V, device="cuda")
+    x["qk".index(name)][[20, 27]] = 0.
+    want = ops.gated_delta_rule(*x, *w, state[0], *lay, 1e-6, 1e-5)
+    x["qk".index(name)][[20, 27]] = 1e20
+    got = ops.gated_delta_rule(*x, *w, state[1], *lay, 1e-6, 1e-5)
+    assert torch.equal(got, want) and torch.equal(state[1], state[0])
+    assert got.isfinite().all() and state.isfinite().all()
+
+
 # ------------------------------------------------------------------ RG-LRU
 
 @pytest.mark.parametrize("mode", MODES)
