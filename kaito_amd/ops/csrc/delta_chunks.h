@@ -18,14 +18,20 @@
 // the operands of the next chunk's products with S (the dims of K are taken in
 // that order), and the results of one product those of the next: S, U and the
 // right-hand side never change lanes. The next chunk's operands are under way
-// while one is multiplied. All in f32.
+// while one is multiplied.
+//
+// S and its products are f32. What is 16 x 16 is f64, from K K^T to U and the
+// read-out: an error there is every dim's at once, and the loop has no such sums.
+// All in f32, states came out up to 1.25 times as far from 64 bits as the loop's
+// and read-outs 1.19 times (f32 inputs, keys of one direction, cosine 0.9, decays
+// from 0.5 to 0.9; both 0.93 to 1.07 elsewhere). Now states 0.78 to 1.01 times
+// (1.07 with those keys at 0.5), read-outs 0.72 to 0.95 (1.04). It costs a tenth:
+// 4 prompts of 2048 tokens, 294 -> 328 us.
 //
 // The token-by-token loop is bound by its chain of sums, 830 cycles a token;
-// here it is instruction issue beside the matrix unit, about 250 with two waves
-// per SIMD (208 of matrix work per token and 16 columns). 64-bit addresses and
+// here it is instruction issue beside the matrix unit. 64-bit addresses and
 // clamps for every load cost a fifth more than buffers that end with their
-// sequence, and two terms per inverse nothing but time. 4 prompts of 2048
-// tokens, 16 heads of 128 x 128, 4 waves: loop 706 us, prep and chunks 20 + 225.
+// sequence. Times beside the loop's: run_chunks.
 #pragma once
 #include "mix_common.h"
 
@@ -35,6 +41,8 @@ namespace delta_chunks {
 constexpr int C = 16;               // tokens of a chunk
 // floats per (chunk, head): inverse times beta, read-out matrix, g, R_15
 constexpr int REC = 2 * C * C + 2 * C;
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 KAITO_DEV f32x4 mfma4(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -54,7 +62,8 @@ __global__ __launch_bounds__(64) void delta_chunk_prep_kernel(
     const int* __restrict__ cu, const int* __restrict__ slots, const int B,
     const int G, const int H, const float qk_eps) {
   constexpr int D = 16 * NJ, P = C + 4;
-  __shared__ __attribute__((aligned(16))) float kk[C][P], qk[C][P];
+  __shared__ __attribute__((aligned(16))) float qk[C][P];
+  __shared__ double kk[C][P];
   __shared__ __attribute__((aligned(16))) double A[4][C][C + 2];
   __shared__ __attribute__((aligned(16))) float dl[4][C], bl[4][C];
   const int id = blockIdx.x, g = blockIdx.y;
@@ -96,7 +105,8 @@ __global__ __launch_bounds__(64) void delta_chunk_prep_kernel(
   // k.k of the unit vectors, as the state has them; q.k of the rows, rounded last.
   // Sums in trees of one instruction's, for their rounding.
   const f32x4 zero{0.f, 0.f, 0.f, 0.f};
-  f32x4 ck[NJ], cq[NJ];
+  f32x4 cq[NJ];
+  f64x4 ck{0., 0., 0., 0.};
 #pragma unroll
   for (int j = 0; j < NJ; j++) {
     const int64_t at = (t * G + g) * D + 16 * j + 4 * hi;
@@ -105,25 +115,21 @@ __global__ __launch_bounds__(64) void delta_chunk_prep_kernel(
       *reinterpret_cast<float4_t*>(kn + at) = ku;
       *reinterpret_cast<float4_t*>(qn + at) = qv[j] * iq;
     }
-    f32x4 pk[4], pq[4];
+    f32x4 pq[4];
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      pk[e] = mfma4(ku[e], ku[e], zero);
+      ck = __builtin_amdgcn_mfma_f64_16x16x4f64(ku[e], ku[e], ck, 0, 0, 0);
       pq[e] = mfma4(qv[j][e], kv[j][e], zero);
     }
-    ck[j] = (pk[0] + pk[1]) + (pk[2] + pk[3]);
     cq[j] = (pq[0] + pq[1]) + (pq[2] + pq[3]);
   }
 #pragma unroll
   for (int w = 1; w < NJ; w *= 2)
 #pragma unroll
-    for (int j = 0; j < NJ; j += 2 * w) {
-      ck[j] += ck[j + w];
-      cq[j] += cq[j + w];
-    }
+    for (int j = 0; j < NJ; j += 2 * w) cq[j] += cq[j + w];
 #pragma unroll
   for (int r = 0; r < 4; r++) {
-    kk[4 * hi + r][lo] = ck[0][r];
+    kk[4 * r + hi][lo] = ck[r];
     // a row whose square is beyond f32 has a unit vector of 0
     const float ir = __shfl(iq, 4 * hi + r, 64);
     qk[4 * hi + r][lo] = ir == 0.f || ik == 0.f ? 0.f : cq[0][r] * ir * ik;
@@ -192,7 +198,7 @@ KAITO_DEV T load1(__amdgpu_buffer_rsrc_t r, const int at) {
 // Rows of a sequence are read and written as buffers that end with it: rows past
 // its last are 0, and not written.
 template <typename T, int NJ, int NW>
-__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void delta_chunk_kernel(
+__global__ __launch_bounds__(64 * NW, 2) void delta_chunk_kernel(
     float* __restrict__ o,                                 // [T, H, V]
     const float* __restrict__ qn, const float* __restrict__ kn,
     const float* __restrict__ rec, const T* __restrict__ v,
@@ -242,6 +248,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void delta_chunk_kernel(
   const int tat = 4 * hi * krow + (d0 + lo) * 4;
   const int vat = 4 * hi * vrow + (v0 + lo) * (int)sizeof(T);
   const int oat = 4 * hi * orow + (v0 + lo) * 4;
+  // the f64 product's row 4 e + hi is the other's 4 hi + e
+  const int irow = lo % 4 * 4 + lo / 4;
   auto fetch = [&](Operands& x, const int c) {
     const float* p = rp + (int64_t)c * H * REC;
     const int kc = kat + c * C * krow, tc = tat + c * C * krow;
@@ -251,8 +259,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void delta_chunk_kernel(
       x.k[j] = load4(kb, kc + j * 64);
       x.q[j] = load4(qb, kc + j * 64);
     }
-    x.inv = *reinterpret_cast<const float4_t*>(p + lo * C + 4 * hi);
-    x.ro = *reinterpret_cast<const float4_t*>(p + C * C + lo * C + 4 * hi);
+    x.inv = *reinterpret_cast<const float4_t*>(p + irow * C + 4 * hi);
+    x.ro = *reinterpret_cast<const float4_t*>(p + C * C + irow * C + 4 * hi);
     x.gam = *reinterpret_cast<const float4_t*>(p + 2 * C * C + 4 * hi);
     x.rest = *reinterpret_cast<const float4_t*>(p + 2 * C * C + C + 4 * hi);
 #pragma unroll
@@ -263,11 +271,12 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void delta_chunk_kernel(
         x.kt[j][e] = load1<float>(kb, tc + e * krow + j * 64);
     }
   };
-  // 16 x 16 matrix times 16 rows; short chains
-  auto times = [&](const float4_t m, const f32x4 y) {
-    const f32x4 zero{0.f, 0.f, 0.f, 0.f};
-    return mfma4(m[1], y[1], mfma4(m[0], y[0], zero)) +
-           mfma4(m[3], y[3], mfma4(m[2], y[2], zero));
+  // 16 x 16 matrix times 16 rows, on top of u
+  auto times = [&](const float4_t m, const f64x4 y, f64x4 u) {
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      u = __builtin_amdgcn_mfma_f64_16x16x4f64((double)m[e], y[e], u, 0, 0, 0);
+    return u;
   };
   auto chunk = [&](const Operands& x, const int c) {
     f32x4 ks[4], qs[4];             // short chains, for their rounding
@@ -300,39 +309,38 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void delta_chunk_kernel(
       }
     }
     const f32x4 zero{0.f, 0.f, 0.f, 0.f};
-    f32x4 rhs, out;
+    const f64x4 none{0., 0., 0., 0.};
+    f64x4 rhs, out;
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      rhs[e] = act_ld(&x.v[e]) - x.gam[e] * sk[e];
-      out[e] = x.gam[e] * sq[e];
+      rhs[e] = (double)act_ld(&x.v[e]) - (double)x.gam[e] * (double)sk[e];
+      out[e] = (double)x.gam[e] * (double)sq[e];
     }
-    f32x4 u = times(x.inv, rhs);
+    f64x4 u = times(x.inv, rhs, none);
     bool finite = true;
 #pragma unroll
-    for (int e = 0; e < 4; e++) finite &= fabsf(u[e]) < INFINITY;
+    for (int e = 0; e < 4; e++) finite &= fabs(u[e]) < (double)INFINITY;
     const bool mine = c % NW == wave;       // writes the chunk's output
     if (__all(finite)) {
-      if (mine)
-        out += times(x.ro, u);
+      if (mine) out = times(x.ro, u, out);
     } else {
       // A value that is not finite reaches the tokens before its own as 0
       // times it: token by token, later ones as 0.
-      const f32x4 base = out;
-      u = zero;
+      const f64x4 base = out;
       for (int i = 0; i < C; i++) {
-        f32x4 y;
+        f64x4 y;
 #pragma unroll
-        for (int e = 0; e < 4; e++) y[e] = 4 * hi + e <= i ? rhs[e] : 0.f;
-        y = times(x.inv, y);
+        for (int e = 0; e < 4; e++) y[e] = 4 * hi + e <= i ? rhs[e] : 0.;
+        y = times(x.inv, y, none);
 #pragma unroll
         for (int e = 0; e < 4; e++)
           if (4 * hi + e == i) u[e] = y[e];
       }
       for (int i = 0; i < C; i++) {
-        f32x4 y;
+        f64x4 y;
 #pragma unroll
-        for (int e = 0; e < 4; e++) y[e] = 4 * hi + e <= i ? u[e] : 0.f;
-        y = base + times(x.ro, y);
+        for (int e = 0; e < 4; e++) y[e] = 4 * hi + e <= i ? u[e] : 0.;
+        y = times(x.ro, y, base);
 #pragma unroll
         for (int e = 0; e < 4; e++)
           if (4 * hi + e == i) out[e] = y[e];
@@ -340,18 +348,32 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void delta_chunk_kernel(
     }
     const float all = __int_as_float(
         __builtin_amdgcn_readlane(__float_as_int(x.gam[3]), 48));   // g_15
-    const f32x4 w = u * x.rest;
+    f32x4 w;
 #pragma unroll
-    for (int j = 0; j < J; j++) S[j] *= all;
+    for (int e = 0; e < 4; e++) w[e] = (float)(u[e] * (double)x.rest[e]);
+    // the chunk's own sum first: S is rounded once, not with every term
+    constexpr int HALF = J > 4 ? 4 : J;     // registers
 #pragma unroll
-    for (int e = 0; e < 4; e++)
+    for (int j0 = 0; j0 < J; j0 += HALF) {
+      f32x4 add[HALF];
 #pragma unroll
-      for (int j = 0; j < J; j++) S[j] = mfma4(x.kt[j][e], w[e], S[j]);
+      for (int j = 0; j < HALF; j++) add[j] = zero;
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+#pragma unroll
+        for (int j = 0; j < HALF; j++)
+          add[j] = mfma4(x.kt[j0 + j][e], w[e], add[j]);
+#pragma unroll
+      for (int j = 0; j < HALF; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          S[j0 + j][e] = fmaf(S[j0 + j][e], all, add[j][e]);
+    }
     if (mine)
 #pragma unroll
       for (int e = 0; e < 4; e++)
         __builtin_amdgcn_raw_buffer_store_b32(
-            __float_as_uint(out[e]), ob, oat + c * C * orow + e * orow, 0, 0);
+            __float_as_uint((float)out[e]), ob, oat + c * C * orow + e * orow, 0, 0);
   };
 
   Operands x0, x1;

@@ -413,17 +413,15 @@ void launch_recurrence(int B, int H, int threads, size_t lds_bytes,
 
 // delta_chunks.h's path, or false where its forms do not fit. Whole op, us,
 // heads of 128 x 128, token loop / one wave / four waves per 16 columns:
-//   4 prompts of 2048 tokens, 16 heads    785 / 536 / 296
-//   1 of 8192                            2390 / 1847 / 657
-//   8 of 1024 (1024 groups of columns)    711 / 352 / 282
-//   16 of 512 (2048)                      537 / 235 / 279
-//   32 of 230                             354 / 240 / 285
-//   32 of 32                               61 / 59 / 67
-//   4 of 24, 1 of 16              23.4, 22.7 / 25.3, 22.6 / 23.6, 22.1
-// hence from 32 tokens per sequence on, four waves up to 1024 groups. 2-norm
-// error against f64, relative, f32 inputs of 300 tokens, loop and chunks:
-// read-out 1.62e-7 and 1.58e-7, state 1.11e-7 and 1.16e-7 (decays around 0.9);
-// 4.87e-7 and 4.45e-7, 1.14e-6 and 1.13e-6 (0.998).
+//   4 prompts of 2048 tokens, 16 heads    784 / 530 / 328
+//   1 of 8192                            2390 / 1783 / 720
+//   8 of 1024 (1024 groups of columns)    715 / 356 / 311
+//   16 of 512 (2048)                      547 / 240 / 297
+//   32 of 230                             348 / 239 / 290
+//   32 of 32                               63 / 59 / 69
+//   4 of 24, 1 of 16              22.2, 21.1 / 22.4, 20.9 / 22.3, 21.0
+// hence from 32 tokens per sequence on, four waves up to 1024 groups. Errors
+// against f64: delta_chunks.h.
 template <typename T>
 bool run_chunks(hipStream_t stream, const at::Tensor& q, const at::Tensor& k,
                 const at::Tensor& v, const at::Tensor& a, const at::Tensor& b,

@@ -230,6 +230,47 @@ def test_delta_rule_long_vectors(name, waves, monkeypatch):
     assert got.isfinite().all() and state.isfinite().all()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("decay", [-2.0, 0.0])
+def test_delta_chunks_keep_the_loops_precision(D, decay, monkeypatch):
+    """2-norm errors against f64 beside the token loop's, over 192 states, for
+    keys that share a direction, where sums between tokens cancel most. Both
+    forms round S once a step, so their errors are of one size: a tenth more is
+    beyond what 192 states scatter, f32 sums between tokens gave a quarter."""
+    B, L, G, H, V = 24, 64, 4, 8, 32
+    x, w, lay = _chunk_inputs([L] * B, G, H, D, V, torch.float32)
+    x[1] += 3 * torch.randn(B, 1, G, D, device="cuda").expand(
+        B, L, G, D).reshape(B * L, G, D)
+    w[0] += 2.0 + decay
+    q, k, v, gate, a, b = (t.double().view(B, L, *t.shape[1:]) for t in x)
+    a_log, dt_bias, norm_w = (t.double() for t in w)
+    unit = lambda t: (t / (t.square().sum(-1, True) + 1e-6).sqrt()
+                      ).repeat_interleave(H // G, 2)
+    q, k = unit(q) * D ** -0.5, unit(k)
+    d = torch.exp(-a_log.exp() * torch.nn.functional.softplus(a + dt_bias))
+    S = torch.zeros(B, H, D, V, dtype=O.F64, device="cuda")
+    want = torch.empty(B, L, H, V, dtype=O.F64, device="cuda")
+    for t in range(L):
+        S = S * d[:, t, :, None, None]
+        u = torch.sigmoid(b[:, t, :, None]) * (
+            v[:, t] - (S * k[:, t, :, :, None]).sum(2))
+        S = S + k[:, t, :, :, None] * u[:, :, None]
+        o = (S * q[:, t, :, :, None]).sum(2)
+        want[:, t] = o / (o.square().mean(-1, True) + 1e-5).sqrt()
+    want = want * norm_w * gate * torch.sigmoid(gate)
+
+    def errors(waves):
+        monkeypatch.setenv("KAITO_DELTA_WAVES", waves)
+        state = torch.zeros(B, H, D, V, device="cuda")
+        out = ops.gated_delta_rule(*x, *w, state, *lay, 1e-6, 1e-5)
+        return (out.view_as(want) - want).norm(), (state - S).norm()
+    loop = errors("0")
+    for waves in ("1", "4"):
+        for mine, its in zip(errors(waves), loop):
+            assert mine <= 1.1 * its
+
+
 # ------------------------------------------------------------------ RG-LRU
 
 @pytest.mark.parametrize("mode", MODES)
