@@ -442,17 +442,19 @@ bool run_chunks(hipStream_t stream, const at::Tensor& q, const at::Tensor& k,
     return row >= 0 && (T_ + dc::C) * row < 1LL << 31;
   };
   // KAITO_DELTA_WAVES=1|4 pins the waves, 0 the token loop (A/B runs, tests)
-  const char* pin = getenv("KAITO_DELTA_WAVES");
+  const char* env = getenv("KAITO_DELTA_WAVES");
+  const int pin = env ? atoi(env) : -1;
+  TORCH_CHECK(!env || pin == 0 || pin == 1 || pin == 4,
+              "KAITO_DELTA_WAVES: 0, 1 or 4");
   if ((D != 64 && D != 128) || V % 16 || T_ < 32 * (int64_t)B ||
       !fours(q) || !fours(k) || !reach(G * (int64_t)D * 4) ||
       !reach(H * (int64_t)V * 4) || !reach(v.stride(0) * v.element_size()) ||
-      (pin && atoi(pin) == 0) ||
-      getenv("KAITO_DELTA_ROWS_PER_LANE"))
+      pin == 0 || getenv("KAITO_DELTA_ROWS_PER_LANE"))
     return false;
   const int64_t chunks = T_ / dc::C + B;
   at::Tensor rec = at::empty({chunks, H, dc::REC}, qn.options());
   const int64_t groups = (int64_t)B * H * (V / 16);
-  const int nw = pin ? atoi(pin) : groups > 1024 ? 1 : 4;
+  const int nw = env ? pin : groups > 1024 ? 1 : 4;
 #define KAITO_DELTA_CHUNKS(NJ_, NW_)                                         \
   if (nw == NW_)                                                             \
     hipLaunchKernelGGL((dc::delta_chunk_kernel<T, NJ_, NW_>),                \

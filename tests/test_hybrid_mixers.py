@@ -271,6 +271,16 @@ def test_delta_chunks_keep_the_loops_precision(D, decay, monkeypatch):
             assert mine <= 1.1 * its
 
 
+@pytest.mark.gpu
+def test_delta_waves_that_do_not_exist(monkeypatch):
+    x, w, lay = _chunk_inputs([50], 1, 2, 64, 32, torch.float32)
+    state = torch.zeros(1, 2, 64, 32, device="cuda")
+    for waves in ("2", "8", "-4"):
+        monkeypatch.setenv("KAITO_DELTA_WAVES", waves)
+        with pytest.raises(RuntimeError, match="KAITO_DELTA_WAVES"):
+            ops.gated_delta_rule(*x, *w, state, *lay, 1e-6, 1e-5)
+
+
 # ------------------------------------------------------------------ RG-LRU
 
 @pytest.mark.parametrize("mode", MODES)
