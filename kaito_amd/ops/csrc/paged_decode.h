@@ -32,9 +32,11 @@
 //
 // BIASED is the form of the hybrid stacks' windowed layers
 // (window_attention.hip): scores with a tanh cap and a distance penalty, the
-// mask on keys and not on values. log1pf in place of the penalty's logf took 5
-// us of 25 (32 rows of a 1024-key window); the argument's rounding, 6e-8, is
-// that of the score it is taken from.
+// mask on keys and not on values. The penalty is a log1pf, whose argument may be
+// far below 1 (ln(1 + 1e-6) by logf is off by a twentieth); on every lane, unused
+// columns too, it took 4 us of 23 (32 rows of a 1024-key window, 4 heads per kv
+// head), shared out over the lanes and read back from LDS none, with 8 heads 2 of
+// 16.
 //
 // Cache layout: [num_blocks, KV_HEADS, BLOCK_SIZE, HEAD_DIM] bf16 | e4m3.
 #pragma once
@@ -139,6 +141,9 @@ void paged_decode_kernel(const DecodeArgs a) {
   constexpr int LV = KT * CV / 64;  // V chunks per lane and tile
   __shared__ __attribute__((aligned(128))) short lds_v[NW][KT * D];
   __shared__ float s_m[NW][16], s_l[NW][16];
+  // BIASED: penalties of a wave's tile, heads by keys
+  constexpr int PH = BIASED ? D <= 128 ? 8 : 4 : 1;
+  __shared__ __attribute__((aligned(16))) float s_pen[BIASED ? NW : 1][PH * KT];
 
   const int seq = blockIdx.x / a.KH, kvh = blockIdx.x % a.KH;
   const int lane = threadIdx.x & 63;
@@ -175,10 +180,16 @@ void paged_decode_kernel(const DecodeArgs a) {
   }
   constexpr float NONE = BIASED ? -INFINITY : -1e30f;
   float m = NONE, l = 0.f;
-  float r1 = 0.f, r2 = 0.f;
+  // Penalties are evaluated once for each head and key, and not by the lanes of
+  // unused columns too: lane % 32 is the key, its heads are lane / 32 + 2 j.
+  float r1[PH / 2 + 1], r2[PH / 2 + 1];
   if (BIASED && a.r1) {
-    r1 = a.r1[kvh * a.G + min(lo, a.G - 1)];
-    r2 = a.r2[kvh * a.G + min(lo, a.G - 1)];
+#pragma unroll
+    for (int j = 0; j < PH / 2; j++) {
+      const int head = kvh * a.G + min((lane >> 5) + 2 * j, a.G - 1);
+      r1[j] = a.r1[head];
+      r2[j] = a.r2[head];
+    }
   }
   f32x4 o[DT];
 #pragma unroll
@@ -267,13 +278,19 @@ void paged_decode_kernel(const DecodeArgs a) {
 #pragma unroll
         for (int i = 0; i < 8; i++)
           s[i / 4][i % 4] = a.cap * tanhf(s[i / 4][i % 4] / a.cap);
-      if (a.r1)
+      if (a.r1) {
+        float* pen = s_pen[wave];
+        const float dist = (float)(seq_len - 1 - key0 - (lane & 31));
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-          const int key = key0 + 16 * (i / 4) + 4 * hi + i % 4;
-          s[i / 4][i % 4] -=
-              r1 * logf(fmaf(r2, (float)(seq_len - 1 - key), 1.f));
-        }
+        for (int j = 0; j < PH / 2; j++)
+          if (2 * j < a.G) pen[lane + 64 * j] = r1[j] * log1pf(r2[j] * dist);
+        __builtin_amdgcn_wave_barrier();
+        const float* mine = pen + min(lo, a.G - 1) * KT + 4 * hi;
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+          s[i] -= *reinterpret_cast<const f32x4*>(mine + 16 * i);
+        __builtin_amdgcn_wave_barrier();
+      }
     }
     auto seen = [&](const int i, const int r) {
       const int key = key0 + 16 * i + 4 * hi + r;

@@ -134,6 +134,33 @@ def test_rglru_very_long_steps(T):
     assert ((one - parts).abs() <= 2.0 ** -14 * (1 + parts.abs())).all()
 
 
+@pytest.mark.parametrize("H,G,D", [(3, 3, 64), (8, 1, 128), (6, 2, 128),
+                                   (8, 2, 256)])
+@pytest.mark.parametrize("r2", [1e-7, 3e-6, 1e-3])
+def test_window_decode_small_penalties(H, G, D, r2):
+    """r1 ln(1 + r2 distance) with r2 distance far below 1 and a large r1: the
+    logarithm keeps f32's relative precision. Two equal keys are in the window,
+    so that the penalty of the older one alone decides its share."""
+    n, BS = 1001, 16
+    pages = -(-n // BS)
+    kc = torch.zeros(pages, G, BS, D, device=DEV, dtype=torch.bfloat16)
+    vc = torch.zeros_like(kc)
+    vc[(n - 2) // BS, :, (n - 2) % BS] = 1.
+    table = torch.arange(pages, dtype=torch.int32, device=DEV)[None]
+    q = torch.ones(1, H, D, device=DEV, dtype=torch.bfloat16)
+    r1 = torch.linspace(1, 8, H, device=DEV) / r2
+    r2 = torch.full((H,), r2, device=DEV)
+    out = ops.window_attention(
+        q, kc, vc, table, torch.zeros(1, dtype=torch.int32, device=DEV),
+        torch.tensor([n - 1], device=DEV), 1.0, 0.0, r1, r2, 2)
+    ref = torch.sigmoid(-r1.double() * torch.log1p(r2.double()))
+    # penalties up to 8, of three roundings: shares within 8 * 3 * 2^-24; then
+    # one rounding to bf16
+    err = (out[0, :, 0].double() - ref).abs()
+    assert (err <= (2.0 ** -8 + 2e-6) * ref).all(), err / ref
+    assert (out == out[..., :1]).all()
+
+
 @pytest.mark.parametrize("T", [1, 31, 32, 33, 1100])
 @pytest.mark.parametrize("B,bw", [(1, 64), (3, 128), (16, 128), (2, 32)])
 def test_rglru_gates(T, B, bw):
