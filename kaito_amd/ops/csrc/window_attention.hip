@@ -869,10 +869,11 @@ void window_attention(at::Tensor out, at::Tensor q, at::Tensor k_cache,
   auto stream0 = at::hip::getCurrentHIPStream();
   // Matrix-core decode (paged_decode.h): softmax over bf16 pages of 16 with any
   // window, cap, penalty, sinks and head gates. us, decode kernel below and
-  // now, 16 heads of 128 on 4 kv heads, window 1024: 32 rows of 2049 keys 39.7
-  // and 19.6, 8 of up to 2000 31.5 and 17.1, 96 of 600 69 and 23, 500 of 250 136
-  // and 44, one of 300 14.3 and 8.7; where it gains least, one head per kv
-  // head: 96 of 600, 8 heads of 128, 40.8 and 38.9, 4 of 256 41.9 and 40.7.
+  // here, 16 heads of 128 on 4 kv heads, window 1024, penalties: 32 rows of 2000
+  // keys 38.5 and 20.9, 8 of 1000 30.6 and 17.9, 96 of 600 69 and 25, 500 of 250
+  // 143 and 47, one of 300 14.6 and 10.9; where it gains least, one head per kv
+  // head: 96 of 600, 8 heads of 128, 40.2 and 40.1, 4 of 256 41.7 and 41.8; one
+  // row of 40, 8 heads per kv head, 8.9 and 9.0.
   const int rep = H / G;
   if (q.dtype() == at::kBFloat16 && D == V && BS == 16 &&
       (D == 64 || D == 128 || D == 256) && rep <= (D == 256 ? 4 : 8) &&
