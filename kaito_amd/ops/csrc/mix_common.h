@@ -25,6 +25,17 @@ template <> KAITO_DEV void act_st<bf16_act>(bf16_act* p, float v) {
   p->v = f32_to_bf16(v);
 }
 
+// v as three bf16 terms, largest first, to its last bit. An infinity or a NaN is
+// the first alone; finite values beyond the largest bf16 stay finite.
+KAITO_DEV void bf16_terms(const float v, __bf16 (&t)[3]) {
+  constexpr float MOST = 0x1.fep127f;
+  const bool finite = fabsf(v) < INFINITY;
+  t[0] = (__bf16)(finite ? fminf(fmaxf(v, -MOST), MOST) : v);
+  const float rest = finite ? v - (float)t[0] : 0.f;
+  t[1] = (__bf16)rest;
+  t[2] = (__bf16)(rest - (float)t[1]);
+}
+
 KAITO_DEV float4_t act_ld4(const float* p) {
   return *reinterpret_cast<const float4_t*>(p);
 }

@@ -86,12 +86,10 @@ __global__ __launch_bounds__(64 * GATE_WAVES, 2) void rglru_gates_kernel(
   for (int k = 0; k < KS; k++)
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-      float v = wp[(16 * k + i) * N];
+      __bf16 t[3];
+      bf16_terms(wp[(16 * k + i) * N], t);
 #pragma unroll
-      for (int n = 0; n < 3; n++) {
-        b[n][k][i] = (__bf16)v;
-        v -= (float)b[n][k][i];
-      }
+      for (int n = 0; n < 3; n++) b[n][k][i] = t[n];
     }
   const float c0 = bias[blk * N + n0 + lr];
   for (int t = blockIdx.z; t < tiles; t += gridDim.z) {

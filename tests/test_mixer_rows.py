@@ -199,6 +199,32 @@ def test_rglru_closed_output_gate(z):
     assert out.abs().max().item() < 1e-30
 
 
+@pytest.mark.parametrize("bw", [64, 128])
+def test_rglru_gates_large_weights(bw):
+    """Weights that are infinite or beyond the largest bf16, with rows that are
+    finite, infinite and NaN, as the f32 product has them."""
+    torch.manual_seed(bw)
+    T, B = 40, 2
+    u = (torch.rand(T, B * bw, device=DEV) / 4 + 0.01).to(torch.bfloat16)
+    u[3, 7], u[4, 9], u[5, 11] = float("inf"), -float("inf"), float("nan")
+    w = torch.randn(B, bw, 2 * bw, device=DEV)
+    big = torch.finfo(torch.float32).max
+    w[0, 9, 1], w[0, 20, 2], w[1, 5, 3] = float("inf"), -float("inf"), \
+        float("nan")
+    w[0, 30, 4], w[1, 30, 5], w[1, 31, 6] = big, -big, 3.395e38
+    b = torch.randn(B, 1, 2 * bw, device=DEV)
+    ub = u.reshape(T, B, bw).transpose(0, 1).contiguous()
+    ref = torch.baddbmm(b.double(), ub.double(), w.double())
+    out = ops.rglru_gates(u, w, b)
+    fine = ref.isfinite()
+    assert torch.equal(out.isnan(), ref.isnan())
+    assert torch.equal(out.double()[ref.isinf()], ref[ref.isinf()])
+    size = torch.baddbmm(b.double().abs(), ub.double().abs(), w.double().abs())
+    err = (out.double() - ref).abs()
+    # an f32 sum of 3 bw products, every rounding at its worst
+    assert (err[fine] <= 3 * bw * 2.0 ** -24 * size[fine]).all()
+
+
 @pytest.mark.parametrize("D,H,G", [(64, 3, 3), (128, 8, 1), (128, 6, 2),
                                    (256, 8, 2)])
 @pytest.mark.parametrize("window,cap,bias,sink,gated",
