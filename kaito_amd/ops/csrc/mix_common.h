@@ -25,15 +25,19 @@ template <> KAITO_DEV void act_st<bf16_act>(bf16_act* p, float v) {
   p->v = f32_to_bf16(v);
 }
 
-// v as three bf16 terms, largest first, to its last bit. An infinity or a NaN is
-// the first alone; finite values beyond the largest bf16 stay finite.
+// v as three bf16 terms, largest first, to its last bit: 8 bits each, cut off, so
+// that no finite value's term is infinite. An infinity or a NaN is the first alone.
 KAITO_DEV void bf16_terms(const float v, __bf16 (&t)[3]) {
-  constexpr float MOST = 0x1.fep127f;
-  const bool finite = fabsf(v) < INFINITY;
-  t[0] = (__bf16)(finite ? fminf(fmaxf(v, -MOST), MOST) : v);
-  const float rest = finite ? v - (float)t[0] : 0.f;
-  t[1] = (__bf16)rest;
-  t[2] = (__bf16)(rest - (float)t[1]);
+  auto top = [](const float f) {
+    return __uint_as_float(__float_as_uint(f) & 0xffff0000u);
+  };
+  // NaN: quiet, which is a bit of the upper half
+  const float a = top(__builtin_canonicalizef(v));
+  const float rest = fabsf(v) < INFINITY ? v - a : 0.f;
+  const float b = top(rest);
+  t[0] = (__bf16)a;
+  t[1] = (__bf16)b;
+  t[2] = (__bf16)(rest - b);
 }
 
 KAITO_DEV float4_t act_ld4(const float* p) {

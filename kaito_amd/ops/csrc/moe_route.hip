@@ -274,13 +274,10 @@ KAITO_DEV void gate_terms(const float* w, skinny::hbf16x8 (&b)[3]) {
   const float4_t hi = *reinterpret_cast<const float4_t*>(w + 4);
 #pragma unroll
   for (int i = 0; i < 8; i++) {
-    float v = i < 4 ? lo[i & 3] : hi[i & 3];
+    __bf16 t[3];
+    bf16_terms(i < 4 ? lo[i & 3] : hi[i & 3], t);
 #pragma unroll
-    for (int n = 0; n < 3; n++) {
-      b[n][i] = (__bf16)v;
-      v -= (float)b[n][i];
-      if (!(fabsf(v) < INFINITY)) v = 0.f;  // behind an infinity, a NaN
-    }
+    for (int n = 0; n < 3; n++) b[n][i] = t[n];
   }
 }
 

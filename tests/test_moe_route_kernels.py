@@ -230,3 +230,22 @@ def test_choice_of_16_rows_not_finite(dtype):
     # weights: logits of unit size, sums of 256 products in another order
     torch.testing.assert_close(long[1][:512], short[1], rtol=1e-5, atol=1e-6,
                                equal_nan=True)
+
+
+@pytest.mark.gpu
+def test_choice_of_16_rows_large_router():
+    """f32 weights beyond the largest bf16 whose logits are finite."""
+    torch.manual_seed(4)
+    x = torch.randn(600, 256, device=DEV).to(torch.bfloat16)
+    gate = torch.randn(8, 256, device=DEV) / 16
+    x[:, 9] = x[:, 9].clamp(-0.5, 0.5)
+    gate[5, 9], gate[2, 9] = torch.finfo(torch.float32).max, -3.4e38
+    a = (3, 8, 1, 1, False, 1.0, "logits")
+    topi, topw, _ = ops.moe_gate_route(x, gate, None, *a)
+    want = R.moe_route((x.double() @ gate.double().T).float(), None, *a)
+    assert topw.isfinite().all()
+    assert torch.equal(topi, want[0])
+    # the products of 256 terms, every rounding at its worst
+    size = (x.double().abs() @ gate.double().abs().T).float().gather(
+        1, topi.long())
+    assert ((topw - want[1]).abs() <= 768 * 2.0 ** -24 * size).all()
