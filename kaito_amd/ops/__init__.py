@@ -608,6 +608,22 @@ def _gate_short(x, gate) -> bool:
     return T <= 512 and T * gate.size(0) <= 8192
 
 
+def _gate_long(T: int, N: int, H: int, f32: bool) -> bool:
+    """Whether tiles of 16 rows form the logits of a long step. us, library and
+    choice, and tiles; T rows, N outputs, rows of H. An f32 router saves the cast
+    of the rows: 8 outputs 15.7, 8.4 and 38.0, 14.4 (600 and 8192 rows of 2048),
+    32 outputs 16.5, 13.0 and 37.7, 26.4; beyond 16 outputs and H of 3072 only from
+    1024 rows on (32 x 7168: 27.7, 34.3 at 257, 33.8, 34.6 at 600, 38.2, 35.0 at
+    1024). A bf16 one has to be small: 8 outputs 9.1, 7.0 and 14.7, 10.8, of 4096
+    9.8, 9.7 and 19.1, 17.9; 16 outputs 9.2, 7.6 and 15.0, 12.1, of 2880 11.3, 9.0,
+    of 3072 9.2, 9.3, of 4096 9.8, 11.0; 32 outputs of 2048 15.7, 16.0 at 8192."""
+    if H % 32 or N > 32:
+        return False
+    if f32:
+        return N <= 16 or H <= 3072 or T >= 1024
+    return N <= 16 and H <= 2880 or N <= 8 and H <= 4096
+
+
 def _gate_in_route(x, gate) -> bool:
     return (x.is_cuda and x.dtype == torch.bfloat16 and gate.size(0) <= 32
             and gate.is_contiguous()
@@ -646,19 +662,15 @@ def moe_gate_route(x, gate, correction, top: int, n_real: int,
                    scale: float = 1.0, mode: str = "softmax"):
     """moe_route of the logits x gate^T, formed in f32. One launch for short
     steps and narrow routers: a workgroup per row reads the whole router, 8
-    outputs after one another, so that wider ones and longer steps take tiles of
-    16 rows or leave the product to the library (us, one launch and two; rows of 2048 and 7168, bf16
-    router: 8 outputs 5.1, 9.4 and 6.1, 13.2 at 32 rows, 5.7, 9.5 and 7.0, 11.4
-    at 512; 32 outputs 9.2, 9.6 and 12.2, 13.7 at 32 rows, 9.6, 9.6 and 13.3,
-    13.7 at 256, 10.3, 9.7 and 16.0, 13.9 at 512; 48 outputs 12.0, 9.5 and
-    16.5, 13.6 at 32). Tiles up to 32 outputs: an f32 router saves the cast of
-    the rows (8192 rows, 8 outputs: 16.3, 38.0 and 38.2, 103; 32 outputs 27.7,
-    38.3), a bf16 one has to be narrow (8 outputs 11.7, 15.5 and 27.4, 26.4; 32
-    outputs 16.0, 15.7; 1024 rows of 7168 to 32 outputs 23.0, 14.6)."""
+    outputs after one another, so that wider ones and longer steps take tiles
+    of 16 rows (_gate_long) or leave the product to the library. us, one launch
+    and two; rows of 2048 and 7168, bf16 router: 8 outputs 5.1, 9.4 and 6.1,
+    13.2 at 32 rows, 5.7, 9.5 and 7.0, 11.4 at 512; 32 outputs 9.2, 9.6 and
+    12.2, 13.7 at 32 rows, 9.6, 9.6 and 13.3, 13.7 at 256, 10.3, 9.7 and 16.0,
+    13.9 at 512; 48 outputs 12.0, 9.5 and 16.5, 13.6 at 32."""
     T = x.size(0)
-    H = x.size(1)
-    long = H % 32 == 0 and (gate.dtype == torch.float32
-                            or gate.size(0) <= 16 and H <= 4096)
+    long = _gate_long(T, gate.size(0), x.size(1),
+                      gate.dtype == torch.float32)
     if (long or _gate_short(x, gate)) and _gate_in_route(x, gate):
         topi, topw, w_id = _route_out(T, top, x.device)
         _K.moe_gate_route(topi, topw, w_id, x, gate, _none(correction, x),

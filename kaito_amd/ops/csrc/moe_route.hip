@@ -259,10 +259,10 @@ __global__ __launch_bounds__(256) void moe_gate_route_kernel(
 // and rows need no cast. Bound by latency up to 2048 rows, behind them by reading
 // rows and router through L2; a workgroup per row reads the router 16 times as
 // often (us, product by the library and choice -> here, rows of 2048, 8 outputs:
-// bf16 router 9.7 -> 7.6 at 600 rows, 15.5 -> 11.7 at 8192 (row by row 20.4); f32
-// 16.3 -> 9.5 and 38.0 -> 16.3 (27.2)). Loads of a round's router ahead of its
-// products cost f32 routers half their waves: 19.3. Error of the weights against
-// f64 logits at 8192 rows: 1.8e-7, of the library's 3.0e-7 and 6.6e-7.
+// bf16 router 9.1 -> 7.0 at 600 rows, 14.7 -> 10.8 at 8192 (row by row 20.4); f32
+// 15.7 -> 8.4 and 38.0 -> 14.4 (27.2)). Loads of a round's router ahead of its
+// products cost f32 routers half their waves: a fifth more. Error of the weights
+// against f64 logits at 8192 rows: 1.8e-7, of the library's 3.0e-7 and 6.6e-7.
 constexpr int GATE_ROWS = 16, GATE_STEPS = 4;
 
 // the terms of 8 elements of the router, largest first

@@ -249,3 +249,15 @@ def test_choice_of_16_rows_large_router():
     size = (x.double().abs() @ gate.double().abs().T).float().gather(
         1, topi.long())
     assert ((topw - want[1]).abs() <= 768 * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.parametrize("T,N,H,f32,tiles", [
+    (600, 8, 2048, False, True), (8192, 16, 2880, False, True),
+    (600, 8, 4096, False, True), (600, 16, 4096, False, False),
+    (2048, 16, 3072, False, False), (8192, 32, 2048, False, False),
+    (257, 32, 2048, True, True), (600, 16, 8192, True, True),
+    (512, 32, 4096, True, False), (600, 24, 8192, True, False),
+    (1024, 32, 8192, True, True), (8192, 8, 2040, True, False)])
+def test_which_steps_choose_by_16_rows(T, N, H, f32, tiles):
+    """The sides of the line on which either was measured to be faster."""
+    assert ops._gate_long(T, N, H, f32) == tiles
