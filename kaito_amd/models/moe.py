@@ -233,7 +233,8 @@ class MoEMLP(nn.Module):
         topi, topw, w_id = chosen if chosen is not None else self._choose(x)
         kernels = self._kernels_for(x)
         # decode-sized steps: every expert finds its rows by itself
-        pairs = kernels == "streamed" and topi.numel() <= ops.PAIRS_MAX
+        pairs = kernels == "streamed" and ops.moe_pairs_pay(
+            topi.numel(), self.e_local, self.w_gate_up.size(1), x.size(1))
         pos = None
         if not pairs:
             # identity outputs sort behind every expert's rows

@@ -505,6 +505,21 @@ def moe_down_rows(y, act, w_down, offsets, e_base: int, n_local_experts: int,
 PAIRS_MAX = 256       # pairs of a step whose experts find their own rows
 
 
+def moe_pairs_pay(pairs: int, n_local: int, up_rows: int, H: int) -> bool:
+    """Whether a step's local experts, of up_rows x H, find their rows among
+    the pairs. The sort's launch is saved, and every workgroup of 16 weight rows,
+    of hit experts or not, scans them. us a layer, sorted and by pairs: 8 experts
+    of 2048 x 2048, top 2, 1 to 128 tokens (2 to 256 pairs) 19.9, 18.6; 26.9,
+    22.6; 43.0, 39.9 (16); 73.8, 71.8; 16 of 2048 x 1024, top 4, 1 to 64 tokens
+    19.9, 20.5; 31.2, 25.8; 45.5, 44.4; 53.0, 53.5; 16 of 2880 x 2880 (8640
+    workgroups) 45.6, 44.5; 127, 125; 183, 181. More workgroups: 8 of 4096 x 14336
+    (16384) 117, 121 and 179, 185 at 1 and 2 tokens, 24 of 2048 x 1024 19.8, 21.1
+    at 1, 32 of 2048 x 2048 (12288) 21.0, 25.2, 128 of 2048 x 768, top 8, 32.4,
+    41.4 and 191, 221 at 1 and 32."""
+    return pairs <= PAIRS_MAX and n_local <= 16 \
+        and n_local * (up_rows + H) <= 16 * 8704
+
+
 def moe_up_pairs(act, x, w_gate_up, topi, n_experts: int, e_base: int,
                  n_local_experts: int, bias=None, act_mode: int = 0,
                  act_limit: float = 7.0) -> None:

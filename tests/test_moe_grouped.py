@@ -255,3 +255,13 @@ def test_norm_and_choice(T, H, N, f32):
     assert (xn != ref).float().mean() < 0.02
     for a, b in zip(chosen, ops.moe_gate_route(xn, gate, None, 2, N)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("pairs,n_local,ff,H,pay", [
+    (2, 8, 2048, 2048, True), (256, 8, 2048, 2048, True),
+    (257, 8, 2048, 2048, False), (4, 16, 2880, 2880, True),
+    (2, 8, 14336, 4096, False), (4, 24, 1024, 2048, False),
+    (2, 32, 2048, 2048, False), (256, 128, 768, 2048, False)])
+def test_which_steps_go_by_pairs(pairs, n_local, ff, H, pay):
+    """The sides of the line on which either was measured to be faster."""
+    assert ops.moe_pairs_pay(pairs, n_local, 2 * ff, H) == pay
