@@ -507,17 +507,23 @@ PAIRS_MAX = 256       # pairs of a step whose experts find their own rows
 
 def moe_pairs_pay(pairs: int, n_local: int, up_rows: int, H: int) -> bool:
     """Whether a step's local experts, of up_rows x H, find their rows among
-    the pairs. The sort's launch is saved, and every workgroup of 16 weight rows,
-    of hit experts or not, scans them. us a layer, sorted and by pairs: 8 experts
-    of 2048 x 2048, top 2, 1 to 128 tokens (2 to 256 pairs) 19.9, 18.6; 26.9,
-    22.6; 43.0, 39.9 (16); 73.8, 71.8; 16 of 2048 x 1024, top 4, 1 to 64 tokens
-    19.9, 20.5; 31.2, 25.8; 45.5, 44.4; 53.0, 53.5; 16 of 2880 x 2880 (8640
-    workgroups) 45.6, 44.5; 127, 125; 183, 181. More workgroups: 8 of 4096 x 14336
-    (16384) 117, 121 and 179, 185 at 1 and 2 tokens, 24 of 2048 x 1024 19.8, 21.1
-    at 1, 32 of 2048 x 2048 (12288) 21.0, 25.2, 128 of 2048 x 768, top 8, 32.4,
-    41.4 and 191, 221 at 1 and 32."""
-    return pairs <= PAIRS_MAX and n_local <= 16 \
-        and n_local * (up_rows + H) <= 16 * 8704
+    the pairs. The sort's launch is saved, and every workgroup of 16 weight rows
+    scans them, of experts that no token chose too. us a layer, sorted and by
+    pairs: 8 experts of 2048 x 2048 (3072 workgroups), top 2, 19.9, 18.5 at 1
+    token, 26.5, 22.6 at 2, 43.0, 39.9 at 16, 73.9, 71.6 at 128; 12 of 2048 x 1408
+    (3648), top 3, 21.7, 19.2 at 1. More workgroups need more pairs: 8 of 4096 x
+    4096 (6144) 43.7, 44.8 at 1, 61.0, 65.1 at 2, 112.4, 112.6 at 8, 127.2, 125.8
+    at 12; with H of 2048, where they stay for several tiles, 16 of 2048 x 1024
+    (4096), top 4, 19.9, 20.5 at 1, 28.6, 25.7 at 2, 16 of 2048 x 2048 (6144) 33.2,
+    34.6 at 3, 36.8, 31.3 at 4. 8 of 4096 x 14336 (16384) 118, 122 and 179, 185 at
+    1 and 2; 32 of 2048 x 2048 (12288) 21.2, 25.3 at 1; 24 of 2048 x 1024, top 4,
+    19.9, 20.9 at 1; 128 of 2048 x 768, top 8, 32.5, 41.2 and 191, 221 at 1 and
+    32."""
+    workgroups = n_local * (up_rows + H) // 16
+    if pairs > PAIRS_MAX or n_local > 16 or workgroups > 8704:
+        return False
+    return workgroups <= 3840 or \
+        pairs >= (n_local // 2 if H == 2048 else 2 * n_local)
 
 
 def moe_up_pairs(act, x, w_gate_up, topi, n_experts: int, e_base: int,

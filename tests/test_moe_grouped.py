@@ -259,7 +259,9 @@ def test_norm_and_choice(T, H, N, f32):
 
 @pytest.mark.parametrize("pairs,n_local,ff,H,pay", [
     (2, 8, 2048, 2048, True), (256, 8, 2048, 2048, True),
-    (257, 8, 2048, 2048, False), (4, 16, 2880, 2880, True),
+    (257, 8, 2048, 2048, False), (32, 16, 2880, 2880, True),
+    (2, 8, 4096, 4096, False), (24, 8, 4096, 4096, True),
+    (4, 16, 1024, 2048, False), (8, 16, 1024, 2048, True),
     (2, 8, 14336, 4096, False), (4, 24, 1024, 2048, False),
     (2, 32, 2048, 2048, False), (256, 128, 768, 2048, False)])
 def test_which_steps_go_by_pairs(pairs, n_local, ff, H, pay):
