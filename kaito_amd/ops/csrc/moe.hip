@@ -270,23 +270,29 @@ void launch_rows(const StreamArgs& a, int64_t E_local, int64_t pairs,
   const bool two = pairs > 12 * E;
   // With K = 2048 and up to 32 experts, workgroups that stay
   // (skinny::stream_tiles), from three tiles per CU on of the experts that are
-  // likely hit. us, per tile and staying: 8 experts of 2048 x 2048, up 17.6 and
-  // 16.1, 26.1 and 24.2, 28.4 and 24.4, 35.7 and 25.7 at 4, 16, 32 and 64
-  // tokens of two experts; down 16.1 and 14.0, 16.9 and 14.2, 21.5 and 16.0 at
-  // 16 to 64, 10.7 and 11.4 at 4 (672 tiles); one token 8.4 and 10.7, 7.2 and
-  // 8.4. 32 of 2048 x 768, top 8, up 28.1 and 26.5 at 4, 51.9 and 37.4 at 64;
-  // 64 of 2048 x 1408, top 6, 39.5 and 53.8 at 4, 99 and 105 at 16: an equal
-  // share per expert leaves CUs idle when some of many are not hit, and equal
-  // runs over those that are cost more to find than they give (26.0 and 15.5
-  // for the 32 tokens). Wider K streams as fast in tiles of their own: 8 of
-  // 28672 x 4096, 16 tokens, 275 and 282.
+  // likely hit, where equal shares of them come out even. us, per tile and
+  // staying. By pairs, 8 experts of 2048 x 2048, top 2, up 15.0 and 12.7, 20.0 and
+  // 18.8, 28.5 and 24.3, 30.1 and 24.4, 40.3 and 25.7 at 2, 4, 16, 32 and 64
+  // tokens; down 14.2 and 12.6, 17.0 and 13.9, 21.5 and 15.3 at 6, 32 and 64; 16
+  // experts up 23.3 and 18.7 at 4, 49.8 and 41.9 at 32, but 21.8 and 24.6 at 3: 6
+  // pairs, 42 workgroups each for 256 tiles. Sorted, 32 of 2048 x 768, top 8, up
+  // 39.5 and 33.7 at 32 tokens (all hit), 31.3 and 30.2 at 8 (0.87 of them), 25.2
+  // and 25.3 at 4 (0.64), 18.3 and 21.4 at 2 (0.4); 8 of 2048 x 8192 78.2 and 80.6
+  // at 8 (0.88), 93.2 and 88.1 at 24: equal shares leave CUs idle when experts are
+  // not hit, and equal runs over those that are cost more to find than they give
+  // (26.0 and 15.5 for the 32 tokens). 64 of 2048 x 1408, top 6, 39.5 and 53.8 at
+  // 4, 99 and 105 at 16. Wider K streams as fast in tiles of their own: 8 of 28672 x
+  // 4096, 16 tokens, 275 and 282.
   const double hit =
       E_local * (1.0 - std::pow(1.0 - 1.0 / E, (double)pairs));
-  if (a.K == 2048 && E_local <= 32 && hit * grid.x >= 768) {
-    // never more than the CUs: a CU with two of them ends late (264
-    // workgroups for the 32 tokens: 31.2 and 18.4)
-    const int most = (int)std::min<int64_t>(E_local, pairs);
-    const int per = std::max(1, std::min<int>(grid.x, 256 / most));
+  // never more than the CUs: a CU with two of them ends late (264
+  // workgroups for the 32 tokens: 31.2 and 18.4)
+  const int most = (int)std::min<int64_t>(E_local, pairs);
+  const int per = std::max(1, std::min<int>(grid.x, 256 / most));
+  const int rounds = (grid.x + per - 1) / per;
+  if (a.K == 2048 && E_local <= 32 && hit * grid.x >= 768 &&
+      rounds * per * 8 <= (int)grid.x * 9 &&
+      (PAIRS || hit >= 0.9 * E_local)) {
     hipLaunchKernelGGL((moe_tiles_kernel<2, KIND, PAIRS>), dim3(per, E_local),
                        block, 0, stream, a, (int)grid.x);
     return;
