@@ -34,7 +34,7 @@ for _g, _names in {
             "moe_grouped_up moe_grouped_down moe_combine moe_combine_norm"),
     "route": "moe_route moe_gate_route moe_norm_gate_route moe_sort",
     "quant": ("w4a16_gemv w4a16_dequant w4a16_gemm w4a16_swiglu "
-              "w4a16_swiglu_fits lora_shrink lora_expand"),
+              "w4a16_in_tiles lora_shrink lora_expand"),
     "comm": ("allreduce_rmsnorm one_shot_ar_rmsnorm ipc_handle ipc_open "
              "ipc_close"),
     "mix": ("causal_conv_update "
@@ -743,7 +743,7 @@ def w4a16_swiglu(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor,
     if not (x.is_cuda and x.dtype == torch.bfloat16 and x.size(0) <= 16
             and qweight.size(0) % 2 == 0 and x.data_ptr() % 16 == 0
             and qweight.data_ptr() % 16 == 0
-            and _K.w4a16_swiglu_fits(x.size(0), N, K, group)):
+            and _K.w4a16_in_tiles(x.size(0), 2 * N, K, group, True)):
         return None
     out = torch.empty(x.size(0), N, dtype=x.dtype, device=x.device)
     _K.w4a16_swiglu(out, x.contiguous(), qweight, scales, zeros, group)

@@ -12,7 +12,8 @@ void w4a16_gemm(at::Tensor out, at::Tensor x, at::Tensor qweight,
                 at::Tensor scales, at::Tensor zeros, int64_t group);
 void w4a16_swiglu(at::Tensor out, at::Tensor x, at::Tensor qweight,
                   at::Tensor scales, at::Tensor zeros, int64_t group);
-bool w4a16_swiglu_fits(int64_t M, int64_t N, int64_t K, int64_t group);
+bool w4a16_in_tiles(int64_t M, int64_t rows, int64_t K, int64_t group,
+                    bool glu);
 void lora_shrink(at::Tensor tmp, at::Tensor x, at::Tensor A, at::Tensor idx,
                  double scale);
 void lora_expand(at::Tensor y, at::Tensor tmp, at::Tensor B, at::Tensor idx);
@@ -23,7 +24,7 @@ TORCH_LIBRARY_FRAGMENT(kaito, m) {
   m.def("w4a16_dequant(Tensor(a!) out, Tensor qweight, Tensor scales, Tensor zeros, int group) -> ()");
   m.def("w4a16_gemm(Tensor(a!) out, Tensor x, Tensor qweight, Tensor scales, Tensor zeros, int group) -> ()");
   m.def("w4a16_swiglu(Tensor(a!) out, Tensor x, Tensor qweight, Tensor scales, Tensor zeros, int group) -> ()");
-  m.def("w4a16_swiglu_fits(int M, int N, int K, int group) -> bool", &kaito::w4a16_swiglu_fits);
+  m.def("w4a16_in_tiles(int M, int rows, int K, int group, bool glu) -> bool", &kaito::w4a16_in_tiles);
   m.def("lora_shrink(Tensor(a!) tmp, Tensor x, Tensor A, Tensor idx, float scale) -> ()");
   m.def("lora_expand(Tensor(a!) y, Tensor tmp, Tensor B, Tensor idx) -> ()");
 }

@@ -297,13 +297,38 @@ __global__ __launch_bounds__(64 * W4_WAVES) void w4a16_tiles_kernel(
 }
 
 // 0, or the stages of a ring with which the sizes fit
-int w4_tiles_depth(int64_t M, int64_t N, int64_t K, int64_t group, int cols) {
-  if (M < 1 || M > 16 || group != 128 || K % W4_K || N % cols ||
-      (N * 2) * (K / 2) >= 1LL << 32)
+int w4_tiles_depth(int64_t M, int64_t rows, int64_t K, int64_t group) {
+  if (M < 1 || M > 16 || group != 128 || K % W4_K || rows % 16 ||
+      rows * (K / 2) >= 1LL << 32)
     return 0;
   const int mr = M <= 4 ? 4 : 16;
   return w4_lds(3, mr, M, K) <= W4_LDS ? 3
       : w4_lds(2, mr, M, K) <= W4_LDS ? 2 : 0;
+}
+
+// Whether they are faster than the row streams (from 5 rows of x on: MFMA from
+// global memory), us, streams and tiles. K = 512 S keeps S of the eight waves
+// busy.
+//   Alone: one row never; two with many weights, 4096 x 14336 13.8 and 11.7,
+// 28672 x 2560 .81 of the time, but 12288 x 2048 7.1 and 8.1, 57344 x 1024 16.9 and
+// 19.9. Three or four of a narrow K with 4096 rows of W (2048 x 2048 4.4 and 4.7,
+// 11008 .84). More, from K of 2048 on (4096 x 1024 3.8 and 4.6 at 5, 57344 x 512 9.7
+// and 20.2), beyond 8 rows at 2048 with 6144 of W (4096: 6.1 and 6.7 at 16).
+//   A pair saves a launch. One row: few rows of W (4096 .83 to .95; 6144 x 4096
+// 7.7 and 8.1, 22016 x 2048 9.7 and 11.7, 28672 x 4096 1.04) and many of a wide K
+// (11008 x 5120 .96, 28672 x 7168 .79). Two: not with many rows of a narrow K
+// (57344 x 2048 20.1 and 21.6). From five on K up to 1024 only with few (22016 x
+// 512 7.4 and 11.0, 22016 x 1024 1.04).
+bool w4_tiles_pay(int64_t M, int64_t rows, int64_t K, bool glu) {
+  if (glu) {
+    if (M == 1) return rows < 6144 || (rows >= 11008 && K >= 5120);
+    if (M == 2) return K > 2048 || rows <= 11008;
+    return M <= 4 || K > 1024 || rows <= 4096;
+  }
+  if (M == 1) return false;
+  if (M == 2) return K > 2048 && rows * K >= 48 << 20;
+  if (M <= 4) return K > 2048 || rows >= 4096;
+  return K > 2048 || (K == 2048 && (M <= 8 || rows >= 6144));
 }
 
 template <bool GLU>
@@ -312,11 +337,7 @@ bool launch_w4_tiles(at::Tensor& out, const at::Tensor& x,
                      const at::Tensor& zeros, int64_t group) {
   const int M = x.size(0), K = x.size(1);
   const int N = qweight.size(0) / (GLU ? 2 : 1);
-  const int depth = w4_tiles_depth(M, N, K, group, GLU ? 8 : 16);
-  // alone, two rows pay from 48 M weights on (4096 x 14336 13.8 and 11.7 us; 4096
-  // x 8192 9.1 and 9.4, 12288 x 2048 7.1 and 8.1), one row never; the pair saves
-  // a launch of 4.6
-  if (!GLU && (M < 2 || (M == 2 && (int64_t)N * K < 48 << 20))) return false;
+  const int depth = w4_tiles_depth(M, qweight.size(0), K, group);
   if (!depth || (uintptr_t)x.data_ptr() % 16 ||
       (uintptr_t)qweight.data_ptr() % 16)
     return false;
@@ -503,7 +524,9 @@ void w4a16_gemv(at::Tensor out, at::Tensor x, at::Tensor qweight,
               "w4a16_gemv: 64|K and 64|group required");
   TORCH_CHECK(x.is_contiguous() && out.is_contiguous());
   if (M == 0 || N == 0) return;
-  if (launch_w4_tiles<false>(out, x, qweight, scales, zeros, group)) return;
+  if (w4_tiles_pay(M, N, K, false) &&
+      launch_w4_tiles<false>(out, x, qweight, scales, zeros, group))
+    return;
   auto stream = at::hip::getCurrentHIPStream();
 #define W4_ARGS                                                               \
   (short*)out.data_ptr(), (const short*)x.data_ptr(),                         \
@@ -542,11 +565,14 @@ void w4a16_gemv(at::Tensor out, at::Tensor x, at::Tensor qweight,
 #undef W4_ARGS
 }
 
-// silu(x Wg^T) * (x Wu^T) of the stacked W = [Wg | Wu], where the tiles take it
-// (w4a16_swiglu_fits)
-bool w4a16_swiglu_fits(int64_t M, int64_t N, int64_t K, int64_t group) {
-  return w4_tiles_depth(M, N, K, group, 8) > 0;
+// Whether M rows of x run in the tiles: alone or as a SwiGLU pair
+bool w4a16_in_tiles(int64_t M, int64_t rows, int64_t K, int64_t group,
+                    bool glu) {
+  return w4_tiles_depth(M, rows, K, group) > 0 &&
+         w4_tiles_pay(M, rows, K, glu);
 }
+
+// silu(x Wg^T) * (x Wu^T) of the stacked W = [Wg | Wu]
 
 void w4a16_swiglu(at::Tensor out, at::Tensor x, at::Tensor qweight,
                   at::Tensor scales, at::Tensor zeros, int64_t group) {

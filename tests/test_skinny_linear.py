@@ -156,6 +156,24 @@ def test_w4_tiles(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,rows,K,alone,pair", [
+    (1, 4096, 4096, False, True), (1, 6144, 4096, False, False),
+    (1, 28672, 4096, False, False), (1, 28672, 7168, False, True),
+    (2, 28672, 4096, True, True), (2, 4096, 14336, True, True),
+    (2, 12288, 2048, False, False), (2, 57344, 1024, False, False),
+    (3, 2048, 2048, False, True), (3, 11008, 2048, True, True),
+    (4, 1024, 4096, True, True), (5, 4096, 1024, False, True),
+    (5, 22016, 512, False, False), (8, 4096, 2048, True, True),
+    (16, 4096, 2048, False, True), (16, 6144, 2048, True, True),
+    (16, 4096, 4096, False, False), (17, 4096, 512, False, False)])
+def test_which_packed_sizes_take_tiles(M, rows, K, alone, pair):
+    """The sides of the lines on which either was measured to be faster."""
+    assert ops._K.w4a16_in_tiles(M, rows, K, 128, False) == alone
+    assert ops._K.w4a16_in_tiles(M, rows, K, 128, True) == pair
+    assert not ops._K.w4a16_in_tiles(M, rows, K, 64, True)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 16, 17, 32])
 @pytest.mark.parametrize("N,K,G", [(1, 64, 64), (40, 128, 128),
                                    (33, 192, 192), (100, 4224, 128),
