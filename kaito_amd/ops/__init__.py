@@ -170,10 +170,13 @@ def _skinny(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
     7168 (2112 x 7168: 12.7, 12.6; 2048 x 8192: 14.6, 13.1); SwiGLU pairs,
     which save a launch, to 8192 (28672 x 4096: 50.3, 60.5), uneven ones
     excepted (5120 x 5120: 19.1, 17.9).
-    K of 2048, where x fits the registers, always (7168 x 2048: 10.5, 13.9 at
-    16; 12288 13.6, 16.6; at 32 4096 x 2048: 8.9, 11.9; 5152 11.4, 12.6; 8192
-    12.8, 14.0; 12288 15.9, 16.9; 32000 29.7, 31.8), and K of 4096 with many
-    rows of W up to 16 (128256 x 4096 168, 186).
+    K of 2048, where x fits the registers (7168 x 2048: 9.9, 12.7 at 16; 12288
+    13.0, 14.8; 128256 91, 103; at 32 4096 x 2048: 8.4, 11.8; 5152 11.1, 11.8;
+    8192 12.4, 12.8; 24576 23.3, 25.1; 128256 98, 105; as a pair 16384 17.3,
+    19.5), but beyond 24 rows the library is ahead on both sides of 12288, three
+    tiles per CU and a tie (10240 14.4, 13.6; 12288 15.2, 14.8; 16384 18.0,
+    17.0); and K of 4096 with many rows of W up to 16 (12288 x 4096 22.0, 28.4;
+    128256 167, 186).
     Up to 32: to 3072 x 2048 (7.4, 11.5; as a pair to 6144 x 2048 12.5, 15.0)
     and K of 4096 (1024 x 4096: 10.1, 11.3 at 24), where beyond 24
     rows the library has another kernel for few rows of W and K of 2560 and
@@ -195,8 +198,9 @@ def _skinny(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
     if K % 64 or N % 16:
         return False
     # x stays in registers while W streams
-    if N * K < 1 << 31 and (
-            K == 2048 or (K == 4096 and M <= 16 and N >= 12288)):
+    if K == 2048 and N * K < 1 << 31:
+        return glu or M <= 24 or not (8192 < N < 12288 or 12544 <= N < 24576)
+    if K == 4096 and M <= 16 and N >= 12288 and N * K < 1 << 31:
         return True
     if M <= 16 and N < 1024 and K > 5120 and not glu:
         return False

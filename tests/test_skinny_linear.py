@@ -68,6 +68,17 @@ def test_staying_workgroups(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,glu,streamed", [
+    (24, 16384, False, True), (32, 8192, False, True),
+    (32, 10240, False, False), (25, 16384, False, False),
+    (32, 16384, True, True), (32, 24576, False, True)])
+def test_which_rows_of_2048_stream(M, N, glu, streamed):
+    x = torch.empty(M, 2048, device=DEV, dtype=torch.bfloat16)
+    w = torch.empty(N, 2048, device=DEV, dtype=torch.bfloat16)
+    assert ops._skinny(x, w, glu) == streamed
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M", [2, 3, 4])
 @pytest.mark.parametrize("N,K", [(4096, 8192), (4128, 8192), (4104, 8192),
                                  (4128, 8200)])
