@@ -5,11 +5,11 @@ catalog (gpt-oss-120b / Qwen MoE presets in
 supported_models.yaml).
 
 The GPU path needs no host read: two launches choose the experts and, beyond
-decode sizes, sort the (token, expert) pairs by expert (ops/csrc/moe_route.hip),
-grouped products gather the rows, apply the activation and go down again behind the device's
-offsets (ops/csrc/moe.hip for decode-sized steps, moe_gemm.hip for prompts),
-and one launch sums every token's rows with their weights, the identity
-experts' share and the shared expert. Worst-case tile grids make every shape
+small steps of few experts, sort the (token, expert) pairs by expert
+(ops/csrc/moe_route.hip), grouped products gather the rows, apply the activation
+and go down again behind the device's offsets (ops/csrc/moe.hip for decode-sized
+steps, moe_gemm.hip for prompts), and one launch sums every token's rows with
+their weights, the identity experts' share and the shared expert. Worst-case tile grids make every shape
 static, so MoE decode steps capture into hipGraphs.
 
 Parallelism at tp>1:

@@ -5,7 +5,9 @@
 //
 //   * tokens are sorted by expert on the GPU (moe_route.hip) and the kernels
 //     get `sorted_ids` (token per sorted row) and `offsets` ([E+1] exclusive
-//     prefix sums, by global expert);
+//     prefix sums, by global expert); in small steps of few experts
+//     (ops.moe_pairs_pay) a workgroup finds its expert's rows among the pairs
+//     (moe_up_pairs, moe_down_pairs);
 //   * moe_gate_silu: act[s] = silu(x[tok] Wg^T) * (x[tok] Wu^T), the rows
 //     gathered through sorted_ids (ungated experts, act_mode 2: relu(.)^2). A
 //     workgroup's 16 weight rows are 8 gate rows and their 8 up rows;
@@ -14,13 +16,12 @@
 //
 // One workgroup per (16 weight rows, expert), or with K = 2048 about one per CU
 // that goes from tile to tile; an expert with more rows than 16 MT is walked in
-// passes, whose weights come back from the caches. Measured
-// on one MI355X (32 tokens, 8 experts of 2048 x 2048, top 2) against 64 x 128
-// tiles with both operands staged behind barriers, on 128 workgroups:
-// 89 us for both products, 47 in tiles of their own, now 38.5 (201 MB of
-// weights: 5.2 TB/s, launches included). 32 experts
-// of 2880 x 2880 (K in stages of 64), top 4, whole layer: 8 tokens 491 -> 178,
-// 64 tokens 440 -> 297.
+// passes, whose weights come back from the caches. Measured on one MI355X (32
+// tokens, 8 experts of 2048 x 2048, top 2) against 64 x 128 tiles with both
+// operands staged behind barriers, on 128 workgroups: 89 us for both products, 47
+// in tiles of their own, now 38.5 (201 MB of weights: 5.2 TB/s, launches
+// included). 32 experts of 2880 x 2880 (K in stages of 64), top 4, whole layer: 8
+// tokens 491 -> 178, 64 tokens 440 -> 297.
 //
 // Expert parallelism: callers pass `e_base` and the LOCAL weights; TP shards
 // the expert intermediate dim. Both use these kernels unchanged.

@@ -14,8 +14,8 @@
 // f32. 28672 x 4096: 44.4 us at M = 8 (library 56.8), 50.9 at 16 (57.4), 72.8 at
 // 32 (48.6): x comes through the caches once per workgroup, so the gain ends
 // where its rows cost what those of W do. Where x fits the registers,
-// workgroups stay for many tiles (stream_tiles): 40.1 at 8, 41.8 at 16. K in stages of 64, 2880 x 2880: 6.5
-// at 8 (16.3), 6.8 at 16 (16.4).
+// workgroups stay for many tiles (stream_tiles): 40.1 at 8, 41.8 at 16. K in
+// stages of 64, 2880 x 2880: 6.5 at 8 (16.3), 6.8 at 16 (16.4).
 //
 // 4-bit weights run as integers. Read as fp8 (e4m3, subnormals and the first
 // binade), a byte of 0 to 15 is exactly q / 512: two masks and four packed

@@ -119,12 +119,15 @@ __global__ __launch_bounds__(256) void w4a16_mfma_kernel(
 // 16 bytes are 32 k of one group, four operands of v_mfma_f32_16x16x32_bf16, so
 // that a nibble is unpacked once and multiplied with every row of x on the matrix
 // unit. x lies in the unpacked nibbles' order, beside its sums over the groups.
-// Bound by the unpacking, about 270 instructions per stage and 2 x 8 waves: the
-// time hardly grows with the rows. us, rows streamed (5 rows and more: MFMA from
-// global memory) and now, at 1, 2, 3, 4, 8 rows: 28672 x 4096 15.8 19.7 23.6 33.2
-// 37.7 and 16.7 17.4 17.4 17.5 18.3; 4096 x 14336 11.4 13.8 and 11.7 11.7 (more rows
-// do not fit); 4096 x 4096 4.6 5.7 7.9 8.8 8.7 and 5.9 6.1 6.6 7.0 7.9. Four waves:
-// 20.5 at 2 rows; sums of two tiles at a time: no change.
+// Bound by the chain of a tile, with two waves per SIMD to cover it: wait, unpack
+// (232 vector instructions per stage), multiply, meet at a barrier, sum. 28672 x
+// 4096, 2 rows: vector unit busy 31 %, matrix cores 9, LDS 16, 3.8 TB/s; of the
+// waves' time 38 % waits for loads and barriers, 30 for issue. The time hardly grows
+// with the rows. us, rows streamed (5 rows and more: MFMA from global memory) and
+// now, at 1, 2, 3, 4, 8 rows: 28672 x 4096 15.8 19.7 23.6 33.2 37.7 and 16.7 17.4
+// 17.4 17.5 18.3; 4096 x 14336 11.4 13.8 and 11.7 11.7 (more rows do not fit); 4096 x
+// 4096 4.6 5.7 7.9 8.8 8.7 and 5.9 6.1 6.6 7.0 7.9. Four waves: 20.5 at 2 rows; sums
+// of two tiles at a time: no change.
 namespace {
 
 constexpr int W4_K = 512;           // k of a stage
