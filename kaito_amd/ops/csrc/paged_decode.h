@@ -321,8 +321,9 @@ void paged_decode_kernel(const DecodeArgs a) {
     for (int i = 0; i < 2; i++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        // a masked key weighs nothing even where a lane saw no other yet
-        const bool live = BIASED ? seen(i, r) : s[i][r] > -1e29f;
+        // a masked key weighs nothing even where a lane saw no other yet; so
+        // does one whose score is -infinity
+        const bool live = BIASED ? s[i][r] != NONE : s[i][r] > -1e29f;
         float w = live ? fold_weight<BIASED>(s[i][r], m) : 0.f;
         l += w;
 #pragma unroll

@@ -134,6 +134,54 @@ def test_rglru_very_long_steps(T):
     assert ((one - parts).abs() <= 2.0 ** -14 * (1 + parts.abs())).all()
 
 
+def _decode_of_700(rows, H, G, D):
+    """q, pages and the table of rows with 700 keys each."""
+    pages = -(-700 // 16)
+    kc, vc = (torch.randn(rows * pages, G, 16, D, device=DEV).to(torch.bfloat16)
+              for _ in range(2))
+    table = torch.arange(rows * pages, dtype=torch.int32,
+                         device=DEV).view(rows, pages)
+    return torch.randn(rows, H, D, device=DEV).to(torch.bfloat16), kc, vc, \
+        table
+
+
+def _check_decode_of_700(q, kc, vc, table, window):
+    """Against f64, with scores beyond f32 as infinities; NaN and infinities
+    where the reference has them."""
+    (rows, H, D), G, n = q.shape, kc.size(1), 700
+    out = ops.window_attention(
+        q, kc, vc, table, torch.arange(rows, dtype=torch.int32, device=DEV),
+        torch.full((rows,), n - 1, device=DEV), D ** -0.5, 0.0, None, None,
+        window)
+    lo = n - window if window else 0
+    for t in (0, rows - 1):
+        k, v = (c[table[t].long()].transpose(1, 2).reshape(-1, G, D)[lo:n]
+                .double().repeat_interleave(H // G, 1) for c in (kc, vc))
+        s = (k * q[t].double()).sum(-1).T * D ** -0.5
+        p = torch.where(s < -1e38, -torch.inf, s).softmax(-1)
+        ref = (p.T[:, :, None] * v).sum(0)
+        got = out[t].double()
+        assert torch.equal(got.isnan(), ref.isnan())
+        assert torch.equal(got[ref.isinf()], ref[ref.isinf()])
+        fine = ref.isfinite()
+        err = (got - ref).abs()[fine]
+        assert (err <= 2.0 ** -8 * ref.abs()[fine] + 2e-5).all()
+    return out
+
+
+@pytest.mark.parametrize("H,G,D", [(3, 3, 64), (8, 1, 128), (4, 1, 256)])
+@pytest.mark.parametrize("window,rows", [(0, 2), (300, 2), (0, 300)])
+def test_window_decode_infinite_scores(H, G, D, window, rows):
+    """Keys whose scores are -infinity weigh nothing, also where a wave has no
+    others."""
+    torch.manual_seed(D + window)
+    q, kc, vc, table = _decode_of_700(rows, H, G, D)
+    q[0, :, 0] = 2.0 ** 100
+    kc[:table.size(1), :, :, 0] = 0
+    kc[512 // 16:640 // 16, :, :, 0] = -2.0 ** 60
+    assert _check_decode_of_700(q, kc, vc, table, window).isfinite().all()
+
+
 @pytest.mark.parametrize("H,G,D", [(3, 3, 64), (8, 1, 128), (6, 2, 128),
                                    (8, 2, 256)])
 @pytest.mark.parametrize("r2", [1e-7, 3e-6, 1e-3])
