@@ -231,148 +231,175 @@ void paged_decode_kernel(const DecodeArgs a) {
     }
   };
 
-  int64_t row0 = 0, row1 = 0;
-  if (t0 < t1) {
-    row0 = page_row(base / BS + t0 * 2);
-    row1 = page_row(base / BS + t0 * 2 + 1);
-    load_k(row0, row1);
-  }
-  for (int t = t0; t < t1; t++) {
-    // ---- V of this tile: slot j * 64 + lane is row s / CV, place s % CV
-    u8x8_t v8[FP8 ? LV : 1];
-#pragma unroll
-    for (int j = 0; j < LV; j++) {
-      const int row = j * (64 / CV) + lane / CV;
-      const int64_t at = (j * (64 / CV) < BS ? row0 : row1) * D;
-      const uint32_t off =
-          row % BS * D + flash::swz_v<D>(row, lane % CV) * 8;
-      if constexpr (FP8)
-        v8[j] = *reinterpret_cast<const u8x8_t*>(
-            (const uint8_t*)a.v + at + off);
-      else
-        flash::lds_copy16((const short*)a.v + at + off, vl + j * 512);
-    }
-    // ---- S^T: keys 16 i + 4 hi + r of head lo
-    f32x4 s[2];
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-      s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kk = 0; kk < KK; kk++) {
-        if constexpr (FP8) kf[i][kk] = widen8(k8[i][kk]);
-        s[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[i][kk], qf[kk],
-                                                       s[i], 0, 0, 0);
-      }
-    }
-    if (t + 1 < t1) {               // K of the next tile, under way with V
-      row0 = page_row(base / BS + t * 2 + 2);
-      row1 = page_row(base / BS + t * 2 + 3);
+  // `wild`: an infinity among the values is multiplied by the leading term of its
+  // weight alone; with a remainder of the other sign, or of 0, it would be NaN.
+  auto walk = [&](const bool wild) {
+    int64_t row0 = 0, row1 = 0;
+    if (t0 < t1) {
+      row0 = page_row(base / BS + t0 * 2);
+      row1 = page_row(base / BS + t0 * 2 + 1);
       load_k(row0, row1);
     }
-    // ---- softmax
-    const int key0 = base + t * KT;
-    const bool whole = key0 >= start && key0 + KT <= seq_len;
-    float mx = NONE;
-    if constexpr (BIASED) {
-#pragma unroll
-      for (int i = 0; i < 2; i++) s[i] *= a.scale;
-      if (a.cap > 0.f)
-#pragma unroll
-        for (int i = 0; i < 8; i++)
-          s[i / 4][i % 4] = a.cap * tanhf(s[i / 4][i % 4] / a.cap);
-      if (a.r1) {
-        float* pen = s_pen[wave];
-        const float dist = (float)(seq_len - 1 - key0 - (lane & 31));
-#pragma unroll
-        for (int j = 0; j < PH / 2; j++)
-          if (2 * j < a.G) pen[lane + 64 * j] = r1[j] * log1pf(r2[j] * dist);
-        __builtin_amdgcn_wave_barrier();
-        const float* mine = pen + min(lo, a.G - 1) * KT + 4 * hi;
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-          s[i] -= *reinterpret_cast<const f32x4*>(mine + 16 * i);
-        __builtin_amdgcn_wave_barrier();
-      }
-    }
-    auto seen = [&](const int i, const int r) {
-      const int key = key0 + 16 * i + 4 * hi + r;
-      return whole || (key >= start && key < seq_len);
-    };
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        if (!BIASED) s[i][r] *= c;
-        if (!seen(i, r)) s[i][r] = NONE;
-        mx = fmaxf(mx, s[i][r]);
-      }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    if (__any(mx > m)) {
-      const float mn = fmaxf(m, mx);
-      const float corr = BIASED && m == mn ? 1.f : fold_weight<BIASED>(m, mn);
-      m = mn;
-      l *= corr;
-#pragma unroll
-      for (int dt = 0; dt < DT; dt++) o[dt] *= corr;
-    }
-    hbf16x8 p[3];                   // the weight's leading bits, the rest
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        // a masked key weighs nothing even where a lane saw no other yet; so
-        // does one whose score is -infinity
-        const bool live = BIASED ? s[i][r] != NONE : s[i][r] > -1e29f;
-        float w = live ? fold_weight<BIASED>(s[i][r], m) : 0.f;
-        l += w;
-#pragma unroll
-        for (int n = 0; n < 3; n++) {
-          p[n][i * 4 + r] = (__bf16)w;
-          w -= (float)p[n][i * 4 + r];
-        }
-      }
-    if constexpr (FP8) {
-#pragma unroll
-      for (int j = 0; j < LV; j++)
-        *reinterpret_cast<hbf16x8*>(vl + (j * 64 + lane) * 8) = widen8(v8[j]);
-    } else {
-      // the direct loads' data: this wave's own, so no barrier
-      __builtin_amdgcn_s_waitcnt(0x0f70);     // vmcnt(0)
-    }
-    if (!whole) {
-      // slots outside the sequence hold what their last user left, and a
-      // weight of zero does not silence an infinity
+    for (int t = t0; t < t1; t++) {
+      // ---- V of this tile: slot j * 64 + lane is row s / CV, place s % CV
+      u8x8_t v8[FP8 ? LV : 1];
 #pragma unroll
       for (int j = 0; j < LV; j++) {
-        const int key = key0 + j * (64 / CV) + lane / CV;
-        if (key < start || key >= seq_len)
-          *reinterpret_cast<short8_t*>(vl + (j * 64 + lane) * 8) =
-              short8_t{0, 0, 0, 0, 0, 0, 0, 0};
+        const int row = j * (64 / CV) + lane / CV;
+        const int64_t at = (j * (64 / CV) < BS ? row0 : row1) * D;
+        const uint32_t off =
+            row % BS * D + flash::swz_v<D>(row, lane % CV) * 8;
+        if constexpr (FP8)
+          v8[j] = *reinterpret_cast<const u8x8_t*>(
+              (const uint8_t*)a.v + at + off);
+        else
+          flash::lds_copy16((const short*)a.v + at + off, vl + j * 512);
       }
-    }
-    __builtin_amdgcn_wave_barrier();
-    // ---- O^T: dims 16 dt + 4 hi + r of head lo
+      // ---- S^T: keys 16 i + 4 hi + r of head lo
+      f32x4 s[2];
 #pragma unroll
-    for (int dt = 0; dt < DT; dt += 2) {    // in pairs: neither waits for itself
-      hbf16x8 vf[2];
+      for (int i = 0; i < 2; i++) {
+        s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int u = 0; u < 2; u++) {
-        const short* at = vl + vrow * D +
-            flash::swz_v<D>(vrow, (dt + u) * 2 + vc) * 8 + ve;
-        const short4_t a4 = flash::read_tr(at);
-        const short4_t b4 = flash::read_tr(at + 16 * D);
-        vf[u] = __builtin_bit_cast(
-            hbf16x8, __builtin_shufflevector(a4, b4, 0, 1, 2, 3, 4, 5, 6, 7));
+        for (int kk = 0; kk < KK; kk++) {
+          if constexpr (FP8) kf[i][kk] = widen8(k8[i][kk]);
+          s[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[i][kk], qf[kk],
+                                                         s[i], 0, 0, 0);
+        }
       }
+      if (t + 1 < t1) {               // K of the next tile, under way with V
+        row0 = page_row(base / BS + t * 2 + 2);
+        row1 = page_row(base / BS + t * 2 + 3);
+        load_k(row0, row1);
+      }
+      // ---- softmax
+      const int key0 = base + t * KT;
+      const bool whole = key0 >= start && key0 + KT <= seq_len;
+      float mx = NONE;
+      if constexpr (BIASED) {
 #pragma unroll
-      for (int n = 2; n >= 0; n--)
+        for (int i = 0; i < 2; i++) s[i] *= a.scale;
+        if (a.cap > 0.f)
 #pragma unroll
-        for (int u = 0; u < 2; u++)
-          o[dt + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              vf[u], p[n], o[dt + u], 0, 0, 0);
+          for (int i = 0; i < 8; i++)
+            s[i / 4][i % 4] = a.cap * tanhf(s[i / 4][i % 4] / a.cap);
+        if (a.r1) {
+          float* pen = s_pen[wave];
+          const float dist = (float)(seq_len - 1 - key0 - (lane & 31));
+#pragma unroll
+          for (int j = 0; j < PH / 2; j++)
+            if (2 * j < a.G) pen[lane + 64 * j] = r1[j] * log1pf(r2[j] * dist);
+          __builtin_amdgcn_wave_barrier();
+          const float* mine = pen + min(lo, a.G - 1) * KT + 4 * hi;
+#pragma unroll
+          for (int i = 0; i < 2; i++)
+            s[i] -= *reinterpret_cast<const f32x4*>(mine + 16 * i);
+          __builtin_amdgcn_wave_barrier();
+        }
+      }
+      auto seen = [&](const int i, const int r) {
+        const int key = key0 + 16 * i + 4 * hi + r;
+        return whole || (key >= start && key < seq_len);
+      };
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          if (!BIASED) s[i][r] *= c;
+          if (!seen(i, r)) s[i][r] = NONE;
+          mx = fmaxf(mx, s[i][r]);
+        }
+      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      if (__any(mx > m)) {
+        const float mn = fmaxf(m, mx);
+        const float corr = BIASED && m == mn ? 1.f : fold_weight<BIASED>(m, mn);
+        m = mn;
+        l *= corr;
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++) o[dt] *= corr;
+      }
+      hbf16x8 p[3];                   // the weight's leading bits, the rest
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          // a masked key weighs nothing even where a lane saw no other yet; so
+          // does one whose score is -infinity
+          const bool live = BIASED ? s[i][r] != NONE : s[i][r] > -1e29f;
+          float w = live ? fold_weight<BIASED>(s[i][r], m) : 0.f;
+          l += w;
+#pragma unroll
+          for (int n = 0; n < 3; n++) {
+            p[n][i * 4 + r] = (__bf16)w;
+            w -= (float)p[n][i * 4 + r];
+          }
+        }
+      if constexpr (FP8) {
+#pragma unroll
+        for (int j = 0; j < LV; j++)
+          *reinterpret_cast<hbf16x8*>(vl + (j * 64 + lane) * 8) = widen8(v8[j]);
+      } else {
+        // the direct loads' data: this wave's own, so no barrier
+        __builtin_amdgcn_s_waitcnt(0x0f70);     // vmcnt(0)
+      }
+      if (!whole) {
+        // slots outside the sequence hold what their last user left, and a
+        // weight of zero does not silence an infinity
+#pragma unroll
+        for (int j = 0; j < LV; j++) {
+          const int key = key0 + j * (64 / CV) + lane / CV;
+          if (key < start || key >= seq_len)
+            *reinterpret_cast<short8_t*>(vl + (j * 64 + lane) * 8) =
+                short8_t{0, 0, 0, 0, 0, 0, 0, 0};
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+      // ---- O^T: dims 16 dt + 4 hi + r of head lo
+#pragma unroll
+      for (int dt = 0; dt < DT; dt += 2) {    // in pairs: neither waits for itself
+        hbf16x8 vf[2];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+          const short* at = vl + vrow * D +
+              flash::swz_v<D>(vrow, (dt + u) * 2 + vc) * 8 + ve;
+          const short4_t a4 = flash::read_tr(at);
+          const short4_t b4 = flash::read_tr(at + 16 * D);
+          vf[u] = __builtin_bit_cast(
+              hbf16x8, __builtin_shufflevector(a4, b4, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+#pragma unroll
+        for (int n = 2; n >= 0; n--)
+#pragma unroll
+          for (int u = 0; u < 2; u++) {
+            hbf16x8 v = vf[u];
+            if (BIASED && wild && n > 0) {
+#pragma unroll
+              for (int e = 0; e < 8; e++)
+                if (!(fabsf((float)v[e]) < INFINITY)) v[e] = (__bf16)0.f;
+            }
+            o[dt + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                v, p[n], o[dt + u], 0, 0, 0);
+          }
+      }
+      __builtin_amdgcn_wave_barrier();
     }
-    __builtin_amdgcn_wave_barrier();
+  };
+  walk(false);
+  if constexpr (BIASED) {
+    bool nan = false;
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) nan |= o[dt][r] != o[dt][r];
+    if (__any(nan)) {
+      m = NONE;
+      l = 0.f;
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      pages_at = -64;
+      walk(true);
+    }
   }
 
   // ---- fold the waves: O of the used heads through LDS (the V stage)

@@ -182,6 +182,22 @@ def test_window_decode_infinite_scores(H, G, D, window, rows):
     assert _check_decode_of_700(q, kc, vc, table, window).isfinite().all()
 
 
+@pytest.mark.parametrize("H,G,D", [(3, 3, 64), (8, 1, 128), (4, 1, 256)])
+@pytest.mark.parametrize("window,rows", [(0, 2), (300, 2), (0, 300)])
+def test_window_decode_infinite_values(H, G, D, window, rows):
+    """Infinities in the values come out as such, NaN where two of them meet, as
+    a sum of weight times value has it. A window behind them, and rows without
+    any, do not see them."""
+    torch.manual_seed(D + window)
+    q, kc, vc, table = _decode_of_700(rows, H, G, D)
+    inf = float("inf")
+    for key, dim, v in ((100, 1, inf), (500, 2, -inf), (500, 3, inf),
+                        (600, 3, -inf), (699, 4, inf), (450, 5, float("nan"))):
+        vc[key // 16, :, key % 16, dim] = v
+    out = _check_decode_of_700(q, kc, vc, table, window)
+    assert out[1:].isfinite().all()
+
+
 @pytest.mark.parametrize("H,G,D", [(3, 3, 64), (8, 1, 128), (6, 2, 128),
                                    (8, 2, 256)])
 @pytest.mark.parametrize("r2", [1e-7, 3e-6, 1e-3])
