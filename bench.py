@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
-"""Flagship serving benchmark (driver contract).
+"""Flagship serving benchmark.
 
-Measures the reference's headline metric (BASELINE.json): output tokens/sec
+Measures the reference's headline metric: output tokens/sec
 (+ p50 TTFT) for Llama-3-8B TP=1, saturated continuous batching, synthetic
 requests of input 200 / output 200 tokens (the reference's Phi-4 CSV
 methodology, website/docs/gpu-benchmarks.md), random-init weights.
@@ -161,7 +161,7 @@ def main():
 
     # ---- saturation ramp (NOT counted against warmup/steps) ----
     # The timed region must measure STEADY-STATE serving, independent of
-    # the driver-chosen steps/warmup: a short run that starts timing at
+    # the chosen steps/warmup: a short run that starts timing at
     # t=0 only measures the initial prefill burst (the whole queue is
     # prefilling, nothing is decoding yet) — and a window that ends
     # before the first requests finish measures pure decode with no
@@ -253,7 +253,7 @@ def main():
             "ms_per_step": round(elapsed / args.steps * 1000, 3),
             "higher_is_better": True,
             "scaling": "weak",
-            # closest same-methodology anchor in BASELINE.md: the
+            # closest same-methodology anchor: the
             # reference's saturated output tok/s on 1xA100 80G
             # (phi-4-mini @64 QPS, 6265 tok/s) — no Llama CSV exists
             "vs_baseline": round(value / 6265.0, 3),

@@ -1,5 +1,5 @@
-"""Paged-KV block pool: the MI355X analog of vLLM's block allocator
-(SURVEY.md §2.3 "Paged-attention ... KV block pool" row). Blocks are
+"""Paged-KV block pool: the MI355X analog of vLLM's block allocator.
+Blocks are
 block_size tokens across all layers; ref-counted for future prefix sharing
 and exposing the same accounting the reference's benchmark probe reads
 (vllm:cache_config_info num_gpu_blocks — see server/metrics.py).

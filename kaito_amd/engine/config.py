@@ -2,7 +2,7 @@
 
 ModelConfig covers the llama-architecture family (Llama-3 8B/70B, Phi-4-mini
 class, Mistral, Qwen dense) — the architectures behind the reference's
-headline benchmarks (BASELINE.md: Llama-3-8B TP=1 / 70B TP=8,
+headline benchmarks (Llama-3-8B TP=1 / 70B TP=8,
 Phi-4-mini serving CSVs).
 """
 from __future__ import annotations

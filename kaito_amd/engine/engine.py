@@ -1,7 +1,7 @@
 """LLMEngine: the continuous-batching serving loop.
 
 The MI355X-native replacement for the vLLM engine the reference's Workspace
-pods launch (SURVEY.md §3.2 "HOT LOOP"). One engine per GPU (DP tier) or per
+pods launch. One engine per GPU (DP tier) or per
 TP group; step() = schedule → forward → sample → append/finish.
 """
 from __future__ import annotations

@@ -1,5 +1,4 @@
-"""Multi-adapter LoRA serving (punica/SGMV-class, reference row
-"LoRA multi-adapter serving" SURVEY.md §2.3; adapters arrive via the
+"""Multi-adapter LoRA serving (punica/SGMV-class; adapters arrive via the
 Workspace adapter spec + /mnt/adapter pulls, preset_inferences.go:886-956).
 
 Adapters are stacked per target module into [num_slots, R_max, K] (A) and

@@ -7,7 +7,7 @@ kernels (rmsnorm, rope, silu_mul, paged/prefill attention).
 
 Reference parity: this is the engine-side replacement for the vLLM model
 executor that KAITO launches via presets/workspace/inference/vllm/
-inference_api.py (SURVEY.md §2.3).
+inference_api.py.
 """
 from __future__ import annotations
 

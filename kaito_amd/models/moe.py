@@ -1,7 +1,7 @@
 """Mixture-of-experts FFN (Mixtral / Qwen-MoE / gpt-oss class).
 
 Replaces vLLM's fused-MoE CUDA path for the MoE presets in the reference
-catalog (SURVEY.md §2.3: gpt-oss-120b / Qwen MoE presets in
+catalog (gpt-oss-120b / Qwen MoE presets in
 supported_models.yaml).
 
 The GPU path needs no host read: two launches choose the experts and, beyond

@@ -1,10 +1,9 @@
 """W4A16 group quantization: pack/repack + the QuantLinear module.
 
-Covers the reference catalog's AWQ/GPTQ presets (SURVEY.md §2.3
-"quantized GEMM" row; supported_models.yaml qwen3-8b-awq etc.). Native
-layout is kernel-first (ops/csrc/w4a16.hip): qweight u32 [N, K/8] with 8
-consecutive K nibbles per word, fp32 scales/zeros [N, K/G], w = s*q - z.
-AWQ checkpoints repack into it at load time.
+Covers the reference catalog's AWQ/GPTQ presets (supported_models.yaml
+qwen3-8b-awq etc.). Native layout is kernel-first (ops/csrc/w4a16.hip):
+qweight u32 [N, K/8] with 8 consecutive K nibbles per word, fp32 scales/zeros
+[N, K/G], w = s*q - z. AWQ checkpoints repack into it at load time.
 """
 from __future__ import annotations
 

@@ -1,7 +1,7 @@
 """Model weight streaming — the MI355X analog of the reference's
 model-streaming subsystem (pkg/workspace/inference/modelstreaming: az://
 path resolution, SAS-token auth via fetch_sas.py init container, RunAI
-streamer --load-format=runai_streamer; SURVEY.md §2 "Model streaming" row).
+streamer --load-format=runai_streamer).
 
 Sources:
   file://path or plain path  → used in place

@@ -3,7 +3,7 @@
 Python re-implementation of the reference's CRD Go structs
 (api/v1beta1/workspace_types.go:298-306, inferenceset_types.go,
 api/v1alpha1/ragengine_types.go:86-112) keeping field names, condition
-types and label keys byte-compatible (SURVEY.md §8 contract appendix) so
+types and label keys byte-compatible so
 ecosystem tooling can diff/consume unchanged.
 """
 from __future__ import annotations

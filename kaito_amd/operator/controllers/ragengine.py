@@ -2,7 +2,7 @@
 pkg/ragengine/controllers (ragengine_controller.go:82 Reconcile,
 preset_rag.go:198 CreatePresetRAG): RAGEngine CR → Deployment + Service
 with the CRD spec wired into the service's env contract
-(pkg/ragengine/manifests/manifests.go:155; env names in SURVEY.md §8),
+(pkg/ragengine/manifests/manifests.go:155),
 guardrails policy ConfigMap, storage volume, GPU node path for local
 embedding, and ServiceReady/RAGEngineSucceeded conditions.
 """

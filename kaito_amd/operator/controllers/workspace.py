@@ -1,6 +1,6 @@
 """Workspace reconciler — the Python re-implementation of the reference's
-pkg/workspace/controllers/workspace_controller.go (1570 L) core path
-(SURVEY.md §3.2): validate → targetNodeCount estimate → provision →
+pkg/workspace/controllers/workspace_controller.go (1570 L) core path:
+validate → targetNodeCount estimate → provision →
 ensure Services → StatefulSet (inference) / Job (tuning) → status sync with
 pod-failure classification → benchmark result ingestion.
 """

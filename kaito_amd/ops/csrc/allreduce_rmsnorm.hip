@@ -1,6 +1,6 @@
 // Fused one-shot all-reduce + RMSNorm for TP decode over xGMI.
 //
-// SURVEY.md hard part #2 / §8: on the 8-GPU MI355X mesh every GPU has a
+// On the 8-GPU MI355X mesh every GPU has a
 // direct link to every peer, so for the SMALL tensors of a decode step
 // ([T<=1024, H] bf16) a one-shot all-reduce — each rank reads all N peer
 // buffers directly over xGMI and reduces locally — beats a ring (which

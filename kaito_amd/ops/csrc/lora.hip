@@ -1,8 +1,7 @@
 // Batched multi-adapter LoRA kernels for gfx950 (BGMV/SGMV class).
 //
-// Replaces vLLM's punica SGMV CUDA kernels (SURVEY.md §2.3 "LoRA
-// multi-adapter serving" row). Per-token adapter indices; adapter weights
-// are stacked [num_adapters, ...]; rank<=64. Both stages are memory-bound
+// Replaces vLLM's punica SGMV CUDA kernels. Per-token adapter indices; adapter
+// weights are stacked [num_adapters, ...]; rank<=64. Both stages are memory-bound
 // on adapter weights — per-adapter slabs are small (r*K) and hit L2/L3
 // across the tokens sharing an adapter.
 //

@@ -1,7 +1,6 @@
 // Paged-attention DECODE kernel for gfx950 (MI355X).
 //
-// Replaces the vLLM decode attention the reference delegates to
-// (SURVEY.md §2.3 row "Paged-attention prefill/decode"). MI355X-first
+// Replaces the vLLM decode attention the reference delegates to. MI355X-first
 // design, NOT a CUDA port:
 //  - memory-bound regime: one (seq, kv_head) workgroup streams the whole
 //    K/V history once and shares it across the GQA group's Q heads.

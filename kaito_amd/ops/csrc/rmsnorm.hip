@@ -1,8 +1,7 @@
 // Fused RMSNorm kernels for gfx950.
 //
 // Replaces the fused CUDA norm ops the reference delegates to vLLM
-// ("RMSNorm / RoPE / SiLU-MLP" row; reference invokes
-// them via presets/workspace/inference/vllm/inference_api.py -> vLLM).
+// (invoked via presets/workspace/inference/vllm/inference_api.py -> vLLM).
 //
 // Memory-bound: target is HBM BW. All bf16 traffic is vectorized as
 // short8 (16 B/lane). One workgroup per token row; grid-stride over rows.

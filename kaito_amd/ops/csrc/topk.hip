@@ -1,7 +1,7 @@
 // Top-K selection kernel for gfx950 — the selection half of flat k-NN
 // search (distances come from an MFMA GEMM; this kernel selects the K best
 // per query row). Replaces faiss-cpu's CPU selection in the reference's
-// RAG engine (SURVEY.md §2.3 "Embedding forward + FAISS" row).
+// RAG engine.
 //
 // One workgroup per query row; each thread keeps its K best over a strided
 // scan in registers (insertion-sorted, K<=32), then K rounds of block-wide

@@ -1,5 +1,4 @@
-// W4A16 group-quantized linear kernels (AWQ/GPTQ-class presets —
-// reference inventory row "quantized GEMM"; the catalog
+// W4A16 group-quantized linear kernels (AWQ/GPTQ-class presets; the catalog
 // carries qwen3-8b-awq etc.).
 //
 // Native layout (loaders repack AWQ checkpoints into this):

@@ -1,6 +1,6 @@
 """One-shot fused all-reduce(+residual)+RMSNorm over xGMI peer mappings.
 
-SURVEY.md hard part #2: on the 8-GPU MI355X mesh every GPU has a direct
+On the 8-GPU MI355X mesh every GPU has a direct
 xGMI link to every peer, so for decode-sized tensors a one-shot
 all-reduce (each rank reads all N peer staging buffers and reduces
 locally) replaces the per-link-bound ring, and fusing the
@@ -8,7 +8,7 @@ residual-add + RMSNorm epilogue saves one full read+write of the hidden
 states (the fusion the reference explicitly disables on NVIDIA,
 interface.go:439-446).
 
-v2 (round 2): the synchronization lives INSIDE the kernel — each rank
+The synchronization lives INSIDE the kernel — each rank
 exchanges hipIpc handles for a staging pair AND a signal page; block
 `row` release-stores a device-side epoch into every peer's signal slot
 and acquire-spins until all peers arrive. With double-buffered staging

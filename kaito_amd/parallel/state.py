@@ -4,8 +4,8 @@ On ROCm the torch.distributed "nccl" backend IS RCCL; xGMI gives every
 MI355X a direct link to every other GPU in the 8-way mesh, so TP
 all-reduces run as single-hop collectives. CPU tests use gloo.
 
-Reference behaviour being replaced: vLLM's NCCL TP groups + Ray bootstrap
-(SURVEY.md §5.8); rendezvous here is plain torch.distributed env-var init
+Reference behaviour being replaced: vLLM's NCCL TP groups + Ray bootstrap;
+rendezvous here is plain torch.distributed env-var init
 (POD_INDEX/headless-service DNS on k8s, 127.0.0.1 standalone).
 """
 from __future__ import annotations

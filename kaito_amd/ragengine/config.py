@@ -1,6 +1,6 @@
 """RAGEngine configuration — env contract kept byte-compatible with the
 reference (presets/ragengine/config.py; wired from the CRD by
-pkg/ragengine/manifests/manifests.go:155; SURVEY.md §8)."""
+pkg/ragengine/manifests/manifests.go:155)."""
 from __future__ import annotations
 
 import os

@@ -1,7 +1,7 @@
 """OpenAI-compatible HTTP front-end on :5000.
 
 Endpoint surface matches what the reference's ecosystem expects from a
-Workspace pod (SURVEY.md §8): /health, /metrics, /v1/models,
+Workspace pod: /health, /metrics, /v1/models,
 /v1/completions, /v1/chat/completions (with SSE streaming). Metric names
 are vLLM-compatible so benchmark_entrypoint / EPP / KEDA integrations work
 unchanged.

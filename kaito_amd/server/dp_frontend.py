@@ -4,7 +4,7 @@ The planner's tier 1 (model < 50% of one 288 GiB MI355X —
 operator/planner.py:50) gives one pod ALL the node's GPUs with
 data-parallel-size=N: N independent TP=1 engine replicas behind one
 OpenAI endpoint (the reference gets this from vLLM's DP engine-core
-replicas; SURVEY.md §2.3 "DP" row).
+replicas).
 
 MI355X shape: one engine PROCESS per GPU (HIP_VISIBLE_DEVICES pinning —
 no multi-GPU process state), a parent asyncio reverse proxy on :5000

@@ -1,5 +1,5 @@
 """Prometheus metrics with the engine metric names the KAITO ecosystem
-scrapes (SURVEY.md §8 contract appendix):
+scrapes:
 
   vllm:cache_config_info          — block pool size (benchmark probe reads
                                     num_gpu_blocks to size saturation

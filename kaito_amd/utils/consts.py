@@ -1,5 +1,4 @@
-"""Contract constants — parity with the reference's pkg/utils/consts
-(SURVEY.md §8 ports/paths table)."""
+"""Contract constants — parity with the reference's pkg/utils/consts."""
 
 PORT_INFERENCE = 5000            # OpenAI API (consts.go:140-141)
 PORT_DECODE_ENGINE = 5001        # decode role engine behind router sidecar

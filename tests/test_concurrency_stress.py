@@ -1,5 +1,5 @@
 """Concurrency stress — the air-gapped analog of the reference's Go
-`-race` CI tier (SURVEY.md §5 "race detection"). Hammers the shared
+`-race` CI tier. Hammers the shared
 serving surfaces from many threads at once and asserts (a) nothing
 deadlocks or raises, (b) greedy results stay DETERMINISTIC per prompt
 under arbitrary interleaving, (c) aborted streams never wedge the

@@ -1,5 +1,5 @@
 """Controller reconcile tests against FakeKubeClient — the reference's
-MockClient unit-test strategy (SURVEY.md §4): no cluster, full reconcile
+MockClient unit-test strategy: no cluster, full reconcile
 paths, golden assertions on created objects and conditions."""
 import json
 

@@ -1,8 +1,5 @@
 """Leader election, webhook cert bootstrap, RAGEngine version
-conversion, and the azure provisioner / NodePool management added in
-round 2 (VERDICT coverage rows: webhooks 'no cert controller / leader
-election', API types 'no v1alpha1↔v1beta1 RAGEngine conversion',
-node provisioning 'no azure-gpu-provisioner / NodePool management')."""
+conversion, and the azure provisioner / NodePool management."""
 import shutil
 
 import pytest

@@ -1,6 +1,6 @@
 """Server tests: OpenAI API surface, SSE streaming, metrics names, 429
 rate limiting — the contract the reference ecosystem (benchmark probe,
-EPP, KEDA) scrapes (SURVEY.md §8).
+EPP, KEDA) scrapes.
 """
 import threading
 import time

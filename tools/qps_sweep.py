@@ -5,7 +5,7 @@
 
 Emits one CSV row per QPS with the columns of the reference's summary
 tables (benchmark-phi4-p1.csv: TTFT and ITL mean/median/p99) plus output
-tok/s, so results are DIRECTLY comparable to BASELINE.md's A100/A10 rows.
+tok/s, so results are DIRECTLY comparable to the reference's A100/A10 rows.
 
 Usage (on a GPU box):
   python tools/qps_sweep.py --model phi-4-mini --qps 1,2,4,8,16,32,64 \
