@@ -373,7 +373,8 @@ __global__ __launch_bounds__(64 * NW, 2) void delta_chunk_kernel(
 #pragma unroll
       for (int e = 0; e < 4; e++)
         __builtin_amdgcn_raw_buffer_store_b32(
-            __float_as_uint((float)out[e]), ob, oat + c * C * orow + e * orow, 0, 0);
+            __float_as_uint((float)out[e]), ob, oat + c * C * orow + e * orow, 0,
+            0);
   };
 
   Operands x0, x1;
