@@ -58,13 +58,26 @@ KAITO_DEV void fp8x8_to_f32(const u8x8_t v, float* __restrict__ out) {
   }
 }
 
+// round to nearest even, one instruction (for two neighbouring results)
 KAITO_DEV short f32_to_bf16(float f) {
-  union { float f; uint32_t i; } v;
-  v.f = f;
-  // round-to-nearest-even
-  uint32_t rounding = 0x7FFF + ((v.i >> 16) & 1);
-  return (short)((v.i + rounding) >> 16);
+  return __builtin_bit_cast(short, (__bf16)f);
 }
+
+// v / (4 d4) as accurate as the division, in half the instructions: the
+// reciprocal's quotient and one correction. The quarter keeps the reciprocal of
+// the largest finite divisors above the values that are flushed. The correction
+// is no number where the quotient is infinite, zero over infinity, or none.
+KAITO_DEV float quotient(float v, float d4) {
+  const float r = __builtin_amdgcn_rcpf(d4), v4 = 0.25f * v, q = v4 * r;
+  const float c = __builtin_fmaf(__builtin_fmaf(-d4, q, v4), r, q);
+  return c == c ? c : q;
+}
+
+// v sigmoid(s v)
+KAITO_DEV float swish_f32(float v, float s) {
+  return quotient(v, __builtin_fmaf(0.25f, __expf(-s * v), 0.25f));
+}
+KAITO_DEV float silu_f32(float v) { return swish_f32(v, 1.f); }
 
 // ---- DPP cross-lane adds (VALU-speed; __shfl_xor lowers to
 // ds_bpermute_b32 which costs a ~30-60 cyc LDS-crossbar trip each).

@@ -70,11 +70,11 @@ struct GemmArgs {
   const int* rows;                  // x row of a sorted row; none: the same
   const int* offsets;               // [.., E + 1]
   int e_base, E, N, K;
-  int act_mode;                     // 0 SwiGLU, 1 clamped, 2 squared relu
   float limit;
 };
 
-enum Kind { UP_GATED, UP_PLAIN, DOWN };
+enum Kind { UP_GATED, UP_CLAMPED, UP_PLAIN, DOWN };
+constexpr bool is_gated(int kind) { return kind <= UP_CLAMPED; }
 
 // 16 bytes per lane from r + lane offset + uniform offset to dst + 16 * lane
 KAITO_DEV void buffer_copy16(__amdgpu_buffer_rsrc_t r, short* dst,
@@ -83,16 +83,15 @@ KAITO_DEV void buffer_copy16(__amdgpu_buffer_rsrc_t r, short* dst,
       r, (__attribute__((address_space(3))) void*)dst, 16, lane_off, off, 0, 0);
 }
 
-KAITO_DEV float silu_of(float v) { return v / (1.f + __expf(-v)); }
-
-// act_mode 1: min(g, limit) sigmoid(1.702 min(g, limit)) (clamp(u) + 1)
-KAITO_DEV float gated(int mode, float g, float u, float limit) {
-  if (mode == 1) {
+// CLAMPED: min(g, limit) sigmoid(1.702 min(g, limit)) (clamp(u) + 1)
+template <int KIND>
+KAITO_DEV float gated(float g, float u, float limit) {
+  if constexpr (KIND == UP_CLAMPED) {
     g = fminf(g, limit);
     u = fminf(fmaxf(u, -limit), limit);
-    return (u + 1.f) * (g / (1.f + __expf(-1.702f * g)));
+    return (u + 1.f) * swish_f32(g, 1.702f);
   }
-  return silu_of(g) * u;
+  return silu_f32(g) * u;
 }
 
 // elements of LDS: two and a half K steps of a whole tile, five of a quarter
@@ -115,7 +114,7 @@ KAITO_DEV void grouped_tile(const GemmArgs& a, short* lds, const int expert,
   // ---- staging slots: slot s (16 bytes) is row s / 8, place s % 8; byte
   // offsets from the tile's first row (gathered rows: from x, which the caller
   // keeps below 4 GB)
-  const int wrows = KIND == UP_GATED ? 2 * a.N : a.N;
+  const int wrows = is_gated(KIND) ? 2 * a.N : a.N;
   const short* we = a.w + ((int64_t)expert * wrows + n0) * a.K;
   const short* xe = a.rows ? a.x : a.x + (int64_t)m0 * a.K;
   const auto xr = __builtin_amdgcn_make_buffer_rsrc(
@@ -143,7 +142,7 @@ KAITO_DEV void grouped_tile(const GemmArgs& a, short* lds, const int expert,
     const int s = j * 512 + threadIdx.x, row = s / CH;
     const int c = place(row, s % CH);
     // gated: every 64 tile rows are 32 gate rows, then their up rows
-    const uint32_t n = KIND == UP_GATED
+    const uint32_t n = is_gated(KIND)
         ? min((row / 64) * 32 + row % 32, a.N - 1 - n0) +
               (row % 64 >= 32 ? a.N : 0)
         : min(row, a.N - 1 - n0);
@@ -271,25 +270,15 @@ KAITO_DEV void grouped_tile(const GemmArgs& a, short* lds, const int expert,
   }
 
   // ---- outputs n = 8 b + 4 h + e of 32-row tile i, token row lr of tile j
-  constexpr int NI = KIND == UP_GATED ? 1 : 2;
+  constexpr int NI = is_gated(KIND) ? 1 : 2;
   constexpr int WC = NI * 32;       // columns of a wave: all exist or none
   const int c0 = n0 + wn * WC;
   if (c0 >= a.N) return;            // N is a multiple of 64; no barrier below
-  if (a.bias) {
-    const short* be = a.bias + (int64_t)expert * wrows + c0;
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int b = 0; b < 4; b++) {
-        const short4_t v = *reinterpret_cast<const short4_t*>(
-            be + (KIND == UP_GATED ? i * a.N : i * 32) + 8 * b + 4 * h);
-#pragma unroll
-        for (int j = 0; j < MT; j++)
-#pragma unroll
-          for (int e = 0; e < 4; e++)
-            acc[i][j][b * 4 + e] += bf16_to_f32(v[e]);
-      }
-  }
+  // added where a value leaves: ahead of that, over all of acc, it cost 132 bytes
+  // of scratch per lane and 55 us of 312 (up, 8 experts of 2048 x 2048, 16384
+  // pairs of uneven experts, weights out of the caches; with the activations'
+  // divisions in half the instructions)
+  const short* be = a.bias + (int64_t)expert * wrows + c0 + 4 * h;
   // bf16 rows pass through the wave's part of LDS (every wave is done with
   // its tiles) and leave as 16 bytes a lane
   constexpr int PITCH = WC + 8, LANES = WC / 8;
@@ -301,12 +290,28 @@ KAITO_DEV void grouped_tile(const GemmArgs& a, short* lds, const int expert,
     for (int i = 0; i < NI; i++)
 #pragma unroll
       for (int b = 0; b < 4; b++) {
-        float4_t v;
+        float4_t v, u;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           v[e] = acc[i][j][b * 4 + e];
-          if constexpr (KIND == UP_GATED) {
-            v[e] = gated(a.act_mode, v[e], acc[1][j][b * 4 + e], a.limit);
+          if constexpr (is_gated(KIND)) u[e] = acc[1][j][b * 4 + e];
+        }
+        if (a.bias) {
+          const short4_t bv =
+              *reinterpret_cast<const short4_t*>(be + i * 32 + 8 * b);
+#pragma unroll
+          for (int e = 0; e < 4; e++) v[e] += bf16_to_f32(bv[e]);
+          if constexpr (is_gated(KIND)) {
+            const short4_t bu =
+                *reinterpret_cast<const short4_t*>(be + a.N + 8 * b);
+#pragma unroll
+            for (int e = 0; e < 4; e++) u[e] += bf16_to_f32(bu[e]);
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          if constexpr (is_gated(KIND)) {
+            v[e] = gated<KIND>(v[e], u[e], a.limit);
           } else if constexpr (KIND == UP_PLAIN) {
             v[e] = fmaxf(v[e], 0.f);
             v[e] *= v[e];
@@ -342,7 +347,7 @@ KAITO_DEV void grouped_tile(const GemmArgs& a, short* lds, const int expert,
 
 template <int BM, int KIND>
 __global__ __launch_bounds__(512, 2) void moe_grouped_kernel(const GemmArgs a) {
-  constexpr int COLS = KIND == UP_GATED ? BN / 2 : BN;   // outputs per tile
+  constexpr int COLS = is_gated(KIND) ? BN / 2 : BN;   // outputs per tile
   constexpr bool QUARTERS = BM == 256;
   __shared__ __attribute__((aligned(128)))
   short lds[BM == 256 ? LDS : 2 * (BM + BN) * BK];
@@ -553,7 +558,7 @@ __global__ __launch_bounds__(256) void moe_combine_norm_kernel(
 
 template <int KIND>
 void launch_grouped(const GemmArgs& a, int64_t TK) {
-  constexpr int COLS = KIND == UP_GATED ? BN / 2 : BN;
+  constexpr int COLS = is_gated(KIND) ? BN / 2 : BN;
   const int64_t ntiles = (a.N + COLS - 1) / COLS;
   auto stream = at::hip::getCurrentHIPStream();
   auto launch = [&](auto bm) {
@@ -615,10 +620,10 @@ void moe_grouped_up(at::Tensor act, at::Tensor x, at::Tensor w,
     a.rows = nullptr;
   }
   a.offsets = offsets.data_ptr<int>();
-  a.act_mode = (int)act_mode;
   a.limit = (float)act_limit;
   if (act.size(0) == 0 || a.E == 0 || a.N == 0) return;
   if (plain) launch_grouped<UP_PLAIN>(a, act.size(0));
+  else if (act_mode == 1) launch_grouped<UP_CLAMPED>(a, act.size(0));
   else launch_grouped<UP_GATED>(a, act.size(0));
 }
 

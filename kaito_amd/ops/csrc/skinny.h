@@ -437,7 +437,7 @@ KAITO_DEV void stream_rows_w4(float (&acc)[M][R],
   }
 }
 
-KAITO_DEV float silu(float v) { return v / (1.f + __expf(-v)); }
+KAITO_DEV float silu(float v) { return silu_f32(v); }
 
 }  // namespace skinny
 }  // namespace kaito

@@ -224,3 +224,27 @@ def test_packed_sums_keep_f32(M, N, K, G):
     out = ops.w4a16_gemv(xd, words.to(DEV), s.to(DEV), z.to(DEV), G).cpu()
     ref = x.double() @ (q.double() - 8).T
     assert torch.equal(out, ref.to(torch.bfloat16))
+
+
+@pytest.mark.gpu
+def test_swiglu_of_every_gate():
+    # all bf16 gates, infinities among them, as the first column of W
+    g = torch.arange(-32768, 32768, dtype=torch.int16, device=DEV).view(
+        torch.bfloat16)
+    w = torch.zeros(2, g.numel(), 8, dtype=torch.bfloat16, device=DEV)
+    w[0, :, 0], w[1, :, 0] = g, 1.5
+    x = torch.zeros(1, 8, dtype=torch.bfloat16, device=DEV)
+    x[0, 0] = 1
+    out = ops.linear_swiglu(x, w.view(-1, 8))[0].double()
+    v = g.double()
+    # beyond the f32 range of exp(-v) the weight is 0
+    ref = torch.where(v < -88.8, -0.0 * v.abs(), v * torch.sigmoid(v)) * 1.5
+    ref = torch.where(v == -float("inf"), float("nan"), ref)
+    ref = torch.where(ref > 2.0 ** 128 - 2.0 ** 119, float("inf"), ref)
+    assert torch.equal(out.isnan(), ref.isnan())
+    both = ~ref.isnan() & (out != ref)
+    err = (out - ref).abs()[both]
+    # half a unit of bf16's 8 bits (f32's part, exp(88) included, is below 2^-16),
+    # and what is left of results below f32's normal range
+    bound = (2.0 ** -8 + 2.0 ** -16) * ref.abs()[both] + 2.0 ** -126
+    assert (err <= bound).all(), (err / bound).max()
