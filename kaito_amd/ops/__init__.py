@@ -26,7 +26,8 @@ _OP_GROUP = {}
 for _g, _names in {
     "core": ("rms_norm fused_add_rms_norm rotary_embedding silu_and_mul "
              "gelu_and_mul gelu layer_norm fused_add_layer_norm "
-             "rope_and_cache reshape_and_cache topk skinny_linear skinny_swiglu"),
+             "rope_and_cache reshape_and_cache topk skinny_linear skinny_swiglu "
+             "batch_linear"),
     "attn": ("paged_attention paged_attention_sp prefill_attention "
              "mla_prefill_attention context_attention mfma_tile_gemm paged_read_bw"),
     "mla": "mla_decode mla_prepare head_rows mla_cache_write",
@@ -153,9 +154,22 @@ def _transformed() -> bool:
         or torch.is_autocast_enabled("cuda")
 
 
+def _plain_rows(x: torch.Tensor, w: torch.Tensor, most: int) -> bool:
+    """1 to `most` rows of bf16 on the GPU, 16-byte aligned rows, nothing to
+    differentiate: what the kernels of small linear layers take."""
+    return x.is_cuda and x.dim() == w.dim() == 2 and 1 <= x.size(0) <= most \
+        and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 \
+        and x.device == w.device and not _transformed() \
+        and w.is_contiguous() and w.size(1) % 8 == 0 and w.numel() > 0 \
+        and x.stride(1) == 1 \
+        and (x.size(0) == 1 or x.stride(0) % 8 == 0) \
+        and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 \
+        and not (torch.is_grad_enabled()
+                 and (x.requires_grad or w.requires_grad))
+
+
 def _skinny(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
-    """Whether x W^T runs on the weight-streaming kernels: a few rows of
-    bf16 on the GPU, 16-byte aligned rows, nothing to differentiate.
+    """Whether x W^T runs on the weight-streaming kernels.
 
     The lines, with us on both sides (streamed, library; weights out of the
     caches): beyond 4 rows x comes through the caches once per 16 rows of W,
@@ -182,15 +196,7 @@ def _skinny(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
     rows the library has another kernel for few rows of W and K of 2560 and
     more (1024 x 2560: 8.0, 6.9; 2048 x 2816: 8.8, 9.5; 1024 x 2816 as a pair
     9.0, 9.5)."""
-    if not (x.is_cuda and x.dim() == w.dim() == 2 and 1 <= x.size(0) <= 32
-            and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
-            and x.device == w.device and not _transformed()
-            and w.is_contiguous() and w.size(1) % 8 == 0 and w.numel() > 0
-            and x.stride(1) == 1
-            and (x.size(0) == 1 or x.stride(0) % 8 == 0)
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and not (torch.is_grad_enabled()
-                     and (x.requires_grad or w.requires_grad))):
+    if not _plain_rows(x, w, 32):
         return False
     M, (N, K) = x.size(0), w.shape
     if M <= 4:
@@ -214,26 +220,84 @@ def _skinny(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
         M <= 24 or K < 2560 or N >= 2048 or glu)
 
 
+def _batched(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
+    """Whether x W^T of up to 256 rows runs on the split kernel
+    (csrc/batch_linear.hip) where the row streams do not take it.
+
+    Both sides in us (split, library; weights out of the caches). The split
+    of K is what the library does not always find: ahead from K of 10240 on
+    (4096 x 14336: 25.4, 26.4 at 16 rows, 27.4, 34.9 at 48, 36.9, 49.4 at 128,
+    45.5, 59.1 at 256; 7168 x 18432 at 256 89, 208), to 16384 rows of W
+    (beyond, W is cut often enough without: 28672 x 14336 at 128 1 % behind).
+    K in no multiple of 512, which the library has few kernels for (4096 x
+    2880: 1.5 to 1.9 times as fast from 17 to 128 rows; behind at 256).
+    K from 4096: to 6144 rows of W (3072 x 5120 at 64 1.26 times, 4096 x 7168
+    at 128 1.6; at K of 4096 only to 64 rows, 4096 x 4096 14.3, 15.3 there and
+    18.6, 17.7 at 128; at K of 8192 only beyond 32 rows, 4096 x 8192 at 24
+    20.6, 17.9); to 8192 between K of 4096 and 8192 (8192 x 7168: 1.02 to 1.47;
+    8192 x 4096 at 64 0.88, 8192 x 8192 at 64 0.84); 16384 and more to 64 rows
+    (1.03 to 1.16). 193 to 256 rows: 6144 to 16384 with K from 7168 (1.06 to
+    1.67; 4096 x 7168 0.91).
+    SwiGLU pairs, which save a launch and a pass: from 12288 rows of W with
+    more than 16 rows, 32 for K of 2048 (28672 x 4096: 48.9, 57.2 at 64, 73.6,
+    79.8 at 256; 12288 x 2048 16.6, 20.2 at 64; 8192 x 4096 0.89), beyond 32768
+    to 64 rows (57344 x 4096: 1.07 to 1.13, 0.90 at 256), at K of 8192 from
+    20480 on (16384 x 8192 0.97)."""
+    if not _plain_rows(x, w, 256):
+        return False
+    M, (N, K) = x.size(0), w.shape
+    if M < 9 or K % 64 or N % (32 if glu else 16) \
+            or (N + 128) * K >= 1 << 31 or M * x.stride(0) >= 1 << 31:
+        return False
+    if glu:
+        return M > (16 if K > 2048 else 32) and K >= 2048 and N >= (
+            20480 if K >= 8192 else 12288) and (N <= 32768 or M <= 64)
+    if K >= 10240:
+        return 1024 <= N <= 16384
+    if M < 17:
+        return False
+    if K % 512:
+        return K >= 2560 and N >= 3072 and M <= 128
+    if K < 4096 or K > 8192 or N < 3072:
+        return False
+    if M > 192:
+        return K >= 7168 and 6144 <= N <= 16384 and (K < 8192 or N <= 12288)
+    if N <= 6144:
+        return M <= 64 if K == 4096 else K < 8192 or M > 32
+    if N <= 8192:
+        return 4096 < K < 8192
+    return N >= 16384 and K < 8192 and M <= 64
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
-    """x W^T (+ bias): the weight-streaming kernels for small decode steps,
-    hipBLASLt otherwise."""
-    if _skinny(x, w) and (bias is None or (
+    """x W^T (+ bias): the weight-streaming kernels for small decode steps, the
+    split kernel for larger ones where it is ahead, hipBLASLt otherwise."""
+    if bias is None or (
             bias.dtype == torch.bfloat16 and bias.is_contiguous()
             and bias.shape == w.shape[:1] and bias.device == w.device
-            and not (torch.is_grad_enabled() and bias.requires_grad))):
-        out = torch.empty(x.size(0), w.size(0), dtype=x.dtype,
-                          device=x.device)
-        _K.skinny_linear(out, x, w, _none(bias, x))
-        return out
+            and not (torch.is_grad_enabled() and bias.requires_grad)):
+        skinny = _skinny(x, w)
+        if skinny or _batched(x, w):
+            out = torch.empty(x.size(0), w.size(0), dtype=x.dtype,
+                              device=x.device)
+            if skinny:
+                _K.skinny_linear(out, x, w, _none(bias, x))
+            else:
+                _K.batch_linear(out, x, w, _none(bias, x), 0, 0, False)
+            return out
     return torch.nn.functional.linear(x, w, bias)
 
 
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x Wg^T) * (x Wu^T) for the stacked W = [Wg | Wu]."""
-    if _skinny(x, w, True):
+    skinny = _skinny(x, w, True)
+    if skinny or _batched(x, w, True):
         out = torch.empty(x.size(0), w.size(0) // 2, dtype=x.dtype,
                           device=x.device)
-        _K.skinny_swiglu(out, x, w)
+        if skinny:
+            _K.skinny_swiglu(out, x, w)
+        else:
+            _K.batch_linear(out, x, w, _none(None, x), 0, 0, True)
         return out
     return silu_and_mul(torch.nn.functional.linear(x, w))
 

@@ -1,0 +1,105 @@
+"""Linear layers of batched decode steps (ops/csrc/batch_linear.hip): rows around
+the tiles, rows of W that end in a tile, K steps that do not divide by the splits.
+Sums are f32, results bf16: half a unit of the 8 bits, and where a sum cancels the
+f32 rounding of its terms (K up to 2^12 of them, 2^-24 each at most: below 2^-12 of
+the typical sum)."""
+import pytest
+import torch
+
+from kaito_amd import ops
+
+DEV = "cuda"
+
+
+def _close(out, ref):
+    assert out.dtype == torch.bfloat16 and torch.isfinite(out).all()
+    err = (out.double() - ref).abs()
+    rms = ref.square().mean().sqrt()
+    assert (err <= 2.0 ** -8 * ref.abs() + 2.0 ** -12 * rms).all(), err.max()
+
+
+def _inputs(M, N, K):
+    g = torch.Generator(device=DEV).manual_seed(M * N + K)
+    big = torch.randn(M, K + 16, device=DEV, generator=g).to(torch.bfloat16)
+    w = torch.randn(N, K, device=DEV, generator=g).to(torch.bfloat16)
+    b = torch.randn(N, device=DEV, generator=g).to(torch.bfloat16)
+    return big[:, 8:8 + K], w, b             # strided rows
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 9, 16, 17, 32, 33, 64, 65, 128, 129, 192,
+                               193, 256])
+@pytest.mark.parametrize("N,K", [(16, 64), (80, 192), (144, 1152),
+                                 (272, 2048)])
+def test_plans(M, N, K):
+    x, w, b = _inputs(M, N, K)
+    ref = x.double() @ w.double().T
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    none = torch.empty(0, device=DEV)
+    for cols in (64, 128):
+        for splits in sorted({1, min(3, K // 64), min(16, K // 64)}):
+            out.fill_(float("nan"))
+            ops._K.batch_linear(out, x, w, none, cols, splits, False)
+            _close(out, ref)
+            ops._K.batch_linear(out, x, w, b, cols, splits, False)
+            _close(out, ref + b.double())
+        if N % 32 == 0 or N == 144:
+            n = N // 2 // 16 * 16
+            g, u = x.double() @ w[:n].double().T, x.double() @ w[
+                n:2 * n].double().T
+            pair = torch.full((M, n), float("nan"), dtype=torch.bfloat16,
+                              device=DEV)
+            ops._K.batch_linear(pair, x, w[:2 * n], none, cols, 1, True)
+            _close(pair, g * torch.sigmoid(g) * u)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,glu", [
+    (9, 1024, 10240, False), (256, 2048, 10240, False),
+    (17, 3072, 2880, False), (100, 4112, 2880, False),
+    (33, 4096, 4096, False), (250, 6144, 7168, False),
+    (33, 12288, 2048, True), (256, 12352, 4096, True)])
+def test_route(M, N, K, glu):
+    x, w, b = _inputs(M, N, K)
+    assert ops._batched(x, w, glu) and not ops._skinny(x, w, glu)
+    # larger than a test wants in 64 bits on the device: f32 of the library
+    ref = (x.float() @ w.float().T).double()
+    if glu:
+        g, u = ref.chunk(2, -1)
+        _close(ops.linear_swiglu(x, w), g * torch.sigmoid(g) * u)
+    else:
+        _close(ops.linear(x, w), ref)
+        _close(ops.linear(x, w, b), ref + b.double())
+
+
+@pytest.mark.gpu
+def test_stays_with_the_library():
+    x, w, _ = _inputs(64, 4096, 4096)
+    assert ops._batched(x, w)
+    for a, b in ((x.float(), w.float()), (x.half(), w.half()),
+                 (x[:8], w), (x[:, :4088], w[:, :4088].contiguous()),
+                 (x, w[:4088]), (x, w.t().contiguous().t())):
+        assert not ops._batched(a, b)
+    with torch.enable_grad():
+        v = w.clone().requires_grad_()
+        assert not ops._batched(x, v)
+        y = ops.linear(x, v)
+        y.sum().backward()
+    assert v.grad is not None
+    assert not ops._batched(x.repeat(5, 1), w)
+
+
+@pytest.mark.gpu
+def test_replayed_graph():
+    x, w, b = _inputs(40, 2048, 10240)
+    x = x.contiguous()
+    ops.linear(x, w, b)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ops.linear(x, w, b)
+    for i in range(3):
+        x.copy_(torch.randn_like(x) + i)
+        eager = ops.linear(x, w, b).clone()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
