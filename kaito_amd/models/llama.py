@@ -154,35 +154,36 @@ class LlamaAttention(nn.Module):
             # by reshape_and_cache, k and v need EQUAL row strides
             v = v.contiguous()
         cs = cos_sin_local if self.local_rope else cos_sin
+        T = x.size(0)
+        sinks = getattr(self, "sinks", None)
+        if kv_cache is not None and not meta.is_prefill:
+            out = ops.rope_paged_attention(
+                positions, q, k, v, self.head_dim, cs, kv_cache[0],
+                kv_cache[1], meta.slot_mapping, meta.block_tables,
+                meta.seq_lens, self.scale, self.window, sinks)
+            return self.o_proj(out.reshape(T, -1))
         if kv_cache is not None:
             q, k = ops.rope_and_cache(positions, q, k, v, self.head_dim, cs,
                                       kv_cache[0], kv_cache[1],
                                       meta.slot_mapping)
         else:
             q, k = ops.rotary_embedding(positions, q, k, self.head_dim, cs)
-        T = x.size(0)
         qh = q.unflatten(-1, (self.num_heads, self.head_dim))
         kh = k.unflatten(-1, (self.num_kv_heads, self.head_dim))
         vh = v.unflatten(-1, (self.num_kv_heads, self.head_dim))
-        sinks = getattr(self, "sinks", None)
-        if meta.is_prefill:
-            tiles = None if meta.tile_seq is None else \
-                (meta.tile_seq, meta.tile_qbase)
-            if meta.kv_lens is not None:
-                # suffix-query attention over the paged cache (the suffix
-                # K/V was just written by rope_and_cache above)
-                out = ops.context_attention(qh, kv_cache[0], kv_cache[1],
-                                            meta.cu_seqlens, meta.kv_lens,
-                                            meta.block_tables, self.scale,
-                                            self.window, sinks, tiles)
-            else:
-                out = ops.prefill_attention(qh, kh, vh, meta.cu_seqlens,
-                                            self.scale, meta.max_seqlen,
-                                            self.window, sinks, tiles)
+        tiles = None if meta.tile_seq is None else \
+            (meta.tile_seq, meta.tile_qbase)
+        if meta.kv_lens is not None:
+            # suffix-query attention over the paged cache (the suffix
+            # K/V was just written by rope_and_cache above)
+            out = ops.context_attention(qh, kv_cache[0], kv_cache[1],
+                                        meta.cu_seqlens, meta.kv_lens,
+                                        meta.block_tables, self.scale,
+                                        self.window, sinks, tiles)
         else:
-            out = ops.paged_attention(qh, kv_cache[0], kv_cache[1],
-                                      meta.block_tables, meta.seq_lens,
-                                      self.scale, self.window, sinks)
+            out = ops.prefill_attention(qh, kh, vh, meta.cu_seqlens,
+                                        self.scale, meta.max_seqlen,
+                                        self.window, sinks, tiles)
         return self.o_proj(out.reshape(T, -1))
 
 

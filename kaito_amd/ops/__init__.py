@@ -28,7 +28,8 @@ for _g, _names in {
              "gelu_and_mul gelu layer_norm fused_add_layer_norm "
              "rope_and_cache reshape_and_cache topk skinny_linear skinny_swiglu "
              "batch_linear"),
-    "attn": ("paged_attention paged_attention_sp prefill_attention "
+    "attn": ("paged_attention paged_attention_sp rope_paged_attention "
+             "prefill_attention "
              "mla_prefill_attention context_attention mfma_tile_gemm paged_read_bw"),
     "mla": "mla_decode mla_prepare head_rows mla_cache_write",
     "moe": ("moe_gate_silu moe_down_rows moe_up_pairs moe_down_pairs "
@@ -311,6 +312,13 @@ def reshape_and_cache(k: torch.Tensor, v: torch.Tensor, k_cache: torch.Tensor,
     torch_ref.reshape_and_cache(k, v, k_cache, v_cache, slot_mapping)
 
 
+def _whole_chunks(*rows: torch.Tensor) -> bool:
+    """bf16 rows of whole 16-byte chunks"""
+    return all(t.dim() == 2 and t.dtype == torch.bfloat16 and t.stride(1) == 1
+               and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
+               for t in rows)
+
+
 def rope_and_cache(positions: torch.Tensor, q: torch.Tensor, k: torch.Tensor,
                    v: torch.Tensor, head_dim: int, cos_sin: torch.Tensor,
                    k_cache: torch.Tensor, v_cache: torch.Tensor,
@@ -318,11 +326,7 @@ def rope_and_cache(positions: torch.Tensor, q: torch.Tensor, k: torch.Tensor,
     """rotary_embedding of q and k [T, heads * head_dim], then
     reshape_and_cache of k and v. Returns (q, k). One launch for rows of
     whole 16-byte chunks."""
-    rows = (q, k, v)
-    if q.is_cuda and all(
-            t.dim() == 2 and t.dtype == torch.bfloat16 and t.stride(1) == 1
-            and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
-            for t in rows) \
+    if q.is_cuda and _whole_chunks(q, k, v) \
             and cos_sin.size(1) % 16 == 0 and cos_sin.size(1) <= head_dim \
             and cos_sin.is_contiguous() and positions.is_contiguous() \
             and head_dim % 8 == 0 and k_cache.size(3) == head_dim \
@@ -373,6 +377,44 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         return out
     return torch_ref.paged_attention(q, k_cache, v_cache, block_tables,
                                      seq_lens, scale, window, sinks)
+
+
+def rope_paged_attention(positions: torch.Tensor, q: torch.Tensor,
+                         k: torch.Tensor, v: torch.Tensor, head_dim: int,
+                         cos_sin: torch.Tensor, k_cache: torch.Tensor,
+                         v_cache: torch.Tensor, slot_mapping: torch.Tensor,
+                         block_tables: torch.Tensor, seq_lens: torch.Tensor,
+                         scale: float, window: int = 0,
+                         sinks: torch.Tensor | None = None) -> torch.Tensor:
+    """rope_and_cache of q, k and v [T, heads * head_dim], then
+    paged_attention: decode rows, each of a sequence of its own with its own
+    key as the last of seq_lens. Returns [T, QH, head_dim]; q and k may or may
+    not be rotated afterwards. One launch for rotations of whole heads, up to
+    8192 (row, kv head) pairs: every wave rotates its queries anew (one launch
+    and two, us, 8 kv heads of 128: 1 row of 217 keys 7.6, 9.3; 16 of 3000 in
+    fp8 27.0, 29.8; 250 of 300 55.3, 56.4; 512 of 300 105, 107; 2048 of 220
+    296, 291)."""
+    QH, KH = q.size(1) // head_dim, k_cache.size(1)
+    if q.is_cuda and _PA_IMPL == "sp" and q.size(0) * KH <= 8192 \
+            and _whole_chunks(q, k, v) and cos_sin.size(1) == head_dim and head_dim in (64, 128, 256) \
+            and k_cache.size(2) == 16 and k_cache.size(3) == head_dim \
+            and k.size(1) == v.size(1) == KH * head_dim \
+            and k_cache.is_contiguous() and v_cache.is_contiguous() \
+            and cos_sin.is_contiguous() and positions.is_contiguous() \
+            and slot_mapping.is_contiguous() \
+            and positions.numel() == slot_mapping.numel() == q.size(0) \
+            == seq_lens.numel():
+        out = torch.empty(q.size(0), QH, head_dim, dtype=q.dtype,
+                          device=q.device)
+        _K.rope_paged_attention(
+            out, positions, q.unflatten(-1, (QH, head_dim)), k, v, cos_sin,
+            k_cache, v_cache, slot_mapping, block_tables, seq_lens, scale,
+            window, _sinks_arg(sinks, q.device))
+        return out
+    q, k = rope_and_cache(positions, q, k, v, head_dim, cos_sin, k_cache,
+                          v_cache, slot_mapping)
+    return paged_attention(q.unflatten(-1, (QH, head_dim)), k_cache, v_cache,
+                           block_tables, seq_lens, scale, window, sinks)
 
 
 def mla_decode(q: torch.Tensor, cache: torch.Tensor,

@@ -38,6 +38,11 @@
 // head), shared out over the lanes and read back from LDS none, with 8 heads 2 of
 // 16.
 //
+// ROPE takes q without its rotation and the row's own key and value beside the
+// pages: a launch of 4.5 us less before it. The wave of the last keys stores them
+// and then reads its pages as ever. The same bits as rope.hip and this kernel
+// behind it; 1 row of 217 keys 9.3 -> 7.6 us, 32 of a 1024-key window 23.1 -> 19.7.
+//
 // Cache layout: [num_blocks, KV_HEADS, BLOCK_SIZE, HEAD_DIM] bf16 | e4m3.
 #pragma once
 #include "flash_prefill.h"
@@ -77,6 +82,12 @@ struct DecodeArgs {
   const float *r1, *r2;             // [QH] or nullptr
   const short* gate;                // [T, ..]: sigmoid of it times the output
   int64_t gate_stride;
+  // ROPE: q comes without its rotation, the row's own key and value outside the
+  // pages; both go to their slot (< 0: none) first. positions as above
+  const short *k_row, *v_row;       // [T, KH * D]
+  int64_t k_stride, v_stride;
+  const float* cos_sin;             // [positions, D]
+  const int64_t* slots;             // [T]
 
   template <bool BIASED> KAITO_DEV int len(const int64_t row) const {
     return BIASED ? (int)positions[row] + 1 : seq_lens[row];
@@ -116,6 +127,53 @@ KAITO_DEV void store_head(const DecodeArgs& a, const int64_t row, const int QH,
   a.out[(row * QH + head) * D + d] = f32_to_bf16(v);
 }
 
+// The rotation of 8 dims x at d and their partners y at d + D / 2 of a head.
+// Products and rounding as the compiler forms them in rope.hip: the same bits.
+template <typename V>
+KAITO_DEV void rotate8(V& x, V& y, const float* cs, const int half) {
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    const float c = cs[j], s = cs[half + j];
+    const float a = (float)x[j], b = (float)y[j];
+    x[j] = (__bf16)__builtin_fmaf(a, c, -(b * s));
+    y[j] = (__bf16)__builtin_fmaf(b, c, a * s);
+  }
+}
+
+// One wave: the row's key, rotated, and its value go to their slot of the pages
+// and can be read from there by this wave.
+template <int D, bool FP8>
+KAITO_DEV void append_row(const DecodeArgs& a, const int64_t row, const int kvh,
+                          const float* cs, const int lane) {
+  const int64_t slot = a.slots[row];
+  if (slot < 0) return;             // uniform
+  const int64_t at = ((slot / BS * a.KH + kvh) * BS + slot % BS) * D;
+  auto put = [&](const void* cache, const int d, const hbf16x8 x) {
+    if constexpr (FP8) {
+      uint32_t w[4];
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        w[j] = f32x2_to_fp8x2((float)x[2 * j], (float)x[2 * j + 1]) & 0xffff;
+      const uint2 o = {w[0] | w[1] << 16, w[2] | w[3] << 16};
+      *reinterpret_cast<uint2*>((uint8_t*)const_cast<void*>(cache) + at + d) = o;
+    } else {
+      *reinterpret_cast<hbf16x8*>((short*)const_cast<void*>(cache) + at + d) = x;
+    }
+  };
+  const short* v = a.v_row + row * a.v_stride + kvh * D;
+  const short* k = a.k_row + row * a.k_stride + kvh * D;
+  if (lane < D / 8)
+    put(a.v, lane * 8, *reinterpret_cast<const hbf16x8*>(v + lane * 8));
+  if (lane < D / 16) {
+    hbf16x8 x = *reinterpret_cast<const hbf16x8*>(k + lane * 8);
+    hbf16x8 y = *reinterpret_cast<const hbf16x8*>(k + D / 2 + lane * 8);
+    rotate8(x, y, cs + lane * 8, D / 2);
+    put(a.k, lane * 8, x);
+    put(a.k, D / 2 + lane * 8, y);
+  }
+  __threadfence_block();            // ahead of this wave's loads of the page
+}
+
 // how a sequence's keys are shared out: 32-key tiles from the page that
 // holds the window's first key on, a contiguous run of `per` for every wave.
 // A split is the share of a workgroup's waves, so that with `used` == 1 the
@@ -134,7 +192,7 @@ KAITO_DEV Spans spans_of(const int seq_len, const int window, const int nsplit,
   return p;
 }
 
-template <int D, bool FP8, int NW, bool SPLIT, bool BIASED>
+template <int D, bool FP8, int NW, bool SPLIT, bool BIASED, bool ROPE>
 __global__ __launch_bounds__(NW * 64, NW <= 4 && D <= 128 ? 3 : 2)
 void paged_decode_kernel(const DecodeArgs a) {
   constexpr int KK = D / 32;        // 16x16x32 steps over the dims
@@ -179,6 +237,15 @@ void paged_decode_kernel(const DecodeArgs a) {
     for (int kk = 0; kk < KK; kk++)
       qf[kk] = *reinterpret_cast<const hbf16x8*>(
           qp + min(lo, a.G - 1) * D + hi * 8 + kk * 32);
+  }
+  if constexpr (ROPE) {
+    const float* cs = a.cos_sin + a.positions[seq] * D;
+    // the wave of the last key, which is the row's own
+    if (sp.tiles ? t0 < t1 && t1 == sp.tiles : wave == 0)
+      append_row<D, FP8>(a, seq, kvh, cs, lane);
+#pragma unroll
+    for (int kk = 0; kk < KK / 2; kk++)
+      rotate8(qf[kk], qf[kk + KK / 2], cs + hi * 8 + kk * 32, D / 2);
   }
   constexpr float NONE = BIASED ? -INFINITY : -1e30f;
   float m = NONE, l = 0.f;
@@ -476,7 +543,7 @@ void paged_fold_kernel(const DecodeArgs a, const int QH, const int splits) {
   store_head<BIASED>(a, row / QH, QH, (int)(row % QH), D, d, num, den);
 }
 
-template <int D, bool FP8, bool BIASED>
+template <int D, bool FP8, bool BIASED, bool ROPE = false>
 void launch_paged_decode(DecodeArgs a, const at::Tensor& out, int T) {
   auto stream = at::hip::getCurrentHIPStream();
   const int64_t pairs = (int64_t)T * a.KH;
@@ -504,7 +571,7 @@ void launch_paged_decode(DecodeArgs a, const at::Tensor& out, int T) {
   int64_t longest = (int64_t)a.max_blocks * BS;
   if (a.window > 0) longest = std::min<int64_t>(longest, a.window + BS);
 #define PA_LAUNCH(NW_, SPLIT_, GRID_)                                         \
-  hipLaunchKernelGGL((paged_decode_kernel<D, FP8, NW_, SPLIT_, BIASED>), GRID_,      \
+  hipLaunchKernelGGL((paged_decode_kernel<D, FP8, NW_, SPLIT_, BIASED, ROPE>), GRID_, \
                      dim3(NW_ * 64), 0, stream, a)
   const int64_t splits = std::min<int64_t>(
       {SPLIT_FILL / pairs, longest / (WIDE * KT * SPLIT_MIN), 64});

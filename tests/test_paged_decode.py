@@ -177,3 +177,50 @@ def test_weights_keep_f32(D, KH, gap, max_blocks):
     ref = (v1 + v2 - w) / (2 + w)
     err = ((out - ref[..., None]) / ref[..., None]).abs()
     assert err.max() < 2.0 ** -6, err.max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("G,KH,D", [(1, 2, 64), (8, 1, 64), (3, 2, 128),
+                                    (4, 8, 128), (4, 1, 256)])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("lens,max_blocks,window", [
+    (EDGES, 20, 0), (EDGES, 20, 40), ([1900, 33, 1, 2047], 128, 0),
+    ([1, 16, 17, 300] * 70, 19, 0)])
+def test_rotated_on_the_way(G, KH, D, fp8, lens, max_blocks, window):
+    """One launch or rope_and_cache and attention behind it: the same pages and
+    results, rows without a slot and slots of no sequence's page among them."""
+    torch.manual_seed(G * D + len(lens))
+    T, pages = len(lens), sum(-(-n // 16) for n in lens) + 2
+    perm = torch.randperm(pages)
+    bt = torch.zeros(T, max_blocks, dtype=torch.int32)
+    slots = torch.full((T,), -1)
+    at = 0
+    for i, n in enumerate(lens):
+        u = -(-n // 16)
+        bt[i, :u] = perm[at:at + u]
+        if n and i % 5 != 3:
+            slots[i] = int(bt[i, (n - 1) // 16]) * 16 + (n - 1) % 16
+        at += u
+    slots[0] = int(perm[-1]) * 16 + 5        # a page that nobody reads
+    dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    caches = [torch.randn(pages, KH, 16, D, device=DEV).to(dt) for _ in "kv"]
+    if fp8:
+        caches = [c.view(torch.uint8) for c in caches]
+    qkv = torch.randn(T, (G + 2) * KH * D + 8, device=DEV).to(torch.bfloat16)
+    q, k, v = qkv[:, 8:].split([G * KH * D, KH * D, KH * D], -1)
+    pos = torch.randint(0, 500, (T,), device=DEV)
+    cs = torch.randn(500, D, device=DEV)
+    bt, slots = bt.to(DEV), slots.to(DEV)
+    sl = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    sinks = torch.randn(G * KH, device=DEV) if window else None
+    a, b = ([c.clone() for c in caches] for _ in "ab")
+    before = qkv.clone()
+    out = ops.rope_paged_attention(pos, q, k, v, D, cs, *a, slots, bt, sl,
+                                   D ** -0.5, window, sinks)
+    assert torch.equal(qkv, before)
+    q, k = ops.rope_and_cache(pos, q, k, v, D, cs, *b, slots)
+    ref = ops.paged_attention(q.unflatten(-1, (-1, D)), *b, bt, sl, D ** -0.5,
+                              window, sinks)
+    for x, y in zip(a, b):
+        assert torch.equal(x, y)
+    assert torch.isfinite(out).all() and torch.equal(out, ref)
