@@ -197,9 +197,13 @@ def _skinny(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
     rows the library has another kernel for few rows of W and K of 2560 and
     more (1024 x 2560: 8.0, 6.9; 2048 x 2816: 8.8, 9.5; 1024 x 2816 as a pair
     9.0, 9.5)."""
-    if not _plain_rows(x, w, 32):
+    M = x.size(0)
+    if M > 32 or w.dim() != 2:
         return False
-    M, (N, K) = x.size(0), w.shape
+    return _skinny_shape(M, *w.shape, glu) and _plain_rows(x, w, 32)
+
+
+def _skinny_shape(M: int, N: int, K: int, glu: bool) -> bool:
     if M <= 4:
         return True
     if K % 64 or N % 16:
@@ -236,23 +240,27 @@ def _batched(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
     at 128 1.6; at K of 4096 only to 64 rows, 4096 x 4096 14.3, 15.3 there and
     18.6, 17.7 at 128; at K of 8192 only beyond 32 rows, 4096 x 8192 at 24
     20.6, 17.9); to 8192 between K of 4096 and 8192 (8192 x 7168: 1.02 to 1.47;
-    8192 x 4096 at 64 0.88, 8192 x 8192 at 64 0.84); 16384 and more to 64 rows
-    (1.03 to 1.16). 193 to 256 rows: 6144 to 16384 with K from 7168 (1.06 to
+    8192 x 4096 at 64 0.88, 8192 x 8192 at 64 0.84); 16384 to 65536 to 64 rows
+    (1.03 to 1.16; 128256 x 4096 at 32 206, 193). 193 to 256 rows: 6144 to 16384 with K from 7168 (1.06 to
     1.67; 4096 x 7168 0.91).
     SwiGLU pairs, which save a launch and a pass: from 12288 rows of W with
     more than 16 rows, 32 for K of 2048 (28672 x 4096: 48.9, 57.2 at 64, 73.6,
     79.8 at 256; 12288 x 2048 16.6, 20.2 at 64; 8192 x 4096 0.89), beyond 32768
     to 64 rows (57344 x 4096: 1.07 to 1.13, 0.90 at 256), at K of 8192 from
     20480 on (16384 x 8192 0.97)."""
-    if not _plain_rows(x, w, 256):
+    M = x.size(0)
+    if not 9 <= M <= 256 or w.dim() != 2:
         return False
-    M, (N, K) = x.size(0), w.shape
-    if M < 9 or K % 64 or N % (32 if glu else 16) \
-            or (N + 128) * K >= 1 << 31 or M * x.stride(0) >= 1 << 31:
+    return _batched_shape(M, *w.shape, glu) and _plain_rows(x, w, 256) \
+        and M * x.stride(0) < 1 << 31
+
+
+def _batched_shape(M: int, N: int, K: int, glu: bool) -> bool:
+    if K % 64 or N % (32 if glu else 16) or (N + 128) * K >= 1 << 31:
         return False
     if glu:
         return M > (16 if K > 2048 else 32) and K >= 2048 and N >= (
-            20480 if K >= 8192 else 12288) and (N <= 32768 or M <= 64)
+            20480 if K >= 8192 else 12288) and (N <= 32768 or (N <= 65536 and M <= 64))
     if K >= 10240:
         return 1024 <= N <= 16384
     if M < 17:
@@ -267,7 +275,7 @@ def _batched(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
         return M <= 64 if K == 4096 else K < 8192 or M > 32
     if N <= 8192:
         return 4096 < K < 8192
-    return N >= 16384 and K < 8192 and M <= 64
+    return 16384 <= N <= 65536 and K < 8192 and M <= 64
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
