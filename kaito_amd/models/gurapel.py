@@ -70,8 +70,12 @@ class HybridLayer(MixerLayerBase):
             y = self.mixer(xa, positions, self._view(cache, self.mixer), meta)
             xa = ops.post_norm_residual(x32, y, self.norm1, eps, dt)
         else:
-            ya = self.attn(xa, positions, self._view(cache, self.attn), meta)
-            yr = self.rglru(xa, positions, self._view(cache, self.rglru), meta)
+            a, r = self.attn, self.rglru
+            pa, pr = ops.linear_pair(xa, a.qkv_proj, xa, r.in_proj, None,
+                                     r.in_bias)
+            oa = a.mix(pa, positions, self._view(cache, a), meta)
+            yo = r.mix(pr, self._view(cache, r), meta)
+            ya, yr = ops.linear_pair(oa, a.o_proj, yo, r.o_proj)
             xa = ops.post_norm_residual(x32, ya, self.norm1, eps, dt, y2=yr,
                                         w_y=self.attn_out_norm,
                                         w_y2=self.rglru_out_norm)

@@ -150,18 +150,20 @@ class RGLRUMixer(nn.Module):
         return 0, max(s.conv_taps - 1, 1) * s.width * esz + s.width * 4
 
     def forward(self, x, positions, cache, meta):
-        s = self.spec
-        T, w = x.size(0), s.width
         p = ops.linear(x, self.in_proj, self.in_bias)
+        return ops.linear(self.mix(p, cache, meta), self.o_proj)
+
+    def mix(self, p, cache, meta):
+        """Between the projections: p, rows of in_proj's result."""
+        w = self.spec.width
         u = ops.causal_conv_update(
             p[:, w:], self.conv_weight, self.conv_bias, cache["conv"],
             meta.cu_seqlens, meta.state_slots, meta.seq_starts,
             meta.token_seq, act=0)
         gates = ops.rglru_gates(u, self.gate_w, self.gate_b)  # [B, T, 2bw]
-        o = ops.rglru_scan(u, gates, p[:, :w], self.decay_rate, cache["lru"],
-                           meta.cu_seqlens, meta.state_slots, meta.seq_starts,
-                           meta.token_seq)
-        return ops.linear(o, self.o_proj)
+        return ops.rglru_scan(u, gates, p[:, :w], self.decay_rate,
+                              cache["lru"], meta.cu_seqlens, meta.state_slots,
+                              meta.seq_starts, meta.token_seq)
 
 
 class BiasedWindowAttention(nn.Module):
@@ -208,9 +210,12 @@ class BiasedWindowAttention(nn.Module):
         return s.kv_heads * block_size * (s.dim + s.vdim) * esz, 0
 
     def forward(self, x, positions, cache, meta):
-        s = self.spec
-        T = x.size(0)
         qkv = ops.linear(x, self.qkv_proj)
+        return ops.linear(self.mix(qkv, positions, cache, meta), self.o_proj)
+
+    def mix(self, qkv, positions, cache, meta):
+        """Between the projections: qkv, rows of qkv_proj's result."""
+        s = self.spec
         q = qkv[:, :self.q_size].unflatten(-1, (s.heads, s.dim))
         k = qkv[:, self.q_size:self.q_size + self.k_size].unflatten(
             -1, (s.kv_heads, s.dim))
@@ -227,7 +232,7 @@ class BiasedWindowAttention(nn.Module):
                                  meta.block_tables, meta.token_seq, positions,
                                  s.scale, s.softcap, self.r1, self.r2,
                                  s.window, tiles=tiles)
-        return ops.linear(o.reshape(T, -1), self.o_proj)
+        return o.reshape(qkv.size(0), -1)
 
 
 class RotaryWindowAttention(nn.Module):

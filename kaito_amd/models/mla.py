@@ -122,24 +122,27 @@ class MLAAttention(nn.Module):
         self.o_proj.fuse_norm = not cfg.parallel_block \
             and not cfg.sandwich_norms and cfg.norm_type == "rmsnorm"
 
-    def _project_q(self, x: torch.Tensor) -> torch.Tensor:
+    def _project(self, x: torch.Tensor):
+        """Queries [T, heads, nope + rope] and latent rows [T, r + rope]."""
+        w = self.kv_a_proj_with_mqa
         if self.cfg.q_lora_rank > 0:
-            qa = ops.linear(x, self.q_a_proj)
+            qa, kv_a = ops.linear_pair(x, self.q_a_proj, x, w)
             qa = ops.rms_norm(qa, self.q_a_layernorm, self.cfg.rms_eps)
             q = self.q_b_proj(qa)
+        elif self.q_proj.is_plain():
+            q, kv_a = ops.linear_pair(x, self.q_proj.weight, x, w)
         else:
-            q = self.q_proj(x)
-        return q.view(-1, self.num_heads, self.qk_dim)
+            q, kv_a = self.q_proj(x), ops.linear(x, w)
+        return q.view(-1, self.num_heads, self.qk_dim), kv_a
 
     def forward(self, x: torch.Tensor, positions: torch.Tensor,
                 kv_cache: Optional[Tuple[torch.Tensor, torch.Tensor]],
                 meta, cos_sin: torch.Tensor,
                 cos_sin_local: Optional[torch.Tensor] = None) -> torch.Tensor:
         T = x.size(0)
-        q = self._project_q(x)                          # [T, Hl, nope+rope]
+        q, kv_a = self._project(x)
         q_nope = q[..., :self.nope]
         q_pe = q[..., self.nope:]                       # [T, Hl, rope]
-        kv_a = ops.linear(x, self.kv_a_proj_with_mqa)
         if x.is_cuda and x.dtype == torch.bfloat16 \
                 and (self.r, self.rope, cos_sin.size(1)) == (512, 64, 64) \
                 and self.nope % 8 == 0 and q.data_ptr() % 16 == 0:

@@ -27,7 +27,7 @@ for _g, _names in {
     "core": ("rms_norm fused_add_rms_norm rotary_embedding silu_and_mul "
              "gelu_and_mul gelu layer_norm fused_add_layer_norm "
              "rope_and_cache reshape_and_cache topk skinny_linear skinny_swiglu "
-             "batch_linear"),
+             "skinny_linear_pair batch_linear"),
     "attn": ("paged_attention paged_attention_sp rope_paged_attention "
              "prefill_attention "
              "mla_prefill_attention context_attention mfma_tile_gemm paged_read_bw"),
@@ -295,6 +295,31 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
                 _K.batch_linear(out, x, w, _none(bias, x), 0, 0, False)
             return out
     return torch.nn.functional.linear(x, w, bias)
+
+
+def linear_pair(x: torch.Tensor, w: torch.Tensor, x2: torch.Tensor,
+                w2: torch.Tensor, bias=None, bias2=None):
+    """(linear(x, w, bias), linear(x2, w2, bias2)): products that do not wait
+    for one another, of the same K. One launch where both stream their weights
+    (us, two launches and one, 32 rows, K of 2048: 3072 and 576 rows of W 14.8, 8.3,
+    3072 and 4096 of one x 16.3, 12.2, 2048 and 2048 of two 14.5, 8.8; one row
+    6.9, 4.9, 9.4, 6.7 and 7.2, 5.1)."""
+    if x.size(0) == x2.size(0) <= 32 and x.dim() == x2.dim() == 2 \
+            and w.size(1) == w2.size(1) and x.device == x2.device \
+            and w.size(0) % 16 == w2.size(0) % 16 == 0 \
+            and _skinny(x, w) and _skinny(x2, w2) and all(
+                b is None or (b.dtype == torch.bfloat16 and b.is_contiguous()
+                              and b.shape == v.shape[:1]
+                              and b.device == v.device
+                              and not (torch.is_grad_enabled()
+                                       and b.requires_grad))
+                for b, v in ((bias, w), (bias2, w2))):
+        out, out2 = (torch.empty(x.size(0), v.size(0), dtype=x.dtype,
+                                 device=x.device) for v in (w, w2))
+        _K.skinny_linear_pair(out, x, w, _none(bias, x), out2, x2, w2,
+                              _none(bias2, x))
+        return out, out2
+    return linear(x, w, bias), linear(x2, w2, bias2)
 
 
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

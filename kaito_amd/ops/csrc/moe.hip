@@ -206,8 +206,8 @@ KAITO_DEV void stream_pass(const StreamArgs& a, const int le, const int ntiles,
   const int64_t wrows = GATED ? 2 * a.N : a.N;
   const int slot = threadIdx.x, l = slot & 63, c = l & 15;
   const bool mine = slot < MT * 64 && !(GATED && c >= 8);
-  skinny::stream_tiles<MT, S>(
-      a.w + le * wrows * a.K,
+  skinny::stream_tiles<MT, S, false>(
+      a.w + le * wrows * a.K, nullptr, 0,
       [&](const int j) {
         const int r = skinny::tile_row<KS>(j, lane);
         const uint32_t n = GATED ? r % 8 + (r >= 8 ? a.N : 0) : r;

@@ -5,6 +5,7 @@
 #include <torch/library.h>
 #include <ATen/ATen.h>
 #include <ATen/hip/HIPContext.h>
+#include <type_traits>
 
 namespace kaito {
 
@@ -12,15 +13,36 @@ namespace {
 
 constexpr int NW = 4;
 
+// One product; two of the same K and rows of x (of one x or of two) share a
+// launch, the second's workgroups behind the first's.
+struct Part {
+  short* out;                       // [M, N]
+  const short* x;
+  int64_t x_stride;
+  const short* w;                   // [N, K]; GLU [2 N, K]
+  const short* bias;                // [N] or nullptr
+  int N;
+};
+struct Parts {
+  Part part[2];
+  int first;                        // workgroups (staying ones: tiles) of part 0
+  int M, K;
+};
+
 // GLU: the wave's two rows are a gate row and its up row (N apart)
 template <int M, int R, bool GLU>
-__global__ __launch_bounds__(NW * 64) void skinny_linear_kernel(
-    short* __restrict__ out, const short* __restrict__ x,
-    const int64_t x_stride, const short* __restrict__ w,
-    const short* __restrict__ bias, const int N, const int K) {
+__global__ __launch_bounds__(NW * 64) void skinny_linear_kernel(const Parts a) {
+  const int second = (int)blockIdx.x >= a.first;
+  const Part p = second ? a.part[1] : a.part[0];
+  short* __restrict__ out = p.out;
+  const short* __restrict__ x = p.x;
+  const short* __restrict__ w = p.w;
+  const short* __restrict__ bias = p.bias;
+  const int64_t x_stride = p.x_stride;
+  const int N = p.N, K = a.K;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n0 = (blockIdx.x * NW + wave) * (GLU ? 1 : R);
+  const int n0 = ((blockIdx.x - second * a.first) * NW + wave) * (GLU ? 1 : R);
   if (n0 >= N) return;
   const short* wp[R];
   float acc[M][R];
@@ -52,16 +74,21 @@ __global__ __launch_bounds__(NW * 64) void skinny_linear_kernel(
 // M <= 16 MT rows; N is a multiple of 16 (GLU: of 8, the workgroup's 16 rows
 // are 8 gate rows and their up rows, N apart), K of the stage
 template <int MT, int KS, bool GLU>
-__global__ __launch_bounds__(256, 2) void skinny_tile_kernel(
-    short* __restrict__ out, const short* __restrict__ x,
-    const int64_t x_stride, const short* __restrict__ w,
-    const short* __restrict__ bias, const int M, const int N, const int K) {
+__global__ __launch_bounds__(256, 2) void skinny_tile_kernel(const Parts a) {
+  const int second = (int)blockIdx.x >= a.first;
+  const Part p = second ? a.part[1] : a.part[0];
+  short* __restrict__ out = p.out;
+  const short* __restrict__ x = p.x;
+  const short* __restrict__ w = p.w;
+  const short* __restrict__ bias = p.bias;
+  const int64_t x_stride = p.x_stride;
+  const int M = a.M, N = p.N, K = a.K;
   constexpr int NI = skinny::tile_loads<KS>();
   __shared__ __attribute__((aligned(128))) short ring[4][2][16 * KS];
   static_assert(sizeof(ring) >= 4 * MT * 64 * sizeof(f32x4), "fold");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n0 = blockIdx.x * (GLU ? 8 : 16);
+  const int n0 = (blockIdx.x - second * a.first) * (GLU ? 8 : 16);
   const short *src[NI], *xp[MT];
 #pragma unroll
   for (int j = 0; j < NI; j++) {
@@ -101,38 +128,42 @@ __global__ __launch_bounds__(256, 2) void skinny_tile_kernel(
   }
 }
 
-// K = 1024 S: see skinny::stream_tiles. gridDim.x workgroups share the tiles.
-template <int MT, int S, bool GLU>
-__global__ __launch_bounds__(256, 2) void skinny_tiles_kernel(
-    short* __restrict__ out, const short* __restrict__ x,
-    const int64_t x_stride, const short* __restrict__ w,
-    const short* __restrict__ bias, const int M, const int N, const int K) {
+// K = 1024 S: see skinny::stream_tiles. gridDim.x workgroups share the tiles of
+// both parts, which have one x.
+template <int MT, int S, bool GLU, bool TWO>
+__global__ __launch_bounds__(256, 2) void skinny_tiles_kernel(const Parts a) {
   constexpr int KS = skinny::TILES_KS, TW = skinny::TILE_NW;
   constexpr int COLS = GLU ? 8 : 16;
   __shared__ __attribute__((aligned(128))) short ring[TW][2][16 * KS];
   __shared__ f32x4 red[2][TW][MT * 64];
+  const Part p = a.part[0], p2 = a.part[TWO];
+  const int M = a.M, K = a.K, first = a.first;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int slot = threadIdx.x, l = slot & 63, c = l & 15;
   const bool mine = slot < MT * 64 && !(GLU && c >= 8);
-  skinny::stream_tiles<MT, S>(
-      w,
+  skinny::stream_tiles<MT, S, TWO>(
+      p.w, p2.w, first,
       [&](const int j) {
         const int r = skinny::tile_row<KS>(j, lane);
-        const uint32_t n = GLU ? r % 8 + (r >= 8 ? N : 0) : r;
+        const uint32_t n = GLU ? r % 8 + (r >= 8 ? p.N : 0) : r;
         return (n * K + skinny::tile_col<KS>(j, lane)) * 2;
       },
-      COLS * K * 2, blockIdx.x, gridDim.x, N / COLS,
+      COLS * K * 2, blockIdx.x, gridDim.x, first + (TWO ? p2.N / COLS : 0),
       [&](const short* (&xp)[MT]) {
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
-          xp[mt] = x + min(mt * 16 + (lane & 15), M - 1) * x_stride +
+          xp[mt] = p.x + min(mt * 16 + (lane & 15), M - 1) * p.x_stride +
               (lane >> 4) * 8;
       },
       ring[wave][0], &red[0][0][0], wave, lane,
       [&](const int t, const f32x4* sums) {
         if (!mine) return;
-        const int n = t * COLS + c;
+        const bool second = TWO && t >= first;
+        const int N = second ? p2.N : p.N;
+        const short* bias = second ? p2.bias : p.bias;
+        short* out = second ? p2.out : p.out;
+        const int n = (second ? t - first : t) * COLS + c;
         f32x4 v = skinny::fold<MT, TW>(sums, slot);
         if constexpr (GLU) {
           const f32x4 u = skinny::fold<MT, TW>(sums, slot + 8);
@@ -172,10 +203,9 @@ bool in_tiles(int64_t M, int64_t N, int64_t K, int64_t cols, int64_t weights) {
 // workgroups per CU are no faster (1792 of a pair 42.8).
 constexpr int WORKGROUPS = 256;
 
-bool many_tiles(int M, int64_t tiles, const at::Tensor& w) {
+bool many_tiles(int M, int64_t tiles, int64_t weights, int64_t K) {
   return tiles >= (M > 16 ? WORKGROUPS + 64 : 3 * WORKGROUPS) &&
-         w.numel() < (1ll << 31) &&
-         (w.size(1) == 2048 || (w.size(1) == 4096 && M <= 16));
+         weights < (1ll << 31) && (K == 2048 || (K == 4096 && M <= 16));
 }
 
 void check(const at::Tensor& out, const at::Tensor& x, const at::Tensor& w,
@@ -194,62 +224,104 @@ void check(const at::Tensor& out, const at::Tensor& x, const at::Tensor& w,
               "more than 4 rows: K in whole stages, N in whole tiles");
 }
 
+template <typename Kernel>
+void launch(Kernel kernel, int64_t workgroups, const Parts& a) {
+  hipLaunchKernelGGL(kernel, dim3(workgroups),
+                     dim3(256), 0, at::hip::getCurrentHIPStream(), a);
+}
+
+// `cols` output columns of a tile or, GLU, half of its 16 rows of W
+template <bool GLU>
+void run(Parts a, bool shared_x) {
+  constexpr int cols = GLU ? 8 : 16;
+  const int64_t K = a.K, N0 = a.part[0].N, N1 = a.part[1].N, N = N0 + N1;
+  const int64_t weights = (GLU ? 2 : 1) * N * K;
+  const int M = a.M;
+  if (in_tiles(M, N0 % cols ? N0 : N, K, cols, weights)) {
+    a.first = (int)(N0 / cols);
+    if (shared_x && many_tiles(M, N / cols, weights, K)) {
+      auto stay = [&](auto two) {
+        constexpr bool TWO = decltype(two)::value;
+        if (K == 4096)
+          launch(&skinny_tiles_kernel<1, 4, GLU, TWO>, WORKGROUPS, a);
+        else if (M > 16)
+          launch(&skinny_tiles_kernel<2, 2, GLU, TWO>, WORKGROUPS, a);
+        else
+          launch(&skinny_tiles_kernel<1, 2, GLU, TWO>, WORKGROUPS, a);
+      };
+      if (GLU || N1 == 0) stay(std::false_type{});
+      else stay(std::bool_constant<!GLU>{});
+    } else if (K % 256 == 0) {
+      if (M > 16) launch(&skinny_tile_kernel<2, 256, GLU>, N / cols, a);
+      else launch(&skinny_tile_kernel<1, 256, GLU>, N / cols, a);
+    } else {
+      if (M > 16) launch(&skinny_tile_kernel<2, 64, GLU>, N / cols, a);
+      else launch(&skinny_tile_kernel<1, 64, GLU>, N / cols, a);
+    }
+    return;
+  }
+  // one row per wave keeps most waves under way for a single x row (N =
+  // 4096, K = 4096: 6.6 us against 6.8 with two); with more, two rows share
+  // the x loads (M = 4, N = 28672: 48 us)
+  const int64_t per = NW * (GLU || M == 1 ? 1 : 2);
+  a.first = (int)((N0 + per - 1) / per);
+  const int64_t grid = a.first + (N1 + per - 1) / per;
+  switch (M) {
+    case 1: launch(&skinny_linear_kernel<1, GLU ? 2 : 1, GLU>, grid, a); break;
+    case 2: launch(&skinny_linear_kernel<2, 2, GLU>, grid, a); break;
+    case 3: launch(&skinny_linear_kernel<3, 2, GLU>, grid, a); break;
+    default: launch(&skinny_linear_kernel<4, 2, GLU>, grid, a); break;
+  }
+}
+
+Part part_of(const at::Tensor& out, const at::Tensor& x, const at::Tensor& w,
+             int64_t N) {
+  return {(short*)out.data_ptr(), (const short*)x.data_ptr(), x.stride(0),
+          (const short*)w.data_ptr(), nullptr, (int)N};
+}
+
+Part part_of(const at::Tensor& out, const at::Tensor& x, const at::Tensor& w,
+             const at::Tensor& bias) {
+  const int64_t N = w.size(0);
+  Part p = part_of(out, x, w, N);
+  if (bias.numel() > 0) {
+    TORCH_CHECK(bias.is_cuda() && bias.is_contiguous() &&
+                bias.dtype() == at::kBFloat16 && bias.numel() == N);
+    p.bias = (const short*)bias.data_ptr();
+  }
+  return p;
+}
+
 }  // namespace
 
 void skinny_linear(at::Tensor out, at::Tensor x, at::Tensor w,
                    at::Tensor bias) {
   const int64_t N = w.size(0);
   check(out, x, w, N, 16);
-  const bool has_bias = bias.numel() > 0;
-  TORCH_CHECK(!has_bias || (bias.is_cuda() && bias.is_contiguous() &&
-                            bias.dtype() == at::kBFloat16 &&
-                            bias.numel() == N));
   if (N == 0) return;
-  // one row per wave keeps most waves under way for a single x row (N =
-  // 4096, K = 4096: 6.6 us against 6.8 with two); with more, two rows share
-  // the x loads (M = 4, N = 28672: 48 us)
-#define SL_LAUNCH(M_, R_)                                                     \
-  hipLaunchKernelGGL((skinny_linear_kernel<M_, R_, false>),                   \
-      dim3((N + NW * R_ - 1) / (NW * R_)), dim3(NW * 64), 0,                  \
-      at::hip::getCurrentHIPStream(), (short*)out.data_ptr(),                 \
-      (const short*)x.data_ptr(), x.stride(0), (const short*)w.data_ptr(),    \
-      has_bias ? (const short*)bias.data_ptr() : nullptr, (int)N,             \
-      (int)w.size(1))
-  const int M = x.size(0);
-#define SLT_LAUNCH(MT_, KS_)                                                  \
-  hipLaunchKernelGGL((skinny_tile_kernel<MT_, KS_, false>), dim3(N / 16),         \
-      dim3(256), 0, at::hip::getCurrentHIPStream(), (short*)out.data_ptr(),   \
-      (const short*)x.data_ptr(), x.stride(0), (const short*)w.data_ptr(),    \
-      has_bias ? (const short*)bias.data_ptr() : nullptr, M, (int)N, (int)w.size(1))
-#define SLTS_LAUNCH(MT_, S_)                                                  \
-  hipLaunchKernelGGL((skinny_tiles_kernel<MT_, S_, false>),                    \
-      dim3(WORKGROUPS), dim3(256), 0, at::hip::getCurrentHIPStream(),         \
-      (short*)out.data_ptr(), (const short*)x.data_ptr(), x.stride(0),        \
-      (const short*)w.data_ptr(),                                             \
-      has_bias ? (const short*)bias.data_ptr() : nullptr, M, (int)N, (int)w.size(1))
-  if (in_tiles(M, N, w.size(1), 16, w.numel())) {
-    if (many_tiles(M, N / 16, w)) {
-      if (w.size(1) == 4096) SLTS_LAUNCH(1, 4);
-      else if (M > 16) SLTS_LAUNCH(2, 2);
-      else SLTS_LAUNCH(1, 2);
-      return;
-    }
-    if (w.size(1) % 256 == 0) {
-      if (M > 16) SLT_LAUNCH(2, 256); else SLT_LAUNCH(1, 256);
-    } else {
-      if (M > 16) SLT_LAUNCH(2, 64); else SLT_LAUNCH(1, 64);
-    }
-    return;
-  }
-#undef SLT_LAUNCH
-#undef SLTS_LAUNCH
-  switch (M) {
-    case 1: SL_LAUNCH(1, 1); break;
-    case 2: SL_LAUNCH(2, 2); break;
-    case 3: SL_LAUNCH(3, 2); break;
-    default: SL_LAUNCH(4, 2); break;
-  }
-#undef SL_LAUNCH
+  Parts a{};
+  a.part[0] = part_of(out, x, w, bias);
+  a.M = (int)x.size(0);
+  a.K = (int)w.size(1);
+  run<false>(a, true);
+}
+
+// two products of as many rows and the same K in one launch
+void skinny_linear_pair(at::Tensor out, at::Tensor x, at::Tensor w,
+                        at::Tensor bias, at::Tensor out2, at::Tensor x2,
+                        at::Tensor w2, at::Tensor bias2) {
+  const int64_t N = w.size(0), N2 = w2.size(0);
+  check(out, x, w, N, 16);
+  check(out2, x2, w2, N2, 16);
+  TORCH_CHECK(x2.size(0) == x.size(0) && w2.size(1) == w.size(1) &&
+              N % 16 == 0 && N2 % 16 == 0 && N > 0 && N2 > 0 &&
+              N + N2 < (1ll << 31));
+  Parts a{};
+  a.part[0] = part_of(out, x, w, bias);
+  a.part[1] = part_of(out2, x2, w2, bias2);
+  a.M = (int)x.size(0);
+  a.K = (int)w.size(1);
+  run<false>(a, x.data_ptr() == x2.data_ptr() && x.stride(0) == x2.stride(0));
 }
 
 void skinny_swiglu(at::Tensor out, at::Tensor x, at::Tensor w) {
@@ -257,56 +329,22 @@ void skinny_swiglu(at::Tensor out, at::Tensor x, at::Tensor w) {
   const int64_t N = w.size(0) / 2;
   check(out, x, w, N, 8);
   if (N == 0) return;
-  const int M = x.size(0);
-#define SGT_LAUNCH(MT_, KS_)                                                  \
-  hipLaunchKernelGGL((skinny_tile_kernel<MT_, KS_, true>), dim3(N / 8),         \
-      dim3(256), 0, at::hip::getCurrentHIPStream(), (short*)out.data_ptr(),   \
-      (const short*)x.data_ptr(), x.stride(0), (const short*)w.data_ptr(),    \
-      nullptr, M, (int)N, (int)w.size(1))
-#define SGTS_LAUNCH(MT_, S_)                                                  \
-  hipLaunchKernelGGL((skinny_tiles_kernel<MT_, S_, true>),                    \
-      dim3(WORKGROUPS), dim3(256), 0, at::hip::getCurrentHIPStream(),         \
-      (short*)out.data_ptr(), (const short*)x.data_ptr(), x.stride(0),        \
-      (const short*)w.data_ptr(),                                             \
-      nullptr, M, (int)N, (int)w.size(1))
-  if (in_tiles(M, N, w.size(1), 8, w.numel())) {
-    if (many_tiles(M, N / 8, w)) {
-      if (w.size(1) == 4096) SGTS_LAUNCH(1, 4);
-      else if (M > 16) SGTS_LAUNCH(2, 2);
-      else SGTS_LAUNCH(1, 2);
-      return;
-    }
-    if (w.size(1) % 256 == 0) {
-      if (M > 16) SGT_LAUNCH(2, 256); else SGT_LAUNCH(1, 256);
-    } else {
-      if (M > 16) SGT_LAUNCH(2, 64); else SGT_LAUNCH(1, 64);
-    }
-    return;
-  }
-#undef SGT_LAUNCH
-#undef SGTS_LAUNCH
-#define SG_LAUNCH(M_)                                                         \
-  hipLaunchKernelGGL((skinny_linear_kernel<M_, 2, true>),                     \
-      dim3((N + NW - 1) / NW), dim3(NW * 64), 0,                              \
-      at::hip::getCurrentHIPStream(), (short*)out.data_ptr(),                 \
-      (const short*)x.data_ptr(), x.stride(0), (const short*)w.data_ptr(),    \
-      nullptr, (int)N, (int)w.size(1))
-  switch (M) {
-    case 1: SG_LAUNCH(1); break;
-    case 2: SG_LAUNCH(2); break;
-    case 3: SG_LAUNCH(3); break;
-    default: SG_LAUNCH(4); break;
-  }
-#undef SG_LAUNCH
+  Parts a{};
+  a.part[0] = part_of(out, x, w, N);
+  a.M = (int)x.size(0);
+  a.K = (int)w.size(1);
+  run<true>(a, true);
 }
 
 }  // namespace kaito
 
 TORCH_LIBRARY_FRAGMENT(kaito, m) {
   m.def("skinny_linear(Tensor(a!) out, Tensor x, Tensor w, Tensor bias) -> ()");
+  m.def("skinny_linear_pair(Tensor(a!) out, Tensor x, Tensor w, Tensor bias, Tensor(b!) out2, Tensor x2, Tensor w2, Tensor bias2) -> ()");
   m.def("skinny_swiglu(Tensor(a!) out, Tensor x, Tensor w) -> ()");
 }
 TORCH_LIBRARY_IMPL(kaito, CUDA, m) {
   m.impl("skinny_linear", &kaito::skinny_linear);
+  m.impl("skinny_linear_pair", &kaito::skinny_linear_pair);
   m.impl("skinny_swiglu", &kaito::skinny_swiglu);
 }

@@ -248,3 +248,28 @@ def test_swiglu_of_every_gate():
     # and what is left of results below f32's normal range
     bound = (2.0 ** -8 + 2.0 ** -16) * ref.abs()[both] + 2.0 ** -126
     assert (err <= bound).all(), (err / bound).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 16, 17, 32])
+@pytest.mark.parametrize("N,N2,K", [
+    (16, 48, 64), (48, 16, 256), (320, 48, 2048), (5136, 16, 2048),
+    (16, 5136, 2048), (6144, 6160, 4096), (112, 80, 1792)])
+def test_pairs(M, N, N2, K):
+    """Two products in one launch: the bits of two launches of a kernel, f32
+    sums of either kernel where the pair has tiles enough to stay."""
+    g = torch.Generator(device=DEV).manual_seed(M * N + K)
+    big = torch.randn(M, K + 16, device=DEV, generator=g).to(torch.bfloat16)
+    x, x2 = big[:, 8:8 + K], big[:, 16:16 + K]
+    w, w2 = (torch.randn(n, K, device=DEV, generator=g).to(torch.bfloat16)
+             for n in (N, N2))
+    b, b2 = (torch.randn(n, device=DEV, generator=g).to(torch.bfloat16)
+             for n in (N, N2))
+    for y in (x, x2):
+        out = [torch.full((M, n), float("nan"), dtype=torch.bfloat16,
+                          device=DEV) for n in (N, N2)]
+        if M <= 16 or K == 2048 or N * K <= 3072 * 2048:
+            _close(ops.linear_pair(x, w, y, w2)[1], y.double() @ w2.double().T)
+        ops._K.skinny_linear_pair(out[0], x, w, b, out[1], y, w2, b2)
+        _close(out[0], x.double() @ w.double().T + b.double())
+        _close(out[1], y.double() @ w2.double().T + b2.double())
