@@ -146,10 +146,16 @@ class MLAAttention(nn.Module):
         if x.is_cuda and x.dtype == torch.bfloat16 \
                 and (self.r, self.rope, cos_sin.size(1)) == (512, 64, 64) \
                 and self.nope % 8 == 0 and q.data_ptr() % 16 == 0:
-            q_pe, c_kv, k_pe = ops.mla_prepare(
-                q_pe, kv_a, self.kv_a_layernorm, self.cfg.rms_eps, positions,
-                cos_sin, None if kv_cache is None else kv_cache[0],
-                None if kv_cache is None else meta.slot_mapping)
+            args = (q_pe, kv_a, self.kv_a_layernorm, self.cfg.rms_eps,
+                    positions, cos_sin,
+                    None if kv_cache is None else kv_cache[0],
+                    None if kv_cache is None else meta.slot_mapping)
+            if not meta.is_prefill:
+                q_c, q_pe, _, _ = ops.mla_prepare_rows(q_nope, self.w_kc,
+                                                       *args)
+                out = self._decode(q_c, q_pe, kv_cache[0], meta)
+                return self.o_proj(out.reshape(T, -1))
+            q_pe, c_kv, k_pe = ops.mla_prepare(*args)
         else:
             q_pe, c_kv, k_pe = self._prepare(q_pe, kv_a, positions, cos_sin,
                                              kv_cache, meta)
@@ -162,7 +168,8 @@ class MLAAttention(nn.Module):
             else:
                 out = self._prefill(q_nope, q_pe, c_kv, k_pe, meta)
         else:
-            out = self._decode(q_nope, q_pe, kv_cache[0], meta)
+            out = self._decode(ops.head_rows(q_nope, self.w_kc), q_pe,
+                               kv_cache[0], meta)
         return self.o_proj(out.reshape(T, -1))
 
     def _prepare(self, q_pe, kv_a, positions, cos_sin, kv_cache, meta):
@@ -190,11 +197,10 @@ class MLAAttention(nn.Module):
         return q_pe.view(T, self.num_heads, self.rope), c_kv, k_pe
 
     # ---- absorbed decode over the latent cache --------------------------
-    def _decode(self, q_nope, q_pe, cache, meta) -> torch.Tensor:
-        T = q_nope.size(0)
-        # q_c[h] = q_nope[h] @ w_kc[h], read by the kernel where the product
-        # leaves it
-        q_c = ops.head_rows(q_nope, self.w_kc)          # [T, Hl, r]
+    def _decode(self, q_c, q_pe, cache, meta) -> torch.Tensor:
+        """q_c [T, Hl, r]: q_nope[h] @ w_kc[h], read by the kernel where the
+        product leaves it."""
+        T = q_c.size(0)
         out_c = ops.mla_decode(q_c, cache, meta.block_tables, meta.seq_lens,
                                self.scale, self.r, q_pe)
         # latent -> per-head v

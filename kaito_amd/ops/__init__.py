@@ -31,7 +31,7 @@ for _g, _names in {
     "attn": ("paged_attention paged_attention_sp rope_paged_attention "
              "prefill_attention "
              "mla_prefill_attention context_attention mfma_tile_gemm paged_read_bw"),
-    "mla": "mla_decode mla_prepare head_rows mla_cache_write",
+    "mla": "mla_decode mla_prepare mla_prepare_rows head_rows mla_cache_write",
     "moe": ("moe_gate_silu moe_down_rows moe_up_pairs moe_down_pairs "
             "moe_grouped_up moe_grouped_down moe_combine moe_combine_norm"),
     "route": "moe_route moe_gate_route moe_norm_gate_route moe_sort",
@@ -485,22 +485,47 @@ def mla_prepare(q: torch.Tensor, kv_a: torch.Tensor, w: torch.Tensor,
     return q_out, c, k
 
 
+def _head_rows_fit(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """The library is ahead from 32 rows of 128 heads on (us, 512 x 128: 14.4,
+    13.8; 24 rows 13.0, 13.6; 64 heads 8.9, 12.9; 16 heads 6.7, 12.8)."""
+    T, H, K = x.shape
+    return x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and T <= 32 \
+        and T * H <= 3072 and K % 64 == 0 and 0 < K <= 512 \
+        and w.size(2) % 32 == 0 and w.is_contiguous() \
+        and w.data_ptr() % 16 == 0 and x.stride(2) == 1 \
+        and x.stride(0) % 4 == 0 and x.stride(1) % 4 == 0 \
+        and x.data_ptr() % 8 == 0
+
+
 def head_rows(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x [T, H, K] (any token and head strides) times w [H, K, N] per head:
     [T, H, N]. One launch for up to 32 rows, a batched library product and
-    its transposition beyond: W is read once per 32 rows. The library is
-    ahead from 32 rows of 128 heads on (us, 512 x 128: 14.4, 13.8; 24 rows
-    13.0, 13.6; 64 heads 8.9, 12.9; 16 heads 6.7, 12.8)."""
-    T, H, K = x.shape
-    if x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and T <= 32 \
-            and T * H <= 3072 and K % 64 == 0 and 0 < K <= 512 and w.size(2) % 32 == 0 \
-            and w.is_contiguous() and w.data_ptr() % 16 == 0 \
-            and x.stride(2) == 1 and x.stride(0) % 4 == 0 \
-            and x.stride(1) % 4 == 0 and x.data_ptr() % 8 == 0:
-        y = torch.empty(T, H, w.size(2), dtype=x.dtype, device=x.device)
+    its transposition beyond: W is read once per 32 rows."""
+    if _head_rows_fit(x, w):
+        y = torch.empty(*x.shape[:2], w.size(2), dtype=x.dtype,
+                        device=x.device)
         _K.head_rows(y, x, w)
         return y
     return torch.bmm(x.transpose(0, 1), w).transpose(0, 1)
+
+
+def mla_prepare_rows(x: torch.Tensor, wx: torch.Tensor, q: torch.Tensor,
+                     kv_a: torch.Tensor, w: torch.Tensor, eps: float,
+                     positions: torch.Tensor, cos_sin: torch.Tensor,
+                     cache: torch.Tensor | None, slots: torch.Tensor | None):
+    """(head_rows(x, wx), *mla_prepare(q, ...)); one launch where head_rows
+    is one."""
+    if not _head_rows_fit(x, wx) or x.size(0) != q.size(0):
+        return head_rows(x, wx), *mla_prepare(q, kv_a, w, eps, positions,
+                                              cos_sin, cache, slots)
+    T, H, P = q.shape
+    y, q_out, c, k = (torch.empty(*s, dtype=q.dtype, device=q.device)
+                      for s in ((T, x.size(1), wx.size(2)), (T, H, P),
+                                (T, w.numel()), (T, P)))
+    _K.mla_prepare_rows(q_out, c, k, _none(cache, q), q, kv_a, w, eps,
+                        positions, cos_sin,
+                        positions if slots is None else slots, y, x, wx)
+    return y, q_out, c, k
 
 
 def mla_cache_write(cache: torch.Tensor, c_kv: torch.Tensor,

@@ -404,19 +404,37 @@ namespace {
 // decode steps. Wave 0 of a token's workgroup has the latent (8 dims a lane),
 // the others rotate 8 pairs a lane; norm and rotation round as the single
 // kernels do.
-__global__ __launch_bounds__(256)
-void mla_prepare_kernel(
-    short* __restrict__ q_out,              // [T, H, P]
-    short* __restrict__ c_out,              // [T, R]
-    short* __restrict__ k_out,              // [T, P]
-    short* __restrict__ cache,              // [NB, BS, DT] or nullptr
-    const short* __restrict__ q, const int64_t q_ts, const int64_t q_hs,
-    const short* __restrict__ kv_a, const int64_t kv_ts,
-    const short* __restrict__ w, const float eps,
-    const int64_t* __restrict__ positions,
-    const float* __restrict__ cos_sin,      // [max_pos, P]
-    const int64_t* __restrict__ slots, const int H) {
-  const int64_t t = blockIdx.x;
+struct PrepareArgs {
+  short* q_out;                     // [T, H, P]
+  short* c_out;                     // [T, R]
+  short* k_out;                     // [T, P]
+  short* cache;                     // [NB, BS, DT] or nullptr
+  const short* q;
+  int64_t q_ts, q_hs;
+  const short* kv_a;
+  int64_t kv_ts;
+  const short* w;
+  float eps;
+  const int64_t* positions;
+  const float* cos_sin;             // [max_pos, P]
+  const int64_t* slots;
+  int H;
+};
+
+KAITO_DEV void prepare_token(const PrepareArgs& a, const int64_t t) {
+  short* __restrict__ q_out = a.q_out;
+  short* __restrict__ c_out = a.c_out;
+  short* __restrict__ k_out = a.k_out;
+  short* __restrict__ cache = a.cache;
+  const short* __restrict__ q = a.q;
+  const short* __restrict__ kv_a = a.kv_a;
+  const short* __restrict__ w = a.w;
+  const float* __restrict__ cos_sin = a.cos_sin;
+  const int64_t* __restrict__ positions = a.positions;
+  const int64_t* __restrict__ slots = a.slots;
+  const int64_t q_ts = a.q_ts, q_hs = a.q_hs, kv_ts = a.kv_ts;
+  const float eps = a.eps;
+  const int H = a.H;
   const int tid = threadIdx.x;
   const int64_t slot = cache ? slots[t] : -1;
   if (tid < 64) {
@@ -468,13 +486,17 @@ void mla_prepare_kernel(
   }
 }
 
+__global__ __launch_bounds__(256)
+void mla_prepare_kernel(const PrepareArgs a) { prepare_token(a, blockIdx.x); }
+
 }  // namespace
 
 // q [T, H, P] of any token and head stride; an empty cache: nothing cached
-void mla_prepare(at::Tensor q_out, at::Tensor c_out, at::Tensor k_out,
-                 at::Tensor cache, at::Tensor q, at::Tensor kv_a, at::Tensor w,
-                 double eps, at::Tensor positions, at::Tensor cos_sin,
-                 at::Tensor slots) {
+static PrepareArgs prepare_args(
+    const at::Tensor& q_out, const at::Tensor& c_out, const at::Tensor& k_out,
+    const at::Tensor& cache, const at::Tensor& q, const at::Tensor& kv_a,
+    const at::Tensor& w, double eps, const at::Tensor& positions,
+    const at::Tensor& cos_sin, const at::Tensor& slots) {
   auto ok = [](const at::Tensor& t) {
     bool fine = t.is_cuda() && t.dtype() == at::kBFloat16 &&
                 t.stride(-1) == 1 && (uintptr_t)t.data_ptr() % 16 == 0;
@@ -499,16 +521,25 @@ void mla_prepare(at::Tensor q_out, at::Tensor c_out, at::Tensor k_out,
                 cache.size(2) == DT && slots.dtype() == at::kLong &&
                 slots.numel() == T && slots.is_contiguous());
   }
-  if (T == 0) return;
-  hipLaunchKernelGGL(mla_prepare_kernel, dim3(T), dim3(256), 0,
-                     at::hip::getCurrentHIPStream(), (short*)q_out.data_ptr(),
-                     (short*)c_out.data_ptr(), (short*)k_out.data_ptr(),
-                     cached ? (short*)cache.data_ptr() : nullptr,
-                     (const short*)q.data_ptr(), q.stride(0), q.stride(1),
-                     (const short*)kv_a.data_ptr(), kv_a.stride(0),
-                     (const short*)w.data_ptr(), (float)eps,
-                     positions.data_ptr<int64_t>(), cos_sin.data_ptr<float>(),
-                     cached ? slots.data_ptr<int64_t>() : nullptr, (int)H);
+  return {(short*)q_out.data_ptr(), (short*)c_out.data_ptr(),
+          (short*)k_out.data_ptr(),
+          cached ? (short*)cache.data_ptr() : nullptr,
+          (const short*)q.data_ptr(), q.stride(0), q.stride(1),
+          (const short*)kv_a.data_ptr(), kv_a.stride(0),
+          (const short*)w.data_ptr(), (float)eps,
+          positions.data_ptr<int64_t>(), cos_sin.data_ptr<float>(),
+          cached ? slots.data_ptr<int64_t>() : nullptr, (int)H};
+}
+
+void mla_prepare(at::Tensor q_out, at::Tensor c_out, at::Tensor k_out,
+                 at::Tensor cache, at::Tensor q, at::Tensor kv_a, at::Tensor w,
+                 double eps, at::Tensor positions, at::Tensor cos_sin,
+                 at::Tensor slots) {
+  const PrepareArgs a = prepare_args(q_out, c_out, k_out, cache, q, kv_a, w,
+                                     eps, positions, cos_sin, slots);
+  if (q.size(0) == 0) return;
+  hipLaunchKernelGGL(mla_prepare_kernel, dim3(q.size(0)), dim3(256), 0,
+                     at::hip::getCurrentHIPStream(), a);
 }
 
 namespace {
@@ -521,15 +552,23 @@ namespace {
 // library products took 12.3 (K = 128) and 4.7 us (K = 512) of which the
 // second needed a copy of 4.7 us to transpose its result, these
 // 5.9 each (32 rows of 16 heads, with the launch).
+struct HeadArgs {
+  short* y;                         // [T, H, N]
+  const short* x;
+  int64_t x_ts, x_hs;
+  const short* w;                   // [H, K, N]
+  int T, H, K, N;
+};
+
+// wt: [K][32]
 template <int MT>
-__global__ __launch_bounds__(256)
-void head_rows_kernel(short* __restrict__ y, const short* __restrict__ x,
-                      const int64_t x_ts, const int64_t x_hs,
-                      const short* __restrict__ w, const int T, const int K,
-                      const int N) {
-  extern __shared__ __attribute__((aligned(128))) short wt[];   // [K][32]
-  __shared__ f32x4 red[2][MT][64];
-  const int n0 = blockIdx.x * 32, head = blockIdx.y, H = gridDim.y;
+KAITO_DEV void head_tile(const HeadArgs& a, short* wt, f32x4 (&red)[2][MT][64],
+                         const int n0, const int head) {
+  short* __restrict__ y = a.y;
+  const short* __restrict__ x = a.x;
+  const short* __restrict__ w = a.w;
+  const int64_t x_ts = a.x_ts, x_hs = a.x_hs;
+  const int T = a.T, H = a.H, K = a.K, N = a.N;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lo = lane & 15, hi = lane >> 4;
@@ -587,10 +626,34 @@ void head_rows_kernel(short* __restrict__ y, const short* __restrict__ x,
   }
 }
 
+template <int MT>
+__global__ __launch_bounds__(256) void head_rows_kernel(const HeadArgs a) {
+  extern __shared__ __attribute__((aligned(128))) short wt[];
+  __shared__ f32x4 red[2][MT][64];
+  head_tile<MT>(a, wt, red, blockIdx.x * 32, blockIdx.y);
+}
+
+// mla_prepare's workgroups and behind them those of head_rows: neither reads what
+// the other writes, and both are little more than a launch (one MI355X, 32 rows of
+// 16 heads: 2.5 and 3.6 us, together 3.7).
+template <int MT>
+__global__ __launch_bounds__(256)
+void mla_prepare_rows_kernel(const PrepareArgs p, const HeadArgs a) {
+  extern __shared__ __attribute__((aligned(128))) short wt[];
+  __shared__ f32x4 red[2][MT][64];
+  if ((int)blockIdx.x < a.T) {
+    prepare_token(p, blockIdx.x);
+  } else {
+    const int b = blockIdx.x - a.T, tiles = a.N / 32;
+    head_tile<MT>(a, wt, red, b % tiles * 32, b / tiles);
+  }
+}
+
 }  // namespace
 
 // y [T, H, N], x [T, H, K] of any token and head stride, w [H, K, N]
-void head_rows(at::Tensor y, at::Tensor x, at::Tensor w) {
+static HeadArgs head_args(const at::Tensor& y, const at::Tensor& x,
+                          const at::Tensor& w) {
   for (const at::Tensor* t : {&y, &x, &w})
     TORCH_CHECK(t->is_cuda() && t->dtype() == at::kBFloat16 && t->dim() == 3);
   const int64_t T = x.size(0), H = x.size(1), K = x.size(2), N = w.size(2);
@@ -601,15 +664,39 @@ void head_rows(at::Tensor y, at::Tensor x, at::Tensor w) {
               x.stride(0) % 4 == 0 && x.stride(1) % 4 == 0 &&
               (uintptr_t)x.data_ptr() % 8 == 0 &&
               (uintptr_t)w.data_ptr() % 16 == 0);
-  if (T == 0 || H == 0 || N == 0) return;
+  return {(short*)y.data_ptr(), (const short*)x.data_ptr(), x.stride(0),
+          x.stride(1), (const short*)w.data_ptr(), (int)T, (int)H, (int)K,
+          (int)N};
+}
+
+void head_rows(at::Tensor y, at::Tensor x, at::Tensor w) {
+  const HeadArgs a = head_args(y, x, w);
+  if (a.T == 0 || a.H == 0 || a.N == 0) return;
   auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(N / 32, H), dim3(256), K * 64,
-        at::hip::getCurrentHIPStream(), (short*)y.data_ptr(),
-        (const short*)x.data_ptr(), x.stride(0), x.stride(1),
-        (const short*)w.data_ptr(), (int)T, (int)K, (int)N);
+    hipLaunchKernelGGL(kernel, dim3(a.N / 32, a.H), dim3(256), a.K * 64,
+                       at::hip::getCurrentHIPStream(), a);
   };
-  if (T <= 16) launch(&head_rows_kernel<1>);
+  if (a.T <= 16) launch(&head_rows_kernel<1>);
   else launch(&head_rows_kernel<2>);
+}
+
+// mla_prepare and head_rows of the same up to 32 rows
+void mla_prepare_rows(at::Tensor q_out, at::Tensor c_out, at::Tensor k_out,
+                      at::Tensor cache, at::Tensor q, at::Tensor kv_a,
+                      at::Tensor w, double eps, at::Tensor positions,
+                      at::Tensor cos_sin, at::Tensor slots, at::Tensor y,
+                      at::Tensor x, at::Tensor wx) {
+  const PrepareArgs p = prepare_args(q_out, c_out, k_out, cache, q, kv_a, w,
+                                     eps, positions, cos_sin, slots);
+  const HeadArgs a = head_args(y, x, wx);
+  TORCH_CHECK(q.size(0) == a.T);
+  if (a.T == 0) return;
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(a.T + a.N / 32 * a.H), dim3(256),
+                       a.K * 64, at::hip::getCurrentHIPStream(), p, a);
+  };
+  if (a.T <= 16) launch(&mla_prepare_rows_kernel<1>);
+  else launch(&mla_prepare_rows_kernel<2>);
 }
 
 // MLA cache write alone: latent row (c_kv ‖ k_rope) scattered to the paged

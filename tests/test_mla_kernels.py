@@ -107,3 +107,29 @@ def test_single_operations_agree():
     b = ops.mla_decode(q[..., :512], cache, bt, sl, 0.1, 512, q[..., 512:])
     assert torch.equal(a, b)
     assert torch.equal(a, R.mla_decode(q, cache, bt, sl, 0.1, 512))
+
+
+@pytest.mark.parametrize("T,H,K,N,cached", [(1, 16, 128, 512, True),
+                                            (16, 3, 64, 96, True),
+                                            (17, 16, 128, 512, False),
+                                            (32, 20, 128, 512, True)])
+def test_prepare_beside_head_rows(T, H, K, N, cached):
+    """One launch or two: the same bits."""
+    torch.manual_seed(T + H)
+    q, w, wx = _bf16(T, H, K + 64), _bf16(512), _bf16(H, K, N)
+    kv_a = _bf16(T, 576)
+    pos = torch.randint(0, 100, (T,), device=DEV)
+    cs = torch.randn(100, 64, device=DEV)
+    slots = torch.randperm(96, device=DEV)[:T]
+    slots[T // 2] = -1
+    a = _bf16(6, 16, 576)
+    b = a.clone()
+    args = (q[..., K:], kv_a, w, 1e-6, pos, cs)
+    got = ops.mla_prepare_rows(q[..., :K], wx, *args, a if cached else None,
+                               slots if cached else None)
+    want = (ops.head_rows(q[..., :K], wx),
+            *ops.mla_prepare(*args, b if cached else None,
+                             slots if cached else None))
+    for x, y in zip(got, want):
+        assert torch.equal(x, y)
+    assert torch.equal(a, b)
