@@ -243,11 +243,12 @@ class MoEMLP(nn.Module):
         if not self.n_identity:
             w_id = None
         shared = None
-        if self.w_shared_gate_up is not None:   # deepseek shared experts
+        # deepseek shared experts; beside the routed ones where they fit
+        beside = pairs and self._shared_fits(T)
+        if self.w_shared_gate_up is not None and not beside:
             h1 = ops.linear_swiglu(x, self.w_shared_gate_up) if self.gated \
                 else ops.relu2(ops.linear(x, self.w_shared_gate_up))
             shared = ops.linear(h1, self.w_shared_down)
-        added = None if split_shared else shared
         if kernels == "loop":
             out = self._routed_start(x, w_id)
             self._forward_loop(x, sorted_tok, gates, offsets, out)
@@ -257,24 +258,24 @@ class MoEMLP(nn.Module):
             if x.data_ptr() % 16:
                 x = x.clone()
             if pairs:
-                y = self._rows_pairs(x, topi)
+                y, beside_y = self._rows_pairs(x, topi, beside)
+                shared = beside_y if beside else shared
             elif kernels == "streamed":
                 y = self._rows_streamed(x, sorted_tok, offsets)
             else:
                 y = self._rows_tiled(x, sorted_tok, offsets)
             rows = MoERows((T, H), torch.float32 if keep_f32 else x.dtype, y,
                            pos, topi, topw, self.e_base, self.e_local, x,
-                           w_id, added)
+                           w_id, None if split_shared else shared)
             if defer and get_state().tp_size == 1:
                 assert not split_shared
                 return rows
             out = rows.tensor()
-            added = None
         if split_shared:
             assert get_state().tp_size == 1
             return out, shared
-        if added is not None:
-            out = out + added
+        if shared is not None and kernels == "loop":
+            out = out + shared
         if get_state().tp_size > 1:
             out = tp_all_reduce(out)
         return out
@@ -287,17 +288,44 @@ class MoEMLP(nn.Module):
 
     # All return the experts' outputs of the sorted rows (or of the pairs), to be
     # summed per token by moe_combine; static shapes, no host read.
-    def _rows_pairs(self, x, topi):
-        act = torch.empty(topi.numel(), self.ie_local, dtype=x.dtype,
-                          device=x.device)
+    def _shared_fits(self, T: int) -> bool:
+        """Whether the shared expert runs as one more of the routed ones: of
+        their sizes, on few tokens (32 rows, 8 experts of 2048 x 2048, top 2,
+        us: up 25.4 and down 14.5 behind 15.4 for products of its own, 30.0 and
+        17.2 with it; 4 rows 19.4, 14.0 and 10.7, 23.7 and 13.5)."""
+        w = self.w_shared_gate_up
+        if w is None or T > 32:
+            return False
+        d = self.w_shared_down
+        return self.gated \
+            and self.act_mode == 0 \
+            and self.b_gate_up is None and self.b_down is None \
+            and w.shape == self.w_gate_up.shape[1:] \
+            and d.shape == self.w_down.shape[1:] \
+            and w.dtype == d.dtype == torch.bfloat16 \
+            and w.is_contiguous() and d.is_contiguous() \
+            and w.data_ptr() % 16 == d.data_ptr() % 16 == 0
+
+    def _rows_pairs(self, x, topi, beside: bool = False):
+        """(rows of the pairs, the shared expert's [T, H] or None)"""
+        def new(rows, cols, dtype):
+            return torch.empty(rows, cols, dtype=dtype, device=x.device)
+
+        T, H = x.shape
+        act = new(topi.numel(), self.ie_local, x.dtype)
+        up, down, all_y = {}, {}, None
+        if beside:
+            all_act, all_y = new(T, self.ie_local, x.dtype), new(T, H, x.dtype)
+            up = dict(all_w=self.w_shared_gate_up, all_act=all_act)
+            down = dict(all_w=self.w_shared_down, all_act=all_act,
+                        all_y=all_y)
         ops.moe_up_pairs(act, x, self.w_gate_up, topi, self.n_route,
                          self.e_base, self.e_local, self.b_gate_up,
-                         self.act_mode, self.act_limit)
-        y = torch.empty(topi.numel(), x.size(1), dtype=torch.float32,
-                        device=x.device)
+                         self.act_mode, self.act_limit, **up)
+        y = new(topi.numel(), H, torch.float32)
         ops.moe_down_pairs(y, act, self.w_down, topi, self.n_route,
-                           self.e_base, self.e_local, self.b_down)
-        return y
+                           self.e_base, self.e_local, self.b_down, **down)
+        return y, all_y
 
     def _rows_tiled(self, x, sorted_tok, offsets):
         TK, H = sorted_tok.numel(), x.size(1)

@@ -696,18 +696,24 @@ def moe_pairs_pay(pairs: int, n_local: int, up_rows: int, H: int) -> bool:
 
 def moe_up_pairs(act, x, w_gate_up, topi, n_experts: int, e_base: int,
                  n_local_experts: int, bias=None, act_mode: int = 0,
-                 act_limit: float = 7.0) -> None:
+                 act_limit: float = 7.0, all_w=None, all_act=None) -> None:
     """moe_gate_silu with the rows of `act` in the order of the pairs of
-    `topi` [T, top] int32, up to PAIRS_MAX of them: no sort (GPU only)."""
+    `topi` [T, top] int32, up to PAIRS_MAX of them: no sort (GPU only).
+    all_w [2 IE, H]: an expert of every token beside them (SwiGLU, no
+    biases), its rows go to all_act [T, IE]."""
     _K.moe_up_pairs(act, x, w_gate_up, topi, _none(bias, x), act_mode,
-                    n_experts, e_base, n_local_experts, act_limit)
+                    n_experts, e_base, n_local_experts, act_limit,
+                    _none(all_w, x), _none(all_act, x))
 
 
 def moe_down_pairs(y, act, w_down, topi, n_experts: int, e_base: int,
-                   n_local_experts: int, bias=None) -> None:
-    """moe_down_rows with rows in the order of the pairs (GPU only)."""
+                   n_local_experts: int, bias=None, all_w=None, all_act=None,
+                   all_y=None) -> None:
+    """moe_down_rows with rows in the order of the pairs (GPU only). all_w
+    [H, IE]: the expert of every token, all_y [T, H] bf16 its result."""
     _K.moe_down_pairs(y, act, w_down, topi, _none(bias, act), n_experts,
-                      e_base, n_local_experts)
+                      e_base, n_local_experts, _none(all_w, y),
+                      _none(all_act, y), _none(all_y, y))
 
 
 def moe_grouped_up(act, x, w, sorted_ids, offsets, e_base: int, bias=None,

@@ -50,6 +50,12 @@ struct StreamArgs {
   float limit;
   short* act;                       // up: [TK, N]
   float* y;                         // down: [TK, N]
+  // an expert of every token behind the local ones, of the same sizes, or none
+  // (PAIRS, without biases): its weights; up: act [T, N]; down: act [T, K], y in
+  // bf16 [T, N]
+  const short* all_w;
+  short* all_act;
+  short* all_y;
 };
 
 enum Kind { UP_GATED, UP_PLAIN, DOWN };
@@ -74,7 +80,7 @@ KAITO_DEV float moe_act_f(int mode, float g, float u, float limit) {
 // token, 2048 x 512, top 8).
 constexpr int PAIRS_MAX = 256;
 
-template <bool PAIRS>
+template <int PAIRS>
 struct Rows {
   int begin, end;
   const unsigned short* list;       // of PAIRS
@@ -83,11 +89,41 @@ struct Rows {
   KAITO_DEV int at(const int m) const { return PAIRS ? list[m] : m; }
 };
 
-template <bool PAIRS>
+// PAIRS: rows by sorted pairs (0), by the pairs themselves (1), so and with an
+// expert of every token (2), which would cost the others 0.7 us of a launch.
+// The arguments as local expert le sees them: the one of all lies behind the rest.
+template <int KIND, int PAIRS>
+KAITO_DEV StreamArgs as_expert(const StreamArgs& a, const int le) {
+  StreamArgs b = a;
+  const int64_t wrows = KIND == UP_GATED ? 2 * a.N : a.N;
+  const bool all = PAIRS == 2 && le == (int)gridDim.y - 1;
+  b.w = all ? a.all_w : a.w + le * wrows * a.K;
+  if (b.bias) b.bias += le * wrows;
+  if constexpr (PAIRS == 2) {
+    if (KIND == DOWN) {
+      b.x = all ? a.all_act : a.x;
+      b.all_y = all ? a.all_y : nullptr;
+    } else {
+      b.act = all ? a.all_act : a.act;
+    }
+    b.pairs = all ? a.pairs / a.top : a.pairs;
+    b.top = all ? 1 : a.top;
+    b.topi = all ? nullptr : a.topi;
+  }
+  return b;
+}
+
+template <int PAIRS>
 KAITO_DEV Rows<PAIRS> rows_of(const StreamArgs& a, const int expert,
                               unsigned short* list, const int lane) {
   if constexpr (!PAIRS)
     return {a.offsets[expert], a.offsets[expert + 1], nullptr};
+  if (PAIRS == 2 && !a.topi) {      // every token
+#pragma unroll
+    for (int i = 0; i < PAIRS_MAX; i += 64) list[i + lane] = i + lane;
+    __builtin_amdgcn_wave_barrier();
+    return {0, a.pairs, list};
+  }
   int n = 0, e[PAIRS_MAX / 64];
 #pragma unroll
   for (int i = 0; i < PAIRS_MAX / 64; i++) {
@@ -108,7 +144,7 @@ KAITO_DEV Rows<PAIRS> rows_of(const StreamArgs& a, const int expert,
 }
 
 // column n of rows m .. m + 3 below the end: v, or gate v and up u
-template <int KIND, bool PAIRS>
+template <int KIND, int PAIRS>
 KAITO_DEV void store_rows(const StreamArgs& a, const f32x4 v, const f32x4 u,
                           const int m0, const Rows<PAIRS>& rows,
                           const int n) {
@@ -122,6 +158,8 @@ KAITO_DEV void store_rows(const StreamArgs& a, const f32x4 v, const f32x4 u,
     } else if constexpr (KIND == UP_PLAIN) {
       const float p = fmaxf(v[r], 0.f);
       a.act[(int64_t)m * a.N + n] = f32_to_bf16(p * p);
+    } else if (PAIRS == 2 && a.all_y) {
+      a.all_y[(int64_t)m * a.N + n] = f32_to_bf16(v[r]);
     } else {
       a.y[(int64_t)m * a.N + n] = v[r];
     }
@@ -129,7 +167,7 @@ KAITO_DEV void store_rows(const StreamArgs& a, const f32x4 v, const f32x4 u,
 }
 
 // x of row m, the last one's past the end
-template <int KIND, bool PAIRS>
+template <int KIND, int PAIRS>
 KAITO_DEV const short* x_row(const StreamArgs& a, const Rows<PAIRS>& rows,
                              const int m) {
   const int r = rows.at(min(m, rows.end - 1));
@@ -137,14 +175,16 @@ KAITO_DEV const short* x_row(const StreamArgs& a, const Rows<PAIRS>& rows,
   return a.x + row * a.K;
 }
 
-template <int MT, int KS, int KIND, bool PAIRS>
-__global__ __launch_bounds__(256, 2) void moe_stream_kernel(const StreamArgs a) {
+template <int MT, int KS, int KIND, int PAIRS>
+__global__ __launch_bounds__(256, 2) void moe_stream_kernel(
+    const StreamArgs args) {
   constexpr int NI = skinny::tile_loads<KS>();
   constexpr bool GATED = KIND == UP_GATED;
   __shared__ __attribute__((aligned(128))) short ring[4][2][16 * KS];
   static_assert(sizeof(ring) >= 4 * MT * 64 * sizeof(f32x4), "fold");
   __shared__ unsigned short list[PAIRS ? 4 : 1][PAIRS ? PAIRS_MAX : 1];
   const int le = blockIdx.y;
+  const StreamArgs a = as_expert<KIND, PAIRS>(args, le);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const auto rows =
@@ -152,18 +192,17 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const StreamArgs a) 
   const int begin = rows.begin, end = rows.end;
   if (begin >= end) return;
   const int n0 = blockIdx.x * (GATED ? 8 : 16);
-  const int64_t wrows = GATED ? 2 * a.N : a.N;
   const short* src[NI];
 #pragma unroll
   for (int j = 0; j < NI; j++) {
     const int r = skinny::tile_row<KS>(j, lane);
     const int64_t n = GATED ? n0 + r % 8 + (r >= 8 ? a.N : 0) : n0 + r;
-    src[j] = a.w + (le * wrows + n) * a.K + skinny::tile_col<KS>(j, lane);
+    src[j] = a.w + n * a.K + skinny::tile_col<KS>(j, lane);
   }
   f32x4* red = reinterpret_cast<f32x4*>(&ring[0][0][0]);
   const int slot = threadIdx.x, l = slot & 63, c = l & 15;
   const bool mine = slot < MT * 64 && !(GATED && c >= 8);
-  const short* be = a.bias ? a.bias + le * wrows + n0 + c : nullptr;
+  const short* be = a.bias ? a.bias + n0 + c : nullptr;
   for (int m0 = begin; m0 < end; m0 += 16 * MT) {
     const short* xp[MT];
 #pragma unroll
@@ -196,18 +235,17 @@ __global__ __launch_bounds__(256, 2) void moe_stream_kernel(const StreamArgs a) 
 
 // K = 1024 S: see skinny::stream_tiles. gridDim.x workgroups share an expert's
 // ntiles tiles; MT row tiles of 16 in a pass.
-template <int MT, int S, int KIND, bool PAIRS>
-KAITO_DEV void stream_pass(const StreamArgs& a, const int le, const int ntiles,
+template <int MT, int S, int KIND, int PAIRS>
+KAITO_DEV void stream_pass(const StreamArgs& a, const int ntiles,
                            const int m0, const Rows<PAIRS>& rows, short* ring,
                            f32x4* red, const int wave, const int lane) {
   constexpr int KS = skinny::TILES_KS, NW = skinny::TILE_NW;
   constexpr bool GATED = KIND == UP_GATED;
   constexpr int COLS = GATED ? 8 : 16;
-  const int64_t wrows = GATED ? 2 * a.N : a.N;
   const int slot = threadIdx.x, l = slot & 63, c = l & 15;
   const bool mine = slot < MT * 64 && !(GATED && c >= 8);
   skinny::stream_tiles<MT, S, false>(
-      a.w + le * wrows * a.K, nullptr, 0,
+      a.w, nullptr, 0,
       [&](const int j) {
         const int r = skinny::tile_row<KS>(j, lane);
         const uint32_t n = GATED ? r % 8 + (r >= 8 ? a.N : 0) : r;
@@ -227,7 +265,7 @@ KAITO_DEV void stream_pass(const StreamArgs& a, const int le, const int ntiles,
         f32x4 v = skinny::fold<MT, NW>(sums, slot), u{0.f, 0.f, 0.f, 0.f};
         if constexpr (GATED) u = skinny::fold<MT, NW>(sums, slot + 8);
         if (a.bias) {
-          const short* be = a.bias + le * wrows + n;
+          const short* be = a.bias + n;
           v += bf16_to_f32(be[0]);
           if constexpr (GATED) u += bf16_to_f32(be[a.N]);
         }
@@ -237,9 +275,9 @@ KAITO_DEV void stream_pass(const StreamArgs& a, const int le, const int ntiles,
   __syncthreads();                  // sums read before the next pass's
 }
 
-template <int S, int KIND, bool PAIRS>
-__global__ __launch_bounds__(256, 2) void moe_tiles_kernel(const StreamArgs a,
-                                                           const int ntiles) {
+template <int S, int KIND, int PAIRS>
+__global__ __launch_bounds__(256, 2) void moe_tiles_kernel(
+    const StreamArgs args, const int ntiles) {
   constexpr int KS = skinny::TILES_KS, NW = skinny::TILE_NW;
   __shared__ __attribute__((aligned(128))) short ring[NW][2][16 * KS];
   __shared__ f32x4 red[2][NW][2 * 64];
@@ -247,24 +285,27 @@ __global__ __launch_bounds__(256, 2) void moe_tiles_kernel(const StreamArgs a,
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   __shared__ unsigned short list[PAIRS ? NW : 1][PAIRS ? PAIRS_MAX : 1];
   const int le = blockIdx.y;
+  const StreamArgs a = as_expert<KIND, PAIRS>(args, le);
   const auto rows =
       rows_of<PAIRS>(a, a.e_base + le, list[PAIRS ? wave : 0], lane);
   // An expert that many tokens share would hold up its workgroups for a second
   // pass: as many row tiles as it has.
   for (int m0 = rows.begin; m0 < rows.end; m0 += 32) {
     if (rows.end - m0 > 16)
-      stream_pass<2, S, KIND>(a, le, ntiles, m0, rows, ring[wave][0],
+      stream_pass<2, S, KIND>(a, ntiles, m0, rows, ring[wave][0],
                               &red[0][0][0], wave, lane);
     else
-      stream_pass<1, S, KIND>(a, le, ntiles, m0, rows, ring[wave][0],
+      stream_pass<1, S, KIND>(a, ntiles, m0, rows, ring[wave][0],
                               &red[0][0][0], wave, lane);
   }
 }
 
 // pairs: (token, expert) pairs of the step, over all E experts
-template <int KIND, bool PAIRS>
+template <int KIND, int PAIRS>
 void launch_rows(const StreamArgs& a, int64_t E_local, int64_t pairs,
                  int64_t E) {
+  const int64_t E_chosen = E_local;
+  E_local += PAIRS == 2;
   const dim3 grid(a.N / (KIND == UP_GATED ? 8 : 16), E_local), block(256);
   auto stream = at::hip::getCurrentHIPStream();
   // two row tiles once most experts have more than one
@@ -285,10 +326,11 @@ void launch_rows(const StreamArgs& a, int64_t E_local, int64_t pairs,
   // 4, 99 and 105 at 16. Wider K streams as fast in tiles of their own: 8 of 28672 x
   // 4096, 16 tokens, 275 and 282.
   const double hit =
-      E_local * (1.0 - std::pow(1.0 - 1.0 / E, (double)pairs));
+      E_chosen * (1.0 - std::pow(1.0 - 1.0 / E, (double)pairs)) +
+      (E_local - E_chosen);
   // never more than the CUs: a CU with two of them ends late (264
   // workgroups for the 32 tokens: 31.2 and 18.4)
-  const int most = (int)std::min<int64_t>(E_local, pairs);
+  const int most = (int)(std::min<int64_t>(E_chosen, pairs) + E_local - E_chosen);
   const int per = std::max(1, std::min<int>(grid.x, 256 / most));
   const int rounds = (grid.x + per - 1) / per;
   if (a.K == 2048 && E_local <= 32 && hit * grid.x >= 768 &&
@@ -312,8 +354,13 @@ void launch_rows(const StreamArgs& a, int64_t E_local, int64_t pairs,
 template <int KIND>
 void launch_stream(const StreamArgs& a, int64_t E_local, int64_t pairs,
                    int64_t E) {
-  if (a.topi) launch_rows<KIND, true>(a, E_local, pairs, E);
-  else launch_rows<KIND, false>(a, E_local, pairs, E);
+  if (a.all_w) {
+    if constexpr (KIND != UP_PLAIN) launch_rows<KIND, 2>(a, E_local, pairs, E);
+  } else if (a.topi) {
+    launch_rows<KIND, 1>(a, E_local, pairs, E);
+  } else {
+    launch_rows<KIND, 0>(a, E_local, pairs, E);
+  }
 }
 
 void check16(const at::Tensor& t) {
@@ -355,7 +402,8 @@ void set_rows(StreamArgs& a, const RowArgs& r, int64_t e_base, int64_t n_local,
 
 void up_rows(at::Tensor& act, const at::Tensor& x, const at::Tensor& w_gate_up,
              const RowArgs& rows, const at::Tensor& bias, int64_t act_mode,
-             int64_t e_base, int64_t n_local, double act_limit) {
+             int64_t e_base, int64_t n_local, double act_limit,
+             const at::Tensor& all_w, const at::Tensor& all_act) {
   check16(act); check16(x); check16(w_gate_up);
   const bool gated = act_mode != 2;
   StreamArgs a{};
@@ -377,13 +425,23 @@ void up_rows(at::Tensor& act, const at::Tensor& x, const at::Tensor& w_gate_up,
   a.act_mode = (int)act_mode;
   a.limit = (float)act_limit;
   a.act = (short*)act.data_ptr();
+  if (all_w.defined() && all_w.numel() > 0) {
+    check16(all_w); check16(all_act);
+    const int64_t T = x.size(0);
+    TORCH_CHECK(rows.topi.defined() && gated && act_mode == 0 && !a.bias &&
+                all_w.numel() == 2 * (int64_t)a.N * a.K &&
+                all_act.numel() == T * a.N && T * a.top == rows.pairs);
+    a.all_w = (const short*)all_w.data_ptr();
+    a.all_act = (short*)all_act.data_ptr();
+  }
   if (gated) launch_stream<UP_GATED>(a, n_local, rows.pairs, rows.E);
   else launch_stream<UP_PLAIN>(a, n_local, rows.pairs, rows.E);
 }
 
 void down_rows(at::Tensor& y, const at::Tensor& act, const at::Tensor& w_down,
                const RowArgs& rows, const at::Tensor& bias, int64_t e_base,
-               int64_t n_local) {
+               int64_t n_local, const at::Tensor& all_w,
+               const at::Tensor& all_act, const at::Tensor& all_y) {
   TORCH_CHECK(y.is_cuda() && y.dtype() == at::kFloat && y.is_contiguous());
   check16(act); check16(w_down);
   StreamArgs a{};
@@ -401,6 +459,15 @@ void down_rows(at::Tensor& y, const at::Tensor& act, const at::Tensor& w_down,
   a.x = (const short*)act.data_ptr();
   a.w = (const short*)w_down.data_ptr();
   a.y = y.data_ptr<float>();
+  if (all_w.defined() && all_w.numel() > 0) {
+    check16(all_w); check16(all_act); check16(all_y);
+    const int64_t T = rows.topi.defined() ? rows.topi.size(0) : -1;
+    TORCH_CHECK(!a.bias && all_w.numel() == (int64_t)a.N * a.K &&
+                all_act.numel() == T * a.K && all_y.numel() == T * a.N);
+    a.all_w = (const short*)all_w.data_ptr();
+    a.all_act = (short*)all_act.data_ptr();
+    a.all_y = (short*)all_y.data_ptr();
+  }
   launch_stream<DOWN>(a, n_local, rows.pairs, rows.E);
 }
 
@@ -413,7 +480,8 @@ void moe_gate_silu(at::Tensor act, at::Tensor x, at::Tensor w_gate_up,
                    double act_limit) {
   up_rows(act, x, w_gate_up,
           {offsets, sorted_ids, {}, sorted_ids.numel(), offsets.numel() - 1},
-          bias, act_mode, e_base, n_local_experts, act_limit);
+          bias, act_mode, e_base, n_local_experts, act_limit,
+          at::Tensor(), at::Tensor());
 }
 
 void moe_down_rows(at::Tensor y, at::Tensor act, at::Tensor w_down,
@@ -421,24 +489,25 @@ void moe_down_rows(at::Tensor y, at::Tensor act, at::Tensor w_down,
                    int64_t n_local_experts) {
   down_rows(y, act, w_down,
             {offsets, {}, {}, y.size(0), offsets.numel() - 1}, bias, e_base,
-            n_local_experts);
+            n_local_experts, at::Tensor(), at::Tensor(), at::Tensor());
 }
 
 void moe_up_pairs(at::Tensor act, at::Tensor x, at::Tensor w_gate_up,
                   at::Tensor topi, at::Tensor bias, int64_t act_mode,
                   int64_t n_experts, int64_t e_base, int64_t n_local_experts,
-                  double act_limit) {
+                  double act_limit, at::Tensor all_w, at::Tensor all_act) {
   TORCH_CHECK(x.size(0) == topi.size(0));
   up_rows(act, x, w_gate_up, {{}, {}, topi, topi.numel(), n_experts}, bias,
-          act_mode, e_base, n_local_experts, act_limit);
+          act_mode, e_base, n_local_experts, act_limit, all_w, all_act);
 }
 
 void moe_down_pairs(at::Tensor y, at::Tensor act, at::Tensor w_down,
                     at::Tensor topi, at::Tensor bias, int64_t n_experts,
-                    int64_t e_base, int64_t n_local_experts) {
+                    int64_t e_base, int64_t n_local_experts, at::Tensor all_w,
+                    at::Tensor all_act, at::Tensor all_y) {
   TORCH_CHECK(y.size(0) == topi.numel());
   down_rows(y, act, w_down, {{}, {}, topi, topi.numel(), n_experts}, bias,
-            e_base, n_local_experts);
+            e_base, n_local_experts, all_w, all_act, all_y);
 }
 
 }  // namespace kaito

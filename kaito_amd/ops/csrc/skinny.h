@@ -152,32 +152,42 @@ constexpr int TILES_KS = 256;
 
 // Sums of the 16 rows of W of tiles first, first + step .. < n. rows(j): byte
 // offset of load j's piece from the start of tile 0, which lies at w, and with TWO
-// so from tile n1, which lies at w2; tile: bytes from a tile to the next; xp: as for stream_tile, asked for once the
-// first weights are under way. ring: [2][16 * 256] of this wave, red:
+// so from tile n1, which lies at w2; tile: bytes from a tile to the next; xp: as
+// for stream_tile, asked for once the first weights are under way. ring: [2][16 * 256] of this wave, red:
 // [2][4][MT * 64] of the workgroup. out(tile, sums): on every thread, the sums
 // of the waves for fold().
 template <int MT, int S, bool TWO, typename Rows, typename X, typename Out>
 KAITO_DEV void stream_tiles(const void* w, const void* w2, const int n1,
-                            const Rows& rows, const uint32_t tile, const int first,
-                            const int step, const int n, const X& x,
-                            short* ring, f32x4* red, const int wave,
-                            const int lane, const Out& out) {
+                            const Rows& rows, const uint32_t tile,
+                            const int first, const int step, const int n,
+                            const X& x, short* ring, f32x4* red,
+                            const int wave, const int lane, const Out& out) {
   constexpr int KS = TILES_KS, NI = tile_loads<KS>(), STEPS = KS / 32;
   static_assert(S % 2 == 0, "a tile starts in ring 0");
   if (first >= n) return;           // uniform
   uint32_t off[NI];
 #pragma unroll
   for (int j = 0; j < NI; j++) off[j] = rows(j);
+  const auto wb = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<void*>(w), 0, 0xffffffff, 0x27000);
+  // past the last tile: loads of nothing, so that the waits stay counts
+  const auto none = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<void*>(w), 0, 0, 0x27000);
   auto fetch = [&](const int t, const int s) {
-    // past the last tile: loads of nothing, so that the waits stay counts
-    const bool second = TWO && t >= n1;
-    const uint64_t from = reinterpret_cast<uint64_t>(second ? w2 : w);
-    const auto r = __builtin_amdgcn_make_buffer_rsrc(
-        reinterpret_cast<void*>(
-            (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)from) |
-            (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(
-                (int)(from >> 32)) << 32),
-        0, __builtin_amdgcn_readfirstlane(t < n ? -1 : 0), 0x27000);
+    auto r = t < n ? wb : none;
+    bool second = false;
+    if constexpr (TWO) {
+      // a descriptor that is scalar for sure: one of two chosen by the tile was
+      // looked for lane by lane, which doubled the time
+      second = t >= n1;
+      const uint64_t from = reinterpret_cast<uint64_t>(second ? w2 : w);
+      r = __builtin_amdgcn_make_buffer_rsrc(
+          reinterpret_cast<void*>(
+              (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)from) |
+              (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(
+                  (int)(from >> 32)) << 32),
+          0, __builtin_amdgcn_readfirstlane(t < n ? -1 : 0), 0x27000);
+    }
     const uint32_t at = __builtin_amdgcn_readfirstlane(
         (second ? t - n1 : t) * tile + (wave + s * TILE_NW) * KS * 2);
 #pragma unroll

@@ -261,3 +261,51 @@ def test_choice_of_16_rows_large_router():
 def test_which_steps_choose_by_16_rows(T, N, H, f32, tiles):
     """The sides of the line on which either was measured to be faster."""
     assert ops._gate_long(T, N, H, f32) == tiles
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 5, 16, 17, 32])
+@pytest.mark.parametrize("E,H,I,top", [(8, 2048, 2048, 2), (16, 2048, 256, 4),
+                                       (4, 512, 192, 1), (6, 2048, 768, 6)])
+def test_expert_of_every_token(T, E, H, I, top):
+    """An expert of every token in the launches of the chosen ones, some of which
+    nobody chose: the routed rows' bits stay, its own rows are two linear layers
+    (f32 sums of up to 2048 terms, one rounding to bf16 each)."""
+    g = torch.Generator(device="cuda").manual_seed(T * E + I)
+
+    def normal(*s):
+        return torch.randn(*s, device="cuda", generator=g)
+    x = normal(T, H).bfloat16()
+    wu, wd = (normal(E, 2 * I, H) * H ** -.5).bfloat16(), \
+        (normal(E, H, I) * I ** -.5).bfloat16()
+    su, sd = (normal(2 * I, H) * H ** -.5).bfloat16(), \
+        (normal(H, I) * I ** -.5).bfloat16()
+    topi = torch.stack([torch.randperm(max(1, E - 1), device="cuda")[:top]
+                        for _ in range(T)]).int() if top < E else \
+        torch.arange(E, device="cuda").int().repeat(T, 1)
+
+    def run(**kw):
+        up = {k: kw[k] for k in ("all_w", "all_act") if k in kw}
+        act = torch.empty(T * top, I, dtype=torch.bfloat16, device="cuda")
+        ops.moe_up_pairs(act, x, wu, topi, E, 0, E, **up)
+        y = torch.empty(T * top, H, device="cuda")
+        down = dict(all_w=kw["all_d"], all_act=kw["all_act"],
+                    all_y=kw["all_y"]) if kw else {}
+        ops.moe_down_pairs(y, act, wd, topi, E, 0, E, **down)
+        return act, y
+    aa = torch.full((T, I), float("nan"), dtype=torch.bfloat16, device="cuda")
+    ay = torch.full((T, H), float("nan"), dtype=torch.bfloat16, device="cuda")
+    plain = run()
+    beside = run(all_w=su, all_d=sd, all_act=aa, all_y=ay)
+    for a, b in zip(plain, beside):
+        assert torch.isfinite(b).all()
+        assert (a.float() - b.float()).norm() <= 2.0 ** -9 * a.float().norm()
+    gu = x.double() @ su.double().T
+    ref = gu[:, :I] * torch.sigmoid(gu[:, :I]) * gu[:, I:]
+    rms = ref.square().mean().sqrt()
+    assert ((aa.double() - ref).abs()
+            <= 2.0 ** -8 * ref.abs() + 2.0 ** -12 * rms).all()
+    ref = aa.double() @ sd.double().T
+    rms = ref.square().mean().sqrt()
+    assert ((ay.double() - ref).abs()
+            <= 2.0 ** -8 * ref.abs() + 2.0 ** -12 * rms).all()
