@@ -245,12 +245,8 @@ class MLAAttention(nn.Module):
         Hl = self.num_heads
         tiles = None if meta.tile_seq is None else \
             (meta.tile_seq, meta.tile_qbase)
-        # decompress: k_nope [T, Hl, nope], v [Hl, T, v]
-        k_nope = ops.linear(
-            c_kv.to(self.w_kc.dtype), self.w_kc.view(Hl * self.nope, self.r)
-        ).view(T, Hl, self.nope)
-        v = torch.matmul(c_kv.to(self.w_vc.dtype).unsqueeze(0), self.w_vc)
-        v = v.transpose(0, 1)                           # [T, Hl, v]
+        # decompress: k_nope [T, Hl, nope], v [T, Hl, v]
+        k_nope, v = ops.latent_kv(c_kv, self.w_kc, self.w_vc)
         if q_nope.is_cuda and q_nope.dtype == torch.bfloat16 and \
                 (self.nope, self.rope, self.v_dim) == (128, 64, 128):
             return ops.mla_prefill_attention(

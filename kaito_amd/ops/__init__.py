@@ -33,7 +33,8 @@ for _g, _names in {
              "mla_prefill_attention context_attention mfma_tile_gemm paged_read_bw"),
     "mla": "mla_decode mla_prepare mla_prepare_rows head_rows mla_cache_write",
     "moe": ("moe_gate_silu moe_down_rows moe_up_pairs moe_down_pairs "
-            "moe_grouped_up moe_grouped_down moe_combine moe_combine_norm"),
+            "moe_grouped_up moe_grouped_down moe_combine moe_combine_norm "
+            "latent_kv"),
     "route": "moe_route moe_gate_route moe_norm_gate_route moe_sort",
     "quant": ("w4a16_gemv w4a16_dequant w4a16_gemm w4a16_swiglu "
               "w4a16_in_tiles lora_shrink lora_expand"),
@@ -552,6 +553,30 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         return out
     return torch_ref.prefill_attention(q, k, v, cu_seqlens, scale, window,
                                        sinks)
+
+
+def latent_kv(c: torch.Tensor, w_kc: torch.Tensor, w_vc: torch.Tensor):
+    """Keys [T, H, D] and values [T, H, V] of latent rows c [T, r]: c times
+    w_kc [H, D, r] and w_vc [H, r, V]. One launch (and a transposition of
+    w_vc) for prompts that fill the chip with 256 x 256 tiles, library products
+    else (us, library and tiles, 128 + 128 dims of 512: 8192 rows of 16 heads
+    59.2, 46.7, 4096 34.0, 27.4, 2048 23.2, 23.5; 4096 of 128 heads 213, 169,
+    512 33.2, 34.5)."""
+    T, (H, D, r), V = c.size(0), w_kc.shape, w_vc.size(2)
+    if c.is_cuda and T * H * (D + V) >= 4096 * 4096 and T < 1 << 22 \
+            and c.dtype == w_kc.dtype == w_vc.dtype == torch.bfloat16 \
+            and H * D % 256 == V % 64 == r % 64 == 0 \
+            and w_vc.shape[:2] == (H, r) and not _transformed() and all(
+                t.is_contiguous() and t.data_ptr() % 16 == 0
+                and not (torch.is_grad_enabled() and t.requires_grad)
+                for t in (c, w_kc, w_vc)):
+        kv = torch.empty(T, H * (D + V), dtype=c.dtype, device=c.device)
+        _K.latent_kv(kv, c, w_kc, w_vc)
+        return kv[:, :H * D].unflatten(-1, (H, D)), \
+            kv[:, H * D:].unflatten(-1, (H, V))
+    k = linear(c.to(w_kc.dtype), w_kc.view(H * D, r)).view(T, H, D)
+    v = torch.matmul(c.to(w_vc.dtype).unsqueeze(0), w_vc)
+    return k, v.transpose(0, 1)
 
 
 def mla_prefill_attention(q, q_pe, k, k_pe, v, cu_seqlens, scale: float,

@@ -422,6 +422,54 @@ __global__ __launch_bounds__(512, 2) void moe_grouped_kernel(const GemmArgs a) {
                                                    n0);
 }
 
+// ---- keys and values of latent rows ----------------------------------------
+// [k | v][t] = c[t] [Wk | Wv^T]^T, tiles of 256 x 256 over both: the tiles of
+// Wk's N1 rows first. Behind one another, as a library product and a batched one
+// of Wv as it is stored, they took 32 + 42 us (8192 rows of 512, 16 heads of 128 +
+// 128; 34 GFLOP, 80 MB), here 47 with the transposition: 8 K steps a tile, whose
+// start and end take as long.
+__global__ __launch_bounds__(512, 2) void latent_kv_kernel(GemmArgs a,
+                                                               const short* w2,
+                                                               const int N1,
+                                                               const int T) {
+  __shared__ __attribute__((aligned(128))) short lds[LDS];
+  const int ntiles = (a.N + BN - 1) / BN, mtiles = (T + 255) / 256;
+  const int total = ntiles * mtiles, share = (total + 7) / 8;
+  const int t = blockIdx.x % 8 * share + blockIdx.x / 8;
+  if ((int)blockIdx.x / 8 >= share || t >= total) return;
+  const int blk = t / (NG * mtiles), in_blk = t - blk * NG * mtiles;
+  const int wide = min(NG, ntiles - blk * NG);
+  const int n0 = (blk * NG + in_blk % wide) * BN, m0 = in_blk / wide * 256;
+  if (n0 >= N1) a.w = w2 - (int64_t)N1 * a.K;
+  grouped_tile<256, BN, 2, 0, DOWN>(a, lds, 0, m0, T, n0);
+}
+
+// w [H, K, V] -> out [H, V, K], by squares of 64
+__global__ __launch_bounds__(256) void transpose_heads_kernel(
+    short* __restrict__ out, const short* __restrict__ w, const int K,
+    const int V) {
+  __shared__ short tile[64][72];
+  const int k0 = blockIdx.x * 64, v0 = blockIdx.y * 64;
+  const int64_t head = (int64_t)blockIdx.z * K * V;
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const int s = i * 256 + threadIdx.x, r = s / 8, c = s % 8 * 8;
+    *reinterpret_cast<short8_t*>(&tile[r][c]) =
+        *reinterpret_cast<const short8_t*>(w + head + (int64_t)(k0 + r) * V +
+                                           v0 + c);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const int s = i * 256 + threadIdx.x, r = s / 8, c = s % 8 * 8;
+    short8_t o;
+#pragma unroll
+    for (int j = 0; j < 8; j++) o[j] = tile[c + j][r];
+    *reinterpret_cast<short8_t*>(out + head + (int64_t)(v0 + r) * K + k0 + c) =
+        o;
+  }
+}
+
 struct CombineArgs {
   const void* y;
   const int *pos, *topi;            // pos: none where rows are the pairs
@@ -659,6 +707,35 @@ void moe_grouped_down(at::Tensor y, at::Tensor act, at::Tensor w,
   launch_grouped<DOWN>(a, y.size(0));
 }
 
+// kv [T, H D + H V]: c [T, K] times wk [H, D, K] (rows K long) and wv [H, K, V]
+void latent_kv(at::Tensor kv, at::Tensor c, at::Tensor wk, at::Tensor wv) {
+  check16(kv); check16(c); check16(wk); check16(wv);
+  TORCH_CHECK(c.dim() == 2 && kv.dim() == 2 && wk.dim() == 3 && wv.dim() == 3);
+  const int64_t T = c.size(0), K = c.size(1), H = wk.size(0), V = wv.size(2);
+  const int64_t N1 = H * wk.size(1);
+  TORCH_CHECK(wk.size(2) == K && wv.size(0) == H && wv.size(1) == K &&
+              kv.size(0) == T && kv.size(1) == N1 + H * V &&
+              K % 64 == 0 && K > 0 && V % 64 == 0 && N1 % BN == 0 &&
+              T < (1ll << 22) && kv.size(1) < (1ll << 22));
+  if (T == 0 || H == 0) return;
+  auto stream = at::hip::getCurrentHIPStream();
+  const at::Tensor wt = at::empty({H, V, K}, wv.options());
+  hipLaunchKernelGGL(transpose_heads_kernel, dim3(K / 64, V / 64, H),
+                     dim3(256), 0, stream, (short*)wt.data_ptr(),
+                     (const short*)wv.data_ptr(), (int)K, (int)V);
+  GemmArgs a{};
+  a.out = (short*)kv.data_ptr();
+  a.x = (const short*)c.data_ptr();
+  a.w = (const short*)wk.data_ptr();
+  a.E = 1;
+  a.N = (int)kv.size(1);
+  a.K = (int)K;
+  const int64_t tiles = (T + 255) / 256 * ((a.N + BN - 1) / BN);
+  hipLaunchKernelGGL(latent_kv_kernel, dim3((tiles + 7) / 8 * 8),
+                     dim3(512), 0, stream, a, (const short*)wt.data_ptr(),
+                     (int)N1, (int)T);
+}
+
 // checks shared by both sums
 static CombineArgs combine_args(const at::Tensor& y, const at::Tensor& pos,
                                 const at::Tensor& topi, const at::Tensor& topw,
@@ -770,6 +847,7 @@ void moe_combine_norm(at::Tensor out, at::Tensor residual, at::Tensor y,
 TORCH_LIBRARY_FRAGMENT(kaito, m) {
   m.def("moe_grouped_up(Tensor(a!) act, Tensor x, Tensor w, Tensor sorted_ids, Tensor offsets, Tensor bias, int act_mode, int e_base, float act_limit) -> ()");
   m.def("moe_grouped_down(Tensor(a!) y, Tensor act, Tensor w, Tensor offsets, Tensor bias, int e_base) -> ()");
+  m.def("latent_kv(Tensor(a!) kv, Tensor c, Tensor wk, Tensor wv) -> ()");
   m.def("moe_combine(Tensor(a!) out, Tensor y, Tensor pos, Tensor topi, Tensor topw, Tensor x, Tensor w_id, Tensor shared, int e_base, int e_local) -> ()");
   m.def("moe_combine_norm(Tensor(a!) out, Tensor(b!) residual, Tensor y, Tensor pos, Tensor topi, Tensor topw, Tensor x, Tensor w_id, Tensor shared, Tensor weight, float eps, int e_base, int e_local) -> ()");
 }
@@ -777,5 +855,6 @@ TORCH_LIBRARY_IMPL(kaito, CUDA, m) {
   m.impl("moe_combine_norm", &kaito::moe_combine_norm);
   m.impl("moe_grouped_up", &kaito::moe_grouped_up);
   m.impl("moe_grouped_down", &kaito::moe_grouped_down);
+  m.impl("latent_kv", &kaito::latent_kv);
   m.impl("moe_combine", &kaito::moe_combine);
 }

@@ -133,3 +133,24 @@ def test_prepare_beside_head_rows(T, H, K, N, cached):
     for x, y in zip(got, want):
         assert torch.equal(x, y)
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("T,H,D,V,K", [(4096, 16, 128, 128, 512),
+                                       (4101, 16, 128, 128, 512),
+                                       (16390, 8, 64, 64, 192),
+                                       (5471, 12, 64, 192, 64)])
+def test_latent_kv(T, H, D, V, K):
+    """Rows and columns that end inside a tile; below the tiles' size the
+    library. Sums of up to 512 f32 products, rounded to bf16 once."""
+    torch.manual_seed(T + K)
+    c = _bf16(T, K)
+    wk, wv = _bf16(H, D, K, scale=K ** -0.5), _bf16(H, K, V, scale=K ** -0.5)
+    for rows in (T, 33):
+        k, v = ops.latent_kv(c[:rows], wk, wv)
+        for out, w in ((k, wk.transpose(1, 2)), (v, wv)):
+            w = w.contiguous()
+            for h in (0, H // 2, H - 1):
+                ref = c[:rows].double() @ w[h].double()
+                rms = ref.square().mean().sqrt()
+                err = (out[:, h].double() - ref).abs()
+                assert (err <= 2.0 ** -8 * ref.abs() + 2.0 ** -12 * rms).all()
