@@ -160,10 +160,9 @@ class RGLRUMixer(nn.Module):
             p[:, w:], self.conv_weight, self.conv_bias, cache["conv"],
             meta.cu_seqlens, meta.state_slots, meta.seq_starts,
             meta.token_seq, act=0)
-        gates = ops.rglru_gates(u, self.gate_w, self.gate_b)  # [B, T, 2bw]
-        return ops.rglru_scan(u, gates, p[:, :w], self.decay_rate,
-                              cache["lru"], meta.cu_seqlens, meta.state_slots,
-                              meta.seq_starts, meta.token_seq)
+        return ops.rglru(u, self.gate_w, self.gate_b, p[:, :w],
+                         self.decay_rate, cache["lru"], meta.cu_seqlens,
+                         meta.state_slots, meta.seq_starts, meta.token_seq)
 
 
 class BiasedWindowAttention(nn.Module):

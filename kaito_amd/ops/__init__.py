@@ -48,7 +48,7 @@ for _g, _names in {
             "scaled_softcap"),
     "latent": ("bigram_embed latent_rope_cache_write latent_attention "
                "latent_expand"),
-    "delta": "gated_delta_rule rglru_gates rglru_scan",
+    "delta": "gated_delta_rule rglru_gates rglru_scan rglru_rows",
     "diag": "diag_delta_rule hgrn2_scan gla_scan",
     "decay": "mlstm_scan ssd_scan",
     "streams": "stream_mix_norm stream_embed",
@@ -1039,19 +1039,40 @@ def gated_delta_rule(q, k, v, gate, a, b, a_log, dt_bias, norm_w, state,
         state_slots, seq_starts, qk_eps, norm_eps).reshape(v.size(0), -1)
 
 
+def _rglru_aligned(u, w, bias):
+    return u.is_cuda and u.dtype == torch.bfloat16 and w.size(1) in (64, 128) \
+        and u.size(0) > 0 and u.stride(1) == 1 and u.stride(0) % 8 == 0 \
+        and u.data_ptr() % 16 == 0 and w.is_contiguous() \
+        and bias.is_contiguous()
+
+
 def rglru_gates(u, w, bias):
     """Gate pre-activations of rglru_scan: u [T, B*bw] by blocks of channels
     times w [B, bw, 2*bw] f32, + bias [B, 1, 2*bw] f32, summed in f32.
     Returns [B, T, 2*bw] f32."""
     T, (B, bw, n) = u.size(0), w.shape
-    if u.is_cuda and u.dtype == torch.bfloat16 and bw in (64, 128) \
-            and T > 0 and u.stride(1) == 1 and u.stride(0) % 8 == 0 \
-            and u.data_ptr() % 16 == 0 and w.is_contiguous() \
-            and bias.is_contiguous():
+    if _rglru_aligned(u, w, bias):
         gates = torch.empty(B, T, n, dtype=torch.float32, device=u.device)
         _K.rglru_gates(gates, u, w, bias)
         return gates
     return torch.baddbmm(bias, u.float().view(T, B, bw).transpose(0, 1), w)
+
+
+def rglru(u, w, bias, y, decay_rate, state, cu_seqlens, state_slots,
+          seq_starts, token_seq=None):
+    """rglru_scan of the rows' own rglru_gates."""
+    T, B = u.size(0), state_slots.size(0)
+    # prompt-sized steps (the rule of the segment-parallel scan): the gates
+    # stay in registers. 65 -> 32 us from 128 tokens on, 173 -> 132 at 8192
+    if token_seq is not None and _rglru_aligned(u, w, bias) \
+            and T >= 4 * B and T >= 128 \
+            and y.dtype == u.dtype and y.stride(1) == 1 and state.is_contiguous():
+        out = torch.empty(u.shape, dtype=u.dtype, device=u.device)
+        _K.rglru_rows(out, u, w, bias, y, decay_rate, state, cu_seqlens,
+                      state_slots, seq_starts, token_seq)
+        return out
+    return rglru_scan(u, rglru_gates(u, w, bias), y, decay_rate, state,
+                      cu_seqlens, state_slots, seq_starts, token_seq)
 
 
 def rglru_scan(u, gates, y, decay_rate, state, cu_seqlens, state_slots,

@@ -105,6 +105,52 @@ def test_rglru_segments(lens, pad, dt):
         at += n
 
 
+def _rows(T, bw, blocks):
+    W = bw * blocks
+    p = torch.randn(T, 2 * W, device=DEV).bfloat16()    # [y | x]
+    u = torch.randn(T, W + 8, device=DEV).bfloat16()[:, :W]
+    w = torch.randn(blocks, bw, 2 * bw, device=DEV) * 2 / bw ** 0.5
+    bias = torch.randn(blocks, 1, 2 * bw, device=DEV)
+    rate = torch.rand(W, device=DEV)
+    rate[::7] = 1e-6                      # states that hardly decay
+    return u, w, bias, p[:, :W], rate
+
+
+@pytest.mark.parametrize("bw", [64, 128])
+@pytest.mark.parametrize("lens,pad", [
+    ([130], 0), ([64, 64, 1, 70], 0), ([7, 200, 9], 5), ([31, 0, 513], 0),
+    ([33, 1, 95], 31), ([2500], 0), ([40000, 3, 30000], 1)])
+def test_rglru_rows_of_prompts(lens, pad, bw):
+    """Gates and recurrence together beside one after the other: the same
+    products and steps, sums of 64 rows in another order, of states of up to
+    some 2^5 here (f32: 2^-24 by the depth of 64 rows and 1100 segments)."""
+    torch.manual_seed(len(lens) + bw)
+    T = sum(lens) + pad
+    u, w, bias, y, rate = _rows(T, bw, 2)
+    u[5, 3], u[70, 9] = float("inf"), float("nan")
+    state = torch.randn(len(lens) + 1, 2 * bw, device=DEV)
+    starts = [3 * (i % 2) for i in range(len(lens))]
+    slots = list(range(len(lens), 0, -1))
+    if len(lens) == 4:
+        slots[1] = -1                     # rows 64 to 127 are of no chunk
+    lay = _layout(lens, starts, slots, pad)
+    one, two = state.clone(), state.clone()
+    out = ops.rglru(u, w, bias, y, rate, one, *lay)
+    ref = ops.rglru_scan(u, ops.rglru_gates(u, w, bias), y, rate, two, *lay)
+    at = 0
+    for n, slot in zip(lens, slots):
+        a, b = out[at:at + n].float(), ref[at:at + n].float()
+        at += n
+        if slot < 0 or n == 0:
+            continue
+        assert torch.equal(a.isfinite(), b.isfinite())
+        tol = 2.0 ** -7 * b.abs() + 1e-4 * y[at - n:at].float().abs()
+        assert ((a - b).abs() <= tol)[b.isfinite()].all()
+    assert torch.equal(one.isfinite(), two.isfinite())
+    ok = two.isfinite()
+    assert ((one - two).abs() <= 1e-4 * (1 + two.abs()))[ok].all()
+
+
 @pytest.mark.parametrize("T", [65536, 65537, 65600, 70000])
 def test_rglru_very_long_steps(T):
     """Both sides of the line from which the carries have a launch of their
