@@ -139,7 +139,11 @@ class LlamaAttention(nn.Module):
                 kv_cache: Optional[Tuple[torch.Tensor, torch.Tensor]],
                 meta: AttnMetadata, cos_sin: torch.Tensor,
                 cos_sin_local: Optional[torch.Tensor] = None) -> torch.Tensor:
-        qkv = self.qkv_proj(x)
+        return self.attend(self.qkv_proj(x), positions, kv_cache, meta,
+                           cos_sin, cos_sin_local)
+
+    def attend(self, qkv, positions, kv_cache, meta, cos_sin, cos_sin_local):
+        """Behind the first projection."""
         # strided views into the fused qkv buffer — the HIP kernels take row
         # strides, so no .contiguous() copies on the hot path.
         q, k, v = qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
@@ -154,7 +158,7 @@ class LlamaAttention(nn.Module):
             # by reshape_and_cache, k and v need EQUAL row strides
             v = v.contiguous()
         cs = cos_sin_local if self.local_rope else cos_sin
-        T = x.size(0)
+        T = qkv.size(0)
         sinks = getattr(self, "sinks", None)
         if kv_cache is not None and not meta.is_prefill:
             out = ops.rope_paged_attention(
@@ -292,6 +296,16 @@ class LlamaDecoderLayer(nn.Module):
             return ops.layer_norm(x, w, b, self.cfg.rms_eps)
         return ops.rms_norm(x, w, self.cfg.rms_eps)
 
+    @staticmethod
+    def _in_product(block, name, hidden, residual, norm) -> bool:
+        """Whether the norm before `block` goes into its first projection
+        (decode steps of 1 and 2 rows)."""
+        p = getattr(block, name, None)
+        return p is not None and isinstance(hidden, torch.Tensor) \
+            and get_state().tp_size == 1 and not block._forward_hooks \
+            and not block._forward_pre_hooks \
+            and p.norms(hidden, residual, norm)
+
     def forward(self, hidden, residual, positions, kv_cache, meta, cos_sin,
                 cos_sin_local=None, defer: bool = False):
         """defer: the first result may be MoERows, for the next layer's norm
@@ -321,6 +335,7 @@ class LlamaDecoderLayer(nn.Module):
             m = self.mlp(y)
             m = self._norm(m, "post_feedforward_layernorm")
             return m, stream
+        qkv = None
         if residual is None:
             residual = hidden
             hidden = self._norm(hidden, "input_layernorm")
@@ -328,6 +343,12 @@ class LlamaDecoderLayer(nn.Module):
             hidden, residual = ops.fused_add_layer_norm(
                 hidden, residual, self.input_layernorm,
                 self.input_layernorm_bias, cfg.rms_eps)
+        elif self._in_product(self.self_attn, "qkv_proj", hidden, residual,
+                              self.input_layernorm):
+            p = self.self_attn.qkv_proj
+            qkv, residual = ops.add_norm_linear(
+                hidden, residual, self.input_layernorm, cfg.rms_eps, p.weight,
+                p.bias)
         else:
             # `hidden` here is the PREVIOUS layer's mlp output — a
             # deferred TP partial when a one-shot group is active and the
@@ -336,7 +357,9 @@ class LlamaDecoderLayer(nn.Module):
                 hidden, residual, self.input_layernorm, cfg.rms_eps,
                 deferred_producer=cfg.num_experts == 0)
         hidden = self.self_attn(hidden, positions, kv_cache, meta, cos_sin,
-                                cos_sin_local)
+                                cos_sin_local) if qkv is None else \
+            self.self_attn.attend(qkv, positions, kv_cache, meta, cos_sin,
+                                  cos_sin_local)
         if cfg.norm_type == "layernorm":
             hidden, residual = ops.fused_add_layer_norm(
                 hidden, residual, self.post_attention_layernorm,
@@ -345,6 +368,14 @@ class LlamaDecoderLayer(nn.Module):
             return self.mlp.forward_add_norm(
                 hidden, residual, self.post_attention_layernorm, cfg.rms_eps,
                 defer=True)
+        elif cfg.gated_mlp and cfg.hidden_act != "gelu_tanh" \
+                and self._in_product(self.mlp, "gate_up_proj", hidden,
+                                     residual, self.post_attention_layernorm) \
+                and self.mlp.gate_up_proj.is_plain():
+            act, residual = ops.add_norm_linear(
+                hidden, residual, self.post_attention_layernorm, cfg.rms_eps,
+                self.mlp.gate_up_proj.weight, glu=True)
+            return self.mlp.down_proj(act), residual
         else:
             hidden, residual = _tp_fused_add_rms_norm(
                 hidden, residual, self.post_attention_layernorm, cfg.rms_eps,

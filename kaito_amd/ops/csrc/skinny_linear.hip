@@ -1,6 +1,7 @@
 // Linear layers of decode steps (skinny.h), M <= 32 rows:
 //   skinny_linear  out = x W^T (+ bias)
 //   skinny_swiglu  out = silu(x Wg^T) * (x Wu^T), W = [Wg | Wu] stacked
+//   skinny_norm    either of them of the RMS norm of x + residual
 #include "skinny.h"
 #include <torch/library.h>
 #include <ATen/ATen.h>
@@ -67,6 +68,150 @@ __global__ __launch_bounds__(NW * 64) void skinny_linear_kernel(const Parts a) {
         if (lane == 0 && n0 + r < N)
           out[(int64_t)m * N + n0 + r] = f32_to_bf16(
               acc[m][r] + (bias ? bf16_to_f32(bias[n0 + r]) : 0.f));
+    }
+  }
+}
+
+// The products of rms(x + residual) * g, with the sum left for later layers. Each
+// workgroup norms the rows for itself, on top of its first weights' way: they are
+// asked for behind x and nothing waits for them before the norm is in LDS, and a
+// launch of its own, with nothing under way, is saved. Bit for bit what the norm's
+// kernel and skinny_linear_kernel leave.
+// With the norm's launch, us, two and one (weights out of the caches): 6144 x 4096
+// 11.9, 10.5 for one row and 13.6, 11.4 for two, silu * up of 2 x 14336 x 4096 39.3,
+// 37.7 and 40.9, 39.0, of 2 x 28672 x 8192 143, 140 and 153, 145, 7680 x 5120 18.0,
+// 16.4 and 19.2, 17.3, 1024 x 512 4.6, 2.9 and 5.0, 3.4.
+struct NormArgs {
+  short* out;                       // [M, N]
+  short* sum;                       // [M, K], x + residual
+  const short *x, *residual;        // [M, K]
+  const short* g;                   // [K]
+  const short* w;                   // [N, K]; GLU [2 N, K]
+  const short* bias;                // [N] or nullptr
+  float eps;
+  int N, K;                         // K: 512 n, at most 2048 ITER; WHOLE: that
+};
+
+// until this wave's reads and writes of LDS are done, and those of all waves;
+// loads stay under way
+KAITO_DEV void lds_barrier() {
+  __builtin_amdgcn_s_waitcnt(0xc07f);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+template <int M, int R, int ITER, bool WHOLE, bool GLU>
+__global__ __launch_bounds__(NW * 64) void skinny_norm_kernel(
+    const NormArgs a) {
+  using skinny::hbf16x8;
+  constexpr int U = 4;              // loads of a row under way, 2048 k
+  __shared__ __attribute__((aligned(16))) short xs[M][ITER * 2048];
+  __shared__ float red[M][NW];
+  const int N = a.N, K = WHOLE ? ITER * 2048 : a.K, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = (blockIdx.x * NW + wave) * (GLU ? 1 : R);
+  const int at = threadIdx.x * 8;
+  short8_t v[M][ITER], u[M][ITER], g[ITER];
+#pragma unroll
+  for (int i = 0; i < ITER; i++) {
+    const int c = min(i * 2048 + at, K - 8);
+#pragma unroll
+    for (int m = 0; m < M; m++) {
+      v[m][i] = *reinterpret_cast<const short8_t*>(a.x + m * K + c);
+      u[m][i] = *reinterpret_cast<const short8_t*>(a.residual + m * K + c);
+    }
+    g[i] = *reinterpret_cast<const short8_t*>(a.g + c);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const short* wp[R];
+  float acc[M][R];
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    wp[r] = a.w + (int64_t)(GLU ? r * N + min(n0, N - 1)
+                                : min(n0 + r, N - 1)) * K + lane * 8;
+#pragma unroll
+    for (int m = 0; m < M; m++) acc[m][r] = 0.f;
+  }
+  hbf16x8 w[2][U][R];
+  auto fetch = [&](const int k0, const int b) {
+#pragma unroll
+    for (int j = 0; j < U; j++)
+#pragma unroll
+      for (int r = 0; r < R; r++)
+        if (k0 + j * 512 < K)       // uniform
+          w[b][j][r] = skinny::load_stream<hbf16x8>(wp[r] + k0 + j * 512);
+  };
+  fetch(0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  float ss[M];
+#pragma unroll
+  for (int m = 0; m < M; m++) {
+    ss[m] = 0.f;
+#pragma unroll
+    for (int i = 0; i < ITER; i++) {
+      if (i * 2048 + at >= K) break;
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        v[m][i][j] = f32_to_bf16(bf16_to_f32(v[m][i][j]) +
+                                 bf16_to_f32(u[m][i][j]));
+        const float f = bf16_to_f32(v[m][i][j]);
+        ss[m] += f * f;
+      }
+    }
+    ss[m] = wave_reduce_sum(ss[m]);
+    if (lane == 0) red[m][wave] = ss[m];
+  }
+  lds_barrier();
+#pragma unroll
+  for (int m = 0; m < M; m++) {
+    const float s = (red[m][0] + red[m][1]) + (red[m][2] + red[m][3]);
+    const float inv = rsqrtf(s / (float)K + a.eps);
+#pragma unroll
+    for (int i = 0; i < ITER; i++) {
+      const int c = i * 2048 + at;
+      if (c >= K) break;
+      short8_t o;
+#pragma unroll
+      for (int j = 0; j < 8; j++)
+        o[j] = f32_to_bf16(bf16_to_f32(v[m][i][j]) * inv * bf16_to_f32(g[i][j]));
+      *reinterpret_cast<short8_t*>(&xs[m][c]) = o;
+      if (blockIdx.x == 0)
+        *reinterpret_cast<short8_t*>(a.sum + m * K + c) = v[m][i];
+    }
+  }
+  lds_barrier();
+#pragma unroll
+  for (int i = 0; i < ITER; i++) {
+    const int k0 = i * 2048;
+    if (k0 >= K) break;             // uniform
+    if (i + 1 < ITER) fetch(k0 + 2048, (i + 1) & 1);
+#pragma unroll
+    for (int j = 0; j < U; j++) {
+      if (k0 + j * 512 >= K) break;
+#pragma unroll
+      for (int m = 0; m < M; m++) {
+        const hbf16x8 xv = skinny::load_x(&xs[m][k0 + j * 512 + lane * 8]);
+#pragma unroll
+        for (int r = 0; r < R; r++)
+          acc[m][r] = skinny::dot8(w[i & 1][j][r], xv, acc[m][r]);
+      }
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < M; m++) {
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[m][r] = wave_reduce_sum(acc[m][r]);
+    if constexpr (GLU) {
+      if (lane == 0 && n0 < N)
+        a.out[(int64_t)m * N + n0] =
+            f32_to_bf16(skinny::silu(acc[m][0]) * acc[m][1]);
+    } else {
+#pragma unroll
+      for (int r = 0; r < R; r++)
+        if (lane == 0 && n0 + r < N)
+          a.out[(int64_t)m * N + n0 + r] = f32_to_bf16(
+              acc[m][r] + (a.bias ? bf16_to_f32(a.bias[n0 + r]) : 0.f));
     }
   }
 }
@@ -324,6 +469,58 @@ void skinny_linear_pair(at::Tensor out, at::Tensor x, at::Tensor w,
   run<false>(a, x.data_ptr() == x2.data_ptr() && x.stride(0) == x2.stride(0));
 }
 
+// of rms(x + residual) * g; sum: x + residual, not one of the others
+void skinny_norm(at::Tensor out, at::Tensor sum, at::Tensor x,
+                 at::Tensor residual, at::Tensor g, double eps, at::Tensor w,
+                 at::Tensor bias, bool glu) {
+  TORCH_CHECK(!glu || (w.dim() == 2 && w.size(0) % 2 == 0 && bias.numel() == 0));
+  const int64_t N = glu ? w.size(0) / 2 : w.size(0);
+  check(out, x, w, N, 1);
+  const int64_t M = x.size(0), K = w.size(1);
+  for (const auto& t : {x, residual, sum})
+    TORCH_CHECK(t.is_cuda() && t.is_contiguous() && t.sizes() == x.sizes() &&
+                t.dtype() == at::kBFloat16 && (uintptr_t)t.data_ptr() % 16 == 0);
+  TORCH_CHECK(g.is_cuda() && g.is_contiguous() && g.numel() == K &&
+              g.dtype() == at::kBFloat16 && (uintptr_t)g.data_ptr() % 16 == 0);
+  TORCH_CHECK(M <= 2 && K % 512 == 0 && K <= 8192 &&
+              sum.data_ptr() != residual.data_ptr() &&
+              sum.data_ptr() != x.data_ptr());
+  if (N == 0) return;
+  const Part p = part_of(out, x, w, bias);
+  const NormArgs a = {p.out, (short*)sum.data_ptr(), p.x,
+                      (const short*)residual.data_ptr(),
+                      (const short*)g.data_ptr(), p.w, p.bias, (float)eps,
+                      (int)N, (int)K};
+  auto run_norm = [&](auto m, auto r, auto is_glu) {
+    constexpr int MM = decltype(m)::value, R = decltype(r)::value;
+    constexpr bool GLU = decltype(is_glu)::value;
+    const int64_t per = NW * (GLU ? 1 : R);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((N + per - 1) / per), dim3(NW * 64), 0,
+                         at::hip::getCurrentHIPStream(), a);
+    };
+    auto iter = [&](auto whole) {
+      constexpr bool WHOLE = decltype(whole)::value;
+      if (K <= 2048) go(&skinny_norm_kernel<MM, R, 1, WHOLE, GLU>);
+      else if (K <= 4096) go(&skinny_norm_kernel<MM, R, 2, WHOLE, GLU>);
+      else if (K <= 6144) go(&skinny_norm_kernel<MM, R, 3, WHOLE, GLU>);
+      else go(&skinny_norm_kernel<MM, R, 4, WHOLE, GLU>);
+    };
+    if (K % 2048) iter(std::false_type{});
+    else iter(std::true_type{});
+  };
+  using std::integral_constant;
+  const integral_constant<int, 1> one;
+  const integral_constant<int, 2> two;
+  if (glu) {
+    if (M == 1) run_norm(one, two, std::true_type{});
+    else run_norm(two, two, std::true_type{});
+  } else {
+    if (M == 1) run_norm(one, one, std::false_type{});
+    else run_norm(two, two, std::false_type{});
+  }
+}
+
 void skinny_swiglu(at::Tensor out, at::Tensor x, at::Tensor w) {
   TORCH_CHECK(w.size(0) % 2 == 0);
   const int64_t N = w.size(0) / 2;
@@ -341,10 +538,12 @@ void skinny_swiglu(at::Tensor out, at::Tensor x, at::Tensor w) {
 TORCH_LIBRARY_FRAGMENT(kaito, m) {
   m.def("skinny_linear(Tensor(a!) out, Tensor x, Tensor w, Tensor bias) -> ()");
   m.def("skinny_linear_pair(Tensor(a!) out, Tensor x, Tensor w, Tensor bias, Tensor(b!) out2, Tensor x2, Tensor w2, Tensor bias2) -> ()");
+  m.def("skinny_norm(Tensor(a!) out, Tensor(b!) sum, Tensor x, Tensor residual, Tensor g, float eps, Tensor w, Tensor bias, bool glu) -> ()");
   m.def("skinny_swiglu(Tensor(a!) out, Tensor x, Tensor w) -> ()");
 }
 TORCH_LIBRARY_IMPL(kaito, CUDA, m) {
   m.impl("skinny_linear", &kaito::skinny_linear);
   m.impl("skinny_linear_pair", &kaito::skinny_linear_pair);
+  m.impl("skinny_norm", &kaito::skinny_norm);
   m.impl("skinny_swiglu", &kaito::skinny_swiglu);
 }

@@ -86,6 +86,13 @@ class ColumnParallelLinear(_QuantMixin, nn.Module):
         return self.bias is None and not self._quantized \
             and not lora_mod.is_active()
 
+    def norms(self, x, residual, norm) -> bool:
+        """Whether this layer's product of the RMS norm of x + residual is one
+        launch (ops.add_norm_linear) and nothing but it."""
+        return not self._quantized and not lora_mod.is_active() \
+            and not self._forward_hooks and not self._forward_pre_hooks \
+            and ops.norm_fits(x, residual, norm, self.weight)
+
     def quantized_swiglu(self, x: torch.Tensor):
         """silu(gate) * up of this layer's packed [gate | up] rows, or None
         where that is not one launch."""

@@ -273,3 +273,44 @@ def test_pairs(M, N, N2, K):
         ops._K.skinny_linear_pair(out[0], x, w, b, out[1], y, w2, b2)
         _close(out[0], x.double() @ w.double().T + b.double())
         _close(out[1], y.double() @ w2.double().T + b2.double())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 2])
+@pytest.mark.parametrize("N,K", [(1, 512), (5, 1024), (64, 2048), (9, 2560),
+                                 (30, 4096), (33, 5120), (7, 6144), (3, 6656),
+                                 (18, 8192)])
+def test_norm_in_the_product(M, N, K):
+    """Bit for bit the norm's kernel and the product behind it; the inputs
+    stay as they are, the sum is a buffer of its own."""
+    torch.manual_seed(M * N + K)
+    x, r = (torch.randn(M, K, device=DEV).to(torch.bfloat16) for _ in "xr")
+    g, b = (torch.randn(n, device=DEV).to(torch.bfloat16) for n in (K, 2 * N))
+    w = torch.randn(2 * N, K, device=DEV).to(torch.bfloat16)
+    x0, r0 = x.clone(), r.clone()
+    assert ops.norm_fits(x, r, g, w)
+    normed, total = ops.fused_add_rms_norm(x, r.clone(), g, 1e-5)
+    for bias, glu in ((None, False), (b, False), (None, True)):
+        out, stream = ops.add_norm_linear(x, r, g, 1e-5, w, bias, glu)
+        want = ops.linear_swiglu(normed, w) if glu \
+            else ops.linear(normed, w, bias)
+        assert torch.equal(out, want) and torch.equal(stream, total)
+        assert torch.equal(x, x0) and torch.equal(r, r0)
+
+
+@pytest.mark.gpu
+def test_norm_beside_the_product():
+    """What the one launch does not take goes by the two."""
+    g = torch.ones(512, device=DEV, dtype=torch.bfloat16)
+    w = torch.randn(16, 512, device=DEV).to(torch.bfloat16)
+    for x in (torch.randn(3, 512, device=DEV).to(torch.bfloat16),
+              torch.randn(2, 512, device=DEV).to(torch.bfloat16)):
+        part = x.size(0) == 2
+        v, k = (w[:, :504].contiguous(), 504) if part else (w, 512)
+        x, n = x[:, :k].contiguous(), g[:k].contiguous()
+        r = torch.randn_like(x)
+        assert not ops.norm_fits(x, r, n, v)
+        normed, total = ops.fused_add_rms_norm(x, r.clone(), n, 1e-5)
+        out, stream = ops.add_norm_linear(x, r, n, 1e-5, v)
+        assert torch.equal(out, ops.linear(normed, v))
+        assert torch.equal(stream, total)
