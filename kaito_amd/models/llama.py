@@ -297,14 +297,31 @@ class LlamaDecoderLayer(nn.Module):
         return ops.rms_norm(x, w, self.cfg.rms_eps)
 
     @staticmethod
-    def _in_product(block, name, hidden, residual, norm) -> bool:
-        """Whether the norm before `block` goes into its first projection
+    def _takes_norm(block, hidden) -> bool:
+        """Whether the norm before `block` may go into its first projection
         (decode steps of 1 and 2 rows)."""
-        p = getattr(block, name, None)
-        return p is not None and isinstance(hidden, torch.Tensor) \
+        return isinstance(hidden, torch.Tensor) and hidden.size(0) <= 2 \
             and get_state().tp_size == 1 and not block._forward_hooks \
-            and not block._forward_pre_hooks \
-            and p.norms(hidden, residual, norm)
+            and not block._forward_pre_hooks
+
+    def _norm_qkv(self, hidden, residual):
+        """qkv of the input norm's rows, and the residual, or None."""
+        if self.cfg.is_mla or not self._takes_norm(self.self_attn, hidden):
+            return None
+        p = self.self_attn.qkv_proj
+        if not p.norms(hidden, residual, self.input_layernorm):
+            return None
+        return ops.add_norm_linear(hidden, residual, self.input_layernorm,
+                                   self.cfg.rms_eps, p.weight, p.bias)
+
+    def _norm_act(self, hidden, residual):
+        """The MLP's inner rows of the norm's, and the residual, or None."""
+        cfg = self.cfg
+        if self.routed or not cfg.gated_mlp or cfg.hidden_act == "gelu_tanh" \
+                or not self._takes_norm(self.mlp, hidden):
+            return None
+        return self.mlp.gate_up_proj.norm_swiglu(
+            hidden, residual, self.post_attention_layernorm, cfg.rms_eps)
 
     def forward(self, hidden, residual, positions, kv_cache, meta, cos_sin,
                 cos_sin_local=None, defer: bool = False):
@@ -343,12 +360,8 @@ class LlamaDecoderLayer(nn.Module):
             hidden, residual = ops.fused_add_layer_norm(
                 hidden, residual, self.input_layernorm,
                 self.input_layernorm_bias, cfg.rms_eps)
-        elif self._in_product(self.self_attn, "qkv_proj", hidden, residual,
-                              self.input_layernorm):
-            p = self.self_attn.qkv_proj
-            qkv, residual = ops.add_norm_linear(
-                hidden, residual, self.input_layernorm, cfg.rms_eps, p.weight,
-                p.bias)
+        elif (took := self._norm_qkv(hidden, residual)) is not None:
+            qkv, residual = took
         else:
             # `hidden` here is the PREVIOUS layer's mlp output — a
             # deferred TP partial when a one-shot group is active and the
@@ -368,13 +381,8 @@ class LlamaDecoderLayer(nn.Module):
             return self.mlp.forward_add_norm(
                 hidden, residual, self.post_attention_layernorm, cfg.rms_eps,
                 defer=True)
-        elif cfg.gated_mlp and cfg.hidden_act != "gelu_tanh" \
-                and self._in_product(self.mlp, "gate_up_proj", hidden,
-                                     residual, self.post_attention_layernorm) \
-                and self.mlp.gate_up_proj.is_plain():
-            act, residual = ops.add_norm_linear(
-                hidden, residual, self.post_attention_layernorm, cfg.rms_eps,
-                self.mlp.gate_up_proj.weight, glu=True)
+        elif (took := self._norm_act(hidden, residual)) is not None:
+            act, residual = took
             return self.mlp.down_proj(act), residual
         else:
             hidden, residual = _tp_fused_add_rms_norm(

@@ -37,6 +37,7 @@ for _g, _names in {
             "latent_kv"),
     "route": "moe_route moe_gate_route moe_norm_gate_route moe_sort",
     "quant": ("w4a16_gemv w4a16_dequant w4a16_gemm w4a16_swiglu "
+              "w4a16_norm_swiglu "
               "w4a16_in_tiles lora_shrink lora_expand"),
     "comm": ("allreduce_rmsnorm one_shot_ar_rmsnorm ipc_handle ipc_open "
              "ipc_close"),
@@ -362,10 +363,14 @@ def add_norm_linear(x: torch.Tensor, residual: torch.Tensor,
 
 def norm_fits(x, residual, norm, w) -> bool:
     """Whether add_norm_linear of these is one launch."""
-    return x.dim() == 2 and x.size(0) <= 2 and w.size(1) % 512 == 0 \
-        and w.size(1) <= 8192 and _plain_rows(x, w, 2) \
-        and x.is_contiguous() and residual.is_contiguous() \
-        and residual.shape == x.shape and norm.is_contiguous() \
+    return x.dim() == 2 and x.size(0) <= 2 and _plain_rows(x, w, 2) \
+        and _norm_rows(x, residual, norm)
+
+
+def _norm_rows(x, residual, norm) -> bool:
+    """Rows that a product can norm on the way."""
+    return x.size(1) % 512 == 0 and x.size(1) <= 8192 and x.is_contiguous() \
+        and residual.is_contiguous() and residual.shape == x.shape and norm.is_contiguous() \
         and all(t.dtype == torch.bfloat16 and t.device == x.device
                 and t.data_ptr() % 16 == 0 for t in (residual, norm)) \
         and not (torch.is_grad_enabled() and (
@@ -982,6 +987,27 @@ def w4a16_swiglu(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor,
     out = torch.empty(x.size(0), N, dtype=x.dtype, device=x.device)
     _K.w4a16_swiglu(out, x.contiguous(), qweight, scales, zeros, group)
     return out
+
+
+def w4a16_norm_swiglu(x, residual, norm, eps: float, qweight, scales, zeros,
+                      group: int):
+    """w4a16_swiglu of fused_add_rms_norm's rows and its residual, of 1 and 2
+    rows in one launch; None for other sizes."""
+    if not (x.is_cuda and x.dim() == 2 and 1 <= x.size(0) <= 2
+            and x.dtype == torch.bfloat16 and x.data_ptr() % 16 == 0
+            and qweight.size(0) % 2 == 0 and qweight.data_ptr() % 16 == 0
+            and _norm_rows(x, residual, norm)
+            and not (torch.is_grad_enabled() and x.requires_grad)
+            and not _transformed()
+            and _K.w4a16_in_tiles(x.size(0), qweight.size(0), x.size(1), group,
+                                  True)):
+        return None
+    out = torch.empty(x.size(0), qweight.size(0) // 2, dtype=x.dtype,
+                      device=x.device)
+    stream = torch.empty_like(x)
+    _K.w4a16_norm_swiglu(out, stream, x, residual, norm, eps, qweight, scales,
+                         zeros, group)
+    return out, stream
 
 
 def w4a16_streams(x: torch.Tensor, group: int) -> bool:

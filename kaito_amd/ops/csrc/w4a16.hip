@@ -149,12 +149,26 @@ KAITO_DEV __amdgpu_buffer_rsrc_t w4_buffer(const void* p,
                                            0x27000);
 }
 
-// MR: rows of x that have a place (4 or 16); GLU: N gate rows, then N up rows
-template <int MR, int DEPTH, bool GLU>
+// The rows are rms(x + residual) * g, with the sum left for later layers: up to 2
+// of them, K up to 2048 W4_NORM
+struct W4Norm {
+  short* sum;                       // [M, K]
+  const short *residual, *g;        // [M, K], [K]
+  float eps;
+};
+constexpr int W4_NORM = 4;
+
+// MR: rows of x that have a place (4 or 16); GLU: N gate rows, then N up rows.
+// NORM: four waves norm a row each workgroup for itself, as the norm's kernel does
+// and to the same bits, while the first weights are on the way; its launch is
+// saved: us, two launches and one, 28672 x 4096 20.1, 17.7 for two rows, 22016 x
+// 5120 21.4, 19.1 for one and 22.2, 19.6, 57344 x 8192 48.2, 44.3 and 53.9, 47.0.
+template <int MR, int DEPTH, bool GLU, bool NORM>
 __global__ __launch_bounds__(64 * W4_WAVES) void w4a16_tiles_kernel(
     short* __restrict__ out, const short* __restrict__ x,
     const uint32_t* __restrict__ qw, const float* __restrict__ scales,
-    const float* __restrict__ zeros, const int M, const int N, const int K) {
+    const float* __restrict__ zeros, const int M, const int N, const int K,
+    const W4Norm norm) {
   using skinny::hbf16x8;
   typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
   constexpr int COLS = GLU ? 8 : 16, LOADS = 6, USED = MR * 4;
@@ -208,11 +222,66 @@ __global__ __launch_bounds__(64 * W4_WAVES) void w4a16_tiles_kernel(
       ft += gridDim.x;
     }
   };
+  const int nm = wave / 4, nat = (threadIdx.x & 255) * 8;     // row, first k
+  short8_t nv[NORM ? W4_NORM : 1], nr[NORM ? W4_NORM : 1],
+      ng[NORM ? W4_NORM : 1];
+  if constexpr (NORM) {             // ahead of the weights: loads end in order
+    const int64_t row = (int64_t)min(nm, M - 1) * K;
+#pragma unroll
+    for (int i = 0; i < W4_NORM; i++) {
+      const int k = i * 2048 + nat;
+      if (k >= K) break;            // uniform in a wave: K is whole stages
+      nv[i] = *reinterpret_cast<const short8_t*>(x + row + k);
+      nr[i] = *reinterpret_cast<const short8_t*>(norm.residual + row + k);
+      ng[i] = *reinterpret_cast<const short8_t*>(norm.g + k);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
 #pragma unroll
   for (int i = 0; i < DEPTH; i++) fetch(i);
 
   // ---- x and its sums over the groups; 16 threads have a group
-  for (int c = threadIdx.x; c < M * K / 8; c += 64 * W4_WAVES) {
+  if constexpr (NORM) {
+    float* const rn = reinterpret_cast<float*>(red);
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < W4_NORM; i++) {
+      if (i * 2048 + nat >= K) break;
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        nv[i][e] = f32_to_bf16(bf16_to_f32(nv[i][e]) + bf16_to_f32(nr[i][e]));
+        const float f = bf16_to_f32(nv[i][e]);
+        ss += f * f;
+      }
+    }
+    ss = wave_reduce_sum(ss);
+    if (lane == 0) rn[wave] = ss;
+    __builtin_amdgcn_s_waitcnt(0xc07f);       // weights stay under way
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const float* s = rn + nm * 4;
+    const float inv =
+        rsqrtf(((s[0] + s[1]) + (s[2] + s[3])) / (float)K + norm.eps);
+#pragma unroll
+    for (int i = 0; i < W4_NORM; i++) {
+      const int k = i * 2048 + nat;
+      if (nm >= M || k >= K) break;           // uniform in a wave
+      hbf16x8 v;
+      float sum = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        v[e] = (__bf16)(bf16_to_f32(nv[i][e]) * inv * bf16_to_f32(ng[i][e]));
+        sum += (float)v[e];
+      }
+      sum = group_reduce_sum<16>(sum);
+      *reinterpret_cast<hbf16x8*>(xl + nm * (K + 8) + k) =
+          skinny::nibble_order(v);
+      if (nat % 128 == 0) xs[k / 128 * MR + nm] = sum;
+      if (blockIdx.x == 0)
+        *reinterpret_cast<short8_t*>(norm.sum + (int64_t)nm * K + k) = nv[i];
+    }
+  } else for (int c = threadIdx.x; c < M * K / 8; c += 64 * W4_WAVES) {
     const int m = c / (K / 8), k = c % (K / 8) * 8;
     const hbf16x8 v = skinny::load_x(x + (int64_t)m * K + k);
     float sum = 0.f;
@@ -333,10 +402,11 @@ bool w4_tiles_pay(int64_t M, int64_t rows, int64_t K, bool glu) {
   return K > 2048 || (K == 2048 && (M <= 8 || rows >= 6144));
 }
 
-template <bool GLU>
+template <bool GLU, bool NORM = false>
 bool launch_w4_tiles(at::Tensor& out, const at::Tensor& x,
                      const at::Tensor& qweight, const at::Tensor& scales,
-                     const at::Tensor& zeros, int64_t group) {
+                     const at::Tensor& zeros, int64_t group,
+                     const W4Norm& norm = {}) {
   const int M = x.size(0), K = x.size(1);
   const int N = qweight.size(0) / (GLU ? 2 : 1);
   const int depth = w4_tiles_depth(M, qweight.size(0), K, group);
@@ -345,14 +415,14 @@ bool launch_w4_tiles(at::Tensor& out, const at::Tensor& x,
     return false;
   const dim3 grid(std::min(256, N / (GLU ? 8 : 16)));
 #define W4T_LAUNCH(MR_, D_)                                                   \
-  hipLaunchKernelGGL((w4a16_tiles_kernel<MR_, D_, GLU>), grid,                \
+  hipLaunchKernelGGL((w4a16_tiles_kernel<MR_, D_, GLU, NORM>), grid,               \
       dim3(64 * W4_WAVES), 0,                                                 \
       at::hip::getCurrentHIPStream(), (short*)out.data_ptr(),                 \
       (const short*)x.data_ptr(), (const uint32_t*)qweight.data_ptr(),        \
-      scales.data_ptr<float>(), zeros.data_ptr<float>(), M, N, K)
+      scales.data_ptr<float>(), zeros.data_ptr<float>(), M, N, K, norm)
   if (M <= 4) {
     if (depth == 3) W4T_LAUNCH(4, 3); else W4T_LAUNCH(4, 2);
-  } else {
+  } else if constexpr (!NORM) {
     if (depth == 3) W4T_LAUNCH(16, 3); else W4T_LAUNCH(16, 2);
   }
 #undef W4T_LAUNCH
@@ -587,6 +657,33 @@ void w4a16_swiglu(at::Tensor out, at::Tensor x, at::Tensor qweight,
               out.size(1) * 2 == qweight.size(0));
   TORCH_CHECK(launch_w4_tiles<true>(out, x, qweight, scales, zeros, group),
               "w4a16_swiglu: sizes of the tiles");
+}
+
+// the same of rms(x + residual) * g; sum: x + residual, not one of the others
+void w4a16_norm_swiglu(at::Tensor out, at::Tensor sum, at::Tensor x,
+                       at::Tensor residual, at::Tensor g, double eps,
+                       at::Tensor qweight, at::Tensor scales, at::Tensor zeros,
+                       int64_t group) {
+  const int64_t M = x.size(0), K = x.size(1);
+  for (const auto& t : {x, residual, sum})
+    TORCH_CHECK(t.is_cuda() && t.is_contiguous() && t.sizes() == x.sizes() &&
+                t.dtype() == at::kBFloat16 && (uintptr_t)t.data_ptr() % 16 == 0);
+  TORCH_CHECK(g.is_cuda() && g.is_contiguous() && g.numel() == K &&
+              g.dtype() == at::kBFloat16 && (uintptr_t)g.data_ptr() % 16 == 0);
+  TORCH_CHECK(out.is_contiguous() && out.dtype() == at::kBFloat16 &&
+              qweight.is_contiguous() && scales.is_contiguous() &&
+              zeros.is_contiguous() && qweight.size(0) % 2 == 0 &&
+              qweight.size(1) * 8 == K && out.size(0) == M &&
+              out.size(1) * 2 == qweight.size(0));
+  TORCH_CHECK(M >= 1 && M <= 2 && K <= 2048 * W4_NORM &&
+              sum.data_ptr() != residual.data_ptr() &&
+              sum.data_ptr() != x.data_ptr());
+  const W4Norm norm = {(short*)sum.data_ptr(),
+                       (const short*)residual.data_ptr(),
+                       (const short*)g.data_ptr(), (float)eps};
+  TORCH_CHECK((launch_w4_tiles<true, true>(out, x, qweight, scales, zeros,
+                                           group, norm)),
+              "w4a16_norm_swiglu: sizes of the tiles");
 }
 
 void w4a16_dequant(at::Tensor out, at::Tensor qweight, at::Tensor scales,

@@ -89,9 +89,26 @@ class ColumnParallelLinear(_QuantMixin, nn.Module):
     def norms(self, x, residual, norm) -> bool:
         """Whether this layer's product of the RMS norm of x + residual is one
         launch (ops.add_norm_linear) and nothing but it."""
-        return not self._quantized and not lora_mod.is_active() \
-            and not self._forward_hooks and not self._forward_pre_hooks \
+        return not self._quantized and self._bare() \
             and ops.norm_fits(x, residual, norm, self.weight)
+
+    def norm_swiglu(self, x, residual, norm, eps: float):
+        """silu(gate) * up of the RMS norm of x + residual, and that sum, or
+        None where that is not one launch."""
+        if self.bias is not None or not self._bare():
+            return None
+        if self._quantized:
+            return ops.w4a16_norm_swiglu(x, residual, norm, eps, self.qweight,
+                                         self.scales, self.zeros, self.q_group)
+        if not ops.norm_fits(x, residual, norm, self.weight):
+            return None
+        return ops.add_norm_linear(x, residual, norm, eps, self.weight,
+                                   glu=True)
+
+    def _bare(self) -> bool:
+        """No adapter, no hooks."""
+        return not lora_mod.is_active() and not self._forward_hooks \
+            and not self._forward_pre_hooks
 
     def quantized_swiglu(self, x: torch.Tensor):
         """silu(gate) * up of this layer's packed [gate | up] rows, or None

@@ -314,3 +314,24 @@ def test_norm_beside_the_product():
         out, stream = ops.add_norm_linear(x, r, n, 1e-5, v)
         assert torch.equal(out, ops.linear(normed, v))
         assert torch.equal(stream, total)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 16, 512), (2, 32, 2560), (2, 4112, 4096),
+                                   (1, 5616, 5120), (2, 48, 8192)])
+def test_norm_in_the_packed_product(M, N, K):
+    """Bit for bit the norm's kernel and the SwiGLU product behind it."""
+    torch.manual_seed(N + K)
+    x, r = (torch.randn(M, K, device=DEV).to(torch.bfloat16) for _ in "xr")
+    g = torch.randn(K, device=DEV).to(torch.bfloat16)
+    packed = quantize_w4(torch.randn(N, K, device=DEV), 128)
+    x0, r0 = x.clone(), r.clone()
+    normed, total = ops.fused_add_rms_norm(x, r.clone(), g, 1e-5)
+    want = ops.w4a16_swiglu(normed, *packed, 128)
+    took = ops.w4a16_norm_swiglu(x, r, g, 1e-5, *packed, 128)
+    assert (took is None) == (want is None)
+    if took is not None:
+        assert torch.equal(took[0], want) and torch.equal(took[1], total)
+        assert torch.equal(x, x0) and torch.equal(r, r0)
+    assert ops.w4a16_norm_swiglu(x.repeat(3, 1), r.repeat(3, 1), g, 1e-5,
+                                 *packed, 128) is None
