@@ -37,12 +37,13 @@ __global__ void delta_prep_kernel(
     float* __restrict__ qn, float* __restrict__ kn,      // [T, G, D]
     float* __restrict__ kq,                               // [T, G] = qn . kn
     float* __restrict__ decay, float* __restrict__ beta,  // [T, H]
+    float* __restrict__ o,                                // [T, H, V]
     const T* __restrict__ q, const int64_t q_s0, const int64_t q_s1,
     const T* __restrict__ k, const int64_t k_s0, const int64_t k_s1,
     const T* __restrict__ a, const int64_t a_s0,
     const T* __restrict__ b, const int64_t b_s0,
     const float* __restrict__ a_log, const float* __restrict__ dt_bias,
-    const int G, const int D, const int H, const float qk_eps) {
+    const int G, const int D, const int H, const int V, const float qk_eps) {
   // one wave per (token, qk head); wave 0 of head 0 also does decay/beta
   const int t = blockIdx.x;
   const int g = blockIdx.y;
@@ -68,6 +69,10 @@ __global__ void delta_prep_kernel(
     ko[d] = act_ld(kr + d) * ik;
   }
   if (lane == 0) kq[(int64_t)t * G + g] = sqk * iq * ik;
+  // rows of padding chunks are never written by the recurrence: the epilogue
+  // reads zeros (a fill of its own was 2.4 us of a decode step)
+  const int n = H / G * V;
+  for (int d = lane; d < n; d += 64) o[((int64_t)t * G + g) * n + d] = 0.f;
   if (g == 0) {
     for (int h = lane; h < H; h += 64) {
       const float av = act_ld(a + (int64_t)t * a_s0 + h);
@@ -451,6 +456,7 @@ bool run_chunks(hipStream_t stream, const at::Tensor& q, const at::Tensor& k,
       !reach(H * (int64_t)V * 4) || !reach(v.stride(0) * v.element_size()) ||
       pin == 0 || getenv("KAITO_DELTA_ROWS_PER_LANE"))
     return false;
+  o.zero_();                        // rows of padding chunks
   const int64_t chunks = T_ / dc::C + B;
   at::Tensor rec = at::empty({chunks, H, dc::REC}, qn.options());
   const int64_t groups = (int64_t)B * H * (V / 16);
@@ -528,11 +534,11 @@ void run_delta(hipStream_t stream, at::Tensor& out, const at::Tensor& q,
   hipLaunchKernelGGL((delta_prep_kernel<T>), dim3(T_, G), dim3(64), 0,
       stream, qn.data_ptr<float>(), kn.data_ptr<float>(),
       kq.data_ptr<float>(), decay.data_ptr<float>(), beta.data_ptr<float>(),
-      (const T*)q.data_ptr(), q.stride(0), q.stride(1),
+      o.data_ptr<float>(), (const T*)q.data_ptr(), q.stride(0), q.stride(1),
       (const T*)k.data_ptr(), k.stride(0), k.stride(1),
       (const T*)a.data_ptr(), a.stride(0), (const T*)b.data_ptr(),
       b.stride(0), a_log.data_ptr<float>(), dt_bias.data_ptr<float>(), G, D,
-      H, qk_eps);
+      H, V, qk_eps);
   int wparts = 1;
   while (wparts * 32 < D) wparts <<= 1;
   if (D % 4 == 0 && wparts <= 8) {
@@ -610,9 +616,7 @@ void gated_delta_rule(at::Tensor out, at::Tensor q, at::Tensor k,
   at::Tensor qn = at::empty({T, G, D}, f32), kn = at::empty({T, G, D}, f32);
   at::Tensor decay = at::empty({T, H}, f32), beta = at::empty({T, H}, f32);
   at::Tensor kq = at::empty({T, G}, f32);
-  // rows of padding chunks are never written by the recurrence: zero so
-  // the epilogue reads defined values
-  at::Tensor o = at::zeros({T, H, V}, f32);
+  at::Tensor o = at::empty({T, H, V}, f32);
 
   // rows per thread (DP) and threads per state column (PARTS)
   int dp = 32, parts = 1;

@@ -456,3 +456,25 @@ def test_post_norm(H, pair, dt):
     ref = X + n(m) * w.double()
     assert ((x32.double() - ref).abs() <= 2e-6 * (1 + ref.abs())).all()
     assert torch.equal(xa, x32.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("D", [64, 96])
+@pytest.mark.parametrize("n", [1, 40])
+def test_delta_rule_of_padding_chunks(n, D):
+    """Rows of a chunk without a slot leave zeros, whatever the scratch held
+    (one token and 40 a chunk: both forms of the recurrence)."""
+    G, H, V = 2, 4, 32
+    lens, slots = [n, n, n], [1, -1, 0]
+    T = sum(lens)
+    r = lambda *s: torch.randn(*s, device=DEV).bfloat16()
+    f = lambda *s: torch.randn(*s, device=DEV)
+    cu, sl, st, _ = _layout(lens, [0, 0, 3], slots)
+    args = (r(T, G, D), r(T, G, D), r(T, H, V), r(T, H, V), r(T, H), r(T, H),
+            f(H), f(H), f(V), f(2, H, D, V), cu, sl, st, 1e-6, 1e-6)
+    for _ in range(2):
+        held = [torch.full((T, H, V), float("nan"), device=DEV)
+                for _ in range(8)]
+        del held
+        out = ops.gated_delta_rule(*args)
+        assert out.isfinite().all() and not out[n:2 * n].any()
+        assert out[:n].any() and out[2 * n:].any()
