@@ -220,20 +220,22 @@ class LlamaMLP(nn.Module):
         tp = get_state().tp_size
         self.inter_per_rank = cfg.intermediate_size // tp
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, defer: bool = False) -> torch.Tensor:
+        """defer: the result may be ops.SplitRows, for the next norm."""
+        down = self.down_proj.for_norm if defer else self.down_proj
         if not self.cfg.gated_mlp:
-            return self.down_proj(ops.gelu(self.up_proj(x)))
+            return down(ops.gelu(self.up_proj(x)))
         p = self.gate_up_proj
         if self.cfg.hidden_act != "gelu_tanh" and p.is_plain():
-            return self.down_proj(ops.linear_swiglu(x, p.weight))
+            return down(ops.linear_swiglu(x, p.weight))
         if self.cfg.hidden_act != "gelu_tanh":
             act = p.quantized_swiglu(x)
             if act is not None:
-                return self.down_proj(act)
+                return down(act)
         gu = p(x)
         act = ops.gelu_and_mul(gu) if self.cfg.hidden_act == "gelu_tanh" \
             else ops.silu_and_mul(gu)
-        return self.down_proj(act)
+        return down(act)
 
 
 def _tp_fused_add_rms_norm(hidden, residual, weight, eps: float,
@@ -325,8 +327,8 @@ class LlamaDecoderLayer(nn.Module):
 
     def forward(self, hidden, residual, positions, kv_cache, meta, cos_sin,
                 cos_sin_local=None, defer: bool = False):
-        """defer: the first result may be MoERows, for the next layer's norm
-        (RMS norms, one rank)."""
+        """defer: the first result may be MoERows or SplitRows, for the next
+        layer's norm (RMS norms, one rank)."""
         cfg = self.cfg
         if cfg.parallel_block:
             # phi-2/falcon: one shared norm; attn and mlp read the same
@@ -388,7 +390,10 @@ class LlamaDecoderLayer(nn.Module):
             hidden, residual = _tp_fused_add_rms_norm(
                 hidden, residual, self.post_attention_layernorm, cfg.rms_eps,
                 deferred_producer=True)   # o_proj always defer-capable
-        hidden = self.mlp(hidden)
+        # residual rows, which the norm behind reads, are bf16 as these
+        defer = defer and not self.routed and not self.mlp._forward_hooks \
+            and hidden.dtype == residual.dtype and residual.is_contiguous()
+        hidden = self.mlp(hidden, defer=True) if defer else self.mlp(hidden)
         return hidden, residual
 
 

@@ -27,7 +27,7 @@ for _g, _names in {
     "core": ("rms_norm fused_add_rms_norm rotary_embedding silu_and_mul "
              "gelu_and_mul gelu layer_norm fused_add_layer_norm "
              "rope_and_cache reshape_and_cache topk skinny_linear skinny_norm skinny_swiglu "
-             "skinny_linear_pair batch_linear"),
+             "skinny_linear_pair batch_linear batch_parts add_rms_norm_parts"),
     "attn": ("paged_attention paged_attention_sp rope_paged_attention "
              "prefill_attention "
              "mla_prefill_attention context_attention mfma_tile_gemm paged_read_bw"),
@@ -297,6 +297,31 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
                 _K.batch_linear(out, x, w, _none(bias, x), 0, 0, False)
             return out
     return torch.nn.functional.linear(x, w, bias)
+
+
+class SplitRows:
+    """A product whose K was split, before the sum of its parts [splits, M, N]
+    f32: whoever normalises it next sums it in the same launch."""
+
+    def __init__(self, part: torch.Tensor):
+        self.part = part
+
+    def add_rms_norm(self, residual, weight, eps: float):
+        """fused_add_rms_norm of it, to the same bits."""
+        out = torch.empty_like(residual)
+        _K.add_rms_norm_parts(out, self.part, residual, weight, eps)
+        return out, residual
+
+
+def linear_parts(x: torch.Tensor, w: torch.Tensor):
+    """linear(x, w) for the add and RMS norm behind it: SplitRows where the
+    product is the split kernel's and in parts, of rows that the norm can sum
+    (always ahead, by 0.4 us of 29 to 4 of 104)."""
+    if w.size(0) <= 8192 and not _skinny(x, w) and _batched(x, w):
+        part = _K.batch_parts(x, w)
+        if part.numel():
+            return SplitRows(part)
+    return linear(x, w)
 
 
 def linear_pair(x: torch.Tensor, w: torch.Tensor, x2: torch.Tensor,

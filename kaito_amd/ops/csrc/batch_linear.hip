@@ -311,21 +311,32 @@ void launch(const BatchArgs& a, int cols) {
 
 }  // namespace
 
-void batch_linear(at::Tensor out, at::Tensor x, at::Tensor w, at::Tensor bias,
-                  int64_t cols, int64_t splits, bool glu) {
-  for (const auto& t : {out, x, w})
+static BatchArgs batch_args(const at::Tensor& x, const at::Tensor& w, bool glu) {
+  for (const auto& t : {x, w})
     TORCH_CHECK(t.is_cuda() && t.dtype() == at::kBFloat16 && t.dim() == 2 &&
                 t.stride(1) == 1 && (uintptr_t)t.data_ptr() % 16 == 0);
   BatchArgs a{};
-  a.M = (int)x.size(0); a.N = (int)out.size(1); a.K = (int)x.size(1);
+  TORCH_CHECK(w.size(0) % (glu ? 2 : 1) == 0 && w.size(0) < (1ll << 31) &&
+              x.size(0) >= 1 && x.size(0) <= 256 && w.size(1) < (1ll << 31));
+  a.M = (int)x.size(0);
+  a.N = (int)(w.size(0) / (glu ? 2 : 1));
+  a.K = (int)w.size(1);
   a.x_stride = x.stride(0);
-  TORCH_CHECK(w.is_contiguous() && out.is_contiguous() && w.size(1) == a.K &&
-              w.size(0) == (glu ? 2 : 1) * (int64_t)a.N &&
-              out.size(0) == a.M && x.size(0) <= 256 && a.M >= 1 &&
+  TORCH_CHECK(w.is_contiguous() && x.size(1) == a.K &&
               (a.M == 1 || a.x_stride % 8 == 0) && a.K % 64 == 0 && a.K > 0 &&
-              a.N % 16 == 0);
-  TORCH_CHECK(w.size(0) < (1ll << 31) && (int64_t)a.M * a.x_stride < (1ll << 31) &&
+              a.N % 16 == 0 && (int64_t)a.M * a.x_stride < (1ll << 31) &&
               ((glu ? a.N : 0) + 128ll) * a.K < (1ll << 31));
+  a.x = (const short*)x.data_ptr();
+  a.w = (const short*)w.data_ptr();
+  return a;
+}
+
+void batch_linear(at::Tensor out, at::Tensor x, at::Tensor w, at::Tensor bias,
+                  int64_t cols, int64_t splits, bool glu) {
+  BatchArgs a = batch_args(x, w, glu);
+  TORCH_CHECK(out.is_cuda() && out.dtype() == at::kBFloat16 && out.dim() == 2 &&
+              out.is_contiguous() && (uintptr_t)out.data_ptr() % 16 == 0 &&
+              out.size(0) == a.M && out.size(1) == a.N);
   const bool has_bias = bias.numel() > 0;
   TORCH_CHECK(!has_bias || (!glu && bias.is_cuda() && bias.is_contiguous() &&
                             bias.dtype() == at::kBFloat16 &&
@@ -339,8 +350,6 @@ void batch_linear(at::Tensor out, at::Tensor x, at::Tensor w, at::Tensor bias,
   TORCH_CHECK((cols == 64 || cols == 128) && splits >= 1 &&
               splits <= a.K / 64 && !(glu && splits > 1));
   a.out = (short*)out.data_ptr();
-  a.x = (const short*)x.data_ptr();
-  a.w = (const short*)w.data_ptr();
   a.bias = has_bias ? (const short*)bias.data_ptr() : nullptr;
   a.splits = (int)splits;
   if (glu) return launch<GLU>(a, cols);
@@ -355,11 +364,26 @@ void batch_linear(at::Tensor out, at::Tensor x, at::Tensor w, at::Tensor bias,
                      a.splits, total, a.N);
 }
 
+// The splits' sums [splits, M, N] f32 of batch_linear's plan; empty if it has one
+at::Tensor batch_parts(at::Tensor x, at::Tensor w) {
+  BatchArgs a = batch_args(x, w, false);
+  const Plan p = plan_for(a.M, a.N, a.K, false);
+  const auto f32 = x.options().dtype(at::kFloat);
+  if (a.N == 0 || p.splits == 1) return at::empty({0}, f32);
+  const at::Tensor part = at::empty({p.splits, a.M, a.N}, f32);
+  a.part = part.data_ptr<float>();
+  a.splits = p.splits;
+  launch<PARTIAL>(a, p.cols);
+  return part;
+}
+
 }  // namespace kaito
 
 TORCH_LIBRARY_FRAGMENT(kaito, m) {
+  m.def("batch_parts(Tensor x, Tensor w) -> Tensor");
   m.def("batch_linear(Tensor(a!) out, Tensor x, Tensor w, Tensor bias, int cols, int splits, bool glu) -> ()");
 }
 TORCH_LIBRARY_IMPL(kaito, CUDA, m) {
+  m.impl("batch_parts", &kaito::batch_parts);
   m.impl("batch_linear", &kaito::batch_linear);
 }

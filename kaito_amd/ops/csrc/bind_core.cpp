@@ -5,6 +5,8 @@
 
 namespace kaito {
 void rms_norm(at::Tensor out, at::Tensor input, at::Tensor weight, double eps);
+void add_rms_norm_parts(at::Tensor out, at::Tensor part, at::Tensor residual,
+                        at::Tensor weight, double eps);
 void fused_add_rms_norm(at::Tensor out, at::Tensor input, at::Tensor residual,
                         at::Tensor weight, double eps);
 void rotary_embedding(at::Tensor positions, at::Tensor q, at::Tensor k,
@@ -28,6 +30,7 @@ void topk(at::Tensor out_vals, at::Tensor out_idx, at::Tensor scores,
 
 TORCH_LIBRARY_FRAGMENT(kaito, m) {
   m.def("rms_norm(Tensor(a!) out, Tensor input, Tensor weight, float eps) -> ()");
+  m.def("add_rms_norm_parts(Tensor(a!) out, Tensor part, Tensor(b!) residual, Tensor weight, float eps) -> ()");
   m.def("fused_add_rms_norm(Tensor(a!) out, Tensor input, Tensor(b!) residual, Tensor weight, float eps) -> ()");
   m.def("rotary_embedding(Tensor positions, Tensor(a!) q, Tensor(b!) k, int head_dim, Tensor cos_sin_cache) -> ()");
   m.def("silu_and_mul(Tensor(a!) out, Tensor x) -> ()");
@@ -42,6 +45,7 @@ TORCH_LIBRARY_FRAGMENT(kaito, m) {
 
 TORCH_LIBRARY_IMPL(kaito, CUDA, m) {
   m.impl("rms_norm", &kaito::rms_norm);
+  m.impl("add_rms_norm_parts", &kaito::add_rms_norm_parts);
   m.impl("fused_add_rms_norm", &kaito::fused_add_rms_norm);
   m.impl("rotary_embedding", &kaito::rotary_embedding);
   m.impl("silu_and_mul", &kaito::silu_and_mul);

@@ -152,6 +152,14 @@ class RowParallelLinear(_QuantMixin, nn.Module):
             torch.empty(out_features, dtype=dtype),
             requires_grad=False) if bias else None
 
+    def for_norm(self, x: torch.Tensor):
+        """forward for an add and RMS norm behind it: rows, or ops.SplitRows."""
+        if self._quantized or self.bias is not None or x.dim() != 2 \
+                or get_state().tp_size > 1 or lora_mod.is_active() \
+                or self._forward_hooks or self._forward_pre_hooks:
+            return self(x)
+        return ops.linear_parts(x, self.weight)
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         out = self._qmatmul(x) if self._quantized \
             else ops.linear(x, self.weight)

@@ -103,3 +103,30 @@ def test_replayed_graph():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(9, 1024, 10240), (16, 4096, 14336),
+                                   (33, 2064, 11008), (250, 4096, 14336),
+                                   (130, 8192, 12288), (64, 4096, 4096)])
+def test_parts_into_the_norm(M, N, K):
+    """Bit for bit the sum's launch and the norm's behind it."""
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K, device="cuda").bfloat16()
+    w = (torch.randn(N, K, device="cuda") * K ** -0.5).bfloat16()
+    r = torch.randn(M, N, device="cuda").bfloat16()
+    g = torch.randn(N, device="cuda").bfloat16()
+    want, total = ops.fused_add_rms_norm(ops.linear(x, w), r.clone(), g, 1e-5)
+    rows = ops.linear_parts(x, w)
+    assert isinstance(rows, ops.SplitRows)
+    out, stream = rows.add_rms_norm(r.clone(), g, 1e-5)
+    assert torch.equal(out, want) and torch.equal(stream, total)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(8, 4096, 14336), (257, 4096, 14336),
+                                   (250, 4096, 4096)])
+def test_no_parts_elsewhere(M, N, K):
+    x = torch.randn(M, K, device="cuda").bfloat16()
+    w = torch.randn(N, K, device="cuda").bfloat16()
+    assert torch.equal(ops.linear_parts(x, w), ops.linear(x, w))
