@@ -32,7 +32,8 @@
 // an XCD's 32 CUs is cut in quarters, 128 x 128, one per CU; so is a small step's
 // only round of up to 16. Measured on one MI355X, 8 experts of 2048 x 2048, top
 // 2, rows as drawn from 16 kinds of tokens, us, two buffers and whole tiles, now:
-// 8192 tokens 317 and 278 (990 TFLOP/s), down 165 and 139; 4096 174 and 149, 106
+// 8192 tokens 317 and 278, with the epilogue of today 254 (1080 TFLOP/s), down 165 and
+// 139; 4096 174 and 149, 106
 // and 86; 2048 114 and 90; 1000 down 60 and 49. 8 of 4096 x 14336, 8192 tokens:
 // 3419 and 3262 (1180 TFLOP/s), 1875 and 1676. 8-byte stores cost a tenth more. A
 // library GEMM per expert with its gathers, casts and index_add took 958 us behind
