@@ -138,12 +138,16 @@ class LlamaAttention(nn.Module):
     def forward(self, x: torch.Tensor, positions: torch.Tensor,
                 kv_cache: Optional[Tuple[torch.Tensor, torch.Tensor]],
                 meta: AttnMetadata, cos_sin: torch.Tensor,
-                cos_sin_local: Optional[torch.Tensor] = None) -> torch.Tensor:
+                cos_sin_local: Optional[torch.Tensor] = None,
+                defer: bool = False) -> torch.Tensor:
         return self.attend(self.qkv_proj(x), positions, kv_cache, meta,
-                           cos_sin, cos_sin_local)
+                           cos_sin, cos_sin_local, defer)
 
-    def attend(self, qkv, positions, kv_cache, meta, cos_sin, cos_sin_local):
-        """Behind the first projection."""
+    def attend(self, qkv, positions, kv_cache, meta, cos_sin, cos_sin_local,
+               defer):
+        """Behind the first projection. defer: the result may be
+        ops.SplitRows, for the next norm."""
+        o_proj = self.o_proj.for_norm if defer else self.o_proj
         # strided views into the fused qkv buffer — the HIP kernels take row
         # strides, so no .contiguous() copies on the hot path.
         q, k, v = qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
@@ -165,7 +169,7 @@ class LlamaAttention(nn.Module):
                 positions, q, k, v, self.head_dim, cs, kv_cache[0],
                 kv_cache[1], meta.slot_mapping, meta.block_tables,
                 meta.seq_lens, self.scale, self.window, sinks)
-            return self.o_proj(out.reshape(T, -1))
+            return o_proj(out.reshape(T, -1))
         if kv_cache is not None:
             q, k = ops.rope_and_cache(positions, q, k, v, self.head_dim, cs,
                                       kv_cache[0], kv_cache[1],
@@ -188,7 +192,7 @@ class LlamaAttention(nn.Module):
             out = ops.prefill_attention(qh, kh, vh, meta.cu_seqlens,
                                         self.scale, meta.max_seqlen,
                                         self.window, sinks, tiles)
-        return self.o_proj(out.reshape(T, -1))
+        return o_proj(out.reshape(T, -1))
 
 
 class LlamaMLP(nn.Module):
@@ -371,10 +375,16 @@ class LlamaDecoderLayer(nn.Module):
             hidden, residual = _tp_fused_add_rms_norm(
                 hidden, residual, self.input_layernorm, cfg.rms_eps,
                 deferred_producer=cfg.num_experts == 0)
-        hidden = self.self_attn(hidden, positions, kv_cache, meta, cos_sin,
-                                cos_sin_local) if qkv is None else \
-            self.self_attn.attend(qkv, positions, kv_cache, meta, cos_sin,
-                                  cos_sin_local)
+        # residual rows, which the norm behind reads, are bf16 as these
+        parts = defer and not self.routed and residual.is_contiguous() \
+            and hidden.dtype == residual.dtype
+        kv = (positions, kv_cache, meta, cos_sin, cos_sin_local)
+        if qkv is not None:
+            hidden = self.self_attn.attend(qkv, *kv, parts)
+        elif parts and not cfg.is_mla and not self.self_attn._forward_hooks:
+            hidden = self.self_attn(hidden, *kv, defer=True)
+        else:
+            hidden = self.self_attn(hidden, *kv)
         if cfg.norm_type == "layernorm":
             hidden, residual = ops.fused_add_layer_norm(
                 hidden, residual, self.post_attention_layernorm,
@@ -390,10 +400,8 @@ class LlamaDecoderLayer(nn.Module):
             hidden, residual = _tp_fused_add_rms_norm(
                 hidden, residual, self.post_attention_layernorm, cfg.rms_eps,
                 deferred_producer=True)   # o_proj always defer-capable
-        # residual rows, which the norm behind reads, are bf16 as these
-        defer = defer and not self.routed and not self.mlp._forward_hooks \
-            and hidden.dtype == residual.dtype and residual.is_contiguous()
-        hidden = self.mlp(hidden, defer=True) if defer else self.mlp(hidden)
+        hidden = self.mlp(hidden, defer=True) \
+            if parts and not self.mlp._forward_hooks else self.mlp(hidden)
         return hidden, residual
 
 
