@@ -26,6 +26,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from ..engine.config import ModelConfig
+from ..parallel.layers import untouched
 from .hybrid_base import HybridStackBase, MixerLayerBase
 from .hybrid_config import LayerSpec, layer_moe_config
 from .mixers import BiasedWindowAttention, GatedDeltaMixer, RGLRUMixer
@@ -71,11 +72,17 @@ class HybridLayer(MixerLayerBase):
             xa = ops.post_norm_residual(x32, y, self.norm1, eps, dt)
         else:
             a, r = self.attn, self.rglru
-            pa, pr = ops.linear_pair(xa, a.qkv_proj, xa, r.in_proj, None,
-                                     r.in_bias)
-            oa = a.mix(pa, positions, self._view(cache, a), meta)
-            yo = r.mix(pr, self._view(cache, r), meta)
-            ya, yr = ops.linear_pair(oa, a.o_proj, yo, r.o_proj)
+            ca, cr = self._view(cache, a), self._view(cache, r)
+            if untouched(a, BiasedWindowAttention) \
+                    and untouched(r, RGLRUMixer):
+                pa, pr = ops.linear_pair(xa, a.qkv_proj, xa, r.in_proj, None,
+                                         r.in_bias)
+                oa = a.mix(pa, positions, ca, meta)
+                yo = r.mix(pr, cr, meta)
+                ya, yr = ops.linear_pair(oa, a.o_proj, yo, r.o_proj)
+            else:
+                ya = a(xa, positions, ca, meta)
+                yr = r(xa, positions, cr, meta)
             xa = ops.post_norm_residual(x32, ya, self.norm1, eps, dt, y2=yr,
                                         w_y=self.attn_out_norm,
                                         w_y2=self.rglru_out_norm)

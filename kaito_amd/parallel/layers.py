@@ -10,10 +10,21 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules import module as _module
 
 from .. import ops
 from .state import get_state, tp_all_reduce
 from ..engine import lora as lora_mod
+
+
+def untouched(module: nn.Module, cls: type) -> bool:
+    """Whether a call of `module` is cls.forward and nothing else: no hooks, no
+    forward of its own in its place. Only then may a layer call its parts."""
+    return type(module).forward is cls.forward \
+        and "forward" not in vars(module) \
+        and not (module._forward_hooks or module._forward_pre_hooks
+                 or _module._global_forward_hooks
+                 or _module._global_forward_pre_hooks)
 
 
 class _QuantMixin:

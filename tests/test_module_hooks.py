@@ -1,0 +1,77 @@
+"""Modules that a caller watches or replaces are called as modules: hooks run, get
+tensors and may change them, whatever the layer would otherwise do in fewer
+launches."""
+import dataclasses
+
+import pytest
+import torch
+
+from kaito_amd.engine import EngineConfig, LLMEngine, SamplingParams
+from kaito_amd.models import get_model_config
+from kaito_amd.parallel.state import init_parallel
+
+DEVICES = ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)]
+
+
+def _engine(device, name, **changes):
+    init_parallel(1)
+    mc = dataclasses.replace(get_model_config(name), **changes)
+    if device == "cpu":
+        mc = dataclasses.replace(mc, dtype=torch.float32)
+    torch.manual_seed(7)
+    return LLMEngine(EngineConfig(
+        model=mc, device=device, max_num_seqs=4, max_model_len=256,
+        num_gpu_blocks=64, enforce_eager=True))
+
+
+def _generate(eng):
+    out = eng.generate([list(range(3, 25))],
+                       SamplingParams(max_tokens=4, temperature=0.0,
+                                      ignore_eos=True))
+    return out[0].output_token_ids
+
+
+def _watch(modules):
+    """Forward hooks on modules; the calls of each, of its tensors' types."""
+    calls = {m: [] for m in modules}
+
+    def seen(m, args, out):
+        first = out[0] if isinstance(out, tuple) else out
+        calls[m].append((type(args[0]), type(first)))
+    handles = [m.register_forward_hook(seen) for m in modules]
+    return calls, handles
+
+
+def _check_watched(eng, modules):
+    calls, handles = _watch(modules)
+    _generate(eng)
+    for h in handles:
+        h.remove()
+    for m, c in calls.items():
+        # a prompt step, then one for each of the other three tokens
+        assert len(c) == 4, (type(m).__name__, c)
+        assert all(issubclass(t, torch.Tensor) for pair in c for t in pair), c
+
+
+@pytest.mark.parametrize("device", DEVICES)
+def test_mixers_of_a_hybrid_layer(device):
+    eng = _engine(device, "tiny-gurapel-test")
+    layers = [l for l in eng.runner.model.layers if l.spec.kind == "parallel"]
+    assert layers
+    _check_watched(eng, [m for l in layers for m in (l.attn, l.rglru)])
+
+
+@pytest.mark.parametrize("device", DEVICES)
+def test_replaced_forward_of_a_mixer(device):
+    """What wraps a module by giving it a forward of its own is not passed by."""
+    eng = _engine(device, "tiny-gurapel-test")
+    layer = next(l for l in eng.runner.model.layers
+                 if l.spec.kind == "parallel")
+    plain, calls = layer.rglru.forward, []
+
+    def forward(*args):
+        calls.append(args[0].size(0))
+        return plain(*args)
+    layer.rglru.forward = forward
+    _generate(eng)
+    assert calls == [22, 1, 1, 1]
