@@ -92,10 +92,9 @@ class ColumnParallelLinear(_QuantMixin, nn.Module):
             requires_grad=False) if bias else None
 
     def is_plain(self) -> bool:
-        """Nothing but the product with the weight: no bias, packed weight
-        or adapter."""
-        return self.bias is None and not self._quantized \
-            and not lora_mod.is_active()
+        """Nothing but the product with the weight: no bias, packed weight,
+        adapter or hook."""
+        return self.bias is None and not self._quantized and self._bare()
 
     def norms(self, x, residual, norm) -> bool:
         """Whether this layer's product of the RMS norm of x + residual is one
@@ -118,14 +117,14 @@ class ColumnParallelLinear(_QuantMixin, nn.Module):
 
     def _bare(self) -> bool:
         """No adapter, no hooks."""
-        return not lora_mod.is_active() and not self._forward_hooks \
-            and not self._forward_pre_hooks
+        return not lora_mod.is_active() \
+            and untouched(self, ColumnParallelLinear)
 
     def quantized_swiglu(self, x: torch.Tensor):
         """silu(gate) * up of this layer's packed [gate | up] rows, or None
         where that is not one launch."""
         if not self._quantized or self.bias is not None \
-                or lora_mod.is_active() or x.dim() != 2:
+                or not self._bare() or x.dim() != 2:
             return None
         return ops.w4a16_swiglu(x, self.qweight, self.scales, self.zeros,
                                 self.q_group)
@@ -167,7 +166,7 @@ class RowParallelLinear(_QuantMixin, nn.Module):
         """forward for an add and RMS norm behind it: rows, or ops.SplitRows."""
         if self._quantized or self.bias is not None or x.dim() != 2 \
                 or get_state().tp_size > 1 or lora_mod.is_active() \
-                or self._forward_hooks or self._forward_pre_hooks:
+                or not untouched(self, RowParallelLinear):
             return self(x)
         return ops.linear_parts(x, self.weight)
 

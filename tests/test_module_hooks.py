@@ -75,3 +75,23 @@ def test_replaced_forward_of_a_mixer(device):
     layer.rglru.forward = forward
     _generate(eng)
     assert calls == [22, 1, 1, 1]
+
+
+@pytest.mark.parametrize("device", DEVICES)
+def test_query_projection_of_latent_attention(device):
+    eng = _engine(device, "tiny-deepseek-test", q_lora_rank=0)
+    _check_watched(eng, [l.self_attn.q_proj for l in eng.runner.model.layers])
+
+
+@pytest.mark.parametrize("device", DEVICES)
+def test_gate_projection(device):
+    eng = _engine(device, "tiny-llama-test")
+    _check_watched(eng, [l.mlp.gate_up_proj for l in eng.runner.model.layers])
+
+
+@pytest.mark.gpu
+def test_packed_gate_projection():
+    eng = _engine("cuda", "tiny-llama-test")
+    for l in eng.runner.model.layers:
+        l.mlp.gate_up_proj.quantize_(128)
+    _check_watched(eng, [l.mlp.gate_up_proj for l in eng.runner.model.layers])
