@@ -307,7 +307,15 @@ class SplitRows:
         self.part = part
 
     def add_rms_norm(self, residual, weight, eps: float):
-        """fused_add_rms_norm of it, to the same bits."""
+        """fused_add_rms_norm of it, to the same bits; one launch for rows
+        and weights in whole 16-byte chunks."""
+        if not (self.part.is_cuda and residual.data_ptr() % 16 == 0
+                and weight.data_ptr() % 16 == 0):
+            rows = self.part[0]
+            for p in self.part[1:]:
+                rows = rows + p
+            return fused_add_rms_norm(rows.to(residual.dtype), residual,
+                                      weight, eps)
         out = torch.empty_like(residual)
         _K.add_rms_norm_parts(out, self.part, residual, weight, eps)
         return out, residual

@@ -130,3 +130,23 @@ def test_no_parts_elsewhere(M, N, K):
     x = torch.randn(M, K, device="cuda").bfloat16()
     w = torch.randn(N, K, device="cuda").bfloat16()
     assert torch.equal(ops.linear_parts(x, w), ops.linear(x, w))
+
+
+@pytest.mark.parametrize("what", ["rows", "weight"])
+def test_parts_that_the_norm_kernel_does_not_take(what):
+    """Residual rows or weights at odd addresses, which the norm of whole rows
+    takes: the parts are summed first, to the same bits."""
+    def at_odd(t):
+        return torch.empty(t.numel() + 1, dtype=t.dtype)[1:].view(
+            t.shape).copy_(t)
+    torch.manual_seed(3)
+    part = torch.randn(3, 20, 64)
+    r, g = torch.randn(20, 64).bfloat16(), torch.randn(64).bfloat16()
+    rows = ((part[0] + part[1]) + part[2]).bfloat16()
+    want, total = ops.fused_add_rms_norm(rows, r.clone(), g, 1e-5)
+    if what == "rows":
+        r = at_odd(r)
+    else:
+        g = at_odd(g)
+    out, stream = ops.SplitRows(part).add_rms_norm(r, g, 1e-5)
+    assert torch.equal(out, want) and torch.equal(stream, total)
