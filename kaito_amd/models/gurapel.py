@@ -87,7 +87,7 @@ class HybridLayer(MixerLayerBase):
                                         w_y=self.attn_out_norm,
                                         w_y2=self.rglru_out_norm)
         if self.mlp is not None:
-            f = self.mlp(xa, defer=True)
+            f = self.mlp(xa, defer=untouched(self.mlp, MoEMLP))
             xa = f.post_norm(x32, self.norm2, eps, dt) \
                 if isinstance(f, MoERows) \
                 else ops.post_norm_residual(x32, f, self.norm2, eps, dt)

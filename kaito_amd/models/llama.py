@@ -22,7 +22,7 @@ from .. import ops
 from ..engine.config import ModelConfig
 from ..parallel.state import get_state
 from ..parallel.layers import (ColumnParallelLinear, RowParallelLinear,
-                               VocabParallelEmbedding)
+                               VocabParallelEmbedding, untouched)
 
 
 @dataclass
@@ -303,16 +303,15 @@ class LlamaDecoderLayer(nn.Module):
         return ops.rms_norm(x, w, self.cfg.rms_eps)
 
     @staticmethod
-    def _takes_norm(block, hidden) -> bool:
+    def _takes_norm(block, cls, hidden) -> bool:
         """Whether the norm before `block` may go into its first projection
         (decode steps of 1 and 2 rows)."""
         return isinstance(hidden, torch.Tensor) and hidden.size(0) <= 2 \
-            and get_state().tp_size == 1 and not block._forward_hooks \
-            and not block._forward_pre_hooks
+            and get_state().tp_size == 1 and untouched(block, cls)
 
     def _norm_qkv(self, hidden, residual):
         """qkv of the input norm's rows, and the residual, or None."""
-        if self.cfg.is_mla or not self._takes_norm(self.self_attn, hidden):
+        if not self._takes_norm(self.self_attn, LlamaAttention, hidden):
             return None
         p = self.self_attn.qkv_proj
         if not p.norms(hidden, residual, self.input_layernorm):
@@ -324,7 +323,7 @@ class LlamaDecoderLayer(nn.Module):
         """The MLP's inner rows of the norm's, and the residual, or None."""
         cfg = self.cfg
         if self.routed or not cfg.gated_mlp or cfg.hidden_act == "gelu_tanh" \
-                or not self._takes_norm(self.mlp, hidden):
+                or not self._takes_norm(self.mlp, LlamaMLP, hidden):
             return None
         return self.mlp.gate_up_proj.norm_swiglu(
             hidden, residual, self.post_attention_layernorm, cfg.rms_eps)
@@ -381,7 +380,7 @@ class LlamaDecoderLayer(nn.Module):
         kv = (positions, kv_cache, meta, cos_sin, cos_sin_local)
         if qkv is not None:
             hidden = self.self_attn.attend(qkv, *kv, parts)
-        elif parts and not cfg.is_mla and not self.self_attn._forward_hooks:
+        elif parts and untouched(self.self_attn, LlamaAttention):
             hidden = self.self_attn(hidden, *kv, defer=True)
         else:
             hidden = self.self_attn(hidden, *kv)
@@ -401,7 +400,7 @@ class LlamaDecoderLayer(nn.Module):
                 hidden, residual, self.post_attention_layernorm, cfg.rms_eps,
                 deferred_producer=True)   # o_proj always defer-capable
         hidden = self.mlp(hidden, defer=True) \
-            if parts and not self.mlp._forward_hooks else self.mlp(hidden)
+            if parts and untouched(self.mlp, LlamaMLP) else self.mlp(hidden)
         return hidden, residual
 
 
@@ -478,13 +477,16 @@ class LlamaForCausalLM(nn.Module):
         # a layer's experts are summed by the norm behind it
         defer = cfg.norm_type != "layernorm" and not cfg.parallel_block \
             and not cfg.sandwich_norms and get_state().tp_size == 1
-        last = len(self.layers) - 1
+        # rows that are no tensor yet pass between layers that nobody watches
+        plain = [defer and untouched(layer, LlamaDecoderLayer)
+                 for layer in self.layers]
+        plain.append(self.is_last)
         for i, layer in enumerate(self.layers):
             kv = kv_caches[i] if kv_caches is not None else None
             hidden, residual = layer(hidden, residual, positions, kv, meta,
                                      self.cos_sin_cache,
                                      self.cos_sin_cache_local,
-                                     defer and (i < last or self.is_last))
+                                     plain[i] and plain[i + 1])
         if self.is_last:
             if self.cfg.norm_type == "layernorm":
                 hidden, _ = ops.fused_add_layer_norm(

@@ -26,6 +26,7 @@ import torch.nn as nn
 
 from .. import ops
 from ..engine.config import ModelConfig
+from ..parallel.layers import untouched
 from ..parallel.state import get_state, tp_all_reduce
 
 
@@ -220,7 +221,8 @@ class MoEMLP(nn.Module):
         (output, residual)."""
         xn, residual, *chosen = ops.moe_norm_gate_route(
             x, residual, weight, eps, *self._choice())
-        return self(xn, defer=defer, chosen=chosen), residual
+        return self(xn, defer=defer and untouched(self, MoEMLP),
+                    chosen=chosen), residual
 
     def forward(self, x: torch.Tensor, keep_f32: bool = False,
                 split_shared: bool = False, defer: bool = False,

@@ -6,6 +6,7 @@ import dataclasses
 import pytest
 import torch
 
+from kaito_amd import ops
 from kaito_amd.engine import EngineConfig, LLMEngine, SamplingParams
 from kaito_amd.models import get_model_config
 from kaito_amd.parallel.state import init_parallel
@@ -95,3 +96,34 @@ def test_packed_gate_projection():
     for l in eng.runner.model.layers:
         l.mlp.gate_up_proj.quantize_(128)
     _check_watched(eng, [l.mlp.gate_up_proj for l in eng.runner.model.layers])
+
+
+def _in_parts(x, w):
+    """Every product as if the split kernel had made it."""
+    y = x.float() @ w.float().t()
+    return ops.SplitRows(torch.stack([y * 0.75, y * 0.25]))
+
+
+@pytest.mark.parametrize("which", [
+    lambda ls: [ls[0]], lambda ls: [ls[1]], lambda ls: [ls[0].self_attn],
+    lambda ls: [ls[0].mlp], lambda ls: [m for l in ls for m in (
+        l, l.self_attn, l.mlp, l.self_attn.o_proj, l.mlp.down_proj)]],
+    ids=["first", "second", "attention", "mlp", "all"])
+def test_decoder_layers_with_products_in_parts(monkeypatch, which):
+    eng = _engine("cpu", "tiny-llama-test")
+    want = _generate(eng)
+    monkeypatch.setattr(ops, "linear_parts", _in_parts)
+    assert _generate(eng) == want
+    _check_watched(eng, which(eng.runner.model.layers))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["tiny-moe-test", "tiny-gurapel-test",
+                                  "tiny-deepseek-test", "tiny-llama-test"])
+@pytest.mark.parametrize("which", ["first", "last", "mlp", "all"])
+def test_layers_on_the_gpu(name, which):
+    eng = _engine("cuda", name)
+    ls = eng.runner.model.layers
+    _check_watched(eng, {
+        "first": [ls[0]], "last": [ls[-1]], "mlp": [l.mlp for l in ls],
+        "all": [m for l in ls for m in (l, l.mlp)]}[which])
