@@ -236,8 +236,19 @@ def _batched(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
     (4096 x 14336: 25.4, 26.4 at 16 rows, 27.4, 34.9 at 48, 36.9, 49.4 at 128,
     45.5, 59.1 at 256; 7168 x 18432 at 256 89, 208), to 16384 rows of W
     (beyond, W is cut often enough without: 28672 x 14336 at 128 1 % behind).
-    K in no multiple of 512, which the library has few kernels for (4096 x
-    2880: 1.5 to 1.9 times as fast from 17 to 128 rows; behind at 256).
+    K in no multiple of 256, which the library has few kernels for (4096 x
+    2880: 1.1 to 1.25 times as fast from 17 to 128 rows, 28672 x 2880 1.24 to
+    1.39; behind at 256). In odd multiples of 256: below 4096 only wide outputs
+    and up to 64 rows (8192 x 2816 1.04 to 1.30, 16384 x 3840 1.05 to 1.18 but
+    0.96 at 96, 4096 x 2816 0.80 to 0.95, 12288 x 3840 at 64 0.90); else to
+    8192 rows of W (4096 x 5376 1.16 to 1.41; 3072 x 4352 0.86 to 0.98), beyond
+    to 64 (16384 x 5376 1.07 to 1.18, at 96 to 128 0.99, 20480 x 5376 0.86 to
+    0.92), to 16384 at K of 8192 and more (16384 x 8960 1.0 to 1.16; 20480 x
+    8960 at 128 0.90). Beyond 32768 rows of W a workgroup has all of K and the
+    library enough tiles: to 32 rows (40960 x 2880 1.20, 49152 x 5376 0.98 to
+    1.02, 131072 x 8960 1.06; at 64 0.93 to 1.09, at 128 0.81 to 0.93), to 96 of
+    a vocabulary of 200000 (201088 x 2880 349, 207 at 17 rows, 357, 272 at 96,
+    266, 287 at 128; 262208 x 5376 581, 455, 639, 612 and 574, 632).
     K from 4096: to 6144 rows of W (3072 x 5120 at 64 1.26 times, 4096 x 7168
     at 128 1.6; at K of 4096 only to 64 rows, 4096 x 4096 14.3, 15.3 there and
     18.6, 17.7 at 128; at K of 8192 only beyond 32 rows, 4096 x 8192 at 24
@@ -268,7 +279,18 @@ def _batched_shape(M: int, N: int, K: int, glu: bool) -> bool:
     if M < 17:
         return False
     if K % 512:
-        return K >= 2560 and N >= 3072 and M <= 128
+        if not (K >= 2560 and N >= 3072 and M <= 128):
+            return False
+        if N > 32768:
+            return M <= 32 or (N >= 196608 and M <= 96)
+        if K % 256:
+            return True
+        if K < 4096:
+            return M <= 64 and N >= 8192 and (
+                M <= 32 or not 12288 <= N < 16384)
+        if N < 4096:
+            return K >= 5120
+        return M <= 64 or N <= (16384 if K >= 8192 else 8192)
     if K < 4096 or K > 8192 or N < 3072:
         return False
     if M > 192:

@@ -72,6 +72,28 @@ def test_route(M, N, K, glu):
         _close(ops.linear(x, w, b), ref + b.double())
 
 
+def _sides(N, K, glu, ahead, behind):
+    for M in ahead:
+        assert ops._batched_shape(M, N, K, glu), (M, N, K)
+    for M in behind:
+        assert not ops._batched_shape(M, N, K, glu), (M, N, K)
+
+
+@pytest.mark.parametrize("N,K,ahead,behind", [
+    (4096, 2880, (17, 128), (129, 256)), (28672, 2880, (17, 128), ()),
+    (40960, 2880, (17, 32), (64, 96, 128)), (57344, 2880, (32,), (96, 128)),
+    (131072, 3840, (32,), (96, 128)), (201088, 2880, (17, 64, 96), (128,)),
+    (262208, 5376, (17, 96), (128,)), (8192, 2816, (17, 64), (96, 128)),
+    (3072, 3840, (), (17, 64)), (4096, 2816, (), (17, 64, 128)),
+    (12288, 3840, (17,), (64, 128)), (16384, 3840, (17, 64), (96, 128)),
+    (3072, 4352, (), (17, 64)), (3072, 5376, (17, 128), ()),
+    (8192, 5376, (17, 128), ()), (20480, 5376, (17, 64), (96, 128)),
+    (16384, 8960, (17, 128), ()), (20480, 8960, (64,), (128,))])
+def test_inner_sizes_in_no_multiple_of_512(N, K, ahead, behind):
+    """The sides of the line on which either was measured to be faster."""
+    _sides(N, K, False, ahead, behind)
+
+
 @pytest.mark.gpu
 def test_stays_with_the_library():
     x, w, _ = _inputs(64, 4096, 4096)
