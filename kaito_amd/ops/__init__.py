@@ -249,13 +249,18 @@ def _batched(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
     1.02, 131072 x 8960 1.06; at 64 0.93 to 1.09, at 128 0.81 to 0.93), to 96 of
     a vocabulary of 200000 (201088 x 2880 349, 207 at 17 rows, 357, 272 at 96,
     266, 287 at 128; 262208 x 5376 581, 455, 639, 612 and 574, 632).
-    K from 4096: to 6144 rows of W (3072 x 5120 at 64 1.26 times, 4096 x 7168
-    at 128 1.6; at K of 4096 only to 64 rows, 4096 x 4096 14.3, 15.3 there and
-    18.6, 17.7 at 128; at K of 8192 only beyond 32 rows, 4096 x 8192 at 24
-    20.6, 17.9); to 8192 between K of 4096 and 8192 (8192 x 7168: 1.02 to 1.47;
-    8192 x 4096 at 64 0.88, 8192 x 8192 at 64 0.84); 16384 to 65536 to 64 rows
-    (1.03 to 1.16; 128256 x 4096 at 32 206, 193). 193 to 256 rows: 6144 to 16384 with K from 7168 (1.06 to
-    1.67; 4096 x 7168 0.91).
+    K from 4096: to 6144 rows of W (3072 x 5120 at 64 1.19 times, 4096 x 7168
+    at 128 1.67), fewer than 4096 only from K of 5120 on (3072 x 4096 0.86 to
+    0.93 to 64 rows, 3072 x 4608 0.88 to 0.97); below 4608 only to 64 rows (4096
+    x 4096 14.2, 14.9 there, ahead once the norm behind it sums the parts, and
+    16.9, 18.8 at 128; 4096 x 4608 1.09 to 1.48 to 192 rows); at K of 8192 only
+    beyond 32 rows (4096 x 8192 0.92 at 32, 1.19 at 33). To 8192 between K of
+    4608 and 8192 (8192 x 7168: 1.02 to 1.47; 8192 x 4096 at 64 0.88, 8192 x
+    8192 at 64 0.84); 16384 to 32768 to 64 rows (1.00 to 1.16), beyond to 32
+    and from K of 5120 (49152 x 7168 at 32 1.08 and 0.96 at 64, 57344 x 5120
+    1.08 and 0.95; 36864 x 4608 0.97, 49152 x 4096 0.82; 128256 x 4096 206,
+    193). 193 to 256 rows: 6144 to 16384 with K from 7168 (1.06 to 1.67; 4096 x
+    7168 0.91).
     SwiGLU pairs, which save a launch and a pass: from 12288 rows of W with
     more than 16 rows, 32 for K of 2048 (28672 x 4096: 48.9, 57.2 at 64, 73.6,
     79.8 at 256; 12288 x 2048 16.6, 20.2 at 64; 8192 x 4096 0.89), beyond 32768
@@ -296,10 +301,13 @@ def _batched_shape(M: int, N: int, K: int, glu: bool) -> bool:
     if M > 192:
         return K >= 7168 and 6144 <= N <= 16384 and (K < 8192 or N <= 12288)
     if N <= 6144:
-        return M <= 64 if K == 4096 else K < 8192 or M > 32
+        return (N >= 4096 or K >= 5120) and (M <= 64 or K >= 4608) \
+            and (M > 32 or K < 8192)
     if N <= 8192:
-        return 4096 < K < 8192
-    return 16384 <= N <= 65536 and K < 8192 and M <= 64
+        return 4608 <= K < 8192
+    if N <= 32768:
+        return N >= 16384 and K < 8192 and M <= 64
+    return N <= 65536 and 5120 <= K < 8192 and M <= 32
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:

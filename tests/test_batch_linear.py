@@ -94,6 +94,19 @@ def test_inner_sizes_in_no_multiple_of_512(N, K, ahead, behind):
     _sides(N, K, False, ahead, behind)
 
 
+@pytest.mark.parametrize("N,K,ahead,behind", [
+    (3072, 4096, (), (17, 32, 64)), (3072, 4608, (), (17, 64, 160)),
+    (3072, 5120, (17, 64, 128), ()), (4096, 4096, (17, 64), (128, 192)),
+    (4096, 4608, (17, 64, 128, 192), ()), (5120, 4096, (17, 64), ()),
+    (4096, 8192, (33, 192), (17, 32)), (8192, 4608, (17, 192), ()),
+    (16384, 4096, (17, 64), ()), (32768, 4096, (17, 64), (65,)),
+    (36864, 4096, (), (17, 64)), (57344, 4096, (), (17, 64)),
+    (36864, 4608, (), (17, 64)), (36864, 5120, (17, 32), (33, 64)),
+    (49152, 7168, (17, 32), (64,)), (128256, 4096, (), (17, 64))])
+def test_inner_sizes_in_multiples_of_512(N, K, ahead, behind):
+    _sides(N, K, False, ahead, behind)
+
+
 @pytest.mark.gpu
 def test_stays_with_the_library():
     x, w, _ = _inputs(64, 4096, 4096)
