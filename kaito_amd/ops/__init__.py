@@ -265,7 +265,10 @@ def _batched(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
     more than 16 rows, 32 for K of 2048 (28672 x 4096: 48.9, 57.2 at 64, 73.6,
     79.8 at 256; 12288 x 2048 16.6, 20.2 at 64; 8192 x 4096 0.89), beyond 32768
     to 64 rows (57344 x 4096: 1.07 to 1.13, 0.90 at 256), at K of 8192 from
-    20480 on (16384 x 8192 0.97)."""
+    20480 on (16384 x 8192 0.97). 20480 rows of W are 160 workgroups of 64 + 64
+    columns, which leaves CUs idle: with K beyond 4096 not from 65 to 128 rows
+    (20480 x 5120 1.14 at 32, 0.94 and 0.87 at 96 and 128, 0.99 at 192; x 7168
+    0.97, 0.92; 22016 x 5120 0.93 at 128, 22528 x 5120 1.01)."""
     M = x.size(0)
     if not 9 <= M <= 256 or w.dim() != 2:
         return False
@@ -277,6 +280,8 @@ def _batched_shape(M: int, N: int, K: int, glu: bool) -> bool:
     if K % 64 or N % (32 if glu else 16) or (N + 128) * K >= 1 << 31:
         return False
     if glu:
+        if 64 < M <= 128 and 16384 < N < 22528 and K > 4096:
+            return False
         return M > (16 if K > 2048 else 32) and K >= 2048 and N >= (
             20480 if K >= 8192 else 12288) and (N <= 32768 or (N <= 65536 and M <= 64))
     if K >= 10240:

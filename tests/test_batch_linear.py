@@ -107,6 +107,15 @@ def test_inner_sizes_in_multiples_of_512(N, K, ahead, behind):
     _sides(N, K, False, ahead, behind)
 
 
+@pytest.mark.parametrize("N,K,ahead,behind", [
+    (20480, 4096, (17, 96, 128), ()), (20480, 5120, (17, 64, 192), (96, 128)),
+    (20480, 8192, (64, 192), (128,)), (22016, 5120, (64,), (128,)),
+    (16384, 5120, (17, 128, 256), ()), (22528, 5120, (17, 128, 256), ()),
+    (28672, 4096, (17, 128, 256), (16,)), (57344, 4096, (64,), (65, 256))])
+def test_sizes_of_pairs(N, K, ahead, behind):
+    _sides(N, K, True, ahead, behind)
+
+
 @pytest.mark.gpu
 def test_stays_with_the_library():
     x, w, _ = _inputs(64, 4096, 4096)
