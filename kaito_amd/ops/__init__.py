@@ -236,6 +236,10 @@ def _batched(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
     (4096 x 14336: 25.4, 26.4 at 16 rows, 27.4, 34.9 at 48, 36.9, 49.4 at 128,
     45.5, 59.1 at 256; 7168 x 18432 at 256 89, 208), to 16384 rows of W
     (beyond, W is cut often enough without: 28672 x 14336 at 128 1 % behind).
+    Fewer than 2048 rows of W with K below 13824 only to 64 rows (1024 x 10240
+    15.1, 16.0 at 64, 17.2, 15.6 at 96, 26.3, 22.2 at 256, and 13.5, 11.5 at 16,
+    where the norm behind it gives most of that back), of inner sizes in
+    multiples of 512 (1024 x 11008 at 32 14.3, 18.0).
     K in no multiple of 256, which the library has few kernels for (4096 x
     2880: 1.1 to 1.25 times as fast from 17 to 128 rows, 28672 x 2880 1.24 to
     1.39; behind at 256). In odd multiples of 256: below 4096 only wide outputs
@@ -247,13 +251,13 @@ def _batched(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
     8960 at 128 0.90). Beyond 32768 rows of W a workgroup has all of K and the
     library enough tiles: to 32 rows (40960 x 2880 1.20, 49152 x 5376 0.98 to
     1.02, 131072 x 8960 1.06; at 64 0.93 to 1.09, at 128 0.81 to 0.93), to 96 of
-    a vocabulary of 200000 (201088 x 2880 349, 207 at 17 rows, 357, 272 at 96,
-    266, 287 at 128; 262208 x 5376 581, 455, 639, 612 and 574, 632).
+    a vocabulary of 200000 (201088 x 2880 207, 349 at 17 rows, 272, 357 at 96,
+    287, 266 at 128; 262208 x 5376 455, 581, 612, 639 and 632, 574).
     K from 4096: to 6144 rows of W (3072 x 5120 at 64 1.19 times, 4096 x 7168
     at 128 1.67), fewer than 4096 only from K of 5120 on (3072 x 4096 0.86 to
     0.93 to 64 rows, 3072 x 4608 0.88 to 0.97); below 4608 only to 64 rows (4096
-    x 4096 14.2, 14.9 there, ahead once the norm behind it sums the parts, and
-    16.9, 18.8 at 128; 4096 x 4608 1.09 to 1.48 to 192 rows); at K of 8192 only
+    x 4096 14.9, 14.2 there, ahead once the norm behind it sums the parts, and
+    18.8, 16.9 at 128; 4096 x 4608 1.09 to 1.48 to 192 rows); at K of 8192 only
     beyond 32 rows (4096 x 8192 0.92 at 32, 1.19 at 33). To 8192 between K of
     4608 and 8192 (8192 x 7168: 1.02 to 1.47; 8192 x 4096 at 64 0.88, 8192 x
     8192 at 64 0.84); 16384 to 32768 to 64 rows (1.00 to 1.16), beyond to 32
@@ -285,7 +289,8 @@ def _batched_shape(M: int, N: int, K: int, glu: bool) -> bool:
         return M > (16 if K > 2048 else 32) and K >= 2048 and N >= (
             20480 if K >= 8192 else 12288) and (N <= 32768 or (N <= 65536 and M <= 64))
     if K >= 10240:
-        return 1024 <= N <= 16384
+        return N <= 16384 and N >= (
+            2048 if M > 64 and K < 13824 and K % 512 == 0 else 1024)
     if M < 17:
         return False
     if K % 512:

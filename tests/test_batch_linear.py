@@ -102,7 +102,10 @@ def test_inner_sizes_in_no_multiple_of_512(N, K, ahead, behind):
     (16384, 4096, (17, 64), ()), (32768, 4096, (17, 64), (65,)),
     (36864, 4096, (), (17, 64)), (57344, 4096, (), (17, 64)),
     (36864, 4608, (), (17, 64)), (36864, 5120, (17, 32), (33, 64)),
-    (49152, 7168, (17, 32), (64,)), (128256, 4096, (), (17, 64))])
+    (49152, 7168, (17, 32), (64,)), (128256, 4096, (), (17, 64)),
+    (1024, 10240, (9, 64), (96, 256)), (1024, 12800, (32,), (128,)),
+    (2048, 10240, (9, 96, 256), ()), (1024, 14336, (9, 256), ()),
+    (1024, 11008, (9, 128), ())])
 def test_inner_sizes_in_multiples_of_512(N, K, ahead, behind):
     _sides(N, K, False, ahead, behind)
 
