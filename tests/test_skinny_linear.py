@@ -335,3 +335,12 @@ def test_norm_in_the_packed_product(M, N, K):
         assert torch.equal(x, x0) and torch.equal(r, r0)
     assert ops.w4a16_norm_swiglu(x.repeat(3, 1), r.repeat(3, 1), g, 1e-5,
                                  *packed, 128) is None
+
+
+@pytest.mark.parametrize("M,N,one,launch", [
+    (1, 25152, False, True), (4, 25152, False, True), (5, 25152, False, False),
+    (32, 25152, False, False), (32, 25152, True, True), (32, 9216, False, True),
+    (33, 4096, True, False)])
+def test_pairs_that_share_a_launch(M, N, one, launch):
+    """The sides of the line on which either was measured to be faster."""
+    assert ops._pair_pays(M, N, one) == launch
