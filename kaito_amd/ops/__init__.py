@@ -379,9 +379,7 @@ def linear_pair(x: torch.Tensor, w: torch.Tensor, x2: torch.Tensor,
     (us, two launches and one, 32 rows, K of 2048: 3072 and 576 rows of W 14.8, 8.3,
     3072 and 4096 of one x 16.3, 12.2, 2048 and 2048 of two 14.5, 8.8; one row
     6.9, 4.9, 9.4, 6.7 and 7.2, 5.1)."""
-    one = x.data_ptr() == x2.data_ptr() and x.stride() == x2.stride()
-    if x.dim() == x2.dim() == 2 and x.size(0) == x2.size(0) \
-            and _pair_pays(x.size(0), w.size(0) + w2.size(0), one) \
+    if x.size(0) == x2.size(0) <= 32 and x.dim() == x2.dim() == 2 \
             and w.size(1) == w2.size(1) and x.device == x2.device \
             and w.size(0) % 16 == w2.size(0) % 16 == 0 \
             and _skinny(x, w) and _skinny(x2, w2) and all(
@@ -390,7 +388,10 @@ def linear_pair(x: torch.Tensor, w: torch.Tensor, x2: torch.Tensor,
                               and b.device == v.device
                               and not (torch.is_grad_enabled()
                                        and b.requires_grad))
-                for b, v in ((bias, w), (bias2, w2))):
+                for b, v in ((bias, w), (bias2, w2))) \
+            and _pair_pays(x.size(0), w.size(0) + w2.size(0),
+                           x.data_ptr() == x2.data_ptr()
+                           and x.stride() == x2.stride()):
         out, out2 = (torch.empty(x.size(0), v.size(0), dtype=x.dtype,
                                  device=x.device) for v in (w, w2))
         _K.skinny_linear_pair(out, x, w, _none(bias, x), out2, x2, w2,
@@ -404,7 +405,7 @@ def _pair_pays(M: int, N: int, one: bool) -> bool:
     and more than 4 rows, the many tiles of wide products are better alone (K of
     2048, one launch as a share of two, 24576 and 576 rows of W at 16 and 32 rows
     1.02 and 1.20, with one x 0.84 and 0.81; 8192 and 1024 at 32 0.89)."""
-    return M <= 32 and (one or M <= 4 or N < 16384)
+    return one or M <= 4 or N < 16384
 
 
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
