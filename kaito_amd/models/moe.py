@@ -292,11 +292,10 @@ class MoEMLP(nn.Module):
     # summed per token by moe_combine; static shapes, no host read.
     def _shared_fits(self, T: int) -> bool:
         """Whether the shared expert runs as one more of the routed ones: of
-        their sizes, on few tokens (32 rows, 8 experts of 2048 x 2048, top 2,
-        us: up 25.4 and down 14.5 behind 15.4 for products of its own, 30.0 and
-        17.2 with it; 4 rows 19.4, 14.0 and 10.7, 23.7 and 13.5)."""
+        their sizes, on few tokens."""
         w = self.w_shared_gate_up
-        if w is None or T > 32:
+        if w is None or not ops.moe_shared_pays(
+                T, T * self.top_k, self.num_experts, w.size(1), w.size(0) // 2):
             return False
         d = self.w_shared_down
         return self.gated \

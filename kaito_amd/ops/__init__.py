@@ -850,6 +850,25 @@ def moe_pairs_pay(pairs: int, n_local: int, up_rows: int, H: int) -> bool:
         pairs >= (n_local // 2 if H == 2048 else 2 * n_local)
 
 
+def moe_shared_pays(T: int, pairs: int, n_experts: int, H: int,
+                    I: int) -> bool:
+    """Whether an expert of every token, of the routed ones' sizes H x I, runs in
+    their launches (us, products of its own and beside, up and down together; 8
+    of 2048 x 2048, top 2: 44.9, 39.2 at 4 tokens, 54.7, 46.9 at 32; 16 of 1024 x
+    512, top 4, 1.05 to 1.41 times as fast, 8 of 7168 x 2048, top 8, 1.03 to 1.07,
+    8 of 4096 x 4096, top 2, 1.05 at 8 to 16). Its rows beyond 16 are a second pass
+    over its weights unless the others have two tiles of rows too (more than 12
+    pairs an expert), which wide or few experts do not win back: 8 of 4096 x 4096
+    0.93 to 0.96 at 17 to 32, 4 of 4096 x 8192, top 1, 0.84 to 0.88, 16 of 5120 x
+    1536, top 6, 0.95 at 32, 4 of 2048 x 2048 0.85 at 24 and 1.01 at 32; 6 of 2880
+    x 2880 1.09 to 1.13. One token of very large ones: 4 of 2048 x 8192 61.8,
+    65.4, 8 of 2048 x 4096 40.5, 37.6."""
+    if T > 16:
+        return T <= 32 and (pairs > 12 * n_experts
+                            or (H < 3072 and n_experts > 4))
+    return T > 1 or I <= 4096
+
+
 def moe_up_pairs(act, x, w_gate_up, topi, n_experts: int, e_base: int,
                  n_local_experts: int, bias=None, act_mode: int = 0,
                  act_limit: float = 7.0, all_w=None, all_act=None) -> None:

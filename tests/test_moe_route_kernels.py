@@ -309,3 +309,20 @@ def test_expert_of_every_token(T, E, H, I, top):
     rms = ref.square().mean().sqrt()
     assert ((ay.double() - ref).abs()
             <= 2.0 ** -8 * ref.abs() + 2.0 ** -12 * rms).all()
+
+
+@pytest.mark.parametrize("E,H,I,top,beside,alone", [
+    (8, 2048, 2048, 2, (1, 4, 16, 17, 32), (33,)),
+    (4, 2048, 2048, 2, (1, 16, 25, 32), (17, 24)),
+    (8, 4096, 4096, 2, (8, 16), (17, 24, 32)),
+    (4, 4096, 8192, 1, (2, 16), (17, 32)),
+    (16, 5120, 1536, 6, (6, 16), (17, 24, 32)),
+    (8, 3584, 2560, 2, (8, 16), (17, 32)), (8, 7168, 2048, 8, (2, 17, 32), ()),
+    (6, 2880, 2880, 2, (1, 17, 32), ()), (1, 2048, 2048, 1, (1, 17, 32), ()),
+    (4, 2048, 8192, 2, (2, 16), (1,)), (8, 2048, 4096, 2, (1, 32), ())])
+def test_which_shared_experts_join(E, H, I, top, beside, alone):
+    """The sides of the line on which either was measured to be faster."""
+    for T in beside:
+        assert ops.moe_shared_pays(T, T * top, E, H, I), T
+    for T in alone:
+        assert not ops.moe_shared_pays(T, T * top, E, H, I), T
