@@ -224,3 +224,26 @@ def test_rotated_on_the_way(G, KH, D, fp8, lens, max_blocks, window):
     for x, y in zip(a, b):
         assert torch.equal(x, y)
     assert torch.isfinite(out).all() and torch.equal(out, ref)
+
+
+@pytest.mark.gpu
+def test_rotations_at_any_address():
+    """A table that does not start on 16 bytes takes the two launches."""
+    D, KH, G = 64, 2, 2
+    table = torch.randn(32 * D + 1, device=DEV)
+    caches = [torch.randn(3, KH, 16, D, device=DEV).bfloat16() for _ in "kv"]
+    qkv = torch.randn(2, (G + 2) * KH * D, device=DEV).bfloat16()
+    pos = torch.tensor([3, 17], device=DEV)
+    slots = torch.tensor([16 + 3, 32 + 1], device=DEV)
+    bt = torch.tensor([[1, 0], [0, 2]], dtype=torch.int32, device=DEV)
+    sl = torch.tensor([4, 18], dtype=torch.int32, device=DEV)
+    outs = []
+    for odd in (False, True):
+        cs = table[1:].view(32, D)
+        assert cs.data_ptr() % 16
+        cs = cs if odd else cs.clone()
+        q, k, v = qkv.clone().split([G * KH * D, KH * D, KH * D], -1)
+        outs.append(ops.rope_paged_attention(
+            pos, q, k, v, D, cs, *(c.clone() for c in caches), slots, bt, sl,
+            D ** -0.5))
+    assert torch.equal(*outs)
