@@ -92,7 +92,8 @@ def test_gate_projection(device):
 
 @pytest.mark.gpu
 def test_packed_gate_projection():
-    eng = _engine("cuda", "tiny-llama-test")
+    eng = _engine("cuda", "tiny-llama-test", hidden_size=1024,
+                  intermediate_size=1024)
     for l in eng.runner.model.layers:
         l.mlp.gate_up_proj.quantize_(128)
     _check_watched(eng, [l.mlp.gate_up_proj for l in eng.runner.model.layers])
