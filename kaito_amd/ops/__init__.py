@@ -233,8 +233,8 @@ def _batched(x: torch.Tensor, w: torch.Tensor, glu: bool = False) -> bool:
 
     Both sides in us (split, library; weights out of the caches). The split
     of K is what the library does not always find: ahead from K of 10240 on
-    (4096 x 14336: 25.4, 26.4 at 16 rows, 27.4, 34.9 at 48, 36.9, 49.4 at 128,
-    45.5, 59.1 at 256; 7168 x 18432 at 256 89, 208), to 16384 rows of W
+    (4096 x 14336: 24.3, 26.4 at 16 rows, 27.4, 34.9 at 48, 38.5, 49.4 at 128,
+    47.3, 59.1 at 256; 7168 x 18432 at 256 88, 208), to 16384 rows of W
     (beyond, W is cut often enough without: 28672 x 14336 at 128 1 % behind).
     Fewer than 2048 rows of W with K below 13824 only to 64 rows (1024 x 10240
     15.1, 16.0 at 64, 17.2, 15.6 at 96, 26.3, 22.2 at 256, and 13.5, 11.5 at 16,

@@ -18,9 +18,9 @@
 // nothing.
 //
 // One MI355X, weights out of the caches, us, hipBLASLt and here (sums included):
-// 4096 x 14336: 33 rows 33.3 and 26.1, 64 36.2 and 29.4, 128 49.4 and 36.8, 256 59.1
-// and 45.5; 7168 x 18432 at 256 208 and 89; 28672 x 4096 as a pair: 64 60.2 and 49,
-// 256 79.8 and 75; 4096 x 4096 at 64 15.3 and 14.3, at 256 20.7 and 26. At 256 rows
+// 4096 x 14336: 33 rows 33.3 and 26.7, 64 36.2 and 30.0, 128 49.4 and 38.5, 256 59.1
+// and 47.3; 7168 x 18432 at 256 208 and 88; 28672 x 4096 as a pair: 64 60.2 and 49,
+// 256 79.8 and 75; 4096 x 4096 at 64 14.2 and 15.0, at 256 20.7 and 26. At 256 rows
 // of 28672 x 4096 the matrix cores' 41 us (1.45 PFLOP/s), 43 us of HBM and 52 of
 // staging do not overlap fully.
 #include "skinny.h"
@@ -271,10 +271,13 @@ struct Plan {
 
 // The plan with the least time by what was measured: staging at 52 B/ns per CU (one
 // workgroup each), W at 5.5 TB/s over the chip, the two overlapping in part, 4 us
-// per round of workgroups and for the second launch, whose sums move at 4 TB/s. Its
-// choice is within 8 % of the best of cols 64 and 128 with 1 to 8 splits (4096 x
-// 14336: 128 x 8 at 256 rows, 46 us where 64 x 4 takes 53; 64 x 4 at 64 rows, 29).
-
+// per round of workgroups, 3 for the second launch, whose sums move at 4 TB/s. Up to
+// 32 rows count as 32 also where the tile holds 64: rows past the last are one
+// line's reads (with 64 of them 4096 x 2880 at 17 rows would take 128 x 8, 12.1 us
+// where 64 x 4 takes 10.8). Against the best of cols 64 and 128 with 1 to 16 splits,
+// 22 sizes of 9 to 256 rows: within 8 % but for 65 rows, which count as 128 (to
+// 25 %), 2048 x 11008 below 17 rows (17 %) and 8192 x 2880 and 8192 x 7232 at 17 (29
+// and 10 %). 4096 x 14336: 128 x 8 at 64 rows 30.0 us, 64 x 4 28.7; at 256 rows 47.3.
 Plan plan_for(int64_t M, int64_t N, int64_t K, bool glu) {
   const int64_t steps = K / 64;
   Plan best{64, 1};

@@ -256,8 +256,9 @@ def test_swiglu_of_every_gate():
     (16, 48, 64), (48, 16, 256), (320, 48, 2048), (5136, 16, 2048),
     (16, 5136, 2048), (6144, 6160, 4096), (112, 80, 1792)])
 def test_pairs(M, N, N2, K):
-    """Two products in one launch: the bits of two launches of a kernel, f32
-    sums of either kernel where the pair has tiles enough to stay."""
+    """Two products in one launch: the bits of two launches where all three run
+    on one kernel (workgroups that stay have sums in another order, and large
+    weights of 3 and 4 rows take tiles)."""
     g = torch.Generator(device=DEV).manual_seed(M * N + K)
     big = torch.randn(M, K + 16, device=DEV, generator=g).to(torch.bfloat16)
     x, x2 = big[:, 8:8 + K], big[:, 16:16 + K]
@@ -265,14 +266,31 @@ def test_pairs(M, N, N2, K):
              for n in (N, N2))
     b, b2 = (torch.randn(n, device=DEV, generator=g).to(torch.bfloat16)
              for n in (N, N2))
+
+    def kernel(n, one=True):
+        if M <= 4:
+            return "tiles" if M > 2 and n * K > 1 << 25 else "rows"
+        stay = n // 16 >= (320 if M > 16 else 768) and (
+            K == 2048 or (K == 4096 and M <= 16))
+        return "staying" if stay and one else "tiles"
+
+    def new():
+        return [torch.full((M, n), float("nan"), dtype=torch.bfloat16,
+                           device=DEV) for n in (N, N2)]
     for y in (x, x2):
-        out = [torch.full((M, n), float("nan"), dtype=torch.bfloat16,
-                          device=DEV) for n in (N, N2)]
         if M <= 16 or K == 2048 or N * K <= 3072 * 2048:
-            _close(ops.linear_pair(x, w, y, w2)[1], y.double() @ w2.double().T)
+            got = ops.linear_pair(x, w, y, w2)
+            _close(got[0], x.double() @ w.double().T)
+            _close(got[1], y.double() @ w2.double().T)
+        out, two = new(), new()
         ops._K.skinny_linear_pair(out[0], x, w, b, out[1], y, w2, b2)
         _close(out[0], x.double() @ w.double().T + b.double())
         _close(out[1], y.double() @ w2.double().T + b2.double())
+        ops._K.skinny_linear(two[0], x, w, b)
+        ops._K.skinny_linear(two[1], y, w2, b2)
+        for o, t, n in zip(out, two, (N, N2)):
+            if kernel(N + N2, y is x) == kernel(n):
+                assert torch.equal(o, t)
 
 
 @pytest.mark.gpu
