@@ -20,11 +20,11 @@ from ..engine import lora as lora_mod
 def untouched(module: nn.Module, cls: type) -> bool:
     """Whether a call of `module` is cls.forward and nothing else: no hooks, no
     forward of its own in its place. Only then may a layer call its parts."""
-    return type(module).forward is cls.forward \
-        and "forward" not in vars(module) \
-        and not (module._forward_hooks or module._forward_pre_hooks
-                 or _module._global_forward_hooks
-                 or _module._global_forward_pre_hooks)
+    own = module.__dict__
+    return not (own["_forward_hooks"] or own["_forward_pre_hooks"]
+                or _module._global_forward_hooks
+                or _module._global_forward_pre_hooks or "forward" in own) \
+        and type(module).forward is cls.forward
 
 
 class _QuantMixin:
