@@ -20,11 +20,13 @@
 // ahead and the loads go out a few at a time. The bound is the way from the
 // caches to LDS: without the products the loads alone take nine tenths of the
 // time, without the loads the rest takes four fifths. At 8 of 28672 x 4096 the matrix
-// cores are busy 67 % of it and waves wait a quarter of theirs, for loads at the
-// barrier; a library product of that width, 84 % busy, has the same hit rate in L2
-// (79 %), bytes per operation and clock (1.5 GHz). (K steps of 32 in four or
-// five buffers, whose rows are half lines: a tenth slower; waves of a SIMD taking
-// turns behind barriers, other starts in K per tile: no change.)
+// cores are busy 72 % of it and waves wait a quarter of theirs, for loads at the
+// barrier; a library product of that width, 83 % busy, has the same hit rate in L2
+// (79 %), bytes per operation and clock (1.57 GHz), but two thirds of the LDS reads
+// per operation: 128 x 64 outputs per wave read 6 fragments for 8 products, 128 x
+// 128 read 8 for 16. (K steps of 32 in four or five buffers, whose rows are half
+// lines: a tenth slower; waves of a SIMD taking turns behind barriers, other starts
+// in K per tile: no change.)
 //
 // Tiles are numbered expert by expert, in blocks of 4 column tiles x all row
 // tiles, and every XCD takes one contiguous eighth of them: the 32 tiles in
@@ -32,9 +34,9 @@
 // an XCD's 32 CUs is cut in quarters, 128 x 128, one per CU; so is a small step's
 // only round of up to 16. Measured on one MI355X, 8 experts of 2048 x 2048, top
 // 2, rows as drawn from 16 kinds of tokens, us, two buffers and whole tiles, now:
-// 8192 tokens 317 and 278, with the epilogue of today 254 (1080 TFLOP/s), down 165 and
-// 139; 4096 174 and 149, 106
-// and 86; 2048 114 and 90; 1000 down 60 and 49. 8 of 4096 x 14336, 8192 tokens:
+// 8192 tokens 317 and 278, with the epilogue of today 254 (1080 TFLOP/s), down 165
+// and 139; 4096 174 and 149, 106 and 86; 2048 114 and 90; 1000 down 60 and 49. 8 of
+// 4096 x 14336, 8192 tokens:
 // 3419 and 3262 (1180 TFLOP/s), 1875 and 1676. 8-byte stores cost a tenth more. A
 // library GEMM per expert with its gathers, casts and index_add took 958 us behind
 // a host read at the first of these.
