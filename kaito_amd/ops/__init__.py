@@ -320,13 +320,18 @@ def _batched_shape(M: int, N: int, K: int, glu: bool) -> bool:
     return N <= 65536 and 5120 <= K < 8192 and M <= 32
 
 
+def _plain_bias(bias, w: torch.Tensor) -> bool:
+    """None, or one that the kernels of small linear layers add."""
+    return bias is None or (
+        bias.dtype == torch.bfloat16 and bias.is_contiguous()
+        and bias.shape == w.shape[:1] and bias.device == w.device
+        and not (torch.is_grad_enabled() and bias.requires_grad))
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
     """x W^T (+ bias): the weight-streaming kernels for small decode steps, the
     split kernel for larger ones where it is ahead, hipBLASLt otherwise."""
-    if bias is None or (
-            bias.dtype == torch.bfloat16 and bias.is_contiguous()
-            and bias.shape == w.shape[:1] and bias.device == w.device
-            and not (torch.is_grad_enabled() and bias.requires_grad)):
+    if _plain_bias(bias, w):
         skinny = _skinny(x, w)
         if skinny or _batched(x, w):
             out = torch.empty(x.size(0), w.size(0), dtype=x.dtype,
@@ -382,13 +387,8 @@ def linear_pair(x: torch.Tensor, w: torch.Tensor, x2: torch.Tensor,
     if x.size(0) == x2.size(0) <= 32 and x.dim() == x2.dim() == 2 \
             and w.size(1) == w2.size(1) and x.device == x2.device \
             and w.size(0) % 16 == w2.size(0) % 16 == 0 \
-            and _skinny(x, w) and _skinny(x2, w2) and all(
-                b is None or (b.dtype == torch.bfloat16 and b.is_contiguous()
-                              and b.shape == v.shape[:1]
-                              and b.device == v.device
-                              and not (torch.is_grad_enabled()
-                                       and b.requires_grad))
-                for b, v in ((bias, w), (bias2, w2))) \
+            and _skinny(x, w) and _skinny(x2, w2) \
+            and _plain_bias(bias, w) and _plain_bias(bias2, w2) \
             and _pair_pays(x.size(0), w.size(0) + w2.size(0),
                            x.data_ptr() == x2.data_ptr()
                            and x.stride() == x2.stride()):
@@ -430,11 +430,7 @@ def add_norm_linear(x: torch.Tensor, residual: torch.Tensor,
     rows, always ahead there (us, two launches and one: 11.9, 10.5 at one row of
     6144 x 4096, 13.6, 11.4 at two); more rows cost every workgroup more than a
     launch is worth."""
-    if norm_fits(x, residual, norm, w) and (
-            bias is None or (bias.dtype == torch.bfloat16
-                             and bias.is_contiguous()
-                             and bias.shape == w.shape[:1]
-                             and bias.device == w.device)):
+    if norm_fits(x, residual, norm, w) and _plain_bias(bias, w):
         out = torch.empty(x.size(0), w.size(0) // (2 if glu else 1),
                           dtype=x.dtype, device=x.device)
         stream = torch.empty_like(x)

@@ -335,6 +335,21 @@ def test_norm_beside_the_product():
 
 
 @pytest.mark.gpu
+def test_bias_that_is_trained_beside_the_norm():
+    """Its gradient is the sum of the product's, as behind the norm's launch."""
+    x, r = (torch.randn(2, 512, device=DEV).bfloat16() for _ in "xr")
+    g, w = (torch.randn(*s, device=DEV).bfloat16() for s in ((512,), (16, 512)))
+    b = torch.randn(16, device=DEV).bfloat16()
+    normed, _ = ops.fused_add_rms_norm(x, r.clone(), g, 1e-5)
+    want = normed.double() @ w.double().T + b.double()
+    b.requires_grad_()
+    out, _ = ops.add_norm_linear(x, r.clone(), g, 1e-5, w, b)
+    _close(out.detach(), want)
+    out.sum().backward()
+    assert torch.equal(b.grad, torch.full_like(b, 2.0))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(1, 16, 512), (2, 32, 2560), (2, 4112, 4096),
                                    (1, 5616, 5120), (2, 48, 8192)])
 def test_norm_in_the_packed_product(M, N, K):
