@@ -32,18 +32,14 @@ struct Parts {
 
 // GLU: the wave's two rows are a gate row and its up row (N apart)
 template <int M, int R, bool GLU>
-__global__ __launch_bounds__(NW * 64) void skinny_linear_kernel(const Parts a) {
-  const int second = (int)blockIdx.x >= a.first;
-  const Part p = second ? a.part[1] : a.part[0];
-  short* __restrict__ out = p.out;
-  const short* __restrict__ x = p.x;
-  const short* __restrict__ w = p.w;
-  const short* __restrict__ bias = p.bias;
-  const int64_t x_stride = p.x_stride;
-  const int N = p.N, K = a.K;
+KAITO_DEV void linear_rows(short* __restrict__ out,
+                           const short* __restrict__ x, const int64_t x_stride,
+                           const short* __restrict__ w,
+                           const short* __restrict__ bias, const int N,
+                           const int K, const int block) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n0 = ((blockIdx.x - second * a.first) * NW + wave) * (GLU ? 1 : R);
+  const int n0 = (block * NW + wave) * (GLU ? 1 : R);
   if (n0 >= N) return;
   const short* wp[R];
   float acc[M][R];
@@ -70,6 +66,26 @@ __global__ __launch_bounds__(NW * 64) void skinny_linear_kernel(const Parts a) {
               acc[m][r] + (bias ? bf16_to_f32(bias[n0 + r]) : 0.f));
     }
   }
+}
+
+// A product alone has a kernel of its own: chosen from two by the workgroup it took
+// (us) 4.9 where it takes 4.6 (576 x 8192, one row), 15.9 and 14.9 (4096 x 8192, four),
+// 6.3 and 6.0 (28672 x 64).
+template <int M, int R, bool GLU>
+__global__ __launch_bounds__(NW * 64) void skinny_linear_kernel(
+    short* __restrict__ out, const short* __restrict__ x,
+    const int64_t x_stride, const short* __restrict__ w,
+    const short* __restrict__ bias, const int, const int N, const int K) {
+  linear_rows<M, R, GLU>(out, x, x_stride, w, bias, N, K, blockIdx.x);
+}
+
+template <int M, int R>
+__global__ __launch_bounds__(NW * 64) void skinny_linear_pair_kernel(
+    const Parts a) {
+  const int second = (int)blockIdx.x >= a.first;
+  const Part p = second ? a.part[1] : a.part[0];
+  linear_rows<M, R, false>(p.out, p.x, p.x_stride, p.w, p.bias, p.N, a.K,
+                           blockIdx.x - second * a.first);
 }
 
 // The products of rms(x + residual) * g, with the sum left for later layers. Each
@@ -219,21 +235,17 @@ __global__ __launch_bounds__(NW * 64) void skinny_norm_kernel(
 // M <= 16 MT rows; N is a multiple of 16 (GLU: of 8, the workgroup's 16 rows
 // are 8 gate rows and their up rows, N apart), K of the stage
 template <int MT, int KS, bool GLU>
-__global__ __launch_bounds__(256, 2) void skinny_tile_kernel(const Parts a) {
-  const int second = (int)blockIdx.x >= a.first;
-  const Part p = second ? a.part[1] : a.part[0];
-  short* __restrict__ out = p.out;
-  const short* __restrict__ x = p.x;
-  const short* __restrict__ w = p.w;
-  const short* __restrict__ bias = p.bias;
-  const int64_t x_stride = p.x_stride;
-  const int M = a.M, N = p.N, K = a.K;
+KAITO_DEV void linear_tile(short* __restrict__ out,
+                           const short* __restrict__ x, const int64_t x_stride,
+                           const short* __restrict__ w,
+                           const short* __restrict__ bias, const int M,
+                           const int N, const int K, const int block) {
   constexpr int NI = skinny::tile_loads<KS>();
   __shared__ __attribute__((aligned(128))) short ring[4][2][16 * KS];
   static_assert(sizeof(ring) >= 4 * MT * 64 * sizeof(f32x4), "fold");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n0 = (blockIdx.x - second * a.first) * (GLU ? 8 : 16);
+  const int n0 = block * (GLU ? 8 : 16);
   const short *src[NI], *xp[MT];
 #pragma unroll
   for (int j = 0; j < NI; j++) {
@@ -271,6 +283,23 @@ __global__ __launch_bounds__(256, 2) void skinny_tile_kernel(const Parts a) {
     const int m = (slot >> 6) * 16 + (l >> 4) * 4 + r;
     if (m < M) out[(int64_t)m * N + n0 + c] = f32_to_bf16(v[r]);
   }
+}
+
+template <int MT, int KS, bool GLU>
+__global__ __launch_bounds__(256, 2) void skinny_tile_kernel(
+    short* __restrict__ out, const short* __restrict__ x,
+    const int64_t x_stride, const short* __restrict__ w,
+    const short* __restrict__ bias, const int M, const int N, const int K) {
+  linear_tile<MT, KS, GLU>(out, x, x_stride, w, bias, M, N, K, blockIdx.x);
+}
+
+template <int MT, int KS>
+__global__ __launch_bounds__(256, 2) void skinny_tile_pair_kernel(
+    const Parts a) {
+  const int second = (int)blockIdx.x >= a.first;
+  const Part p = second ? a.part[1] : a.part[0];
+  linear_tile<MT, KS, false>(p.out, p.x, p.x_stride, p.w, p.bias, a.M, p.N,
+                             a.K, blockIdx.x - second * a.first);
 }
 
 // K = 1024 S: see skinny::stream_tiles. gridDim.x workgroups share the tiles of
@@ -369,10 +398,21 @@ void check(const at::Tensor& out, const at::Tensor& x, const at::Tensor& w,
               "more than 4 rows: K in whole stages, N in whole tiles");
 }
 
+template <int V> using Int = std::integral_constant<int, V>;
+
 template <typename Kernel>
 void launch(Kernel kernel, int64_t workgroups, const Parts& a) {
   hipLaunchKernelGGL(kernel, dim3(workgroups),
                      dim3(256), 0, at::hip::getCurrentHIPStream(), a);
+}
+
+// a product alone
+template <typename Kernel>
+void launch_one(Kernel kernel, int64_t workgroups, const Parts& a) {
+  const Part& p = a.part[0];
+  hipLaunchKernelGGL(kernel, dim3(workgroups), dim3(256), 0,
+                     at::hip::getCurrentHIPStream(), p.out, p.x, p.x_stride,
+                     p.w, p.bias, a.M, p.N, a.K);
 }
 
 // `cols` output columns of a tile or, GLU, half of its 16 rows of W
@@ -396,12 +436,21 @@ void run(Parts a, bool shared_x) {
       };
       if (GLU || N1 == 0) stay(std::false_type{});
       else stay(std::bool_constant<!GLU>{});
-    } else if (K % 256 == 0) {
-      if (M > 16) launch(&skinny_tile_kernel<2, 256, GLU>, N / cols, a);
-      else launch(&skinny_tile_kernel<1, 256, GLU>, N / cols, a);
+      return;
+    }
+    auto tile = [&](auto mt, auto ks) {
+      constexpr int MT = decltype(mt)::value, KS = decltype(ks)::value;
+      if constexpr (!GLU)
+        if (N1 > 0)
+          return launch(&skinny_tile_pair_kernel<MT, KS>, N / cols, a);
+      launch_one(&skinny_tile_kernel<MT, KS, GLU>, N / cols, a);
+    };
+    if (M > 16) {
+      if (K % 256 == 0) tile(Int<2>{}, Int<256>{});
+      else tile(Int<2>{}, Int<64>{});
     } else {
-      if (M > 16) launch(&skinny_tile_kernel<2, 64, GLU>, N / cols, a);
-      else launch(&skinny_tile_kernel<1, 64, GLU>, N / cols, a);
+      if (K % 256 == 0) tile(Int<1>{}, Int<256>{});
+      else tile(Int<1>{}, Int<64>{});
     }
     return;
   }
@@ -410,12 +459,19 @@ void run(Parts a, bool shared_x) {
   // the x loads (M = 4, N = 28672: 48 us)
   const int64_t per = NW * (GLU || M == 1 ? 1 : 2);
   a.first = (int)((N0 + per - 1) / per);
-  const int64_t grid = a.first + (N1 + per - 1) / per;
+  auto rows = [&](auto m, auto r) {
+    constexpr int MM = decltype(m)::value, R = decltype(r)::value;
+    if constexpr (!GLU)
+      if (N1 > 0)
+        return launch(&skinny_linear_pair_kernel<MM, R>,
+                      a.first + (N1 + per - 1) / per, a);
+    launch_one(&skinny_linear_kernel<MM, R, GLU>, a.first, a);
+  };
   switch (M) {
-    case 1: launch(&skinny_linear_kernel<1, GLU ? 2 : 1, GLU>, grid, a); break;
-    case 2: launch(&skinny_linear_kernel<2, 2, GLU>, grid, a); break;
-    case 3: launch(&skinny_linear_kernel<3, 2, GLU>, grid, a); break;
-    default: launch(&skinny_linear_kernel<4, 2, GLU>, grid, a); break;
+    case 1: rows(Int<1>{}, Int<GLU ? 2 : 1>{}); break;
+    case 2: rows(Int<2>{}, Int<2>{}); break;
+    case 3: rows(Int<3>{}, Int<2>{}); break;
+    default: rows(Int<4>{}, Int<2>{}); break;
   }
 }
 
