@@ -280,8 +280,18 @@ KAITO_DEV void grouped_tile(const GemmArgs& a, short* lds, const int expert,
   // added where a value leaves: ahead of that, over all of acc, it cost 132 bytes
   // of scratch per lane and 55 us of 312 (up, 8 experts of 2048 x 2048, 16384
   // pairs of uneven experts, weights out of the caches; with the activations'
-  // divisions in half the instructions)
+  // divisions in half the instructions). Read once: for every 32 rows anew, a down
+  // projection of 8192 tokens by 16 experts of 1024 x 512 took 51.9 us, now 47.9
   const short* be = a.bias + (int64_t)expert * wrows + c0 + 4 * h;
+  short4_t bias[2][4] = {};
+  if (a.bias) {
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int b = 0; b < 4; b++)
+        bias[i][b] = *reinterpret_cast<const short4_t*>(
+            be + (is_gated(KIND) ? i * a.N : i * 32) + 8 * b);
+  }
   // bf16 rows pass through the wave's part of LDS (every wave is done with
   // its tiles) and leave as 16 bytes a lane
   constexpr int PITCH = WC + 8, LANES = WC / 8;
@@ -300,15 +310,10 @@ KAITO_DEV void grouped_tile(const GemmArgs& a, short* lds, const int expert,
           if constexpr (is_gated(KIND)) u[e] = acc[1][j][b * 4 + e];
         }
         if (a.bias) {
-          const short4_t bv =
-              *reinterpret_cast<const short4_t*>(be + i * 32 + 8 * b);
 #pragma unroll
-          for (int e = 0; e < 4; e++) v[e] += bf16_to_f32(bv[e]);
-          if constexpr (is_gated(KIND)) {
-            const short4_t bu =
-                *reinterpret_cast<const short4_t*>(be + a.N + 8 * b);
-#pragma unroll
-            for (int e = 0; e < 4; e++) u[e] += bf16_to_f32(bu[e]);
+          for (int e = 0; e < 4; e++) {
+            v[e] += bf16_to_f32(bias[i][b][e]);
+            if constexpr (is_gated(KIND)) u[e] += bf16_to_f32(bias[1][b][e]);
           }
         }
 #pragma unroll
