@@ -22,7 +22,7 @@ from .. import ops
 from ..engine.config import ModelConfig
 from ..parallel.state import get_state
 from ..parallel.layers import (ColumnParallelLinear, RowParallelLinear,
-                               VocabParallelEmbedding, untouched)
+                               VocabParallelEmbedding, taken_apart, untouched)
 
 
 @dataclass
@@ -95,6 +95,7 @@ def build_cos_sin_cache(cfg: ModelConfig, device, max_pos: Optional[int] = None,
             * mscale).float().contiguous()
 
 
+@taken_apart
 class LlamaAttention(nn.Module):
     def __init__(self, cfg: ModelConfig, layer_idx: int = 0):
         super().__init__()
@@ -195,6 +196,7 @@ class LlamaAttention(nn.Module):
         return o_proj(out.reshape(T, -1))
 
 
+@taken_apart
 class LlamaMLP(nn.Module):
     def __init__(self, cfg: ModelConfig):
         super().__init__()
@@ -263,6 +265,7 @@ def _tp_fused_add_rms_norm(hidden, residual, weight, eps: float,
     return ops.fused_add_rms_norm(hidden, residual, weight, eps)
 
 
+@taken_apart
 class LlamaDecoderLayer(nn.Module):
     def __init__(self, cfg: ModelConfig, layer_idx: int = 0):
         super().__init__()

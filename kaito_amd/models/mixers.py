@@ -36,6 +36,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .. import ops
+from ..parallel.layers import taken_apart
 from .hybrid_config import (DeltaRuleSpec, DenseFFSpec, DiagDeltaSpec,
                             GLASpec, GLUSpec, HGRN2Spec, LatentAttnSpec,
                             MLSTMSpec, RGLRUSpec, RotaryAttnSpec, SSDSpec,
@@ -108,6 +109,7 @@ class GatedDeltaMixer(nn.Module):
         return ops.linear(o.reshape(T, self.n_v), self.o_proj)
 
 
+@taken_apart
 class RGLRUMixer(nn.Module):
     """Recurrent block around a real-gated linear recurrent unit: a
     GELU-activated gate branch y beside a branch u = conv(linear(x)) that
@@ -165,6 +167,7 @@ class RGLRUMixer(nn.Module):
                          meta.state_slots, meta.seq_starts, meta.token_seq)
 
 
+@taken_apart
 class BiasedWindowAttention(nn.Module):
     """Grouped-query softmax attention over the last `window` positions of
     the paged cache. No rotation: position enters through the causal

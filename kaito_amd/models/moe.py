@@ -26,7 +26,7 @@ import torch.nn as nn
 
 from .. import ops
 from ..engine.config import ModelConfig
-from ..parallel.layers import untouched
+from ..parallel.layers import taken_apart, untouched
 from ..parallel.state import get_state, tp_all_reduce
 
 
@@ -65,6 +65,7 @@ class MoERows:
                                       out_dtype)
 
 
+@taken_apart
 class MoEMLP(nn.Module):
     def __init__(self, cfg: ModelConfig):
         super().__init__()

@@ -17,14 +17,22 @@ from .state import get_state, tp_all_reduce
 from ..engine import lora as lora_mod
 
 
+def taken_apart(cls: type) -> type:
+    """A class of modules whose parts callers may call instead: keeps the forward
+    that those stand for, whatever the class is given later."""
+    cls._whole = cls.forward
+    return cls
+
+
 def untouched(module: nn.Module, cls: type) -> bool:
-    """Whether a call of `module` is cls.forward and nothing else: no hooks, no
-    forward of its own in its place. Only then may a layer call its parts."""
+    """Whether a call of `module` is the forward that `cls` was written with and
+    nothing else: no hooks, no other forward in its place. Only then may a layer
+    call its parts."""
     own = module.__dict__
     return not (own["_forward_hooks"] or own["_forward_pre_hooks"]
                 or _module._global_forward_hooks
                 or _module._global_forward_pre_hooks or "forward" in own) \
-        and type(module).forward is cls.forward
+        and type(module).forward is cls._whole
 
 
 class _QuantMixin:
@@ -76,6 +84,7 @@ class _QuantMixin:
         return y.reshape(*shape, -1).to(x.dtype)
 
 
+@taken_apart
 class ColumnParallelLinear(_QuantMixin, nn.Module):
     def __init__(self, in_features: int, out_features: int, bias: bool = False,
                  dtype: torch.dtype = torch.bfloat16):
@@ -139,6 +148,7 @@ class ColumnParallelLinear(_QuantMixin, nn.Module):
         return lora_mod.maybe_apply(self, x, out)
 
 
+@taken_apart
 class RowParallelLinear(_QuantMixin, nn.Module):
     # set True by the model builder on linears whose output feeds a
     # fused allreduce+RMSNorm call site (attention o_proj, MLP

@@ -62,20 +62,48 @@ def test_mixers_of_a_hybrid_layer(device):
     _check_watched(eng, [m for l in layers for m in (l.attn, l.rglru)])
 
 
+@pytest.mark.parametrize("of", ["module", "class"])
 @pytest.mark.parametrize("device", DEVICES)
-def test_replaced_forward_of_a_mixer(device):
-    """What wraps a module by giving it a forward of its own is not passed by."""
+def test_replaced_forward_of_a_mixer(device, of, monkeypatch):
+    """What wraps a module by giving it, or all of its class, a forward of its own
+    is not passed by."""
     eng = _engine(device, "tiny-gurapel-test")
     layer = next(l for l in eng.runner.model.layers
                  if l.spec.kind == "parallel")
-    plain, calls = layer.rglru.forward, []
+    where = layer.rglru if of == "module" else type(layer.rglru)
+    plain, calls = where.forward, []
 
     def forward(*args):
-        calls.append(args[0].size(0))
+        if of == "module" or args[0] is layer.rglru:
+            calls.append(args[-4].size(0))
         return plain(*args)
-    layer.rglru.forward = forward
+    monkeypatch.setattr(where, "forward", forward)
     _generate(eng)
     assert calls == [22, 1, 1, 1]
+
+
+@pytest.mark.parametrize("name,part", [
+    ("LlamaAttention", "self_attn"), ("LlamaMLP", "mlp"),
+    ("RowParallelLinear", "mlp.down_proj")])
+def test_replaced_forward_of_a_class(name, part, monkeypatch):
+    """Nor in a decoder layer, and it is called as it was: without `defer`."""
+    eng = _engine("cpu", "tiny-llama-test")
+    want = _generate(eng)
+    monkeypatch.setattr(ops, "linear_parts", _in_parts)
+    mine = [l.get_submodule(part) for l in eng.runner.model.layers]
+    cls, calls = type(mine[0]), []
+    assert cls.__name__ == name
+    plain = cls.forward
+
+    def forward(self, *args):
+        if self in mine:
+            calls.append(self)
+        out = plain(self, *args)
+        assert isinstance(out, torch.Tensor)
+        return out
+    monkeypatch.setattr(cls, "forward", forward)
+    assert _generate(eng) == want
+    assert len(calls) == 4 * len(mine)
 
 
 @pytest.mark.parametrize("device", DEVICES)
