@@ -24,8 +24,8 @@
 // K and V tiles go to LDS by 16-byte global_load_lds, one tile ahead of the
 // one in use (two buffers, one barrier per tile). The swizzles are applied
 // to the global side of the copy: 16-byte chunk c of K row r sits at
-// c ^ (r & 7), so that the eight rows of a quarter-wave's ds_read_b128 touch
-// all banks; V rows move by 32-byte pairs for the transposing reads.
+// c ^ (r & 15) (D = 128), so that the sixteen rows of a quarter of a ds_read_b128
+// touch all banks; V rows move by 64 bytes for the transposing reads.
 //
 // What bounds it: per 64 keys a wave runs 32 MFMA (1024 cycles at D = 128)
 // beside about 900 cycles of softmax VALU work and a 32 KB LDS read, so two
@@ -87,19 +87,27 @@ struct Args {
   int temp_every;
 };
 
-// chunk of a K row -> its place, free of bank conflicts for 8 rows at once
+// LDS serves 256 bytes per cycle, 16 lanes of a 16-byte read, 32 of an 8-byte
+// one: as many rows have to lie in different sixteenths (eighths) of 256 bytes.
+// Places that do so for 8 rows only take twice as long (1 KB reads by four waves
+// at once: 32 and 16 cycles each, 512 transposed bytes 16 and 10.5). One prompt of
+// 8192, 32/8 heads of 128: 593 -> 584 us; 4 x 2048, 16/4 heads, window 1024: 91 ->
+// 87; with pages 1157 -> 1139 (3627 rows over 20011 keys).
+// chunk of a K row -> its place
 template <int D>
 KAITO_DEV int swz_k(int row, int c) {
-  if constexpr (D == 96) return c ^ ((row >> 1) & 3);
-  else return c ^ (row & 7);
+  if constexpr (D == 96) return c ^ ((row >> 2) & 3);
+  else if constexpr (D % 128 == 0) return c ^ (row & 15);
+  else return c ^ ((row >> 1) & 7);
 }
 
-// chunk of a V row -> its place; pairs of chunks (16 columns) stay together
+// chunk of a V row -> its place; pairs of chunks (16 columns) stay together, and
+// four where a row is 256 bytes or more: 4 rows of them are read at once
 template <int DV>
 KAITO_DEV int swz_v(int row, int c) {
   if constexpr (DV == 32 || DV == 96) return c ^ (((row >> 1) & 1) << 1);
   else if constexpr (DV == 64) return c ^ ((row & 3) << 1);
-  else return c ^ ((row & 7) << 1);
+  else return c ^ ((row & 3) << 2);
 }
 
 KAITO_DEV void lds_copy16(const short* src, short* dst) {
@@ -308,7 +316,7 @@ void flash_prefill_kernel(const Args a) {
   constexpr bool SPLIT_K = !PAGED && D1 < D;
   constexpr int PERIOD = SPLIT_K ? 3 : 1, AHEAD = PERIOD * NT / CK;
   static_assert(!SPLIT_K || (LK % PERIOD == 0 && PERIOD * NT % CK == 0 &&
-                             AHEAD % 8 == 0 && KVT == LK / PERIOD * AHEAD));
+                             AHEAD % 16 == 0 && KVT == LK / PERIOD * AHEAD));
   const short* k_lane[PERIOD];
   const short* v_lane = nullptr;
   if constexpr (SPLIT_K) {
@@ -323,7 +331,7 @@ void flash_prefill_kernel(const Args a) {
     }
     v_lane = (const short*)a.v + (tok + tid / CV) * a.v_ts + kvh * a.v_hs +
         swz_v<DV>(tid / CV, tid % CV) * 8;
-    static_assert(NT / CV % 8 == 0);
+    static_assert(NT / CV % 4 == 0);
   }
   auto stage = [&](const int kv0, short* buf) {
     if constexpr (PAGED) {

@@ -125,7 +125,7 @@ KAITO_DEV void grouped_tile(const GemmArgs& a, short* lds, const int expert,
   const auto wr = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<short*>(we), 0, 0xffffffff, 0x27000);
   constexpr int CH = BK / 8;        // 16-byte chunks of a row
-  auto place = [](const int row, const int c) { return c ^ (row & 7); };
+  auto place = [](const int row, const int c) { return c ^ (row >> 1 & 7); };
   uint32_t xs[LX], ws[LW];
   int src[LX];                      // one wait for all of them
 #pragma unroll

@@ -94,6 +94,14 @@ struct DecodeArgs {
   }
 };
 
+// chunk of a V row -> its place: 8 rows x 16 columns, which half a wave's
+// transposing read takes at once, lie in different eighths of 256 bytes
+template <int D>
+KAITO_DEV int place_v(const int row, const int c) {
+  if constexpr (D == 64) return c ^ ((row >> 1 & 3) << 1);
+  else return c ^ ((row & 7) << 1);
+}
+
 KAITO_DEV hbf16x8 widen8(const u8x8_t raw) {
   float f[8];
   fp8x8_to_f32(raw, f);
@@ -315,7 +323,7 @@ void paged_decode_kernel(const DecodeArgs a) {
         const int row = j * (64 / CV) + lane / CV;
         const int64_t at = (j * (64 / CV) < BS ? row0 : row1) * D;
         const uint32_t off =
-            row % BS * D + flash::swz_v<D>(row, lane % CV) * 8;
+            row % BS * D + place_v<D>(row, lane % CV) * 8;
         if constexpr (FP8)
           v8[j] = *reinterpret_cast<const u8x8_t*>(
               (const uint8_t*)a.v + at + off);
@@ -429,7 +437,7 @@ void paged_decode_kernel(const DecodeArgs a) {
 #pragma unroll
         for (int u = 0; u < 2; u++) {
           const short* at = vl + vrow * D +
-              flash::swz_v<D>(vrow, (dt + u) * 2 + vc) * 8 + ve;
+              place_v<D>(vrow, (dt + u) * 2 + vc) * 8 + ve;
           const short4_t a4 = flash::read_tr(at);
           const short4_t b4 = flash::read_tr(at + 16 * D);
           vf[u] = __builtin_bit_cast(
