@@ -684,8 +684,8 @@ def latent_kv(c: torch.Tensor, w_kc: torch.Tensor, w_vc: torch.Tensor):
     w_kc [H, D, r] and w_vc [H, r, V]. One launch (and a transposition of
     w_vc) for prompts that fill the chip with 256 x 256 tiles, library products
     else (us, library and tiles, 128 + 128 dims of 512: 8192 rows of 16 heads
-    59.2, 46.7, 4096 34.0, 27.4, 2048 23.2, 23.5; 4096 of 128 heads 213, 169,
-    512 33.2, 34.5)."""
+    59.2, 41.0, 4096 34.0, 27.0, 2048 23.2, 22.3; 4096 of 128 heads 213, 149,
+    512 33.2, 33.4)."""
     T, (H, D, r), V = c.size(0), w_kc.shape, w_vc.size(2)
     if c.is_cuda and _latent_tiles(T, H * (D + V), r) and T < 1 << 22 \
             and c.dtype == w_kc.dtype == w_vc.dtype == torch.bfloat16 \
@@ -705,8 +705,9 @@ def latent_kv(c: torch.Tensor, w_kc: torch.Tensor, w_vc: torch.Tensor):
 
 def _latent_tiles(T: int, N: int, r: int) -> bool:
     """More latent columns than 512 need more tiles for the library to be behind
-    (128 heads of 256 dims, 1536 columns, library over tiles: 0.87 to 0.98 from
-    512 to 3000 tokens, 0.99 at 4096, 1.03 at 6000, 1.18 at 8192)."""
+    (128 heads of 256 dims, 1536 columns, library over tiles: 1.07, 1.01, 1.01 at
+    512, 1024, 2048 tokens, 1.16 at 3000, 1.12 at 4096, 1.19 at 6000: the line is
+    where tiles of 8 waves drew level)."""
     return T * N >= 4096 * 4096 * (1 if r <= 512 else 9)
 
 

@@ -7,40 +7,19 @@
 //                     sums in the order of the choice, plus identity and
 //                     shared experts
 //
-// A workgroup of 8 waves (2 over rows x 4 over weight rows) computes BM rows
-// x 256 weight rows (up: 128 gate rows beside their 128 up rows, 32 + 32 per
-// wave, so a lane holds both of a pair) in K steps of 64 on
-// v_mfma_f32_32x32x16_bf16, transposed (C^T = W X^T: a lane owns one token row
-// and 4 neighbouring outputs at a time). Both operands arrive by 16-byte
-// loads straight to LDS (16-byte chunk c of row r at c ^ (r & 7)); as buffer
-// loads, behind which the compiler can count LDS reads (behind the global form
-// it waits for all). At BM = 256 a step is 32 MFMA per wave, 2048 cycles of a
-// SIMD's two waves, against 192 KB of LDS reads (1536 cycles) and 64 KB of
-// staging per CU: all have to overlap, so fragments are read one step of 16 dims
-// ahead and the loads go out a few at a time. The bound is the way from the
-// caches to LDS: without the products the loads alone take nine tenths of the
-// time, without the loads the rest takes four fifths. At 8 of 28672 x 4096 the matrix
-// cores are busy 72 % of it and waves wait a quarter of theirs, for loads at the
-// barrier; a library product of that width, 83 % busy, has the same hit rate in L2
-// (79 %), bytes per operation and clock (1.57 GHz), but two thirds of the LDS reads
-// per operation: 128 x 64 outputs per wave read 6 fragments for 8 products, 128 x
-// 128 read 8 for 16. (K steps of 32 in four or five buffers, whose rows are half
-// lines: a tenth slower; waves of a SIMD taking turns behind barriers, other starts
-// in K per tile: no change.)
-//
-// Tiles are numbered expert by expert, in blocks of 4 column tiles x all row
-// tiles, and every XCD takes one contiguous eighth of them: the 32 tiles in
-// flight behind one L2 share rows and weights. A last round of up to 8 tiles for
-// an XCD's 32 CUs is cut in quarters, 128 x 128, one per CU; so is a small step's
-// only round of up to 16. Measured on one MI355X, 8 experts of 2048 x 2048, top
-// 2, rows as drawn from 16 kinds of tokens, us, two buffers and whole tiles, now:
-// 8192 tokens 317 and 278, with the epilogue of today 254 (1080 TFLOP/s), down 165
-// and 139; 4096 174 and 149, 106 and 86; 2048 114 and 90; 1000 down 60 and 49. 8 of
-// 4096 x 14336, 8192 tokens:
-// 3419 and 3262 (1180 TFLOP/s), 1875 and 1676. 8-byte stores cost a tenth more. A
-// library GEMM per expert with its gathers, casts and index_add took 958 us behind
+// The products' main loop is that of tile_gemm.h; every workgroup stays and takes
+// tile after tile, of the shape that the step's rows need fewest rounds of. Measured
+// on one MI355X, us, 8 waves of 128 x 64 on 32x32x16 products with a workgroup per
+// tile, now: 8 experts of 2048 x 2048, top 2, 8192 tokens up 272 and 238 (1160
+// TFLOP/s), down 131 and 112; 4096 170 and 148, 80 and 69; 2048 93 and 82, 53 and 49;
+// 1000 56 and 53, 49 and 34; 300 33 and 30, 32 and 21; 100 31 and 24, 29 and 19. 8 of
+// 4096 x 14336, 8192 tokens: 3117 and 2736 (1400 TFLOP/s), 1631 and 1438; 128: 383
+// and 357, 297 and 185. 32 of 2048 x 1024, top 4, 2048 tokens 124 and 119, 62 and
+// 50. 64 of 1024 x 512, top 4, 4096 tokens 64 and 54, 40 and 33; 256, where every
+// row of weights is read for 16 tokens at 5.5 TB/s, 24.2 and 25.5, 15.9 and 16.4.
+// A library GEMM per expert with its gathers, casts and index_add took 958 us behind
 // a host read at the first of these.
-#include "flash_prefill.h"
+#include "tile_gemm.h"
 #include <torch/library.h>
 #include <ATen/ATen.h>
 #include <ATen/hip/HIPContext.h>
@@ -50,406 +29,191 @@ namespace kaito {
 
 namespace {
 
-using flash::f32x16;
-using flash::hbf16x8;
-using flash::mfma32;
-
-constexpr int BK = 64;              // K step
-constexpr int BN = 256;             // weight rows per tile
 constexpr int NG = 4;               // column tiles that share row tiles
-constexpr int XCD_CUS = 32;
-// A quarter takes about two fifths of a tile's time, and the last round runs on
-// caches of its own: 17 to 24 tiles in three rounds of quarters lost (2880 x 2880,
-// 4096 tokens, down: 341 and 352 us), 9 to 16 in two broke even or lost 1 %, except
-// where they are the whole step (58 and 50).
-constexpr int QUARTER_REST = XCD_CUS / 4;
+constexpr int CUS = 256;            // 8 XCDs of 32
 
-struct GemmArgs {
-  short* out;                       // [TK, N]
-  float* out32;                     // the same in f32 (DOWN), or nullptr
-  const short* x;                   // up: [T, K]; down: [TK, K]
-  const short* w;                   // [E, rows, K]
-  const short* bias;                // [E, rows] or nullptr
-  const int* rows;                  // x row of a sorted row; none: the same
-  const int* offsets;               // [.., E + 1]
-  int e_base, E, N, K;
-  float limit;
+using tile::BK;
+using tile::GemmArgs;
+using tile::Tile;
+using tile::SILU;
+using tile::CLAMPED;
+using tile::RELU2;
+using tile::PLAIN;
+using tile::PLAIN_F32;
+
+// inclusive sum over the lanes before
+KAITO_DEV int lane_scan(int x) {
+  auto add = [&](auto ctrl, auto rows) {
+    x += __builtin_amdgcn_update_dpp(0, x, decltype(ctrl)::value,
+                                     decltype(rows)::value, 0xf, false);
+  };
+  using std::integral_constant;
+  add(integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});  // row_shr
+  add(integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});
+  add(integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});
+  add(integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});
+  add(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});  // bcast15
+  add(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});  // bcast31
+  return x;
+}
+
+// rows of 64 experts from e0 on, one per lane
+struct Rows {
+  int o0, o1;
+  KAITO_DEV Rows(const GemmArgs& a, const int e0) {
+    const int lane = threadIdx.x & 63, e = a.e_base + e0 + lane;
+    o0 = e0 + lane < a.E ? a.offsets[e] : 0;
+    o1 = e0 + lane < a.E ? a.offsets[e + 1] : 0;
+  }
+  KAITO_DEV int tiles(const int BM) const { return (o1 - o0 + BM - 1) / BM; }
 };
 
-enum Kind { UP_GATED, UP_CLAMPED, UP_PLAIN, DOWN };
-constexpr bool is_gated(int kind) { return kind <= UP_CLAMPED; }
+// Tiles of 32 FM x 32 FN of a launch, numbered expert by expert, in blocks of NG
+// column tiles x all row tiles, column fastest; every XCD takes one contiguous
+// eighth: the 32 in flight behind one L2 share rows and weights.
+template <int FM, int FN, int KIND>
+struct Tiles {
+  static constexpr int BM = 32 * FM, COLS = tile::columns<FN, KIND>();
+  int scan;                         // of the first 64 experts' row tiles
+  int ntiles;                       // column tiles
+  int share, at, here;              // of an XCD; this one's first and number
 
-// 16 bytes per lane from r + lane offset + uniform offset to dst + 16 * lane
-KAITO_DEV void buffer_copy16(__amdgpu_buffer_rsrc_t r, short* dst,
-                             const uint32_t lane_off, const int off) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(
-      r, (__attribute__((address_space(3))) void*)dst, 16, lane_off, off, 0, 0);
-}
-
-// CLAMPED: min(g, limit) sigmoid(1.702 min(g, limit)) (clamp(u) + 1)
-template <int KIND>
-KAITO_DEV float gated(float g, float u, float limit) {
-  if constexpr (KIND == UP_CLAMPED) {
-    g = fminf(g, limit);
-    u = fminf(fmaxf(u, -limit), limit);
-    return (u + 1.f) * swish_f32(g, 1.702f);
+  KAITO_DEV Tiles(const GemmArgs& a, const Rows& first) {
+    ntiles = (a.N + COLS - 1) / COLS;
+    scan = lane_scan(first.tiles(BM));
+    int total = __builtin_amdgcn_readlane(scan, 63);
+    for (int e0 = 64; e0 < a.E; e0 += 64)
+      total += __builtin_amdgcn_readlane(lane_scan(Rows(a, e0).tiles(BM)), 63);
+    total *= ntiles;
+    share = (total + 7) / 8;
+    at = blockIdx.x % 8 * share;
+    here = max(min(share, total - at), 0);
   }
-  return silu_f32(g) * u;
-}
-
-// elements of LDS: two and a half K steps of a whole tile, five of a quarter
-constexpr int LDS = 5 * 256 * BK;
-
-// BM rows x BW weight rows of one expert by 8 waves, WM of them over the rows;
-// NST K steps in LDS, or 0: five slots of BM = BW rows. m0: first row, n0: first
-// output.
-template <int BM, int BW, int WM, int NST, int KIND>
-KAITO_DEV void grouped_tile(const GemmArgs& a, short* lds, const int expert,
-                            const int m0, const int row_end, const int n0) {
-  constexpr int WN = 8 / WM, MT = BM / WM / 32;   // 32-row tiles of a wave
-  constexpr int LX = BM * BK / 8 / 512, LW = BW * BK / 8 / 512;
-  constexpr int STEP = (BM + BW) * BK;
-  static_assert(WN * 64 == BW && NST * STEP <= LDS, "tile");
-  const int lane = threadIdx.x & 63, lr = lane & 31, h = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = wave / WN, wn = wave % WN;
-
-  // ---- staging slots: slot s (16 bytes) is row s / 8, place s % 8; byte
-  // offsets from the tile's first row (gathered rows: from x, which the caller
-  // keeps below 4 GB)
-  const int wrows = is_gated(KIND) ? 2 * a.N : a.N;
-  const short* we = a.w + ((int64_t)expert * wrows + n0) * a.K;
-  const short* xe = a.rows ? a.x : a.x + (int64_t)m0 * a.K;
-  const auto xr = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<short*>(xe), 0, 0xffffffff, 0x27000);
-  const auto wr = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<short*>(we), 0, 0xffffffff, 0x27000);
-  constexpr int CH = BK / 8;        // 16-byte chunks of a row
-  auto place = [](const int row, const int c) { return c ^ (row >> 1 & 7); };
-  uint32_t xs[LX], ws[LW];
-  int src[LX];                      // one wait for all of them
-#pragma unroll
-  for (int j = 0; j < LX; j++)
-    src[j] = min((int)(j * 512 + threadIdx.x) / CH, row_end - 1 - m0);
-  if (a.rows) {
-#pragma unroll
-    for (int j = 0; j < LX; j++) src[j] = a.rows[m0 + src[j]];
-  }
-#pragma unroll
-  for (int j = 0; j < LX; j++) {
-    const int s = j * 512 + threadIdx.x;
-    xs[j] = ((uint32_t)src[j] * a.K + place(s / CH, s % CH) * 8) * 2;
-  }
-#pragma unroll
-  for (int j = 0; j < LW; j++) {
-    const int s = j * 512 + threadIdx.x, row = s / CH;
-    const int c = place(row, s % CH);
-    // gated: every 64 tile rows are 32 gate rows, then their up rows
-    const uint32_t n = is_gated(KIND)
-        ? min((row / 64) * 32 + row % 32, a.N - 1 - n0) +
-              (row % 64 >= 32 ? a.N : 0)
-        : min(row, a.N - 1 - n0);
-    ws[j] = (n * a.K + c * 8) * 2;
-  }
-  auto stage_x = [&](const int k, short* buf, const int j0, const int j1) {
-#pragma unroll
-    for (int j = 0; j < LX; j++)
-      if (j >= j0 && j < j1)
-        buffer_copy16(xr, buf + (j * 512 + wave * 64) * 8, xs[j], k * 2);
-  };
-  auto stage_w = [&](const int k, short* buf) {
-#pragma unroll
-    for (int j = 0; j < LW; j++)
-      buffer_copy16(wr, buf + (j * 512 + wave * 64) * 8, ws[j], k * 2);
-  };
-
-  f32x16 acc[2][MT];
-#pragma unroll
-  for (int i = 0; i < 2; i++)
-#pragma unroll
-    for (int j = 0; j < MT; j++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
-
-  // Fragments of 16 dims of K are read one step ahead of their products, the
-  // first of the next tile beside the last products of this one: the barrier
-  // that frees this tile stands between its last read and its last products.
-  hbf16x8 wf[2][2], xf[2][MT];
-  auto read = [&](const short* xbuf, const short* wbuf, const int kk) {
-    const int c = place(lr, kk * 2 + h) * 8, f = kk & 1;
-    const short* xb = xbuf + (wm * (BM / WM) + lr) * BK + c;
-    const short* wb = wbuf + (wn * 64 + lr) * BK + c;
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-      wf[f][i] = *reinterpret_cast<const hbf16x8*>(wb + i * 32 * BK);
-#pragma unroll
-    for (int j = 0; j < MT; j++)
-      xf[f][j] = *reinterpret_cast<const hbf16x8*>(xb + j * 32 * BK);
-  };
-  auto multiply = [&](const int kk) {
-    const int f = kk & 1;
-    __builtin_amdgcn_sched_barrier(0);      // the next reads are under way
-#pragma unroll
-    for (int j = 0; j < MT; j++)
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-        acc[i][j] = mfma32(wf[f][i], xf[f][j], acc[i][j]);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  // own reads done and own loads landed but for the newest LATER: all's
-  auto meet = [&](auto newest, const bool later) {
-    constexpr int N = decltype(newest)::value;
-    if (N > 0 && later)
-      __builtin_amdgcn_s_waitcnt(0x0070 | (N & 15) | ((N >> 4) << 14));
-    else
-      __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0)
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-  };
-
-  if constexpr (NST == 0) {
-    // x and w by turns through five slots: x(s), w(s) and x(s + 1) are there
-    // when step s begins, w(s + 1) and x(s + 2) are asked for in its course.
-    // All of a step's loads at once, for the next but one, kept the caches busy
-    // in bursts: 514 cycles from request to data where 360 are now.
-    constexpr int SLOT = BM * BK;
-    static_assert(BM == BW && 5 * SLOT <= LDS && BK == 64, "slots");
-    constexpr std::integral_constant<int, LX> newest;
-    stage_w(0, lds + SLOT);
-    stage_x(0, lds, 0, LX);
-    if (BK < a.K) stage_x(BK, lds + 2 * SLOT, 0, LX);
-    meet(newest, BK < a.K);
-    int slot = 0;                   // of x(s); w(s), x(s + 1) .. follow
-    auto nth = [&](const int i) {
-      return lds + (slot + i < 5 ? slot + i : slot + i - 5) * SLOT;
-    };
-    read(nth(0), nth(1), 0);
-    for (int k = 0; k < a.K; k += BK) {
-      const bool more = k + BK < a.K, more2 = k + 2 * BK < a.K;
-      read(nth(0), nth(1), 1);
-      if (more) stage_w(k + BK, nth(3));
-      multiply(0);
-      read(nth(0), nth(1), 2);
-      if (more2) stage_x(k + 2 * BK, nth(4), 0, LX / 2);
-      multiply(1);
-      read(nth(0), nth(1), 3);
-      if (more2) stage_x(k + 2 * BK, nth(4), LX / 2, LX);
-      multiply(2);
-      meet(newest, more2);
-      slot = slot < 3 ? slot + 2 : slot - 3;
-      if (more) read(nth(0), nth(1), 0);
-      multiply(3);
-    }
-  } else {
-    constexpr int STEPS = BK / 16;
-    constexpr std::integral_constant<int, (NST - 2) * (LX + LW)> newest;
-    auto stage = [&](const int k, const int at) {
-      stage_x(k, lds + at * STEP, 0, LX);
-      stage_w(k, lds + at * STEP + BM * BK);
-    };
-    auto next = [&](const int at, const int kk) {
-      read(lds + at * STEP, lds + at * STEP + BM * BK, kk);
-    };
-    stage(0, 0);
-#pragma unroll
-    for (int i = 1; i < NST - 1; i++)
-      if (i * BK < a.K) stage(i * BK, i);
-    meet(newest, (NST - 2) * BK < a.K);
-    if ((NST - 1) * BK < a.K) stage((NST - 1) * BK, NST - 1);
-    next(0, 0);
-    int cur = 0;
-    for (int k = 0; k < a.K; k += BK) {
-#pragma unroll
-      for (int kk = 0; kk < STEPS - 1; kk++) {
-        next(cur, kk + 1);
-        multiply(kk);
+  KAITO_DEV Tile tile(const GemmArgs& a, const Rows& first, int t) const {
+    Tile out{};
+    int mtiles = 1;
+    t += at;
+    auto look = [&](const Rows& r, const int scan, const int e0) {
+      const unsigned long long hit = __ballot(scan * ntiles > t);
+      if (!hit) {
+        t -= __builtin_amdgcn_readlane(scan, 63) * ntiles;
+        return false;
       }
-      meet(newest, k + (NST - 1) * BK < a.K);
-      if (k + NST * BK < a.K) stage(k + NST * BK, cur);
-      cur = cur == NST - 1 ? 0 : cur + 1;
-      if (k + BK < a.K) next(cur, 0);
-      multiply(STEPS - 1);
-    }
-  }
-
-  // ---- outputs n = 8 b + 4 h + e of 32-row tile i, token row lr of tile j
-  constexpr int NI = is_gated(KIND) ? 1 : 2;
-  constexpr int WC = NI * 32;       // columns of a wave: all exist or none
-  const int c0 = n0 + wn * WC;
-  if (c0 >= a.N) return;            // N is a multiple of 64; no barrier below
-  // added where a value leaves: ahead of that, over all of acc, it cost 132 bytes
-  // of scratch per lane and 55 us of 312 (up, 8 experts of 2048 x 2048, 16384
-  // pairs of uneven experts, weights out of the caches; with the activations'
-  // divisions in half the instructions). Read once: for every 32 rows anew, a down
-  // projection of 8192 tokens by 16 experts of 1024 x 512 took 51.9 us, now 47.9
-  const short* be = a.bias + (int64_t)expert * wrows + c0 + 4 * h;
-  short4_t bias[2][4] = {};
-  if (a.bias) {
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int b = 0; b < 4; b++)
-        bias[i][b] = *reinterpret_cast<const short4_t*>(
-            be + (is_gated(KIND) ? i * a.N : i * 32) + 8 * b);
-  }
-  // bf16 rows pass through the wave's part of LDS (every wave is done with
-  // its tiles) and leave as 16 bytes a lane
-  constexpr int PITCH = WC + 8, LANES = WC / 8;
-  short* slab = lds + wave * 32 * PITCH;
-#pragma unroll
-  for (int j = 0; j < MT; j++) {
-    const int mj = m0 + wm * (BM / WM) + j * 32;
-#pragma unroll
-    for (int i = 0; i < NI; i++)
-#pragma unroll
-      for (int b = 0; b < 4; b++) {
-        float4_t v, u;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          v[e] = acc[i][j][b * 4 + e];
-          if constexpr (is_gated(KIND)) u[e] = acc[1][j][b * 4 + e];
-        }
-        if (a.bias) {
-#pragma unroll
-          for (int e = 0; e < 4; e++) {
-            v[e] += bf16_to_f32(bias[i][b][e]);
-            if constexpr (is_gated(KIND)) u[e] += bf16_to_f32(bias[1][b][e]);
-          }
-        }
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          if constexpr (is_gated(KIND)) {
-            v[e] = gated<KIND>(v[e], u[e], a.limit);
-          } else if constexpr (KIND == UP_PLAIN) {
-            v[e] = fmaxf(v[e], 0.f);
-            v[e] *= v[e];
-          }
-        }
-        const int n = i * 32 + 8 * b + 4 * h;
-        if (KIND == DOWN && a.out32) {
-          if (mj + lr < row_end)
-            *reinterpret_cast<float4_t*>(
-                a.out32 + (int64_t)(mj + lr) * a.N + c0 + n) = v;
-        } else {
-          *reinterpret_cast<short4_t*>(slab + lr * PITCH + n) =
-              short4_t{f32_to_bf16(v[0]), f32_to_bf16(v[1]),
-                       f32_to_bf16(v[2]), f32_to_bf16(v[3])};
-        }
-      }
-    if (KIND == DOWN && a.out32) continue;
-    __builtin_amdgcn_wave_barrier();
-    asm volatile("" ::: "memory");
-#pragma unroll
-    for (int r = 0; r < 32; r += 64 / LANES) {
-      const int row = r + lane / LANES, n = lane % LANES * 8;
-      const short8_t v =
-          *reinterpret_cast<const short8_t*>(slab + row * PITCH + n);
-      if (mj + row < row_end)
-        *reinterpret_cast<short8_t*>(a.out + (int64_t)(mj + row) * a.N + c0 +
-                                     n) = v;
-    }
-    __builtin_amdgcn_wave_barrier();
-    asm volatile("" ::: "memory");
-  }
-}
-
-template <int BM, int KIND>
-__global__ __launch_bounds__(512, 2) void moe_grouped_kernel(const GemmArgs a) {
-  constexpr int COLS = is_gated(KIND) ? BN / 2 : BN;   // outputs per tile
-  constexpr bool QUARTERS = BM == 256;
-  __shared__ __attribute__((aligned(128)))
-  short lds[BM == 256 ? LDS : 2 * (BM + BN) * BK];
-  const int lane = threadIdx.x & 63;
-  const int ntiles = (a.N + COLS - 1) / COLS;
-
-  // ---- this workgroup's tile: every wave scans the experts, 64 at a time
-  int total = 0;
-  for (int e0 = 0; e0 < a.E; e0 += 64) {
-    const int e = a.e_base + e0 + lane;
-    int n = e0 + lane < a.E
-        ? (a.offsets[e + 1] - a.offsets[e] + BM - 1) / BM : 0;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
-    total += n;
-  }
-  total = __builtin_amdgcn_readfirstlane(total) * ntiles;
-  const int share = (total + 7) / 8, at = (blockIdx.x % 8) * share;
-  const int here = min(share, total - at);  // tiles of this XCD
-  int rest = here % XCD_CUS;        // of its last round
-  if (!QUARTERS || rest > (here < XCD_CUS ? 2 : 1) * QUARTER_REST) rest = 0;
-  int in_share = blockIdx.x / 8, quarter = -1;
-  if (in_share >= here - rest) {
-    const int p = in_share - (here - rest);
-    if (p >= 4 * rest) return;
-    in_share = here - rest + p / 4;
-    quarter = p % 4;
-  }
-  int t = at + in_share;
-  int expert = -1, mtiles = 0, row0 = 0, row_end = 0;
-  for (int e0 = 0; e0 < a.E && expert < 0; e0 += 64) {
-    const int e = a.e_base + e0 + lane;
-    const int o0 = e0 + lane < a.E ? a.offsets[e] : 0;
-    const int o1 = e0 + lane < a.E ? a.offsets[e + 1] : 0;
-    const int n = (o1 - o0 + BM - 1) / BM;
-    int scan = n;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int add = __shfl_up(scan, off, 64);
-      if (lane >= off) scan += add;
-    }
-    const unsigned long long hit = __ballot(scan * ntiles > t);
-    if (hit) {
       const int src = __builtin_ctzll(hit);
-      expert = a.e_base + e0 + src;
-      mtiles = __builtin_amdgcn_readlane(n, src);
+      mtiles = __builtin_amdgcn_readlane(r.tiles(BM), src);
       t -= (__builtin_amdgcn_readlane(scan, src) - mtiles) * ntiles;
-      row0 = __builtin_amdgcn_readlane(o0, src);
-      row_end = __builtin_amdgcn_readlane(o1, src);
-    } else {
-      t -= __builtin_amdgcn_readlane(scan, 63) * ntiles;
-    }
+      out.expert = a.e_base + e0 + src;
+      out.m0 = __builtin_amdgcn_readlane(r.o0, src);
+      out.row_end = __builtin_amdgcn_readlane(r.o1, src);
+      return true;
+    };
+    if (!look(first, scan, 0))
+      for (int e0 = 64; e0 < a.E; e0 += 64) {
+        const Rows r(a, e0);
+        if (look(r, lane_scan(r.tiles(BM)), e0)) break;
+      }
+    const int blk = t / (NG * mtiles);
+    const int wide = min(NG, ntiles - blk * NG);
+    const int in_blk = t - blk * NG * mtiles;
+    out.n0 = (blk * NG + in_blk % wide) * COLS;
+    out.m0 += in_blk / wide * BM;
+    return out;
   }
-  // blocks of NG column tiles, column fastest
-  const int blk = t / (NG * mtiles);
-  const int wide = min(NG, ntiles - blk * NG);
-  const int in_blk = t - blk * NG * mtiles;
-  const int nt = blk * NG + in_blk % wide, mt0 = in_blk / wide;
+};
 
-  const int m0 = row0 + mt0 * BM, n0 = nt * COLS;
-  if constexpr (QUARTERS) {
-    if (quarter >= 0) {
-      const int m = m0 + quarter / 2 * (BM / 2);
-      const int n = n0 + quarter % 2 * (COLS / 2);
-      if (m < row_end && n < a.N)
-        grouped_tile<BM / 2, BN / 2, 4, 5, KIND>(a, lds, expert, m, row_end,
-                                                 n);
-      return;
-    }
+// One workgroup per CU. Tiles of 256 x 256, those of a small last round in quarters,
+// or of 128 x 256, 256 x 128 or 128 x 128 altogether, whichever is shortest. A round of them takes, where
+// weights and rows come from the caches, about 5 (50 us at K = 2048), 3, 3 and 2
+// (18 us), the quarters as long as those of 128 x 128. 700 tokens by 8 of 2048 x 2048,
+// up: 53, 37, 59 and 41 us; 200: 34, 30, 33 and 24; 4096 tokens by 64 of 1024 x 512:
+// 60, 56, 66 and 55.
+enum { LARGE, WIDE, TALL, SMALL };
+template <int KIND>
+__global__ __launch_bounds__(256, 1) void moe_grouped_kernel(const GemmArgs a) {
+  __shared__ __attribute__((aligned(1024))) short lds[tile::LDS];
+  const Rows rows(a, 0);
+  const Tiles<8, 8, KIND> large(a, rows);
+  const Tiles<8, 4, KIND> tall(a, rows);
+  const Tiles<4, 8, KIND> wide(a, rows);
+  const Tiles<4, 4, KIND> small(a, rows);
+  constexpr int workers = CUS / 8;
+  auto rounds = [&](const int n) { return (n + workers - 1) / workers; };
+  // of n tiles, those that are cut in quarters
+  auto last = [&](const int n) {
+    const int rest = n % workers;
+    return 4 * rest > workers * (n < workers ? 2 : 1) ? 0 : rest;
+  };
+  // the same answer on all XCDs
+  const int over = last(large.share);
+  int best = 5 * rounds(large.share - over) + 2 * rounds(4 * over), mode = LARGE;
+  auto other = [&](const int m, const int cost) {
+    if (cost < best) best = cost, mode = m;
+  };
+  other(WIDE, 3 * rounds(wide.share));
+  other(TALL, 3 * rounds(tall.share));
+  other(SMALL, 2 * rounds(small.share));
+  const int rest = last(large.here);
+  int i = blockIdx.x / 8;
+  if (mode == LARGE)
+    tile::stream<8, 8, KIND>(a, lds, [&](Tile& t) {
+      if (i >= large.here - rest) return false;
+      t = large.tile(a, rows, i);
+      i += workers;
+      return true;
+    });
+  auto all = [&](const auto& tiles) {
+    return [&](Tile& t) {
+      if (i >= tiles.here) return false;
+      t = tiles.tile(a, rows, i);
+      i += workers;
+      return true;
+    };
+  };
+  if (mode == WIDE) {
+    tile::stream<4, 8, KIND>(a, lds, all(wide));
+  } else if (mode == TALL) {
+    tile::stream<8, 4, KIND>(a, lds, all(tall));
+  } else {
+    i = blockIdx.x / 8;
+    const int end = mode == LARGE ? 4 * rest : small.here;
+    tile::stream<4, 4, KIND>(a, lds, [&](Tile& t) {
+      for (; i < end; i += workers) {
+        if (mode == LARGE) {
+          t = large.tile(a, rows, large.here - rest + i / 4);
+          t.m0 += i % 4 / 2 * (large.BM / 2);
+          t.n0 += i % 2 * (large.COLS / 2);
+          if (t.m0 >= t.row_end || t.n0 >= a.N) continue;
+        } else {
+          t = small.tile(a, rows, i);
+        }
+        i += workers;
+        return true;
+      }
+      return false;
+    });
   }
-  grouped_tile<BM, BN, 2, BM == 256 ? 0 : 2, KIND>(a, lds, expert, m0, row_end,
-                                                   n0);
 }
 
 // ---- keys and values of latent rows ----------------------------------------
 // [k | v][t] = c[t] [Wk | Wv^T]^T, tiles of 256 x 256 over both: the tiles of
 // Wk's N1 rows first. Behind one another, as a library product and a batched one
 // of Wv as it is stored, they took 32 + 42 us (8192 rows of 512, 16 heads of 128 +
-// 128; 34 GFLOP, 80 MB), here 47 with the transposition: 8 K steps a tile, whose
-// start and end take as long.
-__global__ __launch_bounds__(512, 2) void latent_kv_kernel(GemmArgs a,
-                                                               const short* w2,
-                                                               const int N1,
-                                                               const int T) {
-  __shared__ __attribute__((aligned(128))) short lds[LDS];
-  const int ntiles = (a.N + BN - 1) / BN, mtiles = (T + 255) / 256;
+// 128; 34 GFLOP, 80 MB), here 41 with the transposition: 8 K steps a tile.
+__global__ __launch_bounds__(256, 1) void latent_kv_kernel(const GemmArgs a,
+                                                           const int T) {
+  __shared__ __attribute__((aligned(1024))) short lds[tile::LDS];
+  const int ntiles = (a.N + 255) / 256, mtiles = (T + 255) / 256;
   const int total = ntiles * mtiles, share = (total + 7) / 8;
-  const int t = blockIdx.x % 8 * share + blockIdx.x / 8;
-  if ((int)blockIdx.x / 8 >= share || t >= total) return;
-  const int blk = t / (NG * mtiles), in_blk = t - blk * NG * mtiles;
-  const int wide = min(NG, ntiles - blk * NG);
-  const int n0 = (blk * NG + in_blk % wide) * BN, m0 = in_blk / wide * 256;
-  if (n0 >= N1) a.w = w2 - (int64_t)N1 * a.K;
-  grouped_tile<256, BN, 2, 0, DOWN>(a, lds, 0, m0, T, n0);
+  const int at = blockIdx.x % 8 * share, here = min(share, total - at);
+  int i = blockIdx.x / 8;
+  tile::stream<8, 8, PLAIN>(a, lds, [&](Tile& t) {
+    if (i >= here) return false;
+    const int blk = (at + i) / (NG * mtiles), in_blk = at + i - blk * NG * mtiles;
+    const int wide = min(NG, ntiles - blk * NG);
+    t = {0, in_blk / wide * 256, T, (blk * NG + in_blk % wide) * 256};
+    i += CUS / 8;
+    return true;
+  });
 }
 
 // w [H, K, V] -> out [H, V, K], by squares of 64
@@ -613,23 +377,9 @@ __global__ __launch_bounds__(256) void moe_combine_norm_kernel(
 }
 
 template <int KIND>
-void launch_grouped(const GemmArgs& a, int64_t TK) {
-  constexpr int COLS = is_gated(KIND) ? BN / 2 : BN;
-  const int64_t ntiles = (a.N + COLS - 1) / COLS;
-  auto stream = at::hip::getCurrentHIPStream();
-  auto launch = [&](auto bm) {
-    constexpr int BM = decltype(bm)::value;
-    // most row tiles that TK rows in E groups can make
-    const int64_t most = TK / BM + std::min<int64_t>(a.E, TK);
-    // per XCD, a rest's quarters in place of its tiles
-    const int64_t quarters = BM == 256 ? 3 * 2 * QUARTER_REST : 0;
-    hipLaunchKernelGGL((moe_grouped_kernel<BM, KIND>),
-        dim3(((most * ntiles + 7) / 8 + quarters) * 8), dim3(512), 0, stream,
-        a);
-  };
-  // half tiles where an expert's rows would leave most of a whole one empty
-  if (TK >= 192 * (int64_t)a.E) launch(std::integral_constant<int, 256>{});
-  else launch(std::integral_constant<int, 128>{});
+void launch_grouped(const GemmArgs& a) {
+  hipLaunchKernelGGL((moe_grouped_kernel<KIND>), dim3(CUS), dim3(256), 0,
+                     at::hip::getCurrentHIPStream(), a);
 }
 
 void check16(const at::Tensor& t) {
@@ -670,7 +420,7 @@ void moe_grouped_up(at::Tensor act, at::Tensor x, at::Tensor w,
   if (a.bias) a.bias -= e_base * 2 * a.N;
   a.rows = sorted_ids.data_ptr<int>();
   at::Tensor gathered;
-  if (x.numel() >= 1LL << 31) {     // beyond 32-bit byte offsets
+  if (x.numel() * 2 > tile::MOST_BYTES) {       // beyond 32-bit offsets
     gathered = x.index_select(0, sorted_ids);
     a.x = (const short*)gathered.data_ptr();
     a.rows = nullptr;
@@ -678,9 +428,9 @@ void moe_grouped_up(at::Tensor act, at::Tensor x, at::Tensor w,
   a.offsets = offsets.data_ptr<int>();
   a.limit = (float)act_limit;
   if (act.size(0) == 0 || a.E == 0 || a.N == 0) return;
-  if (plain) launch_grouped<UP_PLAIN>(a, act.size(0));
-  else if (act_mode == 1) launch_grouped<UP_CLAMPED>(a, act.size(0));
-  else launch_grouped<UP_GATED>(a, act.size(0));
+  if (plain) launch_grouped<RELU2>(a);
+  else if (act_mode == 1) launch_grouped<CLAMPED>(a);
+  else launch_grouped<SILU>(a);
 }
 
 void moe_grouped_down(at::Tensor y, at::Tensor act, at::Tensor w,
@@ -712,7 +462,8 @@ void moe_grouped_down(at::Tensor y, at::Tensor act, at::Tensor w,
   a.w = (const short*)w.data_ptr() - e_base * w.stride(0);
   a.offsets = offsets.data_ptr<int>();
   if (y.size(0) == 0 || a.E == 0 || a.N == 0) return;
-  launch_grouped<DOWN>(a, y.size(0));
+  if (wide) launch_grouped<PLAIN_F32>(a);
+  else launch_grouped<PLAIN>(a);
 }
 
 // kv [T, H D + H V]: c [T, K] times wk [H, D, K] (rows K long) and wv [H, K, V]
@@ -723,7 +474,7 @@ void latent_kv(at::Tensor kv, at::Tensor c, at::Tensor wk, at::Tensor wv) {
   const int64_t N1 = H * wk.size(1);
   TORCH_CHECK(wk.size(2) == K && wv.size(0) == H && wv.size(1) == K &&
               kv.size(0) == T && kv.size(1) == N1 + H * V &&
-              K % 64 == 0 && K > 0 && V % 64 == 0 && N1 % BN == 0 &&
+              K % 64 == 0 && K > 0 && V % 64 == 0 && N1 % 256 == 0 &&
               T < (1ll << 22) && kv.size(1) < (1ll << 22));
   if (T == 0 || H == 0) return;
   auto stream = at::hip::getCurrentHIPStream();
@@ -738,10 +489,10 @@ void latent_kv(at::Tensor kv, at::Tensor c, at::Tensor wk, at::Tensor wv) {
   a.E = 1;
   a.N = (int)kv.size(1);
   a.K = (int)K;
-  const int64_t tiles = (T + 255) / 256 * ((a.N + BN - 1) / BN);
-  hipLaunchKernelGGL(latent_kv_kernel, dim3((tiles + 7) / 8 * 8),
-                     dim3(512), 0, stream, a, (const short*)wt.data_ptr(),
-                     (int)N1, (int)T);
+  a.w2 = (const short*)wt.data_ptr();
+  a.n2 = (int)N1;
+  hipLaunchKernelGGL(latent_kv_kernel, dim3(CUS), dim3(256), 0, stream, a,
+                     (int)T);
 }
 
 // checks shared by both sums

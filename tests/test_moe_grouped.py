@@ -93,6 +93,21 @@ def test_grouped_rounds(counts, H, IE, mode, bias):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("counts,H,IE,mode,bias", [
+    ([1800, 1400, 1100, 700, 500, 300, 120, 81], 2880, 1024, 0, False),
+    ([200] * 15, 320, 1088, 0, True),          # up: 256 rows x 128 weight rows
+    ([250, 130] * 4, 384, 1600, 1, True),      # 128 x 256
+    ([120] * 8, 320, 2048, 0, False),          # 128 x 128, one round
+    ([130, 1] * 9, 576, 2112, 2, False),
+    ([90, 0, 128] * 23, 64, 512, 0, True),     # more experts than lanes
+])
+@pytest.mark.parametrize("f32", [False, True])
+def test_grouped_shapes(counts, H, IE, mode, bias, f32):
+    """Each shape of tiles, several rounds of one, the same one on all XCDs."""
+    test_grouped_step(counts, H, IE, mode, bias, None, f32)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("counts,H,IE,mode,bias,part", [
     ([1], 64, 64, 0, False, None),
     ([3, 0, 16, 17, 1], 256, 192, 0, True, None),
