@@ -12,6 +12,8 @@ time one of its ops is called.
 """
 from __future__ import annotations
 
+import functools
+
 import numpy as np
 import torch
 import torch.autograd.forward_ad as _fwd_ad
@@ -27,7 +29,8 @@ for _g, _names in {
     "core": ("rms_norm fused_add_rms_norm rotary_embedding silu_and_mul "
              "gelu_and_mul gelu layer_norm fused_add_layer_norm "
              "rope_and_cache reshape_and_cache topk skinny_linear skinny_norm skinny_swiglu "
-             "skinny_linear_pair batch_linear batch_parts add_rms_norm_parts"),
+             "skinny_linear_pair batch_linear batch_parts add_rms_norm_parts "
+             "tile_swiglu tile_pair"),
     "attn": ("paged_attention paged_attention_sp rope_paged_attention "
              "prefill_attention "
              "mla_prefill_attention context_attention mfma_tile_gemm paged_read_bw"),
@@ -397,6 +400,12 @@ def linear_pair(x: torch.Tensor, w: torch.Tensor, x2: torch.Tensor,
         _K.skinny_linear_pair(out, x, w, _none(bias, x), out2, x2, w2,
                               _none(bias2, x))
         return out, out2
+    if _pair_tiled(x, w, x2, w2) and _plain_bias(bias, w) \
+            and _plain_bias(bias2, w2):
+        out, out2 = (torch.empty(x.size(0), v.size(0), dtype=x.dtype,
+                                 device=x.device) for v in (w, w2))
+        _K.tile_pair(out, x, w, _none(bias, x), out2, x2, w2, _none(bias2, x))
+        return out, out2
     return linear(x, w, bias), linear(x2, w2, bias2)
 
 
@@ -406,6 +415,74 @@ def _pair_pays(M: int, N: int, one: bool) -> bool:
     2048, one launch as a share of two, 24576 and 576 rows of W at 16 and 32 rows
     1.02 and 1.20, with one x 0.84 and 0.81; 8192 and 1024 at 32 0.89)."""
     return one or M <= 4 or N < 16384
+
+
+@functools.lru_cache(1024)
+def _tile_fill(M: int, N: int) -> float:
+    """What share of its time a product of M rows and N weight rows keeps the
+    chip's 256 workgroups busy for, in the best of the shapes that the tiles'
+    kernels choose from (csrc/tile_gemm.h `run`: the same costs)."""
+    def share(rows, cols):          # tiles of an XCD
+        return -(-(-(-M // rows) * -(-N // cols)) // 8)
+
+    def rounds(n):
+        return -(-n // 32)
+    large = share(256, 256)
+    rest = large % 32
+    if rest > (16 if large < 32 else 8):
+        rest = 0
+    cost = min(5 * rounds(large - rest) + 2 * rounds(4 * rest),
+               3 * rounds(share(128, 256)), 3 * rounds(share(256, 128)),
+               2 * rounds(share(128, 128)))
+    return M * N / (cost * 256 * 65536 / 5)
+
+
+def _tiles_fit(x: torch.Tensor, w: torch.Tensor, cols: int) -> bool:
+    """Operands that the tiles' kernels take."""
+    return _plain_rows(x, w, (1 << 24) - 1) and x.is_contiguous() \
+        and w.size(1) % 64 == 0 and w.size(0) % cols == 0 \
+        and w.size(1) < 1 << 22 and w.numel() <= 0x7fff8000
+
+
+def _tiled(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether a SwiGLU pair of a prompt's rows runs on the tiles, activation
+    included (csrc/tile_linear.hip)."""
+    return w.dim() == 2 and x.dim() == 2 \
+        and _tiled_shape(x.size(0), *w.shape) and _tiles_fit(x, w, 128)
+
+
+def _tiled_shape(M: int, N: int, K: int) -> bool:
+    """The pass over the library's output that tiles spare is worth an unevenly
+    filled last round where the chip is busy for 82 % of the time, or where K is
+    short and the rows are many (us, library and activation, tiles: 28672 x 4096
+    at 512 rows 120, 111, 1500 294, 294, 8192 1385, 1259; 22016 x 4096 at 1500 316,
+    218, at 1000, 73 % busy, 175, 203; 35840 x 5120 at 3000 889, 766; 5760 x 2880 at
+    8192 339, 189, at 1000, 57 %, 43, 54; 16384 x 3072 at 1500, 81 %, 144, 158;
+    4096 x 2048 at 1000 26, 20, 8192 118, 107; 1024 x 2048 at 2048, 31 %, 20, 19 and
+    1500 18, 19; 2816 x 2048 at 1500, 42 %, 28, 27)."""
+    if M <= 256:
+        return False
+    fill = _tile_fill(M, N)
+    return fill >= 0.82 or (K <= 2048 and M >= 1000 and fill >= 0.42)
+
+
+def _pair_tiled(x, w, x2, w2) -> bool:
+    return x.dim() == x2.dim() == w.dim() == w2.dim() == 2 \
+        and x.shape == x2.shape and w.size(0) % 256 == 0 \
+        and _pair_tiled_shape(x.size(0), w.size(0) + w2.size(0), w.size(1)) \
+        and x.device == x2.device \
+        and _tiles_fit(x, w, 256) and _tiles_fit(x2, w2, 64)
+
+
+def _pair_tiled_shape(M: int, N: int, K: int) -> bool:
+    """Whether two products of a prompt's rows, N outputs together, run as one
+    launch of tiles: no last round of their own (us, library twice and tiles, K of
+    2048: 3072 + 576 at 128 rows 20, 16, 700 28, 19, 2048 42, 31, 8192 120, 99, at
+    64 17, 16; 3072 + 4096 at 128 30, 23, 2048 67, 55, 6500 170, 149, but 87, 93 at
+    3000, 100, 102 at 4096 and 187, 191 at 8192; 2048 + 576 at 8192 79, 82). K of
+    5120 and 7168 gave 0.54 to 1.38 times."""
+    return M >= 128 and K <= 2048 and N <= 7168 and (
+        M * N <= 20000000 or _tile_fill(M, N) >= 0.88)
 
 
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -418,6 +495,11 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
             _K.skinny_swiglu(out, x, w)
         else:
             _K.batch_linear(out, x, w, _none(None, x), 0, 0, True)
+        return out
+    if _tiled(x, w):
+        out = torch.empty(x.size(0), w.size(0) // 2, dtype=x.dtype,
+                          device=x.device)
+        _K.tile_swiglu(out, x, w)
         return out
     return silu_and_mul(torch.nn.functional.linear(x, w))
 

@@ -28,7 +28,7 @@ GROUPS: Dict[str, List[str]] = {
     # norms, activations, rope, paged-cache scatter, top-k
     "core": ["bind_core.cpp", "rmsnorm.hip", "activation.hip", "rope.hip",
              "cache.hip", "topk.hip", "skinny_linear.hip",
-             "batch_linear.hip"],
+             "batch_linear.hip", "tile_linear.hip"],
     # rotary-model attention over the paged cache (decode/prefill/context)
     "attn": ["bind_attn.cpp", "paged_attention.hip",
              "paged_attention_sp.hip", "prefill_attention.hip",

@@ -29,10 +29,9 @@ namespace kaito {
 
 namespace {
 
-constexpr int NG = 4;               // column tiles that share row tiles
-constexpr int CUS = 256;            // 8 XCDs of 32
-
 using tile::BK;
+using tile::CUS;
+using tile::NG;
 using tile::GemmArgs;
 using tile::Tile;
 using tile::SILU;
@@ -74,11 +73,13 @@ struct Rows {
 template <int FM, int FN, int KIND>
 struct Tiles {
   static constexpr int BM = 32 * FM, COLS = tile::columns<FN, KIND>();
-  int scan;                         // of the first 64 experts' row tiles
+  const GemmArgs& a;
+  const Rows& first;                // of 64 experts
+  int scan;                         // of their row tiles
   int ntiles;                       // column tiles
   int share, at, here;              // of an XCD; this one's first and number
 
-  KAITO_DEV Tiles(const GemmArgs& a, const Rows& first) {
+  KAITO_DEV Tiles(const GemmArgs& a, const Rows& first) : a(a), first(first) {
     ntiles = (a.N + COLS - 1) / COLS;
     scan = lane_scan(first.tiles(BM));
     int total = __builtin_amdgcn_readlane(scan, 63);
@@ -89,7 +90,7 @@ struct Tiles {
     at = blockIdx.x % 8 * share;
     here = max(min(share, total - at), 0);
   }
-  KAITO_DEV Tile tile(const GemmArgs& a, const Rows& first, int t) const {
+  KAITO_DEV Tile operator()(int t) const {
     Tile out{};
     int mtiles = 1;
     t += at;
@@ -121,77 +122,12 @@ struct Tiles {
   }
 };
 
-// One workgroup per CU. Tiles of 256 x 256, those of a small last round in quarters,
-// or of 128 x 256, 256 x 128 or 128 x 128 altogether, whichever is shortest. A round of them takes, where
-// weights and rows come from the caches, about 5 (50 us at K = 2048), 3, 3 and 2
-// (18 us), the quarters as long as those of 128 x 128. 700 tokens by 8 of 2048 x 2048,
-// up: 53, 37, 59 and 41 us; 200: 34, 30, 33 and 24; 4096 tokens by 64 of 1024 x 512:
-// 60, 56, 66 and 55.
-enum { LARGE, WIDE, TALL, SMALL };
 template <int KIND>
 __global__ __launch_bounds__(256, 1) void moe_grouped_kernel(const GemmArgs a) {
   __shared__ __attribute__((aligned(1024))) short lds[tile::LDS];
   const Rows rows(a, 0);
-  const Tiles<8, 8, KIND> large(a, rows);
-  const Tiles<8, 4, KIND> tall(a, rows);
-  const Tiles<4, 8, KIND> wide(a, rows);
-  const Tiles<4, 4, KIND> small(a, rows);
-  constexpr int workers = CUS / 8;
-  auto rounds = [&](const int n) { return (n + workers - 1) / workers; };
-  // of n tiles, those that are cut in quarters
-  auto last = [&](const int n) {
-    const int rest = n % workers;
-    return 4 * rest > workers * (n < workers ? 2 : 1) ? 0 : rest;
-  };
-  // the same answer on all XCDs
-  const int over = last(large.share);
-  int best = 5 * rounds(large.share - over) + 2 * rounds(4 * over), mode = LARGE;
-  auto other = [&](const int m, const int cost) {
-    if (cost < best) best = cost, mode = m;
-  };
-  other(WIDE, 3 * rounds(wide.share));
-  other(TALL, 3 * rounds(tall.share));
-  other(SMALL, 2 * rounds(small.share));
-  const int rest = last(large.here);
-  int i = blockIdx.x / 8;
-  if (mode == LARGE)
-    tile::stream<8, 8, KIND>(a, lds, [&](Tile& t) {
-      if (i >= large.here - rest) return false;
-      t = large.tile(a, rows, i);
-      i += workers;
-      return true;
-    });
-  auto all = [&](const auto& tiles) {
-    return [&](Tile& t) {
-      if (i >= tiles.here) return false;
-      t = tiles.tile(a, rows, i);
-      i += workers;
-      return true;
-    };
-  };
-  if (mode == WIDE) {
-    tile::stream<4, 8, KIND>(a, lds, all(wide));
-  } else if (mode == TALL) {
-    tile::stream<8, 4, KIND>(a, lds, all(tall));
-  } else {
-    i = blockIdx.x / 8;
-    const int end = mode == LARGE ? 4 * rest : small.here;
-    tile::stream<4, 4, KIND>(a, lds, [&](Tile& t) {
-      for (; i < end; i += workers) {
-        if (mode == LARGE) {
-          t = large.tile(a, rows, large.here - rest + i / 4);
-          t.m0 += i % 4 / 2 * (large.BM / 2);
-          t.n0 += i % 2 * (large.COLS / 2);
-          if (t.m0 >= t.row_end || t.n0 >= a.N) continue;
-        } else {
-          t = small.tile(a, rows, i);
-        }
-        i += workers;
-        return true;
-      }
-      return false;
-    });
-  }
+  tile::run<KIND>(a, lds, Tiles<8, 8, KIND>(a, rows), Tiles<4, 8, KIND>(a, rows),
+                  Tiles<8, 4, KIND>(a, rows), Tiles<4, 4, KIND>(a, rows));
 }
 
 // ---- keys and values of latent rows ----------------------------------------
@@ -206,7 +142,7 @@ __global__ __launch_bounds__(256, 1) void latent_kv_kernel(const GemmArgs a,
   const int total = ntiles * mtiles, share = (total + 7) / 8;
   const int at = blockIdx.x % 8 * share, here = min(share, total - at);
   int i = blockIdx.x / 8;
-  tile::stream<8, 8, PLAIN>(a, lds, [&](Tile& t) {
+  tile::stream<8, 8, PLAIN, true>(a, lds, [&](Tile& t) {
     if (i >= here) return false;
     const int blk = (at + i) / (NG * mtiles), in_blk = at + i - blk * NG * mtiles;
     const int wide = min(NG, ntiles - blk * NG);
@@ -489,6 +425,7 @@ void latent_kv(at::Tensor kv, at::Tensor c, at::Tensor wk, at::Tensor wv) {
   a.E = 1;
   a.N = (int)kv.size(1);
   a.K = (int)K;
+  a.x2 = a.x;
   a.w2 = (const short*)wt.data_ptr();
   a.n2 = (int)N1;
   hipLaunchKernelGGL(latent_kv_kernel, dim3(CUS), dim3(256), 0, stream, a,

@@ -71,7 +71,10 @@ struct GemmArgs {
   float* out32;                     // PLAIN_F32: [rows, N] in place of out
   const short* x;                   // [.., K]
   const short* w;                   // [E, rows, K]
-  const short* w2;                  // rows from n2 on, where n2 > 0
+  // TWO: outputs from n2 on, of rows x2 (no `rows`) and weights w2, which go to
+  // out2 [rows, N - n2]
+  const short *x2, *w2, *bias2;
+  short* out2;                      // nullptr: to out as the others
   int n2;
   const short* bias;                // [E, rows] or nullptr
   const int* rows;                  // x row of an output row; none: the same
@@ -130,8 +133,8 @@ template <int FN, int KIND> constexpr int columns() {
 }
 
 // Tiles of 32 FM rows x 32 FN weight rows, as next(Tile&) names them until it
-// returns false; the same ones for all waves. n2 is a multiple of 32 FN.
-template <int FM, int FN, int KIND, class Next>
+// returns false; the same ones for all waves. TWO: n2 is a multiple of 32 FN.
+template <int FM, int FN, int KIND, bool TWO, class Next>
 KAITO_DEV void stream(const GemmArgs& a, short* lds, Next&& next) {
   constexpr int D = ahead<FM, FN>(), P = FM * FN / 2;   // pairs of products
   constexpr bool GATED = is_gated(KIND);
@@ -161,7 +164,7 @@ KAITO_DEV void stream(const GemmArgs& a, short* lds, Next&& next) {
     return min(j * 32 + eighth, t.row_end - 1 - t.m0);
   };
   auto aim_w = [&](const Tile& t) {
-    at.w = a.n2 > 0 && t.n0 >= a.n2
+    at.w = TWO && t.n0 >= a.n2
         ? a.w2 + (int64_t)(t.n0 - a.n2) * a.K
         : a.w + ((int64_t)t.expert * wrows + t.n0) * a.K;
 #pragma unroll
@@ -173,7 +176,8 @@ KAITO_DEV void stream(const GemmArgs& a, short* lds, Next&& next) {
     }
   };
   auto aim_x = [&](const Tile& t, const int (&src)[FM]) {
-    at.x = a.rows ? a.x : a.x + (int64_t)t.m0 * a.K;
+    at.x = a.rows ? a.x
+        : (TWO && t.n0 >= a.n2 ? a.x2 : a.x) + (int64_t)t.m0 * a.K;
 #pragma unroll
     for (int j = 0; j < FM; j++)
       at.xs[j] = j * 32 + eighth < t.row_end - t.m0
@@ -359,16 +363,18 @@ KAITO_DEV void stream(const GemmArgs& a, short* lds, Next&& next) {
     // this wave's part of the slot that the next step's loads fill first: the
     // same kilobytes that its own copies go to
     constexpr int RPP = 512 / WC;                   // rows in a kilobyte
-    const int c0 = cur.n0 + wn * WC;
+    const bool apart = TWO && a.out2 && cur.n0 >= a.n2;
+    // columns of the rows written, this wave's first one of them
+    const int N = apart ? a.N - a.n2 : TWO && a.out2 ? a.n2 : a.N;
+    const int c0 = cur.n0 + wn * WC - (apart ? a.n2 : 0);
     const int64_t first_row = cur.m0 + wm * FM * 16;
     const int live = cur.row_end - (int)first_row;  // rows that exist
     constexpr int SIZE = F32 ? 4 : 2;
     // rows and columns that do not exist lie beyond the resource's end
     const auto ro = resource(
-        F32 ? (void*)(a.out32 + first_row * a.N + c0)
-            : (void*)(a.out + first_row * a.N + c0),
-        live > 0 && c0 < a.N
-            ? ((live - 1) * a.N + min(WC, a.N - c0)) * SIZE : 0);
+        F32 ? (void*)(a.out32 + first_row * N + c0)
+            : (void*)((apart ? a.out2 : a.out) + first_row * N + c0),
+        live > 0 && c0 < N ? ((live - 1) * N + min(WC, N - c0)) * SIZE : 0);
     constexpr int BEYOND = 0x80000000;
     char* slab = (char*)(x_of(D) + wave * 512);
     auto slab_at = [&](const int row, const int c) {
@@ -381,12 +387,13 @@ KAITO_DEV void stream(const GemmArgs& a, short* lds, Next&& next) {
     for (int r = 0; r < NR; r++) {
       const int row = (r * 64 + lane) / CH, c = lane % CH;
       from[r] = slab_at(row, c);
-      to[r] = c0 + c * 8 < a.N ? (row * a.N + c * 8) * 2 : BEYOND;
+      to[r] = c0 + c * 8 < N ? (row * N + c * 8) * 2 : BEYOND;
     }
     typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
+    const short* bias = apart ? a.bias2
+        : a.bias ? a.bias + (int64_t)cur.expert * wrows : nullptr;
     auto outputs = [&](const bool biased) {
-      const short* be =
-          a.bias + (int64_t)cur.expert * wrows + c0 + 4 * hi;
+      const short* be = bias + c0 + 4 * hi;
       short4_t b[GATED ? 2 : 1][NO];
       if (biased) {
 #pragma unroll
@@ -394,7 +401,7 @@ KAITO_DEV void stream(const GemmArgs& a, short* lds, Next&& next) {
 #pragma unroll
           for (int g = 0; g < (GATED ? 2 : 1); g++) {
             b[g][i] = short4_t{0, 0, 0, 0};
-            if (c0 + i * 16 < a.N)
+            if (c0 + i * 16 < N)
               b[g][i] =
                   *reinterpret_cast<const short4_t*>(be + g * a.N + i * 16);
           }
@@ -404,7 +411,7 @@ KAITO_DEV void stream(const GemmArgs& a, short* lds, Next&& next) {
 #pragma unroll
         for (int r = 0; r < NR; r++)
           __builtin_amdgcn_raw_buffer_store_b128(
-              rows[r], ro, to[r] + j * 32 * a.N, 0, 0);
+              rows[r], ro, to[r] + j * 32 * N, 0, 0);
       };
 #pragma unroll
       for (int j = 0; j < FM; j++) {
@@ -429,8 +436,8 @@ KAITO_DEV void stream(const GemmArgs& a, short* lds, Next&& next) {
           if constexpr (F32) {
             __builtin_amdgcn_raw_buffer_store_b128(
                 __builtin_bit_cast(u32x4, v), ro,
-                c0 + i * 16 < a.N
-                    ? ((j * 16 + lo) * a.N + i * 16 + 4 * hi) * 4 : BEYOND,
+                c0 + i * 16 < N
+                    ? ((j * 16 + lo) * N + i * 16 + 4 * hi) * 4 : BEYOND,
                 0, 0);
           } else {
             *reinterpret_cast<short4_t*>(slab + (write0 ^ i * 32)) =
@@ -452,7 +459,7 @@ KAITO_DEV void stream(const GemmArgs& a, short* lds, Next&& next) {
       }
       if constexpr (!F32) store(FM - 1);
     };
-    if (a.bias) outputs(true);
+    if (bias) outputs(true);
     else outputs(false);
     if (!more) break;
     cur = nxt;
@@ -463,6 +470,73 @@ KAITO_DEV void stream(const GemmArgs& a, short* lds, Next&& next) {
   __builtin_amdgcn_s_waitcnt(0x0070);
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
+}
+
+constexpr int NG = 4;               // column tiles that share row tiles
+constexpr int CUS = 256;            // 8 XCDs of 32
+
+// A launch of CUS workgroups, one per CU: all tiles of a product, of the shape that
+// takes least time. Of each shape: `share` tiles per XCD, `here` on this one, tile
+// i of those by number. Tiles of 256 x 256, those of a small last round in quarters,
+// or of 128 x 256, 256 x 128 or 128 x 128: a round takes, where weights and rows come
+// from the caches, about 5 (50 us at K = 2048), 3, 3 and 2 (18 us), quarters as long
+// as 128 x 128. 700 tokens by 8 experts of 2048 x 2048, up: 53, 37, 59 and 41 us; 200:
+// 34, 30, 33 and 24; 4096 tokens by 64 of 1024 x 512: 60, 56, 66 and 55.
+template <int KIND, bool TWO = false, class Large, class Wide, class Tall,
+          class Small>
+KAITO_DEV void run(const GemmArgs& a, short* lds, const Large& large,
+                   const Wide& wide, const Tall& tall, const Small& small) {
+  constexpr int workers = CUS / 8;
+  enum { LARGE, WIDE, TALL, SMALL };
+  auto rounds = [&](const int n) { return (n + workers - 1) / workers; };
+  // of n tiles, those that are cut in quarters
+  auto last = [&](const int n) {
+    const int rest = n % workers;
+    return 4 * rest > workers * (n < workers ? 2 : 1) ? 0 : rest;
+  };
+  // the same answer on all XCDs, whose tiles are numbered through
+  const int over = last(large.share);
+  int best = 5 * rounds(large.share - over) + 2 * rounds(4 * over), mode = LARGE;
+  auto other = [&](const int m, const int cost) {
+    if (cost < best) best = cost, mode = m;
+  };
+  other(WIDE, 3 * rounds(wide.share));
+  other(TALL, 3 * rounds(tall.share));
+  other(SMALL, 2 * rounds(small.share));
+  const int rest = last(large.here);
+  int i = blockIdx.x / 8;
+  auto all = [&](const auto& tiles, const int end) {
+    return [&, end](Tile& t) {
+      if (i >= end) return false;
+      t = tiles(i);
+      i += workers;
+      return true;
+    };
+  };
+  if (mode == LARGE) stream<8, 8, KIND, TWO>(a, lds, all(large, large.here - rest));
+  if (mode == WIDE) {
+    stream<4, 8, KIND, TWO>(a, lds, all(wide, wide.here));
+  } else if (mode == TALL) {
+    stream<8, 4, KIND, TWO>(a, lds, all(tall, tall.here));
+  } else {
+    i = blockIdx.x / 8;
+    const int end = mode == LARGE ? 4 * rest : small.here;
+    stream<4, 4, KIND, TWO>(a, lds, [&](Tile& t) {
+      for (; i < end; i += workers) {
+        if (mode == LARGE) {
+          t = large(large.here - rest + i / 4);
+          t.m0 += i % 4 / 2 * (large.BM / 2);
+          t.n0 += i % 2 * (large.COLS / 2);
+          if (t.m0 >= t.row_end || t.n0 >= a.N) continue;
+        } else {
+          t = small(i);
+        }
+        i += workers;
+        return true;
+      }
+      return false;
+    });
+  }
 }
 
 }  // namespace tile

@@ -1,0 +1,98 @@
+"""Linear layers of prompts on tiles (ops/csrc/tile_linear.hip): rows and columns
+that end inside a tile, few K steps, each shape of tiles and several rounds. Sums
+of K f32 products, rounded to bf16 once: half a unit of the 8 bits, and where a sum
+cancels the f32 rounding of its terms."""
+import pytest
+import torch
+
+from kaito_amd import ops
+
+DEV = "cuda"
+
+
+def _rand(*shape, std=1.0):
+    return (std * torch.randn(*shape, device=DEV)).to(torch.bfloat16)
+
+
+def _close(out, ref):
+    assert torch.isfinite(out).all()
+    err = (out.double() - ref).abs()
+    rms = ref.square().mean().sqrt()
+    assert (err <= 2.0 ** -8 * ref.abs() + 2.0 ** -12 * rms).all(), err.max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [
+    (1, 64, 64), (127, 192, 128), (257, 320, 192), (300, 2048, 320),
+    (1000, 1408, 576), (2050, 2112, 448), (4200, 1600, 256)])
+def test_swiglu(M, N, K):
+    torch.manual_seed(M)
+    x, w = _rand(M, K), _rand(2 * N, K, std=K ** -0.5)
+    out = torch.full((M, N), float("nan"), device=DEV).to(torch.bfloat16)
+    ops._K.tile_swiglu(out, x, w)
+    g, u = (x.double() @ w.double().T).chunk(2, -1)
+    _close(out, g * torch.sigmoid(g) * u)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,N2,K,b,b2", [
+    (1, 256, 64, 64, True, False), (130, 512, 576, 320, False, True),
+    (1000, 3072, 576, 192, True, True), (3001, 768, 1088, 128, False, False),
+    (5000, 2048, 2048, 256, False, True)])
+@pytest.mark.parametrize("one", [True, False])
+def test_pair(M, N, N2, K, b, b2, one):
+    torch.manual_seed(M)
+    x = _rand(M, K)
+    x2 = x if one else _rand(M, K)
+    w, w2 = _rand(N, K, std=K ** -0.5), _rand(N2, K, std=K ** -0.5)
+    none = torch.empty(0, device=DEV)
+    bias, bias2 = _rand(N) if b else none, _rand(N2) if b2 else none
+    out, out2 = (torch.full((M, n), float("nan"), device=DEV).to(torch.bfloat16)
+                 for n in (N, N2))
+    ops._K.tile_pair(out, x, w, bias, out2, x2, w2, bias2)
+    _close(out, x.double() @ w.double().T + (bias.double() if b else 0))
+    _close(out2, x2.double() @ w2.double().T + (bias2.double() if b2 else 0))
+
+
+@pytest.mark.gpu
+def test_forms_that_tiles_do_not_take():
+    """Strided, misaligned and differentiated operands give what they gave."""
+    torch.manual_seed(0)
+    M, N, K = 1100, 1024, 256
+    big, wide = _rand(M, K + 8), _rand(2 * N * K + 8)
+    w = wide[:-8].view(2 * N, K)
+    forms = [(big[:, 8:], w), (big[:, :K].t().contiguous().t(), w),
+             (big[:, :K].contiguous(), wide[4:-4].view(2 * N, K)),
+             (big[:, :K].contiguous(), w)]
+    for x, v in forms:
+        g, u = (x.double() @ v.double().T).chunk(2, -1)
+        ref = g * torch.sigmoid(g) * u
+        out = ops.linear_swiglu(x, v)
+        # gate and up are rounded too where the library makes them
+        assert (out.double() - ref).norm() <= 2.0 ** -7 * ref.norm()
+        a, b = ops.linear_pair(x, v[:N], x, v[N:])
+        assert (a.double() - g).norm() <= 2.0 ** -8 * g.norm()
+        assert (b.double() - u).norm() <= 2.0 ** -8 * u.norm()
+    x = forms[-1][0].requires_grad_()
+    ops.linear_pair(x, w[:N], x, w[N:])[0].sum().backward()
+    assert x.grad is not None
+
+
+@pytest.mark.parametrize("M,N,K,tiles", [
+    (256, 28672, 4096, False), (512, 28672, 4096, True),
+    (700, 28672, 4096, False), (8192, 28672, 4096, True),
+    (1000, 22016, 4096, False), (1500, 16384, 3072, False),
+    (700, 4096, 2048, False), (1000, 4096, 2048, True),
+    (1500, 1024, 2048, False), (2048, 1024, 2048, False)])
+def test_which_pairs_take_tiles(M, N, K, tiles):
+    """The sides of the line on which either was measured to be faster."""
+    assert ops._tiled_shape(M, N, K) == tiles
+
+
+@pytest.mark.parametrize("M,N,K,tiles", [
+    (127, 3648, 2048, False), (128, 3648, 2048, True),
+    (8192, 3648, 2048, True), (3000, 7168, 2048, False),
+    (6500, 7168, 2048, True), (8192, 2624, 2048, False),
+    (1000, 2112, 7168, False)])
+def test_which_two_products_take_tiles(M, N, K, tiles):
+    assert ops._pair_tiled_shape(M, N, K) == tiles
