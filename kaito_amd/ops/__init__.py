@@ -30,7 +30,7 @@ for _g, _names in {
              "gelu_and_mul gelu layer_norm fused_add_layer_norm "
              "rope_and_cache reshape_and_cache topk skinny_linear skinny_norm skinny_swiglu "
              "skinny_linear_pair batch_linear batch_parts add_rms_norm_parts "
-             "tile_swiglu tile_pair"),
+             "tile_linear tile_swiglu tile_pair"),
     "attn": ("paged_attention paged_attention_sp rope_paged_attention "
              "prefill_attention "
              "mla_prefill_attention context_attention mfma_tile_gemm paged_read_bw"),
@@ -344,6 +344,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
             else:
                 _K.batch_linear(out, x, w, _none(bias, x), 0, 0, False)
             return out
+    if bias is None and w.dim() == 2 and x.dim() == 2 \
+            and _vocabulary_shape(x.size(0), *w.shape) \
+            and _tiles_fit(x, w, 64):
+        out = torch.empty(x.size(0), w.size(0), dtype=x.dtype, device=x.device)
+        _K.tile_linear(out, x, w)
+        return out
     return torch.nn.functional.linear(x, w, bias)
 
 
@@ -464,6 +470,18 @@ def _tiled_shape(M: int, N: int, K: int) -> bool:
         return False
     fill = _tile_fill(M, N)
     return fill >= 0.82 or (K <= 2048 and M >= 1000 and fill >= 0.42)
+
+
+def _vocabulary_shape(M: int, N: int, K: int) -> bool:
+    """Whether a large batch's logits run on the tiles, whose 256 rows are a
+    step's (us, library and tiles: 128256 x 4096 297, 234 at 129 rows, 262, 241 at
+    192, 310, 246 at 256; 151936 x 4096 309, 292 at 129, 363, 321 at 256; 256000 x
+    4096 553, 477; 128256 x 8192 464, 450 at 160, 548, 472 at 256; 128256 x 6144
+    351, 341 at 144, 448, 361 at 256; 131072 x 5120 279, 294 at 144, 338, 313 at
+    256. Fewer rows or a shorter K went either way: 262144 x 2304 0.94 to 0.98,
+    151936 x 4096 1.0 to 1.02 from 33 to 64 rows, 128256 x 8192 0.94 to 1.02)."""
+    return 129 <= M <= 256 and N >= 100000 and K >= 4096 \
+        and (M > 224 or not 4096 < K < 6144)
 
 
 def _pair_tiled(x, w, x2, w2) -> bool:

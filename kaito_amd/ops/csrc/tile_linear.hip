@@ -1,5 +1,6 @@
 // Linear layers of prompts on the tiles of tile_gemm.h:
 //
+//   tile_linear   out = x W^T, for vocabularies
 //   tile_swiglu   out = silu(x Wg^T) (x Wu^T) of W = [Wg | Wu]
 //   tile_pair     out = x W^T (+ bias), out2 = x2 W2^T (+ bias2): one launch, whose
 //                 last round of tiles is not each product's own
@@ -91,6 +92,12 @@ static void launch(const GemmArgs& a, int64_t T) {
                      at::hip::getCurrentHIPStream(), a, (int)T);
 }
 
+void tile_linear(at::Tensor out, at::Tensor x, at::Tensor w) {
+  GemmArgs a = tile_args(out, x, w, out.size(1));
+  a.n2 = a.N;                       // no second product
+  launch<tile::PLAIN, true>(a, x.size(0));
+}
+
 // w [2 N, K]
 void tile_swiglu(at::Tensor out, at::Tensor x, at::Tensor w) {
   launch<tile::SILU, false>(tile_args(out, x, w, 2 * out.size(1)), x.size(0));
@@ -117,10 +124,12 @@ void tile_pair(at::Tensor out, at::Tensor x, at::Tensor w, at::Tensor bias,
 }  // namespace kaito
 
 TORCH_LIBRARY_FRAGMENT(kaito, m) {
+  m.def("tile_linear(Tensor(a!) out, Tensor x, Tensor w) -> ()");
   m.def("tile_swiglu(Tensor(a!) out, Tensor x, Tensor w) -> ()");
   m.def("tile_pair(Tensor(a!) out, Tensor x, Tensor w, Tensor bias, Tensor(b!) out2, Tensor x2, Tensor w2, Tensor bias2) -> ()");
 }
 TORCH_LIBRARY_IMPL(kaito, CUDA, m) {
+  m.impl("tile_linear", &kaito::tile_linear);
   m.impl("tile_swiglu", &kaito::tile_swiglu);
   m.impl("tile_pair", &kaito::tile_pair);
 }

@@ -35,6 +35,17 @@ def test_swiglu(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 64, 64), (250, 4160, 448),
+                                   (129, 33024, 192), (600, 2112, 320)])
+def test_linear(M, N, K):
+    torch.manual_seed(M)
+    x, w = _rand(M, K), _rand(N, K, std=K ** -0.5)
+    out = torch.full((M, N), float("nan"), device=DEV).to(torch.bfloat16)
+    ops._K.tile_linear(out, x, w)
+    _close(out, x.double() @ w.double().T)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,N2,K,b,b2", [
     (1, 256, 64, 64, True, False), (130, 512, 576, 320, False, True),
     (1000, 3072, 576, 192, True, True), (3001, 768, 1088, 128, False, False),
@@ -96,3 +107,12 @@ def test_which_pairs_take_tiles(M, N, K, tiles):
     (1000, 2112, 7168, False)])
 def test_which_two_products_take_tiles(M, N, K, tiles):
     assert ops._pair_tiled_shape(M, N, K) == tiles
+
+
+@pytest.mark.parametrize("M,N,K,tiles", [
+    (128, 128256, 4096, False), (129, 128256, 4096, True),
+    (256, 128256, 4096, True), (257, 128256, 4096, False),
+    (144, 131072, 5120, False), (256, 131072, 5120, True),
+    (256, 262144, 2304, False), (200, 32000, 4096, False)])
+def test_which_vocabularies_take_tiles(M, N, K, tiles):
+    assert ops._vocabulary_shape(M, N, K) == tiles
