@@ -12,7 +12,13 @@
 //     LDS by 16-byte direct loads and comes back by transposing reads.
 // P enters as the sum of three bf16 terms, which hold every bit of the f32
 // weight (two of them 16 of its 24). fp8 (e4m3) pages are widened to bf16,
-// exactly, on the way. The waves of a workgroup, and with SPLIT the
+// exactly, on the way: by pairs straight to bf16, 16 bytes a load (dims of K permuted
+// to match, with q's), V through registers a tile ahead. By way of f32, 8 bytes a
+// load and V asked for at the head of its own tile: 250 rows of 200 to 400 keys 48.9
+// us, now 42.9; 64 of 700 to 1400 34.9, 31.7; 16 of 2050 to 4100 30.8, 28.2. bf16
+// pages are bound by memory (57 us alone for the first, 66 here): the table and K
+// ahead of q's rotation and the row's own key from registers changed nothing there,
+// and cost 0.7 us of 8 where the code is fetched anew for every launch. The waves of a workgroup, and with SPLIT the
 // workgroups of a (sequence, kv head), hold partial (max, sum, O) that are
 // folded at the end.
 //
@@ -55,6 +61,7 @@ namespace {
 
 using flash::hbf16x8;
 using flash::LOG2E;
+typedef uint8_t u8x16_t __attribute__((ext_vector_type(16)));
 
 constexpr int BS = 16;              // tokens per page
 constexpr int KT = 32;              // keys per wave step: two pages
@@ -102,12 +109,22 @@ KAITO_DEV int place_v(const int row, const int c) {
   else return c ^ ((row & 7) << 1);
 }
 
-KAITO_DEV hbf16x8 widen8(const u8x8_t raw) {
-  float f[8];
-  fp8x8_to_f32(raw, f);
+// eight of 16 e4m3 as bf16, exactly: half 0 the first, 1 the last
+KAITO_DEV hbf16x8 widen8(const u8x16_t raw, const int half) {
+  typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
+  typedef __bf16 hbf16x2 __attribute__((ext_vector_type(2)));
+  const u32x4 u = __builtin_bit_cast(u32x4, raw);
   hbf16x8 w;
 #pragma unroll
-  for (int e = 0; e < 8; e++) w[e] = (__bf16)f[e];
+  for (int i = 0; i < 2; i++) {
+    const unsigned x = u[2 * half + i];
+    const hbf16x2 a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x, 1.f, false);
+    const hbf16x2 b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x, 1.f, true);
+    w[4 * i] = a[0];
+    w[4 * i + 1] = a[1];
+    w[4 * i + 2] = b[0];
+    w[4 * i + 3] = b[1];
+  }
   return w;
 }
 
@@ -207,6 +224,12 @@ void paged_decode_kernel(const DecodeArgs a) {
   constexpr int DT = D / 16;        // 16-row tiles of O^T
   constexpr int CV = D / 8;         // 16-byte chunks of a V row
   constexpr int LV = KT * CV / 64;  // V chunks per lane and tile
+  // Dims of a lane in product step kk: 8 from d0 + step_dim(kk) on. fp8 rows of 128
+  // dims and more: those of two steps are one load of 16 bytes
+  constexpr bool QUADS = FP8 && D >= 128;
+  auto step_dim = [](const int kk) {
+    return QUADS ? kk / 2 * 64 + kk % 2 * 8 : kk * 32;
+  };
   __shared__ __attribute__((aligned(128))) short lds_v[NW][KT * D];
   __shared__ float s_m[NW][16], s_l[NW][16];
   // BIASED: penalties of a wave's tile, heads by keys
@@ -237,6 +260,7 @@ void paged_decode_kernel(const DecodeArgs a) {
   const int t1 = min(sp.tiles, t0 + sp.per);
   const int last_page = (seq_len - 1) / BS;
 
+  const int d0 = hi * (QUADS ? 16 : 8);
   hbf16x8 qf[KK];
   {
     const short* qp = a.q + (int64_t)seq * a.q_stride +
@@ -244,7 +268,7 @@ void paged_decode_kernel(const DecodeArgs a) {
 #pragma unroll
     for (int kk = 0; kk < KK; kk++)
       qf[kk] = *reinterpret_cast<const hbf16x8*>(
-          qp + min(lo, a.G - 1) * D + hi * 8 + kk * 32);
+          qp + min(lo, a.G - 1) * D + d0 + step_dim(kk));
   }
   if constexpr (ROPE) {
     const float* cs = a.cos_sin + a.positions[seq] * D;
@@ -253,7 +277,7 @@ void paged_decode_kernel(const DecodeArgs a) {
       append_row<D, FP8>(a, seq, kvh, cs, lane);
 #pragma unroll
     for (int kk = 0; kk < KK / 2; kk++)
-      rotate8(qf[kk], qf[kk + KK / 2], cs + hi * 8 + kk * 32, D / 2);
+      rotate8(qf[kk], qf[kk + KK / 2], cs + d0 + step_dim(kk), D / 2);
   }
   constexpr float NONE = BIASED ? -INFINITY : -1e30f;
   float m = NONE, l = 0.f;
@@ -287,22 +311,43 @@ void paged_decode_kernel(const DecodeArgs a) {
     return ((int64_t)page * a.KH + kvh) * BS;
   };
   hbf16x8 kf[2][KK];
-  u8x8_t k8[FP8 ? 2 : 1][FP8 ? KK : 1];
+  u8x16_t k8[FP8 ? 2 : 1][FP8 ? KK / 2 : 1];
   auto load_k = [&](const int64_t r0, const int64_t r1) {
 #pragma unroll
     for (int i = 0; i < 2; i++) {
       // uniform page address, 32-bit lane offset
       const int64_t at = (i ? r1 : r0) * D;
-      const uint32_t off = lo * D + hi * 8;
+      const uint32_t off = lo * D + d0;
+      if constexpr (FP8) {
 #pragma unroll
-      for (int kk = 0; kk < KK; kk++) {
-        if constexpr (FP8)
-          k8[i][kk] = *reinterpret_cast<const u8x8_t*>(
-              (const uint8_t*)a.k + at + (off + kk * 32));
-        else
+        for (int kk = 0; kk < KK; kk += 2) {
+          const uint8_t* k = (const uint8_t*)a.k + at + (off + step_dim(kk));
+          if constexpr (QUADS) {
+            k8[i][kk / 2] = *reinterpret_cast<const u8x16_t*>(k);
+          } else {
+            const u8x8_t x = *reinterpret_cast<const u8x8_t*>(k);
+            const u8x8_t y = *reinterpret_cast<const u8x8_t*>(k + step_dim(1));
+            k8[i][kk / 2] = __builtin_shufflevector(
+                x, y, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int kk = 0; kk < KK; kk++)
           kf[i][kk] = *reinterpret_cast<const hbf16x8*>(
-              (const short*)a.k + at + (off + kk * 32));
+              (const short*)a.k + at + (off + step_dim(kk)));
       }
+    }
+  };
+  // fp8: V of the tile at r0 and r1, a tile ahead; 16 bytes are two chunks of a row
+  u8x16_t v8[FP8 ? LV / 2 : 1];
+  auto load_v8 = [&](const int64_t r0, const int64_t r1) {
+#pragma unroll
+    for (int j = 0; j < LV / 2; j++) {
+      const int s = (j * 64 + lane) * 2;
+      const int64_t at = (j * 128 / CV < BS ? r0 : r1) * D;
+      v8[j] = *reinterpret_cast<const u8x16_t*>(
+          (const uint8_t*)a.v + at + (uint32_t)(s / CV % BS * D + s % CV * 8));
     }
   };
 
@@ -314,21 +359,19 @@ void paged_decode_kernel(const DecodeArgs a) {
       row0 = page_row(base / BS + t0 * 2);
       row1 = page_row(base / BS + t0 * 2 + 1);
       load_k(row0, row1);
+      if constexpr (FP8) load_v8(row0, row1);
     }
     for (int t = t0; t < t1; t++) {
       // ---- V of this tile: slot j * 64 + lane is row s / CV, place s % CV
-      u8x8_t v8[FP8 ? LV : 1];
+      if constexpr (!FP8) {
 #pragma unroll
-      for (int j = 0; j < LV; j++) {
-        const int row = j * (64 / CV) + lane / CV;
-        const int64_t at = (j * (64 / CV) < BS ? row0 : row1) * D;
-        const uint32_t off =
-            row % BS * D + place_v<D>(row, lane % CV) * 8;
-        if constexpr (FP8)
-          v8[j] = *reinterpret_cast<const u8x8_t*>(
-              (const uint8_t*)a.v + at + off);
-        else
+        for (int j = 0; j < LV; j++) {
+          const int row = j * (64 / CV) + lane / CV;
+          const int64_t at = (j * (64 / CV) < BS ? row0 : row1) * D;
+          const uint32_t off =
+              row % BS * D + place_v<D>(row, lane % CV) * 8;
           flash::lds_copy16((const short*)a.v + at + off, vl + j * 512);
+        }
       }
       // ---- S^T: keys 16 i + 4 hi + r of head lo
       f32x4 s[2];
@@ -337,7 +380,7 @@ void paged_decode_kernel(const DecodeArgs a) {
         s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kk = 0; kk < KK; kk++) {
-          if constexpr (FP8) kf[i][kk] = widen8(k8[i][kk]);
+          if constexpr (FP8) kf[i][kk] = widen8(k8[i][kk / 2], kk & 1);
           s[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[i][kk], qf[kk],
                                                          s[i], 0, 0, 0);
         }
@@ -412,8 +455,15 @@ void paged_decode_kernel(const DecodeArgs a) {
         }
       if constexpr (FP8) {
 #pragma unroll
-        for (int j = 0; j < LV; j++)
-          *reinterpret_cast<hbf16x8*>(vl + (j * 64 + lane) * 8) = widen8(v8[j]);
+        for (int j = 0; j < LV / 2; j++) {
+          const int s0 = (j * 64 + lane) * 2, row = s0 / CV;
+#pragma unroll
+          for (int h = 0; h < 2; h++)
+            *reinterpret_cast<hbf16x8*>(
+                vl + row * D + place_v<D>(row, s0 % CV + h) * 8) =
+                widen8(v8[j], h);
+        }
+        if (t + 1 < t1) load_v8(row0, row1);
       } else {
         // the direct loads' data: this wave's own, so no barrier
         __builtin_amdgcn_s_waitcnt(0x0f70);     // vmcnt(0)

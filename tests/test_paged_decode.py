@@ -247,3 +247,20 @@ def test_rotations_at_any_address():
             pos, q, k, v, D, cs, *(c.clone() for c in caches), slots, bt, sl,
             D ** -0.5))
     assert torch.equal(*outs)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_codes_are_widened_exactly(D):
+    """One key per row weighs 1: the output is its value, whatever its code."""
+    T = 256 // D
+    codes = torch.arange(256, dtype=torch.uint8).view(T, 1, 1, D)
+    kc = torch.full((T, 1, 16, D), 0x38, dtype=torch.uint8)     # 1.0
+    vc = torch.zeros(T, 1, 16, D, dtype=torch.uint8)
+    vc[:, :, :1] = codes
+    bt, sl = torch.arange(T, dtype=torch.int32).view(T, 1), torch.ones(T)
+    out = ops.paged_attention(
+        torch.randn(T, 1, D, dtype=torch.bfloat16, device=DEV), kc.to(DEV),
+        vc.to(DEV), bt.to(DEV), sl.int().to(DEV), D ** -0.5)
+    want = codes.view(torch.float8_e4m3fn).float().view(T, 1, D)
+    assert torch.equal(out.cpu().float().nan_to_num(1e9), want.nan_to_num(1e9))
