@@ -316,11 +316,8 @@ class LlamaDecoderLayer(nn.Module):
         """qkv of the input norm's rows, and the residual, or None."""
         if not self._takes_norm(self.self_attn, LlamaAttention, hidden):
             return None
-        p = self.self_attn.qkv_proj
-        if not p.norms(hidden, residual, self.input_layernorm):
-            return None
-        return ops.add_norm_linear(hidden, residual, self.input_layernorm,
-                                   self.cfg.rms_eps, p.weight, p.bias)
+        return self.self_attn.qkv_proj.norm_linear(
+            hidden, residual, self.input_layernorm, self.cfg.rms_eps)
 
     def _norm_act(self, hidden, residual):
         """The MLP's inner rows of the norm's, and the residual, or None."""

@@ -40,7 +40,7 @@ for _g, _names in {
             "latent_kv"),
     "route": "moe_route moe_gate_route moe_norm_gate_route moe_sort",
     "quant": ("w4a16_gemv w4a16_dequant w4a16_gemm w4a16_swiglu "
-              "w4a16_norm_swiglu "
+              "w4a16_norm_swiglu w4a16_norm_linear w4a16_norm_in_tiles "
               "w4a16_in_tiles lora_shrink lora_expand"),
     "comm": ("allreduce_rmsnorm one_shot_ar_rmsnorm ipc_handle ipc_open "
              "ipc_close"),
@@ -1204,12 +1204,8 @@ def w4a16_norm_swiglu(x, residual, norm, eps: float, qweight, scales, zeros,
                       group: int):
     """w4a16_swiglu of fused_add_rms_norm's rows and its residual, of 1 and 2
     rows in one launch; None for other sizes."""
-    if not (x.is_cuda and x.dim() == 2 and 1 <= x.size(0) <= 2
-            and x.dtype == torch.bfloat16 and x.data_ptr() % 16 == 0
-            and qweight.size(0) % 2 == 0 and qweight.data_ptr() % 16 == 0
-            and _norm_rows(x, residual, norm)
-            and not (torch.is_grad_enabled() and x.requires_grad)
-            and not _transformed()
+    if not (_packed_norm_rows(x, residual, norm, qweight)
+            and qweight.size(0) % 2 == 0
             and _K.w4a16_in_tiles(x.size(0), qweight.size(0), x.size(1), group,
                                   True)):
         return None
@@ -1218,6 +1214,33 @@ def w4a16_norm_swiglu(x, residual, norm, eps: float, qweight, scales, zeros,
     stream = torch.empty_like(x)
     _K.w4a16_norm_swiglu(out, stream, x, residual, norm, eps, qweight, scales,
                          zeros, group)
+    return out, stream
+
+
+def _packed_norm_rows(x, residual, norm, qweight) -> bool:
+    """Rows that a product with packed weights can norm on the way."""
+    return x.is_cuda and x.dim() == 2 and 1 <= x.size(0) <= 2 \
+        and x.dtype == torch.bfloat16 and x.data_ptr() % 16 == 0 \
+        and qweight.data_ptr() % 16 == 0 and _norm_rows(x, residual, norm) \
+        and not (torch.is_grad_enabled() and x.requires_grad) \
+        and not _transformed()
+
+
+def w4a16_norm_linear(x, residual, norm, eps: float, qweight, scales, zeros,
+                      group: int, glu: bool = False):
+    """w4a16_gemv (glu: SwiGLU of the pair) of fused_add_rms_norm's rows and its
+    residual, of 1 and 2 rows in one launch; None for other sizes."""
+    if not (_packed_norm_rows(x, residual, norm, qweight)
+            and qweight.is_contiguous() and scales.is_contiguous()
+            and zeros.is_contiguous() and qweight.size(0) % (2 if glu else 1) == 0
+            and _K.w4a16_norm_in_tiles(x.size(0), qweight.size(0), x.size(1),
+                                       group, glu)):
+        return None
+    out = torch.empty(x.size(0), qweight.size(0) // (2 if glu else 1),
+                      dtype=x.dtype, device=x.device)
+    stream = torch.empty_like(x)
+    _K.w4a16_norm_linear(out, stream, x, residual, norm, eps, qweight, scales,
+                         zeros, group, glu)
     return out, stream
 
 

@@ -121,9 +121,15 @@ __global__ __launch_bounds__(256) void w4a16_mfma_kernel(
 // Bound by the chain of a tile, with two waves per SIMD to cover it: wait, unpack
 // (232 vector instructions per stage), multiply, meet at a barrier, sum. 28672 x
 // 4096, 2 rows: vector unit busy 31 %, matrix cores 9, LDS 16, 3.8 TB/s; of the
-// waves' time 38 % waits for loads and barriers, 30 for issue. The time hardly grows
+// waves' time 38 % waits for loads and barriers, 30 for issue. Hence, from 512 tiles
+// on, two workgroups of four waves per CU, whose barriers do not meet: 12288 x 4096,
+// 2 rows, 10.4 -> 9.2 us, 28672 x 2560 13.2 -> 11.5, as a pair 28672 x 4096 15.9 ->
+// 14.8, with the norm 16.8 -> 15.6 (57344 x 8192 44.6 both; fewer tiles the same or
+// slower). x is asked for ahead of the weights, behind which its loads would end:
+// 4096 x 14336 11.2 -> 9.7, 28672 x 4096 as a pair, 5 rows, 17.3 -> 16.0. The wave
+// that sums by turns: no change. The time hardly grows
 // with the rows. us, rows streamed (5 rows and more: MFMA from global memory) and
-// now, at 1, 2, 3, 4, 8 rows: 28672 x 4096 15.8 19.7 23.6 33.2 37.7 and 16.7 17.4
+// tiles before these two, at 1, 2, 3, 4, 8 rows: 28672 x 4096 15.8 19.7 23.6 33.2 37.7 and 16.7 17.4
 // 17.4 17.5 18.3; 4096 x 14336 11.4 13.8 and 11.7 11.7 (more rows do not fit); 4096 x
 // 4096 4.6 5.7 7.9 8.8 8.7 and 5.9 6.1 6.6 7.0 7.9. Four waves: 20.5 at 2 rows; sums
 // of two tiles at a time: no change.
@@ -131,16 +137,15 @@ namespace {
 
 constexpr int W4_K = 512;           // k of a stage
 constexpr int W4_STAGE = 16 * W4_K / 2 + 2 * 256;
-constexpr int W4_LDS = 160 * 1024;
-constexpr int W4_WAVES = 8;
+constexpr int W4_LDS = 160 * 1024;  // for 8 waves; for 4 half of it
 
 // bytes behind the rings: sums over the waves (twice), sums of x, x
-__host__ __device__ constexpr int w4_red(int mr) {
-  return W4_WAVES * mr * 4 * 16;
+__host__ __device__ constexpr int w4_red(int waves, int mr) {
+  return waves * mr * 4 * 16;
 }
-inline int64_t w4_lds(int depth, int mr, int64_t M, int64_t K) {
-  return W4_WAVES * depth * W4_STAGE + 2 * w4_red(mr) + K / 128 * mr * 4 +
-         M * (K * 2 + 16);
+inline bool w4_fits(int waves, int depth, int mr, int64_t M, int64_t K) {
+  return waves * depth * W4_STAGE + 2 * w4_red(waves, mr) + K / 128 * mr * 4 +
+         M * (K * 2 + 16) <= W4_LDS * waves / 8;
 }
 
 KAITO_DEV __amdgpu_buffer_rsrc_t w4_buffer(const void* p,
@@ -157,14 +162,15 @@ struct W4Norm {
   float eps;
 };
 constexpr int W4_NORM = 4;
+constexpr int W4_AHEAD = 8;         // 16-byte parts of x that a thread asks for first
 
 // MR: rows of x that have a place (4 or 16); GLU: N gate rows, then N up rows.
 // NORM: four waves norm a row each workgroup for itself, as the norm's kernel does
 // and to the same bits, while the first weights are on the way; its launch is
 // saved: us, two launches and one, 28672 x 4096 20.1, 17.7 for two rows, 22016 x
 // 5120 21.4, 19.1 for one and 22.2, 19.6, 57344 x 8192 48.2, 44.3 and 53.9, 47.0.
-template <int MR, int DEPTH, bool GLU, bool NORM>
-__global__ __launch_bounds__(64 * W4_WAVES) void w4a16_tiles_kernel(
+template <int NW, int MR, int DEPTH, bool GLU, bool NORM>
+__global__ __launch_bounds__(64 * NW, 2) void w4a16_tiles_kernel(
     short* __restrict__ out, const short* __restrict__ x,
     const uint32_t* __restrict__ qw, const float* __restrict__ scales,
     const float* __restrict__ zeros, const int M, const int N, const int K,
@@ -172,16 +178,16 @@ __global__ __launch_bounds__(64 * W4_WAVES) void w4a16_tiles_kernel(
   using skinny::hbf16x8;
   typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
   constexpr int COLS = GLU ? 8 : 16, LOADS = 6, USED = MR * 4;
-  __shared__ __attribute__((aligned(128))) char lds[W4_LDS];
+  __shared__ __attribute__((aligned(128))) char lds[W4_LDS * NW / 8];
   const int lane = threadIdx.x & 63, lo = lane & 15, hi = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   char* ring = lds + wave * DEPTH * W4_STAGE;
-  f32x4* red = reinterpret_cast<f32x4*>(lds + W4_WAVES * DEPTH * W4_STAGE);
+  f32x4* red = reinterpret_cast<f32x4*>(lds + NW * DEPTH * W4_STAGE);
   float* xs = reinterpret_cast<float*>(
-      lds + W4_WAVES * DEPTH * W4_STAGE + 2 * w4_red(MR));     // [K / 128][MR]
+      lds + NW * DEPTH * W4_STAGE + 2 * w4_red(NW, MR));     // [K / 128][MR]
   short* xl = reinterpret_cast<short*>(xs + K / 128 * MR);  // [M][K + 8]
   const int ntiles = N / COLS, nst = K / W4_K;
-  const int spt = (nst + W4_WAVES - 1) / W4_WAVES;  // stages of a wave and tile
+  const int spt = (nst + NW - 1) / NW;  // stages of a wave and tile
   if ((int)blockIdx.x >= ntiles) return;
 
   auto n_of = [&](const int r) {    // row of W of row r of tile 0
@@ -198,10 +204,10 @@ __global__ __launch_bounds__(64 * W4_WAVES) void w4a16_tiles_kernel(
   auto fetch = [&](const int slot) {
     // past the last stage: loads of nothing, so that the waits stay counts
     const uint32_t all = __builtin_amdgcn_readfirstlane(
-        ft < ntiles && fs * W4_WAVES + wave < nst ? 0xffffffff : 0);
+        ft < ntiles && fs * NW + wave < nst ? 0xffffffff : 0);
     const auto wr = w4_buffer(qw, all), sr = w4_buffer(scales, all),
                zr = w4_buffer(zeros, all);
-    const int k = (fs * W4_WAVES + wave) * W4_K;
+    const int k = (fs * NW + wave) * W4_K;
     const uint32_t row = ft * COLS;
     const uint32_t at = __builtin_amdgcn_readfirstlane(row * (K / 2) + k / 2);
     const uint32_t sat =
@@ -222,75 +228,105 @@ __global__ __launch_bounds__(64 * W4_WAVES) void w4a16_tiles_kernel(
       ft += gridDim.x;
     }
   };
-  const int nm = wave / 4, nat = (threadIdx.x & 255) * 8;     // row, first k
-  short8_t nv[NORM ? W4_NORM : 1], nr[NORM ? W4_NORM : 1],
+  // four waves norm a row, of four waves both rows one behind the other
+  constexpr int NR = NORM ? 8 / NW : 1;
+  const int nm = wave / 4 * NR, nat = (threadIdx.x & 255) * 8;  // row, first k
+  short8_t nv[NR][NORM ? W4_NORM : 1], nr[NR][NORM ? W4_NORM : 1],
       ng[NORM ? W4_NORM : 1];
-  if constexpr (NORM) {             // ahead of the weights: loads end in order
-    const int64_t row = (int64_t)min(nm, M - 1) * K;
+  hbf16x8 xv[NORM ? 1 : W4_AHEAD];
+  // x ahead of the weights: loads end in order
+  if constexpr (NORM) {
 #pragma unroll
     for (int i = 0; i < W4_NORM; i++) {
       const int k = i * 2048 + nat;
       if (k >= K) break;            // uniform in a wave: K is whole stages
-      nv[i] = *reinterpret_cast<const short8_t*>(x + row + k);
-      nr[i] = *reinterpret_cast<const short8_t*>(norm.residual + row + k);
+#pragma unroll
+      for (int r = 0; r < NR; r++) {
+        const int64_t row = (int64_t)min(nm + r, M - 1) * K;
+        nv[r][i] = *reinterpret_cast<const short8_t*>(x + row + k);
+        nr[r][i] =
+            *reinterpret_cast<const short8_t*>(norm.residual + row + k);
+      }
       ng[i] = *reinterpret_cast<const short8_t*>(norm.g + k);
     }
-    __builtin_amdgcn_sched_barrier(0);
+  } else {
+#pragma unroll
+    for (int i = 0; i < W4_AHEAD; i++)
+      xv[i] = skinny::load_x(
+          x + min(i * 64 * NW + (int)threadIdx.x, M * K / 8 - 1) * 8);
   }
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int i = 0; i < DEPTH; i++) fetch(i);
 
   // ---- x and its sums over the groups; 16 threads have a group
   if constexpr (NORM) {
     float* const rn = reinterpret_cast<float*>(red);
-    float ss = 0.f;
 #pragma unroll
-    for (int i = 0; i < W4_NORM; i++) {
-      if (i * 2048 + nat >= K) break;
+    for (int r = 0; r < NR; r++) {
+      float ss = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; e++) {
-        nv[i][e] = f32_to_bf16(bf16_to_f32(nv[i][e]) + bf16_to_f32(nr[i][e]));
-        const float f = bf16_to_f32(nv[i][e]);
-        ss += f * f;
+      for (int i = 0; i < W4_NORM; i++) {
+        if (i * 2048 + nat >= K) break;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          nv[r][i][e] = f32_to_bf16(bf16_to_f32(nv[r][i][e]) +
+                                    bf16_to_f32(nr[r][i][e]));
+          const float f = bf16_to_f32(nv[r][i][e]);
+          ss += f * f;
+        }
       }
+      ss = wave_reduce_sum(ss);
+      if (lane == 0) rn[(nm + r) * 4 + wave % 4] = ss;
     }
-    ss = wave_reduce_sum(ss);
-    if (lane == 0) rn[wave] = ss;
     __builtin_amdgcn_s_waitcnt(0xc07f);       // weights stay under way
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    const float* s = rn + nm * 4;
-    const float inv =
-        rsqrtf(((s[0] + s[1]) + (s[2] + s[3])) / (float)K + norm.eps);
 #pragma unroll
-    for (int i = 0; i < W4_NORM; i++) {
-      const int k = i * 2048 + nat;
-      if (nm >= M || k >= K) break;           // uniform in a wave
-      hbf16x8 v;
+    for (int r = 0; r < NR; r++) {
+      const int m = nm + r;
+      const float* s = rn + m * 4;
+      const float inv =
+          rsqrtf(((s[0] + s[1]) + (s[2] + s[3])) / (float)K + norm.eps);
+#pragma unroll
+      for (int i = 0; i < W4_NORM; i++) {
+        const int k = i * 2048 + nat;
+        if (m >= M || k >= K) break;          // uniform in a wave
+        hbf16x8 v;
+        float sum = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          v[e] =
+              (__bf16)(bf16_to_f32(nv[r][i][e]) * inv * bf16_to_f32(ng[i][e]));
+          sum += (float)v[e];
+        }
+        sum = group_reduce_sum<16>(sum);
+        *reinterpret_cast<hbf16x8*>(xl + m * (K + 8) + k) =
+            skinny::nibble_order(v);
+        if (nat % 128 == 0) xs[k / 128 * MR + m] = sum;
+        if (blockIdx.x == 0)
+          *reinterpret_cast<short8_t*>(norm.sum + (int64_t)m * K + k) =
+              nv[r][i];
+      }
+    }
+  } else {
+    auto place = [&](const int c, const hbf16x8 v) {
+      const int m = c / (K / 8), k = c % (K / 8) * 8;
       float sum = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; e++) {
-        v[e] = (__bf16)(bf16_to_f32(nv[i][e]) * inv * bf16_to_f32(ng[i][e]));
-        sum += (float)v[e];
-      }
+      for (int e = 0; e < 8; e++) sum += (float)v[e];
       sum = group_reduce_sum<16>(sum);
-      *reinterpret_cast<hbf16x8*>(xl + nm * (K + 8) + k) =
+      *reinterpret_cast<hbf16x8*>(xl + m * (K + 8) + k) =
           skinny::nibble_order(v);
-      if (nat % 128 == 0) xs[k / 128 * MR + nm] = sum;
-      if (blockIdx.x == 0)
-        *reinterpret_cast<short8_t*>(norm.sum + (int64_t)nm * K + k) = nv[i];
-    }
-  } else for (int c = threadIdx.x; c < M * K / 8; c += 64 * W4_WAVES) {
-    const int m = c / (K / 8), k = c % (K / 8) * 8;
-    const hbf16x8 v = skinny::load_x(x + (int64_t)m * K + k);
-    float sum = 0.f;
+      if (c % 16 == 0) xs[k / 128 * MR + m] = sum;
+    };
+    int c = threadIdx.x;
 #pragma unroll
-    for (int e = 0; e < 8; e++) sum += (float)v[e];
-    sum = group_reduce_sum<16>(sum);
-    *reinterpret_cast<hbf16x8*>(xl + m * (K + 8) + k) =
-        skinny::nibble_order(v);
-    if (c % 16 == 0) xs[k / 128 * MR + m] = sum;
+    for (int i = 0; i < W4_AHEAD; i++, c += 64 * NW)
+      if (c < M * K / 8) place(c, xv[i]);     // uniform in 16 lanes
+    for (; c < M * K / 8; c += 64 * NW)
+      place(c, skinny::load_x(x + (int64_t)c * 8));
   }
   skinny::wait_loads<0>();
   __syncthreads();
@@ -303,7 +339,7 @@ __global__ __launch_bounds__(64 * W4_WAVES) void w4a16_tiles_kernel(
     f32x4 acc{0.f, 0.f, 0.f, 0.f};
     for (int st = 0; st < spt; st++) {
       skinny::wait_loads<(DEPTH - 1) * LOADS>();
-      const int k = (st * W4_WAVES + wave) * W4_K;
+      const int k = (st * NW + wave) * W4_K;
       if (k < K) {
         const char* p = ring + slot * W4_STAGE;
         const f32x4 sc = *reinterpret_cast<const f32x4*>(p + 4096 + lo * 16);
@@ -338,7 +374,7 @@ __global__ __launch_bounds__(64 * W4_WAVES) void w4a16_tiles_kernel(
       fetch(slot);
       slot = slot == DEPTH - 1 ? 0 : slot + 1;
     }
-    f32x4* sums = red + par * W4_WAVES * USED;
+    f32x4* sums = red + par * NW * USED;
     if (lane < USED) sums[wave * USED + lane] = acc;
     // own sums written, the next weights still under way; the other half of
     // red is free once all are here
@@ -348,11 +384,11 @@ __global__ __launch_bounds__(64 * W4_WAVES) void w4a16_tiles_kernel(
     if (wave == 0 && lane < USED && !(GLU && lo >= 8)) {
       f32x4 v = sums[lane];
 #pragma unroll
-      for (int w = 1; w < W4_WAVES; w++) v += sums[w * USED + lane];
+      for (int w = 1; w < NW; w++) v += sums[w * USED + lane];
       if constexpr (GLU) {
         f32x4 u = sums[lane + 8];
 #pragma unroll
-        for (int w = 1; w < W4_WAVES; w++) u += sums[w * USED + lane + 8];
+        for (int w = 1; w < NW; w++) u += sums[w * USED + lane + 8];
 #pragma unroll
         for (int r = 0; r < 4; r++) v[r] = skinny::silu(v[r]) * u[r];
       }
@@ -373,16 +409,15 @@ int w4_tiles_depth(int64_t M, int64_t rows, int64_t K, int64_t group) {
       rows * (K / 2) >= 1LL << 32)
     return 0;
   const int mr = M <= 4 ? 4 : 16;
-  return w4_lds(3, mr, M, K) <= W4_LDS ? 3
-      : w4_lds(2, mr, M, K) <= W4_LDS ? 2 : 0;
+  return w4_fits(8, 3, mr, M, K) ? 3 : w4_fits(8, 2, mr, M, K) ? 2 : 0;
 }
 
 // Whether they are faster than the row streams (from 5 rows of x on: MFMA from
 // global memory), us, streams and tiles. K = 512 S keeps S of the eight waves
 // busy.
-//   Alone: one row never; two with many weights, 4096 x 14336 13.8 and 11.7,
-// 28672 x 2560 .81 of the time, but 12288 x 2048 7.1 and 8.1, 57344 x 1024 16.9 and
-// 19.9. Three or four of a narrow K with 4096 rows of W (2048 x 2048 4.4 and 4.7,
+//   Alone: one row never; two with many weights, 4096 x 14336 13.8 and 9.7,
+// 8192 x 4096 8.1 and 7.7, 4096 x 8192 8.5 and 8.2, but 6144 x 4096 7.1 and 7.4,
+// 12288 x 2048 6.4 and 6.6, 16384 x 2048 6.9 and 7.6. Three or four of a narrow K with 4096 rows of W (2048 x 2048 4.4 and 4.7,
 // 11008 .84). More, from K of 2048 on (4096 x 1024 3.8 and 4.6 at 5, 57344 x 512 9.7
 // and 20.2), beyond 8 rows at 2048 with 6144 of W (4096: 6.1 and 6.7 at 16).
 //   A pair saves a launch. One row: few rows of W (4096 .83 to .95; 6144 x 4096
@@ -397,7 +432,7 @@ bool w4_tiles_pay(int64_t M, int64_t rows, int64_t K, bool glu) {
     return M <= 4 || K > 1024 || rows <= 4096;
   }
   if (M == 1) return false;
-  if (M == 2) return K > 2048 && rows * K >= 48 << 20;
+  if (M == 2) return K > 2048 && rows * K >= 32 << 20;
   if (M <= 4) return K > 2048 || rows >= 4096;
   return K > 2048 || (K == 2048 && (M <= 8 || rows >= 6144));
 }
@@ -413,17 +448,21 @@ bool launch_w4_tiles(at::Tensor& out, const at::Tensor& x,
   if (!depth || (uintptr_t)x.data_ptr() % 16 ||
       (uintptr_t)qweight.data_ptr() % 16)
     return false;
-  const dim3 grid(std::min(256, N / (GLU ? 8 : 16)));
-#define W4T_LAUNCH(MR_, D_)                                                   \
-  hipLaunchKernelGGL((w4a16_tiles_kernel<MR_, D_, GLU, NORM>), grid,               \
-      dim3(64 * W4_WAVES), 0,                                                 \
+  const int ntiles = N / (GLU ? 8 : 16);
+  // two workgroups of four waves per CU, where x fits twice
+  const bool two = M <= 4 && ntiles >= 512 && w4_fits(4, 3, 4, M, K);
+#define W4T_LAUNCH(NW_, MR_, D_)                                              \
+  hipLaunchKernelGGL((w4a16_tiles_kernel<NW_, MR_, D_, GLU, NORM>),           \
+      dim3(std::min(2048 / NW_, ntiles)), dim3(64 * NW_), 0,                  \
       at::hip::getCurrentHIPStream(), (short*)out.data_ptr(),                 \
       (const short*)x.data_ptr(), (const uint32_t*)qweight.data_ptr(),        \
       scales.data_ptr<float>(), zeros.data_ptr<float>(), M, N, K, norm)
-  if (M <= 4) {
-    if (depth == 3) W4T_LAUNCH(4, 3); else W4T_LAUNCH(4, 2);
+  if (two) {
+    W4T_LAUNCH(4, 4, 3);
+  } else if (M <= 4) {
+    if (depth == 3) W4T_LAUNCH(8, 4, 3); else W4T_LAUNCH(8, 4, 2);
   } else if constexpr (!NORM) {
-    if (depth == 3) W4T_LAUNCH(16, 3); else W4T_LAUNCH(16, 2);
+    if (depth == 3) W4T_LAUNCH(8, 16, 3); else W4T_LAUNCH(8, 16, 2);
   }
 #undef W4T_LAUNCH
   return true;
@@ -644,6 +683,21 @@ bool w4a16_in_tiles(int64_t M, int64_t rows, int64_t K, int64_t group,
          w4_tiles_pay(M, rows, K, glu);
 }
 
+// Whether the norm of up to two rows goes into their product in the tiles: but for
+// one row of few whole streams (us, norm and what else would follow it, and one
+// launch: one row of 6144 x 4096 8.2 and 8.7, 5120 x 2048 5.7 and 6.3, 10240 x 8192
+// 15.4 and 15.2, 7168 x 5120 11.3 and 10.3, 2048 x 1024 4.8 and 4.6, 28672 x 512 9.6
+// and 7.6; pairs 28672 x 4096 19.5 and 15.8, 57344 x 8192 48.0 and 44.6, 4096 x 512
+// 6.3 and 4.6; two rows of 6144 x 4096 10.0 and 8.8, 10240 x 8192 18.0 and 15.5,
+// 1536 x 512 5.3 and 4.6; pairs 28672 x 4096 18.1 and 16.0, 57344 x 1024 20.9 and
+// 14.1).
+bool w4a16_norm_in_tiles(int64_t M, int64_t rows, int64_t K, int64_t group,
+                         bool glu) {
+  return M <= 2 && K <= 2048 * W4_NORM &&
+         (glu || M == 2 || K % 2048 || rows >= 10240) &&
+         w4_tiles_depth(M, rows, K, group) > 0;
+}
+
 // silu(x Wg^T) * (x Wu^T) of the stacked W = [Wg | Wu]
 
 void w4a16_swiglu(at::Tensor out, at::Tensor x, at::Tensor qweight,
@@ -659,12 +713,13 @@ void w4a16_swiglu(at::Tensor out, at::Tensor x, at::Tensor qweight,
               "w4a16_swiglu: sizes of the tiles");
 }
 
-// the same of rms(x + residual) * g; sum: x + residual, not one of the others
-void w4a16_norm_swiglu(at::Tensor out, at::Tensor sum, at::Tensor x,
+// x W^T of rms(x + residual) * g (glu: the same of the pair); sum: x + residual,
+// not one of the others
+void w4a16_norm_linear(at::Tensor out, at::Tensor sum, at::Tensor x,
                        at::Tensor residual, at::Tensor g, double eps,
                        at::Tensor qweight, at::Tensor scales, at::Tensor zeros,
-                       int64_t group) {
-  const int64_t M = x.size(0), K = x.size(1);
+                       int64_t group, bool glu) {
+  const int64_t M = x.size(0), K = x.size(1), pair = glu ? 2 : 1;
   for (const auto& t : {x, residual, sum})
     TORCH_CHECK(t.is_cuda() && t.is_contiguous() && t.sizes() == x.sizes() &&
                 t.dtype() == at::kBFloat16 && (uintptr_t)t.data_ptr() % 16 == 0);
@@ -672,18 +727,28 @@ void w4a16_norm_swiglu(at::Tensor out, at::Tensor sum, at::Tensor x,
               g.dtype() == at::kBFloat16 && (uintptr_t)g.data_ptr() % 16 == 0);
   TORCH_CHECK(out.is_contiguous() && out.dtype() == at::kBFloat16 &&
               qweight.is_contiguous() && scales.is_contiguous() &&
-              zeros.is_contiguous() && qweight.size(0) % 2 == 0 &&
+              zeros.is_contiguous() && qweight.size(0) % pair == 0 &&
               qweight.size(1) * 8 == K && out.size(0) == M &&
-              out.size(1) * 2 == qweight.size(0));
+              out.size(1) * pair == qweight.size(0));
   TORCH_CHECK(M >= 1 && M <= 2 && K <= 2048 * W4_NORM &&
               sum.data_ptr() != residual.data_ptr() &&
               sum.data_ptr() != x.data_ptr());
   const W4Norm norm = {(short*)sum.data_ptr(),
                        (const short*)residual.data_ptr(),
                        (const short*)g.data_ptr(), (float)eps};
-  TORCH_CHECK((launch_w4_tiles<true, true>(out, x, qweight, scales, zeros,
-                                           group, norm)),
-              "w4a16_norm_swiglu: sizes of the tiles");
+  const bool fits = glu ? launch_w4_tiles<true, true>(out, x, qweight, scales,
+                                                      zeros, group, norm)
+                        : launch_w4_tiles<false, true>(out, x, qweight, scales,
+                                                       zeros, group, norm);
+  TORCH_CHECK(fits, "w4a16_norm_linear: sizes of the tiles");
+}
+
+void w4a16_norm_swiglu(at::Tensor out, at::Tensor sum, at::Tensor x,
+                       at::Tensor residual, at::Tensor g, double eps,
+                       at::Tensor qweight, at::Tensor scales, at::Tensor zeros,
+                       int64_t group) {
+  w4a16_norm_linear(out, sum, x, residual, g, eps, qweight, scales, zeros,
+                    group, true);
 }
 
 void w4a16_dequant(at::Tensor out, at::Tensor qweight, at::Tensor scales,

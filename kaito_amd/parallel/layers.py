@@ -111,14 +111,30 @@ class ColumnParallelLinear(_QuantMixin, nn.Module):
         return not self._quantized and self._bare() \
             and ops.norm_fits(x, residual, norm, self.weight)
 
+    def norm_linear(self, x, residual, norm, eps: float):
+        """This layer's product of the RMS norm of x + residual, and that sum, or
+        None where that is not one launch."""
+        if not self._quantized:
+            return ops.add_norm_linear(x, residual, norm, eps, self.weight,
+                                       self.bias) \
+                if self.norms(x, residual, norm) else None
+        took = ops.w4a16_norm_linear(
+            x, residual, norm, eps, self.qweight, self.scales, self.zeros,
+            self.q_group) if self._bare() else None
+        if took is not None and self.bias is not None:
+            return took[0] + self.bias, took[1]
+        return took
+
     def norm_swiglu(self, x, residual, norm, eps: float):
         """silu(gate) * up of the RMS norm of x + residual, and that sum, or
         None where that is not one launch."""
         if self.bias is not None or not self._bare():
             return None
         if self._quantized:
-            return ops.w4a16_norm_swiglu(x, residual, norm, eps, self.qweight,
-                                         self.scales, self.zeros, self.q_group)
+            args = (x, residual, norm, eps, self.qweight, self.scales,
+                    self.zeros, self.q_group)
+            took = ops.w4a16_norm_swiglu(*args)
+            return ops.w4a16_norm_linear(*args, True) if took is None else took
         if not ops.norm_fits(x, residual, norm, self.weight):
             return None
         return ops.add_norm_linear(x, residual, norm, eps, self.weight,

@@ -167,6 +167,40 @@ def test_w4_tiles(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("N,K", [(4088, 512), (4096, 512), (4112, 1024),
+                                 (8208, 4096), (4112, 5120)])
+def test_w4_tiles_of_two_workgroups(M, N, K):
+    """Around the 512 tiles from which a CU has two workgroups; waves without a
+    stage, more rows than x's room for two."""
+    torch.manual_seed(M * N + K)
+    x = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    packed = [t.to(DEV) for t in quantize_w4(torch.randn(2 * N, K), 128)]
+    w = R.w4a16_unpack(*(t.cpu() for t in packed), 128).to(DEV)
+    ref = x.double() @ w.double().T
+    g, u = ref.chunk(2, -1)
+    _close(ops.w4a16_gemv(x, *packed, 128), ref)
+    out = ops.w4a16_swiglu(x, *packed, 128)
+    if out is not None:
+        _close(out, g * torch.sigmoid(g) * u)
+    # the same rows as a norm's: the kernel's own
+    r = torch.randn(M, K, device=DEV).to(torch.bfloat16)
+    norm = torch.randn(K, device=DEV).to(torch.bfloat16)
+    y, total = ops.fused_add_rms_norm(x.clone(), r.clone(), norm, 1e-5)
+    ref = y.double() @ w.double().T
+    g, u = ref.chunk(2, -1)
+    for glu, want in ((False, ref), (True, g * torch.sigmoid(g) * u)):
+        x0, r0 = x.clone(), r.clone()
+        took = ops.w4a16_norm_linear(x, r, norm, 1e-5, *packed, 128, glu)
+        assert (took is None) == (M > 2 or (not glu and M == 1 and K % 2048 == 0
+                                            and 2 * N < 10240))
+        if took is not None:
+            _close(took[0], want)
+            assert torch.equal(took[1], total)
+            assert torch.equal(x, x0) and torch.equal(r, r0)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,rows,K,alone,pair", [
     (1, 4096, 4096, False, True), (1, 6144, 4096, False, False),
     (1, 28672, 4096, False, False), (1, 28672, 7168, False, True),
