@@ -26,7 +26,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from ..engine.config import ModelConfig
-from ..parallel.layers import untouched
+from ..parallel.layers import looks_up, untouched
 from .hybrid_base import HybridStackBase, MixerLayerBase
 from .hybrid_config import LayerSpec, layer_moe_config
 from .mixers import BiasedWindowAttention, GatedDeltaMixer, RGLRUMixer
@@ -125,9 +125,16 @@ class GurapelForCausalLM(HybridStackBase):
     def forward(self, input_ids, positions, kv_caches, meta,
                 hidden_in=None) -> torch.Tensor:
         cfg = self.cfg
-        x32 = self.embed_tokens(input_ids).float() * cfg.embed_scale \
-            + self.pos_embed[positions].float()
-        xa = x32 if cfg.dtype == torch.float32 else x32.to(cfg.dtype)
+        took = ops.embed_positions(
+            input_ids, positions, self.embed_tokens.weight, self.pos_embed,
+            cfg.embed_scale) if looks_up(self.embed_tokens) \
+            and cfg.dtype == torch.bfloat16 else None
+        if took is not None:
+            x32, xa = took
+        else:
+            x32 = self.embed_tokens(input_ids).float() * cfg.embed_scale \
+                + self.pos_embed[positions].float()
+            xa = x32 if cfg.dtype == torch.float32 else x32.to(cfg.dtype)
         for i, layer in enumerate(self.layers):
             xa = layer(x32, xa, positions, kv_caches[i], meta)
             if self.layer_hook is not None:

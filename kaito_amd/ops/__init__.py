@@ -46,6 +46,7 @@ for _g, _names in {
              "ipc_close"),
     "mix": ("causal_conv_update "
             "qk_norm_cache_write window_attention window_attention_tiles "
+            "embed_positions "
             "post_norm_residual rms_norm_cast residual_add_norm "
             "scaled_residual_add_norm token_shift "
             "clamped_glu sigmoid_mul gelu_glu relu_glu relu2 "
@@ -1497,6 +1498,27 @@ def build_query_tiles(chunk_lens, device, starts=None):
     """query_tiles as int32 tensors (tile_seq, tile_qbase)."""
     return tuple(torch.from_numpy(t).to(device)
                  for t in query_tiles(chunk_lens, starts))
+
+
+def embed_positions(ids, positions, table, where, scale: float):
+    """table[ids] * scale + where[positions] in f32, and its rounding to bf16, in
+    one launch; None for other tables or rows than plain ones of bf16."""
+    if not (table.is_cuda and table.dim() == where.dim() == 2
+            and ids.dim() == positions.dim() == 1
+            and table.size(1) == where.size(1) and table.size(1) % 8 == 0
+            and ids.numel() == positions.numel() and not _transformed()
+            and all(t.is_contiguous() and t.device == table.device
+                    for t in (ids, positions, table, where))
+            and ids.dtype == positions.dtype == torch.int64
+            and all(t.dtype == torch.bfloat16 and t.data_ptr() % 16 == 0
+                    and not (torch.is_grad_enabled() and t.requires_grad)
+                    for t in (table, where))):
+        return None
+    x32 = torch.empty(ids.numel(), table.size(1), dtype=torch.float32,
+                      device=table.device)
+    out = torch.empty_like(x32, dtype=torch.bfloat16)
+    _K.embed_positions(x32, out, ids, positions, table, where, scale)
+    return x32, out
 
 
 def post_norm_residual(x32, y, w, eps: float, out_dtype, y2=None, w_y=None,

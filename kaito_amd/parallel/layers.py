@@ -35,6 +35,19 @@ def untouched(module: nn.Module, cls: type) -> bool:
         and type(module).forward is cls._whole
 
 
+_EMBEDDING = nn.Embedding.forward
+
+
+def looks_up(module: nn.Module) -> bool:
+    """Whether a call of `module` reads the rows of its weight and nothing else."""
+    own = module.__dict__
+    return type(module) is nn.Embedding and module.max_norm is None \
+        and not (own["_forward_hooks"] or own["_forward_pre_hooks"]
+                 or _module._global_forward_hooks
+                 or _module._global_forward_pre_hooks or "forward" in own) \
+        and nn.Embedding.forward is _EMBEDDING
+
+
 class _QuantMixin:
     """Weight-only W4A16 for the parallel linears: quantize_() packs the
     rank-local weight shard into the native 4-bit layout and switches the

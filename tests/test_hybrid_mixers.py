@@ -614,3 +614,31 @@ def test_window_attention_tiled_prompt_kernel(H, G, D, V, window):
         close(got[at:at + n], want, dt)
         close(plain[at:at + n], want, dt)
         at += n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,H", [(1, 8), (3, 520), (32, 2048), (700, 4096)])
+def test_embed_positions(T, H):
+    """The same bits as torch's gathers, product and sum."""
+    torch.manual_seed(T)
+    table = torch.randn(300, H, device="cuda").bfloat16()
+    where = torch.randn(70, H, device="cuda").bfloat16()
+    ids = torch.randint(0, 300, (T,), device="cuda")
+    pos = torch.randint(-70, 70, (T,), device="cuda")
+    x32 = table[ids].float() * 45.2548 + where[pos].float()
+    got = ops.embed_positions(ids, pos, table, where, 45.2548)
+    assert torch.equal(got[0], x32) and torch.equal(got[1], x32.bfloat16())
+    for args in ((ids, pos, table.float(), where), (ids, pos, table.T, where.T),
+                 (ids.int(), pos, table, where)):
+        assert ops.embed_positions(*args, 1.0) is None
+
+
+@pytest.mark.gpu
+def test_hooked_embedding_is_called():
+    from kaito_amd.parallel.layers import looks_up
+    e = torch.nn.Embedding(4, 8)
+    assert looks_up(e)
+    handle = e.register_forward_hook(lambda m, i, o: o + 1)
+    assert not looks_up(e)
+    handle.remove()
+    assert looks_up(e) and not looks_up(torch.nn.Embedding(4, 8, max_norm=1.0))
