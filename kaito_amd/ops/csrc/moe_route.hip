@@ -28,7 +28,7 @@
 // A decode step's choice is launches and latency, not work: as torch ops
 // (product, cast, top-k, softmax, sort, gathers, scatter, scan) it was about
 // 25 launches, 130 us of a layer's 240 at 32 tokens and 8 experts. Now it is
-// 5.1 us for logits and choice (rows of 2048, one launch behind another; 9.5
+// 4.4 us for logits and choice (rows of 2048, one launch behind another; 9.5
 // where the row before has to arrive from its norm) and 4.8 for the sort.
 //
 // An output's place in the row lives in lane e % 64, register e / 64.
@@ -42,14 +42,47 @@ namespace {
 
 constexpr int ROUTE_MAX = 1024;      // router outputs
 
-// largest value over the wave, ties to the lower index
-KAITO_DEV void wave_argmax(float& v, int& i) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const float ov = __shfl_xor(v, off, 64);
-    const int oi = __shfl_xor(i, off, 64);
+// largest value over `width` neighbouring lanes (a power of two), ties to the lower
+// index. A choice is a chain of these: within 16 lanes the neighbours' values come
+// by DPP and not through LDS, and few outputs need few steps (32 rows of 8 outputs
+// in 4 groups, of which 2 stay, top 2: 9.3 us with 6 steps of two LDS exchanges each,
+// one group after the other, now 5.4; 600 rows of 16 14.1 and 9.8; without groups 5.0
+// and 4.4).
+template <int CTRL>
+KAITO_DEV int dpp(const int x) {
+  return __builtin_amdgcn_update_dpp(x, x, CTRL, 0xf, 0xf, false);
+}
+KAITO_DEV void lanes_argmax(float& v, int& i, const int width) {
+  auto take = [&](const float ov, const int oi) {
     if (ov > v || (ov == v && oi < i)) { v = ov; i = oi; }
-  }
+  };
+  // behind a step all lanes of its width agree, so that a mirror is as good as an
+  // exchange
+#define ROUTE_STEP(W_, CTRL_)                                                 \
+  if (width > W_)                                                             \
+    take(__int_as_float(dpp<CTRL_>(__float_as_int(v))), dpp<CTRL_>(i))
+  ROUTE_STEP(1, 0xB1);              // quad_perm 1 0 3 2
+  ROUTE_STEP(2, 0x4E);              // quad_perm 2 3 0 1
+  ROUTE_STEP(4, 0x141);             // row_half_mirror
+  ROUTE_STEP(8, 0x128);             // row_ror 8
+#undef ROUTE_STEP
+  if (width > 16) take(__shfl_xor(v, 16, 64), __shfl_xor(i, 16, 64));
+  if (width > 32) take(__shfl_xor(v, 32, 64), __shfl_xor(i, 32, 64));
+}
+KAITO_DEV float lanes_max(float v, const int width) {
+#define ROUTE_STEP(W_, CTRL_)                                                 \
+  if (width > W_) v = fmaxf(v, __int_as_float(dpp<CTRL_>(__float_as_int(v))))
+  ROUTE_STEP(1, 0xB1);
+  ROUTE_STEP(2, 0x4E);
+  ROUTE_STEP(4, 0x141);
+  ROUTE_STEP(8, 0x128);
+#undef ROUTE_STEP
+  if (width > 16) v = fmaxf(v, __shfl_xor(v, 16, 64));
+  if (width > 32) v = fmaxf(v, __shfl_xor(v, 32, 64));
+  return v;
+}
+KAITO_DEV int lanes_for(const int n) {      // the width that holds n lanes
+  return n <= 1 ? 1 : n > 32 ? 64 : 1 << (32 - __builtin_clz(n - 1));
 }
 
 constexpr int NONE = 1 << 30;        // a lane without a candidate
@@ -88,7 +121,7 @@ KAITO_DEV void route_row(const RouteArgs& a, const float* row, const int64_t t,
                     : -INFINITY;
     }
   } else {
-    mx = wave_reduce_max(mx);
+    mx = lanes_max(mx, NPL == 1 ? lanes_for(N) : 64);
     float sum = 0.f;
 #pragma unroll
     for (int r = 0; r < NPL; r++) {
@@ -114,40 +147,54 @@ KAITO_DEV void route_row(const RouteArgs& a, const float* row, const int64_t t,
   if (a.groups > 1) {
     const int n = N / a.groups;
     float mine = -INFINITY;                 // lane g: group g's score
-    for (int g = 0; g < a.groups; g++) {
-      float m = -INFINITY;
-      int mi = N;
-#pragma unroll
-      for (int r = 0; r < NPL; r++) {
-        const int e = r * 64 + lane;
-        if (e >= g * n && e < (g + 1) * n && (ch[r] > m || mi == N)) {
-          m = ch[r];
-          mi = e;
-        }
+    if (NPL == 1 && (n & (n - 1)) == 0) {   // all at once
+      float score = ch[0];
+      int mi = lane;
+      lanes_argmax(score, mi, n);
+      if (MODE == SIGMOID && n > 1) {
+        float m2 = lane == mi ? -INFINITY : ch[0];      // the second largest
+        int at = lane;
+        lanes_argmax(m2, at, n);
+        score += m2;
       }
-      float score;
-      if constexpr (MODE == SIGMOID) {
-        wave_argmax(m, mi);
-        score = m;
-        float m2 = -INFINITY;               // the second largest
+      score = rank(__shfl(score, lane * n & 63, 64));
+      if (lane < a.groups) mine = score;
+    } else {
+      for (int g = 0; g < a.groups; g++) {
+        float m = -INFINITY;
+        int mi = N;
 #pragma unroll
         for (int r = 0; r < NPL; r++) {
           const int e = r * 64 + lane;
-          if (e >= g * n && e < (g + 1) * n && e != mi) m2 = fmaxf(m2, ch[r]);
+          if (e >= g * n && e < (g + 1) * n && (ch[r] > m || mi == N)) {
+            m = ch[r];
+            mi = e;
+          }
         }
-        if (n > 1) score += wave_reduce_max(m2);
-      } else {
-        score = wave_reduce_max(m);
+        float score;
+        if constexpr (MODE == SIGMOID) {
+          lanes_argmax(m, mi, 64);
+          score = m;
+          float m2 = -INFINITY;               // the second largest
+#pragma unroll
+          for (int r = 0; r < NPL; r++) {
+            const int e = r * 64 + lane;
+            if (e >= g * n && e < (g + 1) * n && e != mi) m2 = fmaxf(m2, ch[r]);
+          }
+          if (n > 1) score += wave_reduce_max(m2);
+        } else {
+          score = wave_reduce_max(m);
+        }
+        if (lane == g) mine = rank(score);
       }
-      if (lane == g) mine = rank(score);
     }
     unsigned long long kept = 0;
     for (int k = 0; k < a.keep; k++) {
       const bool open = lane < a.groups && !((kept >> lane) & 1);
       float v = open ? mine : -INFINITY;
       int i = open ? lane : NONE;
-      wave_argmax(v, i);
-      kept |= 1ull << i;
+      lanes_argmax(v, i, lanes_for(a.groups));
+      kept |= 1ull << __builtin_amdgcn_readfirstlane(i);
     }
 #pragma unroll
     for (int r = 0; r < NPL; r++) {
@@ -170,11 +217,13 @@ KAITO_DEV void route_row(const RouteArgs& a, const float* row, const int64_t t,
         v = ch[r];
         i = r * 64 + lane;
       }
-    wave_argmax(v, i);
+    lanes_argmax(v, i, NPL == 1 ? lanes_for(N) : 64);
+    i = __builtin_amdgcn_readfirstlane(i);
     float sv = 0.f;
 #pragma unroll
     for (int r = 0; r < NPL; r++) {
-      const float b = __shfl(s[r], i & 63, 64);
+      const float b = __int_as_float(
+          __builtin_amdgcn_readlane(__float_as_int(s[r]), i & 63));
       if (r == (i >> 6)) sv = b;
       if (r * 64 + lane == i) open &= ~(1u << r);
     }
