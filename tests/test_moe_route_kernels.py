@@ -346,7 +346,7 @@ def test_which_shared_experts_join(E, H, I, top, beside, alone):
     (2, 2, 1, 1), (3, 1, 1, 3), (16, 1, 1, 2), (17, 1, 1, 5), (32, 4, 2, 3),
     (33, 1, 1, 33), (24, 3, 2, 4), (20, 4, 3, 5), (64, 2, 1, 8), (64, 64, 9, 4),
     (40, 5, 2, 8), (48, 3, 1, 16)])
-def test_choice_at_the_widths_of_lanes(mode, N, groups, keep, top):
+def test_choice_at_the_widths_of_lanes(mode, N, groups, keep, top, monkeypatch):
     """Outputs around the 2 to 64 lanes that a choice looks at, groups of powers of
     two, all at once, and others, ties among them: as in a stable sort."""
     if mode == "logits":
@@ -357,5 +357,8 @@ def test_choice_at_the_widths_of_lanes(mode, N, groups, keep, top):
     z[8] = 0.5
     z[9, N // 2:] = z[9, :N - N // 2].clone()
     a = (top, N, groups, keep, True, 1.0, mode)
-    got, want = ops.moe_route(z, None, *a), R.moe_route(z, None, *a)
-    _check(got, want, N)
+    got = ops.moe_route(z, None, *a)
+    # the lower index first, which topk does not promise
+    monkeypatch.setattr(torch.Tensor, "topk", lambda t, k, d: tuple(
+        v[..., :k] for v in t.sort(dim=d, descending=True, stable=True)))
+    _check(got, R.moe_route(z, None, *a), N)
