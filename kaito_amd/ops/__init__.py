@@ -346,7 +346,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
                 _K.batch_linear(out, x, w, _none(bias, x), 0, 0, False)
             return out
     if bias is None and w.dim() == 2 and x.dim() == 2 \
-            and _vocabulary_shape(x.size(0), *w.shape) \
+            and (_vocabulary_shape(x.size(0), *w.shape)
+                 or _uneven_shape(x.size(0), *w.shape)) \
             and _tiles_fit(x, w, 64):
         out = torch.empty(x.size(0), w.size(0), dtype=x.dtype, device=x.device)
         _K.tile_linear(out, x, w)
@@ -425,10 +426,10 @@ def _pair_pays(M: int, N: int, one: bool) -> bool:
 
 
 @functools.lru_cache(1024)
-def _tile_fill(M: int, N: int) -> float:
-    """What share of its time a product of M rows and N weight rows keeps the
-    chip's 256 workgroups busy for, in the best of the shapes that the tiles'
-    kernels choose from (csrc/tile_gemm.h `run`: the same costs)."""
+def _tile_plan(M: int, N: int):
+    """The tiles that the kernels choose for M rows and N weight rows and the cost of
+    their rounds (csrc/tile_gemm.h `run`): "whole" ones of 256 x 256, "quartered"
+    in the last round, or "smaller" ones."""
     def share(rows, cols):          # tiles of an XCD
         return -(-(-(-M // rows) * -(-N // cols)) // 8)
 
@@ -438,10 +439,18 @@ def _tile_fill(M: int, N: int) -> float:
     rest = large % 32
     if rest > (16 if large < 32 else 8):
         rest = 0
-    cost = min(5 * rounds(large - rest) + 2 * rounds(4 * rest),
-               3 * rounds(share(128, 256)), 3 * rounds(share(256, 128)),
-               2 * rounds(share(128, 128)))
-    return M * N / (cost * 256 * 65536 / 5)
+    whole = 5 * rounds(large - rest) + 2 * rounds(4 * rest)
+    small = min(3 * rounds(share(128, 256)), 3 * rounds(share(256, 128)),
+                2 * rounds(share(128, 128)))
+    if small < whole:
+        return "smaller", small
+    return "quartered" if rest else "whole", whole
+
+
+def _tile_fill(M: int, N: int) -> float:
+    """What share of its time a product of M rows and N weight rows keeps the
+    chip's 256 workgroups busy for."""
+    return M * N / (_tile_plan(M, N)[1] * 256 * 65536 / 5)
 
 
 def _tiles_fit(x: torch.Tensor, w: torch.Tensor, cols: int) -> bool:
@@ -483,6 +492,23 @@ def _vocabulary_shape(M: int, N: int, K: int) -> bool:
     151936 x 4096 1.0 to 1.02 from 33 to 64 rows, 128256 x 8192 0.94 to 1.02)."""
     return 129 <= M <= 256 and N >= 100000 and K >= 4096 \
         and (M > 224 or not 4096 < K < 6144)
+
+
+def _uneven_shape(M: int, N: int, K: int) -> bool:
+    """Whether a product of a prompt's rows whose tiles of 256 x 256 fill no whole
+    number of rounds runs on the tiles, which cut the last round or take smaller
+    ones. Whole rounds are the library's (0.94 to 0.99 times). us, library and
+    tiles: 3072 x 2048 at 8192 rows 91, 84, 5901 86, 65; 5120 x 2048 at 3948 85,
+    68; 2048 x 2048 at 2585 31, 27; 1024 x 1536 at 8192 28, 26, at 4807 21, 22;
+    4096 x 1024 at 4162 56, 39; 3072 x 512 at 6541 51, 25; 4096 x 3072 at 4437
+    112, 93; 8192 x 3072 at 6309 270, 228, but 3072 x 3072 at 6962 112, 113 and
+    5120 x 3072 at 4206 111, 113; 100 sizes, 1.0 to 2.1 times as fast but for those
+    four. K of 4096 with a quartered round 1.06, with smaller tiles 0.99 to 1.02;
+    up to 1024 rows 0.4 to 1.1."""
+    if not (M > 2048 and 1024 <= N <= 8192 and K <= 4096):
+        return False
+    kind = _tile_plan(M, N)[0]
+    return kind == "quartered" or (kind == "smaller" and K <= 3072)
 
 
 def _pair_tiled(x, w, x2, w2) -> bool:

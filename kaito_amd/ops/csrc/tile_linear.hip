@@ -1,6 +1,7 @@
 // Linear layers of prompts on the tiles of tile_gemm.h:
 //
-//   tile_linear   out = x W^T, for vocabularies
+//   tile_linear   out = x W^T, for vocabularies and for products whose large tiles
+//                 fill no whole number of rounds
 //   tile_swiglu   out = silu(x Wg^T) (x Wu^T) of W = [Wg | Wu]
 //   tile_pair     out = x W^T (+ bias), out2 = x2 W2^T (+ bias2): one launch, whose
 //                 last round of tiles is not each product's own

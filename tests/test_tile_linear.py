@@ -116,3 +116,25 @@ def test_which_two_products_take_tiles(M, N, K, tiles):
     (256, 262144, 2304, False), (200, 32000, 4096, False)])
 def test_which_vocabularies_take_tiles(M, N, K, tiles):
     assert ops._vocabulary_shape(M, N, K) == tiles
+
+
+@pytest.mark.parametrize("M,N,K,tiles", [
+    (8192, 3072, 2048, True), (8192, 2048, 2048, False), (2048, 1024, 512, False),
+    (2049, 1024, 512, True), (2049, 1023, 512, False), (8192, 8256, 1024, False),
+    (5901, 3072, 4096, True), (8192, 3072, 3136, False)])
+def test_which_products_of_prompts_take_tiles(M, N, K, tiles):
+    """The sides of the lines on which either was measured to be faster."""
+    assert ops._uneven_shape(M, N, K) == tiles
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(2049, 1024, 64), (2305, 1088, 192),
+                                   (5901, 3072, 128), (8190, 2560, 192),
+                                   (2060, 8192, 320)])
+def test_uneven_products(M, N, K, monkeypatch):
+    """Last rounds in quarters and smaller tiles, rows that end inside one."""
+    torch.manual_seed(M)
+    assert ops._uneven_shape(M, N, K)
+    x, w = _rand(M, K), _rand(N, K, std=K ** -0.5)
+    monkeypatch.setattr(torch.nn.functional, "linear", None)
+    _close(ops.linear(x, w), x.double() @ w.double().T)
