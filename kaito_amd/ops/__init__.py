@@ -457,7 +457,7 @@ def _tiles_fit(x: torch.Tensor, w: torch.Tensor, cols: int) -> bool:
     """Operands that the tiles' kernels take."""
     return _plain_rows(x, w, (1 << 24) - 1) and x.is_contiguous() \
         and w.size(1) % 64 == 0 and w.size(0) % cols == 0 \
-        and w.size(1) < 1 << 22 and w.numel() <= 0x7fff8000
+        and max(w.shape) < 1 << 22 and w.numel() <= 0x7fff8000
 
 
 def _tiled(x: torch.Tensor, w: torch.Tensor) -> bool:

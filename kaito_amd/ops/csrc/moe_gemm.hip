@@ -340,7 +340,8 @@ void moe_grouped_up(at::Tensor act, at::Tensor x, at::Tensor w,
   a.E = (int)w.size(0); a.N = (int)act.size(1); a.K = (int)x.size(1);
   a.e_base = (int)e_base;
   TORCH_CHECK(w.size(1) == (plain ? 1 : 2) * (int64_t)a.N &&
-              w.size(2) == a.K && a.K % BK == 0 && a.N % 64 == 0 && a.K > 0);
+              w.size(2) == a.K && a.K % BK == 0 && a.N % 64 == 0 && a.K > 0 &&
+              act.size(1) < tile::MOST_OUTPUTS);
   TORCH_CHECK(e_base >= 0 && offsets.numel() > e_base + a.E &&
               sorted_ids.numel() == act.size(0));
   TORCH_CHECK(act_mode >= 0 && act_mode <= 2);
@@ -385,7 +386,7 @@ void moe_grouped_down(at::Tensor y, at::Tensor act, at::Tensor w,
   a.E = (int)w.size(0); a.N = (int)y.size(1); a.K = (int)act.size(1);
   a.e_base = (int)e_base;
   TORCH_CHECK(w.size(1) == a.N && w.size(2) == a.K && a.K % BK == 0 &&
-              a.N % 64 == 0 && a.K > 0);
+              a.N % 64 == 0 && a.K > 0 && y.size(1) < tile::MOST_OUTPUTS);
   TORCH_CHECK(e_base >= 0 && offsets.numel() > e_base + a.E);
   if (bias.numel() > 0) {
     check16(bias);
@@ -411,7 +412,7 @@ void latent_kv(at::Tensor kv, at::Tensor c, at::Tensor wk, at::Tensor wv) {
   TORCH_CHECK(wk.size(2) == K && wv.size(0) == H && wv.size(1) == K &&
               kv.size(0) == T && kv.size(1) == N1 + H * V &&
               K % 64 == 0 && K > 0 && V % 64 == 0 && N1 % 256 == 0 &&
-              T < (1ll << 22) && kv.size(1) < (1ll << 22));
+              T < (1ll << 22) && kv.size(1) < tile::MOST_OUTPUTS);
   if (T == 0 || H == 0) return;
   auto stream = at::hip::getCurrentHIPStream();
   const at::Tensor wt = at::empty({H, V, K}, wv.options());

@@ -100,6 +100,8 @@ KAITO_DEV float gated(float g, float u, float limit) {
 
 // bytes of x behind gathered rows, of weights behind a tile's first
 constexpr uint32_t MOST_BYTES = 0xffff0000;
+// outputs of a row are fewer: a wave's 128 rows of them, in f32, end below 2^31
+constexpr int64_t MOST_OUTPUTS = 1 << 22;
 
 struct Tile {
   int expert, m0, row_end, n0;      // first row, rows' end, first output
@@ -368,7 +370,9 @@ KAITO_DEV void stream(const GemmArgs& a, short* lds, Next&& next) {
     const int N = apart ? a.N - a.n2 : TWO && a.out2 ? a.n2 : a.N;
     const int c0 = cur.n0 + wn * WC - (apart ? a.n2 : 0);
     const int64_t first_row = cur.m0 + wm * FM * 16;
-    const int live = cur.row_end - (int)first_row;  // rows that exist
+    // rows of this wave that exist: their bytes, and not all that follow, have to
+    // stay below BEYOND
+    const int live = min(cur.row_end - (int)first_row, FM * 16);
     constexpr int SIZE = F32 ? 4 : 2;
     // rows and columns that do not exist lie beyond the resource's end
     const auto ro = resource(

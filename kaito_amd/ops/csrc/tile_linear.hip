@@ -66,7 +66,7 @@ static GemmArgs tile_args(const at::Tensor& out, const at::Tensor& x,
   const int64_t T = x.size(0), K = x.size(1);
   TORCH_CHECK(out.size(0) == T && w.size(0) == rows && w.size(1) == K &&
               K % tile::BK == 0 && out.size(1) % 64 == 0 && K > 0 &&
-              K < (1 << 22) && T < (1 << 24) && rows < (1 << 24) &&
+              K < (1 << 22) && T < (1 << 24) && rows < tile::MOST_OUTPUTS &&
               w.numel() * 2 <= tile::MOST_BYTES);
   GemmArgs a{};
   a.out = (short*)out.data_ptr();

@@ -138,3 +138,82 @@ def test_uneven_products(M, N, K, monkeypatch):
     x, w = _rand(M, K), _rand(N, K, std=K ** -0.5)
     monkeypatch.setattr(torch.nn.functional, "linear", None)
     _close(ops.linear(x, w), x.double() @ w.double().T)
+
+
+def _all_close(out, ref, rows=1 << 16):
+    for at in range(0, out.size(0), rows):
+        _close(out[at:at + rows], ref(slice(at, at + rows)))
+
+
+# outputs of more than 2 and than 4 GiB, whose last columns end inside a tile
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [560000, 746000])
+@pytest.mark.parametrize("glu", [False, True])
+def test_outputs_of_gigabytes(M, glu):
+    torch.manual_seed(M)
+    N, K = 2880, 64
+    x, w = _rand(M, K), _rand(2 * N if glu else N, K, std=K ** -0.5)
+    out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    (ops._K.tile_swiglu if glu else ops._K.tile_linear)(out, x, w)
+
+    def ref(rows):
+        y = x[rows].double() @ w.double().T
+        if not glu:
+            return y
+        g, u = y.chunk(2, -1)
+        return g * torch.sigmoid(g) * u
+    _all_close(out, ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [560000, 746000])
+@pytest.mark.parametrize("f32", [False, True])
+def test_expert_rows_of_gigabytes(M, f32):
+    """Up where rows are bf16, down where they are f32, half as many for as much."""
+    torch.manual_seed(M)
+    M, N, K = M // (2 if f32 else 1), 2880, 64
+    first = M - 130
+    off = torch.tensor([0, first, M], dtype=torch.int32, device=DEV)
+    none = torch.empty(0, device=DEV)
+    x = _rand(M, K)
+    w = _rand(2, N if f32 else 2 * N, K, std=K ** -0.5)
+    out = torch.full((M, N), float("nan"), device=DEV,
+                     dtype=torch.float32 if f32 else torch.bfloat16)
+    if f32:
+        ops._K.moe_grouped_down(out, x, w, off, none, 0)
+    else:
+        ids = torch.arange(M, dtype=torch.int32, device=DEV)
+        ops._K.moe_grouped_up(out, x, w, ids, off, none, 0, 0, 0.0)
+
+    def ref(rows, e):
+        y = x[rows].double() @ w[e].double().T
+        if f32:
+            return y
+        g, u = y.chunk(2, -1)
+        return g * torch.sigmoid(g) * u
+    _all_close(out[:first], lambda r: ref(slice(r.start, min(r.stop, first)), 0))
+    _close(out[first:], ref(slice(first, M), 1))
+
+
+@pytest.mark.gpu
+def test_latent_keys_and_values_of_gigabytes():
+    torch.manual_seed(0)
+    T, H, D, K = 65600, 128, 128, 64
+    c = _rand(T, K)
+    wk, wv = _rand(H, D, K, std=K ** -0.5), _rand(H, K, D, std=K ** -0.5)
+    assert ops._latent_tiles(T, 2 * H * D, K)
+    k, v = ops.latent_kv(c, wk, wv)
+    rows = wk.view(H * D, K).double().T
+    _all_close(k.reshape(T, H * D), lambda r: c[r].double() @ rows, 1 << 14)
+    rows = wv.transpose(0, 1).reshape(K, H * D).double()
+    _all_close(v.reshape(T, H * D), lambda r: c[r].double() @ rows, 1 << 14)
+
+
+@pytest.mark.gpu
+def test_rows_too_wide_for_the_tiles():
+    """2^22 outputs and more: refused by the kernels, the library's elsewhere."""
+    x, w = _rand(1, 64), _rand(1 << 22, 64)
+    out = torch.empty(1, 1 << 22, dtype=torch.bfloat16, device=DEV)
+    assert not ops._tiles_fit(x, w, 64) and ops._tiles_fit(x, w[:-64], 64)
+    with pytest.raises(RuntimeError):
+        ops._K.tile_linear(out, x, w)
