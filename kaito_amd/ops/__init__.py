@@ -453,9 +453,15 @@ def _tile_fill(M: int, N: int) -> float:
     return M * N / (_tile_plan(M, N)[1] * 256 * 65536 / 5)
 
 
+def _here(x: torch.Tensor) -> bool:
+    """Whether a launch on the current device's stream is one on x's: torch's
+    operations, which a kernel stands in for, find their way by themselves."""
+    return x.device.index == torch.cuda.current_device()
+
+
 def _tiles_fit(x: torch.Tensor, w: torch.Tensor, cols: int) -> bool:
     """Operands that the tiles' kernels take."""
-    return _plain_rows(x, w, (1 << 24) - 1) and x.is_contiguous() \
+    return _plain_rows(x, w, (1 << 24) - 1) and x.is_contiguous() and _here(x) \
         and w.size(1) % 64 == 0 and w.size(0) % cols == 0 \
         and max(w.shape) < 1 << 22 and w.numel() <= 0x7fff8000
 
@@ -1533,6 +1539,7 @@ def embed_positions(ids, positions, table, where, scale: float):
             and ids.dim() == positions.dim() == 1
             and table.size(1) == where.size(1) and table.size(1) % 8 == 0
             and ids.numel() == positions.numel() and not _transformed()
+            and _here(table)
             and all(t.is_contiguous() and t.device == table.device
                     for t in (ids, positions, table, where))
             and ids.dtype == positions.dtype == torch.int64

@@ -12,6 +12,7 @@
 #include <torch/library.h>
 #include <ATen/ATen.h>
 #include <ATen/hip/HIPContext.h>
+#include <c10/hip/HIPFunctions.h>
 
 namespace kaito {
 
@@ -56,6 +57,7 @@ __global__ __launch_bounds__(256, 1) void tile_linear_kernel(const GemmArgs a,
 
 static void check(const at::Tensor& t) {
   TORCH_CHECK(t.is_cuda() && t.dim() == 2 && t.is_contiguous() &&
+              t.get_device() == c10::hip::current_device() &&
               t.dtype() == at::kBFloat16 && (uintptr_t)t.data_ptr() % 16 == 0);
 }
 

@@ -217,3 +217,25 @@ def test_rows_too_wide_for_the_tiles():
     assert not ops._tiles_fit(x, w, 64) and ops._tiles_fit(x, w[:-64], 64)
     with pytest.raises(RuntimeError):
         ops._K.tile_linear(out, x, w)
+
+
+@pytest.mark.gpu
+def test_another_device_is_current(monkeypatch):
+    """Prompts whose device is not the current one are torch's, which switches."""
+    torch.manual_seed(0)
+    x, w, w2 = _rand(2305, 192), _rand(1088, 192), _rand(1024, 192)
+    rows, pair = _rand(1000, 2048), _rand(4096, 2048)
+    table, where = _rand(300, 64), _rand(70, 64)
+    ids = torch.arange(9, device=DEV)
+    assert ops._uneven_shape(2305, 1088, 192) and ops._tiles_fit(x, w, 64)
+    assert ops._pair_tiled(x, w2, x, w) and ops._tiled(rows, pair)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: x.device.index + 1)
+    for op in ("tile_linear", "tile_pair", "tile_swiglu", "embed_positions"):
+        monkeypatch.setattr(ops._K, op, None, raising=False)
+    F = torch.nn.functional
+    assert torch.equal(ops.linear(x, w), F.linear(x, w))
+    a, b = ops.linear_pair(x, w2, x, w)
+    assert torch.equal(a, F.linear(x, w2)) and torch.equal(b, F.linear(x, w))
+    assert torch.equal(ops.linear_swiglu(rows, pair),
+                       ops.silu_and_mul(F.linear(rows, pair)))
+    assert ops.embed_positions(ids, ids, table, where, 1.0) is None
