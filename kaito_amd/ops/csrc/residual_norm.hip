@@ -529,8 +529,8 @@ void token_shift(at::Tensor out, at::Tensor h, at::Tensor mu, at::Tensor state,
 }
 
 // 8 columns per thread; products and sums are rounded each for itself. Numbers
-// outside a table end the launch, as they do in torch's gathers; positions count
-// from the end where they are negative.
+// outside a table add nothing, as ids outside a rank's part of a vocabulary do;
+// positions count from the end where they are negative.
 __global__ void embed_positions_kernel(
     float* __restrict__ x32, short* __restrict__ xo,
     const short* __restrict__ table, const short* __restrict__ where,
@@ -540,10 +540,13 @@ __global__ void embed_positions_kernel(
   const int64_t row = blockIdx.x, id = ids[row];
   int64_t pos = positions[row];
   if (pos < 0) pos += P;
-  if (id < 0 || id >= V || pos < 0 || pos >= P) __builtin_trap();
+  const bool in_table = id >= 0 && id < V, in_where = pos >= 0 && pos < P;
   for (int k = threadIdx.x * 8; k < H; k += blockDim.x * 8) {
-    const short8_t a = *reinterpret_cast<const short8_t*>(table + id * H + k);
-    const short8_t b = *reinterpret_cast<const short8_t*>(where + pos * H + k);
+    short8_t a = {0, 0, 0, 0, 0, 0, 0, 0}, b = a;
+    if (in_table)
+      a = *reinterpret_cast<const short8_t*>(table + id * H + k);
+    if (in_where)
+      b = *reinterpret_cast<const short8_t*>(where + pos * H + k);
     f32x4 v[2];
     short8_t o;
 #pragma unroll

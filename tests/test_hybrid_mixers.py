@@ -634,6 +634,23 @@ def test_embed_positions(T, H):
 
 
 @pytest.mark.gpu
+def test_embed_positions_outside_a_table():
+    """An id or a position that a table does not hold adds nothing."""
+    torch.manual_seed(0)
+    table = torch.randn(300, 520, device="cuda").bfloat16()
+    where = torch.randn(70, 520, device="cuda").bfloat16()
+    ids = torch.tensor([5, -1, 300, 1 << 40, 7, 299, -301], device="cuda")
+    pos = torch.tensor([3, 4, -70, 69, 70, -71, 1 << 40], device="cuda")
+    a = torch.where(((ids >= 0) & (ids < 300))[:, None],
+                    table[ids.clamp(0, 299)].float() * 3.5, 0.0)
+    b = torch.where(((pos >= -70) & (pos < 70))[:, None],
+                    where[pos.clamp(-70, 69)].float(), 0.0)
+    got = ops.embed_positions(ids, pos, table, where, 3.5)
+    assert torch.equal(got[0], a + b)
+    assert torch.equal(got[1], (a + b).bfloat16())
+
+
+@pytest.mark.gpu
 def test_hooked_embedding_is_called():
     from kaito_amd.parallel.layers import looks_up
     e = torch.nn.Embedding(4, 8)
