@@ -40,7 +40,7 @@ for _g, _names in {
             "latent_kv"),
     "route": "moe_route moe_gate_route moe_norm_gate_route moe_sort",
     "quant": ("w4a16_gemv w4a16_dequant w4a16_gemm w4a16_swiglu "
-              "w4a16_norm_swiglu w4a16_norm_linear w4a16_norm_in_tiles "
+              "w4a16_norm_linear w4a16_norm_in_tiles "
               "w4a16_in_tiles lora_shrink lora_expand"),
     "comm": ("allreduce_rmsnorm one_shot_ar_rmsnorm ipc_handle ipc_open "
              "ipc_close"),
@@ -1231,23 +1231,6 @@ def w4a16_swiglu(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor,
     out = torch.empty(x.size(0), N, dtype=x.dtype, device=x.device)
     _K.w4a16_swiglu(out, x.contiguous(), qweight, scales, zeros, group)
     return out
-
-
-def w4a16_norm_swiglu(x, residual, norm, eps: float, qweight, scales, zeros,
-                      group: int):
-    """w4a16_swiglu of fused_add_rms_norm's rows and its residual, of 1 and 2
-    rows in one launch; None for other sizes."""
-    if not (_packed_norm_rows(x, residual, norm, qweight)
-            and qweight.size(0) % 2 == 0
-            and _K.w4a16_in_tiles(x.size(0), qweight.size(0), x.size(1), group,
-                                  True)):
-        return None
-    out = torch.empty(x.size(0), qweight.size(0) // 2, dtype=x.dtype,
-                      device=x.device)
-    stream = torch.empty_like(x)
-    _K.w4a16_norm_swiglu(out, stream, x, residual, norm, eps, qweight, scales,
-                         zeros, group)
-    return out, stream
 
 
 def _packed_norm_rows(x, residual, norm, qweight) -> bool:

@@ -10,10 +10,6 @@ void w4a16_dequant(at::Tensor out, at::Tensor qweight, at::Tensor scales,
                    at::Tensor zeros, int64_t group);
 void w4a16_gemm(at::Tensor out, at::Tensor x, at::Tensor qweight,
                 at::Tensor scales, at::Tensor zeros, int64_t group);
-void w4a16_norm_swiglu(at::Tensor out, at::Tensor sum, at::Tensor x,
-                       at::Tensor residual, at::Tensor g, double eps,
-                       at::Tensor qweight, at::Tensor scales, at::Tensor zeros,
-                       int64_t group);
 void w4a16_swiglu(at::Tensor out, at::Tensor x, at::Tensor qweight,
                   at::Tensor scales, at::Tensor zeros, int64_t group);
 void w4a16_norm_linear(at::Tensor out, at::Tensor sum, at::Tensor x,
@@ -33,7 +29,6 @@ TORCH_LIBRARY_FRAGMENT(kaito, m) {
   m.def("w4a16_gemv(Tensor(a!) out, Tensor x, Tensor qweight, Tensor scales, Tensor zeros, int group) -> ()");
   m.def("w4a16_dequant(Tensor(a!) out, Tensor qweight, Tensor scales, Tensor zeros, int group) -> ()");
   m.def("w4a16_gemm(Tensor(a!) out, Tensor x, Tensor qweight, Tensor scales, Tensor zeros, int group) -> ()");
-  m.def("w4a16_norm_swiglu(Tensor(a!) out, Tensor(b!) sum, Tensor x, Tensor residual, Tensor g, float eps, Tensor qweight, Tensor scales, Tensor zeros, int group) -> ()");
   m.def("w4a16_swiglu(Tensor(a!) out, Tensor x, Tensor qweight, Tensor scales, Tensor zeros, int group) -> ()");
   m.def("w4a16_norm_linear(Tensor(a!) out, Tensor(b!) sum, Tensor x, Tensor residual, Tensor g, float eps, Tensor qweight, Tensor scales, Tensor zeros, int group, bool glu) -> ()");
   m.def("w4a16_norm_in_tiles(int M, int rows, int K, int group, bool glu) -> bool", &kaito::w4a16_norm_in_tiles);
@@ -46,7 +41,6 @@ TORCH_LIBRARY_IMPL(kaito, CUDA, m) {
   m.impl("w4a16_gemv", &kaito::w4a16_gemv);
   m.impl("w4a16_dequant", &kaito::w4a16_dequant);
   m.impl("w4a16_gemm", &kaito::w4a16_gemm);
-  m.impl("w4a16_norm_swiglu", &kaito::w4a16_norm_swiglu);
   m.impl("w4a16_norm_linear", &kaito::w4a16_norm_linear);
   m.impl("w4a16_swiglu", &kaito::w4a16_swiglu);
   m.impl("lora_shrink", &kaito::lora_shrink);

@@ -743,14 +743,6 @@ void w4a16_norm_linear(at::Tensor out, at::Tensor sum, at::Tensor x,
   TORCH_CHECK(fits, "w4a16_norm_linear: sizes of the tiles");
 }
 
-void w4a16_norm_swiglu(at::Tensor out, at::Tensor sum, at::Tensor x,
-                       at::Tensor residual, at::Tensor g, double eps,
-                       at::Tensor qweight, at::Tensor scales, at::Tensor zeros,
-                       int64_t group) {
-  w4a16_norm_linear(out, sum, x, residual, g, eps, qweight, scales, zeros,
-                    group, true);
-}
-
 void w4a16_dequant(at::Tensor out, at::Tensor qweight, at::Tensor scales,
                    at::Tensor zeros, int64_t group) {
   const int N = qweight.size(0), K = out.size(1);

@@ -144,10 +144,9 @@ class ColumnParallelLinear(_QuantMixin, nn.Module):
         if self.bias is not None or not self._bare():
             return None
         if self._quantized:
-            args = (x, residual, norm, eps, self.qweight, self.scales,
-                    self.zeros, self.q_group)
-            took = ops.w4a16_norm_swiglu(*args)
-            return ops.w4a16_norm_linear(*args, True) if took is None else took
+            return ops.w4a16_norm_linear(x, residual, norm, eps, self.qweight,
+                                         self.scales, self.zeros, self.q_group,
+                                         True)
         if not ops.norm_fits(x, residual, norm, self.weight):
             return None
         return ops.add_norm_linear(x, residual, norm, eps, self.weight,

@@ -67,7 +67,6 @@ def _step(m, T):
 def _alone(mp):
     """A launch for each norm, product and sum."""
     mp.setattr(ops, "norm_fits", lambda *a: False)
-    mp.setattr(ops, "w4a16_norm_swiglu", lambda *a: None)
     mp.setattr(ops, "w4a16_norm_linear", lambda *a: None)
     mp.setattr(ops, "linear_parts", ops.linear)
 
@@ -95,7 +94,6 @@ def _compare(m, T, fused, rel=0.0):
         mp.setattr(ops, name, call)
     with pytest.MonkeyPatch.context() as mp:
         count("add_norm_linear", lambda o: True)
-        count("w4a16_norm_swiglu", lambda o: o is not None)
         count("w4a16_norm_linear", lambda o: o is not None)
         count("linear_parts", lambda o: isinstance(o, ops.SplitRows))
         got, ours = _step(m, T)

@@ -395,13 +395,18 @@ def test_norm_in_the_packed_product(M, N, K):
     x0, r0 = x.clone(), r.clone()
     normed, total = ops.fused_add_rms_norm(x, r.clone(), g, 1e-5)
     want = ops.w4a16_swiglu(normed, *packed, 128)
-    took = ops.w4a16_norm_swiglu(x, r, g, 1e-5, *packed, 128)
-    assert (took is None) == (want is None)
-    if took is not None:
-        assert torch.equal(took[0], want) and torch.equal(took[1], total)
-        assert torch.equal(x, x0) and torch.equal(r, r0)
-    assert ops.w4a16_norm_swiglu(x.repeat(3, 1), r.repeat(3, 1), g, 1e-5,
-                                 *packed, 128) is None
+    took = ops.w4a16_norm_linear(x, r, g, 1e-5, *packed, 128, True)
+    if want is None:                  # one row whose product alone is streamed
+        assert M == 1
+        w = R.w4a16_unpack(*(t.cpu() for t in packed), 128).to(DEV)
+        gate, up = (normed.double() @ w.double().T).chunk(2, -1)
+        _close(took[0], gate * torch.sigmoid(gate) * up)
+    else:
+        assert torch.equal(took[0], want)
+    assert torch.equal(took[1], total)
+    assert torch.equal(x, x0) and torch.equal(r, r0)
+    assert ops.w4a16_norm_linear(x.repeat(3, 1), r.repeat(3, 1), g, 1e-5,
+                                 *packed, 128, True) is None
 
 
 @pytest.mark.parametrize("M,N,one,launch", [
