@@ -214,9 +214,11 @@ KAITO_DEV void stream(const GemmArgs& a, short* lds, Next&& next) {
           xs + x_at + c + (n ? n - FN : 0) * 16 * BK);
   };
   // Sums of weight rows 16 i and x rows 16 j are a[4 (FN j + i)] to the third
-  // behind, by name: left to the compiler, they moved. It keeps nothing there
-  // (`fence`). Fragments come from LDS alone, so that no product follows a vector
-  // instruction that writes its operands.
+  // behind, by name: left to the compiler, they moved. Every statement that names
+  // one clobbers all, so that no value of the compiler's outlives a statement there;
+  // that none lives between two either is looked at in what was built
+  // (tests/test_tile_linear.py). Fragments come from LDS alone, so that no product
+  // follows a vector instruction that writes its operands.
   auto fence = [&] { asm volatile("" ::: KAITO_SUMS); };
   auto products = [&](const int kk, const int j, const int i0, const int i1,
                       const bool first) {
@@ -225,12 +227,14 @@ KAITO_DEV void stream(const GemmArgs& a, short* lds, Next&& next) {
       asm volatile("v_mfma_f32_16x16x32_bf16 a[%0:%1], %4, %6, 0\n\t"
                    "v_mfma_f32_16x16x32_bf16 a[%2:%3], %5, %6, 0"
                    :: "n"(a0), "n"(a0 + 3), "n"(a1), "n"(a1 + 3),
-                      "v"(wf[kk][i0]), "v"(wf[kk][i1]), "v"(xf[kk][j]));
+                      "v"(wf[kk][i0]), "v"(wf[kk][i1]), "v"(xf[kk][j])
+                   : KAITO_SUMS);
     else
       asm volatile("v_mfma_f32_16x16x32_bf16 a[%0:%1], %4, %6, a[%0:%1]\n\t"
                    "v_mfma_f32_16x16x32_bf16 a[%2:%3], %5, %6, a[%2:%3]"
                    :: "n"(a0), "n"(a0 + 3), "n"(a1), "n"(a1 + 3),
-                      "v"(wf[kk][i0]), "v"(wf[kk][i1]), "v"(xf[kk][j]));
+                      "v"(wf[kk][i0]), "v"(wf[kk][i1]), "v"(xf[kk][j])
+                   : KAITO_SUMS);
   };
   auto settle = [&] {               // the last products' results are there
     asm volatile("s_nop 15\n\ts_nop 15" ::: KAITO_SUMS);
@@ -238,7 +242,7 @@ KAITO_DEV void stream(const GemmArgs& a, short* lds, Next&& next) {
   auto sum = [&](const int i, const int j, const int e) {
     float v;
     asm volatile("v_accvgpr_read_b32 %0, a[%1]"
-                 : "=v"(v) : "n"(4 * (FN * j + i) + e));
+                 : "=v"(v) : "n"(4 * (FN * j + i) + e) : KAITO_SUMS);
     return v;
   };
 

@@ -2,10 +2,15 @@
 that end inside a tile, few K steps, each shape of tiles and several rounds. Sums
 of K f32 products, rounded to bf16 once: half a unit of the 8 bits, and where a sum
 cancels the f32 rounding of its terms."""
+import os
+import re
+import subprocess
+
 import pytest
 import torch
 
 from kaito_amd import ops
+from kaito_amd.ops import _build
 
 DEV = "cuda"
 
@@ -239,3 +244,40 @@ def test_another_device_is_current(monkeypatch):
     assert torch.equal(ops.linear_swiglu(rows, pair),
                        ops.silu_and_mul(F.linear(rows, pair)))
     assert ops.embed_positions(ids, ids, table, where, 1.0) is None
+
+
+@pytest.mark.parametrize("group,kernels", [
+    ("core", ["tile_linear_kernel"]),
+    ("moe", ["moe_grouped_kernel", "latent_kv_kernel"])])
+def test_sums_are_the_products_alone(group, kernels, tmp_path):
+    """Sums are in accumulation registers by name, unknown to the compiler between
+    two statements: in what it built nothing but products writes to one, and nothing
+    but the reads of sums looks at one."""
+    objdump = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"),
+                           "llvm/bin/llvm-objdump")
+    lib = _build.so_path(group)
+    if not (os.path.exists(objdump) and lib.exists()):
+        pytest.skip("nothing built, or no disassembler")
+    here = tmp_path / lib.name          # code objects are put beside it
+    here.symlink_to(lib)
+    subprocess.run([objdump, "--offloading", here.name], cwd=tmp_path, check=True,
+                   stdout=subprocess.DEVNULL)
+    found = dict.fromkeys(kernels, 0)
+    for obj in tmp_path.glob("*amdgcn*"):
+        text = subprocess.run([objdump, "-d", obj.name], cwd=tmp_path, check=True,
+                              capture_output=True, text=True).stdout
+        for body in re.split(r"\n(?=[0-9a-f]+ <)", text):
+            name = next((k for k in kernels if k in body.split("\n", 1)[0]), None)
+            if name is None:
+                continue
+            products = 0
+            for line in body.split("\n")[1:]:
+                code = line.split("//")[0].split(None, 1)
+                if len(code) < 2 or not re.search(r"\ba(\d|\[)", code[1]):
+                    continue
+                assert code[0] in ("v_mfma_f32_16x16x32_bf16",
+                                   "v_accvgpr_read_b32"), line
+                products += code[0].startswith("v_mfma")
+            assert products
+            found[name] += 1
+    assert all(found.values()), found
