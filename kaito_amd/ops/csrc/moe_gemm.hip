@@ -15,8 +15,8 @@
 // 1000 56 and 53, 49 and 34; 300 33 and 30, 32 and 21; 100 31 and 24, 29 and 19. 8 of
 // 4096 x 14336, 8192 tokens: 3117 and 2736 (1400 TFLOP/s), 1631 and 1438; 128: 383
 // and 357, 297 and 185. 32 of 2048 x 1024, top 4, 2048 tokens 124 and 119, 62 and
-// 50. 64 of 1024 x 512, top 4, 4096 tokens 64 and 54, 40 and 33; 256, where every
-// row of weights is read for 16 tokens at 5.5 TB/s, 24.2 and 25.5, 15.9 and 16.4.
+// 50. 64 of 1024 x 512, top 4, weights from memory, 4096 tokens 64 and 54, 37 and 29;
+// 256, where every row of weights is read for 16 tokens, 29.1 and 27.9, 15.0 and 14.7.
 // A library GEMM per expert with its gathers, casts and index_add took 958 us behind
 // a host read at the first of these.
 #include "tile_gemm.h"
@@ -122,12 +122,28 @@ struct Tiles {
   }
 };
 
+// What a round takes where the weights come from memory and serve one expert's rows:
+// 128 x 256 tiles, which read as much of them as large ones, more than where rows and
+// weights are shared, small ones, with four steps under way, a little less. us, weights
+// from memory, large, 128 x 256, 256 x 128 and small: 64 experts of 1024 x 512, 1024
+// pairs, up 33.5, 30.0, 38.7, 27.2; 32 of 2880 x 2880, 512 pairs, down 130, 126, 131,
+// 97, 8192 pairs, up, 345, 423, 416, 398; 64 of 2048 x 1408, 18000 pairs, up, 252,
+// 286, 286, 300; 8 of 2048 x 2048, 1400 pairs, up, 50, 44, 42, 47. With 5, 3, 3, 2
+// (tile_linear.hip) 92 of 240 such products took 5 % or more longer than with the best
+// shape, and the first four here were slower than with a workgroup per tile.
+//   Two small tiles for one of 128 x 256 are ahead while rows are few and K is short
+// (their rows of x are read twice as often): 64 of 2048 x 1408, up, 1.05 at 24 rows
+// an expert, 1.01 at 48, 0.99 at 66; 128 of 4096 x 1536, up, 0.99 at 16, 0.94 at 64;
+// 64 of 1024 x 512, down, 1.09 at 16, 1.08 at 64. Of fewer weights than 64 MB they are
+// two chains of latencies for one: 24 of 1536 x 768, down, 0.94 to 0.97.
 template <int KIND>
-__global__ __launch_bounds__(256, 1) void moe_grouped_kernel(const GemmArgs a) {
+__global__ __launch_bounds__(256, 1) void moe_grouped_kernel(const GemmArgs a,
+                                                             const int small) {
   __shared__ __attribute__((aligned(1024))) short lds[tile::LDS];
   const Rows rows(a, 0);
-  tile::run<KIND>(a, lds, Tiles<8, 8, KIND>(a, rows), Tiles<4, 8, KIND>(a, rows),
-                  Tiles<8, 4, KIND>(a, rows), Tiles<4, 4, KIND>(a, rows));
+  tile::run<KIND>(a, lds, {50, 40, 30, small}, Tiles<8, 8, KIND>(a, rows),
+                  Tiles<4, 8, KIND>(a, rows), Tiles<8, 4, KIND>(a, rows),
+                  Tiles<4, 4, KIND>(a, rows));
 }
 
 // ---- keys and values of latent rows ----------------------------------------
@@ -312,10 +328,14 @@ __global__ __launch_bounds__(256) void moe_combine_norm_kernel(
   }
 }
 
+// rows: of all experts, which `offsets` ends; w: this rank's
 template <int KIND>
-void launch_grouped(const GemmArgs& a) {
+void launch_grouped(const GemmArgs& a, const int64_t rows,
+                    const at::Tensor& offsets, const at::Tensor& w) {
+  const int64_t of_one = rows / std::max<int64_t>(offsets.numel() - 1, 1);
+  const bool few = a.K + 32 * of_one < 4096 && w.numel() >= 1 << 25;
   hipLaunchKernelGGL((moe_grouped_kernel<KIND>), dim3(CUS), dim3(256), 0,
-                     at::hip::getCurrentHIPStream(), a);
+                     at::hip::getCurrentHIPStream(), a, few ? 19 : 20);
 }
 
 void check16(const at::Tensor& t) {
@@ -365,9 +385,9 @@ void moe_grouped_up(at::Tensor act, at::Tensor x, at::Tensor w,
   a.offsets = offsets.data_ptr<int>();
   a.limit = (float)act_limit;
   if (act.size(0) == 0 || a.E == 0 || a.N == 0) return;
-  if (plain) launch_grouped<RELU2>(a);
-  else if (act_mode == 1) launch_grouped<CLAMPED>(a);
-  else launch_grouped<SILU>(a);
+  if (plain) launch_grouped<RELU2>(a, act.size(0), offsets, w);
+  else if (act_mode == 1) launch_grouped<CLAMPED>(a, act.size(0), offsets, w);
+  else launch_grouped<SILU>(a, act.size(0), offsets, w);
 }
 
 void moe_grouped_down(at::Tensor y, at::Tensor act, at::Tensor w,
@@ -399,8 +419,8 @@ void moe_grouped_down(at::Tensor y, at::Tensor act, at::Tensor w,
   a.w = (const short*)w.data_ptr() - e_base * w.stride(0);
   a.offsets = offsets.data_ptr<int>();
   if (y.size(0) == 0 || a.E == 0 || a.N == 0) return;
-  if (wide) launch_grouped<PLAIN_F32>(a);
-  else launch_grouped<PLAIN>(a);
+  if (wide) launch_grouped<PLAIN_F32>(a, y.size(0), offsets, w);
+  else launch_grouped<PLAIN>(a, y.size(0), offsets, w);
 }
 
 // kv [T, H D + H V]: c [T, K] times wk [H, D, K] (rows K long) and wv [H, K, V]

@@ -483,17 +483,21 @@ KAITO_DEV void stream(const GemmArgs& a, short* lds, Next&& next) {
 constexpr int NG = 4;               // column tiles that share row tiles
 constexpr int CUS = 256;            // 8 XCDs of 32
 
+// What a round of tiles of a shape takes, beside those of the others; quarters are
+// small tiles
+struct Rounds {
+  int large, wide, tall, small;
+};
+
 // A launch of CUS workgroups, one per CU: all tiles of a product, of the shape that
 // takes least time. Of each shape: `share` tiles per XCD, `here` on this one, tile
 // i of those by number. Tiles of 256 x 256, those of a small last round in quarters,
-// or of 128 x 256, 256 x 128 or 128 x 128: a round takes, where weights and rows come
-// from the caches, about 5 (50 us at K = 2048), 3, 3 and 2 (18 us), quarters as long
-// as 128 x 128. 700 tokens by 8 experts of 2048 x 2048, up: 53, 37, 59 and 41 us; 200:
-// 34, 30, 33 and 24; 4096 tokens by 64 of 1024 x 512: 60, 56, 66 and 55.
+// or of 128 x 256, 256 x 128 or 128 x 128.
 template <int KIND, bool TWO = false, class Large, class Wide, class Tall,
           class Small>
-KAITO_DEV void run(const GemmArgs& a, short* lds, const Large& large,
-                   const Wide& wide, const Tall& tall, const Small& small) {
+KAITO_DEV void run(const GemmArgs& a, short* lds, const Rounds takes,
+                   const Large& large, const Wide& wide, const Tall& tall,
+                   const Small& small) {
   constexpr int workers = CUS / 8;
   enum { LARGE, WIDE, TALL, SMALL };
   auto rounds = [&](const int n) { return (n + workers - 1) / workers; };
@@ -504,13 +508,15 @@ KAITO_DEV void run(const GemmArgs& a, short* lds, const Large& large,
   };
   // the same answer on all XCDs, whose tiles are numbered through
   const int over = last(large.share);
-  int best = 5 * rounds(large.share - over) + 2 * rounds(4 * over), mode = LARGE;
+  int best = takes.large * rounds(large.share - over) +
+             takes.small * rounds(4 * over);
+  int mode = LARGE;
   auto other = [&](const int m, const int cost) {
     if (cost < best) best = cost, mode = m;
   };
-  other(WIDE, 3 * rounds(wide.share));
-  other(TALL, 3 * rounds(tall.share));
-  other(SMALL, 2 * rounds(small.share));
+  other(WIDE, takes.wide * rounds(wide.share));
+  other(TALL, takes.tall * rounds(tall.share));
+  other(SMALL, takes.small * rounds(small.share));
   const int rest = last(large.here);
   int i = blockIdx.x / 8;
   auto all = [&](const auto& tiles, const int end) {

@@ -45,12 +45,17 @@ struct Tiles {
   }
 };
 
+// where weights and rows come from the caches (K = 2048: 50 us for a large one, 18
+// for a small one); ops/__init__.py `_tile_plan` counts with the same
+constexpr tile::Rounds TAKES = {5, 3, 3, 2};
+
 template <int KIND, bool TWO>
 __global__ __launch_bounds__(256, 1) void tile_linear_kernel(const GemmArgs a,
                                                              const int T) {
   __shared__ __attribute__((aligned(1024))) short lds[tile::LDS];
-  tile::run<KIND, TWO>(a, lds, Tiles<8, 8, KIND>(a, T), Tiles<4, 8, KIND>(a, T),
-                       Tiles<8, 4, KIND>(a, T), Tiles<4, 4, KIND>(a, T));
+  tile::run<KIND, TWO>(a, lds, TAKES, Tiles<8, 8, KIND>(a, T),
+                       Tiles<4, 8, KIND>(a, T), Tiles<8, 4, KIND>(a, T),
+                       Tiles<4, 4, KIND>(a, T));
 }
 
 }  // namespace

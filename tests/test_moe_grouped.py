@@ -96,9 +96,10 @@ def test_grouped_rounds(counts, H, IE, mode, bias):
 @pytest.mark.parametrize("counts,H,IE,mode,bias", [
     ([1800, 1400, 1100, 700, 500, 300, 120, 81], 2880, 1024, 0, False),
     ([200] * 15, 320, 1088, 0, True),          # up: 256 rows x 128 weight rows
-    ([250, 130] * 4, 384, 1600, 1, True),      # 128 x 256
+    ([250, 130] * 4, 384, 1600, 1, True),
     ([120] * 8, 320, 2048, 0, False),          # 128 x 128, one round
-    ([130, 1] * 9, 576, 2112, 2, False),
+    ([20] * 64, 1024, 512, 0, False),          # two of them
+    ([130, 1] * 9, 576, 2112, 2, False),       # 128 x 256
     ([90, 0, 128] * 23, 64, 512, 0, True),     # more experts than lanes
 ])
 @pytest.mark.parametrize("f32", [False, True])
