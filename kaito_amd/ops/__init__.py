@@ -817,8 +817,8 @@ def latent_kv(c: torch.Tensor, w_kc: torch.Tensor, w_vc: torch.Tensor):
     w_kc [H, D, r] and w_vc [H, r, V]. One launch (and a transposition of
     w_vc) for prompts that fill the chip with 256 x 256 tiles, library products
     else (us, library and tiles, 128 + 128 dims of 512: 8192 rows of 16 heads
-    59.2, 41.0, 4096 34.0, 27.0, 2048 23.2, 22.3; 4096 of 128 heads 213, 149,
-    512 33.2, 33.4)."""
+    59.2, 41.0, 4096 34.0, 27.0, 2048 21.5, 21.6; 4096 of 128 heads 208, 134,
+    512 31.9, 32.7)."""
     T, (H, D, r), V = c.size(0), w_kc.shape, w_vc.size(2)
     if c.is_cuda and _latent_tiles(T, H * (D + V), r) and T < 1 << 22 \
             and c.dtype == w_kc.dtype == w_vc.dtype == torch.bfloat16 \
@@ -837,11 +837,14 @@ def latent_kv(c: torch.Tensor, w_kc: torch.Tensor, w_vc: torch.Tensor):
 
 
 def _latent_tiles(T: int, N: int, r: int) -> bool:
-    """More latent columns than 512 need more tiles for the library to be behind
-    (128 heads of 256 dims, 1536 columns, library over tiles: 1.07, 1.01, 1.01 at
-    512, 1024, 2048 tokens, 1.16 at 3000, 1.12 at 4096, 1.19 at 6000: the line is
-    where tiles of 8 waves drew level)."""
-    return T * N >= 4096 * 4096 * (1 if r <= 512 else 9)
+    """From a product of 4096 x 4096 on (library over tiles; 16 to 128 heads of 256
+    dims there: 1.19, 1.22, 1.14 with 256 latent columns, 1.19, 1.26, 1.12 with 512,
+    1.20, 1.18, 1.07 with 1024, 1.19, 1.15, 1.10 with 1536; half as large 1.02, 0.99,
+    0.90, 0.99, 0.79, 0.91, 0.95, 0.89; larger 1.1 to 2.0). Few tokens of many heads
+    are about even to 512 columns (128 heads of 512 tokens 0.93, 0.98, 256 of 256
+    0.99), beyond not before 640 (128 heads 0.96 at 512, 1.02 at 513, 1.20 at 640; 256
+    heads 0.71 at 256, 0.80 at 512)."""
+    return T * N >= 4096 * 4096 and (r <= 512 or T >= 640)
 
 
 def mla_prefill_attention(q, q_pe, k, k_pe, v, cu_seqlens, scale: float,

@@ -158,7 +158,9 @@ def test_latent_kv(T, H, D, V, K):
 
 @pytest.mark.parametrize("T,N,r,tiles", [
     (4096, 4096, 512, True), (4095, 4096, 512, False), (512, 32768, 512, True),
-    (3000, 32768, 1536, False), (6000, 32768, 1536, True),
+    (3000, 32768, 1536, True), (512, 32768, 1536, False),
+    (640, 32768, 1536, True), (2048, 4096, 1024, False),
+    (4096, 4096, 1536, True), (6000, 32768, 1536, True),
     (8192, 2048, 256, True)])
 def test_which_prompts_take_tiles(T, N, r, tiles):
     """The sides of the line on which either was measured to be faster."""
