@@ -505,16 +505,20 @@ def _uneven_shape(M: int, N: int, K: int) -> bool:
     number of rounds runs on the tiles, which cut the last round or take smaller
     ones. Whole rounds are the library's (0.94 to 0.99 times). us, library and
     tiles: 3072 x 2048 at 8192 rows 91, 84, 5901 86, 65; 5120 x 2048 at 3948 85,
-    68; 2048 x 2048 at 2585 31, 27; 1024 x 1536 at 8192 28, 26, at 4807 21, 22;
-    4096 x 1024 at 4162 56, 39; 3072 x 512 at 6541 51, 25; 4096 x 3072 at 4437
-    112, 93; 8192 x 3072 at 6309 270, 228, but 3072 x 3072 at 6962 112, 113 and
-    5120 x 3072 at 4206 111, 113; 100 sizes, 1.0 to 2.1 times as fast but for those
-    four. K of 4096 with a quartered round 1.06, with smaller tiles 0.99 to 1.02;
-    up to 1024 rows 0.4 to 1.1."""
+    68; 2048 x 2048 at 2585 31, 27; 1024 x 1536 at 8192 28, 26; 4096 x 1024 at 4162
+    56, 39; 3072 x 512 at 6541 51, 25; 4096 x 3072 at 4437 112, 93; 8192 x 3072 at
+    6309 270, 228. K of 4096 with a quartered round 1.06, with smaller tiles 0.99 to
+    1.02; up to 1024 rows 0.4 to 1.1. Smaller tiles that leave much of their rounds
+    idle are behind (1024 x 3072 at 4192 rows, 43 % busy, 31, 38; 2048 x 2560 at 2315,
+    47 %, 29, 34; 1024 x 1536 at 4807, 49 %, 21, 23; 2048 x 1536 at 2700, 55 %, 22, 23),
+    from 56 % on not: of 159 further sizes none is more than 1.4 % behind (1536 x 3072
+    at 16041 rows 118, 120; 5120 x 3072 at 4206 112, 113), 1.16 times as fast in the
+    mean."""
     if not (M > 2048 and 1024 <= N <= 8192 and K <= 4096):
         return False
     kind = _tile_plan(M, N)[0]
-    return kind == "quartered" or (kind == "smaller" and K <= 3072)
+    return kind == "quartered" or (kind == "smaller" and K <= 3072
+                                   and _tile_fill(M, N) >= 0.555)
 
 
 def _pair_tiled(x, w, x2, w2) -> bool:

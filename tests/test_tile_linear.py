@@ -126,7 +126,9 @@ def test_which_vocabularies_take_tiles(M, N, K, tiles):
 @pytest.mark.parametrize("M,N,K,tiles", [
     (8192, 3072, 2048, True), (8192, 2048, 2048, False), (2048, 1024, 512, False),
     (2049, 1024, 512, True), (2049, 1023, 512, False), (8192, 8256, 1024, False),
-    (5901, 3072, 4096, True), (8192, 3072, 3136, False)])
+    (5901, 3072, 4096, True), (8192, 3072, 3136, False),
+    (4807, 1024, 1536, False), (2700, 2048, 1536, False),
+    (2258, 2496, 2752, True), (6962, 3072, 3072, True)])
 def test_which_products_of_prompts_take_tiles(M, N, K, tiles):
     """The sides of the lines on which either was measured to be faster."""
     assert ops._uneven_shape(M, N, K) == tiles
