@@ -490,14 +490,19 @@ def _tiled_shape(M: int, N: int, K: int) -> bool:
 
 def _vocabulary_shape(M: int, N: int, K: int) -> bool:
     """Whether a large batch's logits run on the tiles, whose 256 rows are a
-    step's (us, library and tiles: 128256 x 4096 297, 234 at 129 rows, 262, 241 at
-    192, 310, 246 at 256; 151936 x 4096 309, 292 at 129, 363, 321 at 256; 256000 x
-    4096 553, 477; 128256 x 8192 464, 450 at 160, 548, 472 at 256; 128256 x 6144
-    351, 341 at 144, 448, 361 at 256; 131072 x 5120 279, 294 at 144, 338, 313 at
-    256. Fewer rows or a shorter K went either way: 262144 x 2304 0.94 to 0.98,
-    151936 x 4096 1.0 to 1.02 from 33 to 64 rows, 128256 x 8192 0.94 to 1.02)."""
-    return 129 <= M <= 256 and N >= 100000 and K >= 4096 \
-        and (M > 224 or not 4096 < K < 6144)
+    step's (us, library and tiles: 128256 x 4096 290, 220 at 129 rows, 258, 225 at
+    192, 299, 239 at 256; 151936 x 4096 303, 293 at 129, 356, 311 at 256; 256000 x
+    4096 553, 477; 128256 x 8192 460, 427 at 160, 547, 469 at 256; 128256 x 6144
+    361, 352 at 160, 446, 362 at 256; 131072 x 5120 279, 294 at 144, 338, 313 at
+    256; 100352 x 4096 230, 201 at 129, 202, 203 at 160, 229, 205 at 256, x 6144 306,
+    303 at 160, but x 8192 358, 390 at 160 and 385, 390 at 224. Fewer rows or a shorter
+    K went either way: 262144 x 2304 0.94 to 0.98, 128256 x 2048 0.95 to 1.24, 151936 x
+    4096 1.0 to 1.02 from 33 to 64 rows, 128256 x 8192 0.94 to 1.02. So do smaller
+    vocabularies, by how full their last round is: 92416 x 4096 to 8192 0.73 to 0.91,
+    81920 1.04 to 1.25, 65536 0.93 to 1.09, 49152 0.93 to 1.11, 32000 0.73 to
+    0.95)."""
+    return 129 <= M <= 256 and N >= (128000 if K >= 8192 else 100000) \
+        and K >= 4096 and (M > 224 or not 4096 < K < 6144)
 
 
 def _uneven_shape(M: int, N: int, K: int) -> bool:

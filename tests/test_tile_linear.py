@@ -118,7 +118,9 @@ def test_which_two_products_take_tiles(M, N, K, tiles):
     (128, 128256, 4096, False), (129, 128256, 4096, True),
     (256, 128256, 4096, True), (257, 128256, 4096, False),
     (144, 131072, 5120, False), (256, 131072, 5120, True),
-    (256, 262144, 2304, False), (200, 32000, 4096, False)])
+    (256, 262144, 2304, False), (200, 32000, 4096, False),
+    (160, 100352, 8192, False), (160, 100352, 6144, True),
+    (160, 128256, 8192, True)])
 def test_which_vocabularies_take_tiles(M, N, K, tiles):
     assert ops._vocabulary_shape(M, N, K) == tiles
 
