@@ -126,7 +126,13 @@ __global__ __launch_bounds__(256) void w4a16_mfma_kernel(
 // 2 rows, 10.4 -> 9.2 us, 28672 x 2560 13.2 -> 11.5, as a pair 28672 x 4096 15.9 ->
 // 14.8, with the norm 16.8 -> 15.6 (57344 x 8192 44.6 both; fewer tiles the same or
 // slower). x is asked for ahead of the weights, behind which its loads would end:
-// 4096 x 14336 11.2 -> 9.7, 28672 x 4096 as a pair, 5 rows, 17.3 -> 16.0. The wave
+// 4096 x 14336 11.2 -> 9.7, 28672 x 4096 as a pair, 5 rows, 17.3 -> 16.0. Little of it
+// is not: 8 loads of a thread, most of them of nothing new, hold the weights up for
+// longer than x behind them takes (2 rows, pairs, x ahead and behind, 2048 x 2048 4.9
+// and 4.5, 4096 x 1024 4.9 and 4.5, 7168 x 2048 6.4 and 6.1, one row of 4096 x 4096 5.7
+// and 5.4, 16 of 4096 x 512 5.3 and 4.9, but 16 of 4096 x 2048 6.6 and 6.9, 6144 x 4096
+// 7.4 and 7.8; asked for only where there is some: 5.1, 4.7, and 5.9 -> 6.2 of 8704 x
+// 2048, as the waits count for either). The wave
 // that sums by turns: no change. The time hardly grows
 // with the rows. us, rows streamed (5 rows and more: MFMA from global memory) and
 // tiles before these two, at 1, 2, 3, 4, 8 rows: 28672 x 4096 15.8 19.7 23.6 33.2 37.7 and 16.7 17.4
@@ -169,7 +175,7 @@ constexpr int W4_AHEAD = 8;         // 16-byte parts of x that a thread asks for
 // and to the same bits, while the first weights are on the way; its launch is
 // saved: us, two launches and one, 28672 x 4096 20.1, 17.7 for two rows, 22016 x
 // 5120 21.4, 19.1 for one and 22.2, 19.6, 57344 x 8192 48.2, 44.3 and 53.9, 47.0.
-template <int NW, int MR, int DEPTH, bool GLU, bool NORM>
+template <int NW, int MR, int DEPTH, bool GLU, bool NORM, int AHEAD = W4_AHEAD>
 __global__ __launch_bounds__(64 * NW, 2) void w4a16_tiles_kernel(
     short* __restrict__ out, const short* __restrict__ x,
     const uint32_t* __restrict__ qw, const float* __restrict__ scales,
@@ -233,7 +239,7 @@ __global__ __launch_bounds__(64 * NW, 2) void w4a16_tiles_kernel(
   const int nm = wave / 4 * NR, nat = (threadIdx.x & 255) * 8;  // row, first k
   short8_t nv[NR][NORM ? W4_NORM : 1], nr[NR][NORM ? W4_NORM : 1],
       ng[NORM ? W4_NORM : 1];
-  hbf16x8 xv[NORM ? 1 : W4_AHEAD];
+  hbf16x8 xv[NORM || !AHEAD ? 1 : AHEAD];
   // x ahead of the weights: loads end in order
   if constexpr (NORM) {
 #pragma unroll
@@ -251,7 +257,7 @@ __global__ __launch_bounds__(64 * NW, 2) void w4a16_tiles_kernel(
     }
   } else {
 #pragma unroll
-    for (int i = 0; i < W4_AHEAD; i++)
+    for (int i = 0; i < AHEAD; i++)
       xv[i] = skinny::load_x(
           x + min(i * 64 * NW + (int)threadIdx.x, M * K / 8 - 1) * 8);
   }
@@ -323,7 +329,7 @@ __global__ __launch_bounds__(64 * NW, 2) void w4a16_tiles_kernel(
     };
     int c = threadIdx.x;
 #pragma unroll
-    for (int i = 0; i < W4_AHEAD; i++, c += 64 * NW)
+    for (int i = 0; i < AHEAD; i++, c += 64 * NW)
       if (c < M * K / 8) place(c, xv[i]);     // uniform in 16 lanes
     for (; c < M * K / 8; c += 64 * NW)
       place(c, skinny::load_x(x + (int64_t)c * 8));
@@ -451,8 +457,11 @@ bool launch_w4_tiles(at::Tensor& out, const at::Tensor& x,
   const int ntiles = N / (GLU ? 8 : 16);
   // two workgroups of four waves per CU, where x fits twice
   const bool two = M <= 4 && ntiles >= 512 && w4_fits(4, 3, 4, M, K);
-#define W4T_LAUNCH(NW_, MR_, D_)                                              \
-  hipLaunchKernelGGL((w4a16_tiles_kernel<NW_, MR_, D_, GLU, NORM>),           \
+  const bool brief =
+      K <= 2048 ? M * K <= 16384 : M * K <= 8192 && ntiles <= 256;
+#define W4T_LAUNCH(NW_, MR_, D_, ...)                                         \
+  hipLaunchKernelGGL(                                                         \
+      (w4a16_tiles_kernel<NW_, MR_, D_, GLU, NORM, ##__VA_ARGS__>),           \
       dim3(std::min(2048 / NW_, ntiles)), dim3(64 * NW_), 0,                  \
       at::hip::getCurrentHIPStream(), (short*)out.data_ptr(),                 \
       (const short*)x.data_ptr(), (const uint32_t*)qweight.data_ptr(),        \
@@ -460,9 +469,13 @@ bool launch_w4_tiles(at::Tensor& out, const at::Tensor& x,
   if (two) {
     W4T_LAUNCH(4, 4, 3);
   } else if (M <= 4) {
-    if (depth == 3) W4T_LAUNCH(8, 4, 3); else W4T_LAUNCH(8, 4, 2);
+    if (!NORM && brief) W4T_LAUNCH(8, 4, 3, 0);
+    else if (depth == 3) W4T_LAUNCH(8, 4, 3);
+    else W4T_LAUNCH(8, 4, 2);
   } else if constexpr (!NORM) {
-    if (depth == 3) W4T_LAUNCH(8, 16, 3); else W4T_LAUNCH(8, 16, 2);
+    if (brief) W4T_LAUNCH(8, 16, 3, 0);
+    else if (depth == 3) W4T_LAUNCH(8, 16, 3);
+    else W4T_LAUNCH(8, 16, 2);
   }
 #undef W4T_LAUNCH
   return true;
