@@ -426,15 +426,16 @@ int w4_tiles_depth(int64_t M, int64_t rows, int64_t K, int64_t group) {
 // 12288 x 2048 6.4 and 6.6, 16384 x 2048 6.9 and 7.6. Three or four of a narrow K with 4096 rows of W (2048 x 2048 4.4 and 4.7,
 // 11008 .84). More, from K of 2048 on (4096 x 1024 3.8 and 4.6 at 5, 57344 x 512 9.7
 // and 20.2), beyond 8 rows at 2048 with 6144 of W (4096: 6.1 and 6.7 at 16).
-//   A pair saves a launch. One row: few rows of W (4096 .83 to .95; 6144 x 4096
-// 7.7 and 8.1, 22016 x 2048 9.7 and 11.7, 28672 x 4096 1.04) and many of a wide K
-// (11008 x 5120 .96, 28672 x 7168 .79). Two: not with many rows of a narrow K
-// (57344 x 2048 20.1 and 21.6). From five on K up to 1024 only with few (22016 x
-// 512 7.4 and 11.0, 22016 x 1024 1.04).
+//   A pair saves a launch. One row: but for some 400 tiles, which are neither two
+// rounds of one workgroup per CU nor enough for two (6144 x 2048 5.5 and 5.7, x 4096
+// 7.0 and 7.2, x 8192 10.5 and 10.4; 4096 x 4096 6.5 and 5.4, 5120 x 2048 5.4 and 5.5,
+// 7168 x 2048 6.0 and 5.9, x 4096 8.2 and 7.5, 28672 x 4096 17.6 and 15.1, 57344 x 8192
+// 60.9 and 46.9, others 1.03 to 1.35). Two: always (6144 x 2048 6.8 and 5.9, 28672 x
+// 4096 18.1 and 15.7, 57344 x 1024 18.9 and 13.2). From five on K up to 1024 only with
+// few (22016 x 512 7.4 and 11.0, 22016 x 1024 1.04).
 bool w4_tiles_pay(int64_t M, int64_t rows, int64_t K, bool glu) {
   if (glu) {
-    if (M == 1) return rows < 6144 || (rows >= 11008 && K >= 5120);
-    if (M == 2) return K > 2048 || rows <= 11008;
+    if (M <= 2) return M == 2 || rows < 6144 || rows >= 7168;
     return M <= 4 || K > 1024 || rows <= 4096;
   }
   if (M == 1) return false;

@@ -203,9 +203,11 @@ def test_w4_tiles_of_two_workgroups(M, N, K):
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,rows,K,alone,pair", [
     (1, 4096, 4096, False, True), (1, 6144, 4096, False, False),
-    (1, 28672, 4096, False, False), (1, 28672, 7168, False, True),
+    (1, 28672, 4096, False, True), (1, 28672, 7168, False, True),
+    (1, 5120, 2048, False, True), (1, 6656, 2048, False, False),
+    (1, 7168, 2048, False, True),
     (2, 28672, 4096, True, True), (2, 4096, 14336, True, True),
-    (2, 12288, 2048, False, False), (2, 57344, 1024, False, False),
+    (2, 12288, 2048, False, True), (2, 57344, 1024, False, True),
     (3, 2048, 2048, False, True), (3, 11008, 2048, True, True),
     (4, 1024, 4096, True, True), (5, 4096, 1024, False, True),
     (5, 22016, 512, False, False), (8, 4096, 2048, True, True),
