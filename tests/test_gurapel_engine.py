@@ -341,3 +341,22 @@ def test_preemption_recomputes_state(tmp_path_factory):
     assert [o.output_token_ids for o in got] == want
     assert tight.state_pool.num_free == 4
     assert tight.pool.num_free == tight.pool.num_blocks
+
+
+@pytest.mark.parametrize("mode", [("cpu", "float32"), pytest.param(
+    ("cuda", "bfloat16"), marks=pytest.mark.gpu)])
+def test_hooked_embedding_is_called(tmp_path_factory, mode):
+    """By the model too, whose own launch would pass the hook by."""
+    cfg, _, folder = checkpoint(tmp_path_factory, "c")
+    m = engine(folder, mode).runner.model
+    m.layers = torch.nn.ModuleList()
+    ids = torch.tensor(tokens(cfg, 9, 3), device=m.lm_head.device)
+    pos = torch.arange(9, device=ids.device)
+    plain = m(ids, pos, [], None)
+    rows = m.embed_tokens.weight[ids].float() * m.cfg.embed_scale
+    assert torch.equal(plain, rows + m.pos_embed[pos].float())
+    handle = m.embed_tokens.register_forward_hook(lambda mod, i, o: o * 2)
+    assert torch.equal(m(ids, pos, [], None),
+                       rows * 2 + m.pos_embed[pos].float())
+    handle.remove()
+    assert torch.equal(m(ids, pos, [], None), plain)

@@ -650,9 +650,8 @@ def test_embed_positions_outside_a_table():
     assert torch.equal(got[1], (a + b).bfloat16())
 
 
-@pytest.mark.gpu
-def test_hooked_embedding_is_called():
-    from kaito_amd.parallel.layers import looks_up
+def test_embeddings_that_only_look_up():
+    from kaito_amd.models.gurapel import looks_up
     e = torch.nn.Embedding(4, 8)
     assert looks_up(e)
     handle = e.register_forward_hook(lambda m, i, o: o + 1)

@@ -94,6 +94,85 @@ def test_forms_that_tiles_do_not_take():
     assert x.grad is not None
 
 
+@pytest.mark.gpu
+def test_rows_without_a_value_stay_among_themselves():
+    """A row or a weight row of infinities or NaN, in tiles of finite ones."""
+    torch.manual_seed(0)
+    M, N, K = 300, 576, 192
+    x, w, pair = _rand(M, K), _rand(N, K), _rand(2 * N, K)
+    x[5, 7], x[131, 0], x[299] = float("inf"), float("nan"), float("-inf")
+    w[64, 3], pair[N + 64, 3] = float("nan"), float("nan")
+    rows = torch.ones(M, dtype=torch.bool, device=DEV)
+    rows[[5, 131, 299]] = False
+    cols = torch.ones(N, dtype=torch.bool, device=DEV)
+    cols[64] = False
+    out, act = (torch.empty(M, N, device=DEV).to(torch.bfloat16) for _ in "oa")
+    ops._K.tile_linear(out, x, w)
+    ops._K.tile_swiglu(act, x, pair)
+    g, u = (x.double() @ pair.double().T).chunk(2, -1)
+    for y, ref in ((out, x.double() @ w.double().T),
+                   (act, g * torch.sigmoid(g) * u)):
+        _close(y[rows][:, cols], ref[rows][:, cols])
+        assert y[131].isnan().all() and y[:, 64].isnan().all()
+    assert not out[[5, 299]].isfinite().any()
+    # the same rows as two experts'
+    off = torch.tensor([0, 131, M], dtype=torch.int32, device=DEV)
+    y = torch.empty(M, N, device=DEV)
+    ops._K.moe_grouped_down(y, x, w[None].repeat(2, 1, 1), off,
+                            torch.empty(0, device=DEV), 0)
+    ref = x.double() @ w.double().T
+    _close(y[rows][:, cols], ref[rows][:, cols])
+    assert y[131].isnan().all() and y[:, 64].isnan().all()
+
+
+@pytest.mark.gpu
+def test_another_stream():
+    """What the caller's stream holds is waited for, and no other stream is."""
+    torch.manual_seed(0)
+    x, w, pair = _rand(3000, 1024), _rand(2112, 1024), _rand(4096, 1024)
+    assert ops._uneven_shape(3000, 2112, 1024) and ops._tiled(x, pair)
+    want = [ops.linear(x, w), ops.linear_swiglu(x, pair)]
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        z = _rand(4096, 4096)
+        for _ in range(20):
+            z = z @ z * 2 ** -7
+        late = torch.empty_like(x).copy_(x)   # behind them
+        got = [ops.linear(late, w), ops.linear_swiglu(late, pair)]
+    side.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.gpu
+def test_operands_that_the_kernels_refuse():
+    x, w, out = _rand(40, 128), _rand(64, 128), _rand(40, 64)
+    wide, none = _rand(40 * 128 + 8), torch.empty(0, device=DEV)
+    linear = [
+        (out.float(), x, w), (out, x.float(), w), (out, x, w.half()),
+        (out, x.cpu(), w), (out[:, ::2], x, w[::2].contiguous()),
+        (out, x[:, :64], w[:, :64]), (out, wide[4:-4].view(40, 128), w),
+        (out, x[:, :32].contiguous(), w[:, :32].contiguous()),
+        (out[:20], x, w), (out, x, w[:32]), (out, x, _rand(64, 192)),
+        (_rand(40, 32), x, w[:32].contiguous())]
+    for args in linear:
+        with pytest.raises(RuntimeError):
+            ops._K.tile_linear(*args)
+    with pytest.raises(RuntimeError):
+        ops._K.tile_swiglu(out, x, w)
+    big, big_out = _rand(256, 128), _rand(40, 256)
+    pairs = [
+        (out, x, w, none, out, x, w, none),           # first not by 256
+        (big_out, x, big, _rand(64), out, x, w, none),
+        (big_out, x, big, none, out, x, w, torch.zeros(64, device=DEV)),
+        (big_out, x, big, none, _rand(41, 64), _rand(41, 128), w, none)]
+    for args in pairs:
+        with pytest.raises(RuntimeError):
+            ops._K.tile_pair(*args)
+    ops._K.tile_pair(big_out, x, big, none, out, x, w, none)
+    _close(out, x.double() @ w.double().T)
+
+
 @pytest.mark.parametrize("M,N,K,tiles", [
     (256, 28672, 4096, False), (512, 28672, 4096, True),
     (700, 28672, 4096, False), (8192, 28672, 4096, True),
