@@ -334,7 +334,9 @@ def _plain_bias(bias, w: torch.Tensor) -> bool:
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
     """x W^T (+ bias): the weight-streaming kernels for small decode steps, the
-    split kernel for larger ones where it is ahead, hipBLASLt otherwise."""
+    split kernel for larger ones where it is ahead, the tiles for large batches'
+    logits and for prompts whose large tiles fill no whole number of rounds,
+    hipBLASLt otherwise."""
     if _plain_bias(bias, w):
         skinny = _skinny(x, w)
         if skinny or _batched(x, w):

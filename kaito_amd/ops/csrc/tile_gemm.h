@@ -10,9 +10,10 @@
 // What bounds large products here is power: the clock drops until the chip stays
 // within its budget. Hence (one MI355X, 8192 x 4096 x 14336, where a library product
 // reaches 1600 TFLOP/s; 8 waves of 128 x 64 on 32 x 32 tiles, as before: 1180):
-//   - 16x16x32 instead of 32x32x16: alone, on random data, 2065 and 1818 TFLOP/s;
+//   - 16x16x32 instead of 32x32x16: alone, on random data, 1940 TFLOP/s at 2.0 GHz
+//     and 1780 at 1.8 (on zeros 2330 and 2410, at 2.4 and 2.3);
 //   - 128 x 128 per wave: a fragment that is read serves 8 products, of 128 x 64 some
-//     5.3; LDS is busy a third of the time instead of all of it;
+//     5.3; LDS is busy 20 % of the time instead of 55;
 //   - sums in accumulation registers through inline assembly, by name: with the
 //     intrinsic the compiler moved 17 of 64 tiles of sums between the files in
 //     every step;
