@@ -458,8 +458,11 @@ bool launch_w4_tiles(at::Tensor& out, const at::Tensor& x,
   const int ntiles = N / (GLU ? 8 : 16);
   // two workgroups of four waves per CU, where x fits twice
   const bool two = M <= 4 && ntiles >= 512 && w4_fits(4, 3, 4, M, K);
-  const bool brief =
-      K <= 2048 ? M * K <= 16384 : M * K <= 8192 && ntiles <= 256;
+  // little of x, asked for behind the weights; few tiles: 3 rows, x ahead and behind,
+  // 1024 x 3072 5.1 and 4.8, 4096 x 3584 5.84 and 5.72, but 4096 x 4096 5.9 and 6.1, 5 of
+  // 1024 x 3584 5.2 and 5.5, 6 of 4608 x 3072 6.7 and 7.1
+  const bool brief = K <= 2048
+      ? M * K <= 16384 : ntiles <= 256 && M * K <= (K < 4096 ? 16384 : 8192);
 #define W4T_LAUNCH(NW_, MR_, D_, ...)                                         \
   hipLaunchKernelGGL(                                                         \
       (w4a16_tiles_kernel<NW_, MR_, D_, GLU, NORM, ##__VA_ARGS__>),           \

@@ -149,7 +149,7 @@ def test_transformed_calls_are_seen():
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8, 14, 16])
 @pytest.mark.parametrize("N,K", [(8, 512), (24, 4608), (2056, 1536),
-                                 (2080, 2048), (16, 14336)])
+                                 (2080, 2048), (40, 3584), (16, 14336)])
 def test_w4_tiles(M, N, K):
     """x in LDS: fewer tiles than workgroups and several each, waves without a
     stage, rings of two and three stages, sizes that do not fit."""
