@@ -542,8 +542,13 @@ def _pair_tiled_shape(M: int, N: int, K: int) -> bool:
     2048: 3072 + 576 at 128 rows 20, 16, 700 28, 19, 2048 42, 31, 8192 120, 99, at
     64 17, 16; 3072 + 4096 at 128 30, 23, 2048 67, 55, 6500 170, 149, but 87, 93 at
     3000, 100, 102 at 4096 and 187, 191 at 8192; 2048 + 576 at 8192 79, 82). K of
-    5120 and 7168 gave 0.54 to 1.38 times."""
+    5120 and 7168 gave 0.54 to 1.38 times. Few outputs of a long K gain little with
+    weights from memory and lose with those that are in the caches (512 + 320 of 2048 at
+    168 rows 16.3, 16.2 and 11.2, 16.0; 512 + 64 at 653 17.4, 16.5 and 14.3, 16.4; 2048 +
+    64 of 1536 at 154 14.2, 13.5 and 12.1, 13.2), more of them with neither (3072 + 576 at
+    241 17.5, 16.6 from the caches)."""
     return M >= 128 and K <= 2048 and N <= 7168 and (
+        M * N >= 400000 or K <= 1024) and (
         M * N <= 20000000 or _tile_fill(M, N) >= 0.88)
 
 

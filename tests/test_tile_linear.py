@@ -188,6 +188,8 @@ def test_which_pairs_take_tiles(M, N, K, tiles):
     (127, 3648, 2048, False), (128, 3648, 2048, True),
     (8192, 3648, 2048, True), (3000, 7168, 2048, False),
     (6500, 7168, 2048, True), (8192, 2624, 2048, False),
+    (168, 832, 2048, False), (154, 2112, 1536, False), (168, 832, 1024, True),
+    (241, 3648, 2048, True),
     (1000, 2112, 7168, False)])
 def test_which_two_products_take_tiles(M, N, K, tiles):
     assert ops._pair_tiled_shape(M, N, K) == tiles
