@@ -496,15 +496,23 @@ def _vocabulary_shape(M: int, N: int, K: int) -> bool:
     192, 299, 239 at 256; 151936 x 4096 303, 293 at 129, 356, 311 at 256; 256000 x
     4096 553, 477; 128256 x 8192 460, 427 at 160, 547, 469 at 256; 128256 x 6144
     361, 352 at 160, 446, 362 at 256; 131072 x 5120 279, 294 at 144, 338, 313 at
-    256; 100352 x 4096 230, 201 at 129, 202, 203 at 160, 229, 205 at 256, x 6144 306,
-    303 at 160, but x 8192 358, 390 at 160 and 385, 390 at 224. Fewer rows or a shorter
+    256; 100352 x 4096 230, 201 at 129, 202, 203 at 160, 229, 205 at 256, but x 8192 358,
+    390 at 160 and 385, 390 at 224. Fewer rows or a shorter
     K went either way: 262144 x 2304 0.94 to 0.98, 128256 x 2048 0.95 to 1.24, 151936 x
     4096 1.0 to 1.02 from 33 to 64 rows, 128256 x 8192 0.94 to 1.02. So do smaller
     vocabularies, by how full their last round is: 92416 x 4096 to 8192 0.73 to 0.91,
     81920 1.04 to 1.25, 65536 0.93 to 1.09, 49152 0.93 to 1.11, 32000 0.73 to
-    0.95)."""
-    return 129 <= M <= 256 and N >= (128000 if K >= 8192 else 100000) \
-        and K >= 4096 and (M > 224 or not 4096 < K < 6144)
+    0.95). Of a K of 6144 and more, up to 192 rows are ahead only where the last round
+    is full (library over tiles at 144 and 160 rows, 128256 x 7168 1.08, 1.08, 102400
+    0.96, 0.94, 120832 0.97, 0.94, 151936 0.93, 1.05, x 8192 0.90, 1.02, x 6144 0.95,
+    1.03, 112640 x 6144 0.97, 0.96; at 208 and 256 102400 x 7168 1.09, 1.08, 151936 x
+    8192 1.03, 1.14)."""
+    if not (129 <= M <= 256 and K >= 4096
+            and N >= (128000 if K >= 8192 else 100000)
+            and (M > 224 or not 4096 < K < 6144)):
+        return False
+    tiles = -(-N // 256)
+    return K < 6144 or M > 200 or tiles >= 0.95 * 256 * -(-tiles // 256)
 
 
 def _uneven_shape(M: int, N: int, K: int) -> bool:

@@ -200,8 +200,10 @@ def test_which_two_products_take_tiles(M, N, K, tiles):
     (256, 128256, 4096, True), (257, 128256, 4096, False),
     (144, 131072, 5120, False), (256, 131072, 5120, True),
     (256, 262144, 2304, False), (200, 32000, 4096, False),
-    (160, 100352, 8192, False), (160, 100352, 6144, True),
-    (160, 128256, 8192, True)])
+    (160, 100352, 8192, False), (160, 100352, 6144, False),
+    (160, 128256, 8192, True), (160, 128256, 7168, True),
+    (160, 102400, 7168, False), (256, 102400, 7168, True),
+    (144, 151936, 8192, False), (144, 151936, 4096, True)])
 def test_which_vocabularies_take_tiles(M, N, K, tiles):
     assert ops._vocabulary_shape(M, N, K) == tiles
 
