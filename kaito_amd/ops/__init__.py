@@ -526,14 +526,21 @@ def _uneven_shape(M: int, N: int, K: int) -> bool:
     1.02; up to 1024 rows 0.4 to 1.1. Smaller tiles that leave much of their rounds
     idle are behind (1024 x 3072 at 4192 rows, 43 % busy, 31, 38; 2048 x 2560 at 2315,
     47 %, 29, 34; 1024 x 1536 at 4807, 49 %, 21, 23; 2048 x 1536 at 2700, 55 %, 22, 23),
-    from 56 % on not: of 159 further sizes none is more than 1.4 % behind (1536 x 3072
-    at 16041 rows 118, 120; 5120 x 3072 at 4206 112, 113), 1.16 times as fast in the
-    mean."""
-    if not (M > 2048 and 1024 <= N <= 8192 and K <= 4096):
+    from 56 % on not; 128 x 256 with a K of 1024 and more from 62 % on (1536 x 2048 at
+    4000, 61 %, 27.0, 28.1, 1408 x 2560 at 4176, 58 %, 33, 35, 2560 x 1280 at 2233, 57 %,
+    20, 21). One round of quarters is even or behind
+    below 45 % (1024 rows of W at 2570, 39 %: x 256 6.8, 7.2, x 512 10.8, 8.2, x 1024 11.3,
+    11.6, x 4096 27.9, 30.0; at 47 % x 4096 1.05). K below 256 went either way (0.81 to
+    1.6). Of 480 sizes 2 are more than 1.5 % behind (2560 x 2560 at 8445 97.9, 100.3),
+    1.20 times as fast in the mean."""
+    if not (M > 2048 and 1024 <= N <= 8192 and 256 <= K <= 4096):
         return False
-    kind = _tile_plan(M, N)[0]
-    return kind == "quartered" or (kind == "smaller" and K <= 3072
-                                   and _tile_fill(M, N) >= 0.555)
+    kind, cost = _tile_plan(M, N)
+    fill = _tile_fill(M, N)
+    if cost == 2 and fill < 0.45 and not 256 < K <= 512:
+        return False
+    return kind == "quartered" or (kind == "smaller" and K <= 3072 and fill >= (
+        0.555 if K < 1024 or cost == 2 else 0.62))
 
 
 def _pair_tiled(x, w, x2, w2) -> bool:

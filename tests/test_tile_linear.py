@@ -213,7 +213,10 @@ def test_which_vocabularies_take_tiles(M, N, K, tiles):
     (2049, 1024, 512, True), (2049, 1023, 512, False), (8192, 8256, 1024, False),
     (5901, 3072, 4096, True), (8192, 3072, 3136, False),
     (4807, 1024, 1536, False), (2700, 2048, 1536, False),
-    (2258, 2496, 2752, True), (6962, 3072, 3072, True)])
+    (2377, 2496, 2752, False), (6962, 3072, 3072, True),
+    (2570, 1024, 256, False), (2570, 1024, 512, True), (2570, 1024, 4096, False),
+    (3100, 1024, 4096, True), (4000, 1536, 2048, False), (4000, 1536, 768, True),
+    (2826, 2048, 3072, False), (5000, 4096, 128, False)])
 def test_which_products_of_prompts_take_tiles(M, N, K, tiles):
     """The sides of the lines on which either was measured to be faster."""
     assert ops._uneven_shape(M, N, K) == tiles
@@ -222,14 +225,19 @@ def test_which_products_of_prompts_take_tiles(M, N, K, tiles):
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(2049, 1024, 64), (2305, 1088, 192),
                                    (5901, 3072, 128), (8190, 2560, 192),
-                                   (2060, 8192, 320)])
+                                   (2060, 8192, 320), (2305, 1088, 320),
+                                   (3000, 2112, 256)])
 def test_uneven_products(M, N, K, monkeypatch):
     """Last rounds in quarters and smaller tiles, rows that end inside one."""
     torch.manual_seed(M)
-    assert ops._uneven_shape(M, N, K)
     x, w = _rand(M, K), _rand(N, K, std=K ** -0.5)
-    monkeypatch.setattr(torch.nn.functional, "linear", None)
-    _close(ops.linear(x, w), x.double() @ w.double().T)
+    out = torch.full((M, N), float("nan"), device=DEV).to(torch.bfloat16)
+    ops._K.tile_linear(out, x, w)
+    _close(out, x.double() @ w.double().T)
+    assert ops._uneven_shape(M, N, K) == (K >= 256)
+    if K >= 256:
+        monkeypatch.setattr(torch.nn.functional, "linear", None)
+        assert torch.equal(ops.linear(x, w), out)
 
 
 def _all_close(out, ref, rows=1 << 16):
@@ -315,11 +323,11 @@ def test_rows_too_wide_for_the_tiles():
 def test_another_device_is_current(monkeypatch):
     """Prompts whose device is not the current one are torch's, which switches."""
     torch.manual_seed(0)
-    x, w, w2 = _rand(2305, 192), _rand(1088, 192), _rand(1024, 192)
+    x, w, w2 = _rand(2305, 320), _rand(1088, 320), _rand(1024, 320)
     rows, pair = _rand(1000, 2048), _rand(4096, 2048)
     table, where = _rand(300, 64), _rand(70, 64)
     ids = torch.arange(9, device=DEV)
-    assert ops._uneven_shape(2305, 1088, 192) and ops._tiles_fit(x, w, 64)
+    assert ops._uneven_shape(2305, 1088, 320) and ops._tiles_fit(x, w, 64)
     assert ops._pair_tiled(x, w2, x, w) and ops._tiled(rows, pair)
     monkeypatch.setattr(torch.cuda, "current_device", lambda: x.device.index + 1)
     for op in ("tile_linear", "tile_pair", "tile_swiglu", "embed_positions"):
