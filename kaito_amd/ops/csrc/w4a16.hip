@@ -701,17 +701,20 @@ bool w4a16_in_tiles(int64_t M, int64_t rows, int64_t K, int64_t group,
 }
 
 // Whether the norm of up to two rows goes into their product in the tiles: but for
-// one row of few whole streams (us, norm and what else would follow it, and one
-// launch: one row of 6144 x 4096 8.2 and 8.7, 5120 x 2048 5.7 and 6.3, 10240 x 8192
-// 15.4 and 15.2, 7168 x 5120 11.3 and 10.3, 2048 x 1024 4.8 and 4.6, 28672 x 512 9.6
-// and 7.6; pairs 28672 x 4096 19.5 and 15.8, 57344 x 8192 48.0 and 44.6, 4096 x 512
-// 6.3 and 4.6; two rows of 6144 x 4096 10.0 and 8.8, 10240 x 8192 18.0 and 15.5,
-// 1536 x 512 5.3 and 4.6; pairs 28672 x 4096 18.1 and 16.0, 57344 x 1024 20.9 and
+// one row of few whole streams and of some 350 tiles (us, norm and what else would
+// follow it, and one launch: one row of 6144 x 4096 8.2 and 8.7, 5120 x 2048 5.7 and
+// 6.3, 20480 x 2048 9.0 and 9.4, 28672 x 2048 1.06, 10240 x 4096 9.7 and 9.9, 12288 x
+// 4096 1.10, 10240 x 8192 1.06; 6144 x 512 5.0 and 5.4, x 1024 5.2 and 5.6, 5120 x 5120
+// 9.3 and 9.5, but 7168 x 5120 11.3 and 10.3, 4096 x 1024 1.06; 2048 x 1024 4.8 and 4.6,
+// 28672 x 512 9.6 and 7.6; pairs 28672 x 4096 19.5 and 15.8, 57344 x 8192 48.0 and 44.6,
+// 4096 x 512 6.3 and 4.6; two rows of 6144 x 4096 10.0 and 8.8, 10240 x 8192 18.0 and
+// 15.5, 1536 x 512 5.3 and 4.6; pairs 28672 x 4096 18.1 and 16.0, 57344 x 1024 20.9 and
 // 14.1).
 bool w4a16_norm_in_tiles(int64_t M, int64_t rows, int64_t K, int64_t group,
                          bool glu) {
-  return M <= 2 && K <= 2048 * W4_NORM &&
-         (glu || M == 2 || K % 2048 || rows >= 10240) &&
+  const bool one = K % 2048 ? rows <= 4096 || rows >= 7168
+                            : rows >= 10240 && rows * K >= 48 << 20;
+  return M <= 2 && K <= 2048 * W4_NORM && (glu || M == 2 || one) &&
          w4_tiles_depth(M, rows, K, group) > 0;
 }
 

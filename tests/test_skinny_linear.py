@@ -221,6 +221,19 @@ def test_which_packed_sizes_take_tiles(M, rows, K, alone, pair):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows,K,alone", [
+    (4096, 1024, True), (5120, 1024, False), (6144, 512, False),
+    (7168, 5120, True), (6144, 4096, False), (20480, 2048, False),
+    (28672, 2048, True), (10240, 4096, False), (12288, 4096, True),
+    (8192, 8192, False), (10240, 8192, True)])
+def test_which_packed_products_take_one_row_s_norm(rows, K, alone):
+    """The sides of the lines on which either was measured to be faster."""
+    assert ops._K.w4a16_norm_in_tiles(1, rows, K, 128, False) == alone
+    assert ops._K.w4a16_norm_in_tiles(1, rows, K, 128, True)
+    assert ops._K.w4a16_norm_in_tiles(2, rows, K, 128, False)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 16, 17, 32])
 @pytest.mark.parametrize("N,K,G", [(1, 64, 64), (40, 128, 128),
                                    (33, 192, 192), (100, 4224, 128),
