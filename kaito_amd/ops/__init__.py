@@ -484,14 +484,14 @@ def _tiled_shape(M: int, N: int, K: int) -> bool:
     8192 339, 189, at 1000, 57 %, 43, 54; 16384 x 3072 at 1500, 81 %, 144, 158;
     4096 x 2048 at 1000 26, 20, 8192 118, 107; 1024 x 2048 at 2048, 31 %, 20, 19 and
     1500 18, 19; 2816 x 2048 at 1500, 42 %, 28, 27; in one round of 256 x 256 3584 x 2048
-    at 2378, 51 %, 39.6, 41.3, 2816 x 2048 at 3176, 53 %, 40.3, 41.0, 3584 x 2048 at 2635,
-    56 %, 41.3, 41.2). Of 410 sizes none is more than 1 % behind, 1.38 times as fast in the
-    mean."""
+    at 2378, 51 %, 39.6, 41.3, 2816 x 2048 at 3176, 53 %, 40.3, 41.0, at 3069 48.8, 42.8;
+    six layers with 2048 x 2048 at 4379 rows, 53 %, are 60 us slower with the library). Of
+    410 sizes one is more than 1 % behind, 1.38 times as fast in the mean."""
     if M <= 256:
         return False
     fill = _tile_fill(M, N)
     return fill >= 0.82 or (K <= 2048 and M >= 1000 and fill >= (
-        0.535 if K > 1536 and _tile_plan(M, N)[0] == "whole" else 0.42))
+        0.52 if K > 1536 and _tile_plan(M, N)[0] == "whole" else 0.42))
 
 
 def _vocabulary_shape(M: int, N: int, K: int) -> bool:

@@ -179,7 +179,8 @@ def test_operands_that_the_kernels_refuse():
     (1000, 22016, 4096, False), (1500, 16384, 3072, False),
     (700, 4096, 2048, False), (1000, 4096, 2048, True),
     (1500, 1024, 2048, False), (2048, 1024, 2048, False),
-    (2378, 3584, 2048, False), (2635, 3584, 2048, True)])
+    (2378, 3584, 2048, False), (2635, 3584, 2048, True),
+    (4379, 2048, 2048, True)])
 def test_which_pairs_take_tiles(M, N, K, tiles):
     """The sides of the line on which either was measured to be faster."""
     assert ops._tiled_shape(M, N, K) == tiles
