@@ -484,8 +484,8 @@ def _tiled_shape(M: int, N: int, K: int) -> bool:
     8192 339, 189, at 1000, 57 %, 43, 54; 16384 x 3072 at 1500, 81 %, 144, 158;
     4096 x 2048 at 1000 26, 20, 8192 118, 107; 1024 x 2048 at 2048, 31 %, 20, 19 and
     1500 18, 19; 2816 x 2048 at 1500, 42 %, 28, 27; in one round of 256 x 256 3584 x 2048
-    at 2378, 51 %, 39.6, 41.3, 2816 x 2048 at 3176, 53 %, 40.3, 41.0, at 3069 48.8, 42.8;
-    six layers with 2048 x 2048 at 4379 rows, 53 %, are 60 us slower with the library). Of
+    at 2378, 51 %, 39.6, 41.3, with weights from memory 44.2, 44.6, 2816 x 2048 at 3176,
+    53 %, 40.3, 41.0 and 45.1, 43.8, 2048 x 2048 at 4379, 53 %, from memory 51.2, 43.3). Of
     410 sizes one is more than 1 % behind, 1.38 times as fast in the mean."""
     if M <= 256:
         return False
